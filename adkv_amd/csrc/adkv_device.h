@@ -193,66 +193,82 @@ __device__ __forceinline__ int quantize(h1 x, h1 zp, h1 sc)
     return (int)r;
 }
 
-// The encoder's form of quantize(): the same value with as few dependent instructions between
-// one token's state and the next as the arithmetic allows.
-//  * x - zp is one mixed-precision fma on the fp16 halves in place (f32(x)*1 - f32(zp), rounded
-//    once: exactly the reference's fp32 difference) instead of two conversions and a subtract.
-//  * rsc is the hardware reciprocal of sc (1 ulp), taken as soon as sc is known.  r = d*rsc is
-//    within 2^-22 relative of the exact quotient u, so for |r| < 16 it is within 2^-18 absolute:
-//    unless r lies closer than 2^-16 to a rounding boundary k + 1/2, rint(r) == rint(u) (exact
-//    ties always land in that band).  For |r| >= 16 both u and r are beyond the clamp on the same
-//    side, whatever rint gives.  Inside the band, and for NaN (which ends as code 0, like CUDA's
-//    __float2int_rn), the exact divide decides; that branch is taken by about one element in
-//    30 000.
-//  * The result is the clamped code as a float (an integer in [QLO, QHI]): the fp16 operands of
-//    the state update are converted from it directly, the integer for the code word off the
-//    critical path.
-// xw / zpw hold the fp16 operands in their low (HI = false) or high (HI = true) halves.
-template <int BITS, bool HI>
-__device__ __forceinline__ float quantize_enc_fast(uint32_t xw, uint32_t zpw, h1 sc, float rsc)
+// The encoder's fast form of quantize(): x - zp is one mixed-precision fma on the fp16 halves in
+// place (f32(x)*1 - f32(zp), rounded once: exactly the reference's fp32 difference) instead of two
+// conversions and a subtract.
+template <bool HI>
+__device__ __forceinline__ float enc_diff(uint32_t xw, uint32_t zpw)
 {
     float d;
     if (HI)
         asm("v_fma_mix_f32 %0, %1, 1.0, -%2 op_sel:[1,0,1] op_sel_hi:[1,0,1]" : "=v"(d) : "v"(xw), "v"(zpw));
     else
         asm("v_fma_mix_f32 %0, %1, 1.0, -%2 op_sel_hi:[1,0,1]" : "=v"(d) : "v"(xw), "v"(zpw));
-    const float r = d * rsc;
-    float n = __builtin_rintf(r);
-    if (__builtin_expect(!(__builtin_fabsf(r - n) < 0.5f - 0x1p-16f), 0)) {
-        n = __builtin_rintf(d / (float)sc);
-        n = (n != n) ? 0.0f : n;
-    }
-    return __builtin_amdgcn_fmed3f(n, (float)Code<BITS>::QLO, (float)Code<BITS>::QHI);
+    return d;
+}
+// The IEEE fp32 quotient d / s for d a difference of two fp16 numbers and s an fp16 number, from
+// rs = v_rcp_f32(s) (1 ulp).  q = d*rs is within an ulp or so of the quotient, rem = d - q*s is then
+// exact, and q + rem*rs = (d/s)(1 + 2^-46) before its one rounding.  That rounds like d/s itself:
+// s has 11 significant bits, so a d/s that is not the midpoint of two fp32 neighbours differs from
+// every midpoint (25 bits) by at least 2^-37 of itself, and it cannot be a midpoint, whose product
+// with s needs 25 bits or more where d has 24.  Neither overflow nor underflow can occur (|d| from
+// 2^-24 to 2^17, |s| from 2^-24 to 2^16).  For s = 0 or a non-finite operand the result is a NaN.
+__device__ __forceinline__ float enc_quotient(float d, float s, float rs)
+{
+    const float q = d * rs;
+    const float rem = __builtin_fmaf(-q, s, d);
+    return __builtin_fmaf(rem, rs, q);
+}
+// NaN once any of its operands is (the others only have to be there)
+__device__ __forceinline__ float enc_collect_nan(float acc, float a, float b)
+{
+    float r;
+    asm("v_maximum3_f32 %0, %1, %2, %3" : "=v"(r) : "v"(acc), "v"(a), "v"(b));
+    return r;
 }
 
-// quantize_enc_fast without its branch, for lanes whose wave is alone on its SIMD and pays every
-// dependent instruction in full: the code is taken from the reciprocal product unconditionally and
-// the squared distance of r from its integer is folded into `worst` as an unsigned maximum (a NaN
-// has the largest bit pattern of all).  A caller that finds worst >= ENC_SPEC_LIMIT afterwards
-// must discard the codes and the state derived from them and redo the tokens with
-// quantize_enc_fast.  Squaring is monotonic, so every |r - n| >= 0.5 - 2^-16 is caught.
-constexpr float ENC_SPEC_EDGE = 0.5f - 0x1p-16f;
-constexpr float ENC_SPEC_LIMIT = ENC_SPEC_EDGE * ENC_SPEC_EDGE;
-template <int BITS, bool HI>
-__device__ __forceinline__ float quantize_enc_spec(uint32_t xw, uint32_t zpw, float rsc, uint32_t &worst)
+// Eight tokens of one channel per lane, 14 instructions each (16 issue slots: v_fma_f16 and v_rcp_f32
+// take two) and laid out by hand.  The state keeps the scale in the HIGH half of qs_sc, so that one
+// packed multiply by (code, f) gives both the code's value q*sc (low) and the next scale sc*f
+// (high); f = be*|q| + omt is written by v_fma_f16 into the high half of the register that holds q.
+// Waits the hardware does not make by itself, filled with useful instructions where there is one:
+// a packed or half-register result is not read by the next instruction, nor is v_rcp_f32's.
+struct Chan1 {
+    uint32_t zp;    // low half; the high half is never read
+    uint32_t qs_sc; // high half: the scale
+    float rs;       // v_rcp_f32 of the scale
+};
+template <int BITS>
+__device__ __forceinline__ void enc_eight_tokens(Chan1 &c, const uint16_t *x, uint32_t al, uint32_t be, uint32_t omt,
+                                                 float lo, float hi, uint32_t &word, float &nan)
 {
-    float d;
-    if (HI)
-        asm("v_fma_mix_f32 %0, %1, 1.0, -%2 op_sel:[1,0,1] op_sel_hi:[1,0,1]" : "=v"(d) : "v"(xw), "v"(zpw));
-    else
-        asm("v_fma_mix_f32 %0, %1, 1.0, -%2 op_sel_hi:[1,0,1]" : "=v"(d) : "v"(xw), "v"(zpw));
-    const float r = d * rsc;
-    const float n = __builtin_rintf(r);
-    const float e = r - n;
-    const uint32_t e2 = __float_as_uint(e * e);
-    worst = worst > e2 ? worst : e2;
-    return __builtin_amdgcn_fmed3f(n, (float)Code<BITS>::QLO, (float)Code<BITS>::QHI);
-}
-
-// Two small integers held as floats -> fp16 pair (exact, so the rounding mode is irrelevant).
-__device__ __forceinline__ h2 pack_codes(float a, float b)
-{
-    return __builtin_bit_cast(h2, __builtin_amdgcn_cvt_pkrtz(a, b));
+    float d, r0, r1, t;
+    uint32_t u, q;
+#define ADKV_ENC_TOKEN(X, R, FILL)                                                                       \
+    "v_fma_mix_f32 %[d], " X ", 1.0, -%[zp] op_sel_hi:[1,0,1]\n\t"                                       \
+    "v_mul_f32 " R ", %[d], %[rs]\n\t"                                                                  \
+    "v_fma_mix_f32 %[t], -" R ", %[ss], %[d] op_sel:[0,1,0] op_sel_hi:[0,1,0]\n\t"                      \
+    "v_fmac_f32 " R ", %[t], %[rs]\n\t"                                                                 \
+    "v_add_f32 %[u], 0x4b400000, " R "\n\t"                                                             \
+    "v_med3_f32 %[u], %[u], %[lo], %[hi]\n\t"                                                           \
+    "v_cvt_f16_i16 %[q], %[u]\n\t"                                                                      \
+    "v_fma_f16 %[q], %[be], |%[q]|, %[omt] op_sel:[0,0,0,1]\n\t"                                        \
+    "v_alignbit_b32 %[w], %[u], %[w], %[bits]\n\t"                                                      \
+    "v_pk_mul_f16 %[ss], %[ss], %[q] op_sel:[1,0] op_sel_hi:[1,1]\n\t"                                  \
+    FILL "\n\t"                                                                                         \
+    "v_cvt_f32_f16_sdwa %[t], %[ss] dst_sel:DWORD dst_unused:UNUSED_PAD src0_sel:WORD_1\n\t"            \
+    "v_pk_fma_f16 %[zp], %[al], %[ss], %[zp]\n\t"                                                       \
+    "v_rcp_f32 %[rs], %[t]\n\t"
+#define ADKV_ENC_PAIR(X0, X1)                       \
+    ADKV_ENC_TOKEN(X0, "%[r0]", "s_nop 0")         \
+    ADKV_ENC_TOKEN(X1, "%[r1]", "v_maximum3_f32 %[nan], %[nan], %[r0], %[r1]")
+    asm(ADKV_ENC_PAIR("%[x0]", "%[x1]") ADKV_ENC_PAIR("%[x2]", "%[x3]") ADKV_ENC_PAIR("%[x4]", "%[x5]") ADKV_ENC_PAIR("%[x6]", "%[x7]")
+        : [zp] "+v"(c.zp), [ss] "+v"(c.qs_sc), [rs] "+v"(c.rs), [w] "+v"(word), [nan] "+v"(nan), [d] "=&v"(d), [t] "=&v"(t),
+          [u] "=&v"(u), [q] "=&v"(q), [r0] "=&v"(r0), [r1] "=&v"(r1)
+        : [x0] "v"(x[0]), [x1] "v"(x[1]), [x2] "v"(x[2]), [x3] "v"(x[3]), [x4] "v"(x[4]), [x5] "v"(x[5]), [x6] "v"(x[6]),
+          [x7] "v"(x[7]), [al] "v"(al), [be] "v"(be), [omt] "v"(omt), [lo] "s"(lo), [hi] "v"(hi), [bits] "n"(BITS));
+#undef ADKV_ENC_PAIR
+#undef ADKV_ENC_TOKEN
 }
 
 __device__ __forceinline__ h2 codes_to_h2(int q0, int q1) { return (h2){(h1)q0, (h1)q1}; }

@@ -425,13 +425,28 @@ __device__ __forceinline__ void init_pairs(Pair *st, const h1 *zp, const h1 *sc,
 // ---------------------------------------------------------------------------------------------
 // The state at token t depends on every code before it, so the encoder is one serial chain per
 // channel and nothing but B*H*D is parallel.  A lane owns CPL consecutive channels (1 or 2, the
-// launcher's choice).  With few channels every wave has a SIMD to itself and the time per token
-// is the length of its instruction stream, so that stream is kept short: the dependent chain from
-// one token's state to the next is mixed-precision fma -> mul -> rint -> med3 -> pack -> packed
-// mul -> packed fma, input rows are loaded two groups of 8 tokens ahead with nothing waiting on
-// them, codes are summed as signed q << 4t in floats (one fma each) and biased once by 0x8888...,
-// row pointers advance by addition, checkpoints are found by comparison.
-constexpr int ENC_PF = 3; // supergroup input buffers in rotation
+// launcher's choice).  With few channels a wave has its SIMD to itself, and a wave alone issues one
+// instruction every 4 cycles whether or not it depends on the one before (8 for v_rcp_f32 and
+// v_fma_f16; s_nop, s_waitcnt and scalar instructions take a slot as well): the time per token is
+// the NUMBER of instructions, and the loop below is written for that number.
+//  * rows come through buffer loads (16 bits per lane with one channel, 32 with two): one
+//    instruction per token and nothing else, because the row offsets within a group of 8 tokens
+//    sit in scalar registers and loads past the end of the stream are dropped by the bounds check
+//    instead of being guarded;
+//  * the quotient takes three instructions on top of the reciprocal and is the IEEE one
+//    (enc_quotient), so nothing has to be checked or repeated for finite values: a form that takes
+//    the reciprocal product alone and repeats the groups of 8 tokens in which it comes near a
+//    rounding boundary repeats one group in seven, because exact ties are common (both sides of the
+//    division have few significant bits);
+//  * adding 1.5 * 2^23 + bias rounds the quotient to the nearest integer and leaves the code in the
+//    low bits, clamped by one med3; v_alignbit shifts it into the code word (one instruction per
+//    code), v_cvt_f16_i16 (one channel) or a byte permute and one packed fma (two) turn it into the
+//    fp16 operand of the update.
+// Only a quotient that is not a number (a non-finite input or state, a zero scale) sends its
+// group of 8 tokens through the plain division; half an instruction per token looks for one.
+constexpr int ENC_PF1 = 8;    // buffers of 8 rows in rotation, one channel per lane (one wave per SIMD: nothing else hides HBM)
+constexpr int ENC_AHEAD1 = 6; // groups loaded ahead: 56 loads and their groups' stores fit the 63 the counter holds
+constexpr int ENC_PF2 = 4; // two channels per lane (many waves)
 
 // Where the new rows are: element strides between batches, heads and tokens (channels are
 // contiguous).  The encoder reads each row once, 256 bytes per head, so a [B, T, H, D] projection
@@ -439,6 +454,12 @@ constexpr int ENC_PF = 3; // supergroup input buffers in rotation
 struct RowStrides {
     long b, h, t;
 };
+
+__device__ __forceinline__ uint64_t wave_uniform(uint64_t v)
+{
+    const uint32_t lo = __builtin_amdgcn_readfirstlane((uint32_t)v), hi = __builtin_amdgcn_readfirstlane((uint32_t)(v >> 32));
+    return ((uint64_t)hi << 32) | lo;
+}
 
 template <int BITS, int CPL, int BLK, bool BF16 = false>
 __device__ __forceinline__ void encode_body(
@@ -450,104 +471,68 @@ __device__ __forceinline__ void encode_body(
 {
     // Quantises tokens [T0, T) of a stream whose first T0 tokens are already in the cache; kv_new
     // holds the T - T0 new rows; state_in is the state after token T0-1 (ignored when T0 == 0).
-    constexpr int NP = CPL >= 2 ? CPL / 2 : 1;
+    static_assert(CPL == 1 || CPL == 2, "one channel per lane, or one packed pair");
     constexpr int TPW = Code<BITS>::TPW; // tokens per channel word
     constexpr int G8 = TPW / 8;          // 8-token input groups per word
-    const long total = (long)BH * D;
-    long ci = ((long)blockIdx.x * BLK + threadIdx.x) * CPL;
-    const bool active = ci < total;
-    if (!active)
-        ci = total - CPL;
-    const int bx = (int)(ci / D), c0 = (int)(ci % D);
+    constexpr int PF = CPL == 1 ? ENC_PF1 : ENC_PF2;
+    constexpr int AHEAD = CPL == 1 ? ENC_AHEAD1 : PF - 1;
+    // a wave's 64 * CPL channels lie inside one head (D is a multiple of 128), so everything but
+    // the channel itself is uniform over the wave and a wave past the end has no work at all
+    const int lane = threadIdx.x & 63;
+    const long ci = ((long)blockIdx.x * BLK + (threadIdx.x & ~63)) * CPL; // the wave's first channel
+    if (ci >= (long)BH * D)
+        return;
+    const int bx = __builtin_amdgcn_readfirstlane((int)(ci / D));
+    const int cw0 = __builtin_amdgcn_readfirstlane((int)(ci % D));
+    const int c0 = cw0 + lane * CPL;
     const int h = bx % H;
 
-    Pair st[NP];
-    if (CPL >= 2) {
-#pragma unroll
-        for (int p = 0; p < NP; p++)
-            load_pair(st[p], zp, sc, al, be, tg, h * D + c0 + 2 * p);
+    Pair st;
+    if (CPL == 2) {
+        load_pair(st, zp, sc, al, be, tg, h * D + c0);
     } else {
         const int pi = h * D + c0;
-        st[0].zp = splat(zp[pi]);
-        st[0].sc = splat(sc[pi]);
-        st[0].al = splat(al[pi]);
-        st[0].be = splat(be[pi]);
-        st[0].omt = splat((h1)1.0f) - st[0].be * splat(tg[pi]);
+        st.zp = splat(zp[pi]);
+        st.sc = splat(sc[pi]);
+        st.al = splat(al[pi]);
+        st.be = splat(be[pi]);
+        st.omt = splat((h1)1.0f) - st.be * splat(tg[pi]);
     }
     if (T0 > 0) {
         const h1 *si = state_in + ((size_t)bx * D + c0) * 2;
-        if (CPL >= 2) {
-            load_state<CPL>(si, st);
+        if (CPL == 2) {
+            load_state<2>(si, &st);
         } else {
-            st[0].zp = splat(si[0]);
-            st[0].sc = splat(si[1]);
+            st.zp = splat(si[0]);
+            st.sc = splat(si[1]);
         }
     }
 
-    uint32_t *cw = cache + (size_t)bx * n_super_cap * D + c0;
-    const h1 *xb = kv_new + (long)(bx / H) * xs.b + (long)h * xs.h + c0; // rows of tokens T0.. of this head
+    uint32_t *cw = cache + (size_t)bx * n_super_cap * D + cw0;                                 // the wave's code words
+    const h1 *xb = kv_new + (long)(bx / H) * xs.b + (long)h * xs.h + cw0 - (long)T0 * xs.t;    // its row of token 0
 
-    // One token's CPL channels as NP aligned 32-bit words of the input row (an fp16 pair each; a
-    // one-channel lane takes the word its channel lies in and shifts at use).  The loads carry no
-    // arithmetic, and no 16-bit values the compiler would pack in pairs across the loop edge, so
-    // nothing waits for a load until its token is quantised.
-    using XW = uint32_t;
-    const h1 *xbw = xb - (CPL == 1 ? (c0 & 1) : 0);
-    const uint32_t xsh = CPL == 1 ? (uint32_t)(c0 & 1) * 16u : 0u;
-    auto load_tok = [&](int t, XW *x) {
-#pragma unroll
-        for (int p = 0; p < NP; p++)
-            x[p] = *reinterpret_cast<const XW *>(xbw + (long)(t - T0) * xs.t + 2 * p);
+    // one token's input: a word with an fp16 (or bf16) pair, or one 16-bit value
+    using XW = typename std::conditional<CPL == 2, uint32_t, uint16_t>::type;
+    auto as_f16 = [](XW w) -> XW {
+        if (!BF16)
+            return w;
+        // bf16 -> fp32 is exact, fp32 -> fp16 rounds to nearest even: torch's .to(float16)
+        const h1 lo = (h1)__uint_as_float((uint32_t)w << 16);
+        if constexpr (CPL == 1)
+            return __builtin_bit_cast(uint16_t, lo);
+        else
+            return as_u32((h2){lo, (h1)__uint_as_float(w & 0xFFFF0000u)});
     };
-    // reciprocal of the current scale, refreshed right after every update (see quantize_enc_fast)
-    float rs[NP][2];
-    auto refresh = [&](int p) {
-        rs[p][0] = __builtin_amdgcn_rcpf((float)st[p].sc.x);
-        rs[p][1] = CPL >= 2 ? __builtin_amdgcn_rcpf((float)st[p].sc.y) : rs[p][0];
+    // exact step with the IEEE divide: partial words and groups that failed the check
+    auto step = [&](XW xw, int *qi) {
+        const h2 x = as_h2((uint32_t)as_f16(xw));
+        qi[0] = quantize<BITS>(x.x, st.zp.x, st.sc.x);
+        if (CPL == 2)
+            qi[1] = quantize<BITS>(x.y, st.zp.y, st.sc.y);
+        const h2 q = codes_to_h2(qi[0], qi[CPL - 1]);
+        update_pair(st, q, q * st.sc);
     };
-#pragma unroll
-    for (int p = 0; p < NP; p++)
-        refresh(p);
-    // quantise one token with the current state, advance the state; qf = the codes as floats.
-    // spec: branch-free speculative form (see quantize_enc_spec), the caller checks `worst`.
-    uint32_t worst = 0u;
-    auto advance = [&](auto spec, const XW *x, float *qf) {
-#pragma unroll
-        for (int p = 0; p < NP; p++) {
-            XW xw = CPL == 1 ? x[p] >> xsh : x[p];
-            if (BF16) {
-                // bf16 -> fp32 is exact, fp32 -> fp16 rounds to nearest even: torch's .to(float16)
-                const h1 lo = (h1)__uint_as_float(xw << 16);
-                const h1 hi = CPL == 1 ? lo : (h1)__uint_as_float(xw & 0xFFFF0000u);
-                xw = as_u32((h2){lo, hi});
-            }
-            const uint32_t zw = __builtin_bit_cast(uint32_t, st[p].zp);
-            float q0, q1;
-            if constexpr (decltype(spec)::value) {
-                q0 = quantize_enc_spec<BITS, false>(xw, zw, rs[p][0], worst);
-                q1 = CPL >= 2 ? quantize_enc_spec<BITS, true>(xw, zw, rs[p][1], worst) : q0;
-            } else {
-                q0 = quantize_enc_fast<BITS, false>(xw, zw, st[p].sc.x, rs[p][0]);
-                q1 = CPL >= 2 ? quantize_enc_fast<BITS, true>(xw, zw, st[p].sc.y, rs[p][1]) : q0;
-            }
-            qf[CPL >= 2 ? 2 * p : 0] = q0;
-            if (CPL >= 2)
-                qf[2 * p + 1] = q1;
-            const h2 q = pack_codes(q0, q1);
-            update_pair_abs(st[p], pack_codes(__builtin_fabsf(q0), __builtin_fabsf(q1)), q * st[p].sc);
-            refresh(p);
-        }
-    };
-    using Exact = std::integral_constant<bool, false>;
-    using Spec = std::integral_constant<bool, true>;
-    // partial words: token slot known at run time only
-    auto step = [&](const XW *x, int tt, uint32_t *w) {
-        float qf[CPL];
-        advance(Exact{}, x, qf);
-#pragma unroll
-        for (int c = 0; c < CPL; c++)
-            w[c] += (uint32_t)(int)qf[c] << (BITS * tt);
-    };
+    auto load_tok = [&](int t) { return *reinterpret_cast<const XW *>(xb + (long)t * xs.t + lane * CPL); };
     // Checkpoints: entry j is the state before token (j+1)*interval.  Words are stored in order,
     // so the next boundary is tracked by comparison instead of a division per word.
     int ck_next = -1, ck_j = 0;
@@ -556,174 +541,208 @@ __device__ __forceinline__ void encode_body(
         ck_j = (first_end + sa.ckpt_interval - 1) / sa.ckpt_interval - 1;
         ck_next = (ck_j + 1) * sa.ckpt_interval;
     }
-    // bias adds -QLO to the codes written now; keep selects codes of earlier tokens to preserve
-    auto store_sg = [&](int sg, const uint32_t *w, uint32_t bias, uint32_t keep) {
-        const int tend = sg * TPW + TPW;
-        const bool ck_here = tend == ck_next;
-        if (ck_here) {
-            ck_next += sa.ckpt_interval;
-            ck_j++;
-        }
-        if (!active)
+    auto checkpoint = [&](int tend) {
+        if (__builtin_expect(tend != ck_next, 1))
             return;
-        uint32_t *dst = cw + (size_t)sg * D;
-        uint32_t o[CPL];
-#pragma unroll
-        for (int c = 0; c < CPL; c++)
-            o[c] = w[c] + bias;
-        if (keep) {
-#pragma unroll
-            for (int c = 0; c < CPL; c++)
-                o[c] = (o[c] & ~keep) | (dst[c] & keep);
-        }
-        if (CPL == 4)
-            *reinterpret_cast<uint4 *>(dst) = make_uint4(o[0], o[1], o[2], o[3]);
-        else if (CPL == 2)
-            *reinterpret_cast<uint2 *>(dst) = make_uint2(o[0], o[1]);
-        else
-            dst[0] = o[0];
-        if (ck_here && tend <= T && ck_j - 1 < sa.n_ckpt_cap)
-            store_state_n<CPL>(sa.ckpt + (((size_t)bx * sa.n_ckpt_cap + (ck_j - 1)) * D + c0) * 2, st);
+        if (tend <= T && ck_j < sa.n_ckpt_cap)
+            store_state_n<CPL>(sa.ckpt + (((size_t)bx * sa.n_ckpt_cap + ck_j) * D + c0) * 2, &st);
+        ck_next += sa.ckpt_interval;
+        ck_j++;
     };
-
-    auto nib_mask = [](int k) { return k >= TPW ? 0xFFFFFFFFu : ((1u << (BITS * k)) - 1u); };
-    constexpr uint32_t BIAS = Code<BITS>::BIAS;
-
-    // a stream that resumes inside a word first completes it (codes below T0 are kept)
-    int t = T0;
-    if ((t % TPW) && t < T) {
-        const int lo = t % TPW, sg = t / TPW;
+    // a word of which only the codes of tokens [lo, hi) are new (codes below lo are kept, the fields
+    // from hi on are zero)
+    auto partial_word = [&](int sg, int lo, int hi) {
+        uint32_t *dst = cw + (size_t)sg * D + lane * CPL;
+        const uint32_t keep = lo ? (1u << (BITS * lo)) - 1u : 0u;
         uint32_t w[CPL];
 #pragma unroll
         for (int c = 0; c < CPL; c++)
-            w[c] = 0u;
-        for (; t < T && t / TPW == sg; t++) {
-            XW x[NP];
-            load_tok(t, x);
-            step(x, t % TPW, w);
-        }
-        const int hi = t / TPW == sg ? t % TPW : TPW;
-        store_sg(sg, w, BIAS & nib_mask(hi) & ~nib_mask(lo), nib_mask(lo));
-    }
-
-    // full words: no per-token conditions, inputs ENC_PF-1 groups of 8 tokens ahead.  The loads
-    // are unconditional (index clamped to the last group): a load under a condition has to land
-    // before the code after the condition runs, which would expose the memory latency per group.
-    const int sgb = t / TPW;                    // first full word
-    const int nfull = (T - t) / TPW;
-    const int ng = nfull * G8;
-    XW xbuf[ENC_PF][8][NP];
-    uint32_t w[CPL];
-#pragma unroll
-    for (int c = 0; c < CPL; c++)
-        w[c] = 0u;
-    // loads the next group of 8 rows; past the last group the same rows are loaded again
-    const h1 *xnext = xbw + (long)(t - T0) * xs.t;
-    int gnext = 0;
-    auto load_next = [&](XW (*xg)[NP]) {
-#pragma unroll
-        for (int tt = 0; tt < 8; tt++) {
-#pragma unroll
-            for (int p = 0; p < NP; p++)
-                xg[tt][p] = *reinterpret_cast<const XW *>(xnext + (long)tt * xs.t + 2 * p);
-        }
-        if (gnext < ng - 1) {
-            xnext += 8 * xs.t;
-            gnext++;
-        }
-    };
-    // The codes of 16/BITS tokens fill 16 bits; their signed sum q << BITS*k is exact in one
-    // float (|sum| < 2^20), one fma per code, and two halves make the 32-bit word.
-    constexpr int TPA = 16 / BITS; // tokens per half word
-    constexpr int NA = 8 / TPA;    // half words an 8-token group fills
-    auto run_group = [&](auto spec, const XW (*xg)[NP], float (*acc)[NA]) {
-#pragma unroll
-        for (int tt = 0; tt < 8; tt++) {
-            float qf[CPL];
-            advance(spec, xg[tt], qf);
-#pragma unroll
-            for (int c = 0; c < CPL; c++) {
-                if (tt % TPA == 0)
-                    acc[c][tt / TPA] = qf[c];
-                else
-                    acc[c][tt / TPA] = __builtin_fmaf(qf[c], (float)(1u << (BITS * (tt % TPA))),
-                                                      acc[c][tt / TPA]);
-            }
-        }
-    };
-    // Lanes of one channel belong to waves that have a SIMD to themselves (that is when the
-    // launcher picks them), so they run a group speculatively without the per-token branch and
-    // repeat it exactly from the saved state when any lane of the wave came near a rounding
-    // boundary (about one group in sixty).
-    constexpr bool SPECULATE = CPL == 1;
-    auto do_group = [&](int g, const XW (*xg)[NP]) {
-        float acc[CPL][NA];
-        if (SPECULATE) {
-            Pair saved[NP];
-#pragma unroll
-            for (int p = 0; p < NP; p++)
-                saved[p] = st[p];
-            worst = 0u;
-            run_group(Spec{}, xg, acc);
-            if (__any(worst >= __float_as_uint(ENC_SPEC_LIMIT))) {
-#pragma unroll
-                for (int p = 0; p < NP; p++) {
-                    st[p] = saved[p];
-                    refresh(p);
-                }
-                run_group(Exact{}, xg, acc);
-            }
-        } else {
-            run_group(Exact{}, xg, acc);
-        }
-#pragma unroll
-        for (int c = 0; c < CPL; c++) {
-            uint32_t v = (uint32_t)(int)acc[c][0];
-            if (NA == 2)
-                v += (uint32_t)(int)acc[c][NA - 1] << 16;
-            w[c] += G8 == 1 ? v : v << (16 * (g % G8));
-        }
-        if (G8 == 1 || g % G8 == G8 - 1) {
-            store_sg(sgb + g / G8, w, BIAS, 0u);
+            w[c] = keep ? dst[c] & keep : 0u;
+        for (int tt = lo; tt < hi; tt++) {
+            int qi[CPL];
+            step(load_tok(sg * TPW + tt), qi);
 #pragma unroll
             for (int c = 0; c < CPL; c++)
-                w[c] = 0u;
+                w[c] |= (uint32_t)(qi[c] - Code<BITS>::QLO) << (BITS * tt);
         }
-    };
-    if (ng > 0) {
-#pragma unroll
-        for (int i = 0; i < ENC_PF - 1; i++)
-            load_next(xbuf[i]);
-        int g0 = 0;
-        for (; g0 + ENC_PF <= ng; g0 += ENC_PF) {
-#pragma unroll
-            for (int i = 0; i < ENC_PF; i++) {
-                load_next(xbuf[(i + ENC_PF - 1) % ENC_PF]);
-                do_group(g0 + i, xbuf[i]);
-            }
-        }
-        // at most ENC_PF-1 groups left; their inputs are already in xbuf[0 .. ENC_PF-2]
-#pragma unroll
-        for (int i = 0; i < ENC_PF - 1; i++)
-            if (g0 + i < ng)
-                do_group(g0 + i, xbuf[i]);
-    }
-    // ragged last word: codes of the tokens present, zero fields after them
-    t += nfull * TPW;
-    if (t < T) {
-        const int ntail = T - t;
 #pragma unroll
         for (int c = 0; c < CPL; c++)
-            w[c] = 0u;
-        for (int tt = 0; tt < ntail; tt++) {
-            XW x[NP];
-            load_tok(t + tt, x);
-            step(x, tt, w);
-        }
-        store_sg(t / TPW, w, BIAS & nib_mask(ntail), 0u);
+            dst[c] = w[c];
+        checkpoint(sg * TPW + TPW);
+    };
+
+    // a stream that resumes inside a word first completes it
+    int sg = T0 / TPW;
+    if (T0 % TPW && T0 < T) {
+        partial_word(sg, T0 % TPW, T / TPW == sg ? T % TPW : TPW);
+        sg++;
     }
-    if (state_out != nullptr && active)
-        store_state_n<CPL>(state_out + ((size_t)bx * D + c0) * 2, st);
+
+    // Full words.  MAGIC + n is exact for the integers that matter, and its low bits are those of n.
+    // With two channels n is biased by -QLO, so that they are the stored code (the byte permute
+    // needs it non-negative); with one they are n's two's complement, as v_cvt_f16_i16 takes it, and
+    // the finished word is biased (an exclusive or with the sign bits).
+    constexpr float BIASF = CPL == 2 ? (float)-Code<BITS>::QLO : 0.0f;
+    constexpr uint32_t WORD_BIAS = CPL == 2 ? 0u : Code<BITS>::BIAS;
+    constexpr float MAGIC = 12582912.0f + BIASF; // 1.5 * 2^23
+    constexpr float ULO = MAGIC + (float)Code<BITS>::QLO, UHI = MAGIC + (float)Code<BITS>::QHI;
+    float uhi = UHI; // med3 takes one scalar operand
+    asm volatile("" : "+v"(uhi));
+    uint32_t w[CPL];
+    float nan = 0.0f; // becomes a NaN when a quotient was one
+    // two channels: the scale in fp32 and its reciprocal
+    float scf[2], rs[2];
+    // one channel: see enc_eight_tokens
+    Chan1 ch;
+    auto enter = [&]() {
+        if (CPL == 1) {
+            ch.zp = as_u32(st.zp);
+            ch.qs_sc = as_u32((h2){(h1)0.0f, st.sc.x});
+            ch.rs = __builtin_amdgcn_rcpf((float)st.sc.x);
+        } else {
+            scf[0] = (float)st.sc.x;
+            scf[1] = (float)st.sc.y;
+            rs[0] = __builtin_amdgcn_rcpf(scf[0]);
+            rs[1] = __builtin_amdgcn_rcpf(scf[1]);
+        }
+        nan = 0.0f;
+    };
+    auto leave = [&]() {
+        if (CPL == 1) {
+            st.zp = splat(as_h2(ch.zp).x);
+            st.sc = splat(as_h2(ch.qs_sc).y);
+        }
+    };
+    auto tokens8 = [&](const XW *x) {
+        if constexpr (CPL == 1) {
+            uint16_t y[8];
+#pragma unroll
+            for (int k = 0; k < 8; k++)
+                y[k] = as_f16(x[k]);
+            enc_eight_tokens<BITS>(ch, y, as_u32(st.al), as_u32(st.be), as_u32(st.omt), ULO, uhi, w[0], nan);
+        } else {
+#pragma unroll
+            for (int k = 0; k < 8; k++) {
+                const uint32_t xw = as_f16(x[k]), zw = as_u32(st.zp);
+                const float r0 = enc_quotient(enc_diff<false>(xw, zw), scf[0], rs[0]);
+                const float r1 = enc_quotient(enc_diff<true>(xw, zw), scf[1], rs[1]);
+                const uint32_t u0 = __float_as_uint(__builtin_amdgcn_fmed3f(r0 + MAGIC, ULO, uhi));
+                const uint32_t u1 = __float_as_uint(__builtin_amdgcn_fmed3f(r1 + MAGIC, ULO, uhi));
+                w[0] = __builtin_amdgcn_alignbit(u0, w[0], BITS);
+                w[CPL - 1] = __builtin_amdgcn_alignbit(u1, w[CPL - 1], BITS);
+                nan = enc_collect_nan(nan, r0, r1);
+                // bytes 3 and 0 of each: 0x4B, code = the fp16 number 14 + code/128
+                const h2 b = as_h2(__builtin_amdgcn_perm(u1, u0, 0x07040300u));
+                const h2 q = pk_fma(b, splat((h1)128.0f), splat((h1)(-1792.0f - BIASF)));
+                update_pair(st, q, q * st.sc);
+                scf[0] = (float)st.sc.x;
+                scf[1] = (float)st.sc.y;
+                rs[0] = __builtin_amdgcn_rcpf(scf[0]);
+                rs[1] = __builtin_amdgcn_rcpf(scf[1]);
+            }
+        }
+    };
+    // Streams longer than what a buffer descriptor can span are taken in pieces (and rows too far
+    // apart for one word's worth in a descriptor the slow way).
+    if (xs.t > (1L << 24))
+        for (; (sg + 1) * TPW <= T; sg++)
+            partial_word(sg, 0, TPW);
+    const int sg_end = T / TPW;
+    const long span_words = (1L << 30) / (xs.t * 2 * TPW);
+    const int piece = (int)(span_words >= PF ? span_words / PF * PF : max(span_words, 1L)); // whole runs where it can
+    while (sg < sg_end) {
+        const int nw = min(piece, sg_end - sg), ng = nw * G8; // words, 8-token groups of this piece
+        const uint32_t xbytes = (uint32_t)(((long)ng * 8 - 1) * xs.t * 2 + 128 * CPL);
+        const __amdgpu_buffer_rsrc_t xr = __builtin_amdgcn_make_buffer_rsrc(
+            (void *)wave_uniform((uint64_t)(xb + (long)sg * TPW * xs.t)), 0, (int)xbytes, 0x00027000);
+        uint32_t xoff = (uint32_t)lane * 2u * CPL;
+        const uint32_t row = (uint32_t)(xs.t * 2);
+        XW xbuf[PF][8];
+        auto load_next = [&](XW *xg) {
+#pragma unroll
+            for (int tt = 0; tt < 8; tt++)
+                xg[tt] = CPL == 2 ? (XW)__builtin_amdgcn_raw_buffer_load_b32(xr, (int)xoff, (int)(row * tt), 0)
+                                  : (XW)__builtin_amdgcn_raw_buffer_load_b16(xr, (int)xoff, (int)(row * tt), 0);
+            xoff += row * 8;
+        };
+        uint32_t *dst = cw + (size_t)sg * D + lane * CPL;
+        // group k of a run that starts at word sg; a word is stored when its last group is done
+        auto do_group = [&](auto kc, XW *xg, auto may_checkpoint) {
+            constexpr int k = decltype(kc)::value;
+            // one wait for the group's rows instead of one per token
+            asm volatile("" ::"v"(xg[0]), "v"(xg[1]), "v"(xg[2]), "v"(xg[3]), "v"(xg[4]), "v"(xg[5]), "v"(xg[6]), "v"(xg[7]));
+            tokens8(xg);
+            if constexpr (k % G8 == G8 - 1) {
+                if (CPL == 2)
+                    *reinterpret_cast<uint2 *>(dst) = make_uint2(w[0], w[CPL - 1]);
+                else
+                    *dst = w[0] ^ WORD_BIAS;
+                dst += D;
+                if constexpr (decltype(may_checkpoint)::value) {
+                    leave();
+                    checkpoint((sg + k / G8 + 1) * TPW);
+                }
+            }
+        };
+        // Quotients are looked at once per run of groups; a run that met a NaN is done again from
+        // its first word with the plain division.
+        auto run = [&](int words, auto &&groups) {
+            const Pair saved = st;
+            const int saved_next = ck_next, saved_j = ck_j;
+            groups();
+            leave();
+            if (__builtin_expect(__any(nan != nan), 0)) {
+                st = saved;
+                ck_next = saved_next;
+                ck_j = saved_j;
+                for (int i = 0; i < words; i++)
+                    partial_word(sg + i, 0, TPW);
+                enter();
+            }
+            sg += words;
+        };
+        enter();
+#pragma unroll
+        for (int i = 0; i < AHEAD; i++)
+            load_next(xbuf[i]);
+        int g = 0;
+        // Two copies of the loop rather than a test in it: where the paths met again, the buffers
+        // in flight would be copied, and waited for.
+        auto runs = [&](auto inner_checkpoints) __attribute__((always_inline)) {
+            for (; g + PF <= ng; g += PF) {
+                run(PF / G8, [&]() __attribute__((always_inline)) {
+                    static_for<PF>([&](auto ic) __attribute__((always_inline)) {
+                        // loads moved up over the last use of their buffer would be copied into it
+                        __builtin_amdgcn_sched_barrier(0);
+                        load_next(xbuf[(decltype(ic)::value + AHEAD) % PF]);
+                        __builtin_amdgcn_sched_barrier(0);
+                        do_group(ic, xbuf[decltype(ic)::value], inner_checkpoints);
+                    });
+                });
+                if constexpr (!decltype(inner_checkpoints)::value)
+                    checkpoint(sg * TPW);
+            }
+        };
+        // Checkpoint boundaries fall between runs (every 64 tokens with one channel per lane) for any
+        // usual interval and a stream that starts at one; only other plans look after every word.
+        if (sa.ckpt == nullptr || (sa.ckpt_interval % (8 * PF) == 0 && sg * TPW % (8 * PF) == 0))
+            runs(std::integral_constant<bool, false>{});
+        else
+            runs(std::integral_constant<bool, true>{});
+        if (g < ng) // at most PF-1 groups, whole words; the first AHEAD of their inputs are in xbuf already
+            run((ng - g) / G8, [&]() __attribute__((always_inline)) {
+                static_for<PF - 1 - AHEAD>([&](auto ic) __attribute__((always_inline)) { load_next(xbuf[AHEAD + decltype(ic)::value]); });
+                static_for<PF - 1>([&](auto ic) __attribute__((always_inline)) {
+                    if (g + decltype(ic)::value < ng)
+                        do_group(ic, xbuf[decltype(ic)::value], std::integral_constant<bool, true>{});
+                });
+            });
+    }
+    // ragged last word: codes of the tokens present, zero fields after them
+    if (T0 < T && sg * TPW < T)
+        partial_word(sg, 0, T - sg * TPW);
+    if (state_out != nullptr)
+        store_state_n<CPL>(state_out + ((size_t)bx * D + c0) * 2, &st);
 }
 
 template <int BITS, int CPL, int BLK>
@@ -2350,15 +2369,15 @@ static int encode_common(void *cache, const void *kv_new,
     seg.intervals = 0;
     seg.phys_per_head = 0;
     seg.skew = 0;
-    // Lane width, measured on an MI355X (4096 tokens, ms for 65 536 / 131 072 / 196 608 / 262 144 /
-    // 524 288 channels): one channel per lane 0.29 / 0.44 / 0.60 / 0.74 / 1.38, two 0.43 / 0.44 /
-    // 0.55 / 0.60 / 1.17, four 0.78 / 0.78 / 0.78 / 0.79 / 1.18.  Up to two waves per SIMD the
-    // one-channel lanes win (each wave is paced by its own dependent chain, and only they run the
-    // branch-free speculative form); beyond that two channels share the packed fp16 updates.
-    // Four channels per lane never win and are not instantiated.
+    // Lane width: one channel per lane while every wave then has a SIMD to itself (its time per token is
+    // its instruction count, 17 against 30 with two channels), two channels beyond (they share the
+    // packed updates and the wave's fixed cost).  ns per token, fp16 rows of 8192 tokens, 4-bit codes, at
+    // 0.25 / 1 / 1.5 / 2 one-channel waves per SIMD: one channel 37 / 42 / 67 / 71, two - / - / 64 / 69
+    // (4.8 TB/s, what the memory gives).  Before the loop was written for its instruction count: 61 at
+    // one wave per SIMD.
     const long channels = (long)BH * D;
     const long tensors = second ? 2 : 1;
-    int cpl = tensors * channels > 2L * 64 * n_simd() + 32768 ? 2 : 1;
+    int cpl = tensors * channels > 64L * n_simd() ? 2 : 1;
     const long lanes = channels / cpl;
     const dim3 grid((unsigned)((lanes + 255) / 256), (unsigned)tensors), block(256);
     EncTensor first;
