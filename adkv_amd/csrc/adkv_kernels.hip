@@ -96,6 +96,7 @@ struct Seg {
     int intervals;
     int phys_per_head;
     unsigned skew;      // shares of the four wave slots, oldest first, one byte each, in sixteenths
+    int fresh;          // encoder: the cache and checkpoint memory is uninitialised, write what is past the tokens too
 };
 
 __host__ __device__ inline int ft_skew(unsigned skew, int k) { return (int)((skew >> (8 * k)) & 0xFFu); }
@@ -741,6 +742,17 @@ __device__ __forceinline__ void encode_body(
     // ragged last word: codes of the tokens present, zero fields after them
     if (T0 < T && sg * TPW < T)
         partial_word(sg, 0, T - sg * TPW);
+    if (sa.fresh) { // free slots are zero, as the appending kernels expect
+        for (int i = (T + TPW - 1) / TPW; i < n_super_cap; i++)
+#pragma unroll
+            for (int c = 0; c < CPL; c++)
+                cw[(size_t)i * D + lane * CPL + c] = 0u;
+        if (sa.ckpt != nullptr)
+            for (int j = T / sa.ckpt_interval; j < sa.n_ckpt_cap; j++)
+#pragma unroll
+                for (int c = 0; c < CPL; c++)
+                    reinterpret_cast<uint32_t *>(sa.ckpt)[((size_t)bx * sa.n_ckpt_cap + j) * D + c0 + c] = 0u;
+    }
     if (state_out != nullptr)
         store_state_n<CPL>(state_out + ((size_t)bx * D + c0) * 2, &st);
 }
@@ -1276,85 +1288,6 @@ __global__ __launch_bounds__(256) void ov_finalize_wide_kernel(const float *__re
 }
 
 // ---------------------------------------------------------------------------------------------
-// Rotary position embedding of q and k in one launch   (llama_adkv.py:336-337 calls transformers'
-// apply_rotary_pos_emb: x * cos + rotate_half(x) * sin, ten elementwise launches)
-// ---------------------------------------------------------------------------------------------
-// Every operation is rounded to the activations' type the way torch's elementwise kernels round
-// it (operands widened to fp32, one fp32 operation, result rounded to nearest even), so the
-// output equals that of the torch expression bit for bit.  A row is one (batch, token, head)
-// vector of D values; a lane takes two adjacent values of the first half and their partners in
-// the second.
-template <bool BF16>
-__device__ __forceinline__ float act_to_f32(uint32_t bits16)
-{
-    if (BF16)
-        return __uint_as_float(bits16 << 16);
-    return (float)__builtin_bit_cast(h1, (uint16_t)bits16);
-}
-template <bool BF16>
-__device__ __forceinline__ uint32_t f32_to_act(float f)
-{
-    if (BF16) {
-        const uint32_t u = __float_as_uint(f);
-        if ((u & 0x7FFFFFFFu) > 0x7F800000u)
-            return 0x7FC0u; // torch's bfloat16 NaN
-        return (u + 0x7FFFu + ((u >> 16) & 1u)) >> 16;
-    }
-    return (uint32_t)__builtin_bit_cast(uint16_t, (h1)f);
-}
-// r(r(x*c) + r(y*s)) with y already negated where rotate_half negates
-template <bool BF16>
-__device__ __forceinline__ uint32_t rope_one(uint32_t x, uint32_t c, uint32_t y, bool neg_y, uint32_t s)
-{
-    const float a = act_to_f32<BF16>(f32_to_act<BF16>(act_to_f32<BF16>(x) * act_to_f32<BF16>(c)));
-    const float yy = neg_y ? -act_to_f32<BF16>(y) : act_to_f32<BF16>(y);
-    const float b = act_to_f32<BF16>(f32_to_act<BF16>(yy * act_to_f32<BF16>(s)));
-    return f32_to_act<BF16>(a + b);
-}
-
-struct RopeSide {
-    const uint16_t *x;
-    uint16_t *out;
-    long sb, sh, st; // element strides of x over batch, head, token (channels contiguous)
-    int heads;
-};
-
-// grid: (lanes of one token's Hq + H rows in workgroups of 256, token, batch)
-template <bool BF16>
-__global__ __launch_bounds__(256) void rope_kernel(RopeSide q, RopeSide k, const uint16_t *__restrict__ cos,
-                                                   const uint16_t *__restrict__ sin, long cb, long ct,
-                                                   int T, int D, int t0, int b0)
-{
-    const unsigned lpr = (unsigned)D >> 2;                   // lanes per row
-    const unsigned idx = blockIdx.x * 256u + threadIdx.x;
-    const unsigned hh = idx / lpr;
-    if (hh >= (unsigned)(q.heads + k.heads))
-        return;
-    const int i = (int)(idx - hh * lpr) * 2;                 // first of this lane's two channels
-    const int t = t0 + (int)blockIdx.y;
-    const long b = (long)b0 + (long)blockIdx.z;
-    const RopeSide &sd = hh < (unsigned)q.heads ? q : k;
-    const int h = hh < (unsigned)q.heads ? (int)hh : (int)hh - q.heads;
-    const uint16_t *x = sd.x + b * sd.sb + h * sd.sh + t * sd.st;
-    uint16_t *o = sd.out + ((b * sd.heads + h) * T + t) * D;
-    const uint16_t *c = cos + b * cb + t * ct, *s = sin + b * cb + t * ct;
-    const int half = D >> 1;
-    const uint32_t x1 = *reinterpret_cast<const uint32_t *>(x + i);
-    const uint32_t x2 = *reinterpret_cast<const uint32_t *>(x + half + i);
-    const uint32_t c1 = *reinterpret_cast<const uint32_t *>(c + i);
-    const uint32_t c2 = *reinterpret_cast<const uint32_t *>(c + half + i);
-    const uint32_t s1 = *reinterpret_cast<const uint32_t *>(s + i);
-    const uint32_t s2 = *reinterpret_cast<const uint32_t *>(s + half + i);
-    // first half: x1*cos + (-x2)*sin; second half: x2*cos + x1*sin
-    const uint32_t lo0 = rope_one<BF16>(x1 & 0xFFFFu, c1 & 0xFFFFu, x2 & 0xFFFFu, true, s1 & 0xFFFFu);
-    const uint32_t lo1 = rope_one<BF16>(x1 >> 16, c1 >> 16, x2 >> 16, true, s1 >> 16);
-    const uint32_t hi0 = rope_one<BF16>(x2 & 0xFFFFu, c2 & 0xFFFFu, x1 & 0xFFFFu, false, s2 & 0xFFFFu);
-    const uint32_t hi1 = rope_one<BF16>(x2 >> 16, c2 >> 16, x1 >> 16, false, s2 >> 16);
-    *reinterpret_cast<uint32_t *>(o + i) = lo0 | (lo1 << 16);
-    *reinterpret_cast<uint32_t *>(o + half + i) = hi0 | (hi1 << 16);
-}
-
-// ---------------------------------------------------------------------------------------------
 // softmax(float(logits)*scaling + mask) -> fp16   (llama_adkv.py:266-271)
 // ---------------------------------------------------------------------------------------------
 constexpr int SM_BLOCK = 256;
@@ -1776,7 +1709,7 @@ using namespace adkv;
 
 static thread_local int g_last_hip_error = 0;
 
-static int check_launch()
+int adkv::check_launch()
 {
     const hipError_t e = hipGetLastError();
     if (e != hipSuccess) {
@@ -1848,6 +1781,7 @@ static Seg plan_segments(void *ckpt, int n_ckpt_cap, int ckpt_interval, int BH, 
     s.intervals = 0;
     s.phys_per_head = 0;
     s.skew = 0;
+    s.fresh = 0;
     if (!ckpt || ckpt_interval <= 0 || T <= ckpt_interval)
         return s;
     const int avail = (T + ckpt_interval - 1) / ckpt_interval;               // finest split
@@ -2268,7 +2202,7 @@ static int check_ckpt(const void *ckpt, int n_ckpt_cap, int ckpt_interval, int b
 
 extern "C" {
 
-int adkv_abi_version(void) { return 16; }
+int adkv_abi_version(void) { return 17; }
 
 void adkv_set_fused_step(int mode) { g_fused_step.store(mode > 0 ? 1 : 0, std::memory_order_relaxed); }
 
@@ -2318,7 +2252,7 @@ static int encode_common(void *cache, const void *kv_new,
                          const void *state_in, void *state_out, void *ckpt_out, int n_ckpt_cap,
                          int ckpt_interval, void *stream, int bits = 4,
                          const EncTensor *second = nullptr, const RowStrides *first_strides = nullptr,
-                         bool bf16 = false)
+                         bool bf16 = false, bool fresh = false)
 {
     if (!cache || !kv_new || !zp || !sc || !alpha || !beta || !tgt)
         return ADKV_E_NULL;
@@ -2369,6 +2303,7 @@ static int encode_common(void *cache, const void *kv_new,
     seg.intervals = 0;
     seg.phys_per_head = 0;
     seg.skew = 0;
+    seg.fresh = fresh ? 1 : 0;
     // Lane width: one channel per lane while every wave then has a SIMD to itself (its time per token is
     // its instruction count, 17 against 30 with two channels), two channels beyond (they share the
     // packed updates and the wave's fixed cost).  ns per token, fp16 rows of 8192 tokens, 4-bit codes, at
@@ -2450,7 +2385,7 @@ int adkv_append_kv(void *cache, const void *kv_new,
                          bits);
 }
 
-int adkv_append_kv_pair(void *k_cache, void *v_cache, const void *k_new, const void *v_new,
+static int encode_pair(bool fresh, void *k_cache, void *v_cache, const void *k_new, const void *v_new,
                         int kv_dtype, const int64_t *k_strides, const int64_t *v_strides,
                         const void *const *k_params, const void *const *v_params,
                         int B, int H, int T0, int n_new, int D, int n_super_cap, int bits,
@@ -2482,7 +2417,33 @@ int adkv_append_kv_pair(void *k_cache, void *v_cache, const void *k_new, const v
     return encode_common(k_cache, k_new, k_params[0], k_params[1], k_params[2], k_params[3],
                          k_params[4], B, H, T0, T0 + n_new, D, n_super_cap, k_state_io, k_state_io,
                          k_ckpt, n_ckpt_cap, ckpt_interval, stream, bits, &v, &ks,
-                         kv_dtype == ADKV_DT_BF16);
+                         kv_dtype == ADKV_DT_BF16, fresh);
+}
+
+int adkv_append_kv_pair(void *k_cache, void *v_cache, const void *k_new, const void *v_new,
+                        int kv_dtype, const int64_t *k_strides, const int64_t *v_strides,
+                        const void *const *k_params, const void *const *v_params,
+                        int B, int H, int T0, int n_new, int D, int n_super_cap, int bits,
+                        void *k_state_io, void *v_state_io, void *k_ckpt, void *v_ckpt,
+                        int n_ckpt_cap, int ckpt_interval, void *stream)
+{
+    return encode_pair(false, k_cache, v_cache, k_new, v_new, kv_dtype, k_strides, v_strides, k_params, v_params,
+                       B, H, T0, n_new, D, n_super_cap, bits, k_state_io, v_state_io, k_ckpt, v_ckpt, n_ckpt_cap,
+                       ckpt_interval, stream);
+}
+
+int adkv_prefill_kv_pair(void *k_cache, void *v_cache, const void *k_new, const void *v_new,
+                         int kv_dtype, const int64_t *k_strides, const int64_t *v_strides,
+                         const void *const *k_params, const void *const *v_params,
+                         int B, int H, int n_new, int D, int n_super_cap, int bits,
+                         void *k_state_out, void *v_state_out, void *k_ckpt, void *v_ckpt,
+                         int n_ckpt_cap, int ckpt_interval, void *stream)
+{
+    if (n_new <= 0)
+        return ADKV_E_SHAPE; // nothing would be written
+    return encode_pair(true, k_cache, v_cache, k_new, v_new, kv_dtype, k_strides, v_strides, k_params, v_params,
+                       B, H, 0, n_new, D, n_super_cap, bits, k_state_out, v_state_out, k_ckpt, v_ckpt, n_ckpt_cap,
+                       ckpt_interval, stream);
 }
 
 int adkv_encode_kv(void *cache, const void *kv_new,
@@ -3006,41 +2967,6 @@ int adkv_softmax(const void *logits, void *weights, const void *mask,
 {
     return adkv_softmax_ex(logits, weights, mask, rows, n, 0, rows_per_mask_row, scaling, nullptr, 0,
                            stream);
-}
-
-int adkv_rope_qk(const void *q, const void *k, const void *cos, const void *sin, void *q_out, void *k_out,
-                 int B, int Hq, int H, int T, int D,
-                 int64_t q_sb, int64_t q_sh, int64_t q_st, int64_t k_sb, int64_t k_sh, int64_t k_st,
-                 int64_t cs_sb, int64_t cs_st, int bf16, void *stream)
-{
-    if (!q || !k || !cos || !sin || !q_out || !k_out)
-        return ADKV_E_NULL;
-    if (B <= 0 || Hq <= 0 || H <= 0 || T <= 0 || D <= 0 || (D & 3))
-        return ADKV_E_SHAPE;
-    // 4-byte accesses: every base and every stride a multiple of two elements
-    if (((uintptr_t)q | (uintptr_t)k | (uintptr_t)cos | (uintptr_t)sin | (uintptr_t)q_out | (uintptr_t)k_out) & 3)
-        return ADKV_E_ALIGN;
-    if ((q_sb | q_sh | q_st | k_sb | k_sh | k_st | cs_sb | cs_st) & 1)
-        return ADKV_E_ALIGN;
-    if ((long)(Hq + H) * (D >> 2) > (long)INT32_MAX)
-        return ADKV_E_SHAPE;
-    const RopeSide qs = {(const uint16_t *)q, (uint16_t *)q_out, (long)q_sb, (long)q_sh, (long)q_st, Hq};
-    const RopeSide ks = {(const uint16_t *)k, (uint16_t *)k_out, (long)k_sb, (long)k_sh, (long)k_st, H};
-    const unsigned gx = (unsigned)(((long)(Hq + H) * (D >> 2) + 255) / 256);
-    constexpr int GMAX = 65535; // grid limit of the token and batch axes: longer ones take several launches
-    for (int b0 = 0; b0 < B; b0 += GMAX)
-        for (int t0 = 0; t0 < T; t0 += GMAX) {
-            const dim3 grid(gx, (unsigned)min(T - t0, GMAX), (unsigned)min(B - b0, GMAX));
-            if (bf16)
-                hipLaunchKernelGGL(rope_kernel<true>, grid, dim3(256), 0, (hipStream_t)stream, qs, ks,
-                                   (const uint16_t *)cos, (const uint16_t *)sin, (long)cs_sb, (long)cs_st, T, D,
-                                   t0, b0);
-            else
-                hipLaunchKernelGGL(rope_kernel<false>, grid, dim3(256), 0, (hipStream_t)stream, qs, ks,
-                                   (const uint16_t *)cos, (const uint16_t *)sin, (long)cs_sb, (long)cs_st, T, D,
-                                   t0, b0);
-        }
-    return check_launch();
 }
 
 static int64_t pad256(int64_t n) { return (n + 255) & ~(int64_t)255; }

@@ -101,25 +101,35 @@ class KVCacheLayer_ADKV:
     def _n_ckpt(self, cap_tokens: int) -> int:
         return cap_tokens // self._ckpt_interval + 1 if self._ckpt_interval else 0
 
-    def _new_buffers(self, cap_tokens: int):
+    def _new_buffers(self, cap_tokens: int, alloc=torch.zeros):
         ns = self._n_super(cap_tokens)
         shape = (self._B, self._H, ns, self._C // 4, 4, 4)
-        mk = lambda: torch.zeros(shape, dtype=torch.uint8, device=self._device)
-        ck = (lambda: torch.zeros((self._B, self._H, self._n_ckpt(ns * (32 // self._bits)), self._C, 2),
-                                  dtype=torch.float16, device=self._device)) \
+        mk = lambda: alloc(shape, dtype=torch.uint8, device=self._device)
+        ck = (lambda: alloc((self._B, self._H, self._n_ckpt(ns * (32 // self._bits)), self._C, 2),
+                            dtype=torch.float16, device=self._device)) \
             if self._ckpt_interval else (lambda: None)
         return ns * (32 // self._bits), mk(), mk(), ck(), ck()
 
-    def _init_buffers(self, B: int, H: int, C: int, device: torch.device):
+    @staticmethod
+    def _capacity(cap: int, T: int) -> int:
+        """Token slots of a cache of ``cap`` slots once it has room for ``T`` tokens."""
+        if T <= cap:
+            return cap
+        return -(-max(T, int(cap * GROWTH)) // CAP_LEN) * CAP_LEN
+
+    def _set_geometry(self, B: int, H: int, C: int, device: torch.device):
         if C not in _HEAD_DIMS:
             raise ValueError(f"ADKV kernels support head_dim in (128, 256, 512), got {C}")
         if self._bits == 2 and C != 128:
             raise ValueError("2-bit ADKV codes need head_dim 128")
         self._B, self._H, self._C, self._device = B, H, C, device
         self._quant_len = 0
+
+    def _init_buffers(self, B: int, H: int, C: int, device: torch.device, tokens: int = INIT_SEQ_LEN, alloc=torch.zeros):
+        self._set_geometry(B, H, C, device)
         (self._cap_len, self._key_buf, self._value_buf,
-         self._key_ckpt, self._value_ckpt) = self._new_buffers(INIT_SEQ_LEN)
-        mk = lambda: torch.zeros((B, H, C, 2), dtype=torch.float16, device=device)
+         self._key_ckpt, self._value_ckpt) = self._new_buffers(tokens, alloc)
+        mk = lambda: alloc((B, H, C, 2), dtype=torch.float16, device=device)
         self._key_state, self._value_state, self._state_valid = mk(), mk(), True
 
     def _cap_buffers(self, T: int):
@@ -128,9 +138,7 @@ class KVCacheLayer_ADKV:
             return
         if self._shares_storage:
             raise RuntimeError("a batch view cannot grow: reserve() the parent cache for the whole context")
-        want = max(T, int(self._cap_len * GROWTH))
-        want = -(-want // CAP_LEN) * CAP_LEN
-        cap, key, value, kck, vck = self._new_buffers(want)
+        cap, key, value, kck, vck = self._new_buffers(self._capacity(self._cap_len, T))
         old = self._key_buf.shape[2]
         key[:, :, :old].copy_(self._key_buf)
         value[:, :, :old].copy_(self._value_buf)
@@ -198,7 +206,8 @@ class KVCacheLayer_ADKV:
     # ------------------------------------------------------------------ quantise
     def _append_tokens(self, key_states, value_states,
                        key_zp_init, key_scale_init, key_alpha, key_beta, key_quant_target,
-                       value_zp_init, value_scale_init, value_alpha, value_beta, value_quant_target):
+                       value_zp_init, value_scale_init, value_alpha, value_beta, value_quant_target,
+                       fresh: bool = False):
         """Quantise ``[B, H, T, C]`` keys/values as tokens ``quant_len ..`` of the stream."""
         v = self._view
         S = self._ckpt_interval
@@ -209,7 +218,7 @@ class KVCacheLayer_ADKV:
             (v(value_zp_init), v(value_scale_init), v(value_alpha), v(value_beta),
              v(value_quant_target)),
             self._quant_len, self._key_state, self._value_state,
-            k_ckpt=self._key_ckpt, v_ckpt=self._value_ckpt, ckpt_interval=S, bits=self._bits)
+            k_ckpt=self._key_ckpt, v_ckpt=self._value_ckpt, ckpt_interval=S, bits=self._bits, fresh=fresh)
         self._quant_len += key_states.shape[2]
 
     def prefill(self, key_states, value_states,
@@ -219,6 +228,21 @@ class KVCacheLayer_ADKV:
         B, H, T, C = key_states.shape
         if value_states.shape != key_states.shape:
             raise ValueError("key/value shapes differ")
+        if self._key_buf is None and T > 0:
+            # a new cache is allocated for the prompt at once and left uninitialised: the launch that
+            # quantises the prompt writes all of it
+            try:
+                self._init_buffers(B, H, C, key_states.device, self._capacity(INIT_SEQ_LEN, T), torch.empty)
+                self._append_tokens(key_states, value_states,
+                                    key_zp_init, key_scale_init, key_alpha, key_beta, key_quant_target,
+                                    value_zp_init, value_scale_init, value_alpha, value_beta,
+                                    value_quant_target, fresh=True)
+            except BaseException:
+                self._key_buf = self._value_buf = self._key_ckpt = self._value_ckpt = None
+                self._key_state = self._value_state = None
+                self._state_valid, self._cap_len = False, 0
+                raise
+            return
         self._check_geometry(B, H, C, key_states.device)
         if T == 0:
             return

@@ -386,6 +386,7 @@ def append_kv_pair(
     v_ckpt: torch.Tensor | None = None,
     ckpt_interval: int = 0,
     bits: int = 4,
+    fresh: bool = False,
 ) -> None:
     """``append_kv`` for the K and V rows of the same tokens in one launch (the two calls of
     src/adkv/hf/llama_adkv.py:144-153 made together).  Results are byte-identical to two
@@ -397,6 +398,9 @@ def append_kv_pair(
     are read, like the reference's ``.to(torch.float16)``, llama_adkv.py:141-142) and need not be
     packed: a ``[B, n, nh, DIM]`` projection output viewed with the head axis first is read in
     place.
+
+    ``fresh``: the caches, states and checkpoints are uninitialised memory (``torch.empty``) and the
+    tokens are their first (``T0 == 0``); the launch also zeroes the slots and checkpoints past them.
     """
     _chk(k_new.dtype == v_new.dtype and k_new.dtype in (torch.float16, torch.bfloat16),
          "kv_new must be float16 or bfloat16 (K and V alike)")
@@ -411,6 +415,7 @@ def append_kv_pair(
     n_super_cap = k_cache.shape[2]
     _chk(k_cache.shape[3] * _TILE == DIM, "kv_cache channel groups do not match kv_new head dim")
     _chk(T0 >= 0, "T0 must be non-negative")
+    _chk(not fresh or (T0 == 0 and n > 0), "a fresh cache starts at token 0")
     _chk(bits in (2, 4), "bits must be 2 or 4")
     tps = 32 // bits
     need = (T0 + n + tps - 1) // tps
@@ -431,11 +436,12 @@ def append_kv_pair(
     xv, vs = _row_strides(v_new)
     arr = _lib.C.c_void_p * 5
     with _lib.device_guard(dev):
-        rc = _lib.lib().adkv_append_kv_pair(
+        entry, at = (_lib.lib().adkv_prefill_kv_pair, ()) if fresh else (_lib.lib().adkv_append_kv_pair, (T0,))
+        rc = entry(
             k_cache.data_ptr(), v_cache.data_ptr(), xk.data_ptr(), xv.data_ptr(),
             _DT_BF16 if k_new.dtype == torch.bfloat16 else _DT_F16, ks, vs,
             arr(*[t.data_ptr() for t in kp]), arr(*[t.data_ptr() for t in vp]),
-            B, nh, T0, n, DIM, n_super_cap, bits, k_state.data_ptr(), v_state.data_ptr(),
+            B, nh, *at, n, DIM, n_super_cap, bits, k_state.data_ptr(), v_state.data_ptr(),
             kc, vc, ccap, civ, _lib.current_stream_ptr(dev))
     _lib.check(rc, "append_kv_pair")
 

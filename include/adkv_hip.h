@@ -183,6 +183,19 @@ int adkv_append_kv_pair(void *k_cache, void *v_cache, const void *k_new, const v
                         void *k_state_io, void *v_state_io, void *k_ckpt, void *v_ckpt,
                         int n_ckpt_cap, int ckpt_interval, void *stream);
 
+/*
+ * The first tokens of NEW caches: adkv_append_kv_pair with T0 == 0 into memory that nobody has
+ * written yet.  The launch also zeroes the slots past the tokens, up to n_super_cap, and the unused
+ * checkpoint entries, so an allocation needs no fill of its own.  Meant for caches not much longer
+ * than the prompt: the zeroes are written by the same lanes, one word after the other.
+ */
+int adkv_prefill_kv_pair(void *k_cache, void *v_cache, const void *k_new, const void *v_new,
+                         int kv_dtype, const int64_t *k_strides, const int64_t *v_strides,
+                         const void *const *k_params, const void *const *v_params,
+                         int B, int H, int n_new, int D, int n_super_cap, int bits,
+                         void *k_state_out, void *v_state_out, void *k_ckpt, void *v_ckpt,
+                         int n_ckpt_cap, int ckpt_interval, void *stream);
+
 int adkv_forward_qk_ex(const void *q, void *k_cache, const void *k_new, void *logits,
                        const void *zp, const void *sc, const void *alpha, const void *beta,
                        const void *tgt,
