@@ -53,6 +53,7 @@ PROTOTYPES = {
     "adkv_decode_segments": (_i, [_i] * 8 + [_vp, _i, _vp]),
     "adkv_rope_qk": (_i, [_vp] * 6 + [_i] * 5 + [C.c_int64] * 8 + [_i, _vp]),
     "adkv_quant_f32": (_i, [_vp] * 12 + [_i] * 3 + [C.c_int64, C.c_int64] + [_i] * 3 + [_f, _f, _vp]),
+    "adkv_quant_f32_pair": (_i, [_vp] * 7 + [_i] * 6 + [_f, _f, _vp]),
     "adkv_fp16_decode_workspace_bytes": (C.c_int64, [_i] * 3),
     "adkv_fp16_decode": (_i, [_vp] * 5 + [C.c_int64] + [_i] * 4 + [_f, _vp]),
 }

@@ -17,6 +17,7 @@ namespace adkv {
 
 // ADKV_OK, or ADKV_E_LAUNCH with the HIP code kept for adkv_last_hip_error() (host; adkv_kernels.hip)
 int check_launch();
+int cu_count(); // of the current device (host; adkv_kernels.hip)
 
 typedef _Float16 h1;
 typedef _Float16 h2 __attribute__((ext_vector_type(2)));

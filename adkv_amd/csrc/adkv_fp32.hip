@@ -8,9 +8,15 @@
 //   s  = max(sc, 1e-8);  q = clamp(rint((x - zp) / s), QL, QU);  r = q*s;  xhat = r + zp
 //   zp = zp + alpha*r;   sc = clamp(sc + (sc*beta)*(|q| - tgt), sc_min, sc_max)
 //
-// One lane owns one channel and walks the tokens in order; loads run three groups of 8 tokens
-// ahead of the dependent chain.  The path is bound by the length of that chain per token, not by
-// memory.
+// The recurrence is serial in t and only channels are parallel (64 to 1024 waves in the sizes this
+// form is used at, at most one per SIMD).  A wave alone on its SIMD issues one instruction every 4
+// cycles whether or not it depends on the one before, so the time per token is the NUMBER of
+// instructions of the wave that carries the chain.  quant_kernel therefore gives a workgroup two
+// waves: one does nothing but the recurrence, out of LDS and into LDS (two tokens per LDS
+// instruction); the other moves rows between memory and LDS, four channels per lane and a 16-byte
+// access per four rows, and converts types.  4096 channels x 1024 tokens of fp32 take 45 us, 44 ns per
+// token (18.5 issue slots at the 2.0-2.3 ns a lone wave pays for one); with everything in one wave it
+// was 65 us, the rest being loads, stores, their addresses and the guards of the rounding.
 #include <hip/hip_runtime.h>
 #include <hip/hip_bf16.h>
 #include <stdint.h>
@@ -22,29 +28,42 @@
 
 namespace adkv_fp32 {
 
-constexpr int BLK = 64;
-
 template <typename T> struct IO;
 template <> struct IO<float> {
-    static __device__ __forceinline__ float ld(const float *p) { return *p; }
-    static __device__ __forceinline__ void st(float *p, float v) { *p = v; }
+    typedef float Bits;
+    static __device__ __forceinline__ float up(float v) { return v; }
+    static __device__ __forceinline__ float down(float v) { return v; }
 };
 template <> struct IO<_Float16> {
-    static __device__ __forceinline__ float ld(const _Float16 *p) { return (float)*p; }
-    static __device__ __forceinline__ void st(_Float16 *p, float v) { *p = (_Float16)v; }
+    typedef uint16_t Bits;
+    static __device__ __forceinline__ float up(uint16_t v) { return (float)__builtin_bit_cast(_Float16, v); }
+    static __device__ __forceinline__ uint16_t down(float v) { return __builtin_bit_cast(uint16_t, (_Float16)v); }
 };
 template <> struct IO<__hip_bfloat16> {
-    static __device__ __forceinline__ float ld(const __hip_bfloat16 *p)
-    {
-        return __uint_as_float((uint32_t)*reinterpret_cast<const uint16_t *>(p) << 16);
-    }
-    static __device__ __forceinline__ void st(__hip_bfloat16 *p, float v)
+    typedef uint16_t Bits;
+    static __device__ __forceinline__ float up(uint16_t v) { return __uint_as_float((uint32_t)v << 16); }
+    static __device__ __forceinline__ uint16_t down(float v)
     {
         // round to nearest even; NaN stays NaN
-        uint32_t u = __float_as_uint(v);
-        uint16_t h = (v != v) ? (uint16_t)((u >> 16) | 0x40) : (uint16_t)((u + 0x7FFF + ((u >> 16) & 1)) >> 16);
-        *reinterpret_cast<uint16_t *>(p) = h;
+        const uint32_t u = __float_as_uint(v);
+        return (v != v) ? (uint16_t)((u >> 16) | 0x40) : (uint16_t)((u + 0x7FFF + ((u >> 16) & 1)) >> 16);
     }
+};
+
+// One tensor of a launch.  Either starting state may be absent: zp0 / sc0 are [C], zp_io / sc_io [B, C].
+struct Tensor {
+    const void *x;
+    void *xhat;
+    int8_t *codes;
+    float *zp_io, *sc_io;
+    const float *zp0, *sc0, *alpha, *beta, *tgt;
+    float *zp_seq, *sc_seq;
+    long xs_b, xs_t, os_b, os_t; // element strides of x and xhat; channels are contiguous
+};
+
+struct Limits {
+    float ql, qu, sc_min, sc_max;
+    float sure; // see Chan::step_spec
 };
 
 // torch.clamp semantics: NaN passes through
@@ -55,29 +74,39 @@ __device__ __forceinline__ float clamp_keep_nan(float x, float lo, float hi)
     return x < lo ? lo : (x > hi ? hi : x);
 }
 
-// One token of one channel.  The quotient is first taken with the hardware reciprocal of s (kept
-// from the previous token, off the dependent chain): r = d*rs is within 2^-22 relative of the
-// exact u = d/s, so rint(r) == rint(u) unless r lies closer than 2^-16 + |r|*2^-20 (four times the
-// error bound) to a rounding boundary k + 1/2, or is NaN; in that band the IEEE divide decides.
-// Everything after the rounding is the reference's separately rounded fp32 sequence.
+// NaN once an operand is one
+__device__ __forceinline__ float collect_abs(float acc, float a, float b)
+{
+    float r;
+    asm("v_maximum3_f32 %0, %1, |%2|, |%3|" : "=v"(r) : "v"(acc), "v"(a), "v"(b));
+    return r;
+}
+
+constexpr int GRP = 8; // tokens per speculative group
+
 struct Chan {
     float zp, sc, s, rs; // s = max(sc, 1e-8) (NaN kept), rs ~ 1/s
     float al, be, tg;
+    __device__ __forceinline__ void init(const Tensor &a, int b, int c, int C)
+    {
+        zp = a.zp0 ? a.zp0[c] : a.zp_io[(long)b * C + c];
+        set_scale(a.sc0 ? a.sc0[c] : a.sc_io[(long)b * C + c]);
+        al = a.alpha[c];
+        be = a.beta[c];
+        tg = a.tgt[c];
+    }
     __device__ __forceinline__ void set_scale(float v)
     {
         sc = v;
         s = (v != v) ? v : (v < 1e-8f ? 1e-8f : v);
-        rs = __builtin_amdgcn_rcpf(s);
+        // a scale whose reciprocal could be subnormal is left to the division
+        rs = s <= 0x1p100f ? __builtin_amdgcn_rcpf(s) : __builtin_nanf("");
     }
-    __device__ __forceinline__ float step(float xv, float ql, float qu, float sc_min, float sc_max, float &q)
+    // One token with the reference's operations and nothing else.
+    __device__ __forceinline__ float step(float xv, const Limits &l, float &q)
     {
         const float d = xv - zp;
-        const float r = d * rs;
-        float n = __builtin_rintf(r);
-        const float margin = __builtin_fmaf(__builtin_fabsf(r), 0x1p-20f, 0x1p-16f);
-        if (__builtin_expect(!(__builtin_fabsf(r - n) < 0.5f - margin), 0))
-            n = __builtin_rintf(d / s);
-        q = clamp_keep_nan(n, ql, qu);
+        q = clamp_keep_nan(__builtin_rintf(d / s), l.ql, l.qu);
         const float xr = q * s;
         const float xh = xr + zp;
         const float ax = al * xr;
@@ -85,25 +114,28 @@ struct Chan {
         const float sb = sc * be;
         const float sbe = sb * e;
         zp = zp + ax;
-        set_scale(clamp_keep_nan(sc + sbe, sc_min, sc_max));
+        set_scale(clamp_keep_nan(sc + sbe, l.sc_min, l.sc_max));
         return xh;
     }
-    // The same token without a branch or a NaN test, for lanes that pay every dependent
-    // instruction in full (few channels: each wave has a SIMD to itself).  The result is only
-    // valid if `worst` stays below SPEC_LIMIT: it takes the unsigned maximum of the bit patterns
-    // of  |r - n| + |r|*2^-20  (at or above 0.5 - 2^-15 whenever step() would have divided; a NaN
-    // or infinite r gives a NaN, whose pattern is above every number's) and of  raw - raw  for the
-    // unclamped new scale (0, or a NaN when raw is not finite: the clamps here drop NaNs, the
-    // reference's keep them).  A caller that finds worst >= SPEC_LIMIT restores the state it
-    // saved and redoes the tokens with step().
-    __device__ __forceinline__ float step_spec(float xv, float ql, float qu, float sc_min, float sc_max,
-                                               float &q, uint32_t &worst)
+    // The same token for a group that is checked afterwards: 16 instructions (rcp takes two slots).
+    //
+    // The quotient is r = d*rs with the reciprocal kept from the token before.  |r - u| <= |u|*2^-22
+    // for the IEEE quotient u (reciprocal 2^-23, two roundings 2^-24 each).  With L the largest code
+    // magnitude, |u| > L + 1 is clamped either way, and below that rint(r) == rint(u) unless r lies
+    // closer than (L + 1)*2^-22 to k + 1/2, that is unless |r - rint(r)| >= sure = 1/2 - (L + 1)*2^-21
+    // (twice the bound).  `off` returns r - rint(r), a NaN when r is infinite or one; `raw` the unclamped
+    // scale, whose NaN the clamp here drops and the reference's keeps.  The caller repeats the group
+    // with step() if any |off| is not below `sure` or any raw is a NaN: about one group of 8 tokens x 64
+    // channels in 120 with 4-bit codes.
+    // FLOOR: sc_min is below 1e-8 (otherwise s and sc are the same number).
+    template <bool FLOOR>
+    __device__ __forceinline__ float step_spec(float xv, const Limits &l, float &q, float &off, float &raw)
     {
         const float d = xv - zp;
         const float r = d * rs;
         const float n = __builtin_rintf(r);
-        q = __builtin_amdgcn_fmed3f(n, ql, qu);
-        const float t = __builtin_fmaf(__builtin_fabsf(r), 0x1p-20f, __builtin_fabsf(r - n));
+        off = r - n;
+        q = __builtin_amdgcn_fmed3f(n, l.ql, l.qu);
         const float xr = q * s;
         const float xh = xr + zp;
         const float ax = al * xr;
@@ -111,145 +143,428 @@ struct Chan {
         const float sb = sc * be;
         const float sbe = sb * e;
         zp = zp + ax;
-        const float raw = sc + sbe;
-        const float u = raw - raw;
-        const uint32_t tb = __float_as_uint(t), ub = __float_as_uint(u);
-        worst = max(worst, max(tb, ub));
-        sc = __builtin_amdgcn_fmed3f(raw, sc_min, sc_max);
-        s = __builtin_amdgcn_fmed3f(sc, 1e-8f, __builtin_inff()); // max(sc, 1e-8) without a NaN pass
+        raw = sc + sbe;
+        sc = __builtin_amdgcn_fmed3f(raw, l.sc_min, l.sc_max);
+        s = FLOOR ? __builtin_amdgcn_fmed3f(sc, 1e-8f, __builtin_inff()) : sc;
         rs = __builtin_amdgcn_rcpf(s);
         return xh;
     }
+    // GRP tokens; zs, ss: the state before each.
+    template <bool FLOOR>
+    __device__ __forceinline__ void steps(const float *x, const Limits &l, float *xh, float *q, float *zs, float *ss)
+    {
+        const Chan saved = *this;
+        float off[GRP], raw[GRP], worst = 0.0f, nan = 0.0f;
+#pragma unroll
+        for (int k = 0; k < GRP; k++) {
+            zs[k] = zp;
+            ss[k] = sc;
+            xh[k] = step_spec<FLOOR>(x[k], l, q[k], off[k], raw[k]);
+            if (k & 1) {
+                worst = collect_abs(worst, off[k - 1], off[k]);
+                nan = adkv::enc_collect_nan(nan, raw[k - 1], raw[k]);
+            }
+        }
+        if (__builtin_expect(__any(!(worst < l.sure) || nan != nan), 0)) {
+            *this = saved;
+#pragma unroll
+            for (int k = 0; k < GRP; k++) {
+                zs[k] = zp;
+                ss[k] = sc;
+                xh[k] = step(x[k], l, q[k]);
+            }
+        }
+    }
 };
-constexpr float SPEC_LIMIT = 0.5f - 0x1p-15f;
 
-constexpr int GRP = 8;  // tokens per group: the unit of speculation and of the input rotation
-constexpr int NBUF = 4; // groups of input in rotation (loads run NBUF-1 groups ahead)
+constexpr int CH = 32; // tokens per chunk, the unit in which the two waves of a workgroup hand rows over
+constexpr int NIN = 3, NOUT = 2;
 
-// x and xhat are declared non-aliasing although the caller may pass the same buffer (in-place
-// use): every element is loaded before the token that stores to it is computed and is never read
-// again, so no ordering between a store and a later load matters; without the promise the
-// compiler serialises every prefetched load behind the stores.
-//
-// WIDE (16-bit inputs only): a lane loads the aligned 32-bit word its channel lies in and picks
-// its half at use, so the values in flight are plain 32-bit registers with no arithmetic on
-// them; 16-bit loads would be zero-extended or packed in pairs at the loop edge, which makes
-// every group wait out the memory latency.  The launcher uses it when the layout allows (even C
-// and strides, 4-byte aligned base).
-template <typename T, bool WIDE, bool SEQ, bool OUT, bool CODES>
-__global__ __launch_bounds__(BLK) void quant_kernel(
-    const T *__restrict__ x, T *__restrict__ xhat, int8_t *__restrict__ codes, float *__restrict__ zp_io,
-    float *__restrict__ sc_io, const float *__restrict__ zp0, const float *__restrict__ sc0,
-    const float *__restrict__ alpha, const float *__restrict__ beta, const float *__restrict__ tgt,
-    float *__restrict__ zp_seq, float *__restrict__ sc_seq,
-    int Tn, int C, long stride_b, long stride_t, float ql, float qu, float sc_min, float sc_max)
+// One array of rows a workgroup reads or writes: 64 channels from c0, rows `stride` elements apart.
+// WIDE: whole 4-channel vectors; the array has to be `aligned` and all 64 channels inside the row.
+template <typename T, bool WIDE>
+struct Rows {
+    typedef typename IO<T>::Bits Bits;
+    struct alignas(4 * sizeof(Bits)) Vec {
+        Bits v[4];
+    };
+    Bits *base;
+    long stride;
+    int c, C; // this lane's first channel (of 4)
+    __device__ __forceinline__ Rows(void *p, long offset, long stride_, int c0, int C_)
+        : stride(stride_), c(c0 + (threadIdx.x & 15) * 4), C(C_)
+    {
+        base = (Bits *)p + offset;
+    }
+    static __device__ __forceinline__ bool aligned(const void *p, long offset, long stride)
+    {
+        return ((uintptr_t)p & (sizeof(Vec) - 1)) == 0 && offset % 4 == 0 && stride % 4 == 0;
+    }
+    __device__ __forceinline__ void load(long row, Vec &d) const
+    {
+        const Bits *p = base + row * stride + c;
+        if (WIDE) {
+            d = *reinterpret_cast<const Vec *>(p);
+        } else {
+#pragma unroll
+            for (int k = 0; k < 4; k++)
+                d.v[k] = c + k < C ? p[k] : (Bits)0;
+        }
+    }
+    __device__ __forceinline__ void store(long row, const float4 &f) const
+    {
+        Bits *p = base + row * stride + c;
+        const Vec d = {{IO<T>::down(f.x), IO<T>::down(f.y), IO<T>::down(f.z), IO<T>::down(f.w)}};
+        if (WIDE) {
+            *reinterpret_cast<Vec *>(p) = d;
+        } else {
+#pragma unroll
+            for (int k = 0; k < 4; k++)
+                if (c + k < C)
+                    p[k] = d.v[k];
+        }
+    }
+};
+
+// orders LDS accesses across the workgroup's barrier; global accesses in flight are not waited for
+__device__ __forceinline__ void hand_over()
 {
-    static_assert(!WIDE || sizeof(T) == 2, "wide loads are for 16-bit inputs");
-    using Raw = typename std::conditional<sizeof(T) == 4, float, typename std::conditional<WIDE, uint32_t, T>::type>::type;
-    const int c = blockIdx.x * BLK + threadIdx.x;
-    const int b = blockIdx.y;
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+}
+
+// 40 KB without the optional outputs: four workgroups on a CU
+template <bool SEQ, bool CODES>
+struct Shared {
+    static constexpr int Q = 1, ZP = CODES ? 2 : 1, SC = ZP + 1; // out[0] is xhat
+    float in[NIN][CH][64];
+    float out[1 + CODES + 2 * SEQ][NOUT][CH][64];
+};
+
+// Chunk i is in `in[i % 3]` from the barrier before phase i-1 on (so the recurrence reads its first
+// group before the barrier that ends phase i-1); its results are in slot i % 2 of the output
+// buffers from the barrier after phase i on.  In phase i the mover
+//   writes chunk i+2 (loaded during phase i-1) to the slot chunk i-1 has left,
+//   issues the loads of chunk i+3, which have until phase i+2 (a phase is about 1 us) to arrive, and
+//   stores the results of chunk i-1.
+// Both waves pass nch + 1 barriers.
+template <typename T, bool SEQ, bool CODES, bool WIDE>
+__device__ __forceinline__ void move_rows(Shared<SEQ, CODES> &sm, const Tensor &a, int b, int c0, int Tn, int C, int nch)
+{
+    const Rows<T, WIDE> x(const_cast<void *>(a.x), b * a.xs_b, a.xs_t, c0, C);
+    const Rows<T, WIDE> xo(a.xhat, b * a.os_b, a.os_t, c0, C);
+    const long dense = (long)b * Tn * C; // codes and state sequences are [B, T, C]
+    const Rows<float, WIDE> zo(a.zp_seq, dense, C, c0, C), so(a.sc_seq, dense, C, c0, C);
+    const int r0 = (threadIdx.x & 63) >> 4, col = (threadIdx.x & 15) * 4;
+
+    typename Rows<T, WIDE>::Vec v[CH / 4];
+    auto load = [&](int i) __attribute__((always_inline)) {
+#pragma unroll
+        for (int j = 0; j < CH / 4; j++)
+            x.load(min(i * CH + j * 4 + r0, Tn - 1), v[j]);
+    };
+    auto fill = [&](int slot) __attribute__((always_inline)) {
+#pragma unroll
+        for (int j = 0; j < CH / 4; j++)
+            *reinterpret_cast<float4 *>(&sm.in[slot][j * 4 + r0][col]) =
+                make_float4(IO<T>::up(v[j].v[0]), IO<T>::up(v[j].v[1]), IO<T>::up(v[j].v[2]), IO<T>::up(v[j].v[3]));
+    };
+    auto drain = [&](int i) __attribute__((always_inline)) {
+        const int slot = i & 1;
+#pragma unroll
+        for (int j = 0; j < CH / 4; j++) {
+            const int row = j * 4 + r0;
+            const int t = i * CH + row;
+            if (t >= Tn)
+                break;
+            auto get = [&](const float *p) { return *reinterpret_cast<const float4 *>(p + col); };
+            if (a.xhat)
+                xo.store(t, get(sm.out[0][slot][row]));
+            if constexpr (SEQ) {
+                zo.store(t, get(sm.out[sm.ZP][slot][row]));
+                so.store(t, get(sm.out[sm.SC][slot][row]));
+            }
+            if constexpr (CODES) {
+                const float4 f = get(sm.out[sm.Q][slot][row]);
+                auto code = [](float q) { return (q != q) ? (int8_t)0 : (int8_t)q; };
+                const char4 k = make_char4(code(f.x), code(f.y), code(f.z), code(f.w));
+                int8_t *p = a.codes + dense + (long)t * C + c0 + col;
+                if (WIDE) {
+                    *reinterpret_cast<char4 *>(p) = k;
+                } else {
+                    const int8_t kk[4] = {k.x, k.y, k.z, k.w};
+#pragma unroll
+                    for (int e = 0; e < 4; e++)
+                        if (c0 + col + e < C)
+                            p[e] = kk[e];
+                }
+            }
+        }
+    };
+    load(0);
+    fill(0);
+    if (nch > 1) {
+        load(1);
+        fill(1);
+    }
+    if (nch > 2)
+        load(2);
+    hand_over();
+    int slot = 2; // (i + 2) % 3
+    for (int i = 0; i < nch; i++) {
+        if (i + 2 < nch)
+            fill(slot);
+        if (i + 3 < nch)
+            load(i + 3);
+        if (i > 0)
+            drain(i - 1);
+        slot = slot == 2 ? 0 : slot + 1;
+        hand_over();
+    }
+    drain(nch - 1);
+}
+
+// ~18 instructions per token: 16 of step_spec, half an LDS read and half an LDS write, the two halves of
+// the check.
+template <bool SEQ, bool CODES, bool FLOOR>
+__device__ __forceinline__ void recurrence(Shared<SEQ, CODES> &sm, const Tensor &a, int b, int c0, int Tn, int C, int nch,
+                                           Limits l)
+{
+    const int lane = threadIdx.x & 63;
+    const int c = c0 + lane;
+    Chan ch;
+    ch.init(a, b, min(c, C - 1), C);
+    // med3 takes one scalar operand: the other bound of each pair lives in a vector register
+    asm volatile("" : "+v"(l.qu), "+v"(l.sc_max));
+
+    // tokens `row`.. of a chunk: results of GRP tokens into slot `o`
+    auto group = [&](const float *x, int row, int o) __attribute__((always_inline)) {
+        float xh[GRP], q[GRP], zs[GRP], ss[GRP];
+        ch.template steps<FLOOR>(x, l, xh, q, zs, ss);
+#pragma unroll
+        for (int k = 0; k < GRP; k++) {
+            sm.out[0][o][row + k][lane] = xh[k];
+            if constexpr (CODES)
+                sm.out[sm.Q][o][row + k][lane] = q[k];
+            if constexpr (SEQ) {
+                sm.out[sm.ZP][o][row + k][lane] = zs[k];
+                sm.out[sm.SC][o][row + k][lane] = ss[k];
+            }
+        }
+    };
+    auto read = [&](float *x, int slot, int row) __attribute__((always_inline)) {
+#pragma unroll
+        for (int k = 0; k < GRP; k++)
+            x[k] = sm.in[slot][row + k][lane];
+    };
+
+    hand_over();
+    const int nfull = Tn / CH;
+    float x[2][GRP];
+    read(x[0], 0, 0);
+    int slot = 0;
+    for (int i = 0; i < nfull; i++) {
+        const int next = slot == 2 ? 0 : slot + 1;
+#pragma unroll
+        for (int g = 0; g < CH / GRP; g++) {
+            // the next group's rows (past the last chunk: whatever the slot holds, never used)
+            read(x[(g + 1) & 1], g + 1 < CH / GRP ? slot : next, (g + 1) * GRP % CH);
+            group(x[g & 1], g * GRP, i & 1);
+        }
+        slot = next;
+        hand_over();
+    }
+    if (nfull < nch) {
+        const int o = nfull & 1, n = Tn - nfull * CH;
+        int row = 0;
+        for (; row + GRP <= n; row += GRP) {
+            read(x[0], slot, row);
+            group(x[0], row, o);
+        }
+        for (; row < n; row++) {
+            if constexpr (SEQ) {
+                sm.out[sm.ZP][o][row][lane] = ch.zp;
+                sm.out[sm.SC][o][row][lane] = ch.sc;
+            }
+            float q;
+            sm.out[0][o][row][lane] = ch.step(sm.in[slot][row][lane], l, q);
+            if constexpr (CODES)
+                sm.out[sm.Q][o][row][lane] = q;
+        }
+        hand_over();
+    }
+    if (a.zp_io && c < C) {
+        a.zp_io[(long)b * C + c] = ch.zp;
+        a.sc_io[(long)b * C + c] = ch.sc;
+    }
+}
+
+// grid: (64-channel blocks, batch, tensors)
+template <typename T, bool SEQ, bool CODES, bool FLOOR>
+__global__ __launch_bounds__(128) void quant_kernel(Tensor a0, Tensor a1, int Tn, int C, Limits l)
+{
+    __shared__ Shared<SEQ, CODES> sm;
+    const Tensor a = blockIdx.z ? a1 : a0;
+    const int c0 = blockIdx.x * 64, b = blockIdx.y, nch = (Tn + CH - 1) / CH;
+    if (threadIdx.x < 64)
+        recurrence<SEQ, CODES, FLOOR>(sm, a, b, c0, Tn, C, nch, l);
+    else {
+        using R = Rows<T, true>;
+        const bool dense_ok = C % 4 == 0 && (((uintptr_t)a.zp_seq | (uintptr_t)a.sc_seq) & 15) == 0 && ((uintptr_t)a.codes & 3) == 0;
+        if (c0 + 64 <= C && R::aligned(a.x, b * a.xs_b, a.xs_t) && (!a.xhat || R::aligned(a.xhat, b * a.os_b, a.os_t)) &&
+            ((!SEQ && !CODES) || dense_ok))
+            move_rows<T, SEQ, CODES, true>(sm, a, b, c0, Tn, C, nch);
+        else
+            move_rows<T, SEQ, CODES, false>(sm, a, b, c0, Tn, C, nch);
+    }
+}
+
+constexpr int NBUF = 2; // groups of rows in rotation (3 and 4 were measured: fewer waves fit, 2-10 % slower)
+
+// A lane per channel straight from memory, in groups of GRP tokens.
+// SPEC = false: limits that step_spec does not cover, the reference's operations only.
+// EXTRA: codes or states are wanted.
+template <typename T, bool SPEC, bool EXTRA>
+__global__ __launch_bounds__(64) void quant_direct_kernel(Tensor a0, Tensor a1, int Tn, int C, Limits l)
+{
+    typedef typename IO<T>::Bits Bits;
+    const Tensor a = blockIdx.z ? a1 : a0;
+    const int c = blockIdx.x * 64 + threadIdx.x, b = blockIdx.y;
     if (c >= C)
         return;
-    const long bc = (long)b * C + c;
     Chan ch;
-    ch.zp = zp0 ? zp0[c] : zp_io[bc];
-    ch.set_scale(sc0 ? sc0[c] : sc_io[bc]);
-    ch.al = alpha[c];
-    ch.be = beta[c];
-    ch.tg = tgt[c];
-    const T *xp = x + b * stride_b + c;
-    T *op = OUT ? xhat + b * stride_b + c : nullptr;
-    const long dense = (long)b * Tn * C + c; // codes / zp_seq / sc_seq are contiguous [B, T, C]
-    const uint32_t half_shift = WIDE ? (uint32_t)(c & 1) * 16u : 0u;
-
-    auto load_raw = [&](long t) __attribute__((always_inline)) -> Raw {
-        if constexpr (WIDE)
-            return *reinterpret_cast<const uint32_t *>(xp - (c & 1) + t * stride_t);
-        else if constexpr (sizeof(T) == 4)
-            return *reinterpret_cast<const float *>(xp + t * stride_t);
-        else
-            return xp[t * stride_t];
-    };
-    auto value = [&](Raw r) __attribute__((always_inline)) -> float {
-        if constexpr (WIDE) {
-            const uint16_t hb = (uint16_t)(r >> half_shift);
-            return IO<T>::ld(reinterpret_cast<const T *>(&hb));
-        } else if constexpr (sizeof(T) == 4) {
-            return r;
-        } else {
-            return IO<T>::ld(&r);
+    ch.init(a, b, c, C);
+    const Bits *xp = (const Bits *)a.x + b * a.xs_b + c;
+    Bits *op = a.xhat ? (Bits *)a.xhat + b * a.os_b + c : nullptr;
+    const long dense = (long)b * Tn * C + c;
+    int8_t *cp = a.codes ? a.codes + dense : nullptr;
+    float *zq = a.zp_seq ? a.zp_seq + dense : nullptr, *sq = a.zp_seq ? a.sc_seq + dense : nullptr;
+    // the next token's results
+    auto emit = [&](float xh, float q, float zp, float sc) __attribute__((always_inline)) {
+        if (op) {
+            *op = IO<T>::down(xh);
+            op += a.os_t;
+        }
+        if (EXTRA && cp) {
+            *cp = (q != q) ? (int8_t)0 : (int8_t)q;
+            cp += C;
+        }
+        if (EXTRA && zq) {
+            *zq = zp;
+            *sq = sc;
+            zq += C;
+            sq += C;
         }
     };
-    auto emit = [&](int t, float xh, float q) __attribute__((always_inline)) {
-        if (OUT)
-            IO<T>::st(op + (long)t * stride_t, xh);
-        if (CODES)
-            codes[dense + (long)t * C] = (q != q) ? (int8_t)0 : (int8_t)q;
-    };
-    // exact path, token by token (also records the state sequence)
-    auto one = [&](float xv, int t) __attribute__((always_inline)) {
-        if (SEQ) {
-            zp_seq[dense + (long)t * C] = ch.zp;
-            sc_seq[dense + (long)t * C] = ch.sc;
-        }
-        float q;
-        const float xh = ch.step(xv, ql, qu, sc_min, sc_max, q);
-        emit(t, xh, q);
-    };
-
-    // Full groups of GRP tokens.  Inputs are loaded NBUF-1 groups ahead, unconditionally (past
-    // the last group the same rows are loaded again).  A group is first run speculatively with
-    // its results held in registers; if any lane of the wave came near a rounding boundary or met
-    // a non-finite value (about one group in thirty) the state is restored and the group is
-    // redone exactly.  Recording the state sequence needs the state before every token, so that
-    // variant runs the exact path only.
-    const int ng = Tn / GRP;
-    Raw buf[NBUF][GRP];
-    long tnext = 0; // first token of the next group to load
-    auto load_next = [&](Raw *dst) __attribute__((always_inline)) {
+    const int ng = SPEC ? Tn / GRP : 0;
+    Bits buf[NBUF][GRP];
+    auto load = [&](int g, Bits *dst) __attribute__((always_inline)) {
 #pragma unroll
-        for (int i = 0; i < GRP; i++)
-            dst[i] = load_raw(tnext + i);
-        if (tnext + GRP < (long)ng * GRP)
-            tnext += GRP;
-    };
-    auto do_group = [&](int g, const Raw *xg) __attribute__((always_inline)) {
-        if (SEQ) {
-#pragma unroll
-            for (int i = 0; i < GRP; i++)
-                one(value(xg[i]), g * GRP + i);
-            return;
-        }
-        const Chan saved = ch;
-        uint32_t worst = 0u;
-        float xh[GRP], q[GRP];
-#pragma unroll
-        for (int i = 0; i < GRP; i++)
-            xh[i] = ch.step_spec(value(xg[i]), ql, qu, sc_min, sc_max, q[i], worst);
-        if (__any(worst >= __float_as_uint(SPEC_LIMIT))) {
-            ch = saved;
-#pragma unroll
-            for (int i = 0; i < GRP; i++)
-                xh[i] = ch.step(value(xg[i]), ql, qu, sc_min, sc_max, q[i]);
-        }
-#pragma unroll
-        for (int i = 0; i < GRP; i++)
-            emit(g * GRP + i, xh[i], q[i]);
+        for (int k = 0; k < GRP; k++)
+            dst[k] = xp[(long)(g * GRP + k) * a.xs_t];
     };
     if (ng > 0) {
-        adkv::static_for<NBUF - 1>([&](auto ic) { load_next(buf[decltype(ic)::value]); });
+        adkv::static_for<NBUF - 1>([&](auto ic) { load(min(decltype(ic)::value, ng - 1), buf[decltype(ic)::value]); });
         adkv::rotate_over<NBUF>(ng, [&](int g, auto ic) __attribute__((always_inline)) {
             constexpr int i = decltype(ic)::value;
-            load_next(buf[(i + NBUF - 1) % NBUF]);
-            do_group(g, buf[i]);
+            // past the last group the same rows again: a condition would make the next wait cover every load
+            load(min(g + NBUF - 1, ng - 1), buf[(i + NBUF - 1) % NBUF]);
+            float x[GRP], xh[GRP], q[GRP], zs[GRP], ss[GRP];
+#pragma unroll
+            for (int k = 0; k < GRP; k++)
+                x[k] = IO<T>::up(buf[i][k]);
+            ch.template steps<true>(x, l, xh, q, zs, ss);
+#pragma unroll
+            for (int k = 0; k < GRP; k++)
+                emit(xh[k], q[k], zs[k], ss[k]);
         });
     }
-    for (int t = ng * GRP; t < Tn; t++)
-        one(value(load_raw(t)), t);
-    if (zp_io) {
-        zp_io[bc] = ch.zp;
-        sc_io[bc] = ch.sc;
+    for (int t = ng * GRP; t < Tn; t++) {
+        const float zp = ch.zp, sc = ch.sc;
+        float q;
+        const float xh = ch.step(IO<T>::up(xp[t * a.xs_t]), l, q);
+        emit(xh, q, zp, sc);
     }
+    if (a.zp_io) {
+        a.zp_io[(long)b * C + c] = ch.zp;
+        a.sc_io[(long)b * C + c] = ch.sc;
+    }
+}
+
+// Which kernel: quant_kernel while all its workgroups are resident at once (its LDS allows four on a
+// CU, two with codes or states, one with both), quant_direct_kernel beyond, where many waves hide what
+// quant_kernel moves out of the chain.  us, both kernels, one tensor of
+// fp32, 64-channel blocks x tokens, quant_kernel / quant_direct_kernel: 64 x 1024 45 / 121, 512 x 512
+// 30 / 66, 1024 x 64 9.5 / 12.1, 1024 x 256 23 / 37; 2048 x 64 20 / 12.7, 8192 x 32 36 / 23.
+static int launch(const Tensor *a, int n, int B, int T, int C, int x_dtype, int lower_limit, int upper_limit,
+                  float sc_min, float sc_max, hipStream_t st)
+{
+    for (int i = 0; i < n; i++) {
+        if (!a[i].x || !a[i].alpha || !a[i].beta || !a[i].tgt)
+            return ADKV_E_NULL;
+        if ((a[i].zp_io == nullptr) != (a[i].sc_io == nullptr) || (a[i].zp0 == nullptr) != (a[i].sc0 == nullptr))
+            return ADKV_E_NULL;
+        if (!a[i].zp_io && !a[i].zp0)
+            return ADKV_E_NULL; // no starting state at all
+        if ((a[i].zp_seq == nullptr) != (a[i].sc_seq == nullptr))
+            return ADKV_E_NULL;
+    }
+    if (B <= 0 || C <= 0 || T < 0 || B > 65535)
+        return ADKV_E_SHAPE;
+    for (int i = 0; i < n; i++)
+        if (a[i].xs_t < C || a[i].xs_b < 0 || a[i].os_t < C || a[i].os_b < 0)
+            return ADKV_E_SHAPE;
+    if (lower_limit > 0 || upper_limit < 0 || lower_limit < -128 || upper_limit > 127)
+        return ADKV_E_UNSUPPORTED;
+    if (x_dtype != ADKV_DT_F32 && x_dtype != ADKV_DT_F16 && x_dtype != ADKV_DT_BF16)
+        return ADKV_E_UNSUPPORTED;
+    if (T == 0 && !(a[0].zp0 && a[0].zp_io))
+        return ADKV_OK;
+    const int largest = -lower_limit > upper_limit ? -lower_limit : upper_limit;
+    const Limits l = {(float)lower_limit, (float)upper_limit, sc_min, sc_max, 0.5f - (float)(largest + 1) * 0x1p-21f};
+    const Tensor &a1 = a[n - 1];
+    const dim3 grid((unsigned)((C + 63) / 64), (unsigned)B, (unsigned)n);
+    const bool spec = sc_min <= sc_max && sc_max >= 1e-8f && sc_max <= 0x1p100f; // what step_spec relies on
+    const bool seq = a[0].zp_seq != nullptr, codes = a[0].codes != nullptr, floored = sc_min < 1e-8f;
+    const long resident = adkv::cu_count() * (seq && codes ? 1L : seq || codes ? 2L : 4L);
+    const bool direct = (long)grid.x * grid.y * grid.z > resident;
+#define ADKV_Q32_K(TYPE, SEQ, CODES, FLOOR)                                                                \
+    hipLaunchKernelGGL((quant_kernel<TYPE, SEQ, CODES, FLOOR>), grid, dim3(128), 0, st, a[0], a1, T, C, l)
+#define ADKV_Q32_F(TYPE, SEQ, CODES)                                                                       \
+    do {                                                                                                   \
+        if (floored)                                                                                       \
+            ADKV_Q32_K(TYPE, SEQ, CODES, true);                                                            \
+        else                                                                                               \
+            ADKV_Q32_K(TYPE, SEQ, CODES, false);                                                           \
+    } while (0)
+#define ADKV_Q32(TYPE)                                                                                     \
+    do {                                                                                                   \
+        if (T < 2 || !spec)                                                                                \
+            hipLaunchKernelGGL((quant_direct_kernel<TYPE, false, true>), grid, dim3(64), 0, st, a[0], a1, T, C, l); \
+        else if (direct && (seq || codes))                                                                 \
+            hipLaunchKernelGGL((quant_direct_kernel<TYPE, true, true>), grid, dim3(64), 0, st, a[0], a1, T, C, l); \
+        else if (direct)                                                                                   \
+            hipLaunchKernelGGL((quant_direct_kernel<TYPE, true, false>), grid, dim3(64), 0, st, a[0], a1, T, C, l); \
+        else if (seq && codes)                                                                             \
+            ADKV_Q32_F(TYPE, true, true);                                                                  \
+        else if (seq)                                                                                      \
+            ADKV_Q32_F(TYPE, true, false);                                                                 \
+        else if (codes)                                                                                    \
+            ADKV_Q32_F(TYPE, false, true);                                                                 \
+        else                                                                                               \
+            ADKV_Q32_F(TYPE, false, false);                                                                \
+    } while (0)
+    if (x_dtype == ADKV_DT_F32)
+        ADKV_Q32(float);
+    else if (x_dtype == ADKV_DT_F16)
+        ADKV_Q32(_Float16);
+    else
+        ADKV_Q32(__hip_bfloat16);
+#undef ADKV_Q32
+#undef ADKV_Q32_F
+#undef ADKV_Q32_K
+    return adkv::check_launch();
 }
 
 } // namespace adkv_fp32
@@ -261,68 +576,26 @@ extern "C" int adkv_quant_f32(const void *x, void *xhat, void *codes, void *zp_s
                               int lower_limit, int upper_limit, float sc_min, float sc_max,
                               void *stream)
 {
-    using namespace adkv_fp32;
-    if (!x || !alpha || !beta || !tgt)
+    const adkv_fp32::Tensor a = {x, xhat, (int8_t *)codes, (float *)zp_state, (float *)sc_state, (const float *)zp_init,
+                                 (const float *)sc_init, (const float *)alpha, (const float *)beta, (const float *)tgt,
+                                 (float *)zp_seq, (float *)sc_seq, (long)stride_b, (long)stride_t, (long)stride_b,
+                                 (long)stride_t};
+    return adkv_fp32::launch(&a, 1, B, T, C, x_dtype, lower_limit, upper_limit, sc_min, sc_max, (hipStream_t)stream);
+}
+
+extern "C" int adkv_quant_f32_pair(const void *const *x, const int64_t *x_strides, void *const *xhat,
+                                   const int64_t *xhat_strides, void *const *state, const void *const *init,
+                                   const void *const *params, int B, int T, int C, int x_dtype, int lower_limit,
+                                   int upper_limit, float sc_min, float sc_max, void *stream)
+{
+    if (!x || !x_strides || !xhat || !xhat_strides || !state || !params)
         return ADKV_E_NULL;
-    if ((zp_state == nullptr) != (sc_state == nullptr) || (zp_init == nullptr) != (sc_init == nullptr))
-        return ADKV_E_NULL;
-    if (!zp_state && !zp_init)
-        return ADKV_E_NULL; // no starting state at all
-    if ((zp_seq == nullptr) != (sc_seq == nullptr))
-        return ADKV_E_NULL;
-    if (B <= 0 || C <= 0 || T < 0 || B > 65535 || stride_t < C || stride_b < 0)
-        return ADKV_E_SHAPE;
-    if (lower_limit > 0 || upper_limit < 0 || lower_limit < -128 || upper_limit > 127)
-        return ADKV_E_UNSUPPORTED;
-    if (T == 0 && !(zp_init && zp_state))
-        return ADKV_OK;
-    const dim3 grid((unsigned)((C + BLK - 1) / BLK), (unsigned)B), block(BLK);
-    hipStream_t st = (hipStream_t)stream;
-#define ADKV_Q32_(TYPE, WIDE, SEQ, OUT, CODES)                                                      \
-    hipLaunchKernelGGL((quant_kernel<TYPE, WIDE, SEQ, OUT, CODES>), grid, block, 0, st,             \
-                       (const TYPE *)x, (TYPE *)xhat,                                               \
-                       (int8_t *)codes, (float *)zp_state, (float *)sc_state, (const float *)zp_init, \
-                       (const float *)sc_init, (const float *)alpha, (const float *)beta,           \
-                       (const float *)tgt, (float *)zp_seq, (float *)sc_seq, T, C, (long)stride_b,  \
-                       (long)stride_t, (float)lower_limit, (float)upper_limit, sc_min, sc_max)
-#define ADKV_Q32_O(TYPE, WIDE, SEQ)                                                                 \
-    do {                                                                                            \
-        if (xhat && codes)                                                                          \
-            ADKV_Q32_(TYPE, WIDE, SEQ, true, true);                                                 \
-        else if (xhat)                                                                              \
-            ADKV_Q32_(TYPE, WIDE, SEQ, true, false);                                                \
-        else if (codes)                                                                             \
-            ADKV_Q32_(TYPE, WIDE, SEQ, false, true);                                                \
-        else                                                                                        \
-            ADKV_Q32_(TYPE, WIDE, SEQ, false, false);                                               \
-    } while (0)
-#define ADKV_Q32(TYPE, WIDE)                                                                        \
-    do {                                                                                            \
-        if (zp_seq)                                                                                 \
-            ADKV_Q32_O(TYPE, WIDE, true);                                                           \
-        else                                                                                        \
-            ADKV_Q32_O(TYPE, WIDE, false);                                                          \
-    } while (0)
-#define ADKV_Q32_16(TYPE)                                                                           \
-    do {                                                                                            \
-        if (wide)                                                                                   \
-            ADKV_Q32(TYPE, true);                                                                   \
-        else                                                                                        \
-            ADKV_Q32(TYPE, false);                                                                  \
-    } while (0)
-    // 16-bit inputs: aligned 32-bit loads when every row starts on a 4-byte boundary and no
-    // channel's word reaches past its row
-    const bool wide = (C % 2 == 0) && (stride_t % 2 == 0) && (stride_b % 2 == 0) &&
-                      (((uintptr_t)x & 3) == 0);
-    switch (x_dtype) {
-    case ADKV_DT_F32: ADKV_Q32(float, false); break;
-    case ADKV_DT_F16: ADKV_Q32_16(_Float16); break;
-    case ADKV_DT_BF16: ADKV_Q32_16(__hip_bfloat16); break;
-    default: return ADKV_E_UNSUPPORTED;
-    }
-#undef ADKV_Q32_16
-#undef ADKV_Q32
-#undef ADKV_Q32_O
-#undef ADKV_Q32_
-    return hipGetLastError() == hipSuccess ? ADKV_OK : ADKV_E_LAUNCH;
+    adkv_fp32::Tensor a[2];
+    for (int i = 0; i < 2; i++)
+        a[i] = {x[i], xhat[i], nullptr, (float *)state[2 * i], (float *)state[2 * i + 1],
+                init ? (const float *)init[2 * i] : nullptr, init ? (const float *)init[2 * i + 1] : nullptr,
+                (const float *)params[3 * i], (const float *)params[3 * i + 1], (const float *)params[3 * i + 2],
+                nullptr, nullptr, (long)x_strides[2 * i], (long)x_strides[2 * i + 1], (long)xhat_strides[2 * i],
+                (long)xhat_strides[2 * i + 1]};
+    return adkv_fp32::launch(a, 2, B, T, C, x_dtype, lower_limit, upper_limit, sc_min, sc_max, (hipStream_t)stream);
 }

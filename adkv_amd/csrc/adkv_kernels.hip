@@ -1760,6 +1760,7 @@ static int cus()
     return n;
 }
 static int n_simd() { return 4 * cus(); }
+int adkv::cu_count() { return cus(); }
 
 // Segment plan for a decode launch.  Starting from the fewest segments that give every SIMD its
 // target of waves, finer splits are taken when they shorten the launch: 16-wave workgroups run one

@@ -4,8 +4,9 @@ kept dequantised, attention is the regular dense one.
 Counterpart of the reference's ``adkv.hf.llama_adkv_eval`` (src/adkv/hf/llama_adkv_eval.py): same
 class names, ``update`` signature and state fields (``key_dc``, ``key_scale``, ...).  The Triton
 kernel of the reference (llama_adkv_eval.py:34-118) is replaced by the gfx950 fp32 quantiser
-(``adkv_quant_f32``), which walks every newly appended token of K and of V in one launch each
-instead of 32-token tiles, in place on the cache buffer.
+(``adkv_quant_f32_pair``), which walks every newly appended token of K and of V in one launch instead
+of 32-token tiles per tensor, from where the rows are into the cache buffer (in place on the buffer
+where they have to be copied there first).
 """
 from __future__ import annotations
 
@@ -23,7 +24,7 @@ from transformers.models.llama.modeling_llama import (
 )
 from transformers.modeling_utils import ALL_ATTENTION_FUNCTIONS
 
-from ..train.train_model import quant_f32
+from ..train.train_model import quant_f32_pair
 from .llama_adkv import ADKV_PARAM_FIELDS, ADKVConfig  # noqa: F401
 
 SCALE_MIN = math.exp(-4.0)
@@ -84,19 +85,25 @@ class KVCacheLayer_ADKV:
         self._recent_len += T
 
     def _quantize_new_tokens(self, key_alpha, key_beta, key_quant_target,
-                             value_alpha, value_beta, value_quant_target):
-        """Quantise on write: every token appended since the last call, in place."""
+                             value_alpha, value_beta, value_quant_target, source=None, init=None):
+        """Quantise on write: every token appended since the last call, in place, or read from
+        ``source`` where the rows have not been copied into the buffers."""
         a, b = self._quant_len, self._recent_len
         if b == a:
             return
-        for buf, dc, scale, al, be, tg in (
-                (self._key_buf, self.key_dc, self.key_scale, key_alpha, key_beta, key_quant_target),
-                (self._value_buf, self.value_dc, self.value_scale, value_alpha, value_beta,
-                 value_quant_target)):
-            view = buf[:, a:b]
-            quant_f32(view, al, be, tg, QUANT_LOWER, QUANT_UPPER, SCALE_MIN, SCALE_MAX,
-                      zp_state=dc, sc_state=scale, out=view)
+        view = (self._key_buf[:, a:b], self._value_buf[:, a:b])
+        quant_f32_pair(view if source is None else source,
+                       ((key_alpha, key_beta, key_quant_target), (value_alpha, value_beta, value_quant_target)),
+                       QUANT_LOWER, QUANT_UPPER, SCALE_MIN, SCALE_MAX, out=view, init=init,
+                       states=((self.key_dc, self.key_scale), (self.value_dc, self.value_scale)))
         self._quant_len = b
+
+    def _reads_in_place(self, x) -> bool:
+        # rows the quantiser can take from where they are: type and device of the buffers, contiguous
+        # channels, forward strides, and no graph that the copy into the buffer would be part of
+        return x.dtype == self._key_buf.dtype and x.device == self._key_buf.device and x.dim() == 3 and x.stride(2) == 1 \
+            and x.stride(1) >= x.shape[2] and x.dtype in (torch.float32, torch.float16, torch.bfloat16) \
+            and not (torch.is_grad_enabled() and x.requires_grad) and type(x) in (torch.Tensor, nn.Parameter)
 
     @property
     def key_states(self):
@@ -113,14 +120,32 @@ class KVCacheLayer_ADKV:
         B, T, C = key_states.shape
         if self._key_buf is None:
             self._init_buffers(B, C, key_states.device, key_states.dtype)
+        init = None
+        direct = T > 0 and (B, C) == (self._key_buf.shape[0], self._key_buf.shape[2]) \
+            and value_states.shape == key_states.shape and self._reads_in_place(key_states) and self._reads_in_place(value_states)
         if self.key_dc is None:
-            f = lambda p: p.detach().to(torch.float32).reshape(1, C).repeat(B, 1).contiguous()
+            if direct:
+                init = ((key_zp_init, key_scale_init), (value_zp_init, value_scale_init))
+                f = lambda p: torch.empty(B, C, dtype=torch.float32, device=key_states.device)
+            else:
+                f = lambda p: p.detach().to(torch.float32).reshape(1, C).repeat(B, 1).contiguous()
             self.key_dc, self.key_scale = f(key_zp_init), f(key_scale_init)
             self.value_dc, self.value_scale = f(value_zp_init), f(value_scale_init)
         self._cap_buffers(T)
-        self._append_tokens(key_states, value_states)
-        self._quantize_new_tokens(key_alpha, key_beta, key_quant_target,
-                                  value_alpha, value_beta, value_quant_target)
+        if not direct:
+            self._append_tokens(key_states, value_states)
+            self._quantize_new_tokens(key_alpha, key_beta, key_quant_target,
+                                      value_alpha, value_beta, value_quant_target)
+            return self.key_states, self.value_states
+        try:
+            self._recent_len += T
+            self._quantize_new_tokens(key_alpha, key_beta, key_quant_target,
+                                      value_alpha, value_beta, value_quant_target, (key_states, value_states), init)
+        except BaseException:   # the rows were never written: they are not in the cache
+            self._recent_len -= T
+            if init is not None:
+                self.key_dc = self.key_scale = self.value_dc = self.value_scale = None
+            raise
         return self.key_states, self.value_states
 
 

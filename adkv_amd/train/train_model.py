@@ -73,6 +73,34 @@ def quant_f32(x: torch.Tensor, alpha: torch.Tensor, beta: torch.Tensor, target: 
     return out, codes, zs, ss
 
 
+def quant_f32_pair(x, params, lower_limit: int, upper_limit: int, sc_min: float, sc_max: float, *, states, out, init=None) -> None:
+    """``quant_f32`` for the K and V rows of the same tokens in one launch, from ``x`` into ``out``.
+
+    Pairs, K first: ``x`` and ``out`` ``[B, T, C]`` (one shape and type, channel stride 1; ``out[i]`` may be
+    ``x[i]`` but not overlap it otherwise), ``params`` the vectors ``(alpha, beta, target)``, ``states`` the
+    fp32 ``[B, C]`` tensors ``(zp, sc)`` updated in place, ``init`` optional ``[C]`` vectors ``(zp, sc)`` to
+    start from instead.
+    """
+    B, T, C = x[0].shape
+    for t, o in zip(x, out):
+        _chk(t.dtype == x[0].dtype and t.dtype in _DTYPES and t.shape == x[0].shape and t.stride(2) == 1, "x must be [B, T, C] with unit channel stride")
+        _chk(o.shape == t.shape and o.dtype == t.dtype and o.stride(2) == 1, "out must match x in shape and dtype")
+    params = [_f32vec(v, C, n) for p in params for v, n in zip(p, ("alpha", "beta", "target"))]
+    init = [_f32vec(v, C, n) for p in init for v, n in zip(p, ("zp_init", "sc_init"))] if init else []
+    for t in (states := [t for p in states for t in p]):
+        _chk(t.dtype == torch.float32 and t.is_contiguous() and t.shape == (B, C), "states must be contiguous fp32 [B, C]")
+    dev = _need_device(*x, *out, *states, *params, *init)
+    ptrs = lambda ts: (_lib.C.c_void_p * len(ts))(*[t.data_ptr() for t in ts])
+    strides = lambda ts: (_lib.C.c_int64 * 4)(*[s for t in ts for s in (t.stride(0) if B > 1 else T * max(t.stride(1), C),
+                                                                        t.stride(1) if T > 1 else C)])
+    with _lib.device_guard(dev):
+        rc = _lib.lib().adkv_quant_f32_pair(
+            ptrs(x), strides(x), ptrs(out), strides(out), ptrs(states), ptrs(init) if init else None, ptrs(params),
+            B, T, C, _DTYPES[x[0].dtype], int(lower_limit), int(upper_limit), float(sc_min), float(sc_max),
+            _lib.current_stream_ptr(dev))
+    _lib.check(rc, "quant_f32_pair")
+
+
 def adkv_chunk_forward(kv_cache_chunk, current_zp, current_sc, alpha, beta, target,
                        upper_limit, lower_limit, sc_min, sc_max, output_states):
     """Same contract as the reference's ``_adkv_chunk_forward`` (train_model.py:46-86):

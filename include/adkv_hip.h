@@ -353,6 +353,21 @@ int adkv_quant_f32(const void *x, void *xhat, void *codes, void *zp_state, void 
                    int lower_limit, int upper_limit, float sc_min, float sc_max, void *stream);
 
 /*
+ * The same for two tensors of one shape and type (the K and V rows of the same tokens, the two calls
+ * of llama_adkv_eval.py:254-287) in one launch, each from where its rows are to where its result
+ * belongs.  Arrays of two, K first:
+ *   x, xhat                  pointers; xhat[i] may be x[i] (same strides) but not overlap it otherwise
+ *   x_strides, xhat_strides  {batch, token} element strides of each tensor
+ *   state                    {zp, sc} of each: fp32 [B, C], read unless init is given, always written
+ *   init                     {zp, sc} of each: fp32 [C], or NULL
+ *   params                   {alpha, beta, tgt} of each: fp32 [C]
+ */
+int adkv_quant_f32_pair(const void *const *x, const int64_t *x_strides, void *const *xhat,
+                        const int64_t *xhat_strides, void *const *state, const void *const *init,
+                        const void *const *params, int B, int T, int C, int x_dtype, int lower_limit,
+                        int upper_limit, float sc_min, float sc_max, void *stream);
+
+/*
  * Rotary position embedding of the query and key rows in one launch: x * cos + rotate_half(x) * sin
  * with every operation rounded to the activations' type as torch rounds it, bit-identical to
  * transformers' apply_rotary_pos_emb that the attention module calls before the cache

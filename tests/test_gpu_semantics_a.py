@@ -152,6 +152,37 @@ def test_quant_f32_half_inputs_in_place_and_chunked(gpu, oracle, dtype):
     assert torch.count_nonzero(buf[:, T:]) == 0
 
 
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("T,C,offset", [(8, 64, 0), (9, 64, 0), (31, 68, 0), (32, 64, 1), (33, 66, 0), (63, 63, 0), (64, 128, 2),
+                                        (65, 1, 0), (96, 132, 4), (97, 129, 3), (131, 192, 0)])
+def test_quant_f32_pair_at_chunk_and_block_edges(gpu, oracle, T, C, offset, dtype):
+    """K and V in one launch, from rows of one pitch into rows of another: around a chunk of 32 tokens
+    and a block of 64 channels, rows aligned for 4-channel accesses and not; a starting state per channel
+    with a scale under its floor."""
+    from adkv_amd.train.train_model import quant_f32_pair
+    B = 2
+    lo = torch.full((C,), -0.25)
+    tensors, wants = [], []
+    for i in range(2):
+        p = _params(C, 40 + i, 4)
+        p["sc"][::5] = lo[::5]
+        x = (torch.randn(B, T, C, generator=torch.Generator().manual_seed(T + i)) * 1.5).to(dtype)
+        wants.append(oracle.quant_f32(x.float().numpy(), *[p[k].numpy() for k in ("zp", "sc", "alpha", "beta", "tgt")]))
+        src = torch.empty(B, T, C + 2 * offset, dtype=dtype, device=gpu)[:, :, offset:offset + C]
+        src.copy_(x)
+        dst = torch.zeros(B, T + 3, C, dtype=dtype, device=gpu)
+        tensors.append((src, dst, {k: v.to(gpu) for k, v in p.items()}, [torch.empty(B, C, device=gpu) for _ in range(2)]))
+    quant_f32_pair([t[0] for t in tensors], [(t[2]["alpha"], t[2]["beta"], t[2]["tgt"]) for t in tensors], -8, 7,
+                   math.exp(-4.0), math.exp(4.0), states=[t[3] for t in tensors], out=[t[1][:, :T] for t in tensors],
+                   init=[(t[2]["zp"], t[2]["sc"]) for t in tensors])
+    torch.cuda.synchronize()
+    for (_, dst, _, (zp, sc)), want in zip(tensors, wants):
+        assert torch.equal(dst[:, :T].cpu(), torch.from_numpy(want["xhat"]).to(dtype))
+        assert torch.count_nonzero(dst[:, T:]) == 0
+        assert np.array_equal(_bits(zp).numpy(), want["zp"].view(np.int32))
+        assert np.array_equal(_bits(sc).numpy(), want["sc"].view(np.int32))
+
+
 def test_train_model_forward_and_chunk_forward(gpu, oracle):
     from adkv_amd.train import ADKVTrainModel, adkv_chunk_forward
     torch.manual_seed(3)
