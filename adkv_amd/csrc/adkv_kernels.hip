@@ -1828,22 +1828,32 @@ static Seg plan_segments(void *ckpt, int n_ckpt_cap, int ckpt_interval, int BH, 
     return s;
 }
 
-template <typename F256, typename FBIG>
-static void launch_units(long threads, int big, F256 f256, FBIG fbig)
+// Threads per workgroup of a shared-table launch.  The table takes 64 KB of a CU's 160 KB of LDS, so a
+// CU holds two workgroups: 4-wave ones (which spread over the CUs best) put at most two waves on a
+// SIMD, and a launch with more than that ran in two rounds although registers allow four.  Launches
+// of 9-12 waves per CU therefore take 12-wave workgroups and larger ones 16-wave ones, one table for
+// all of them.  us per step, 4-wave workgroups (matrix-core kernels: 8-wave) before /
+// now, batch x KV heads x tokens: 64 x 32 x 663 86 / 73, 90 x 32 x 300 77 / 58, 12 x 8 x 8190 of 256
+// channels 88 / 78; grouped queries 25 x 8 x 9000 110 / 102, 2-bit 40 x 8 x 4096 99 / 75.
+static int threads_per_workgroup(long threads)
 {
-    // 16-wave workgroups share one lookup table and let a CU hold 4 waves per SIMD; small launches
-    // use 4-wave workgroups so that they still spread over the CUs
-    if (big > 256 && threads >= (long)big * cus())
-        fbig(dim3((unsigned)((threads + big - 1) / big)), dim3(big));
-    else
-        f256(dim3((unsigned)((threads + 255) / 256)), dim3(256));
+    const long per_cu = (threads / 64 + cus() - 1) / cus();
+    return per_cu <= 8 ? 256 : per_cu <= 12 ? 768 : 1024;
 }
 
-#define ADKV_LAUNCH(KERNEL, DD, CC, BIG, ...)                                                   \
-    launch_units(                                                                               \
-        padded_units<DD / CC>(BH, seg.nseg) * (DD / CC), BIG,                                                  \
-        [&](dim3 g, dim3 b) { hipLaunchKernelGGL((KERNEL<DD, CC, 256>), g, b, 0, st, __VA_ARGS__); }, \
-        [&](dim3 g, dim3 b) { hipLaunchKernelGGL((KERNEL<DD, CC, BIG>), g, b, 0, st, __VA_ARGS__); })
+#define ADKV_LAUNCH_(KERNEL, DD, CC, BLK, ...)                                                      \
+    hipLaunchKernelGGL((KERNEL<DD, CC, BLK>), dim3((unsigned)((threads + (BLK)-1) / (BLK))), dim3(BLK), 0, st, __VA_ARGS__)
+#define ADKV_LAUNCH(KERNEL, DD, CC, ...)                                                            \
+    do {                                                                                            \
+        const long threads = padded_units<DD / CC>(BH, seg.nseg) * (DD / CC);                       \
+        const int blk = threads_per_workgroup(threads);                                       \
+        if (blk == 1024)                                                                            \
+            ADKV_LAUNCH_(KERNEL, DD, CC, 1024, __VA_ARGS__);                                        \
+        else if (blk == 768)                                                                        \
+            ADKV_LAUNCH_(KERNEL, DD, CC, 768, __VA_ARGS__);                                         \
+        else                                                                                        \
+            ADKV_LAUNCH_(KERNEL, DD, CC, 256, __VA_ARGS__);                                         \
+    } while (0)
 
 // Head dim 128 has a second shape, two channels per lane (a head per wave): twice the waves, each
 // with half the instruction stream per token.  It pays when every wave has a SIMD to itself and
@@ -1852,20 +1862,23 @@ static void launch_units(long threads, int big, F256 f256, FBIG fbig)
 #define ADKV_DISPATCH_D(KERNEL, ...)                  \
     switch (D) {                                      \
     case 128:                                         \
-        if (padded_units<32>(BH, seg.nseg) / 2 <= n_simd()) \
-            ADKV_LAUNCH(KERNEL, 128, 2, 256, __VA_ARGS__); \
-        else                                          \
-            ADKV_LAUNCH(KERNEL, 128, 4, 1024, __VA_ARGS__); \
+        if (padded_units<32>(BH, seg.nseg) / 2 <= n_simd()) { \
+            const long threads = padded_units<64>(BH, seg.nseg) * 64; \
+            ADKV_LAUNCH_(KERNEL, 128, 2, 256, __VA_ARGS__); \
+        } else                                        \
+            ADKV_LAUNCH(KERNEL, 128, 4, __VA_ARGS__); \
         break;                                        \
     case 256:                                         \
-        ADKV_LAUNCH(KERNEL, 256, 4, 1024, __VA_ARGS__); \
+        ADKV_LAUNCH(KERNEL, 256, 4, __VA_ARGS__);     \
         break;                                        \
-    default:                                          \
-        ADKV_LAUNCH(KERNEL, 512, 8, 256, __VA_ARGS__); \
+    default: {                                        \
+        const long threads = padded_units<64>(BH, seg.nseg) * 64; \
+        ADKV_LAUNCH_(KERNEL, 512, 8, 256, __VA_ARGS__); \
         break;                                        \
+    }                                                 \
     }
 
-// Matrix-core kernels (head dim 128): 16-wave workgroups for big launches, 8-wave ones otherwise
+// Matrix-core kernels (head dim 128): the same rule, with 8-wave workgroups for small launches
 // (their LDS tile leaves room for one workgroup per CU either way).  Eight query heads per KV head
 // need ~138 registers per lane, more than the 128 a 16-wave workgroup leaves: qk_gqa_kernel still
 // gains from four waves per SIMD with a dozen cold values spilled (cfg5 KV shape, 64 query heads:
@@ -1875,9 +1888,13 @@ static void launch_units(long threads, int big, F256 f256, FBIG fbig)
     do {                                                                                            \
         const long threads = padded_units<32>(BH, seg.nseg) * 32;                                   \
         constexpr int GBIG = (GQV <= 4 || BIG8) ? GQV : 1; /* unused instantiation otherwise */     \
-        if ((GQV <= 4 || BIG8) && threads >= 1024L * cus())                                         \
+        const int blk = (GQV <= 4 || BIG8) ? threads_per_workgroup(threads) : 512;            \
+        if (blk == 1024)                                                                            \
             hipLaunchKernelGGL((KERNEL<BB, GBIG, 1024>), dim3((unsigned)((threads + 1023) / 1024)), \
                                dim3(1024), 0, st, __VA_ARGS__);                                     \
+        else if (blk == 768)                                                                        \
+            hipLaunchKernelGGL((KERNEL<BB, GBIG, 768>), dim3((unsigned)((threads + 767) / 768)),    \
+                               dim3(768), 0, st, __VA_ARGS__);                                      \
         else                                                                                        \
             hipLaunchKernelGGL((KERNEL<BB, GQV, 512>), dim3((unsigned)((threads + 511) / 512)),     \
                                dim3(512), 0, st, __VA_ARGS__);                                      \
@@ -2473,9 +2490,10 @@ static const char *decode_kernel_name(int B, int Hq, int H, int T, int D, int bi
     const Seg seg = plan_segments(n_ckpt_cap > 0 && ckpt_interval > 0 ? &dummy : nullptr, n_ckpt_cap,
                                   ckpt_interval, B * H, T, D);
     if (D == 128 && (GQ > 1 || bits != 4 || mfma_for_mha())) {
-        const long threads = padded_units<32>(B * H, seg.nseg) * 32;
-        return threads >= 1024L * cus() ? "gqa_kernel, 16-wave workgroups (matrix cores)"
-                                      : "gqa_kernel, 8-wave workgroups (matrix cores)";
+        const int blk = threads_per_workgroup(padded_units<32>(B * H, seg.nseg) * 32);
+        return blk == 1024 ? "gqa_kernel, 16-wave workgroups (matrix cores)"
+               : blk == 768 ? "gqa_kernel, 12-wave workgroups (matrix cores)"
+                            : "gqa_kernel, 8-wave workgroups (matrix cores)";
     }
     if (use_head_table(B, H, GQ, bits, D, seg)) {
         Seg s2 = seg;
@@ -2490,7 +2508,10 @@ static const char *decode_kernel_name(int B, int Hq, int H, int T, int D, int bi
         const long units = padded_units<32>(B * H, seg.nseg);
         if (units / 2 <= n_simd())
             return "kernel<128,2,256> (shared table, two channels per lane)";
-        return units * 32 >= 1024L * cus() ? "kernel<128,4,1024> (shared table)" : "kernel<128,4,256> (shared table)";
+        const int blk = threads_per_workgroup(units * 32);
+        return blk == 1024 ? "kernel<128,4,1024> (shared table)"
+               : blk == 768 ? "kernel<128,4,768> (shared table)"
+                            : "kernel<128,4,256> (shared table)";
     }
     return D == 256 ? "kernel<256,4,*> (shared table)" : "kernel<512,8,256> (shared table)";
 }

@@ -877,6 +877,40 @@ def test_paired_append_reads_projection_outputs_in_place(gpu, oracle, dtype, str
         assert np.array_equal(_np16(states[i]).view(np.uint16), want[i][1]), i
 
 
+@pytest.mark.parametrize("B,Hkv,G,D,bits,T", [(66, 32, 1, 128, 4, 20), (93, 32, 1, 128, 4, 33), (37, 32, 1, 256, 4, 20),
+                                              (55, 32, 1, 256, 4, 17), (263, 8, 1, 128, 2, 19), (263, 8, 2, 128, 4, 19),
+                                              (263, 8, 8, 128, 2, 19)])
+def test_launches_of_9_to_16_waves_per_cu(gpu, oracle, B, Hkv, G, D, bits, T):
+    """12- and 16-wave workgroups of launches that do not fill the device, the last one ragged: sequences
+    at both ends and in the middle against the oracle."""
+    S, tps = 16, 32 // bits
+    x, p = _inputs(B, Hkv, T + 1, D, seed=G, bits=bits)
+    pn, pg = [_np16(t) for t in p.astuple()], [t.to(gpu) for t in p.astuple()]
+    g = torch.Generator().manual_seed(60 + G)
+    q = torch.randn(B, Hkv * G, 1, D, generator=g).half()
+    attn = torch.softmax(2.0 * torch.randn(B, Hkv * G, T + 1, generator=g), dim=-1).half()
+    cache = synth.alloc_cache(B, Hkv, T + tps, D, gpu, bits=bits)
+    st = torch.zeros(B, Hkv, D, 2, dtype=torch.float16, device=gpu)
+    ck = torch.zeros(B, Hkv, 3, D, 2, dtype=torch.float16, device=gpu)
+    gemv.append_kv(cache, x[:, :, :T].to(gpu), *pg, 0, st, ckpt=ck, ckpt_interval=S, bits=bits)
+    kc, vc, xnew = cache.clone(), cache.clone(), x[:, :, T:].to(gpu)
+    logits = gemv.forward_qk(q.to(gpu), kc, xnew, *pg, T, SMIN, SMAX, ckpt=ck, ckpt_interval=S, bits=bits)
+    out = gemv.forward_ov(attn.to(gpu), vc, xnew, *pg, SMIN, SMAX, ckpt=ck.clone(), ckpt_interval=S, bits=bits)
+    some = [0, B // 2, B - 1]
+    lg, og = _np16(logits[some]).reshape(3, Hkv, G, T + 1), _np16(out[some]).reshape(3, Hkv, G, D)
+    qn, an, xn = _np16(q[some]).reshape(3, Hkv, G, 1, D), _np16(attn[some]).reshape(3, Hkv, G, T + 1), _np16(x[some])
+    with oracle.code_bits(bits):
+        base = oracle.alloc_cache(3, Hkv, T + tps, D)
+        oracle.encode_kv_f16(base, xn[:, :, :T], *pn)
+        for j in range(G):
+            want = base.copy()
+            l, _ = oracle.forward_qk_f16(np.ascontiguousarray(qn[:, :, j]), want, xn[:, :, T:], *pn, T)
+            o, _ = oracle.forward_ov_f16(np.ascontiguousarray(an[:, :, j]), base.copy(), xn[:, :, T:], *pn)
+            assert np.all(np.abs(lg[:, :, j].astype(np.float64) - l) <= _ulp16(l) + 1e-3)
+            assert np.all(np.abs(og[:, :, j].astype(np.float64) - o) <= _ulp16(o) + 1e-3)
+    assert np.array_equal(kc[some].cpu().numpy(), want) and np.array_equal(vc[some].cpu().numpy(), want)
+
+
 @pytest.mark.parametrize("G,bits", [(4, 4), (8, 4), (2, 2), (4, 2), (8, 2)])
 def test_grouped_query_kernels_in_16_wave_workgroups(gpu, oracle, G, bits):
     """A launch big enough for the 16-wave workgroups (128 KV heads x 64 segments = 8192 units):
