@@ -136,12 +136,22 @@ constexpr int LUT_ENTRIES = 256;
 constexpr int LUT_COPIES = 32;
 constexpr int LUT_WORDS64 = LUT_ENTRIES * LUT_COPIES; // uint2 elements = 64 KB
 
-__device__ __forceinline__ void lut_fill(uint2 *lut, int tid, int nthreads)
+// nthreads: a multiple of 256.  16 lanes write a row, two copies each; the low nibble of a lane's
+// entries never changes and the high one is known once the loop is unrolled.  (An entry per lane and
+// iteration, computed from its index, took a 4-wave workgroup 544 instructions per wave, about 1 us.)
+template <int NT>
+__device__ __forceinline__ void lut_fill(uint2 *lut, int tid)
 {
-    for (int i = tid; i < LUT_WORDS64; i += nthreads) {
-        const int b = i / LUT_COPIES;
-        const h2 q = (h2){(h1)((b & 15) - 8), (h1)((b >> 4) - 8)};
-        lut[i] = make_uint2(as_u32(q), as_u32(q) & 0x7FFF7FFFu);
+    static_assert(NT % 256 == 0, "whole groups of 256 entries' 16 lanes");
+    uint4 *l4 = reinterpret_cast<uint4 *>(lut);
+    const uint32_t lo = as_u32((h2){(h1)(((tid >> 4) & 15) - 8), (h1)0.0f});
+#pragma unroll
+    for (int i = 0; i < LUT_WORDS64 / 2; i += NT) {
+        if (LUT_WORDS64 / 2 % NT != 0 && i + tid >= LUT_WORDS64 / 2)
+            break;
+        const uint32_t hi = as_u32((h2){(h1)0.0f, (h1)(((i + tid) >> 8) - 8)});
+        const uint32_t q = lo | hi, a = q & 0x7FFF7FFFu;
+        l4[i + tid] = make_uint4(q, a, q, a);
     }
 }
 
@@ -170,6 +180,60 @@ __device__ __forceinline__ void update_pair_abs(Pair &p, h2 qabs, h2 qs)
     const h2 f = pk_fma(p.be, qabs, p.omt);
     p.sc = p.sc * f;
 }
+
+// Eight tokens of one channel pair per lane, laid out by hand for a wave that has its SIMD to itself
+// (one instruction every 4 cycles, whatever it is, wait states included): q*sc, the next scale, the
+// value, the next zero-point and the next token's f, in an order in which no packed result is read by
+// the very next instruction, so that no wait state is needed.  x[t] = value of token t.
+#define ADKV_REPLAY_TOKEN(Q, VAL)                       \
+    "v_pk_mul_f16 %[qs], " Q ", %[sc]\n\t"              \
+    "v_pk_mul_f16 %[sc], %[sc], %[f]\n\t"               \
+    "v_pk_add_f16 " VAL ", %[qs], %[zp]\n\t"            \
+    "v_pk_fma_f16 %[zp], %[al], %[qs], %[zp]\n\t"
+#define ADKV_REPLAY_F(A) "v_pk_fma_f16 %[f], %[be], " A ", %[omt]\n\t"
+__device__ __forceinline__ void replay_eight(Pair &p, const uint2 *e, uint32_t *x)
+{
+    uint32_t zp = as_u32(p.zp), sc = as_u32(p.sc), qs, f;
+    asm(ADKV_REPLAY_F("%[a0]") ADKV_REPLAY_TOKEN("%[q0]", "%[x0]") ADKV_REPLAY_F("%[a1]") ADKV_REPLAY_TOKEN("%[q1]", "%[x1]")
+        ADKV_REPLAY_F("%[a2]") ADKV_REPLAY_TOKEN("%[q2]", "%[x2]") ADKV_REPLAY_F("%[a3]") ADKV_REPLAY_TOKEN("%[q3]", "%[x3]")
+        ADKV_REPLAY_F("%[a4]") ADKV_REPLAY_TOKEN("%[q4]", "%[x4]") ADKV_REPLAY_F("%[a5]") ADKV_REPLAY_TOKEN("%[q5]", "%[x5]")
+        ADKV_REPLAY_F("%[a6]") ADKV_REPLAY_TOKEN("%[q6]", "%[x6]") ADKV_REPLAY_F("%[a7]") ADKV_REPLAY_TOKEN("%[q7]", "%[x7]")
+        "s_nop 0"
+        : [zp] "+v"(zp), [sc] "+v"(sc), [qs] "=&v"(qs), [f] "=&v"(f), [x0] "=&v"(x[0]), [x1] "=&v"(x[1]), [x2] "=&v"(x[2]),
+          [x3] "=&v"(x[3]), [x4] "=&v"(x[4]), [x5] "=&v"(x[5]), [x6] "=&v"(x[6]), [x7] "=&v"(x[7])
+        : [q0] "v"(e[0].x), [q1] "v"(e[1].x), [q2] "v"(e[2].x), [q3] "v"(e[3].x), [q4] "v"(e[4].x), [q5] "v"(e[5].x),
+          [q6] "v"(e[6].x), [q7] "v"(e[7].x), [a0] "v"(e[0].y), [a1] "v"(e[1].y), [a2] "v"(e[2].y), [a3] "v"(e[3].y),
+          [a4] "v"(e[4].y), [a5] "v"(e[5].y), [a6] "v"(e[6].y), [a7] "v"(e[7].y), [al] "v"(as_u32(p.al)),
+          [be] "v"(as_u32(p.be)), [omt] "v"(as_u32(p.omt)));
+    p.zp = as_h2(zp);
+    p.sc = as_h2(sc);
+}
+// The same, each value multiplied by its token's weight (two per word of w) and added to acc in fp32.
+#define ADKV_REPLAY_ADD(W, HI)                                                            \
+    "v_fma_mix_f32 %[c0], " W ", %[x], %[c0] op_sel:[" HI ",0,0] op_sel_hi:[1,1,0]\n\t"   \
+    "v_fma_mix_f32 %[c1], " W ", %[x], %[c1] op_sel:[" HI ",1,0] op_sel_hi:[1,1,0]\n\t"
+#define ADKV_REPLAY_TWO(Q0, Q1, A1, A2, W)                                                            \
+    ADKV_REPLAY_TOKEN(Q0, "%[x]") ADKV_REPLAY_F(A1) ADKV_REPLAY_ADD(W, "0")                           \
+    ADKV_REPLAY_TOKEN(Q1, "%[x]") ADKV_REPLAY_F(A2) ADKV_REPLAY_ADD(W, "1")
+__device__ __forceinline__ void replay_eight_weighted(Pair &p, const uint2 *e, const uint4 &w, float *acc)
+{
+    uint32_t zp = as_u32(p.zp), sc = as_u32(p.sc), qs, f, x;
+    asm(ADKV_REPLAY_F("%[a0]") ADKV_REPLAY_TWO("%[q0]", "%[q1]", "%[a1]", "%[a2]", "%[w0]")
+        ADKV_REPLAY_TWO("%[q2]", "%[q3]", "%[a3]", "%[a4]", "%[w1]") ADKV_REPLAY_TWO("%[q4]", "%[q5]", "%[a5]", "%[a6]", "%[w2]")
+        ADKV_REPLAY_TOKEN("%[q6]", "%[x]") ADKV_REPLAY_F("%[a7]") ADKV_REPLAY_ADD("%[w3]", "0")
+        ADKV_REPLAY_TOKEN("%[q7]", "%[x]") ADKV_REPLAY_ADD("%[w3]", "1")
+        : [zp] "+v"(zp), [sc] "+v"(sc), [qs] "=&v"(qs), [f] "=&v"(f), [x] "=&v"(x), [c0] "+v"(acc[0]), [c1] "+v"(acc[1])
+        : [q0] "v"(e[0].x), [q1] "v"(e[1].x), [q2] "v"(e[2].x), [q3] "v"(e[3].x), [q4] "v"(e[4].x), [q5] "v"(e[5].x),
+          [q6] "v"(e[6].x), [q7] "v"(e[7].x), [a0] "v"(e[0].y), [a1] "v"(e[1].y), [a2] "v"(e[2].y), [a3] "v"(e[3].y),
+          [a4] "v"(e[4].y), [a5] "v"(e[5].y), [a6] "v"(e[6].y), [a7] "v"(e[7].y), [w0] "v"(w.x), [w1] "v"(w.y),
+          [w2] "v"(w.z), [w3] "v"(w.w), [al] "v"(as_u32(p.al)), [be] "v"(as_u32(p.be)), [omt] "v"(as_u32(p.omt)));
+    p.zp = as_h2(zp);
+    p.sc = as_h2(sc);
+}
+#undef ADKV_REPLAY_TWO
+#undef ADKV_REPLAY_ADD
+#undef ADKV_REPLAY_F
+#undef ADKV_REPLAY_TOKEN
 
 // Code width.  4 bits is the reference's format (8 tokens per 32-bit channel word, codes in
 // [-8, 7], stored as q + 8).  2 bits is the same recurrence over codes in [-2, 1] (the range the

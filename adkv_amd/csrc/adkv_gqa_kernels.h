@@ -135,13 +135,13 @@ struct Lookups {
     }
 };
 
-template <int BITS>
-__device__ __forceinline__ void fill_table(uint2 *lut, int tid, int nthreads)
+template <int BITS, int NT>
+__device__ __forceinline__ void fill_table(uint2 *lut, int tid)
 {
     if (BITS == 4)
-        lut_fill(lut, tid, nthreads);
+        lut_fill<NT>(lut, tid);
     else
-        lut2_fill(lut, tid, nthreads);
+        lut2_fill(lut, tid, NT);
 }
 
 template <int BITS>
@@ -169,7 +169,7 @@ __global__ __launch_bounds__(BLK) void qk_gqa_kernel(
     using G = Geo<D, CPL>;
     __shared__ uint2 smem[LUT_WORDS64 + (BLK / 64) * TILE_WORDS64];
     const uint2 *lut = smem;
-    fill_table<BITS>(smem, threadIdx.x, BLK);
+    fill_table<BITS, BLK>(smem, threadIdx.x);
     __syncthreads();
 
     const int lane = threadIdx.x & 63;
@@ -351,7 +351,7 @@ __global__ __launch_bounds__(BLK) void ov_gqa_kernel(
     static_assert((GPF * UPS) % WPF == 0, "weight ring must line up with the unrolled loop");
     using G = Geo<D, CPL>;
     __shared__ uint2 lut[LUT_WORDS64];
-    fill_table<BITS>(lut, threadIdx.x, BLK);
+    fill_table<BITS, BLK>(lut, threadIdx.x);
     __syncthreads();
     const int lane = threadIdx.x & 63;
     const uint32_t lane_copy = table_lane_offset<BITS>(lane);

@@ -31,6 +31,9 @@
 namespace adkv {
 
 constexpr int PF = 4; // supergroups in flight per lane (2, 6 and 8 were measured: no difference)
+// two channels per lane: 64 tokens ahead of a loop that takes 29 ns per token (with 32 it ran into the
+// memory's latency: forward_ov of 32 x 32 heads x 1024 tokens 38 us, with 64 32)
+constexpr int PF_PAIR = 8;
 
 template <int D, int CPL>
 struct Geo {
@@ -157,6 +160,9 @@ __host__ __device__ inline int seg_end(const Seg &sa, int seg)
                      : (seg + 1) * sa.seg_tokens;
 }
 __host__ __device__ inline bool seg_is_last(const Seg &sa, int seg) { return segment_of_slot(sa, seg) == sa.nseg - 1; }
+
+// waits for every LDS and scalar access in flight, as an instruction that the compiler counts with
+__device__ __forceinline__ void wait_lgkm() { __builtin_amdgcn_s_waitcnt(0xC07F); }
 
 __device__ __forceinline__ float wave_xor_add(float v, int mask)
 {
@@ -856,6 +862,9 @@ __device__ __forceinline__ void pair_bytes_of(const typename Geo<D, CPL>::Vec *u
 // Per lane and supergroup: 8 fp32 partial logits (v_dot2_f32_f16 over the lane's channel pairs).
 // They are summed across the head's lanes and scattered by reduce8_head (masked DPP adds and row
 // swaps, no LDS): afterwards every quad of lanes holds the total of one token.
+typedef _Float16 h8v __attribute__((ext_vector_type(8))); // operand of v_mfma_f32_16x16x32_f16
+constexpr int PAIR_TILE = 16 * 256; // bytes of a wave's key tile in the two-channel form of qk_kernel
+
 template <int D, int CPL, int BLK>
 __global__ __launch_bounds__(BLK) void qk_kernel(
     const h1 *__restrict__ q, uint4 *__restrict__ cache, const h1 *__restrict__ k_new,
@@ -865,10 +874,13 @@ __global__ __launch_bounds__(BLK) void qk_kernel(
     int BH, int H, int T, int n_super_cap, h1 *__restrict__ state_out, Seg sa)
 {
     using G = Geo<D, CPL>;
+    sa.groups = 0; // only even plans come here (a fifth of the code was the other kind's cuts)
+    // two channels per lane: the head fills the wave, see the loop below
+    constexpr bool PAIR = CPL == 2;
     // the only LDS object: the table sits at LDS offset 0 (its byte address is used as is)
-    __shared__ uint2 smem[LUT_WORDS64];
+    __shared__ uint2 smem[LUT_WORDS64 + (PAIR ? (BLK / 64) * PAIR_TILE / 8 : 0)];
     const uint2 *lut = smem;
-    lut_fill(smem, threadIdx.x, BLK);
+    lut_fill<BLK>(smem, threadIdx.x);
     __syncthreads();
 
     const int lane = threadIdx.x & 63;
@@ -906,76 +918,172 @@ __global__ __launch_bounds__(BLK) void qk_kernel(
             ob[sg * 8 + tk] = (h1)s;
     };
 
-    // ---- software pipeline over the full supergroups.  Global loads run PF supergroups ahead.
-    // Table lookups run one supergroup ahead and are issued token by token between the arithmetic
-    // of the current supergroup (the LDS counter holds only 15 outstanding operations, so issuing a
-    // whole supergroup's lookups at once would stall on them).  The logits of supergroup sg-1 are
-    // reduced and stored at the start of iteration sg, while the first lookups are in flight.
-    // The lookup for the next supergroup goes into the slot the current token has just vacated, so
-    // one supergroup's worth of registers holds both.
-    auto token = [&](int t, uint2 (*e)[8], const uint32_t (*nb)[2], float &out_t) {
-        float acc;
+    if constexpr (PAIR) {
+        // A wave has its SIMD (nearly) to itself and pays for every instruction, so what is left per
+        // token is the lookup, the replay (replay_eight) and half a write: the values of 16 tokens go
+        // to an LDS tile, from which the matrix cores take them as columns against the query as every
+        // row.  All rows of the product are equal, so lane t (modulo 16) receives token t's logit
+        // whichever row it holds, and nothing is summed across lanes.  ~10 issue slots per token
+        // where the dot product, its reduction over the lanes and the wait states made it 19
+        // (32 x 32 heads x 1024 tokens, one segment: 49 -> 34 us; ov_kernel with replay_eight_weighted
+        // 38 -> 32).
+        // The tile: row t = token t, 256 bytes; its 16-byte pieces are permuted by (t / 2) % 8 so that
+        // both halves of an access to 16 rows at once spread over the banks.
+        char *tile = reinterpret_cast<char *>(smem + LUT_WORDS64) + (threadIdx.x >> 6) * PAIR_TILE;
+        const int row = lane & 15, kb = lane >> 4;
+        h8v qa[4];
+        int rd[4], wr[8];
 #pragma unroll
-        for (int p = 0; p < G::NP; p++) {
-            Pair &s = st[p];
-            const h2 qs = as_h2(e[p][t].x) * s.sc;
-            const h2 kh = qs + s.zp;
-            if (p == 0)
-                acc = dot2_from_zero(qv[p], kh);
-            else
-                acc = __builtin_amdgcn_fdot2(qv[p], kh, acc, false);
-            update_pair_abs(s, as_h2(e[p][t].y), qs);
+        for (int m = 0; m < 4; m++) {
+            const h1 *src = q + (size_t)bx * D + m * 32 + kb * 8;
+            const h2 a = load_act2(src, sa.act_bf16), b = load_act2(src + 2, sa.act_bf16);
+            const h2 c = load_act2(src + 4, sa.act_bf16), d = load_act2(src + 6, sa.act_bf16);
+            qa[m] = (h8v){a.x, a.y, b.x, b.y, c.x, c.y, d.x, d.y};
+            rd[m] = row * 256 + (((m * 4 + kb) ^ (row >> 1)) << 4);
         }
-        out_t = acc;
 #pragma unroll
-        for (int p = 0; p < G::NP; p++)
-            e[p][t] = lut_get(lut, nb[p][t & 1], lane_copy, t >> 1);
-        __builtin_amdgcn_sched_barrier(0);
-    };
-
-    Vec buf[PF][G::NV];
-    uint2 lk[G::NP][8];
-    uint32_t nb[G::NP][2];
-    float part[8] = {0, 0, 0, 0, 0, 0, 0, 0};
+        for (int j = 0; j < 8; j++)
+            wr[j] = (lane * 4) ^ (j << 4);
+        auto lookup = [&](uint2 *e, const Vec *u) __attribute__((always_inline)) {
+            uint32_t nb[1][2];
+            pair_bytes_of<D, CPL>(u, nb);
 #pragma unroll
-    for (int i = 0; i < PF; i++) {
+            for (int t = 0; t < 8; t++)
+                e[t] = lut_get(lut, nb[0][t & 1], lane_copy, t >> 1);
+        };
+        h8v kv[4] = {};
+        f4v d;
+        auto fetch = [&]() __attribute__((always_inline)) {
 #pragma unroll
-        for (int v = 0; v < G::NV; v++)
-            buf[i][v] = (i < nfull) ? load_codes(cb + (size_t)i * G::VPS + v) : vec_zero<Vec>();
-    }
-    if (nfull > 0) {
-        pair_bytes_of<D, CPL>(buf[0], nb);
+            for (int m = 0; m < 4; m++)
+                kv[m] = *reinterpret_cast<const h8v *>(tile + rd[m]);
+        };
+        auto multiply = [&]() __attribute__((always_inline)) {
+            d = (f4v){0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
-        for (int t = 0; t < 8; t++)
+            for (int m = 0; m < 4; m++)
+                d = __builtin_amdgcn_mfma_f32_16x16x32_f16(qa[m], kv[m], d, 0, 0, 0);
+        };
+        auto emit = [&](int sg, int ntok) __attribute__((always_inline)) { // sg: first supergroup of the tile
+            if (active && lane < ntok)
+                ob[sg * 8 + lane] = (h1)d.x;
+        };
+        if (nfull > 0) {
+            Vec buf[PF_PAIR][G::NV];
+            uint2 e[2][8];
+            // unconditional loads, here and in the loop, and no scalar load in flight when it starts:
+            // otherwise the waits inside it have to cover what this entry leaves open
+#pragma unroll
+            for (int i = 0; i < PF_PAIR; i++) {
+                buf[i][0] = load_codes(cb + (size_t)min(i, nfull - 1) * G::VPS);
+                __builtin_amdgcn_sched_barrier(0);
+            }
+            lookup(e[0], buf[0]);
+            wait_lgkm();
+            rotate_over<PF_PAIR>(nfull, [&](int sg, auto ic) __attribute__((always_inline)) {
+                constexpr int i = decltype(ic)::value, half = i & 1;
+                lookup(e[half ^ 1], buf[(i + 1) % PF_PAIR]); // stale past the end: looked up, never used
+                buf[i][0] = load_codes(cb + (size_t)min(sg + PF_PAIR, nfull - 1) * G::VPS);
+                __builtin_amdgcn_sched_barrier(0);
+                uint32_t kh[8];
+                replay_eight(st[0], e[half], kh);
+#pragma unroll
+                for (int t = 0; t < 8; t++)
+                    *reinterpret_cast<uint32_t *>(tile + (half * 8 + t) * 256 + wr[half * 4 + t / 2]) = kh[t];
+                __builtin_amdgcn_sched_barrier(0);
+                // the tile before this one: fetched when it was complete, multiplied half a tile later,
+                // stored another half later
+                if constexpr (half == 0) {
+                    multiply();
+                } else {
+                    emit(sg - 3, sg > 1 ? 16 : 0);
+                    fetch();
+                }
+                __builtin_amdgcn_sched_barrier(0);
+            });
+            const int last_sg = nfull - 1;
+            if (last_sg & 1) {
+                multiply();
+                emit(last_sg - 1, 16);
+            } else { // half a tile, and the one before it is not stored yet
+                emit(last_sg - 2, last_sg > 0 ? 16 : 0);
+                fetch();
+                multiply();
+                emit(last_sg, 8);
+            }
+        }
+    } else {
+        // ---- software pipeline over the full supergroups.  Global loads run PF supergroups ahead.
+        // Table lookups run one supergroup ahead and are issued token by token between the arithmetic
+        // of the current supergroup (the LDS counter holds only 15 outstanding operations, so issuing a
+        // whole supergroup's lookups at once would stall on them).  The logits of supergroup sg-1 are
+        // reduced and stored at the start of iteration sg, while the first lookups are in flight.
+        // The lookup for the next supergroup goes into the slot the current token has just vacated, so
+        // one supergroup's worth of registers holds both.
+        auto token = [&](int t, uint2 (*e)[8], const uint32_t (*nb)[2], float &out_t) {
+            float acc;
+#pragma unroll
+            for (int p = 0; p < G::NP; p++) {
+                Pair &s = st[p];
+                const h2 qs = as_h2(e[p][t].x) * s.sc;
+                const h2 kh = qs + s.zp;
+                if (p == 0)
+                    acc = dot2_from_zero(qv[p], kh);
+                else
+                    acc = __builtin_amdgcn_fdot2(qv[p], kh, acc, false);
+                update_pair_abs(s, as_h2(e[p][t].y), qs);
+            }
+            out_t = acc;
 #pragma unroll
             for (int p = 0; p < G::NP; p++)
-                lk[p][t] = lut_get(lut, nb[p][t & 1], lane_copy, t >> 1);
-    }
-    // One supergroup; i = its buffer in the rotation (compile-time).  Nothing in here is
-    // conditional: the trip count is wave-uniform, the prefetch index is clamped, and the
-    // reduction of the previous supergroup stores nothing when there is none (sg == 0).
-    auto body = [&](int sg, auto ic) {
-        constexpr int i = decltype(ic)::value;
-        // bytes of supergroup sg+1 (stale data past the end: looked up, never used)
-        pair_bytes_of<D, CPL>(buf[(i + 1) % PF], nb);
-        {
-            // unconditional, clamped to the segment's last supergroup: a load inside a branch
-            // makes the next wait cover every load in flight, this one included
-            const int sgp = min(sg + PF, nfull - 1);
+                e[p][t] = lut_get(lut, nb[p][t & 1], lane_copy, t >> 1);
+            __builtin_amdgcn_sched_barrier(0);
+        };
+
+        Vec buf[PF][G::NV];
+        uint2 lk[G::NP][8];
+        uint32_t nb[G::NP][2];
+        float part[8] = {0, 0, 0, 0, 0, 0, 0, 0};
+#pragma unroll
+        for (int i = 0; i < PF; i++) {
 #pragma unroll
             for (int v = 0; v < G::NV; v++)
-                buf[i][v] = load_codes(cb + (size_t)sgp * G::VPS + v);
+                buf[i][v] = (i < nfull) ? load_codes(cb + (size_t)i * G::VPS + v) : vec_zero<Vec>();
         }
-        __builtin_amdgcn_sched_barrier(0);
-        finish(part, sg - 1, sg > 0 ? 8 : 0);
-        __builtin_amdgcn_sched_barrier(0);
+        if (nfull > 0) {
+            pair_bytes_of<D, CPL>(buf[0], nb);
 #pragma unroll
-        for (int t = 0; t < 8; t++)
-            token(t, lk, nb, part[t]);
-    };
-    rotate_over<PF>(nfull, body);
-    if (nfull > 0)
-        finish(part, nfull - 1, 8);
+            for (int t = 0; t < 8; t++)
+#pragma unroll
+                for (int p = 0; p < G::NP; p++)
+                    lk[p][t] = lut_get(lut, nb[p][t & 1], lane_copy, t >> 1);
+        }
+        // One supergroup; i = its buffer in the rotation (compile-time).  Nothing in here is
+        // conditional: the trip count is wave-uniform, the prefetch index is clamped, and the
+        // reduction of the previous supergroup stores nothing when there is none (sg == 0).
+        auto body = [&](int sg, auto ic) {
+            constexpr int i = decltype(ic)::value;
+            // bytes of supergroup sg+1 (stale data past the end: looked up, never used)
+            pair_bytes_of<D, CPL>(buf[(i + 1) % PF], nb);
+            {
+                // unconditional, clamped to the segment's last supergroup: a load inside a branch
+                // makes the next wait cover every load in flight, this one included
+                const int sgp = min(sg + PF, nfull - 1);
+#pragma unroll
+                for (int v = 0; v < G::NV; v++)
+                    buf[i][v] = load_codes(cb + (size_t)sgp * G::VPS + v);
+            }
+            __builtin_amdgcn_sched_barrier(0);
+            finish(part, sg - 1, sg > 0 ? 8 : 0);
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int t = 0; t < 8; t++)
+                token(t, lk, nb, part[t]);
+        };
+        rotate_over<PF>(nfull, body);
+        if (nfull > 0)
+            finish(part, nfull - 1, 8);
+    }
     if (!last)
         return;
 
@@ -1037,8 +1145,10 @@ __global__ __launch_bounds__(BLK) void ov_kernel(
     int BH, int H, int T, int n_super_cap, h1 *__restrict__ state_out, Seg sa)
 {
     using G = Geo<D, CPL>;
+    constexpr int AHEAD = CPL == 2 ? PF_PAIR : PF;
+    sa.groups = 0; // only even plans come here
     __shared__ uint2 lut[LUT_WORDS64];
-    lut_fill(lut, threadIdx.x, BLK);
+    lut_fill<BLK>(lut, threadIdx.x);
     __syncthreads();
     const uint32_t lane_copy = (uint32_t)(threadIdx.x & (LUT_COPIES - 1)) * 8u;
 
@@ -1082,27 +1192,6 @@ __global__ __launch_bounds__(BLK) void ov_kernel(
         __builtin_memcpy(&r, wb + (size_t)sg * 8, 16); // row base is only 2-byte aligned
         return r;
     };
-    // one token of the current supergroup, followed by the lookups of the same token slot of the
-    // next supergroup (see qk_kernel for why they are interleaved)
-    auto token = [&](int t, uint2 (*e)[8], const uint32_t (*nb)[2], const uint4 wv) {
-        const uint32_t ww[4] = {wv.x, wv.y, wv.z, wv.w};
-        const h2 wp = as_h2(ww[t >> 1]);
-        const float wt = (t & 1) ? (float)wp.y : (float)wp.x;
-#pragma unroll
-        for (int p = 0; p < G::NP; p++) {
-            Pair &s = st[p];
-            const h2 qs = as_h2(e[p][t].x) * s.sc;
-            const h2 vd = qs + s.zp;
-            acc[2 * p] = __builtin_fmaf(wt, (float)vd.x, acc[2 * p]);
-            acc[2 * p + 1] = __builtin_fmaf(wt, (float)vd.y, acc[2 * p + 1]);
-            update_pair_abs(s, as_h2(e[p][t].y), qs);
-        }
-#pragma unroll
-        for (int p = 0; p < G::NP; p++)
-            e[p][t] = lut_get(lut, nb[p][t & 1], lane_copy, t >> 1);
-        __builtin_amdgcn_sched_barrier(0);
-    };
-
     // two tokens of the current supergroup on the matrix cores, then the lookups of the same two
     // slots of the next one
     auto token2 = [&](int t, uint2 (*e)[8], const uint32_t (*nb)[2], const uint4 wv) {
@@ -1130,48 +1219,55 @@ __global__ __launch_bounds__(BLK) void ov_kernel(
         __builtin_amdgcn_sched_barrier(0);
     };
 
-    Vec buf[PF][G::NV];
-    uint4 wbuf[PF];
-    uint2 lk[G::NP][8];
+    Vec buf[AHEAD][G::NV];
+    uint4 wbuf[AHEAD];
+    uint2 lk[MM ? G::NP : 2][8]; // two channels per lane: this supergroup's lookups and the next one's
     uint32_t nb[G::NP][2];
-#pragma unroll
-    for (int i = 0; i < PF; i++) {
-#pragma unroll
-        for (int v = 0; v < G::NV; v++)
-            buf[i][v] = (i < nfull) ? load_codes(cb + (size_t)i * G::VPS + v) : vec_zero<Vec>();
-        wbuf[i] = (i < nfull) ? load_w(i) : make_uint4(0, 0, 0, 0);
-    }
     if (nfull > 0) {
+        // unconditional, in the loop's order: see qk_kernel
+#pragma unroll
+        for (int i = 0; i < AHEAD; i++) {
+            const int sg = min(i, nfull - 1);
+#pragma unroll
+            for (int v = 0; v < G::NV; v++)
+                buf[i][v] = load_codes(cb + (size_t)sg * G::VPS + v);
+            wbuf[i] = load_w(sg);
+            __builtin_amdgcn_sched_barrier(0);
+        }
         pair_bytes_of<D, CPL>(buf[0], nb);
 #pragma unroll
         for (int t = 0; t < 8; t++)
 #pragma unroll
             for (int p = 0; p < G::NP; p++)
                 lk[p][t] = lut_get(lut, nb[p][t & 1], lane_copy, t >> 1);
+        wait_lgkm();
     }
     // one supergroup, nothing conditional in it (see qk_kernel); i = its buffer in the rotation
     auto body = [&](int sg, auto ic) {
         constexpr int i = decltype(ic)::value;
-        pair_bytes_of<D, CPL>(buf[(i + 1) % PF], nb);
-        const int sgp = min(sg + PF, nfull - 1);
+        pair_bytes_of<D, CPL>(buf[(i + 1) % AHEAD], nb);
+        const int sgp = min(sg + AHEAD, nfull - 1);
 #pragma unroll
         for (int v = 0; v < G::NV; v++)
             buf[i][v] = load_codes(cb + (size_t)sgp * G::VPS + v);
         __builtin_amdgcn_sched_barrier(0);
-        if (MM) {
+        if constexpr (MM) {
 #pragma unroll
             for (int t = 0; t < 8; t += 2)
                 token2(t, lk, nb, wbuf[i]);
         } else {
+            // a wave (nearly) alone on its SIMD: see replay_eight
 #pragma unroll
             for (int t = 0; t < 8; t++)
-                token(t, lk, nb, wbuf[i]);
+                lk[(i & 1) ^ 1][t] = lut_get(lut, nb[0][t & 1], lane_copy, t >> 1);
+            replay_eight_weighted(st[0], lk[i & 1], wbuf[i], acc);
+            __builtin_amdgcn_sched_barrier(0);
         }
         // the weights are reloaded once their last token is done: loading them earlier into a
         // second register set costs copies at the loop edge, which wait for the load they move
         wbuf[i] = load_w(sgp);
     };
-    rotate_over<PF>(nfull, body);
+    rotate_over<AHEAD>(nfull, body);
     if (MM) {
 #pragma unroll
         for (int p = 0; p < G::NP; p++) {

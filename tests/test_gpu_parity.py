@@ -877,6 +877,14 @@ def test_paired_append_reads_projection_outputs_in_place(gpu, oracle, dtype, str
         assert np.array_equal(_np16(states[i]).view(np.uint16), want[i][1]), i
 
 
+@pytest.mark.parametrize("B,H,T,S", [(1, 3, T, 256) for T in (1, 8, 9, 15, 16, 17, 24, 31, 64, 72, 73, 128, 136, 250)]
+                         + [(5, 7, 100, 24), (3, 4, 16 * 9, 16)])
+def test_two_channel_lanes_around_tiles_of_16_tokens(gpu, oracle, B, H, T, S):
+    """Head per wave: whole, half and missing tiles of 16 tokens, fewer supergroups than are kept in
+    flight, one segment and several."""
+    test_checkpointed_segments(gpu, oracle, B, H, T, 128, S)
+
+
 @pytest.mark.parametrize("B,Hkv,G,D,bits,T", [(66, 32, 1, 128, 4, 20), (93, 32, 1, 128, 4, 33), (37, 32, 1, 256, 4, 20),
                                               (55, 32, 1, 256, 4, 17), (263, 8, 1, 128, 2, 19), (263, 8, 2, 128, 4, 19),
                                               (263, 8, 8, 128, 2, 19)])
