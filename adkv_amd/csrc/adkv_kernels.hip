@@ -863,7 +863,111 @@ __device__ __forceinline__ void pair_bytes_of(const typename Geo<D, CPL>::Vec *u
 // They are summed across the head's lanes and scattered by reduce8_head (masked DPP adds and row
 // swaps, no LDS): afterwards every quad of lanes holds the total of one token.
 typedef _Float16 h8v __attribute__((ext_vector_type(8))); // operand of v_mfma_f32_16x16x32_f16
-constexpr int PAIR_TILE = 16 * 256; // bytes of a wave's key tile in the two-channel form of qk_kernel
+constexpr int PAIR_TILE = 16 * 256; // bytes of a wave's key tile
+
+// forward_qk of a segment with the head over a whole wave, two channels per lane.
+// A wave has its SIMD (nearly) to itself and pays for every instruction, so what is left per
+// token is the lookup, the replay (replay_eight) and half a write: the values of 16 tokens go
+// to an LDS tile, from which the matrix cores take them as columns against the query as every
+// row.  All rows of the product are equal, so lane t (modulo 16) receives token t's logit
+// whichever row it holds, and nothing is summed across lanes.  ~10 issue slots per token
+// where the dot product, its reduction over the lanes and the wait states made it 19
+// (32 x 32 heads x 1024 tokens, one segment: 49 -> 34 us; ov_kernel with replay_eight_weighted
+// 38 -> 32).
+// The tile: row t = token t, 256 bytes; its 16-byte pieces are permuted by (t / 2) % 8 so that
+// both halves of an access to 16 rows at once spread over the banks.
+// put(token, logit) is called for token 0.. of the segment, one lane per token.
+template <typename PUT>
+__device__ __forceinline__ void pair_scores(const uint2 *lut, char *tile, int lane, uint32_t lane_copy, Pair &st,
+                                            const h1 *qrow, int act_bf16, const uint2 *cb, int nfull, PUT &&put)
+{
+    using G = Geo<128, 2>;
+    using Vec = G::Vec;
+    constexpr int D = 128, CPL = 2;
+    const int row = lane & 15, kb = lane >> 4;
+    h8v qa[4];
+    int rd[4], wr[8];
+#pragma unroll
+    for (int m = 0; m < 4; m++) {
+        const h1 *src = qrow + m * 32 + kb * 8;
+        const h2 a = load_act2(src, act_bf16), b = load_act2(src + 2, act_bf16);
+        const h2 c = load_act2(src + 4, act_bf16), d = load_act2(src + 6, act_bf16);
+        qa[m] = (h8v){a.x, a.y, b.x, b.y, c.x, c.y, d.x, d.y};
+        rd[m] = row * 256 + (((m * 4 + kb) ^ (row >> 1)) << 4);
+    }
+#pragma unroll
+    for (int j = 0; j < 8; j++)
+        wr[j] = (lane * 4) ^ (j << 4);
+    auto lookup = [&](uint2 *e, const Vec *u) __attribute__((always_inline)) {
+        uint32_t nb[1][2];
+        pair_bytes_of<D, CPL>(u, nb);
+#pragma unroll
+        for (int t = 0; t < 8; t++)
+            e[t] = lut_get(lut, nb[0][t & 1], lane_copy, t >> 1);
+    };
+    h8v kv[4] = {};
+    f4v d;
+    auto fetch = [&]() __attribute__((always_inline)) {
+#pragma unroll
+        for (int m = 0; m < 4; m++)
+            kv[m] = *reinterpret_cast<const h8v *>(tile + rd[m]);
+    };
+    auto multiply = [&]() __attribute__((always_inline)) {
+        d = (f4v){0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+        for (int m = 0; m < 4; m++)
+            d = __builtin_amdgcn_mfma_f32_16x16x32_f16(qa[m], kv[m], d, 0, 0, 0);
+    };
+    auto emit = [&](int sg, int ntok) __attribute__((always_inline)) { // sg: first supergroup of the tile
+        if (lane < ntok)
+            put(sg * 8 + lane, (h1)d.x);
+    };
+    if (nfull > 0) {
+        Vec buf[PF_PAIR][G::NV];
+        uint2 e[2][8];
+        // unconditional loads, here and in the loop, and no scalar load in flight when it starts:
+        // otherwise the waits inside it have to cover what this entry leaves open
+#pragma unroll
+        for (int i = 0; i < PF_PAIR; i++) {
+            buf[i][0] = load_codes(cb + (size_t)min(i, nfull - 1) * G::VPS);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        lookup(e[0], buf[0]);
+        wait_lgkm();
+        rotate_over<PF_PAIR>(nfull, [&](int sg, auto ic) __attribute__((always_inline)) {
+            constexpr int i = decltype(ic)::value, half = i & 1;
+            lookup(e[half ^ 1], buf[(i + 1) % PF_PAIR]); // stale past the end: looked up, never used
+            buf[i][0] = load_codes(cb + (size_t)min(sg + PF_PAIR, nfull - 1) * G::VPS);
+            __builtin_amdgcn_sched_barrier(0);
+            uint32_t kh[8];
+            replay_eight(st, e[half], kh);
+#pragma unroll
+            for (int t = 0; t < 8; t++)
+                *reinterpret_cast<uint32_t *>(tile + (half * 8 + t) * 256 + wr[half * 4 + t / 2]) = kh[t];
+            __builtin_amdgcn_sched_barrier(0);
+            // the tile before this one: fetched when it was complete, multiplied half a tile later,
+            // stored another half later
+            if constexpr (half == 0) {
+                multiply();
+            } else {
+                emit(sg - 3, sg > 1 ? 16 : 0);
+                fetch();
+            }
+            __builtin_amdgcn_sched_barrier(0);
+        });
+        const int last_sg = nfull - 1;
+        if (last_sg & 1) {
+            multiply();
+            emit(last_sg - 1, 16);
+        } else { // half a tile, and the one before it is not stored yet
+            emit(last_sg - 2, last_sg > 0 ? 16 : 0);
+            fetch();
+            multiply();
+            emit(last_sg, 8);
+        }
+    }
+}
+
 
 template <int D, int CPL, int BLK>
 __global__ __launch_bounds__(BLK) void qk_kernel(
@@ -919,99 +1023,12 @@ __global__ __launch_bounds__(BLK) void qk_kernel(
     };
 
     if constexpr (PAIR) {
-        // A wave has its SIMD (nearly) to itself and pays for every instruction, so what is left per
-        // token is the lookup, the replay (replay_eight) and half a write: the values of 16 tokens go
-        // to an LDS tile, from which the matrix cores take them as columns against the query as every
-        // row.  All rows of the product are equal, so lane t (modulo 16) receives token t's logit
-        // whichever row it holds, and nothing is summed across lanes.  ~10 issue slots per token
-        // where the dot product, its reduction over the lanes and the wait states made it 19
-        // (32 x 32 heads x 1024 tokens, one segment: 49 -> 34 us; ov_kernel with replay_eight_weighted
-        // 38 -> 32).
-        // The tile: row t = token t, 256 bytes; its 16-byte pieces are permuted by (t / 2) % 8 so that
-        // both halves of an access to 16 rows at once spread over the banks.
-        char *tile = reinterpret_cast<char *>(smem + LUT_WORDS64) + (threadIdx.x >> 6) * PAIR_TILE;
-        const int row = lane & 15, kb = lane >> 4;
-        h8v qa[4];
-        int rd[4], wr[8];
-#pragma unroll
-        for (int m = 0; m < 4; m++) {
-            const h1 *src = q + (size_t)bx * D + m * 32 + kb * 8;
-            const h2 a = load_act2(src, sa.act_bf16), b = load_act2(src + 2, sa.act_bf16);
-            const h2 c = load_act2(src + 4, sa.act_bf16), d = load_act2(src + 6, sa.act_bf16);
-            qa[m] = (h8v){a.x, a.y, b.x, b.y, c.x, c.y, d.x, d.y};
-            rd[m] = row * 256 + (((m * 4 + kb) ^ (row >> 1)) << 4);
-        }
-#pragma unroll
-        for (int j = 0; j < 8; j++)
-            wr[j] = (lane * 4) ^ (j << 4);
-        auto lookup = [&](uint2 *e, const Vec *u) __attribute__((always_inline)) {
-            uint32_t nb[1][2];
-            pair_bytes_of<D, CPL>(u, nb);
-#pragma unroll
-            for (int t = 0; t < 8; t++)
-                e[t] = lut_get(lut, nb[0][t & 1], lane_copy, t >> 1);
-        };
-        h8v kv[4] = {};
-        f4v d;
-        auto fetch = [&]() __attribute__((always_inline)) {
-#pragma unroll
-            for (int m = 0; m < 4; m++)
-                kv[m] = *reinterpret_cast<const h8v *>(tile + rd[m]);
-        };
-        auto multiply = [&]() __attribute__((always_inline)) {
-            d = (f4v){0.0f, 0.0f, 0.0f, 0.0f};
-#pragma unroll
-            for (int m = 0; m < 4; m++)
-                d = __builtin_amdgcn_mfma_f32_16x16x32_f16(qa[m], kv[m], d, 0, 0, 0);
-        };
-        auto emit = [&](int sg, int ntok) __attribute__((always_inline)) { // sg: first supergroup of the tile
-            if (active && lane < ntok)
-                ob[sg * 8 + lane] = (h1)d.x;
-        };
-        if (nfull > 0) {
-            Vec buf[PF_PAIR][G::NV];
-            uint2 e[2][8];
-            // unconditional loads, here and in the loop, and no scalar load in flight when it starts:
-            // otherwise the waits inside it have to cover what this entry leaves open
-#pragma unroll
-            for (int i = 0; i < PF_PAIR; i++) {
-                buf[i][0] = load_codes(cb + (size_t)min(i, nfull - 1) * G::VPS);
-                __builtin_amdgcn_sched_barrier(0);
-            }
-            lookup(e[0], buf[0]);
-            wait_lgkm();
-            rotate_over<PF_PAIR>(nfull, [&](int sg, auto ic) __attribute__((always_inline)) {
-                constexpr int i = decltype(ic)::value, half = i & 1;
-                lookup(e[half ^ 1], buf[(i + 1) % PF_PAIR]); // stale past the end: looked up, never used
-                buf[i][0] = load_codes(cb + (size_t)min(sg + PF_PAIR, nfull - 1) * G::VPS);
-                __builtin_amdgcn_sched_barrier(0);
-                uint32_t kh[8];
-                replay_eight(st[0], e[half], kh);
-#pragma unroll
-                for (int t = 0; t < 8; t++)
-                    *reinterpret_cast<uint32_t *>(tile + (half * 8 + t) * 256 + wr[half * 4 + t / 2]) = kh[t];
-                __builtin_amdgcn_sched_barrier(0);
-                // the tile before this one: fetched when it was complete, multiplied half a tile later,
-                // stored another half later
-                if constexpr (half == 0) {
-                    multiply();
-                } else {
-                    emit(sg - 3, sg > 1 ? 16 : 0);
-                    fetch();
-                }
-                __builtin_amdgcn_sched_barrier(0);
-            });
-            const int last_sg = nfull - 1;
-            if (last_sg & 1) {
-                multiply();
-                emit(last_sg - 1, 16);
-            } else { // half a tile, and the one before it is not stored yet
-                emit(last_sg - 2, last_sg > 0 ? 16 : 0);
-                fetch();
-                multiply();
-                emit(last_sg, 8);
-            }
-        }
+        pair_scores(lut, reinterpret_cast<char *>(smem + LUT_WORDS64) + (threadIdx.x >> 6) * PAIR_TILE, lane, lane_copy,
+                    st[0], q + (size_t)bx * D, sa.act_bf16, cb, nfull,
+                    [&](int t, h1 v) __attribute__((always_inline)) {
+                        if (active)
+                            ob[t] = v;
+                    });
     } else {
         // ---- software pipeline over the full supergroups.  Global loads run PF supergroups ahead.
         // Table lookups run one supergroup ahead and are issued token by token between the arithmetic
@@ -1830,6 +1847,7 @@ static inline int lanes_per_head(int D) { return D == 128 ? 32 : 64; }
 
 #include "adkv_gqa_kernels.h"
 #include "adkv_ft_kernels.h"
+#include "adkv_small_step.h"
 
 // Waves a SIMD should hold for packed-f16 issue to run near full rate, and SIMDs on the device.
 constexpr int WAVES_PER_SIMD_TARGET = 4;
@@ -2300,6 +2318,27 @@ static int fused_step_plan(Seg &ka, Seg &va, int B, int Hq, int H, int T, int D,
     if (lanes != lanes_v || ka.nseg != 4 || va.nseg != 4 || ka.phys_per_head != W || va.phys_per_head != W)
         return 0;
     return lanes;
+}
+
+static thread_local hipEvent_t g_stage_events[4] = {nullptr, nullptr, nullptr, nullptr};
+
+// Whether a step runs as small_step_kernel, and its plan: a workgroup per (sequence, head), one per CU, a
+// wave per segment.  us per step on the device, three or four launches /
+// one, sequences x heads x tokens: 1 x 32 x 603 25.6 / 20.3 (and 15 us of host time / 5), 8 x 32 x 1000
+// 27.7 / 22.4, 4 x 32 x 200 20.4 / 18.1, 2 x 8 x 64 12.8 / 11.4.  With five to eight segments two waves
+// share a SIMD while other CUs idle, and beyond one workgroup per CU (its LDS allows no second) a launch
+// takes two rounds: those stay with the separate launches, as do callers that time the stages.
+static bool small_step_plan(Seg &seg, int B, int Hq, int H, int T, int D, int bits, void *k_ckpt, void *v_ckpt,
+                            int n_ckpt_cap, int ckpt_interval)
+{
+    if (D != 128 || bits != 4 || Hq != H || T < 0 || T + 1 > SMALL_ROW || (long)B * H > cus() || !k_ckpt != !v_ckpt ||
+        g_mha_kernel.load(std::memory_order_relaxed) >= 0 || mha_kernel_default())
+        return false;
+    for (const hipEvent_t e : g_stage_events)
+        if (e != nullptr)
+            return false;
+    seg = plan_segments(k_ckpt, n_ckpt_cap, ckpt_interval, B * H, T, D);
+    return seg.nseg <= 4;
 }
 
 static int check_ckpt(const void *ckpt, int n_ckpt_cap, int ckpt_interval, int bits = 4)
@@ -3090,7 +3129,6 @@ int adkv_softmax(const void *logits, void *weights, const void *mask,
 static int64_t pad256(int64_t n) { return (n + 255) & ~(int64_t)255; }
 
 // Events adkv_decode_step records around its stages in this thread (a measurement hook).
-static thread_local hipEvent_t g_stage_events[4] = {nullptr, nullptr, nullptr, nullptr};
 
 void adkv_set_stage_events(void *const *events)
 {
@@ -3126,6 +3164,36 @@ int64_t adkv_decode_step_workspace_bytes(int B, int Hq, int H, int T, int D, int
     const int64_t mat = pad256((int64_t)B * Hq * adkv_row_pitch(T + 1) * 2);
     return 2 * mat + pad256(adkv_softmax_workspace_bytes(B * Hq, T + 1)) +
            adkv_forward_ov_gqa_workspace_bytes(B, Hq, H, T, D, n_ckpt_cap, ckpt_interval);
+}
+
+static FtParams ft_params(const void *const *p)
+{
+    return {(const h1 *)p[0], (const h1 *)p[1], (const h1 *)p[2], (const h1 *)p[3], (const h1 *)p[4]};
+}
+
+// What forward_qk and forward_ov would refuse, for the steps that run as one launch (4-bit codes, one
+// query head per KV head).
+static int check_step(const void *q, const void *k_cache, const void *v_cache, const void *k_new, const void *v_new,
+                      const void *const *k_params, const void *const *v_params, const void *out, const void *weights, int B,
+                      int H, int T, int D, int n_super_cap, int bits, const void *k_ckpt, const void *v_ckpt, int n_ckpt_cap,
+                      int ckpt_interval)
+{
+    int rc = check_common(B, H, T, D, n_super_cap);
+    if (rc)
+        return rc;
+    if (T / 8 >= n_super_cap)
+        return ADKV_E_CAPACITY;
+    if (!q || !k_cache || !v_cache || !k_new || !v_new || !out)
+        return ADKV_E_NULL;
+    for (int i = 0; i < 5; i++)
+        if (!k_params[i] || !v_params[i])
+            return ADKV_E_NULL;
+    if (((uintptr_t)k_cache & 15) || ((uintptr_t)v_cache & 15) || ((uintptr_t)q & 7) || ((uintptr_t)k_new & 3) ||
+        ((uintptr_t)v_new & 3) || ((uintptr_t)out & 3) || ((uintptr_t)weights & 1))
+        return ADKV_E_ALIGN;
+    if ((rc = check_ckpt(k_ckpt, n_ckpt_cap, ckpt_interval, bits)))
+        return rc;
+    return check_ckpt(v_ckpt, n_ckpt_cap, ckpt_interval, bits);
 }
 
 int adkv_decode_step(const void *q, void *k_cache, void *v_cache, const void *k_new, const void *v_new,
@@ -3165,27 +3233,13 @@ int adkv_decode_step(const void *q, void *k_cache, void *v_cache, const void *k_
         Seg ka, va;
         const int lanes = mask ? 0 : fused_step_plan(ka, va, B, Hq, H, T, D, bits, k_ckpt, v_ckpt, n_ckpt_cap, ckpt_interval);
         if (lanes) {
-            if ((rc = check_common(B, H, T, D, n_super_cap)))
-                return rc;
-            if (T / 8 >= n_super_cap)
-                return ADKV_E_CAPACITY;
-            if (!q || !k_cache || !v_cache || !k_new || !v_new || !out)
-                return ADKV_E_NULL;
-            for (int i = 0; i < 5; i++)
-                if (!k_params[i] || !v_params[i])
-                    return ADKV_E_NULL;
-            if (((uintptr_t)k_cache & 15) || ((uintptr_t)v_cache & 15) || ((uintptr_t)q & 7) || ((uintptr_t)k_new & 3) ||
-                ((uintptr_t)v_new & 3) || ((uintptr_t)out & 3) || ((uintptr_t)weights & 1))
-                return ADKV_E_ALIGN;
-            if ((rc = check_ckpt(k_ckpt, n_ckpt_cap, ckpt_interval, bits)) || (rc = check_ckpt(v_ckpt, n_ckpt_cap, ckpt_interval, bits)))
+            if ((rc = check_step(q, k_cache, v_cache, k_new, v_new, k_params, v_params, out, weights, B, H, T, D, n_super_cap,
+                                 bits, k_ckpt, v_ckpt, n_ckpt_cap, ckpt_interval)))
                 return rc;
             ka.row_pitch = va.row_pitch = ld;
             ka.act_bf16 = va.act_bf16 = act_bf16;
             va.combine = 1;
-            const FtParams kp = {(const h1 *)k_params[0], (const h1 *)k_params[1], (const h1 *)k_params[2],
-                                 (const h1 *)k_params[3], (const h1 *)k_params[4]};
-            const FtParams vp = {(const h1 *)v_params[0], (const h1 *)v_params[1], (const h1 *)v_params[2],
-                                 (const h1 *)v_params[3], (const h1 *)v_params[4]};
+            const FtParams kp = ft_params(k_params), vp = ft_params(v_params);
             const auto kernel = lanes == 16 ? decode_ft_kernel<16> : decode_ft_kernel<32>;
             hipLaunchKernelGGL(kernel, dim3((unsigned)(H * ka.phys_per_head)), dim3(FT_BLK), 0, (hipStream_t)stream,
                                (const h1 *)q, (uint4 *)k_cache, (const h1 *)k_new, (uint4 *)v_cache, (const h1 *)v_new,
@@ -3196,6 +3250,26 @@ int adkv_decode_step(const void *q, void *k_cache, void *v_cache, const void *k_
                 if ((rc = stage_mark(i, stream)))
                     return rc;
             return ADKV_OK;
+        }
+    }
+    {
+        Seg ka;
+        if (small_step_plan(ka, B, Hq, H, T, D, bits, k_ckpt, v_ckpt, n_ckpt_cap, ckpt_interval)) {
+            if ((rc = check_step(q, k_cache, v_cache, k_new, v_new, k_params, v_params, out, weights, B, H, T, D, n_super_cap,
+                                 bits, k_ckpt, v_ckpt, n_ckpt_cap, ckpt_interval)))
+                return rc;
+            if (mask && rows_per_mask_row <= 0)
+                return ADKV_E_SHAPE;
+            ka.row_pitch = ld;
+            ka.act_bf16 = act_bf16;
+            Seg va = ka;
+            va.ckpt = (h1 *)v_ckpt;
+            const FtParams kp = ft_params(k_params), vp = ft_params(v_params);
+            hipLaunchKernelGGL(small_step_kernel, dim3((unsigned)(B * H)), dim3(256), 0, (hipStream_t)stream, (const h1 *)q,
+                               (uint2 *)k_cache, (const h1 *)k_new, (uint2 *)v_cache, (const h1 *)v_new, (const float *)mask,
+                               mask ? rows_per_mask_row : 1, (h1 *)weights, (h1 *)out, kp, vp, H, T,
+                               n_super_cap, scaling, ka, va);
+            return check_launch();
         }
     }
     rc = forward_qk_impl(q, k_cache, k_new, logits, k_params[0], k_params[1], k_params[2],

@@ -885,6 +885,58 @@ def test_two_channel_lanes_around_tiles_of_16_tokens(gpu, oracle, B, H, T, S):
     test_checkpointed_segments(gpu, oracle, B, H, T, 128, S)
 
 
+@pytest.mark.parametrize("masked", [False, True])
+@pytest.mark.parametrize("B,H,T,S", [(1, 1, 0, 0), (2, 3, 1, 64), (1, 2, 63, 64), (2, 2, 64, 64), (1, 3, 130, 64), (2, 2, 192, 64),
+                                     (1, 2, 255, 64), (1, 2, 256, 64), (3, 1, 511, 0), (1, 2, 512, 256), (1, 2, 1023, 256),
+                                     (1, 1, 1535, 0)])
+def test_step_of_few_short_sequences_in_one_launch(gpu, oracle, B, H, T, S, masked):
+    """One to four segments, ragged and whole last ones, rows up to the longest, with and without a mask:
+    codes, checkpoints and, against the separate launches, the same logits to within one rounding."""
+    from adkv_amd import _lib
+    D = 128
+    (xk, pk), (xv, pv) = (_inputs(B, H, T + 1, D, seed=T + i) for i in range(2))
+    pn = [[_np16(t) for t in p.astuple()] for p in (pk, pv)]
+    kp, vp = (tuple(t.to(gpu) for t in p.astuple()) for p in (pk, pv))
+    g = torch.Generator().manual_seed(T)
+    q = torch.randn(B, H, 1, D, generator=g).half()
+    mask = None
+    if masked:
+        mask = torch.zeros(B, 1, 1, T + 1)
+        mask[:, :, :, :T // 3] = torch.finfo(torch.float16).min
+    base = []
+    for x, p in ((xk, kp), (xv, vp)):
+        c, st = synth.alloc_cache(B, H, T + 9, D, gpu), torch.zeros(B, H, D, 2, dtype=torch.float16, device=gpu)
+        ck = torch.zeros(B, H, T // S + 2, D, 2, dtype=torch.float16, device=gpu) if S else None
+        if T:
+            gemv.append_kv(c, x[:, :, :T].to(gpu), *p, 0, st, ckpt=ck, ckpt_interval=S)
+        base.append((c, ck))
+    got = []
+    for family in (-1, 0):   # one launch; the separate ones
+        _lib.lib().adkv_set_mha_kernel(family)
+        try:
+            bufs = [(c.clone(), None if ck is None else ck.clone()) for c, ck in base]
+            out, w = gemv.decode_step(q.to(gpu), bufs[0][0], bufs[1][0], xk[:, :, T:].to(gpu), xv[:, :, T:].to(gpu), kp, vp, T,
+                                      D ** -0.5, None if mask is None else mask.to(gpu), k_ckpt=bufs[0][1], v_ckpt=bufs[1][1],
+                                      ckpt_interval=S)
+            torch.cuda.synchronize()
+        finally:
+            _lib.lib().adkv_set_mha_kernel(-1)
+        got.append((bufs, _np16(out).astype(np.float64), _np16(w).astype(np.float64)))
+    for (c1, k1), (c2, k2) in zip(got[0][0], got[1][0]):
+        assert torch.equal(c1, c2) and (k1 is None or torch.equal(k1.view(torch.int16), k2.view(torch.int16)))
+    kc, vc = (c.cpu().numpy().copy() for c, _ in base)
+    want, ww, logits = oracle.decode_step_f16(_np16(q), kc, vc, _np16(xk)[:, :, T:], _np16(xv)[:, :, T:], *pn, T, D ** -0.5,
+                                              None if mask is None else mask[:, :, 0].numpy())
+    assert np.array_equal(got[0][0][0][0].cpu().numpy(), kc) and np.array_equal(got[0][0][1][0].cpu().numpy(), vc)
+    # a logit that rounds the other way moves its weight by one fp16 step of it times the scaling; the sum of
+    # the exponentials by no more than the largest of these; a weight is rounded to 11 bits (subnormal: 2^-24)
+    step = 2.0 ** -10 * np.abs(logits).max() * D ** -0.5
+    vmax = 2 * float(xv.abs().max())   # the weights sum to one: an output moves by no more than that share of the largest value
+    for _, out, w in got:
+        assert np.all(np.abs(w - ww.astype(np.float64)) <= ww.astype(np.float64) * (2 * step + 2.0 ** -10) + 2.0 ** -24)
+        assert np.all(np.abs(out - want) <= _ulp16(want) + (2 * step + 2.0 ** -10) * vmax)
+
+
 @pytest.mark.parametrize("B,Hkv,G,D,bits,T", [(66, 32, 1, 128, 4, 20), (93, 32, 1, 128, 4, 33), (37, 32, 1, 256, 4, 20),
                                               (55, 32, 1, 256, 4, 17), (263, 8, 1, 128, 2, 19), (263, 8, 2, 128, 4, 19),
                                               (263, 8, 8, 128, 2, 19)])
