@@ -885,6 +885,32 @@ def test_two_channel_lanes_around_tiles_of_16_tokens(gpu, oracle, B, H, T, S):
     test_checkpointed_segments(gpu, oracle, B, H, T, 128, S)
 
 
+@pytest.mark.parametrize("B,H,T,D,S,bits", [(1, 2, 1, 128, 16, 4), (2, 3, 7, 128, 16, 4), (2, 2, 63, 128, 16, 4), (1, 3, 64, 128, 64, 4),
+                                            (1, 2, 65, 128, 64, 2), (2, 1, 577, 256, 64, 4), (3, 2, 129, 512, 0, 4),
+                                            (80, 32, 130, 128, 64, 4)])
+def test_first_tokens_of_an_uninitialised_cache(gpu, oracle, B, H, T, D, S, bits):
+    """``fresh``: caches, states and checkpoints full of garbage end up as zeroed ones do, to the last free
+    slot; one and two channels per lane, whole runs of groups and less, with and without checkpoints."""
+    tps = 32 // bits
+    (xk, pk), (xv, pv) = (_inputs(B, H, T, D, seed=T + i, bits=bits) for i in range(2))
+    kp, vp = (tuple(t.to(gpu) for t in p.astuple()) for p in (pk, pv))
+    k, v = xk.to(gpu), xv.to(gpu)
+    res = []
+    for fresh in (False, True):
+        fill = 0x5B if fresh else 0
+        cs = [torch.full_like(synth.alloc_cache(B, H, T + 3 * tps, D, gpu, bits=bits), fill) for _ in range(2)]
+        st = [torch.full((B, H, D, 2), 7.0 * fresh, dtype=torch.float16, device=gpu) for _ in range(2)]
+        ck = [torch.full((B, H, T // S + 2, D, 2), 7.0 * fresh, dtype=torch.float16, device=gpu) if S else None for _ in range(2)]
+        gemv.append_kv_pair(*cs, k, v, kp, vp, 0, *st, k_ckpt=ck[0], v_ckpt=ck[1], ckpt_interval=S, bits=bits, fresh=fresh)
+        res.append(cs + [t.view(torch.int16) for t in st + ck if t is not None])
+    torch.cuda.synchronize()
+    assert all(torch.equal(a, b) for a, b in zip(*res))
+    with oracle.code_bits(bits):
+        want = oracle.alloc_cache(1, H, T + 3 * tps, D)
+        oracle.encode_kv_f16(want, _np16(xk)[-1:], *[_np16(t) for t in pk.astuple()])
+    assert np.array_equal(res[1][0][-1:].cpu().numpy(), want)
+
+
 @pytest.mark.parametrize("masked", [False, True])
 @pytest.mark.parametrize("B,H,T,S", [(1, 1, 0, 0), (2, 3, 1, 64), (1, 2, 63, 64), (2, 2, 64, 64), (1, 3, 130, 64), (2, 2, 192, 64),
                                      (1, 2, 255, 64), (1, 2, 256, 64), (3, 1, 511, 0), (1, 2, 512, 256), (1, 2, 1023, 256),

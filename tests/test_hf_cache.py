@@ -767,3 +767,13 @@ def test_rope_equals_transformers_bit_for_bit(gpu, dtype, B, Hq, H, T, D, shared
     # packed inputs and a table that is a slice (odd storage offset in bytes / 4 is fine, strides even)
     got_q2, _ = gemv.rope_qk(q.contiguous(), k.contiguous(), cos, sin)
     assert torch.equal(as_bits(got_q2), as_bits(want_q))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("B,Hq,H,T,D", [(1, 4, 3, 733, 128), (2, 32, 8, 129, 128), (1, 5, 2, 800, 256), (3, 32, 32, 300, 128),
+                                        (40, 64, 64, 1, 128), (39, 64, 64, 1, 128), (1, 6, 1, 1024, 48)])
+def test_rope_in_16_byte_pieces(gpu, dtype, B, Hq, H, T, D):
+    """Enough rows for the 16-byte form: one and four heads per lane, head counts, token counts and row
+    lengths that leave lanes over; and the last size below it."""
+    test_rope_equals_transformers_bit_for_bit(gpu, dtype, B, Hq, H, T, D, T % 2 == 0)
