@@ -14,6 +14,7 @@ import math
 
 import torch
 from torch import nn
+from torch.autograd import forward_ad
 from transformers.models.llama.modeling_llama import (
     LlamaAttention,
     LlamaDecoderLayer,
@@ -98,12 +99,22 @@ class KVCacheLayer_ADKV:
                        states=((self.key_dc, self.key_scale), (self.value_dc, self.value_scale)))
         self._quant_len = b
 
-    def _reads_in_place(self, x) -> bool:
+    @staticmethod
+    def _only_bytes(x, buf) -> bool:
+        """Whether copying ``x`` into ``buf`` would move values and do nothing else.  The quantiser reads
+        memory and sees neither a graph (of the rows, or of rows copied into the buffer earlier) nor a
+        forward-mode tangent, a transform's wrapper, a pending negation or a recording of the copy."""
+        return type(x) in (torch.Tensor, nn.Parameter) and not x.is_neg() \
+            and not (torch.is_grad_enabled() and (x.requires_grad or buf.requires_grad)) \
+            and not torch._C._functorch.is_functorch_wrapped_tensor(x) \
+            and forward_ad.unpack_dual(x).tangent is None \
+            and not torch.jit.is_tracing() and torch._C._len_torch_dispatch_stack() == 0
+
+    def _reads_in_place(self, x, buf) -> bool:
         # rows the quantiser can take from where they are: type and device of the buffers, contiguous
-        # channels, forward strides, and no graph that the copy into the buffer would be part of
-        return x.dtype == self._key_buf.dtype and x.device == self._key_buf.device and x.dim() == 3 and x.stride(2) == 1 \
-            and x.stride(1) >= x.shape[2] and x.dtype in (torch.float32, torch.float16, torch.bfloat16) \
-            and not (torch.is_grad_enabled() and x.requires_grad) and type(x) in (torch.Tensor, nn.Parameter)
+        # channels, forward strides
+        return x.dtype == buf.dtype and x.device == buf.device and x.dim() == 3 and x.stride(2) == 1 \
+            and x.stride(1) >= x.shape[2] and x.dtype in (torch.float32, torch.float16, torch.bfloat16) and self._only_bytes(x, buf)
 
     @property
     def key_states(self):
@@ -122,7 +133,8 @@ class KVCacheLayer_ADKV:
             self._init_buffers(B, C, key_states.device, key_states.dtype)
         init = None
         direct = T > 0 and (B, C) == (self._key_buf.shape[0], self._key_buf.shape[2]) \
-            and value_states.shape == key_states.shape and self._reads_in_place(key_states) and self._reads_in_place(value_states)
+            and value_states.shape == key_states.shape and self._reads_in_place(key_states, self._key_buf) \
+            and self._reads_in_place(value_states, self._value_buf)
         if self.key_dc is None:
             if direct:
                 init = ((key_zp_init, key_scale_init), (value_zp_init, value_scale_init))
