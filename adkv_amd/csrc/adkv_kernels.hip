@@ -2320,23 +2320,18 @@ static int fused_step_plan(Seg &ka, Seg &va, int B, int Hq, int H, int T, int D,
     return lanes;
 }
 
-static thread_local hipEvent_t g_stage_events[4] = {nullptr, nullptr, nullptr, nullptr};
-
 // Whether a step runs as small_step_kernel, and its plan: a workgroup per (sequence, head), one per CU, a
 // wave per segment.  us per step on the device, three or four launches /
 // one, sequences x heads x tokens: 1 x 32 x 603 25.6 / 20.3 (and 15 us of host time / 5), 8 x 32 x 1000
 // 27.7 / 22.4, 4 x 32 x 200 20.4 / 18.1, 2 x 8 x 64 12.8 / 11.4.  With five to eight segments two waves
 // share a SIMD while other CUs idle, and beyond one workgroup per CU (its LDS allows no second) a launch
-// takes two rounds: those stay with the separate launches, as do callers that time the stages.
+// takes two rounds: those stay with the separate launches.
 static bool small_step_plan(Seg &seg, int B, int Hq, int H, int T, int D, int bits, void *k_ckpt, void *v_ckpt,
                             int n_ckpt_cap, int ckpt_interval)
 {
     if (D != 128 || bits != 4 || Hq != H || T < 0 || T + 1 > SMALL_ROW || (long)B * H > cus() || !k_ckpt != !v_ckpt ||
         g_mha_kernel.load(std::memory_order_relaxed) >= 0 || mha_kernel_default())
         return false;
-    for (const hipEvent_t e : g_stage_events)
-        if (e != nullptr)
-            return false;
     seg = plan_segments(k_ckpt, n_ckpt_cap, ckpt_interval, B * H, T, D);
     return seg.nseg <= 4;
 }
@@ -3128,7 +3123,9 @@ int adkv_softmax(const void *logits, void *weights, const void *mask,
 
 static int64_t pad256(int64_t n) { return (n + 255) & ~(int64_t)255; }
 
-// Events adkv_decode_step records around its stages in this thread (a measurement hook).
+// Events adkv_decode_step records around its stages in this thread (a measurement hook: what runs does
+// not depend on it).
+static thread_local hipEvent_t g_stage_events[4] = {nullptr, nullptr, nullptr, nullptr};
 
 void adkv_set_stage_events(void *const *events)
 {
@@ -3146,6 +3143,15 @@ static int stage_mark(int i, void *stream)
         return ADKV_E_LAUNCH;
     }
     return ADKV_OK;
+}
+
+// after a launch that is all three stages
+static int mark_one_launch(void *stream)
+{
+    int rc = ADKV_OK;
+    for (int i = 1; i <= 3 && !rc; i++)
+        rc = stage_mark(i, stream);
+    return rc;
 }
 
 int64_t adkv_forward_ov_gqa_workspace_bytes(int B, int Hq, int H, int T, int D, int n_ckpt_cap,
@@ -3244,12 +3250,7 @@ int adkv_decode_step(const void *q, void *k_cache, void *v_cache, const void *k_
             hipLaunchKernelGGL(kernel, dim3((unsigned)(H * ka.phys_per_head)), dim3(FT_BLK), 0, (hipStream_t)stream,
                                (const h1 *)q, (uint4 *)k_cache, (const h1 *)k_new, (uint4 *)v_cache, (const h1 *)v_new,
                                (h1 *)logits, (h1 *)weights, (h1 *)out, kp, vp, B, H, T, n_super_cap, scaling, ka, va);
-            if ((rc = check_launch()))
-                return rc;
-            for (int i = 1; i <= 3; i++)
-                if ((rc = stage_mark(i, stream)))
-                    return rc;
-            return ADKV_OK;
+            return (rc = check_launch()) ? rc : mark_one_launch(stream);
         }
     }
     {
@@ -3269,7 +3270,7 @@ int adkv_decode_step(const void *q, void *k_cache, void *v_cache, const void *k_
                                (uint2 *)k_cache, (const h1 *)k_new, (uint2 *)v_cache, (const h1 *)v_new, (const float *)mask,
                                mask ? rows_per_mask_row : 1, (h1 *)weights, (h1 *)out, kp, vp, H, T,
                                n_super_cap, scaling, ka, va);
-            return check_launch();
+            return (rc = check_launch()) ? rc : mark_one_launch(stream);
         }
     }
     rc = forward_qk_impl(q, k_cache, k_new, logits, k_params[0], k_params[1], k_params[2],

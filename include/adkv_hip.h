@@ -322,7 +322,8 @@ int adkv_decode_segments(int B, int Hq, int H, int T, int D, int bits, int n_ckp
  * timing enabled, or NULL to switch the hook off.  While set, every adkv_decode_step call of
  * THIS host thread records them on its stream: [0] before the QK launch, [1] after it, [2] after
  * the softmax, [3] after the OV launch and the sum of its segments, so the stages of the product
- * path can be timed without taking it apart.
+ * path can be timed without taking it apart.  What a call launches does not depend on the hook: a step
+ * that is one launch (adkv_decode_step_is_fused) records [0] before it and the other three after it.
  */
 void adkv_set_stage_events(void *const *events);
 

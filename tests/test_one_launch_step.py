@@ -1,0 +1,50 @@
+"""adkv_decode_step where it is one launch: what the measurement hook does to it, and what the library
+says about it."""
+import ctypes
+
+import pytest
+import torch
+
+from adkv_amd import _lib, synth
+from adkv_amd.kernel import gemv
+
+D = 128
+
+
+def _step(gpu, B, H, T, S, workspace):
+    kp, vp = (tuple(t.to(gpu) for t in synth.make_params(H, D, seed=3 + i).astuple()) for i in range(2))
+    k, v = (f(B, H, T + 1, D, seed=5, dtype=torch.float16, device=gpu) for f in (synth.make_k, synth.make_v))
+    q = synth.make_q(B, H, D, seed=6, device=gpu)
+    caches = [synth.alloc_cache(B, H, T + 8, D, gpu) for _ in range(2)]
+    cks = [torch.zeros(B, H, T // S + 1, D, 2, dtype=torch.float16, device=gpu) for _ in range(2)]
+    states = [torch.zeros(B, H, D, 2, dtype=torch.float16, device=gpu) for _ in range(2)]
+    gemv.append_kv_pair(*caches, k[:, :, :T].contiguous(), v[:, :, :T].contiguous(), kp, vp, 0, *states, k_ckpt=cks[0],
+                        v_ckpt=cks[1], ckpt_interval=S)
+    out, w = gemv.decode_step(q, *caches, k[:, :, T:].contiguous(), v[:, :, T:].contiguous(), kp, vp, T, D ** -0.5,
+                              k_ckpt=cks[0], v_ckpt=cks[1], ckpt_interval=S, workspace=workspace)
+    torch.cuda.synchronize()
+    return [out, w.contiguous(), *caches, *cks]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("B,H,T", [(1, 4, 603), (2, 3, 64), (1, 2, 1000)])
+def test_stage_events_do_not_change_what_runs(gpu, B, H, T):
+    """A one-launch step keeps its logits and weights out of the workspace, the separate launches do not:
+    with the events set the workspace stays untouched and every bit of the result is the same."""
+    S = 256
+    need = gemv.decode_step_workspace_bytes(B, H, H, T, D, T // S + 1, S)
+    ws = torch.full((need,), 0xA5, dtype=torch.uint8, device=gpu)
+    plain = _step(gpu, B, H, T, S, ws)
+    assert bool((ws == 0xA5).all())
+    events = [torch.cuda.Event(enable_timing=True) for _ in range(4)]
+    for e in events:
+        e.record()
+    _lib.lib().adkv_set_stage_events((ctypes.c_void_p * 4)(*[e.cuda_event for e in events]))
+    try:
+        timed = _step(gpu, B, H, T, S, ws)
+    finally:
+        _lib.lib().adkv_set_stage_events(None)
+    assert bool((ws == 0xA5).all())
+    for a, b in zip(plain, timed):
+        assert torch.equal(a.view(torch.uint8), b.view(torch.uint8))
+    assert events[0].elapsed_time(events[1]) > 0 and events[0].elapsed_time(events[3]) >= events[0].elapsed_time(events[1])
