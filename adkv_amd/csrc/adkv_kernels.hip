@@ -2360,9 +2360,11 @@ int adkv_decode_step_is_fused(int B, int Hq, int H, int T, int D, int bits, int 
     int dummy = 0;
     Seg ka, va;
     void *ck = n_ckpt_cap > 0 && ckpt_interval > 0 ? &dummy : nullptr;
-    if (masked || B <= 0 || H <= 0 || Hq <= 0 || T < 0)
+    if (B <= 0 || H <= 0 || Hq <= 0 || T < 0)
         return 0;
-    return fused_step_plan(ka, va, B, Hq, H, T, D, bits, ck, ck, n_ckpt_cap, ckpt_interval) ? 1 : 0;
+    if (!masked && fused_step_plan(ka, va, B, Hq, H, T, D, bits, ck, ck, n_ckpt_cap, ckpt_interval))
+        return 1;
+    return small_step_plan(ka, B, Hq, H, T, D, bits, ck, ck, n_ckpt_cap, ckpt_interval) ? 1 : 0;
 }
 
 void adkv_set_mha_kernel(int use_matrix_cores)

@@ -386,6 +386,8 @@ def decode_record(args, B, Hq, H, D, T, bits, S, NL, steps, warmup, headline=Tru
     L = _lib.lib()
     ncap_arg = ncap if S else 0
     kernel = L.adkv_decode_kernel_name(B, Hq, H, T, D, bits, ncap_arg, S).decode()
+    # few short sequences: the whole step is one launch, and what its events bracket is that launch
+    one_launch = L.adkv_decode_step_is_fused(B, Hq, H, T, D, bits, ncap_arg, S, 0) == 1
     ws = torch.empty(gemv.decode_step_workspace_bytes(B, Hq, H, T, D, ncap_arg, S), dtype=torch.uint8, device=dev)
 
     def fused(l):
@@ -467,15 +469,16 @@ def decode_record(args, B, Hq, H, D, T, bits, S, NL, steps, warmup, headline=Tru
         torch.cuda.synchronize()
         graph_ms = (time.perf_counter() - t0) * 1e3 / steps
 
+    qk_kernel, ov_kernel = ("small_step_kernel", None) if one_launch else ("qk_" + kernel, "ov_" + kernel)
     code_bytes = B * H * T * D * bits / 8.0             # one tensor's codes: bytes per QK launch
-    achieved = code_bytes / (qk_ms * 1e-3) / 1e9
+    achieved = (2 if one_launch else 1) * code_bytes / (qk_ms * 1e-3) / 1e9
     tokens_s = B / (N_LAYERS_MODEL * ms_step * 1e-3)
     workload_key = f"decode B={B} Hq={Hq} H={H} d={D} ctx={T} bits={bits} ckpt={S}"
     traffic = None
     try:
         with open(os.path.join(ROOT, "profiles", "hbm_traffic.json")) as f:
             rec = json.load(f).get(workload_key)
-        if rec and rec.get("kernel") == "qk_" + kernel.split(" ")[0].rstrip(","):
+        if rec and rec.get("kernel") == qk_kernel.split(" ")[0].rstrip(","):
             traffic = rec["bytes_per_launch"]
     except (OSError, ValueError):
         pass
@@ -505,7 +508,7 @@ def decode_record(args, B, Hq, H, D, T, bits, S, NL, steps, warmup, headline=Tru
                       "step_device_median": dev_ms, "steps_with_events": len(marks)},
         "step_code_GBps": 2 * code_bytes / (ms_step * 1e-3) / 1e9,
         "roofline": {
-            "kernel": "qk_" + kernel,
+            "kernel": qk_kernel,
             "bound": "hbm",
             "achieved": achieved,
             "peak": HBM_PEAK_GBPS,
@@ -515,11 +518,13 @@ def decode_record(args, B, Hq, H, D, T, bits, S, NL, steps, warmup, headline=Tru
             # known size; kept beside the profile it came from (profiles/hbm_traffic.json)
             "traffic": traffic,
         },
-        # the second big launch of the step, same algorithmic bytes (the V codes)
-        "roofline_ov": {"kernel": "ov_" + kernel, "bound": "hbm", "achieved": code_bytes / (ov_ms * 1e-3) / 1e9,
-                        "peak": HBM_PEAK_GBPS, "unit": "GB/s", "frac": code_bytes / (ov_ms * 1e-3) / 1e9 / HBM_PEAK_GBPS,
-                        "note": "forward_ov stage incl. the partial-sum kernel"},
     }
+    if one_launch:
+        res["kernel_ms"] = {"one_launch": qk_ms, "step_device_median": dev_ms, "steps_with_events": len(marks)}
+    else:  # the second big launch of the step, same algorithmic bytes (the V codes)
+        res["roofline_ov"] = {"kernel": ov_kernel, "bound": "hbm", "achieved": code_bytes / (ov_ms * 1e-3) / 1e9,
+                              "peak": HBM_PEAK_GBPS, "unit": "GB/s", "frac": code_bytes / (ov_ms * 1e-3) / 1e9 / HBM_PEAK_GBPS,
+                              "note": "forward_ov stage incl. the partial-sum kernel"}
     # what the memory system itself delivers for these kernels' access pattern with nothing else
     # running (a loads-only probe; result and method in profiles/hbm_pattern_ceiling.json)
     try:
@@ -545,10 +550,10 @@ def decode_record(args, B, Hq, H, D, T, bits, S, NL, steps, warmup, headline=Tru
     try:
         with open(os.path.join(ROOT, "profiles", "valu_issue.json")) as f:
             vrec = json.load(f).get(workload_key)
-        if vrec and vrec.get("kernel") == "qk_" + kernel.split(" ")[0].rstrip(","):
+        if vrec and vrec.get("kernel") == qk_kernel.split(" ")[0].rstrip(","):
             slots = vrec["valu_insts_per_launch"] * 4.0 / 1024.0          # issue cycles per SIMD
             res["roofline_valu"] = {
-                "kernel": "qk_" + kernel, "bound": "valu",
+                "kernel": qk_kernel, "bound": "valu",
                 "achieved": vrec["valu_insts_per_launch"] / (qk_ms * 1e-3) / 1e12,
                 "peak": 1024 * 2.4e9 / 4.0 / 1e12, "unit": "T wave64 instructions/s",
                 "frac": slots / (qk_ms * 1e-3 * 2.4e9),

@@ -47,11 +47,16 @@ void adkv_set_mha_kernel(int use_matrix_cores);
 /* Tuning knob, no counterpart in the reference (whose module chains the three kernels,
  * llama_adkv.py:264-274): mode > 0 lets adkv_decode_step run forward_qk, the softmax and
  * forward_ov as ONE launch wherever both stages run the per-head-table kernels on four segments
- * per sequence, there is no mask and the context is at most 8703 tokens; 0 (the default) always
- * takes three launches.  The fused launch computes what the three launches compute (the softmax
+ * per sequence, there is no mask and the context is at most 8703 tokens; 0 (the default) takes the
+ * separate launches there.  The fused launch computes what they compute (the softmax
  * sums in a different, fixed order: weights and outputs agree to an fp16 ulp; codes, state and
  * checkpoints are identical) in the same time, measured; it saves the host two launches.
- * adkv_decode_step_is_fused tells which a call with these sizes takes under the current mode. */
+ * Whatever the mode, a step of few short sequences is one launch of its own (small_step_kernel:
+ * head dim 128, 4-bit codes, as many query heads as KV heads, no more heads in the batch than the
+ * device has CUs, at most four segments and 1535 cached tokens, mask or not; not while
+ * adkv_set_mha_kernel or ADKV_MFMA picks a family).
+ * adkv_decode_step_is_fused: 1 if a call with these sizes, masked or not, is one launch of either
+ * kind under the current settings, else 0. */
 void adkv_set_fused_step(int mode);
 int adkv_decode_step_is_fused(int B, int Hq, int H, int T, int D, int bits, int n_ckpt_cap,
                               int ckpt_interval, int masked);
@@ -301,7 +306,8 @@ int adkv_decode_step(const void *q, void *k_cache, void *v_cache, const void *k_
 
 /* Which of the library's decode kernels adkv_forward_qk_gqa / adkv_forward_ov_gqa /
  * adkv_decode_step launch for these sizes ("qk_" / "ov_" + the returned text): a static string,
- * for benchmark records and tests; "invalid" for sizes the entry points reject. */
+ * for benchmark records and tests; "invalid" for sizes the entry points reject.  An adkv_decode_step
+ * that adkv_decode_step_is_fused reports runs in one launch instead of these. */
 const char *adkv_decode_kernel_name(int B, int Hq, int H, int T, int D, int bits, int n_ckpt_cap,
                                     int ckpt_interval);
 

@@ -48,3 +48,32 @@ def test_stage_events_do_not_change_what_runs(gpu, B, H, T):
     for a, b in zip(plain, timed):
         assert torch.equal(a.view(torch.uint8), b.view(torch.uint8))
     assert events[0].elapsed_time(events[1]) > 0 and events[0].elapsed_time(events[3]) >= events[0].elapsed_time(events[1])
+
+
+def test_library_says_which_steps_are_one_launch():
+    """Without a GPU: the rule of the sizes (256 CUs), masked or not, and the knobs that turn it off."""
+    L = _lib.lib()
+    fused = lambda B, Hq, H, T, S=256, D=D, bits=4, masked=0: L.adkv_decode_step_is_fused(
+        B, Hq, H, T, D, bits, T // S + 1 if S else 0, S, masked)
+    for masked in (0, 1):
+        assert fused(1, 32, 32, 603, masked=masked) == 1
+        assert fused(8, 32, 32, 1000, masked=masked) == 1
+        assert fused(1, 32, 32, 1535, 0, masked=masked) == 1
+        assert fused(1, 32, 32, 0, masked=masked) == 1
+        assert fused(9, 32, 32, 600, masked=masked) == 0          # more heads than CUs
+        assert fused(1, 32, 32, 1536, 0, masked=masked) == 0      # a row too long
+        assert fused(1, 32, 8, 600, masked=masked) == 0           # grouped queries
+        assert fused(1, 32, 32, 600, bits=2, masked=masked) == 0
+        assert fused(1, 8, 8, 600, D=256, masked=masked) == 0
+        assert fused(128, 32, 32, 4096, masked=masked) == 0       # the other kind, not asked for
+    for kernel in (0, 1, 2, 3, 4):
+        L.adkv_set_mha_kernel(kernel)
+        try:
+            assert fused(1, 32, 32, 603) == 0
+        finally:
+            L.adkv_set_mha_kernel(-1)
+    L.adkv_set_fused_step(1)
+    try:
+        assert fused(128, 32, 32, 4096) == 1 and fused(128, 32, 32, 4096, masked=1) == 0 and fused(1, 32, 32, 603) == 1
+    finally:
+        L.adkv_set_fused_step(0)
