@@ -605,7 +605,7 @@ __device__ __forceinline__ void encode_body(
         if (CPL == 1) {
             ch.zp = as_u32(st.zp);
             ch.qs_sc = as_u32((h2){(h1)0.0f, st.sc.x});
-            ch.rs = __builtin_amdgcn_rcpf((float)st.sc.x);
+            ch.s = (float)st.sc.x;
         } else {
             scf[0] = (float)st.sc.x;
             scf[1] = (float)st.sc.y;
