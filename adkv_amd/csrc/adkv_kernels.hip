@@ -449,8 +449,9 @@ __device__ __forceinline__ void init_pairs(Pair *st, const h1 *zp, const h1 *sc,
 //    low bits, clamped by one med3; v_alignbit shifts it into the code word (one instruction per
 //    code), v_cvt_f16_i16 (one channel) or a byte permute and one packed fma (two) turn it into the
 //    fp16 operand of the update.
-// Only a quotient that is not a number (a non-finite input or state, a zero scale) sends its
-// group of 8 tokens through the plain division; half an instruction per token looks for one.
+// Only a quotient that is not a number (a non-finite input or state, a zero scale) sends its run
+// of tokens (64 with one channel per lane, 32 with two) through the plain division; half an instruction
+// per token looks for one.
 constexpr int ENC_PF1 = 8;    // buffers of 8 rows in rotation, one channel per lane (one wave per SIMD: nothing else hides HBM)
 constexpr int ENC_AHEAD1 = 6; // groups loaded ahead: 56 loads and their groups' stores fit the 63 the counter holds
 constexpr int ENC_PF2 = 4; // two channels per lane (many waves)
@@ -530,7 +531,7 @@ __device__ __forceinline__ void encode_body(
         else
             return as_u32((h2){lo, (h1)__uint_as_float(w & 0xFFFF0000u)});
     };
-    // exact step with the IEEE divide: partial words and groups that failed the check
+    // exact step with the IEEE divide: partial words and runs that met a NaN
     auto step = [&](XW xw, int *qi) {
         const h2 x = as_h2((uint32_t)as_f16(xw));
         qi[0] = quantize<BITS>(x.x, st.zp.x, st.sc.x);
@@ -656,6 +657,7 @@ __device__ __forceinline__ void encode_body(
             partial_word(sg, 0, TPW);
     const int sg_end = T / TPW;
     const long span_words = (1L << 30) / (xs.t * 2 * TPW);
+    int redo = PF / G8, resumed = -1; // words done with the plain division after a NaN; where the last such stretch ended
     const int piece = (int)(span_words >= PF ? span_words / PF * PF : max(span_words, 1L)); // whole runs where it can
     while (sg < sg_end) {
         const int nw = min(piece, sg_end - sg), ng = nw * G8; // words, 8-token groups of this piece
@@ -691,9 +693,9 @@ __device__ __forceinline__ void encode_body(
                 }
             }
         };
-        // Quotients are looked at once per run of groups; a run that met a NaN is done again from
-        // its first word with the plain division.
-        auto run = [&](int words, auto &&groups) {
+        // Quotients are looked at once per run of groups.  False: one of them was a NaN, and everything
+        // but the code words is as it was before the run.
+        auto run = [&](int words, auto &&groups) -> bool {
             const Pair saved = st;
             const int saved_next = ck_next, saved_j = ck_j;
             groups();
@@ -702,22 +704,22 @@ __device__ __forceinline__ void encode_body(
                 st = saved;
                 ck_next = saved_next;
                 ck_j = saved_j;
-                for (int i = 0; i < words; i++)
-                    partial_word(sg + i, 0, TPW);
-                enter();
+                return false;
             }
             sg += words;
+            return true;
         };
         enter();
 #pragma unroll
         for (int i = 0; i < AHEAD; i++)
             load_next(xbuf[i]);
         int g = 0;
+        bool clean = true;
         // Two copies of the loop rather than a test in it: where the paths met again, the buffers
         // in flight would be copied, and waited for.
         auto runs = [&](auto inner_checkpoints) __attribute__((always_inline)) {
             for (; g + PF <= ng; g += PF) {
-                run(PF / G8, [&]() __attribute__((always_inline)) {
+                clean = run(PF / G8, [&]() __attribute__((always_inline)) {
                     static_for<PF>([&](auto ic) __attribute__((always_inline)) {
                         // loads moved up over the last use of their buffer would be copied into it
                         __builtin_amdgcn_sched_barrier(0);
@@ -726,6 +728,8 @@ __device__ __forceinline__ void encode_body(
                         do_group(ic, xbuf[decltype(ic)::value], inner_checkpoints);
                     });
                 });
+                if (!clean)
+                    return;
                 if constexpr (!decltype(inner_checkpoints)::value)
                     checkpoint(sg * TPW);
             }
@@ -736,14 +740,48 @@ __device__ __forceinline__ void encode_body(
             runs(std::integral_constant<bool, false>{});
         else
             runs(std::integral_constant<bool, true>{});
-        if (g < ng) // at most PF-1 groups, whole words; the first AHEAD of their inputs are in xbuf already
-            run((ng - g) / G8, [&]() __attribute__((always_inline)) {
+        if (clean && g < ng) // at most PF-1 groups, whole words; the first AHEAD of their inputs are in xbuf already
+            clean = run((ng - g) / G8, [&]() __attribute__((always_inline)) {
                 static_for<PF - 1 - AHEAD>([&](auto ic) __attribute__((always_inline)) { load_next(xbuf[AHEAD + decltype(ic)::value]); });
                 static_for<PF - 1>([&](auto ic) __attribute__((always_inline)) {
                     if (g + decltype(ic)::value < ng)
                         do_group(ic, xbuf[decltype(ic)::value], std::integral_constant<bool, true>{});
                 });
             });
+        if (clean)
+            continue;
+        // The run that met a NaN again with the plain division, the rows of the next group on their way
+        // during this one's steps; then the loop above starts anew behind it.  A channel whose scale is
+        // zero, or whose state is a NaN, meets one in every run: as long as no run is clean, twice as many
+        // words are taken here each time (up to 16 runs), so that such a wave hardly tries the fast form:
+        // 86 ns per token of one channel against 38 in the loop above (145 with a load per token).
+        redo = sg == resumed ? min(redo * 2, 16 * (PF / G8)) : PF / G8;
+        dst = cw + (size_t)sg * D + lane * CPL;
+        xoff = (uint32_t)lane * 2u * CPL + row * 8u * (uint32_t)g;
+        load_next(xbuf[0]);
+        for (int left = min(redo * G8, ng - g); left > 0; left--) {
+            XW x[8];
+#pragma unroll
+            for (int tt = 0; tt < 8; tt++)
+                x[tt] = xbuf[0][tt];
+            load_next(xbuf[0]);
+#pragma unroll
+            for (int tt = 0; tt < 8; tt++) {
+                int qi[CPL];
+                step(x[tt], qi);
+#pragma unroll
+                for (int c = 0; c < CPL; c++)
+                    w[c] = __builtin_amdgcn_alignbit((uint32_t)(qi[c] - Code<BITS>::QLO), w[c], BITS);
+            }
+            if (G8 == 1 || (left & 1)) { // whole words: an odd number of groups is left at a word's last
+#pragma unroll
+                for (int c = 0; c < CPL; c++)
+                    dst[c] = w[c];
+                dst += D;
+                checkpoint(++sg * TPW);
+            }
+        }
+        resumed = sg;
     }
     // ragged last word: codes of the tokens present, zero fields after them
     if (T0 < T && sg * TPW < T)
@@ -763,8 +801,9 @@ __device__ __forceinline__ void encode_body(
         store_state_n<CPL>(state_out + ((size_t)bx * D + c0) * 2, &st);
 }
 
+// five waves per SIMD with two channels per lane (many waves): 96 registers
 template <int BITS, int CPL, int BLK>
-__global__ __launch_bounds__(BLK) void encode_kernel(
+__global__ __launch_bounds__(BLK, CPL == 2 ? 5 : 1) void encode_kernel(
     uint32_t *__restrict__ cache, const h1 *__restrict__ kv_new,
     const h1 *__restrict__ zp, const h1 *__restrict__ sc, const h1 *__restrict__ al,
     const h1 *__restrict__ be, const h1 *__restrict__ tg,
@@ -788,7 +827,7 @@ struct EncTensor {
 
 // BF16: the new rows are bfloat16 (same strides, in elements) and are rounded to fp16 on the fly.
 template <int BITS, int CPL, int BLK, bool BF16>
-__global__ __launch_bounds__(BLK) void encode_pair_kernel(EncTensor k, EncTensor v, int BH, int H,
+__global__ __launch_bounds__(BLK, CPL == 2 ? 5 : 1) void encode_pair_kernel(EncTensor k, EncTensor v, int BH, int H,
                                                           int T0, int T, int D, int n_super_cap,
                                                           Seg sa)
 {
