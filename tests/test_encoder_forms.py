@@ -123,3 +123,45 @@ def test_one_bad_channel_does_not_stall_the_launch(gpu, form, T):
     bad = best()
     print(f"{form}: {clean * 1e6:.0f} us, with a bad channel {bad * 1e6:.0f} us")
     assert bad < 3 * clean
+
+
+@pytest.mark.parametrize("form", FORMS)
+@pytest.mark.parametrize("bits", (4, 2))
+def test_rounding_ties(gpu, oracle, form, bits):
+    """(x - zp) / sc = k + 1/2 exactly (ties go to even) and one fp16 step to either side, with scales that are
+    powers of two and not, in whole runs and in the tokens behind them."""
+    B, H = FORMS[form]
+    T = 75
+    g = torch.Generator().manual_seed(11 + bits)
+    sc = torch.tensor([0.25, 0.5, 1.0, 2.0, 0.75, 1.5, 3.0, 0.3330078125])[torch.randint(0, 8, (H, D), generator=g)].half()
+    k = torch.randint(-11, 11, (B, H, T, D), generator=g).float()
+    x = ((k + 0.5) * sc.float()[None, :, None, :]).half()
+    x = (x.view(torch.int16) + torch.randint(-1, 2, x.shape, generator=g).to(torch.int16)).view(torch.float16)
+    zero = torch.zeros(H, D).half()
+    _check(gpu, oracle, form, bits, x, [zero, sc, zero, zero, torch.full((H, D), 3.5 if bits == 4 else 0.5).half()], 0)
+
+
+@pytest.mark.parametrize("form,H", [("one_channel", 3), ("two_channels", 32)])
+@pytest.mark.parametrize("bits,cuts", [(4, (0, 75)), (4, (0, 37, 150)), (2, (0, 107)), (2, (0, 21, 150))])
+def test_bfloat16_pair(gpu, oracle, form, H, bits, cuts):
+    """K and V in one launch from bfloat16 projection outputs, in whole runs and resumed inside a word."""
+    B, T = (1 if form == "one_channel" else 9), cuts[-1]          # 36 864 channels per tensor, 73 728 in the launch
+    rows, params, want = [], [], []
+    for i in range(2):
+        ps = [t.clone() for t in synth.make_params(H, D, bits=bits, seed=4 + i).astuple()]
+        ps[1][H - 1, 3] = 0.0
+        x = (2.0 * torch.randn(B, T, H, D, generator=torch.Generator().manual_seed(i))).to(torch.bfloat16)
+        x[0, T // 2, 0, 9] = float("nan")
+        rows.append(x.to(gpu).transpose(1, 2))
+        params.append(tuple(t.to(gpu) for t in ps))
+        with oracle.code_bits(bits):
+            c = oracle.alloc_cache(B, H, T + 16, D)
+            st = oracle.encode_kv_f16(c, _np16(x.transpose(1, 2).to(torch.float16)), *[_np16(t) for t in ps])
+        want.append((c, st))
+    caches = [synth.alloc_cache(B, H, T + 16, D, gpu, bits=bits) for _ in range(2)]
+    states = [torch.zeros(B, H, D, 2, dtype=torch.float16, device=gpu) for _ in range(2)]
+    for a, b in zip(cuts, cuts[1:]):
+        gemv.append_kv_pair(*caches, *(r[:, :, a:b] for r in rows), *params, a, *states, bits=bits)
+    torch.cuda.synchronize()
+    for c, s, (wc, ws) in zip(caches, states, want):
+        assert np.array_equal(c.cpu().numpy(), wc) and _same16(_np16(s), ws)

@@ -793,7 +793,7 @@ def _gqa_case(gpu, oracle, B, Hkv, G, T, S, seed=0, bits=4):
 @pytest.mark.parametrize("bits,B,H,D,cuts,S", [
     (4, 2, 3, 128, (0, 5, 8, 19, 64, 100), 16),   # one channel per lane (few channels)
     (4, 1, 2, 512, (0, 3, 24), 0),
-    (4, 16, 32, 128, (0, 40), 8),                 # 65 536 channels per tensor: still one per lane
+    (4, 16, 32, 128, (0, 40), 8),                 # 65 536 channels per tensor, 131 072 in the launch: two per lane
     (4, 64, 32, 128, (0, 17), 0),                 # 262 144 channels per tensor: two per lane
     (2, 2, 2, 128, (0, 33, 34, 64, 150), 32),
 ])
@@ -1349,8 +1349,8 @@ def test_non_finite_values_in_logits_and_outputs(gpu, oracle, kernels):
 def test_encode_rounding_boundaries(gpu, oracle, bits):
     """Inputs on and next to the quantiser's rounding boundaries: (x - zp) / sc = k + 1/2 exactly
     (ties go to even), one fp16 step to either side, and scales that are not powers of two.  The
-    encoder decides most elements with a reciprocal multiply and must fall back to the exact
-    divide for these; codes have to match the oracle bit for bit."""
+    encoder's quotient is the IEEE one, from a reciprocal and one correction; codes have to match the
+    oracle bit for bit."""
     B, H, D, T = 1, 2, 128, 96
     g = torch.Generator().manual_seed(11 + bits)
     sc_choices = torch.tensor([0.25, 0.5, 1.0, 2.0, 0.75, 1.5, 3.0, 0.3330078125])
