@@ -2497,8 +2497,8 @@ static int encode_common(void *cache, const void *kv_new,
     // its instruction count, 17 against 30 with two channels), two channels beyond (they share the
     // packed updates and the wave's fixed cost).  ns per token, fp16 rows of 8192 tokens, 4-bit codes, at
     // 0.25 / 1 / 1.5 / 2 one-channel waves per SIMD: one channel 37 / 42 / 67 / 71, two - / - / 64 / 69
-    // (4.8 TB/s, what the memory gives).  Before the loop was written for its instruction count: 61 at
-    // one wave per SIMD.
+    // (4.8 TB/s; with 8 two-channel waves per SIMD 4.5 TB/s and the vector pipe 85 % busy).  Before the
+    // loop was written for its instruction count: 61 at one wave per SIMD.
     const long channels = (long)BH * D;
     const long tensors = second ? 2 : 1;
     int cpl = tensors * channels > 64L * n_simd() ? 2 : 1;

@@ -112,7 +112,7 @@ def cpu_baseline(args, T, D):
                   f"then single-query attention) = {dt:.2f} s; value = {Bs} / (32 layers x that time), "
                   f"i.e. the rate at batch {Bs}, not extrapolated",
     }
-    # secondary: the C oracle of the fp16 recurrence (bit-exact checker), one core
+    # secondary: the C oracle of the fp16 recurrence (bit-exact), one core
     hs = min(H, 8)
     np16 = lambda t: t.detach().cpu().contiguous().view(torch.int16).numpy().view(np.float16)
     kq = synth.make_params(H, D, seed=3)
