@@ -77,3 +77,11 @@ def test_library_says_which_steps_are_one_launch():
         assert fused(128, 32, 32, 4096) == 1 and fused(128, 32, 32, 4096, masked=1) == 0 and fused(1, 32, 32, 603) == 1
     finally:
         L.adkv_set_fused_step(0)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("H,T,S", [(4, 200, 64), (3, 600, 256)])
+def test_one_launch_step_replays_from_a_captured_graph(gpu, H, T, S):
+    from tests.test_gpu_parity import test_decode_step_replays_from_a_captured_graph as replays
+    assert _lib.lib().adkv_decode_step_is_fused(2, H, H, T, D, 4, (T + 8) // S + 1, S, 0) == 1
+    replays(gpu, H, H, T, S, 4)
