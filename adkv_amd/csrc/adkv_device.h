@@ -68,13 +68,13 @@ __device__ __forceinline__ void rotate_over(int n, F &&body)
 // nearest even: torch's .to(float16)) and the fp16 result is rounded to bf16 as it is written
 // (torch's .to(bfloat16)), so values are those of the reference's conversions around its kernels
 // (src/adkv/hf/llama_adkv.py:248-250, 274).  `bf16` is uniform over the launch.
-__device__ __forceinline__ h2 load_act2(const h1 *p, int bf16)
+__device__ __forceinline__ h2 act2(uint32_t w, int bf16)
 {
-    const uint32_t w = *reinterpret_cast<const uint32_t *>(p);
     if (bf16)
         return (h2){(h1)__uint_as_float(w << 16), (h1)__uint_as_float(w & 0xFFFF0000u)};
     return as_h2(w);
 }
+__device__ __forceinline__ h2 load_act2(const h1 *p, int bf16) { return act2(*reinterpret_cast<const uint32_t *>(p), bf16); }
 
 __device__ __forceinline__ uint32_t bf16_bits(h1 v)
 {

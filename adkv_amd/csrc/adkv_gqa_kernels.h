@@ -27,7 +27,6 @@ namespace adkv {
 
 
 constexpr int GQA_D = 128;
-constexpr int GQA_CPL = 4;
 // The key tile of a wave: 8 token rows of 8-byte words (a lane's two channel pairs).  The LDS
 // serves an 8-byte access of 16 lanes per clock from 32 four-byte banks, so a group of 16 lanes has
 // to touch 16 different 8-byte slots modulo 16.  Writes: lane L of a head goes to column
@@ -70,31 +69,33 @@ __device__ __forceinline__ float quarter_sum(f4v d)
 
 
 // The code words of one supergroup -> the per-pair byte streams the table is indexed with.
-template <int BITS>
-__device__ __forceinline__ void code_bytes(const uint4 &u, uint32_t (*nb)[2])
+template <int BITS, typename V>
+__device__ __forceinline__ void code_bytes(const V &u, uint32_t (*nb)[2])
 {
-    if (BITS == 4) {
-        pair_bytes(u.x, u.y, nb[0][0], nb[0][1]);
-        pair_bytes(u.z, u.w, nb[1][0], nb[1][1]);
-    } else {
-        pair_bytes2(u.x, u.y, nb[0][0], nb[0][1]);
-        pair_bytes2(u.z, u.w, nb[1][0], nb[1][1]);
+    uint32_t w[sizeof(V) / 4];
+    vec_words(u, w);
+#pragma unroll
+    for (int p = 0; p < (int)sizeof(V) / 8; p++) {
+        if (BITS == 4)
+            pair_bytes(w[2 * p], w[2 * p + 1], nb[p][0], nb[p][1]);
+        else
+            pair_bytes2(w[2 * p], w[2 * p + 1], nb[p][0], nb[p][1]);
     }
 }
 
 // Table entries of one 8-token unit held in registers, and how a token finds its (q, |q|):
 //   4-bit: slot t, 8 bytes.   2-bit: slot 2*(t/4) + (t&1), 16 bytes, second half for t&2.
-template <int BITS>
+template <int BITS, int NP>
 struct Lookups {
     static constexpr int SLOTS = BITS == 4 ? 8 : 4;
     using Entry = typename std::conditional<BITS == 4, uint2, uint4>::type;
-    Entry e[2][SLOTS];
+    Entry e[NP][SLOTS];
 
     // all lookups of unit `half` (0 or 1 within the supergroup) of the words `nb`
     __device__ __forceinline__ void fill(const uint2 *lut, const uint32_t (*nb)[2], uint32_t lane_copy, int half)
     {
 #pragma unroll
-        for (int p = 0; p < 2; p++) {
+        for (int p = 0; p < NP; p++) {
             if constexpr (BITS == 4) {
 #pragma unroll
                 for (int t = 0; t < 8; t++)
@@ -123,12 +124,12 @@ struct Lookups {
     {
         if constexpr (BITS == 4) {
 #pragma unroll
-            for (int p = 0; p < 2; p++)
+            for (int p = 0; p < NP; p++)
                 e[p][t] = lut_get(lut, nb[p][t & 1], lane_copy, t >> 1);
         } else {
             if (t & 2) {
 #pragma unroll
-                for (int p = 0; p < 2; p++)
+                for (int p = 0; p < NP; p++)
                     e[p][2 * (t >> 2) + (t & 1)] = lut2_get(lut, nb[p][t & 1], lane_copy, 2 * next_half + (t >> 2));
             }
         }
@@ -150,18 +151,76 @@ __device__ __forceinline__ uint32_t table_lane_offset(int lane)
     return BITS == 4 ? (uint32_t)(lane & (LUT_COPIES - 1)) * 8u : (uint32_t)(lane & (LUT2_COPIES - 1)) * 16u;
 }
 
+// forward_qk of one segment, two channels per lane: a KV head fills the wave (see PairScores).
+template <int BITS, int GQ, int BLK>
+__device__ __forceinline__ void qk_gqa_pair(
+    uint2 *smem, const h1 *q, uint4 *__restrict__ cache, const h1 *k_new, h1 *__restrict__ out,
+    const h1 *zp, const h1 *sc, const h1 *al, const h1 *be,
+    const h1 *tg, int BH, int H, int T, int n_super_cap, h1 *__restrict__ state_out, Seg sa)
+{
+    sa.groups = 0; // only even plans come here
+    constexpr int D = GQA_D, CPL = 2, TPW = Code<BITS>::TPW;
+    using G = Geo<D, CPL>;
+    const Unit<D, CPL, BLK> un(BH, sa.nseg);
+    const int bx = un.bx, lane = un.lh, c0 = un.c0;
+    PairScores<BITS, GQ> scores(reinterpret_cast<char *>(smem + LUT_WORDS64) + (threadIdx.x >> 6) * PAIR_TILE, lane,
+                                q + (size_t)bx * GQ * D);
+    SegLoads<D, CPL, BITS, PairScores<BITS, GQ>::AHEAD> s;
+    s.start(cache, zp, sc, al, be, tg, bx % H, bx, lane, un.seg, T, n_super_cap, sa);
+    fill_table<BITS, BLK>(smem, threadIdx.x);
+    __syncthreads();
+    if (!un.wave_active)
+        return; // padding waves
+    Pair st[1];
+    s.state(st);
+    scores.ready(sa.act_bf16);
+    const bool last = s.last;
+    const int t0 = s.t0, t1 = s.t1, nfull = s.nfull;
+    uint2 *cbh = s.cbh;
+    const uint2 *cb = s.cb;
+    h1 *ob = out + (size_t)bx * GQ * sa.row_pitch + t0;
+    auto put = [&](int t, int g, h1 v) __attribute__((always_inline)) { ob[(size_t)g * sa.row_pitch + t] = v; };
+    scores.run(smem, table_lane_offset<BITS>(lane), st[0], s, put);
+    if (!last)
+        return;
+    // ragged tail and the appended token: at most a tile
+    const int ntail = (t1 - t0) % TPW;
+    if (ntail) {
+        const uint2 w = cb[(size_t)nfull * G::VPS];
+        for (int tt = 0; tt < ntail; tt++) {
+            const h2 qc = extract_pair<BITS>(w.x, w.y, tt);
+            const h2 qs = qc * st[0].sc;
+            scores.write(tt, as_u32(qs + st[0].zp));
+            update_pair(st[0], qc, qs);
+        }
+    }
+    publish_state<D, CPL>(st, state_out, sa, bx, c0, T);
+    h2 deq[1];
+    append_new_token<D, CPL, BITS>(cbh, T, k_new + (size_t)bx * D + c0, st, deq, true, sa.act_bf16);
+    scores.write(ntail, as_u32(deq[0]));
+    scores.fetch();
+    scores.multiply();
+    scores.emit(nfull * TPW, ntail + 1, put);
+}
+
 // ---------------------------------------------------------------------------------------------
 // forward_qk with GQ query heads per KV head
 // ---------------------------------------------------------------------------------------------
-template <int BITS, int GQ, int BLK>
+template <int BITS, int GQ, int BLK, int CPL>
 __global__ __launch_bounds__(BLK) void qk_gqa_kernel(
-    const h1 *__restrict__ q, uint4 *__restrict__ cache, const h1 *__restrict__ k_new,
+    const h1 *q, uint4 *__restrict__ cache, const h1 *k_new,
     h1 *__restrict__ out,
-    const h1 *__restrict__ zp, const h1 *__restrict__ sc, const h1 *__restrict__ al,
-    const h1 *__restrict__ be, const h1 *__restrict__ tg,
+    const h1 *zp, const h1 *sc, const h1 *al,
+    const h1 *be, const h1 *tg,
     int BH, int H, int T, int n_super_cap, h1 *__restrict__ state_out, Seg sa)
 {
-    constexpr int D = GQA_D, CPL = GQA_CPL;
+    if constexpr (CPL == 2) {
+        __shared__ uint2 smem[LUT_WORDS64 + (BLK / 64) * PAIR_TILE / 8];
+        qk_gqa_pair<BITS, GQ, BLK>(smem, q, cache, k_new, out, zp, sc, al, be, tg, BH, H, T,
+                                   n_super_cap, state_out, sa);
+        return;
+    } else {
+    constexpr int D = GQA_D;
     constexpr int NB = (GQ + 3) / 4; // column sets of four heads
     constexpr int TPW = Code<BITS>::TPW, UPS = TPW / 8;
     // supergroups in flight per lane: fewer where a supergroup is 16 tokens or registers are short
@@ -169,23 +228,23 @@ __global__ __launch_bounds__(BLK) void qk_gqa_kernel(
     using G = Geo<D, CPL>;
     __shared__ uint2 smem[LUT_WORDS64 + (BLK / 64) * TILE_WORDS64];
     const uint2 *lut = smem;
-    fill_table<BITS, BLK>(smem, threadIdx.x);
-    __syncthreads();
-
     const int lane = threadIdx.x & 63;
     const uint32_t lane_copy = table_lane_offset<BITS>(lane);
     uint2 *tile = smem + LUT_WORDS64 + (threadIdx.x >> 6) * TILE_WORDS64;
 
-    const Unit<D, CPL, BLK> un(BH, sa.nseg);
-    if (!un.wave_active)
-        return; // padding waves
+    const Unit<D, CPL, BLK> un(BH, sa.nseg); // a padding wave's is valid too: it loads and leaves
     const int bx = un.bx, lh = un.lh, c0 = un.c0;
     const bool active = un.active;
-    const bool last = seg_is_last(sa, un.seg);
-    const int h = bx % H;
+    SegLoads<D, CPL, BITS, GPF> s;
+    s.start(cache, zp, sc, al, be, tg, bx % H, bx, lh, un.seg, T, n_super_cap, sa);
+    fill_table<BITS, BLK>(smem, threadIdx.x);
+    __syncthreads();
+    if (!un.wave_active)
+        return; // padding waves
+    const bool last = s.last;
 
     Pair st[G::NP];
-    init_pairs<D, CPL>(st, zp, sc, al, be, tg, h, bx, c0, un.seg, sa);
+    s.state(st);
 
     // matrix-core roles of this lane: block (hh, tg4, qd), row/column r
     const int r = lane & 3, qd = (lane >> 2) & 3, tg4 = (lane >> 4) & 1;
@@ -205,11 +264,10 @@ __global__ __launch_bounds__(BLK) void qk_gqa_kernel(
     const uint2 *arow = tile + (tg4 * 4 + r) * TILE_ROW64 + (lane >> 5) * TILE_HEAD64 + tile_col(qd * 8);
     const int wcol = (lane >> 5) * TILE_HEAD64 + tile_col(lane & 31); // where this lane's values go in a row
 
-    const int t0 = seg_begin(sa, un.seg);
-    const int t1 = last ? T : seg_end(sa, un.seg);
-    uint4 *cbh = cache + (size_t)bx * n_super_cap * G::VPS + lh * G::NV;
-    const uint4 *cb = cbh + (size_t)(t0 / TPW) * G::VPS;
-    const int nfull = (t1 - t0) / TPW;
+    const int t0 = s.t0, t1 = s.t1, nfull = s.nfull;
+    uint4 *cbh = s.cbh;
+    const uint4 *cb = s.cb;
+    auto &buf = s.buf;
 
     // logits of the tile's tokens: read the A operands, run the instructions, add the quarters,
     // lane (.., qd, r) stores token tg4*4+qd of head r.  `unit` counts 8-token units from t0.
@@ -233,7 +291,7 @@ __global__ __launch_bounds__(BLK) void qk_gqa_kernel(
         }
     };
 
-    Lookups<BITS> lk;
+    Lookups<BITS, G::NP> lk;
     // token t of the current unit; then the lookups that reuse its slot for the unit after it
     auto token = [&](int t, const uint32_t (*nbnext)[2], int next_half) {
         uint32_t kh[G::NP];
@@ -251,24 +309,20 @@ __global__ __launch_bounds__(BLK) void qk_gqa_kernel(
         __builtin_amdgcn_sched_barrier(0);
     };
 
-    uint4 buf[GPF];
     uint32_t nbc[G::NP][2], nbn[G::NP][2]; // byte streams of the current / the next supergroup
     uint2 areg[8] = {}; // read (and discarded) once before the first unit has filled it
-#pragma unroll
-    for (int i = 0; i < GPF; i++)
-        buf[i] = (i < nfull) ? load_codes(cb + (size_t)i * G::VPS) : make_uint4(0, 0, 0, 0);
     if (nfull > 0) {
-        code_bytes<BITS>(buf[0], nbc);
+        code_bytes<BITS>(buf[0][0], nbc);
         lk.fill(lut, nbc, lane_copy, 0);
     }
     // one supergroup, nothing conditional in it; i = its buffer in the rotation
     auto body = [&](int sg, auto ic) {
         constexpr int i = decltype(ic)::value;
         // bytes of supergroup sg+1 (stale data past the end: looked up, never used)
-        code_bytes<BITS>(buf[(i + 1) % GPF], nbn);
+        code_bytes<BITS>(buf[(i + 1) % GPF][0], nbn);
         // unconditional, clamped to the segment's last supergroup: a load inside a branch makes
         // the next wait cover every load in flight, this one included
-        buf[i] = load_codes(cb + (size_t)min(sg + GPF, nfull - 1) * G::VPS);
+        buf[i][0] = load_codes(cb + (size_t)min(sg + GPF, nfull - 1) * G::VPS);
         __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
         for (int hf = 0; hf < UPS; hf++) {
@@ -330,20 +384,23 @@ __global__ __launch_bounds__(BLK) void qk_gqa_kernel(
     tile[row * TILE_ROW64 + wcol] = make_uint2(as_u32(deq[0]), as_u32(deq[1]));
     emit_read(areg);
     emit_finish(areg, unit, row + 1);
+    }
 }
 
 // ---------------------------------------------------------------------------------------------
 // forward_ov with GQ query heads per KV head
 // ---------------------------------------------------------------------------------------------
-template <int BITS, int GQ, int BLK>
+template <int BITS, int GQ, int BLK, int CPL>
 __global__ __launch_bounds__(BLK) void ov_gqa_kernel(
-    const h1 *__restrict__ attn, uint4 *__restrict__ cache, const h1 *__restrict__ v_new,
+    const h1 *attn, uint4 *__restrict__ cache, const h1 *v_new,
     h1 *__restrict__ out, float *__restrict__ partial,
-    const h1 *__restrict__ zp, const h1 *__restrict__ sc, const h1 *__restrict__ al,
-    const h1 *__restrict__ be, const h1 *__restrict__ tg,
+    const h1 *zp, const h1 *sc, const h1 *al,
+    const h1 *be, const h1 *tg,
     int BH, int H, int T, int n_super_cap, h1 *__restrict__ state_out, Seg sa)
 {
-    constexpr int D = GQA_D, CPL = GQA_CPL;
+    constexpr int D = GQA_D;
+    if (CPL == 2)
+        sa.groups = 0; // only even plans come here
     constexpr int NB = (GQ + 3) / 4;
     constexpr int TPW = Code<BITS>::TPW, UPS = TPW / 8;
     constexpr int GPF = (BITS == 2 || NB > 1) ? 2 : PF;    // supergroups in flight per lane
@@ -351,48 +408,53 @@ __global__ __launch_bounds__(BLK) void ov_gqa_kernel(
     static_assert((GPF * UPS) % WPF == 0, "weight ring must line up with the unrolled loop");
     using G = Geo<D, CPL>;
     __shared__ uint2 lut[LUT_WORDS64];
-    fill_table<BITS, BLK>(lut, threadIdx.x);
-    __syncthreads();
     const int lane = threadIdx.x & 63;
     const uint32_t lane_copy = table_lane_offset<BITS>(lane);
 
     const Unit<D, CPL, BLK> un(BH, sa.nseg);
-    if (!un.wave_active)
-        return; // padding waves
     const int bx = un.bx, lh = un.lh, c0 = un.c0;
     const bool active = un.active;
-    const bool last = seg_is_last(sa, un.seg);
-    const int h = bx % H;
     const int r = lane & 3;
+    using Vec = typename G::Vec;
+    SegLoads<D, CPL, BITS, GPF> s;
+    s.start(cache, zp, sc, al, be, tg, bx % H, bx, lh, un.seg, T, n_super_cap, sa);
+    const bool last = s.last;
+    const int t0 = s.t0, t1 = s.t1, nfull = s.nfull;
+    Vec *cbh = s.cbh;
+    const Vec *cb = s.cb;
+    auto &buf = s.buf;
+    const int nunits = nfull * UPS;
+    // A operand rows: the weights of head r (+4 per column set) of this lane's KV head; lanes of no head
+    // repeat one, into rows of the product that nobody reads
+    const h1 *wb[NB];
+#pragma unroll
+    for (int n = 0; n < NB; n++)
+        wb[n] = attn + ((size_t)bx * GQ + min(4 * n + r, GQ - 1)) * sa.row_pitch + t0;
+    auto load_w = [&](int n, int unit) {
+        uint4 v;
+        __builtin_memcpy(&v, wb[n] + (size_t)unit * 8, 16); // rows are only 2-byte aligned
+        return v;
+    };
+    uint4 wbuf[WPF][NB];
+    if (nunits > 0)
+#pragma unroll
+        for (int i = 0; i < WPF; i++)
+#pragma unroll
+            for (int n = 0; n < NB; n++)
+                wbuf[i][n] = load_w(n, min(i, nunits - 1));
+    fill_table<BITS, BLK>(lut, threadIdx.x);
+    __syncthreads();
+    if (!un.wave_active)
+        return; // padding waves
 
     Pair st[G::NP];
-    init_pairs<D, CPL>(st, zp, sc, al, be, tg, h, bx, c0, un.seg, sa);
+    s.state(st);
     f4v acc[NB][CPL]; // [column set][channel of this lane], element i = head 4n+i
 #pragma unroll
     for (int n = 0; n < NB; n++)
 #pragma unroll
         for (int c = 0; c < CPL; c++)
             acc[n][c] = (f4v){0.0f, 0.0f, 0.0f, 0.0f};
-
-    const int t0 = seg_begin(sa, un.seg);
-    const int t1 = last ? T : seg_end(sa, un.seg);
-    uint4 *cbh = cache + (size_t)bx * n_super_cap * G::VPS + lh * G::NV;
-    const uint4 *cb = cbh + (size_t)(t0 / TPW) * G::VPS;
-    const int nfull = (t1 - t0) / TPW;
-    const int nunits = nfull * UPS;
-    // A operand rows: the weights of head r (+4 per column set) of this lane's KV head
-    const h1 *wb[NB];
-    bool wok[NB];
-#pragma unroll
-    for (int n = 0; n < NB; n++) {
-        wok[n] = 4 * n + r < GQ;
-        wb[n] = attn + ((size_t)bx * GQ + (wok[n] ? 4 * n + r : 0)) * sa.row_pitch + t0;
-    }
-    auto load_w = [&](int n, int unit) {
-        uint4 v;
-        __builtin_memcpy(&v, wb[n] + (size_t)unit * 8, 16); // rows are only 2-byte aligned
-        return wok[n] ? v : make_uint4(0u, 0u, 0u, 0u);
-    };
 
     // four tokens of dequantised values, token-major pairs -> per-channel h4 -> four instructions
     auto contract = [&](const uint32_t (*kh)[4], const uint4 *wv, int half) {
@@ -413,7 +475,7 @@ __global__ __launch_bounds__(BLK) void ov_gqa_kernel(
         }
     };
     uint32_t kh[G::NP][4];
-    Lookups<BITS> lk;
+    Lookups<BITS, G::NP> lk;
     auto token = [&](int t, const uint32_t (*nbnext)[2], int next_half) {
 #pragma unroll
         for (int p = 0; p < G::NP; p++) {
@@ -428,26 +490,16 @@ __global__ __launch_bounds__(BLK) void ov_gqa_kernel(
         __builtin_amdgcn_sched_barrier(0);
     };
 
-    uint4 buf[GPF];
-    uint4 wbuf[WPF][NB];
     uint32_t nbc[G::NP][2], nbn[G::NP][2];
-#pragma unroll
-    for (int i = 0; i < GPF; i++)
-        buf[i] = (i < nfull) ? load_codes(cb + (size_t)i * G::VPS) : make_uint4(0, 0, 0, 0);
-#pragma unroll
-    for (int i = 0; i < WPF; i++)
-#pragma unroll
-        for (int n = 0; n < NB; n++)
-            wbuf[i][n] = (i < nunits) ? load_w(n, i) : make_uint4(0, 0, 0, 0);
     if (nfull > 0) {
-        code_bytes<BITS>(buf[0], nbc);
+        code_bytes<BITS>(buf[0][0], nbc);
         lk.fill(lut, nbc, lane_copy, 0);
     }
     // one supergroup, nothing conditional in it; i = its buffer in the rotation
     auto body = [&](int sg, auto ic) {
         constexpr int i = decltype(ic)::value;
-        code_bytes<BITS>(buf[(i + 1) % GPF], nbn);
-        buf[i] = load_codes(cb + (size_t)min(sg + GPF, nfull - 1) * G::VPS); // unconditional: see qk_gqa_kernel
+        code_bytes<BITS>(buf[(i + 1) % GPF][0], nbn);
+        buf[i][0] = load_codes(cb + (size_t)min(sg + GPF, nfull - 1) * G::VPS); // unconditional: see qk_gqa_kernel
 #pragma unroll
         for (int hf = 0; hf < UPS; hf++) {
             const int unit = sg * UPS + hf;
@@ -492,12 +544,12 @@ __global__ __launch_bounds__(BLK) void ov_gqa_kernel(
         };
         const int ntail = (t1 - t0) % TPW;
         if (ntail) {
-            const uint4 u = cb[(size_t)nfull * G::VPS];
-            const uint32_t w[4] = {u.x, u.y, u.z, u.w};
+            uint32_t w[CPL];
+            vec_words(cb[(size_t)nfull * G::VPS], w);
             for (int tt = 0; tt < ntail; tt++) {
-                h2 vd[2];
+                h2 vd[G::NP];
 #pragma unroll
-                for (int pp = 0; pp < 2; pp++) {
+                for (int pp = 0; pp < G::NP; pp++) {
                     Pair &s = st[pp];
                     const h2 qc = extract_pair<BITS>(w[2 * pp], w[2 * pp + 1], tt);
                     const h2 qs = qc * s.sc;
@@ -518,14 +570,19 @@ __global__ __launch_bounds__(BLK) void ov_gqa_kernel(
 #pragma unroll
     for (int g = 0; g < GQ; g++) {
         const size_t row = (size_t)bx * GQ + g;
-        const float o0 = acc[g >> 2][0][g & 3], o1 = acc[g >> 2][1][g & 3];
-        const float o2 = acc[g >> 2][2][g & 3], o3 = acc[g >> 2][3][g & 3];
-        if (sa.nseg == 1) {
-            store_act2(out + row * D + c0, o0, o1, sa.act_bf16);
-            store_act2(out + row * D + c0 + 2, o2, o3, sa.act_bf16);
-        } else {
-            *reinterpret_cast<float4 *>(partial + ((size_t)un.seg * BH * GQ + row) * D + c0) =
-                make_float4(o0, o1, o2, o3);
+        float o[CPL];
+#pragma unroll
+        for (int c = 0; c < CPL; c++)
+            o[c] = acc[g >> 2][c][g & 3];
+#pragma unroll
+        for (int c = 0; c < CPL; c += 2) {
+            if (sa.nseg == 1)
+                store_act2(out + row * D + c0 + c, o[c], o[c + 1], sa.act_bf16);
+            else if (CPL == 2)
+                *reinterpret_cast<float2 *>(partial + ((size_t)un.seg * BH * GQ + row) * D + c0) = make_float2(o[0], o[1]);
+            else if (c == 0)
+                *reinterpret_cast<float4 *>(partial + ((size_t)un.seg * BH * GQ + row) * D + c0) =
+                    make_float4(o[0], o[1], o[CPL - 2], o[CPL - 1]);
         }
     }
 }

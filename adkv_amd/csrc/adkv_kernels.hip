@@ -87,6 +87,7 @@ struct Seg {
     int n_ckpt_cap;
     int ckpt_interval;  // 0 when ckpt is null
     int seg_tokens;     // >= T when there is one segment
+    int seg_intervals;  // checkpoint intervals of an even segment (0 when there is one segment)
     int nseg;
     long row_pitch;     // elements between rows of the logits / attention-weight matrix (>= T + 1)
     int act_bf16;       // q, the new token and the output are bfloat16 (see load_act2 / store_act2)
@@ -153,6 +154,11 @@ __host__ __device__ inline int segment_of_slot(const Seg &sa, int seg) { return 
 __host__ __device__ inline int seg_begin(const Seg &sa, int seg)
 {
     return sa.groups ? uneven_cut(seg ^ 3, sa.groups, sa.intervals, sa.skew) * sa.ckpt_interval : seg * sa.seg_tokens;
+}
+// the same in checkpoint intervals (0 when there is one segment)
+__host__ __device__ inline int seg_first_interval(const Seg &sa, int seg)
+{
+    return sa.groups ? uneven_cut(seg ^ 3, sa.groups, sa.intervals, sa.skew) : seg * sa.seg_intervals;
 }
 __host__ __device__ inline int seg_end(const Seg &sa, int seg)
 {
@@ -412,20 +418,68 @@ struct Unit {
     }
 };
 
-// Parameters plus the state this segment starts from.
-template <int D, int CPL>
-__device__ __forceinline__ void init_pairs(Pair *st, const h1 *zp, const h1 *sc, const h1 *al,
-                                           const h1 *be, const h1 *tg, int h, int bx, int c0, int seg,
-                                           const Seg &sa)
-{
+// What a unit reads before it can decode: parameters, the state its segment starts from, the first
+// supergroups of codes.  start() issues the loads and waits for none of them, so they travel while
+// the workgroup writes its table; state() is for after it.  One after the other behind the table (parameters, the
+// checkpoint, then codes) these trips to memory took 5 of the 28 us of a segment of 256 tokens at
+// four waves per SIMD.  (Kernels take what is read here without __restrict__: the compiler moves loads
+// of memory that it knows to be constant past the barrier to their first use.)
+template <int D, int CPL, int BITS, int AHEAD>
+struct SegLoads {
+    using G = Geo<D, CPL>;
+    using Vec = typename G::Vec;
+    static constexpr int TPW = Code<BITS>::TPW;
+    Vec *cbh;       // this head, this lane
+    const Vec *cb;  // this segment
+    int t0, t1, nfull; // tokens [t0, t1), whole supergroups
+    bool last;
+    bool from_ckpt;
+    uint32_t zp[CPL / 2], sc[CPL / 2], al[CPL / 2], be[CPL / 2], tg[CPL / 2], ck[CPL];
+    Vec buf[AHEAD][G::NV];
+
+    __device__ __forceinline__ void start(uint4 *cache, const h1 *zp_, const h1 *sc_, const h1 *al_, const h1 *be_, const h1 *tg_,
+                                          int h, int bx, int lh, int seg, int T, int n_super_cap, const Seg &sa)
+    {
+        const int c0 = lh * CPL, pi = h * D + c0;
+        const int iv = seg_first_interval(sa, seg);
+        last = seg_is_last(sa, seg);
+        t0 = iv * sa.ckpt_interval;
+        t1 = last ? T : seg_end(sa, seg);
+        nfull = (t1 - t0) / TPW;
+        cbh = reinterpret_cast<Vec *>(cache) + (size_t)bx * n_super_cap * G::VPS + lh * G::NV;
+        cb = cbh + (size_t)(t0 / TPW) * G::VPS;
+        from_ckpt = iv > 0;
+        if (from_ckpt)
+            __builtin_memcpy(ck, sa.ckpt + (((size_t)bx * sa.n_ckpt_cap + iv - 1) * D + c0) * 2, 4 * CPL);
+        // parameters and checkpoints are 4-byte aligned at least
+        __builtin_memcpy(zp, zp_ + pi, 2 * CPL);
+        __builtin_memcpy(sc, sc_ + pi, 2 * CPL);
+        __builtin_memcpy(al, al_ + pi, 2 * CPL);
+        __builtin_memcpy(be, be_ + pi, 2 * CPL);
+        __builtin_memcpy(tg, tg_ + pi, 2 * CPL);
+        // unconditional (a segment without a whole supergroup reads its partial one): with a condition
+        // the waits inside the loop have to cover what this entry leaves open
 #pragma unroll
-    for (int p = 0; p < CPL / 2; p++)
-        load_pair(st[p], zp, sc, al, be, tg, h * D + c0 + 2 * p);
-    if (seg_begin(sa, seg) > 0) {
-        const int j = seg_begin(sa, seg) / sa.ckpt_interval - 1;
-        load_state<CPL>(sa.ckpt + (((size_t)bx * sa.n_ckpt_cap + j) * D + c0) * 2, st);
+        for (int i = 0; i < AHEAD; i++) {
+#pragma unroll
+            for (int v = 0; v < G::NV; v++)
+                buf[i][v] = load_codes(cb + (size_t)min(i, max(nfull - 1, 0)) * G::VPS + v);
+        }
     }
-}
+    __device__ __forceinline__ void state(Pair *st) const
+    {
+#pragma unroll
+        for (int p = 0; p < CPL / 2; p++) {
+            const h2 a = as_h2(ck[2 * p]), b = as_h2(ck[2 * p + 1]);
+            st[p].zp = from_ckpt ? (h2){a.x, b.x} : as_h2(zp[p]);
+            st[p].sc = from_ckpt ? (h2){a.y, b.y} : as_h2(sc[p]);
+            st[p].al = as_h2(al[p]);
+            st[p].be = as_h2(be[p]);
+            // omt = 1 - beta*target with both steps rounded to fp16 (gemv.cu:220-221)
+            st[p].omt = splat((h1)1.0f) - st[p].be * as_h2(tg[p]);
+        }
+    }
+};
 
 // ---------------------------------------------------------------------------------------------
 // encode_kv  (gemv.cu:168-308)
@@ -904,116 +958,176 @@ __device__ __forceinline__ void pair_bytes_of(const typename Geo<D, CPL>::Vec *u
 typedef _Float16 h8v __attribute__((ext_vector_type(8))); // operand of v_mfma_f32_16x16x32_f16
 constexpr int PAIR_TILE = 16 * 256; // bytes of a wave's key tile
 
-// forward_qk of a segment with the head over a whole wave, two channels per lane.
+// forward_qk of a segment with the head over a whole wave, two channels per lane, for GQ query heads.
 // A wave has its SIMD (nearly) to itself and pays for every instruction, so what is left per
 // token is the lookup, the replay (replay_eight) and half a write: the values of 16 tokens go
-// to an LDS tile, from which the matrix cores take them as columns against the query as every
-// row.  All rows of the product are equal, so lane t (modulo 16) receives token t's logit
-// whichever row it holds, and nothing is summed across lanes.  ~10 issue slots per token
+// to an LDS tile, from which the matrix cores take them as columns against the queries as
+// rows.  Row r is head r * GQ / 16, so that lane (token, quarter of the rows) receives its head's
+// logit of its token as it is, and nothing is summed across lanes.  ~10 issue slots per token
 // where the dot product, its reduction over the lanes and the wait states made it 19
 // (32 x 32 heads x 1024 tokens, one segment: 49 -> 34 us; ov_kernel with replay_eight_weighted
 // 38 -> 32).
 // The tile: row t = token t, 256 bytes; its 16-byte pieces are permuted by (t / 2) % 8 so that
 // both halves of an access to 16 rows at once spread over the banks.
-// put(token, logit) is called for token 0.. of the segment, one lane per token.
-template <typename PUT>
-__device__ __forceinline__ void pair_scores(const uint2 *lut, char *tile, int lane, uint32_t lane_copy, Pair &st,
-                                            const h1 *qrow, int act_bf16, const uint2 *cb, int nfull, PUT &&put)
-{
+template <int BITS, int GQ>
+struct PairScores {
     using G = Geo<128, 2>;
     using Vec = G::Vec;
-    constexpr int D = 128, CPL = 2;
-    const int row = lane & 15, kb = lane >> 4;
-    h8v qa[4];
-    int rd[4], wr[8];
-#pragma unroll
-    for (int m = 0; m < 4; m++) {
-        const h1 *src = qrow + m * 32 + kb * 8;
-        const h2 a = load_act2(src, act_bf16), b = load_act2(src + 2, act_bf16);
-        const h2 c = load_act2(src + 4, act_bf16), d = load_act2(src + 6, act_bf16);
-        qa[m] = (h8v){a.x, a.y, b.x, b.y, c.x, c.y, d.x, d.y};
-        rd[m] = row * 256 + (((m * 4 + kb) ^ (row >> 1)) << 4);
-    }
-#pragma unroll
-    for (int j = 0; j < 8; j++)
-        wr[j] = (lane * 4) ^ (j << 4);
-    auto lookup = [&](uint2 *e, const Vec *u) __attribute__((always_inline)) {
-        uint32_t nb[1][2];
-        pair_bytes_of<D, CPL>(u, nb);
-#pragma unroll
-        for (int t = 0; t < 8; t++)
-            e[t] = lut_get(lut, nb[0][t & 1], lane_copy, t >> 1);
-    };
-    h8v kv[4] = {};
+    static constexpr int TPW = Code<BITS>::TPW, UPS = TPW / 8; // tokens, units of eight tokens per supergroup
+    static constexpr int AHEAD = PF_PAIR / UPS;                // supergroups in flight
+    char *tile;
+    int lane;
+    h8v qa[4], kv[4];
     f4v d;
-    auto fetch = [&]() __attribute__((always_inline)) {
+    int rd[4], wr[8];
+
+    // loads the queries (rows are 8-byte aligned); ready() once the rest of the workgroup's loads are out
+    __device__ __forceinline__ PairScores(char *tile_, int lane_, const h1 *q) : tile(tile_), lane(lane_)
+    {
+        const int row = lane & 15, kb = lane >> 4;
+#pragma unroll
+        for (int m = 0; m < 4; m++) {
+            const uint2 *src = reinterpret_cast<const uint2 *>(q + (row * GQ >> 4) * 128 + m * 32 + kb * 8);
+            const uint2 a = src[0], b = src[1];
+            qa[m] = __builtin_bit_cast(h8v, make_uint4(a.x, a.y, b.x, b.y));
+        }
+    }
+    __device__ __forceinline__ void ready(int act_bf16)
+    {
+        const int row = lane & 15, kb = lane >> 4;
+#pragma unroll
+        for (int m = 0; m < 4; m++) {
+            if (act_bf16) {
+                const uint4 u = __builtin_bit_cast(uint4, qa[m]);
+                qa[m] = __builtin_bit_cast(h8v, make_uint4(as_u32(act2(u.x, 1)), as_u32(act2(u.y, 1)),
+                                                           as_u32(act2(u.z, 1)), as_u32(act2(u.w, 1))));
+            }
+            kv[m] = (h8v){};
+            rd[m] = row * 256 + (((m * 4 + kb) ^ (row >> 1)) << 4);
+        }
+#pragma unroll
+        for (int j = 0; j < 8; j++)
+            wr[j] = (lane * 4) ^ (j << 4);
+    }
+    // this lane's channel pair of the token in `row` of the tile
+    __device__ __forceinline__ void write(int row, uint32_t x)
+    {
+        *reinterpret_cast<uint32_t *>(tile + row * 256 + ((lane * 4) ^ (row >> 1 << 4))) = x;
+    }
+    __device__ __forceinline__ void fetch()
+    {
 #pragma unroll
         for (int m = 0; m < 4; m++)
             kv[m] = *reinterpret_cast<const h8v *>(tile + rd[m]);
-    };
-    auto multiply = [&]() __attribute__((always_inline)) {
+    }
+    __device__ __forceinline__ void multiply()
+    {
         d = (f4v){0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
         for (int m = 0; m < 4; m++)
             d = __builtin_amdgcn_mfma_f32_16x16x32_f16(qa[m], kv[m], d, 0, 0, 0);
-    };
-    auto emit = [&](int sg, int ntok) __attribute__((always_inline)) { // sg: first supergroup of the tile
-        if (lane < ntok)
-            put(sg * 8 + lane, (h1)d.x);
-    };
-    if (nfull > 0) {
-        Vec buf[PF_PAIR][G::NV];
-        uint2 e[2][8];
-        // unconditional loads, here and in the loop, and no scalar load in flight when it starts:
-        // otherwise the waits inside it have to cover what this entry leaves open
-#pragma unroll
-        for (int i = 0; i < PF_PAIR; i++) {
-            buf[i][0] = load_codes(cb + (size_t)min(i, nfull - 1) * G::VPS);
-            __builtin_amdgcn_sched_barrier(0);
-        }
-        lookup(e[0], buf[0]);
-        wait_lgkm();
-        rotate_over<PF_PAIR>(nfull, [&](int sg, auto ic) __attribute__((always_inline)) {
-            constexpr int i = decltype(ic)::value, half = i & 1;
-            lookup(e[half ^ 1], buf[(i + 1) % PF_PAIR]); // stale past the end: looked up, never used
-            buf[i][0] = load_codes(cb + (size_t)min(sg + PF_PAIR, nfull - 1) * G::VPS);
-            __builtin_amdgcn_sched_barrier(0);
-            uint32_t kh[8];
-            replay_eight(st, e[half], kh);
-#pragma unroll
-            for (int t = 0; t < 8; t++)
-                *reinterpret_cast<uint32_t *>(tile + (half * 8 + t) * 256 + wr[half * 4 + t / 2]) = kh[t];
-            __builtin_amdgcn_sched_barrier(0);
-            // the tile before this one: fetched when it was complete, multiplied half a tile later,
-            // stored another half later
-            if constexpr (half == 0) {
-                multiply();
-            } else {
-                emit(sg - 3, sg > 1 ? 16 : 0);
-                fetch();
-            }
-            __builtin_amdgcn_sched_barrier(0);
-        });
-        const int last_sg = nfull - 1;
-        if (last_sg & 1) {
-            multiply();
-            emit(last_sg - 1, 16);
-        } else { // half a tile, and the one before it is not stored yet
-            emit(last_sg - 2, last_sg > 0 ? 16 : 0);
-            fetch();
-            multiply();
-            emit(last_sg, 8);
+    }
+    // put(token, head, logit) for the first ntok tokens of the tile that starts at `token`
+    template <typename PUT>
+    __device__ __forceinline__ void emit(int token, int ntok, PUT &&put)
+    {
+        const int t = lane & 15, quarter = lane >> 4;
+        if (t >= ntok || (GQ == 1 && quarter) || (GQ == 2 && (quarter & 1)))
+            return;
+        if constexpr (GQ == 8) {
+            put(token + t, 2 * quarter, (h1)d.x);
+            put(token + t, 2 * quarter + 1, (h1)d.z);
+        } else {
+            put(token + t, quarter * GQ >> 2, (h1)d.x);
         }
     }
-}
+
+    // all whole supergroups of a segment; put is given tokens from 0
+    template <typename PUT>
+    __device__ __forceinline__ void run(const uint2 *lut, uint32_t lane_copy, Pair &st, SegLoads<128, 2, BITS, AHEAD> &s, PUT &&put)
+    {
+        const int nfull = s.nfull;
+        if (nfull <= 0)
+            return;
+        const Vec *cb = s.cb;
+        auto &buf = s.buf;
+        uint2 e[2][8];
+        uint32_t nb[2];
+        auto bytes = [&](const Vec &u) __attribute__((always_inline)) {
+            if constexpr (BITS == 4)
+                pair_bytes(u.x, u.y, nb[0], nb[1]);
+            else
+                pair_bytes2(u.x, u.y, nb[0], nb[1]);
+        };
+        auto lookup = [&](uint2 *l, int unit) __attribute__((always_inline)) {
+            if constexpr (BITS == 4) {
+#pragma unroll
+                for (int t = 0; t < 8; t++)
+                    l[t] = lut_get(lut, nb[t & 1], lane_copy, t >> 1);
+            } else { // an entry is tokens s and s + 2
+#pragma unroll
+                for (int s = 0; s < 4; s++) {
+                    const int t = 4 * (s >> 1) + (s & 1);
+                    const uint4 v = lut2_get(lut, nb[s & 1], lane_copy, 2 * unit + (s >> 1));
+                    l[t] = make_uint2(v.x, v.y);
+                    l[t + 2] = make_uint2(v.z, v.w);
+                }
+            }
+        };
+        // no scalar load in flight when the loop starts: its waits would have to cover it
+        bytes(buf[0][0]);
+        lookup(e[0], 0);
+        wait_lgkm();
+        rotate_over<AHEAD>(nfull, [&](int sg, auto ic) __attribute__((always_inline)) {
+            constexpr int i = decltype(ic)::value;
+            static_for<UPS>([&](auto hc) __attribute__((always_inline)) {
+                constexpr int hf = decltype(hc)::value, half = (i * UPS + hf) & 1;
+                const int unit = sg * UPS + hf;
+                if constexpr (hf == UPS - 1) {
+                    bytes(buf[(i + 1) % AHEAD][0]); // stale past the end: looked up, never used
+                    lookup(e[half ^ 1], 0);
+                    buf[i][0] = load_codes(cb + (size_t)min(sg + AHEAD, nfull - 1) * G::VPS);
+                } else {
+                    lookup(e[half ^ 1], hf + 1);
+                }
+                __builtin_amdgcn_sched_barrier(0);
+                uint32_t kh[8];
+                replay_eight(st, e[half], kh);
+#pragma unroll
+                for (int t = 0; t < 8; t++)
+                    *reinterpret_cast<uint32_t *>(tile + (half * 8 + t) * 256 + wr[half * 4 + t / 2]) = kh[t];
+                __builtin_amdgcn_sched_barrier(0);
+                // the tile before this one: fetched when it was complete, multiplied half a tile later,
+                // stored another half later
+                if constexpr (half == 0) {
+                    multiply();
+                } else {
+                    emit((unit - 3) * 8, unit > 1 ? 16 : 0, put);
+                    fetch();
+                }
+                __builtin_amdgcn_sched_barrier(0);
+            });
+        });
+        const int last = nfull * UPS - 1;
+        if (last & 1) {
+            multiply();
+            emit((last - 1) * 8, 16, put);
+        } else { // half a tile, and the one before it is not stored yet
+            emit((last - 2) * 8, last > 0 ? 16 : 0, put);
+            fetch();
+            multiply();
+            emit(last * 8, 8, put);
+        }
+    }
+};
 
 
 template <int D, int CPL, int BLK>
 __global__ __launch_bounds__(BLK) void qk_kernel(
-    const h1 *__restrict__ q, uint4 *__restrict__ cache, const h1 *__restrict__ k_new,
+    const h1 *q, uint4 *__restrict__ cache, const h1 *k_new,
     h1 *__restrict__ out,
-    const h1 *__restrict__ zp, const h1 *__restrict__ sc, const h1 *__restrict__ al,
-    const h1 *__restrict__ be, const h1 *__restrict__ tg,
+    const h1 *zp, const h1 *sc, const h1 *al,
+    const h1 *be, const h1 *tg,
     int BH, int H, int T, int n_super_cap, h1 *__restrict__ state_out, Seg sa)
 {
     using G = Geo<D, CPL>;
@@ -1023,34 +1137,36 @@ __global__ __launch_bounds__(BLK) void qk_kernel(
     // the only LDS object: the table sits at LDS offset 0 (its byte address is used as is)
     __shared__ uint2 smem[LUT_WORDS64 + (PAIR ? (BLK / 64) * PAIR_TILE / 8 : 0)];
     const uint2 *lut = smem;
-    lut_fill<BLK>(smem, threadIdx.x);
-    __syncthreads();
-
     const int lane = threadIdx.x & 63;
     const uint32_t lane_copy = (uint32_t)(lane & (LUT_COPIES - 1)) * 8u;
 
-    const Unit<D, CPL, BLK> un(BH, sa.nseg);
-    if (!un.wave_active)
-        return; // padding waves
+    const Unit<D, CPL, BLK> un(BH, sa.nseg); // a padding wave's is valid too: it loads and leaves
     const int bx = un.bx, lh = un.lh, c0 = un.c0;
     const bool active = un.active;
-    const bool last = seg_is_last(sa, un.seg);
-    const int h = bx % H;
+    using Vec = typename G::Vec;
+    uint32_t qw[G::NP];
+    __builtin_memcpy(qw, q + (size_t)bx * D + c0, 2 * CPL);
+    PairScores<4, 1> scores(reinterpret_cast<char *>(smem + LUT_WORDS64) + (threadIdx.x >> 6) * PAIR_TILE, lane,
+                            q + (size_t)bx * D); // two channels per lane only
+    SegLoads<D, CPL, 4, PAIR ? PF_PAIR : PF> s;
+    s.start(cache, zp, sc, al, be, tg, bx % H, bx, lh, un.seg, T, n_super_cap, sa);
+    lut_fill<BLK>(smem, threadIdx.x);
+    __syncthreads();
+    if (!un.wave_active)
+        return; // padding waves
 
     Pair st[G::NP];
     h2 qv[G::NP];
-    init_pairs<D, CPL>(st, zp, sc, al, be, tg, h, bx, c0, un.seg, sa);
+    s.state(st);
 #pragma unroll
     for (int p = 0; p < G::NP; p++)
-        qv[p] = load_act2(q + (size_t)bx * D + c0 + 2 * p, sa.act_bf16);
+        qv[p] = act2(qw[p], sa.act_bf16);
 
-    const int t0 = seg_begin(sa, un.seg);
-    const int t1 = last ? T : seg_end(sa, un.seg);
-    using Vec = typename G::Vec;
-    Vec *cbh = reinterpret_cast<Vec *>(cache) + (size_t)bx * n_super_cap * G::VPS + lh * G::NV; // this head, this lane
-    const Vec *cb = cbh + (size_t)(t0 >> 3) * G::VPS;                                           // this segment
+    const bool last = s.last;
+    const int t0 = s.t0, t1 = s.t1, nfull = s.nfull;
+    Vec *cbh = s.cbh;
+    const Vec *cb = s.cb;
     h1 *ob = out + (size_t)bx * sa.row_pitch + t0;
-    const int nfull = (t1 - t0) >> 3;
     // the token whose total this lane's quad ends up with, and the one lane per token that stores
     // it (a 64-lane head holds every total twice, once per half)
     const int tk = token_of_lane(lane);
@@ -1062,12 +1178,11 @@ __global__ __launch_bounds__(BLK) void qk_kernel(
     };
 
     if constexpr (PAIR) {
-        pair_scores(lut, reinterpret_cast<char *>(smem + LUT_WORDS64) + (threadIdx.x >> 6) * PAIR_TILE, lane, lane_copy,
-                    st[0], q + (size_t)bx * D, sa.act_bf16, cb, nfull,
-                    [&](int t, h1 v) __attribute__((always_inline)) {
-                        if (active)
-                            ob[t] = v;
-                    });
+        scores.ready(sa.act_bf16);
+        scores.run(lut, lane_copy, st[0], s, [&](int t, int, h1 v) __attribute__((always_inline)) {
+            if (active)
+                ob[t] = v;
+        });
     } else {
         // ---- software pipeline over the full supergroups.  Global loads run PF supergroups ahead.
         // Table lookups run one supergroup ahead and are issued token by token between the arithmetic
@@ -1096,16 +1211,10 @@ __global__ __launch_bounds__(BLK) void qk_kernel(
             __builtin_amdgcn_sched_barrier(0);
         };
 
-        Vec buf[PF][G::NV];
+        auto &buf = s.buf;
         uint2 lk[G::NP][8];
         uint32_t nb[G::NP][2];
         float part[8] = {0, 0, 0, 0, 0, 0, 0, 0};
-#pragma unroll
-        for (int i = 0; i < PF; i++) {
-#pragma unroll
-            for (int v = 0; v < G::NV; v++)
-                buf[i][v] = (i < nfull) ? load_codes(cb + (size_t)i * G::VPS + v) : vec_zero<Vec>();
-        }
         if (nfull > 0) {
             pair_bytes_of<D, CPL>(buf[0], nb);
 #pragma unroll
@@ -1194,31 +1303,49 @@ __global__ __launch_bounds__(BLK) void qk_kernel(
 // `partial` [nseg, B*H, D] and ov_finalize_kernel adds them up.
 template <int D, int CPL, int BLK>
 __global__ __launch_bounds__(BLK) void ov_kernel(
-    const h1 *__restrict__ attn, uint4 *__restrict__ cache, const h1 *__restrict__ v_new,
+    const h1 *attn, uint4 *__restrict__ cache, const h1 *v_new,
     h1 *__restrict__ out, float *__restrict__ partial,
-    const h1 *__restrict__ zp, const h1 *__restrict__ sc, const h1 *__restrict__ al,
-    const h1 *__restrict__ be, const h1 *__restrict__ tg,
+    const h1 *zp, const h1 *sc, const h1 *al,
+    const h1 *be, const h1 *tg,
     int BH, int H, int T, int n_super_cap, h1 *__restrict__ state_out, Seg sa)
 {
     using G = Geo<D, CPL>;
     constexpr int AHEAD = CPL == 2 ? PF_PAIR : PF;
     sa.groups = 0; // only even plans come here
     __shared__ uint2 lut[LUT_WORDS64];
-    lut_fill<BLK>(lut, threadIdx.x);
-    __syncthreads();
     const uint32_t lane_copy = (uint32_t)(threadIdx.x & (LUT_COPIES - 1)) * 8u;
 
     const Unit<D, CPL, BLK> un(BH, sa.nseg);
-    if (!un.wave_active)
-        return; // padding waves
     const int bx = un.bx, lh = un.lh, c0 = un.c0;
     const bool active = un.active;
-    const bool last = seg_is_last(sa, un.seg);
-    const int h = bx % H;
+    using Vec = typename G::Vec;
+    SegLoads<D, CPL, 4, AHEAD> s;
+    s.start(cache, zp, sc, al, be, tg, bx % H, bx, lh, un.seg, T, n_super_cap, sa);
+    const bool last = s.last;
+    const int t0 = s.t0, t1 = s.t1, nfull = s.nfull;
+    Vec *cbh = s.cbh;
+    const Vec *cb = s.cb;
+    auto &buf = s.buf;
+    const h1 *wrow = attn + (size_t)bx * sa.row_pitch;
+    const h1 *wb = wrow + t0;
+    auto load_w = [&](int sg) {
+        uint4 r;
+        __builtin_memcpy(&r, wb + (size_t)sg * 8, 16); // row base is only 2-byte aligned
+        return r;
+    };
+    uint4 wbuf[AHEAD];
+    if (nfull > 0)
+#pragma unroll
+        for (int i = 0; i < AHEAD; i++)
+            wbuf[i] = load_w(min(i, nfull - 1));
+    lut_fill<BLK>(lut, threadIdx.x);
+    __syncthreads();
+    if (!un.wave_active)
+        return; // padding waves
 
     Pair st[G::NP];
     float acc[CPL];
-    init_pairs<D, CPL>(st, zp, sc, al, be, tg, h, bx, c0, un.seg, sa);
+    s.state(st);
 #pragma unroll
     for (int c = 0; c < CPL; c++)
         acc[c] = 0.0f;
@@ -1234,20 +1361,6 @@ __global__ __launch_bounds__(BLK) void ov_kernel(
     const uint32_t sel_a0 = role == 0 ? 0x0C0C0100u : role == 1 ? 0x01000C0Cu : 0x0C0C0C0Cu;
     const uint32_t sel_a1 = role == 0 ? 0x0C0C0302u : role == 1 ? 0x03020C0Cu : 0x0C0C0C0Cu;
 
-    const int t0 = seg_begin(sa, un.seg);
-    const int t1 = last ? T : seg_end(sa, un.seg);
-    using Vec = typename G::Vec;
-    Vec *cbh = reinterpret_cast<Vec *>(cache) + (size_t)bx * n_super_cap * G::VPS + lh * G::NV;
-    const Vec *cb = cbh + (size_t)(t0 >> 3) * G::VPS;
-    const h1 *wrow = attn + (size_t)bx * sa.row_pitch;
-    const h1 *wb = wrow + t0;
-    const int nfull = (t1 - t0) >> 3;
-
-    auto load_w = [&](int sg) {
-        uint4 r;
-        __builtin_memcpy(&r, wb + (size_t)sg * 8, 16); // row base is only 2-byte aligned
-        return r;
-    };
     // two tokens of the current supergroup on the matrix cores, then the lookups of the same two
     // slots of the next one
     auto token2 = [&](int t, uint2 (*e)[8], const uint32_t (*nb)[2], const uint4 wv) {
@@ -1275,21 +1388,9 @@ __global__ __launch_bounds__(BLK) void ov_kernel(
         __builtin_amdgcn_sched_barrier(0);
     };
 
-    Vec buf[AHEAD][G::NV];
-    uint4 wbuf[AHEAD];
     uint2 lk[MM ? G::NP : 2][8]; // two channels per lane: this supergroup's lookups and the next one's
     uint32_t nb[G::NP][2];
     if (nfull > 0) {
-        // unconditional, in the loop's order: see qk_kernel
-#pragma unroll
-        for (int i = 0; i < AHEAD; i++) {
-            const int sg = min(i, nfull - 1);
-#pragma unroll
-            for (int v = 0; v < G::NV; v++)
-                buf[i][v] = load_codes(cb + (size_t)sg * G::VPS + v);
-            wbuf[i] = load_w(sg);
-            __builtin_amdgcn_sched_barrier(0);
-        }
         pair_bytes_of<D, CPL>(buf[0], nb);
 #pragma unroll
         for (int t = 0; t < 8; t++)
@@ -1927,6 +2028,7 @@ static Seg plan_segments(void *ckpt, int n_ckpt_cap, int ckpt_interval, int BH, 
     s.n_ckpt_cap = n_ckpt_cap;
     s.ckpt_interval = ckpt ? ckpt_interval : 0;
     s.seg_tokens = T > 0 ? T : 1;
+    s.seg_intervals = 0;
     s.nseg = 1;
     s.row_pitch = T + 1;
     s.act_bf16 = 0;
@@ -1977,6 +2079,7 @@ static Seg plan_segments(void *ckpt, int n_ckpt_cap, int ckpt_interval, int BH, 
     if (best < 0 || best >= avail)
         return s;
     s.seg_tokens = best * ckpt_interval;
+    s.seg_intervals = best;
     s.nseg = (T + s.seg_tokens - 1) / s.seg_tokens;
     return s;
 }
@@ -2031,26 +2134,36 @@ static int threads_per_workgroup(long threads)
     }                                                 \
     }
 
-// Matrix-core kernels (head dim 128): the same rule, with 8-wave workgroups for small launches
-// (their LDS tile leaves room for one workgroup per CU either way).  Eight query heads per KV head
-// need ~138 registers per lane, more than the 128 a 16-wave workgroup leaves: qk_gqa_kernel still
-// gains from four waves per SIMD with a dozen cold values spilled (cfg5 KV shape, 64 query heads:
-// 563 -> 530 us with 4-bit codes, 518 -> 425 us with 2-bit ones), ov_gqa_kernel spills
-// accumulators and loses (421 -> 533 us, 346 -> 747 us), so BIG8 says which of the two this is.
+// Matrix-core kernels (head dim 128), four channels per lane: 12- or 16-wave workgroups by the same
+// rule.  Eight query heads per KV head need ~138 registers per lane, more than the 128 a 16-wave
+// workgroup leaves: qk_gqa_kernel still gains from four waves per SIMD with a dozen cold values spilled
+// (16 x 8 KV heads x 131072 tokens, 64 query heads: 563 -> 530 us with 4-bit codes, 518 -> 425 us with
+// 2-bit ones), ov_gqa_kernel spills accumulators and loses (421 -> 533 us, 346 -> 747 us), so BIG8 says
+// which of the two this is, and the latter takes 8-wave workgroups.
+// A launch that would leave at most two waves on a SIMD takes two channels per lane instead (a KV head
+// per wave): twice the waves, forward_qk without the reduction over the quarters of a head.  8 x 8 KV
+// heads x 16001 tokens, four query heads each (16 waves per CU instead of 8), kernel times: forward_qk
+// 31.3 / 28.3 us, forward_ov 27.9 / 27.5.  With more waves than that the four-channel lanes have enough
+// of them and spend fewer instructions on what a wave does once per token.
+static bool gqa_pair(long BH, int nseg) { return padded_units<64>((int)BH, nseg) <= 4L * n_simd(); }
+#define ADKV_LAUNCH_GQA_(KERNEL, BB, GQV, BLK, CPLV, ...)                                          \
+    hipLaunchKernelGGL((KERNEL<BB, GQV, BLK, CPLV>), dim3((unsigned)((threads + (BLK)-1) / (BLK))), dim3(BLK), 0, st, __VA_ARGS__)
 #define ADKV_LAUNCH_GQA(KERNEL, BIG8, BB, GQV, ...)                                                \
     do {                                                                                            \
-        const long threads = padded_units<32>(BH, seg.nseg) * 32;                                   \
-        constexpr int GBIG = (GQV <= 4 || BIG8) ? GQV : 1; /* unused instantiation otherwise */     \
-        const int blk = (GQV <= 4 || BIG8) ? threads_per_workgroup(threads) : 512;            \
-        if (blk == 1024)                                                                            \
-            hipLaunchKernelGGL((KERNEL<BB, GBIG, 1024>), dim3((unsigned)((threads + 1023) / 1024)), \
-                               dim3(1024), 0, st, __VA_ARGS__);                                     \
-        else if (blk == 768)                                                                        \
-            hipLaunchKernelGGL((KERNEL<BB, GBIG, 768>), dim3((unsigned)((threads + 767) / 768)),    \
-                               dim3(768), 0, st, __VA_ARGS__);                                      \
-        else                                                                                        \
-            hipLaunchKernelGGL((KERNEL<BB, GQV, 512>), dim3((unsigned)((threads + 511) / 512)),     \
-                               dim3(512), 0, st, __VA_ARGS__);                                      \
+        const bool pair = gqa_pair(BH, seg.nseg);                                                   \
+        const long threads = pair ? padded_units<64>(BH, seg.nseg) * 64 : padded_units<32>(BH, seg.nseg) * 32; \
+        const int blk = threads_per_workgroup(threads);                                             \
+        constexpr bool BIG = GQV <= 4 || BIG8;                                                      \
+        if (pair && blk == 1024)                                                                    \
+            ADKV_LAUNCH_GQA_(KERNEL, BB, GQV, 1024, 2, __VA_ARGS__);                                \
+        else if (pair && blk == 768)                                                                \
+            ADKV_LAUNCH_GQA_(KERNEL, BB, GQV, 768, 2, __VA_ARGS__);                                 \
+        else if (pair)                                                                              \
+            ADKV_LAUNCH_GQA_(KERNEL, BB, GQV, 256, 2, __VA_ARGS__);                                 \
+        else if (blk == 1024 || !BIG)                                                               \
+            ADKV_LAUNCH_GQA_(KERNEL, BB, GQV, (BIG ? 1024 : 512), 4, __VA_ARGS__);                  \
+        else /* more than eight waves per CU: never 256 */                                          \
+            ADKV_LAUNCH_GQA_(KERNEL, BB, GQV, (BIG ? 768 : 512), 4, __VA_ARGS__);                   \
     } while (0)
 
 #define ADKV_DISPATCH_GQ_BITS(KERNEL, BIG8, BB, ...)                                               \
@@ -2661,10 +2774,11 @@ static const char *decode_kernel_name(int B, int Hq, int H, int T, int D, int bi
     const Seg seg = plan_segments(n_ckpt_cap > 0 && ckpt_interval > 0 ? &dummy : nullptr, n_ckpt_cap,
                                   ckpt_interval, B * H, T, D);
     if (D == 128 && (GQ > 1 || bits != 4 || mfma_for_mha())) {
-        const int blk = threads_per_workgroup(padded_units<32>(B * H, seg.nseg) * 32);
-        return blk == 1024 ? "gqa_kernel, 16-wave workgroups (matrix cores)"
-               : blk == 768 ? "gqa_kernel, 12-wave workgroups (matrix cores)"
-                            : "gqa_kernel, 8-wave workgroups (matrix cores)";
+        if (gqa_pair(B * H, seg.nseg))
+            return "gqa_kernel, two channels per lane (matrix cores)";
+        return threads_per_workgroup(padded_units<32>(B * H, seg.nseg) * 32) == 1024
+                   ? "gqa_kernel, 16-wave workgroups (matrix cores)"
+                   : "gqa_kernel, 12-wave workgroups (matrix cores)";
     }
     if (use_head_table(B, H, GQ, bits, D, seg)) {
         Seg s2 = seg;
@@ -3308,7 +3422,7 @@ int adkv_decode_step(const void *q, void *k_cache, void *v_cache, const void *k_
             va.ckpt = (h1 *)v_ckpt;
             const FtParams kp = ft_params(k_params), vp = ft_params(v_params);
             hipLaunchKernelGGL(small_step_kernel, dim3((unsigned)(B * H)), dim3(256), 0, (hipStream_t)stream, (const h1 *)q,
-                               (uint2 *)k_cache, (const h1 *)k_new, (uint2 *)v_cache, (const h1 *)v_new, (const float *)mask,
+                               (uint4 *)k_cache, (const h1 *)k_new, (uint4 *)v_cache, (const h1 *)v_new, (const float *)mask,
                                mask ? rows_per_mask_row : 1, (h1 *)weights, (h1 *)out, kp, vp, H, T,
                                n_super_cap, scaling, ka, va);
             return (rc = check_launch()) ? rc : mark_one_launch(stream);

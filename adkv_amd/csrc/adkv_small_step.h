@@ -14,8 +14,8 @@ namespace adkv {
 constexpr int SMALL_ROW = 3 * 64 * SM_VEC; // longest row of logits: three vectors per lane
 
 __global__ __launch_bounds__(256) void small_step_kernel(
-    const h1 *__restrict__ q, uint2 *__restrict__ k_cache, const h1 *__restrict__ k_new, uint2 *__restrict__ v_cache,
-    const h1 *__restrict__ v_new, const float *__restrict__ mask, int rows_per_mask_row, h1 *__restrict__ weights,
+    const h1 *q, uint4 *__restrict__ k_cache, const h1 *k_new, uint4 *__restrict__ v_cache,
+    const h1 *v_new, const float *__restrict__ mask, int rows_per_mask_row, h1 *__restrict__ weights,
     h1 *__restrict__ out, FtParams kp, FtParams vp, int H, int T, int n_super_cap, float scaling, Seg ka, Seg va)
 {
     constexpr int D = 128, CPL = 2;
@@ -31,23 +31,23 @@ __global__ __launch_bounds__(256) void small_step_kernel(
     h1 *logits = reinterpret_cast<h1 *>(lds + LUT_WORDS64 * 8 + 4 * PAIR_TILE);
     float *partial = reinterpret_cast<float *>(lds + LUT_WORDS64 * 8 + 4 * PAIR_TILE + SMALL_ROW * 2);
     ka.groups = va.groups = 0;
-    lut_fill<256>(lut, threadIdx.x);
-
     const int bx = blockIdx.x, h = bx % H, c0 = lane * 2, n = T + 1;
-    const bool works = seg < ka.nseg, last = seg == ka.nseg - 1;
-    const int t0 = works ? seg_begin(ka, seg) : 0, t1 = !works ? 0 : last ? T : seg_end(ka, seg);
-    const int nfull = (t1 - t0) >> 3, ntail = (t1 - t0) & 7; // only the last segment has a tail
+    const bool works = seg < ka.nseg;
     const uint32_t lane_copy = (uint32_t)(lane & (LUT_COPIES - 1)) * 8u;
-    const size_t head = (size_t)bx * n_super_cap * G::VPS + lane;
-    Pair st[1];
-    if (works)
-        init_pairs<D, CPL>(st, kp.zp, kp.sc, kp.al, kp.be, kp.tg, h, bx, c0, seg, ka);
+    PairScores<4, 1> scores(tile, lane, q + (size_t)bx * D);
+    SegLoads<D, CPL, 4, PF_PAIR> s;
+    s.start(k_cache, kp.zp, kp.sc, kp.al, kp.be, kp.tg, h, bx, lane, works ? seg : 0, T, n_super_cap, ka);
+    const bool last = works && s.last;
+    const int t0 = s.t0, nfull = s.nfull, ntail = (s.t1 - s.t0) & 7; // only the last segment has a tail
+    lut_fill<256>(lut, threadIdx.x);
     __syncthreads();
 
+    Pair st[1];
     if (works) {
-        const uint2 *cb = k_cache + head + (size_t)(t0 >> 3) * G::VPS;
-        pair_scores(lut, tile, lane, lane_copy, st[0], q + (size_t)bx * D, ka.act_bf16, cb, nfull,
-                    [&](int t, h1 v) __attribute__((always_inline)) { logits[t0 + t] = v; });
+        const uint2 *cb = s.cb;
+        s.state(st);
+        scores.ready(ka.act_bf16);
+        scores.run(lut, lane_copy, st[0], s, [&](int t, int, h1 v) __attribute__((always_inline)) { logits[t0 + t] = v; });
         if (last) {
             const h2 qv = load_act2(q + (size_t)bx * D + c0, ka.act_bf16);
             if (ntail) {
@@ -69,13 +69,13 @@ __global__ __launch_bounds__(256) void small_step_kernel(
             }
             publish_state<D, CPL>(st, nullptr, ka, bx, c0, T);
             h2 deq[1];
-            append_new_token<D, CPL>(k_cache + head, T, k_new + (size_t)bx * D + c0, st, deq, true, ka.act_bf16);
+            append_new_token<D, CPL>(s.cbh, T, k_new + (size_t)bx * D + c0, st, deq, true, ka.act_bf16);
             const float self = head_allreduce<64>(__builtin_amdgcn_fdot2(qv, deq[0], 0.0f, false));
             if (lane == 0)
                 logits[T] = (h1)self;
         }
-        // the V segment's state is on its way while the other waves finish
-        init_pairs<D, CPL>(st, vp.zp, vp.sc, vp.al, vp.be, vp.tg, h, bx, c0, seg, va);
+        // the V segment's state and codes are on their way while the other waves finish
+        s.start(v_cache, vp.zp, vp.sc, vp.al, vp.be, vp.tg, h, bx, lane, seg, T, n_super_cap, va);
     }
     __syncthreads();
 
@@ -102,11 +102,13 @@ __global__ __launch_bounds__(256) void small_step_kernel(
         if (seg == 0)
             softmax_store_chunk<SMALL_ROW / 512, 64>(weights + (size_t)bx * ka.row_pitch, n, 0, x, 1.0f / sum, lane);
 
-        const uint2 *cb = v_cache + head + (size_t)(t0 >> 3) * G::VPS;
+        const uint2 *cb = s.cb;
+        s.state(st);
         float acc[2] = {0.0f, 0.0f};
         if (nfull > 0) {
             auto weights_of = [&](int sg) { return *reinterpret_cast<const uint4 *>(w + t0 + sg * 8); };
-            uint2 buf[PF_PAIR][1], e[2][8];
+            auto &buf = s.buf;
+            uint2 e[2][8];
             uint4 wv[2];
             uint32_t nb[1][2];
             auto lookup = [&](uint2 *d, const uint2 *u) __attribute__((always_inline)) {
@@ -115,11 +117,6 @@ __global__ __launch_bounds__(256) void small_step_kernel(
                 for (int t = 0; t < 8; t++)
                     d[t] = lut_get(lut, nb[0][t & 1], lane_copy, t >> 1);
             };
-#pragma unroll
-            for (int i = 0; i < PF_PAIR; i++) {
-                buf[i][0] = load_codes(cb + (size_t)min(i, nfull - 1) * G::VPS);
-                __builtin_amdgcn_sched_barrier(0);
-            }
             lookup(e[0], buf[0]);
             wv[0] = weights_of(0);
             wait_lgkm();
@@ -149,7 +146,7 @@ __global__ __launch_bounds__(256) void small_step_kernel(
             }
             publish_state<D, CPL>(st, nullptr, va, bx, c0, T);
             h2 deq[1];
-            append_new_token<D, CPL>(v_cache + head, T, v_new + (size_t)bx * D + c0, st, deq, true, va.act_bf16);
+            append_new_token<D, CPL>(s.cbh, T, v_new + (size_t)bx * D + c0, st, deq, true, va.act_bf16);
             add((float)w[T], deq[0]);
         }
         reinterpret_cast<float2 *>(partial)[seg * 64 + lane] = make_float2(acc[0], acc[1]);
