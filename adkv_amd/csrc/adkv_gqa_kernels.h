@@ -152,25 +152,14 @@ __device__ __forceinline__ uint32_t table_lane_offset(int lane)
 }
 
 // forward_qk of one segment, two channels per lane: a KV head fills the wave (see PairScores).
-template <int BITS, int GQ, int BLK>
-__device__ __forceinline__ void qk_gqa_pair(
-    uint2 *smem, const h1 *q, uint4 *__restrict__ cache, const h1 *k_new, h1 *__restrict__ out,
-    const h1 *zp, const h1 *sc, const h1 *al, const h1 *be,
-    const h1 *tg, int BH, int H, int T, int n_super_cap, h1 *__restrict__ state_out, Seg sa)
+template <int BITS, int GQ>
+__device__ __forceinline__ void qk_gqa_pair_segment(const uint2 *lut, int lane, int bx, PairScores<BITS, GQ> &scores,
+                                                    SegLoads<GQA_D, 2, BITS, PairScores<BITS, GQ>::AHEAD> &s,
+                                                    const h1 *k_new, h1 *out, int T, h1 *state_out, const Seg &sa)
 {
-    sa.groups = 0; // only even plans come here
     constexpr int D = GQA_D, CPL = 2, TPW = Code<BITS>::TPW;
     using G = Geo<D, CPL>;
-    const Unit<D, CPL, BLK> un(BH, sa.nseg);
-    const int bx = un.bx, lane = un.lh, c0 = un.c0;
-    PairScores<BITS, GQ> scores(reinterpret_cast<char *>(smem + LUT_WORDS64) + (threadIdx.x >> 6) * PAIR_TILE, lane,
-                                q + (size_t)bx * GQ * D);
-    SegLoads<D, CPL, BITS, PairScores<BITS, GQ>::AHEAD> s;
-    s.start(cache, zp, sc, al, be, tg, bx % H, bx, lane, un.seg, T, n_super_cap, sa);
-    fill_table<BITS, BLK>(smem, threadIdx.x);
-    __syncthreads();
-    if (!un.wave_active)
-        return; // padding waves
+    const int c0 = lane * CPL;
     Pair st[1];
     s.state(st);
     scores.ready(sa.act_bf16);
@@ -180,7 +169,7 @@ __device__ __forceinline__ void qk_gqa_pair(
     const uint2 *cb = s.cb;
     h1 *ob = out + (size_t)bx * GQ * sa.row_pitch + t0;
     auto put = [&](int t, int g, h1 v) __attribute__((always_inline)) { ob[(size_t)g * sa.row_pitch + t] = v; };
-    scores.run(smem, table_lane_offset<BITS>(lane), st[0], s, put);
+    scores.run(lut, table_lane_offset<BITS>(lane), st[0], s, put);
     if (!last)
         return;
     // ragged tail and the appended token: at most a tile
@@ -215,10 +204,17 @@ __global__ __launch_bounds__(BLK) void qk_gqa_kernel(
     int BH, int H, int T, int n_super_cap, h1 *__restrict__ state_out, Seg sa)
 {
     if constexpr (CPL == 2) {
+        sa.groups = 0; // only even plans come here
         __shared__ uint2 smem[LUT_WORDS64 + (BLK / 64) * PAIR_TILE / 8];
-        qk_gqa_pair<BITS, GQ, BLK>(smem, q, cache, k_new, out, zp, sc, al, be, tg, BH, H, T,
-                                   n_super_cap, state_out, sa);
-        return;
+        const Unit<GQA_D, 2, BLK> un(BH, sa.nseg);
+        PairScores<BITS, GQ> scores(reinterpret_cast<char *>(smem + LUT_WORDS64) + (threadIdx.x >> 6) * PAIR_TILE, un.lh,
+                                    q + (size_t)un.bx * GQ * GQA_D);
+        SegLoads<GQA_D, 2, BITS, PairScores<BITS, GQ>::AHEAD> s;
+        s.start(cache, zp, sc, al, be, tg, un.bx % H, un.bx, un.lh, un.seg, T, n_super_cap, sa);
+        fill_table<BITS, BLK>(smem, threadIdx.x);
+        __syncthreads();
+        if (un.wave_active)
+            qk_gqa_pair_segment<BITS, GQ>(smem, un.lh, un.bx, scores, s, k_new, out, T, state_out, sa);
     } else {
     constexpr int D = GQA_D;
     constexpr int NB = (GQ + 3) / 4; // column sets of four heads
@@ -390,66 +386,30 @@ __global__ __launch_bounds__(BLK) void qk_gqa_kernel(
 // ---------------------------------------------------------------------------------------------
 // forward_ov with GQ query heads per KV head
 // ---------------------------------------------------------------------------------------------
-template <int BITS, int GQ, int BLK, int CPL>
-__global__ __launch_bounds__(BLK) void ov_gqa_kernel(
-    const h1 *attn, uint4 *__restrict__ cache, const h1 *v_new,
-    h1 *__restrict__ out, float *__restrict__ partial,
-    const h1 *zp, const h1 *sc, const h1 *al,
-    const h1 *be, const h1 *tg,
-    int BH, int H, int T, int n_super_cap, h1 *__restrict__ state_out, Seg sa)
+// forward_ov of one segment for GQ query heads: acc[column set][channel of this lane], element i = head
+// 4n + i.  w8(n, unit): the weights of the unit's eight tokens for this lane's row of column set n, the
+// first two units' in wbuf; w1(head, t): the weight of the segment's token t.
+constexpr int GQA_WPF = 2; // weight vectors (8 tokens each) in flight
+template <int BITS, int GQ, int CPL>
+constexpr int gqa_ahead() { return (BITS == 2 || GQ > 4) ? 2 : PF; } // supergroups in flight per lane
+template <int BITS, int GQ, int CPL, typename W8, typename W1>
+__device__ __forceinline__ void ov_gqa_segment(const uint2 *lut, uint32_t lane_copy, int bx, int c0, bool active,
+                                               SegLoads<GQA_D, CPL, BITS, gqa_ahead<BITS, GQ, CPL>()> &s,
+                                               uint4 (*wbuf)[(GQ + 3) / 4], W8 &&w8, W1 &&w1, const h1 *v_new, int T,
+                                               h1 *state_out, const Seg &sa, f4v (*acc)[CPL])
 {
-    constexpr int D = GQA_D;
-    if (CPL == 2)
-        sa.groups = 0; // only even plans come here
-    constexpr int NB = (GQ + 3) / 4;
-    constexpr int TPW = Code<BITS>::TPW, UPS = TPW / 8;
-    constexpr int GPF = (BITS == 2 || NB > 1) ? 2 : PF;    // supergroups in flight per lane
-    constexpr int WPF = 2;                                 // weight vectors (8 tokens each) in flight
+    constexpr int D = GQA_D, NB = (GQ + 3) / 4, TPW = Code<BITS>::TPW, UPS = TPW / 8;
+    constexpr int GPF = gqa_ahead<BITS, GQ, CPL>(), WPF = GQA_WPF;
     static_assert((GPF * UPS) % WPF == 0, "weight ring must line up with the unrolled loop");
     using G = Geo<D, CPL>;
-    __shared__ uint2 lut[LUT_WORDS64];
-    const int lane = threadIdx.x & 63;
-    const uint32_t lane_copy = table_lane_offset<BITS>(lane);
-
-    const Unit<D, CPL, BLK> un(BH, sa.nseg);
-    const int bx = un.bx, lh = un.lh, c0 = un.c0;
-    const bool active = un.active;
-    const int r = lane & 3;
     using Vec = typename G::Vec;
-    SegLoads<D, CPL, BITS, GPF> s;
-    s.start(cache, zp, sc, al, be, tg, bx % H, bx, lh, un.seg, T, n_super_cap, sa);
     const bool last = s.last;
-    const int t0 = s.t0, t1 = s.t1, nfull = s.nfull;
+    const int t0 = s.t0, t1 = s.t1, nfull = s.nfull, nunits = nfull * UPS;
     Vec *cbh = s.cbh;
     const Vec *cb = s.cb;
     auto &buf = s.buf;
-    const int nunits = nfull * UPS;
-    // A operand rows: the weights of head r (+4 per column set) of this lane's KV head; lanes of no head
-    // repeat one, into rows of the product that nobody reads
-    const h1 *wb[NB];
-#pragma unroll
-    for (int n = 0; n < NB; n++)
-        wb[n] = attn + ((size_t)bx * GQ + min(4 * n + r, GQ - 1)) * sa.row_pitch + t0;
-    auto load_w = [&](int n, int unit) {
-        uint4 v;
-        __builtin_memcpy(&v, wb[n] + (size_t)unit * 8, 16); // rows are only 2-byte aligned
-        return v;
-    };
-    uint4 wbuf[WPF][NB];
-    if (nunits > 0)
-#pragma unroll
-        for (int i = 0; i < WPF; i++)
-#pragma unroll
-            for (int n = 0; n < NB; n++)
-                wbuf[i][n] = load_w(n, min(i, nunits - 1));
-    fill_table<BITS, BLK>(lut, threadIdx.x);
-    __syncthreads();
-    if (!un.wave_active)
-        return; // padding waves
-
     Pair st[G::NP];
     s.state(st);
-    f4v acc[NB][CPL]; // [column set][channel of this lane], element i = head 4n+i
 #pragma unroll
     for (int n = 0; n < NB; n++)
 #pragma unroll
@@ -518,7 +478,7 @@ __global__ __launch_bounds__(BLK) void ov_gqa_kernel(
             // loop edge, which wait for the load they move
 #pragma unroll
             for (int n = 0; n < NB; n++)
-                wbuf[ws][n] = load_w(n, min(unit + WPF, nunits - 1));
+                wbuf[ws][n] = w8(n, min(unit + WPF, nunits - 1));
         }
 #pragma unroll
         for (int p = 0; p < G::NP; p++) {
@@ -533,7 +493,7 @@ __global__ __launch_bounds__(BLK) void ov_gqa_kernel(
         auto add_token = [&](const h2 *vd, int t) {
 #pragma unroll
             for (int g = 0; g < GQ; g++) {
-                const float wt = (float)attn[((size_t)bx * GQ + g) * sa.row_pitch + t];
+                const float wt = (float)w1(g, t);
 #pragma unroll
                 for (int p = 0; p < G::NP; p++) {
                     acc[g >> 2][2 * p][g & 3] = __builtin_fmaf(wt, (float)vd[p].x, acc[g >> 2][2 * p][g & 3]);
@@ -556,15 +516,69 @@ __global__ __launch_bounds__(BLK) void ov_gqa_kernel(
                     vd[pp] = qs + s.zp;
                     update_pair(s, qc, qs);
                 }
-                add_token(vd, t0 + nfull * TPW + tt);
+                add_token(vd, nfull * TPW + tt);
             }
         }
         if (active)
             publish_state<D, CPL>(st, state_out, sa, bx, c0, T);
         h2 deq[G::NP];
         append_new_token<D, CPL, BITS>(cbh, T, v_new + (size_t)bx * D + c0, st, deq, active, sa.act_bf16);
-        add_token(deq, T);
+        add_token(deq, T - t0);
     }
+}
+
+template <int BITS, int GQ, int BLK, int CPL>
+__global__ __launch_bounds__(BLK) void ov_gqa_kernel(
+    const h1 *attn, uint4 *__restrict__ cache, const h1 *v_new,
+    h1 *__restrict__ out, float *__restrict__ partial,
+    const h1 *zp, const h1 *sc, const h1 *al,
+    const h1 *be, const h1 *tg,
+    int BH, int H, int T, int n_super_cap, h1 *__restrict__ state_out, Seg sa)
+{
+    constexpr int D = GQA_D;
+    if (CPL == 2)
+        sa.groups = 0; // only even plans come here
+    constexpr int NB = (GQ + 3) / 4;
+    constexpr int TPW = Code<BITS>::TPW, UPS = TPW / 8;
+    constexpr int GPF = gqa_ahead<BITS, GQ, CPL>(), WPF = GQA_WPF;
+    __shared__ uint2 lut[LUT_WORDS64];
+    const int lane = threadIdx.x & 63;
+    const uint32_t lane_copy = table_lane_offset<BITS>(lane);
+
+    const Unit<D, CPL, BLK> un(BH, sa.nseg);
+    const int bx = un.bx, lh = un.lh, c0 = un.c0;
+    const bool active = un.active;
+    const int r = lane & 3;
+    SegLoads<D, CPL, BITS, GPF> s;
+    s.start(cache, zp, sc, al, be, tg, bx % H, bx, lh, un.seg, T, n_super_cap, sa);
+    const int nunits = s.nfull * UPS;
+    // A operand rows: the weights of head r (+4 per column set) of this lane's KV head; lanes of no head
+    // repeat one, into rows of the product that nobody reads
+    const h1 *wb[NB];
+#pragma unroll
+    for (int n = 0; n < NB; n++)
+        wb[n] = attn + ((size_t)bx * GQ + min(4 * n + r, GQ - 1)) * sa.row_pitch + s.t0;
+    auto load_w = [&](int n, int unit) {
+        uint4 v;
+        __builtin_memcpy(&v, wb[n] + (size_t)unit * 8, 16); // rows are only 2-byte aligned
+        return v;
+    };
+    uint4 wbuf[WPF][NB];
+    if (nunits > 0)
+#pragma unroll
+        for (int i = 0; i < WPF; i++)
+#pragma unroll
+            for (int n = 0; n < NB; n++)
+                wbuf[i][n] = load_w(n, min(i, nunits - 1));
+    fill_table<BITS, BLK>(lut, threadIdx.x);
+    __syncthreads();
+    if (!un.wave_active)
+        return; // padding waves
+
+    f4v acc[NB][CPL];
+    ov_gqa_segment<BITS, GQ, CPL>(lut, lane_copy, bx, c0, active, s, wbuf, load_w,
+                                  [&](int g, int t) { return attn[((size_t)bx * GQ + g) * sa.row_pitch + s.t0 + t]; }, v_new, T,
+                                  state_out, sa, acc);
     if (!active)
         return;
 #pragma unroll

@@ -1122,39 +1122,16 @@ struct PairScores {
 };
 
 
-template <int D, int CPL, int BLK>
-__global__ __launch_bounds__(BLK) void qk_kernel(
-    const h1 *q, uint4 *__restrict__ cache, const h1 *k_new,
-    h1 *__restrict__ out,
-    const h1 *zp, const h1 *sc, const h1 *al,
-    const h1 *be, const h1 *tg,
-    int BH, int H, int T, int n_super_cap, h1 *__restrict__ state_out, Seg sa)
+// forward_qk of one (head, segment), from the loads that s.start() and the caller have sent off.
+// Writes the segment's logits to out + bx * row_pitch and, with the context's last segment, appends.
+template <int D, int CPL>
+__device__ __forceinline__ void qk_segment(const uint2 *lut, uint32_t lane_copy, int lane, int bx, int lh, int c0, bool active,
+                                           PairScores<4, 1> &scores, SegLoads<D, CPL, 4, CPL == 2 ? PF_PAIR : PF> &s,
+                                           const uint32_t *qw, const h1 *k_new, h1 *out, int T, h1 *state_out, const Seg &sa)
 {
     using G = Geo<D, CPL>;
-    sa.groups = 0; // only even plans come here (a fifth of the code was the other kind's cuts)
-    // two channels per lane: the head fills the wave, see the loop below
-    constexpr bool PAIR = CPL == 2;
-    // the only LDS object: the table sits at LDS offset 0 (its byte address is used as is)
-    __shared__ uint2 smem[LUT_WORDS64 + (PAIR ? (BLK / 64) * PAIR_TILE / 8 : 0)];
-    const uint2 *lut = smem;
-    const int lane = threadIdx.x & 63;
-    const uint32_t lane_copy = (uint32_t)(lane & (LUT_COPIES - 1)) * 8u;
-
-    const Unit<D, CPL, BLK> un(BH, sa.nseg); // a padding wave's is valid too: it loads and leaves
-    const int bx = un.bx, lh = un.lh, c0 = un.c0;
-    const bool active = un.active;
     using Vec = typename G::Vec;
-    uint32_t qw[G::NP];
-    __builtin_memcpy(qw, q + (size_t)bx * D + c0, 2 * CPL);
-    PairScores<4, 1> scores(reinterpret_cast<char *>(smem + LUT_WORDS64) + (threadIdx.x >> 6) * PAIR_TILE, lane,
-                            q + (size_t)bx * D); // two channels per lane only
-    SegLoads<D, CPL, 4, PAIR ? PF_PAIR : PF> s;
-    s.start(cache, zp, sc, al, be, tg, bx % H, bx, lh, un.seg, T, n_super_cap, sa);
-    lut_fill<BLK>(smem, threadIdx.x);
-    __syncthreads();
-    if (!un.wave_active)
-        return; // padding waves
-
+    constexpr bool PAIR = CPL == 2; // the head fills the wave: see PairScores
     Pair st[G::NP];
     h2 qv[G::NP];
     s.state(st);
@@ -1294,6 +1271,40 @@ __global__ __launch_bounds__(BLK) void qk_kernel(
         out[(size_t)bx * sa.row_pitch + T] = (h1)self;
 }
 
+template <int D, int CPL, int BLK>
+__global__ __launch_bounds__(BLK) void qk_kernel(
+    const h1 *q, uint4 *__restrict__ cache, const h1 *k_new,
+    h1 *__restrict__ out,
+    const h1 *zp, const h1 *sc, const h1 *al,
+    const h1 *be, const h1 *tg,
+    int BH, int H, int T, int n_super_cap, h1 *__restrict__ state_out, Seg sa)
+{
+    using G = Geo<D, CPL>;
+    sa.groups = 0; // only even plans come here (a fifth of the code was the other kind's cuts)
+    constexpr bool PAIR = CPL == 2;
+    // the only LDS object: the table sits at LDS offset 0 (its byte address is used as is)
+    __shared__ uint2 smem[LUT_WORDS64 + (PAIR ? (BLK / 64) * PAIR_TILE / 8 : 0)];
+    const uint2 *lut = smem;
+    const int lane = threadIdx.x & 63;
+    const uint32_t lane_copy = (uint32_t)(lane & (LUT_COPIES - 1)) * 8u;
+
+    const Unit<D, CPL, BLK> un(BH, sa.nseg); // a padding wave's is valid too: it loads and leaves
+    const int bx = un.bx, lh = un.lh, c0 = un.c0;
+    const bool active = un.active;
+    uint32_t qw[G::NP];
+    __builtin_memcpy(qw, q + (size_t)bx * D + c0, 2 * CPL);
+    PairScores<4, 1> scores(reinterpret_cast<char *>(smem + LUT_WORDS64) + (threadIdx.x >> 6) * PAIR_TILE, lane,
+                            q + (size_t)bx * D); // two channels per lane only
+    SegLoads<D, CPL, 4, PAIR ? PF_PAIR : PF> s;
+    s.start(cache, zp, sc, al, be, tg, bx % H, bx, lh, un.seg, T, n_super_cap, sa);
+    lut_fill<BLK>(smem, threadIdx.x);
+    __syncthreads();
+    if (!un.wave_active)
+        return; // padding waves
+
+    qk_segment<D, CPL>(lut, lane_copy, lane, bx, lh, c0, active, scores, s, qw, k_new, out, T, state_out, sa);
+}
+
 // ---------------------------------------------------------------------------------------------
 // forward_ov  (gemv.cu:946-1178)
 // ---------------------------------------------------------------------------------------------
@@ -1301,50 +1312,22 @@ __global__ __launch_bounds__(BLK) void qk_kernel(
 // reference accumulates in fp16 for the whole sequence (gemv.cu:1087,1096).  With one segment the
 // result is rounded to fp16 and stored; with several, each segment stores its fp32 partial into
 // `partial` [nseg, B*H, D] and ov_finalize_kernel adds them up.
-template <int D, int CPL, int BLK>
-__global__ __launch_bounds__(BLK) void ov_kernel(
-    const h1 *attn, uint4 *__restrict__ cache, const h1 *v_new,
-    h1 *__restrict__ out, float *__restrict__ partial,
-    const h1 *zp, const h1 *sc, const h1 *al,
-    const h1 *be, const h1 *tg,
-    int BH, int H, int T, int n_super_cap, h1 *__restrict__ state_out, Seg sa)
+// forward_ov of one (head, segment): acc = this lane's channels.  w8(sg): the weights of the eight tokens of
+// the segment's supergroup sg, of which the first WR are in wbuf; w1(t): the weight of its token t.
+template <int D, int CPL, int WR, typename W8, typename W1>
+__device__ __forceinline__ void ov_segment(const uint2 *lut, uint32_t lane_copy, int bx, int c0, bool active,
+                                           SegLoads<D, CPL, 4, CPL == 2 ? PF_PAIR : PF> &s, uint4 *wbuf, W8 &&w8, W1 &&w1,
+                                           const h1 *v_new, int T, h1 *state_out, const Seg &sa, float *acc)
 {
     using G = Geo<D, CPL>;
-    constexpr int AHEAD = CPL == 2 ? PF_PAIR : PF;
-    sa.groups = 0; // only even plans come here
-    __shared__ uint2 lut[LUT_WORDS64];
-    const uint32_t lane_copy = (uint32_t)(threadIdx.x & (LUT_COPIES - 1)) * 8u;
-
-    const Unit<D, CPL, BLK> un(BH, sa.nseg);
-    const int bx = un.bx, lh = un.lh, c0 = un.c0;
-    const bool active = un.active;
     using Vec = typename G::Vec;
-    SegLoads<D, CPL, 4, AHEAD> s;
-    s.start(cache, zp, sc, al, be, tg, bx % H, bx, lh, un.seg, T, n_super_cap, sa);
+    constexpr int AHEAD = CPL == 2 ? PF_PAIR : PF;
     const bool last = s.last;
     const int t0 = s.t0, t1 = s.t1, nfull = s.nfull;
     Vec *cbh = s.cbh;
     const Vec *cb = s.cb;
     auto &buf = s.buf;
-    const h1 *wrow = attn + (size_t)bx * sa.row_pitch;
-    const h1 *wb = wrow + t0;
-    auto load_w = [&](int sg) {
-        uint4 r;
-        __builtin_memcpy(&r, wb + (size_t)sg * 8, 16); // row base is only 2-byte aligned
-        return r;
-    };
-    uint4 wbuf[AHEAD];
-    if (nfull > 0)
-#pragma unroll
-        for (int i = 0; i < AHEAD; i++)
-            wbuf[i] = load_w(min(i, nfull - 1));
-    lut_fill<BLK>(lut, threadIdx.x);
-    __syncthreads();
-    if (!un.wave_active)
-        return; // padding waves
-
     Pair st[G::NP];
-    float acc[CPL];
     s.state(st);
 #pragma unroll
     for (int c = 0; c < CPL; c++)
@@ -1411,18 +1394,18 @@ __global__ __launch_bounds__(BLK) void ov_kernel(
         if constexpr (MM) {
 #pragma unroll
             for (int t = 0; t < 8; t += 2)
-                token2(t, lk, nb, wbuf[i]);
+                token2(t, lk, nb, wbuf[i % WR]);
         } else {
             // a wave (nearly) alone on its SIMD: see replay_eight
 #pragma unroll
             for (int t = 0; t < 8; t++)
                 lk[(i & 1) ^ 1][t] = lut_get(lut, nb[0][t & 1], lane_copy, t >> 1);
-            replay_eight_weighted(st[0], lk[i & 1], wbuf[i], acc);
+            replay_eight_weighted(st[0], lk[i & 1], wbuf[i % WR], acc);
             __builtin_amdgcn_sched_barrier(0);
         }
         // the weights are reloaded once their last token is done: loading them earlier into a
         // second register set costs copies at the loop edge, which wait for the load they move
-        wbuf[i] = load_w(sgp);
+        wbuf[i % WR] = w8(min(sg + WR, nfull - 1));
     };
     rotate_over<AHEAD>(nfull, body);
     if (MM) {
@@ -1449,7 +1432,7 @@ __global__ __launch_bounds__(BLK) void ov_kernel(
                         const h2 qc = codes_to_h2((int)na - 8, (int)nbb - 8);
                         const h2 qs = qc * s.sc;
                         const h2 vd = qs + s.zp;
-                        const float wt = (float)wb[nfull * 8 + tt];
+                        const float wt = (float)w1(nfull * 8 + tt);
                         const int c = G::WPV * v + 2 * pp;
                         acc[c] = __builtin_fmaf(wt, (float)vd.x, acc[c]);
                         acc[c + 1] = __builtin_fmaf(wt, (float)vd.y, acc[c + 1]);
@@ -1463,13 +1446,54 @@ __global__ __launch_bounds__(BLK) void ov_kernel(
 
         h2 deq[G::NP];
         append_new_token<D, CPL>(cbh, T, v_new + (size_t)bx * D + c0, st, deq, active, sa.act_bf16);
-        const float wT = (float)wrow[T];
+        const float wT = (float)w1(T - t0);
 #pragma unroll
         for (int p = 0; p < G::NP; p++) {
             acc[2 * p] = __builtin_fmaf(wT, (float)deq[p].x, acc[2 * p]);
             acc[2 * p + 1] = __builtin_fmaf(wT, (float)deq[p].y, acc[2 * p + 1]);
         }
     }
+}
+
+template <int D, int CPL, int BLK>
+__global__ __launch_bounds__(BLK) void ov_kernel(
+    const h1 *attn, uint4 *__restrict__ cache, const h1 *v_new,
+    h1 *__restrict__ out, float *__restrict__ partial,
+    const h1 *zp, const h1 *sc, const h1 *al,
+    const h1 *be, const h1 *tg,
+    int BH, int H, int T, int n_super_cap, h1 *__restrict__ state_out, Seg sa)
+{
+    using G = Geo<D, CPL>;
+    constexpr int AHEAD = CPL == 2 ? PF_PAIR : PF;
+    sa.groups = 0; // only even plans come here
+    __shared__ uint2 lut[LUT_WORDS64];
+    const uint32_t lane_copy = (uint32_t)(threadIdx.x & (LUT_COPIES - 1)) * 8u;
+
+    const Unit<D, CPL, BLK> un(BH, sa.nseg);
+    const int bx = un.bx, lh = un.lh, c0 = un.c0;
+    const bool active = un.active;
+    SegLoads<D, CPL, 4, AHEAD> s;
+    s.start(cache, zp, sc, al, be, tg, bx % H, bx, lh, un.seg, T, n_super_cap, sa);
+    const int nfull = s.nfull;
+    const h1 *wb = attn + (size_t)bx * sa.row_pitch + s.t0;
+    auto load_w = [&](int sg) {
+        uint4 r;
+        __builtin_memcpy(&r, wb + (size_t)sg * 8, 16); // row base is only 2-byte aligned
+        return r;
+    };
+    uint4 wbuf[AHEAD];
+    if (nfull > 0)
+#pragma unroll
+        for (int i = 0; i < AHEAD; i++)
+            wbuf[i] = load_w(min(i, nfull - 1));
+    lut_fill<BLK>(lut, threadIdx.x);
+    __syncthreads();
+    if (!un.wave_active)
+        return; // padding waves
+
+    float acc[CPL];
+    ov_segment<D, CPL, AHEAD>(lut, lane_copy, bx, c0, active, s, wbuf, load_w, [&](int t) { return wb[t]; }, v_new, T,
+                              state_out, sa, acc);
     if (!active)
         return;
     if (sa.nseg == 1) {
@@ -1988,6 +2012,7 @@ static inline int lanes_per_head(int D) { return D == 128 ? 32 : 64; }
 #include "adkv_gqa_kernels.h"
 #include "adkv_ft_kernels.h"
 #include "adkv_small_step.h"
+#include "adkv_segment_step.h"
 
 // Waves a SIMD should hold for packed-f16 issue to run near full rate, and SIMDs on the device.
 constexpr int WAVES_PER_SIMD_TARGET = 4;
@@ -2486,6 +2511,85 @@ static bool small_step_plan(Seg &seg, int B, int Hq, int H, int T, int D, int bi
         return false;
     seg = plan_segments(k_ckpt, n_ckpt_cap, ckpt_interval, B * H, T, D);
     return seg.nseg <= 4;
+}
+
+// Whether a step runs as step_segments_kernel + step_combine_kernel, its plan and its channels per lane.
+// Every segment has to fit the LDS of its wave and all waves have to be resident: at most four per SIMD
+// (two with 184 registers at head dim 512).  us per step on the device, three to four launches / two,
+// sequences x query heads x KV heads x tokens (4-bit, head dim 128, checkpoints every 256 unless said):
+// 1 x 32 x 8 x 603 50.8 / 21.9, 4 x 32 x 8 x 3000 51.3 / 24.2, 8 x 32 x 8 x 16001 (bf16, with the rotary embedding)
+// 65.6 / 58.0, 2 x 64 x 8 x 4000 2-bit 54.8 / 25.1, 1 x 32 x 32 x 2000 28.1 / 20.7, 16 x 32 x 32 x 1500 55.3 /
+// 40.4, 64 x 32 x 32 x 663 masked (bf16, with the rotary embedding) 74.3 / 66.0; head dim 256, 16 x 16 heads x
+// 4000 93.6 / 90.0, 1 x 8 x 1000 34.5 / 30.6; head dim 512, 8 x 8 x 2000 57.3 / 50.1.
+// With one query head two channels per lane are taken as long as four waves per SIMD hold them (12 x 32 heads x
+// 2000 tokens: 48.4 with four channels, 40.6 with two), four beyond.
+// Segments cut finer than 128 tokens (by checkpoints closer than that) with one query head per KV head stay
+// with the separate launches: such a step is the three calls bit for bit, where here a weight is rounded
+// before it is divided by its row's sum, at 15.0 us instead of 11.0 (2 x 3 heads x 530, every 64).
+static bool segment_step_plan(Seg &seg, int &cpl, int B, int Hq, int H, int T, int D, int bits, void *k_ckpt, void *v_ckpt,
+                              int n_ckpt_cap, int ckpt_interval)
+{
+    const int GQ = Hq / H;
+    if ((GQ != 1 && GQ != 2 && GQ != 4 && GQ != 8) || (bits != 4 && bits != 2) || !k_ckpt != !v_ckpt ||
+        g_mha_kernel.load(std::memory_order_relaxed) >= 0 || mha_kernel_default())
+        return false;
+    const int BH = B * H;
+    seg = plan_segments(k_ckpt, n_ckpt_cap, ckpt_interval, BH, T, D);
+    const int longest = seg.nseg > 1 ? seg.seg_tokens : T;
+    if (longest + 1 > (GQ == 8 ? step_cap<8>() : step_cap<1>()) || (GQ == 1 && bits == 4 && seg.nseg > 1 && longest < 128))
+        return false;
+    const long room = (D == 512 ? 2L : 4L) * n_simd();
+    cpl = D == 512 ? 8 : D == 256 ? 4 : 2;
+    long waves = padded_units<64>(BH, seg.nseg);
+    if (waves > room && GQ == 1 && bits == 4 && D == 128) {
+        cpl = 4;
+        waves = padded_units<32>(BH, seg.nseg) / 2;
+    }
+    return waves <= room;
+}
+
+template <int D, int CPL, int BITS, int GQ, typename... Args>
+static int launch_step_shape(long waves, hipStream_t st, Args... args)
+{
+    const long per_cu = (waves + cus() - 1) / cus();
+#define ADKV_STEP(BLK)                                                                              \
+    hipLaunchKernelGGL((step_segments_kernel<D, CPL, BITS, GQ, BLK>), dim3((unsigned)((waves * 64 + BLK - 1) / BLK)), dim3(BLK), 0, st, args...)
+    if (per_cu <= 4) {
+        ADKV_STEP(256);
+    } else if (D == 512 || per_cu <= 8) {
+        ADKV_STEP(512);
+    } else if constexpr (D != 512) { // 184 registers: at most two waves per SIMD
+        if (per_cu <= 12)
+            ADKV_STEP(768);
+        else
+            ADKV_STEP(1024);
+    }
+#undef ADKV_STEP
+    return check_launch();
+}
+
+template <int BITS, typename... Args>
+static int launch_step_grouped(int GQ, long waves, hipStream_t st, Args... args)
+{
+    switch (GQ) {
+    case 1: return launch_step_shape<128, 2, BITS, 1>(waves, st, args...);
+    case 2: return launch_step_shape<128, 2, BITS, 2>(waves, st, args...);
+    case 4: return launch_step_shape<128, 2, BITS, 4>(waves, st, args...);
+    default: return launch_step_shape<128, 2, BITS, 8>(waves, st, args...);
+    }
+}
+
+template <typename... Args>
+static int launch_step_segments(int cpl, int GQ, int bits, int D, int BH, int nseg, hipStream_t st, Args... args)
+{
+    const long units = padded_units<64>(BH, nseg);
+    if (D == 512)
+        return launch_step_shape<512, 8, 4, 1>(units, st, args...);
+    if (D == 256)
+        return launch_step_shape<256, 4, 4, 1>(units, st, args...);
+    if (cpl == 4)
+        return launch_step_shape<128, 4, 4, 1>(padded_units<32>(BH, nseg) / 2, st, args...);
+    return bits == 4 ? launch_step_grouped<4>(GQ, units, st, args...) : launch_step_grouped<2>(GQ, units, st, args...);
 }
 
 static int check_ckpt(const void *ckpt, int n_ckpt_cap, int ckpt_interval, int bits = 4)
@@ -3323,8 +3427,13 @@ int64_t adkv_decode_step_workspace_bytes(int B, int Hq, int H, int T, int D, int
     if (B <= 0 || H <= 0 || Hq <= 0 || T < 0)
         return 0;
     const int64_t mat = pad256((int64_t)B * Hq * adkv_row_pitch(T + 1) * 2);
-    return 2 * mat + pad256(adkv_softmax_workspace_bytes(B * Hq, T + 1)) +
-           adkv_forward_ov_gqa_workspace_bytes(B, Hq, H, T, D, n_ckpt_cap, ckpt_interval);
+    const int64_t ov = adkv_forward_ov_gqa_workspace_bytes(B, Hq, H, T, D, n_ckpt_cap, ckpt_interval);
+    // a step in two launches leaves a maximum, two sums and D partial outputs per row and segment
+    int dummy = 0;
+    const int64_t nseg = H > 0 ? plan_segments(n_ckpt_cap > 0 && ckpt_interval > 0 ? &dummy : nullptr, n_ckpt_cap, ckpt_interval,
+                                               B * H, T, D).nseg : 1;
+    const int64_t step = pad256(nseg * B * Hq * 16) + nseg * B * Hq * D * 4;
+    return 2 * mat + std::max(pad256(adkv_softmax_workspace_bytes(B * Hq, T + 1)) + ov, step);
 }
 
 static FtParams ft_params(const void *const *p)
@@ -3332,17 +3441,18 @@ static FtParams ft_params(const void *const *p)
     return {(const h1 *)p[0], (const h1 *)p[1], (const h1 *)p[2], (const h1 *)p[3], (const h1 *)p[4]};
 }
 
-// What forward_qk and forward_ov would refuse, for the steps that run as one launch (4-bit codes, one
-// query head per KV head).
+// What forward_qk and forward_ov would refuse, for the steps that run otherwise.
 static int check_step(const void *q, const void *k_cache, const void *v_cache, const void *k_new, const void *v_new,
                       const void *const *k_params, const void *const *v_params, const void *out, const void *weights, int B,
-                      int H, int T, int D, int n_super_cap, int bits, const void *k_ckpt, const void *v_ckpt, int n_ckpt_cap,
-                      int ckpt_interval)
+                      int Hq, int H, int T, int D, int n_super_cap, int bits, const void *k_ckpt, const void *v_ckpt,
+                      int n_ckpt_cap, int ckpt_interval)
 {
     int rc = check_common(B, H, T, D, n_super_cap);
     if (rc)
         return rc;
-    if (T / 8 >= n_super_cap)
+    if ((Hq > H || bits != 4) && D != 128)
+        return ADKV_E_UNSUPPORTED;
+    if (T / (32 / bits) >= n_super_cap)
         return ADKV_E_CAPACITY;
     if (!q || !k_cache || !v_cache || !k_new || !v_new || !out)
         return ADKV_E_NULL;
@@ -3394,7 +3504,7 @@ int adkv_decode_step(const void *q, void *k_cache, void *v_cache, const void *k_
         Seg ka, va;
         const int lanes = mask ? 0 : fused_step_plan(ka, va, B, Hq, H, T, D, bits, k_ckpt, v_ckpt, n_ckpt_cap, ckpt_interval);
         if (lanes) {
-            if ((rc = check_step(q, k_cache, v_cache, k_new, v_new, k_params, v_params, out, weights, B, H, T, D, n_super_cap,
+            if ((rc = check_step(q, k_cache, v_cache, k_new, v_new, k_params, v_params, out, weights, B, Hq, H, T, D, n_super_cap,
                                  bits, k_ckpt, v_ckpt, n_ckpt_cap, ckpt_interval)))
                 return rc;
             ka.row_pitch = va.row_pitch = ld;
@@ -3411,7 +3521,7 @@ int adkv_decode_step(const void *q, void *k_cache, void *v_cache, const void *k_
     {
         Seg ka;
         if (small_step_plan(ka, B, Hq, H, T, D, bits, k_ckpt, v_ckpt, n_ckpt_cap, ckpt_interval)) {
-            if ((rc = check_step(q, k_cache, v_cache, k_new, v_new, k_params, v_params, out, weights, B, H, T, D, n_super_cap,
+            if ((rc = check_step(q, k_cache, v_cache, k_new, v_new, k_params, v_params, out, weights, B, Hq, H, T, D, n_super_cap,
                                  bits, k_ckpt, v_ckpt, n_ckpt_cap, ckpt_interval)))
                 return rc;
             if (mask && rows_per_mask_row <= 0)
@@ -3426,6 +3536,38 @@ int adkv_decode_step(const void *q, void *k_cache, void *v_cache, const void *k_
                                mask ? rows_per_mask_row : 1, (h1 *)weights, (h1 *)out, kp, vp, H, T,
                                n_super_cap, scaling, ka, va);
             return (rc = check_launch()) ? rc : mark_one_launch(stream);
+        }
+    }
+    {
+        Seg ka;
+        int cpl;
+        if (segment_step_plan(ka, cpl, B, Hq, H, T, D, bits, k_ckpt, v_ckpt, n_ckpt_cap, ckpt_interval)) {
+            if ((rc = check_step(q, k_cache, v_cache, k_new, v_new, k_params, v_params, out, weights, B, Hq, H, T, D, n_super_cap,
+                                 bits, k_ckpt, v_ckpt, n_ckpt_cap, ckpt_interval)))
+                return rc;
+            if (mask && rows_per_mask_row <= 0)
+                return ADKV_E_SHAPE;
+            ka.row_pitch = ld;
+            ka.act_bf16 = act_bf16;
+            Seg va = ka;
+            va.ckpt = (h1 *)v_ckpt;
+            const long rows = (long)B * Hq;
+            const StepMask mk = {(const float *)mask, mask ? rows_per_mask_row : 1};
+            float4 *ml = (float4 *)(ws + 2 * mat);
+            float *partial = (float *)(ws + 2 * mat + pad256(ka.nseg * rows * 16));
+            if ((rc = launch_step_segments(cpl, Hq / H, bits, D, B * H, ka.nseg, (hipStream_t)stream, (const h1 *)q, (uint4 *)k_cache,
+                                           (const h1 *)k_new, (uint4 *)v_cache, (const h1 *)v_new, mk, (h1 *)logits, partial, ml,
+                                           ft_params(k_params), ft_params(v_params), B * H, H, T, n_super_cap, scaling, ka, va)))
+                return rc;
+            for (int i = 1; i <= 2; i++)
+                if ((rc = stage_mark(i, stream)))
+                    return rc;
+            const int out_waves = ka.nseg > 16 ? D / 16 : D / 128;
+            const long waves = rows * ((T + 1 + 511) / 512 + out_waves);
+            hipLaunchKernelGGL(step_combine_kernel, dim3((unsigned)((waves + 3) / 4)), dim3(256), 0, (hipStream_t)stream,
+                               (const h1 *)logits, (h1 *)weights, (h1 *)out, mk, partial, ml, rows, T + 1, (long)ld, D, ka.nseg,
+                               scaling, out_waves, act_bf16);
+            return (rc = check_launch()) ? rc : stage_mark(3, stream);
         }
     }
     rc = forward_qk_impl(q, k_cache, k_new, logits, k_params[0], k_params[1], k_params[2],

@@ -278,10 +278,12 @@ int adkv_forward_ov_noalloc(const void *attn, void *v_cache, const void *v_new, 
  * One decode-attention step of one layer in a single library call: the launches of forward_qk,
  * scale/mask/softmax and forward_ov (plus the sum of forward_ov's segments) issued back to back
  * on `stream`, appending k_new / v_new at slot T of both caches.  It is one CALL, not one kernel:
- * logits and weights pass through the workspace between the launches.  (A single kernel was
- * evaluated and not built: the softmax arithmetic costs the same vector instructions wherever it
- * runs, these kernels are bound by vector-instruction issue and not by the logits' round trip, and
- * the per-head table that the QK and OV kernels each build needs the whole LDS of a CU for itself.)
+ * logits and weights pass through the workspace between the launches.  Steps that are not the big launches
+ * of long segments run as fewer: few short sequences in one, segments of up to 512 tokens in two,
+ * one that takes every segment through keys, softmax and values and one that puts the segments
+ * together.  In two launches a weight is rounded to fp16 relative to its segment's largest before the
+ * division by its row's sum, after it otherwise, so outputs agree to about an fp16 ulp of the weights;
+ * codes, state and checkpoints are identical.
  * Replaces the body of KVCacheLayer_ADKV.decode (src/adkv/hf/llama_adkv.py:245-276).
  * q: fp16 [B, Hq, D] with Hq a multiple of the H KV heads (Hq == H is the reference's case).
  * k_params / v_params: host arrays of five device pointers {zp, sc, alpha, beta, tgt}, each
@@ -329,7 +331,8 @@ int adkv_decode_segments(int B, int Hq, int H, int T, int D, int bits, int n_ckp
  * THIS host thread records them on its stream: [0] before the QK launch, [1] after it, [2] after
  * the softmax, [3] after the OV launch and the sum of its segments, so the stages of the product
  * path can be timed without taking it apart.  What a call launches does not depend on the hook: a step
- * that is one launch (adkv_decode_step_is_fused) records [0] before it and the other three after it.
+ * that is one launch (adkv_decode_step_is_fused) records [0] before it and the other three after it, a step
+ * of short segments [1] and [2] between its two launches.
  */
 void adkv_set_stage_events(void *const *events);
 
