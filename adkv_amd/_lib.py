@@ -86,6 +86,25 @@ def lib() -> C.CDLL:
     return _lib
 
 
+_host = None
+
+
+def host():
+    """The module of the host calls (csrc/host_calls.cpp).  Like the library, it has to be there."""
+    global _host
+    if _host is None:
+        lib()
+        try:
+            from . import _host as module
+        except ImportError as e:
+            raise ADKVLibraryError(f"adkv_amd/_host.so is missing or does not load ({e}): build it with "
+                                   "`python -m adkv_amd.build`.") from e
+        module.init(_raw_stream if _raw_stream is not None else
+                    lambda index: torch.cuda.current_stream(index).cuda_stream)
+        _host = module
+    return _host
+
+
 def check(rc: int, what: str) -> None:
     if rc != 0:
         L = lib()

@@ -114,14 +114,9 @@ constexpr unsigned pack_skew(unsigned a, unsigned b, unsigned c, unsigned d) { r
 // takes the group's last segment (the longest), the youngest its first (see segment_of_slot).
 // Needs at least four intervals per group.  The same function plans on the host and indexes on
 // the device.
-__host__ __device__ inline int uneven_cut(int seg, int groups, int intervals, unsigned skew)
+__host__ __device__ inline void uneven_parts(int n, unsigned skew, int *part) // of a group of n intervals, by wave slot, oldest first
 {
-    const int g = seg >> 2, k = seg & 3;
-    const int lo = (int)((long)intervals * g / groups);
-    if (k == 0)
-        return lo;
-    const int n = (int)((long)intervals * (g + 1) / groups) - lo;
-    int part[4], left = n; // by wave slot, oldest first
+    int left = n;
     for (int i = 0; i < 4; i++) {
         part[i] = n * ft_skew(skew, i) / 16;
         if (part[i] < 1)
@@ -135,6 +130,15 @@ __host__ __device__ inline int uneven_cut(int seg, int groups, int intervals, un
             part[i]--;
             left++;
         }
+}
+__host__ __device__ inline int uneven_cut(int seg, int groups, int intervals, unsigned skew)
+{
+    const int g = seg >> 2, k = seg & 3;
+    const int lo = (int)((long)intervals * g / groups);
+    if (k == 0)
+        return lo;
+    int part[4];
+    uneven_parts((int)((long)intervals * (g + 1) / groups) - lo, skew, part);
     int c = lo;
     for (int i = 0; i < k; i++)
         c += part[3 - i];
@@ -2066,8 +2070,9 @@ static Seg plan_segments(void *ckpt, int n_ckpt_cap, int ckpt_interval, int BH, 
     if (!ckpt || ckpt_interval <= 0 || T <= ckpt_interval)
         return s;
     const int avail = (T + ckpt_interval - 1) / ckpt_interval;               // finest split
+    const int n_cus = cus(); // asks the runtime for the device: once per plan
     const int lph = lanes ? lanes : lanes_per_head(D); // lanes: 16 for the two-pass per-head-table kernels
-    const long units_target = (long)n_simd() * WAVES_PER_SIMD_TARGET * (64 / lph);
+    const long units_target = 4L * n_cus * WAVES_PER_SIMD_TARGET * (64 / lph);
     long want = (units_target + BH - 1) / BH;
     if (want < 1)
         want = 1;
@@ -2080,10 +2085,10 @@ static Seg plan_segments(void *ckpt, int n_ckpt_cap, int ckpt_interval, int BH, 
     auto cost = [&](int m) {
         const int nseg = (avail + m - 1) / m;
         const long threads = (lph == 16 ? padded_units<16>(BH, nseg) : lph == 32 ? padded_units<32>(BH, nseg) : padded_units<64>(BH, nseg)) * lph;
-        if (D == 512 || threads < 1024L * cus())
+        if (D == 512 || threads < 1024L * n_cus)
             return (double)m;                        // small workgroups: no round structure to model
         const long wgs = (threads + 1023) / 1024;
-        return (double)((wgs + cus() - 1) / cus()) * m;
+        return (double)((wgs + n_cus - 1) / n_cus) * m;
     };
     int best = -1;
     double best_cost = 0.0;
@@ -2301,13 +2306,15 @@ constexpr int FT_MAX_GROUPS = 16;
 
 // Longest segment of an uneven cut, in checkpoint intervals (the oldest wave slot's of the group
 // that got the most intervals).
+// The groups have intervals / groups intervals, rounded down or up, so two are looked at.
 static int uneven_longest(int groups, int intervals, unsigned skew)
 {
-    int longest = 0;
-    for (int g = 0; g < groups; g++) {
-        const int n = uneven_cut(4 * g + 4, groups, intervals, skew) - uneven_cut(4 * g + 3, groups, intervals, skew);
-        if (n > longest)
-            longest = n;
+    int part[4], longest;
+    uneven_parts(intervals / groups, skew, part);
+    longest = part[0];
+    if (intervals % groups) {
+        uneven_parts(intervals / groups + 1, skew, part);
+        longest = std::max(longest, part[0]);
     }
     return longest;
 }
@@ -2326,6 +2333,7 @@ constexpr int FT_UNIT_OVERHEAD_TOKENS = 32;
 static void plan_head_table(Seg &seg, int B, int H, int T, unsigned skew, int upw, bool virtual_ok = true)
 {
     seg.groups = 0;
+    const int n_cus = cus(); // asks the runtime for the device: once per plan
     seg.skew = skew;
     seg.phys_per_head = ft_wgs_per_head(B, seg.nseg, upw);
     if (!seg.ckpt || seg.ckpt_interval <= 0 || skew == 0)
@@ -2344,7 +2352,7 @@ static void plan_head_table(Seg &seg, int B, int H, int T, unsigned skew, int up
         const int W = ft_wgs_per_head(B, 4 * G, upw);
         const double unit = (double)uneven_longest(G, avail, skew) * iv + FT_UNIT_OVERHEAD_TOKENS;
         for (int P = virtual_ok ? 1 : W; P <= W; P++) {
-            const double cost = (double)(((long)H * P + cus() - 1) / cus()) * ((W + P - 1) / P) * unit;
+            const double cost = (double)(((long)H * P + n_cus - 1) / n_cus) * ((W + P - 1) / P) * unit;
             if (best_cost < 0.0 || cost < 0.999 * best_cost) {
                 best_g = G;
                 best_p = P;

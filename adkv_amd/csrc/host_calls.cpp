@@ -1,0 +1,381 @@
+// The library calls of an attention layer, and of the fp32 quantiser, from Python without Python: rotary embedding,
+// attention of one token, quantising of new tokens.  On few sequences a step is over on the device in some 20 us,
+// and the checks, views, allocations and argument conversions of the Python functions took twice that on the host
+// (1 x 32 heads x 603 tokens: 38.2 us per step, now 21.0 and bound by the device).
+//
+// Each function here takes exactly the arguments that need nothing done to them first (plain device tensors
+// of one current device, of the right shapes, dtypes and layouts, a workspace that is large enough) and
+// returns None for all others: the Python function that called it then goes its own way, with its own
+// conversions and error messages.  A number is the library's return code.
+#include <torch/csrc/autograd/python_variable.h>
+
+#include <ATen/ATen.h>
+#include <ATen/PythonTorchFunctionTLS.h>
+#include <c10/core/impl/LocalDispatchKeySet.h>
+#include <c10/core/impl/DeviceGuardImplInterface.h>
+
+#include "../../include/adkv_hip.h"
+
+namespace {
+
+PyObject *raw_stream = nullptr; // device index -> the current stream as a number
+
+// An ordinary tensor of an ordinary device: no subclass, no transform, no pending negation, no other backend.
+const at::Tensor *plain(PyObject *o)
+{
+    static const c10::DispatchKeySet allowed =
+        c10::DispatchKeySet(c10::DispatchKey::CUDA) | c10::DispatchKeySet(c10::DispatchKey::ADInplaceOrView) |
+        c10::getAutogradRelatedKeySetFromBackend(c10::BackendComponent::CUDABit) |
+        c10::getAutocastRelatedKeySetFromBackend(c10::BackendComponent::CUDABit);
+    if (!THPVariable_CheckExact(o))
+        return nullptr;
+    const at::Tensor &t = THPVariable_Unpack(o);
+    return t.defined() && t.is_cuda() && (t.key_set() | allowed) == allowed ? &t : nullptr;
+}
+
+// Nothing watches or transforms what this thread does with tensors: no mode, no tracer, no functorch layer.
+bool unwatched()
+{
+    static const c10::DispatchKeySet ordinary = c10::default_included_set |
+                                                c10::DispatchKeySet(c10::DispatchKey::ADInplaceOrView) |
+                                                c10::DispatchKeySet(c10::DispatchKey::BackendSelect);
+    return (c10::impl::tls_local_dispatch_key_set().included_ | ordinary) == ordinary && !at::impl::torch_function_mode_enabled();
+}
+
+bool half_type(const at::Tensor &t) { return t.scalar_type() == at::kHalf || t.scalar_type() == at::kBFloat16; }
+
+// whether `device` is the thread's current one; its current stream
+bool current(c10::Device device, void *&stream)
+{
+    if (c10::impl::getDeviceGuardImpl(c10::DeviceType::CUDA)->getDevice() != device)
+        return false;
+    PyObject *i = PyLong_FromLong(device.index());
+    PyObject *s = i ? PyObject_CallOneArg(raw_stream, i) : nullptr;
+    Py_XDECREF(i);
+    if (!s) {
+        PyErr_Clear();
+        return false;
+    }
+    stream = PyLong_AsVoidPtr(s);
+    Py_DECREF(s);
+    if (PyErr_Occurred()) {
+        PyErr_Clear();
+        return false;
+    }
+    return true;
+}
+
+PyObject *pair(at::Tensor &&a, at::Tensor &&b)
+{
+    PyObject *x = THPVariable_Wrap(std::move(a)), *y = THPVariable_Wrap(std::move(b));
+    PyObject *r = x && y ? PyTuple_Pack(2, x, y) : nullptr;
+    Py_XDECREF(x);
+    Py_XDECREF(y);
+    return r;
+}
+
+// rows read in place: channels contiguous, even strides, 4-byte aligned base
+bool rows(const at::Tensor &t)
+{
+    const auto st = t.strides();
+    for (size_t i = 0; i + 1 < st.size(); i++)
+        if (st[i] % 2)
+            return false;
+    return st.back() == 1 && (uintptr_t)t.const_data_ptr() % 4 == 0;
+}
+
+// rope_qk(q, k, cos, sin)
+PyObject *rope_qk(PyObject *, PyObject *const *args, Py_ssize_t n)
+{
+    if (n != 4 || !unwatched())
+        Py_RETURN_NONE;
+    const at::Tensor *t[4];
+    for (int i = 0; i < 4; i++)
+        if (!(t[i] = plain(args[i])) || t[i]->scalar_type() != t[0]->scalar_type() || t[i]->device() != t[0]->device())
+            Py_RETURN_NONE;
+    const at::Tensor &q = *t[0], &k = *t[1], &c = *t[2], &s = *t[3];
+    if (!half_type(q) || q.dim() != 4 || k.dim() != 4 || c.dim() != 3 || s.dim() != 3)
+        Py_RETURN_NONE;
+    const int64_t B = q.size(0), Hq = q.size(1), T = q.size(2), D = q.size(3), H = k.size(1);
+    if (k.size(0) != B || k.size(2) != T || k.size(3) != D || c.sizes() != s.sizes() || c.strides() != s.strides() ||
+        c.size(1) != T || c.size(2) != D || (c.size(0) != 1 && c.size(0) != B) || D % 4 || B * Hq * T * D <= 0 || H <= 0 ||
+        B * std::max(Hq, H) * T > INT32_MAX || !rows(q) || !rows(k) || !rows(c) || !rows(s))
+        Py_RETURN_NONE;
+    void *stream;
+    if (!current(q.device(), stream))
+        Py_RETURN_NONE;
+    at::Tensor qo, ko;
+    int rc;
+    try {
+        qo = at::empty({B, Hq, T, D}, q.options());
+        ko = at::empty({B, H, T, D}, q.options());
+        if (!qo.has_storage() || !ko.has_storage())
+            Py_RETURN_NONE;
+        void *qp = qo.mutable_data_ptr(), *kp = ko.mutable_data_ptr();
+        Py_BEGIN_ALLOW_THREADS
+        rc = adkv_rope_qk(q.const_data_ptr(), k.const_data_ptr(), c.const_data_ptr(), s.const_data_ptr(), qp, kp, (int)B, (int)Hq,
+                          (int)H, (int)T, (int)D, q.stride(0), q.stride(1), q.stride(2), k.stride(0), k.stride(1), k.stride(2),
+                          c.size(0) == B && B > 1 ? c.stride(0) : 0, c.stride(1), q.scalar_type() == at::kBFloat16, stream);
+        Py_END_ALLOW_THREADS
+    } catch (const std::exception &) {
+        Py_RETURN_NONE; // out of memory, or a mode that allocates otherwise: the Python function meets it too
+    }
+    return rc ? PyLong_FromLong(rc) : pair(std::move(qo), std::move(ko));
+}
+
+// n contiguous tensors of `type` and `numel` elements each on `device` in a tuple -> their addresses
+bool pointers(PyObject *tuple, Py_ssize_t n, at::ScalarType type, int64_t numel, c10::Device device, const void **out)
+{
+    if (!PyTuple_CheckExact(tuple) || PyTuple_GET_SIZE(tuple) != n)
+        return false;
+    for (Py_ssize_t i = 0; i < n; i++) {
+        const at::Tensor *p = plain(PyTuple_GET_ITEM(tuple, i));
+        if (!p || p->scalar_type() != type || p->numel() != numel || !p->is_contiguous() || p->device() != device)
+            return false;
+        out[i] = p->const_data_ptr();
+    }
+    return true;
+}
+
+// both checkpoint tensors [B, H, n, D, 2] or neither
+bool checkpoints(PyObject *const *args, int64_t B, int64_t H, int64_t D, long interval, long bits, c10::Device device, void **ck,
+                 int64_t &n)
+{
+    ck[0] = ck[1] = nullptr;
+    n = 0;
+    if (args[0] == Py_None && args[1] == Py_None)
+        return true;
+    for (int i = 0; i < 2; i++) {
+        const at::Tensor *c = plain(args[i]);
+        if (!c || c->scalar_type() != at::kHalf || c->dim() != 5 || c->size(0) != B || c->size(1) != H || c->size(2) < 1 ||
+            c->size(2) > INT32_MAX || c->size(3) != D || c->size(4) != 2 || !c->is_contiguous() || c->device() != device ||
+            (i && c->size(2) != n) || interval <= 0 || interval % (32 / bits) || interval > INT32_MAX)
+            return false;
+        n = c->size(2);
+        ck[i] = c->mutable_data_ptr();
+    }
+    return true;
+}
+
+// decode(q, k_new, v_new, params (ten), key codes, value codes, key checkpoints, value checkpoints, interval,
+//        bits, T, scaling, mask or None, workspaces {(device index, stream): uint8 tensor})
+PyObject *decode(PyObject *, PyObject *const *args, Py_ssize_t nargs)
+{
+    if (nargs != 14 || !unwatched() || !PyFloat_CheckExact(args[11]) ||
+        !PyDict_CheckExact(args[13]))
+        Py_RETURN_NONE;
+    const at::Tensor *qt = plain(args[0]), *kn = plain(args[1]), *vn = plain(args[2]), *kc = plain(args[4]), *vc = plain(args[5]);
+    if (!qt || !kn || !vn || !kc || !vc)
+        Py_RETURN_NONE;
+    const at::Tensor &q = *qt;
+    const long interval = PyLong_AsLong(args[8]), bits = PyLong_AsLong(args[9]), T = PyLong_AsLong(args[10]);
+    if (PyErr_Occurred()) {
+        PyErr_Clear();
+        Py_RETURN_NONE;
+    }
+    if (!half_type(q) || kn->scalar_type() != q.scalar_type() || vn->scalar_type() != q.scalar_type() || q.dim() != 4 ||
+        kc->dim() != 6 || kc->scalar_type() != at::kByte || vc->scalar_type() != at::kByte || kc->sizes() != vc->sizes() ||
+        (bits != 2 && bits != 4) || T < 0 || T >= INT32_MAX)
+        Py_RETURN_NONE;
+    const int64_t B = q.size(0), Hq = q.size(1), D = q.size(3), H = kc->size(1), n_super = kc->size(2);
+    if (q.size(2) != 1 || B <= 0 || H <= 0 || kc->size(0) != B || kc->size(3) * 4 != D || kc->size(4) != 4 || kc->size(5) != 4 ||
+        Hq % H || (Hq / H != 1 && Hq / H != 2 && Hq / H != 4 && Hq / H != 8) || (D != 128 && D != 256 && D != 512) ||
+        ((Hq != H || bits != 4) && D != 128) || T / (32 / bits) >= n_super || n_super > INT32_MAX || B * Hq > INT32_MAX)
+        Py_RETURN_NONE;
+    const int64_t token[4] = {B, H, 1, D};
+    if (kn->sizes() != at::IntArrayRef(token) || vn->sizes() != at::IntArrayRef(token) || !q.is_contiguous() || !kn->is_contiguous() || !vn->is_contiguous() ||
+        !kc->is_contiguous() || !vc->is_contiguous())
+        Py_RETURN_NONE;
+    for (const at::Tensor *t : {kn, vn, kc, vc})
+        if (t->device() != q.device())
+            Py_RETURN_NONE;
+    const void *params[10];
+    void *ck[2];
+    int64_t n_ckpt;
+    if (!pointers(args[3], 10, at::kHalf, H * D, q.device(), params) ||
+        !checkpoints(args + 6, B, H, D, interval, bits, q.device(), ck, n_ckpt))
+        Py_RETURN_NONE;
+    const int64_t n = T + 1;
+    const at::Tensor *mask = nullptr;
+    int rows_per_mask_row = 1;
+    if (args[12] != Py_None) {
+        mask = plain(args[12]);
+        if (!mask || mask->device() != q.device() || !at::isFloatingType(mask->scalar_type()) ||
+            (mask->dim() != 3 && !(mask->dim() == 4 && mask->size(2) == 1)) || mask->size(0) != B ||
+            (mask->size(1) != 1 && mask->size(1) != Hq) || mask->size(-1) != n)
+            Py_RETURN_NONE;
+        rows_per_mask_row = mask->size(1) == 1 ? (int)Hq : 1;
+    }
+    void *stream;
+    if (!current(q.device(), stream))
+        Py_RETURN_NONE;
+    PyObject *key = Py_BuildValue("(iN)", (int)q.device().index(), PyLong_FromVoidPtr(stream));
+    PyObject *w = key ? PyDict_GetItem(args[13], key) : nullptr; // borrowed
+    Py_XDECREF(key);
+    const at::Tensor *ws = w ? plain(w) : nullptr;
+    const int64_t need = adkv_decode_step_workspace_bytes((int)B, (int)Hq, (int)H, (int)T, (int)D, (int)n_ckpt, (int)interval);
+    if (!ws || ws->scalar_type() != at::kByte || ws->numel() < need || !ws->is_contiguous() || ws->device() != q.device())
+        Py_RETURN_NONE;
+    at::Tensor out, weights, m32, scratch = *ws; // held: another thread may replace the dictionary's entry
+    int rc;
+    try {
+        if (mask) {
+            m32 = mask->to(at::kFloat).contiguous();
+            if (!m32.has_storage())
+                Py_RETURN_NONE;
+        }
+        const int64_t pitch = adkv_row_pitch((int)n);
+        out = at::empty({B, Hq, D}, q.options());
+        weights = at::empty({B, Hq, pitch}, q.options().dtype(at::kHalf));
+        if (!out.has_storage() || !weights.has_storage())
+            Py_RETURN_NONE;
+        void *op = out.mutable_data_ptr(), *wp = weights.mutable_data_ptr();
+        const void *mp = mask ? m32.const_data_ptr() : nullptr;
+        const double scaling = PyFloat_AS_DOUBLE(args[11]);
+        Py_BEGIN_ALLOW_THREADS
+        rc = adkv_decode_step(q.const_data_ptr(), kc->mutable_data_ptr(), vc->mutable_data_ptr(), kn->const_data_ptr(),
+                              vn->const_data_ptr(), params, params + 5, mp, rows_per_mask_row, (float)scaling, op, wp, pitch, (int)B,
+                              (int)Hq, (int)H, (int)T, (int)D, (int)n_super, (int)bits,
+                              q.scalar_type() == at::kBFloat16 ? ADKV_DT_BF16 : ADKV_DT_F16, ck[0], ck[1], (int)n_ckpt, (int)interval,
+                              scratch.mutable_data_ptr(), scratch.numel(), stream);
+        Py_END_ALLOW_THREADS
+        const int64_t sizes[3] = {B, Hq, n}, strides[3] = {Hq * pitch, pitch, 1};
+        weights.unsafeGetTensorImpl()->set_sizes_and_strides(at::IntArrayRef(sizes), at::IntArrayRef(strides));
+    } catch (const std::exception &) {
+        Py_RETURN_NONE;
+    }
+    return rc ? PyLong_FromLong(rc) : pair(std::move(out), std::move(weights));
+}
+
+// append(key codes, value codes, k rows, v rows, key params (five), value params (five), T0, key state,
+//        value state, key checkpoints, value checkpoints, interval, bits, fresh)
+PyObject *append(PyObject *, PyObject *const *args, Py_ssize_t nargs)
+{
+    if (nargs != 14 || !unwatched())
+        Py_RETURN_NONE;
+    const at::Tensor *t[6];
+    const int at_arg[6] = {0, 1, 2, 3, 7, 8};
+    for (int i = 0; i < 6; i++)
+        if (!(t[i] = plain(args[at_arg[i]])) || t[i]->device() != t[0]->device())
+            Py_RETURN_NONE;
+    const at::Tensor &kc = *t[0], &vc = *t[1], &k = *t[2], &v = *t[3];
+    const long T0 = PyLong_AsLong(args[6]), interval = PyLong_AsLong(args[11]), bits = PyLong_AsLong(args[12]);
+    if (PyErr_Occurred()) {
+        PyErr_Clear();
+        Py_RETURN_NONE;
+    }
+    const bool fresh = args[13] == Py_True;
+    if (!half_type(k) || v.scalar_type() != k.scalar_type() || k.dim() != 4 || v.sizes() != k.sizes() || kc.dim() != 6 ||
+        kc.scalar_type() != at::kByte || vc.scalar_type() != at::kByte || kc.sizes() != vc.sizes() || !kc.is_contiguous() ||
+        !vc.is_contiguous() || (bits != 2 && bits != 4) || T0 < 0 || (fresh && T0 != 0))
+        Py_RETURN_NONE;
+    const int64_t B = k.size(0), H = k.size(1), n = k.size(2), D = k.size(3), n_super = kc.size(2), tps = 32 / bits;
+    if (B <= 0 || H <= 0 || n <= 0 || kc.size(0) != B || kc.size(1) != H || kc.size(3) * 4 != D || kc.size(4) != 4 ||
+        kc.size(5) != 4 || (D != 128 && D != 256 && D != 512) || (T0 + n + tps - 1) / tps > n_super || n_super * tps > INT32_MAX ||
+        B * H > INT32_MAX / D)
+        Py_RETURN_NONE;
+    int64_t strides[2][3];
+    for (int i = 0; i < 2; i++) {
+        const at::Tensor &x = *t[2 + i];
+        for (int j = 0; j < 3; j++)
+            strides[i][j] = x.stride(j);
+        if (!x.is_contiguous() && (!rows(x) || x.stride(2) < D || x.stride(0) < 0 || x.stride(1) < 0))
+            Py_RETURN_NONE;
+        const at::Tensor &st = *t[4 + i];
+        if (st.scalar_type() != at::kHalf || !st.is_contiguous() || st.numel() != B * H * D * 2)
+            Py_RETURN_NONE;
+    }
+    const void *kp[5], *vp[5];
+    void *ck[2], *stream;
+    int64_t n_ckpt;
+    if (!pointers(args[4], 5, at::kHalf, H * D, kc.device(), kp) || !pointers(args[5], 5, at::kHalf, H * D, kc.device(), vp) ||
+        !checkpoints(args + 9, B, H, D, interval, bits, kc.device(), ck, n_ckpt) || !current(kc.device(), stream))
+        Py_RETURN_NONE;
+    const int dtype = k.scalar_type() == at::kBFloat16 ? ADKV_DT_BF16 : ADKV_DT_F16;
+    const int64_t *ks = k.is_contiguous() ? nullptr : strides[0], *vs = v.is_contiguous() ? nullptr : strides[1];
+    const int iv = ck[0] ? (int)interval : 0;
+    void *out[4] = {kc.mutable_data_ptr(), vc.mutable_data_ptr(), t[4]->mutable_data_ptr(), t[5]->mutable_data_ptr()};
+    const void *in[2] = {k.const_data_ptr(), v.const_data_ptr()};
+    int rc;
+    Py_BEGIN_ALLOW_THREADS
+    rc = fresh ? adkv_prefill_kv_pair(out[0], out[1], in[0], in[1], dtype, ks, vs, kp, vp, (int)B, (int)H, (int)n, (int)D,
+                                      (int)n_super, (int)bits, out[2], out[3], ck[0], ck[1], (int)n_ckpt, iv, stream)
+               : adkv_append_kv_pair(out[0], out[1], in[0], in[1], dtype, ks, vs, kp, vp, (int)B, (int)H, (int)T0, (int)n, (int)D,
+                                     (int)n_super, (int)bits, out[2], out[3], ck[0], ck[1], (int)n_ckpt, iv, stream);
+    Py_END_ALLOW_THREADS
+    return PyLong_FromLong(rc);
+}
+
+// quant_f32(x, (alpha, beta, target, zp_init, sc_init), lower, upper, sc_min, sc_max, output_states)
+//   -> (xhat, zp sequence or None, sc sequence or None)
+PyObject *quant_f32(PyObject *, PyObject *const *args, Py_ssize_t nargs)
+{
+    if (nargs != 7 || !unwatched() || !PyFloat_CheckExact(args[4]) || !PyFloat_CheckExact(args[5]))
+        Py_RETURN_NONE;
+    const at::Tensor *x = plain(args[0]);
+    const long lower = PyLong_AsLong(args[2]), upper = PyLong_AsLong(args[3]);
+    if (PyErr_Occurred()) {
+        PyErr_Clear();
+        Py_RETURN_NONE;
+    }
+    if (!x || x->dim() != 3 || !x->is_contiguous() || (!half_type(*x) && x->scalar_type() != at::kFloat))
+        Py_RETURN_NONE;
+    const int64_t B = x->size(0), T = x->size(1), C = x->size(2);
+    const void *p[5];
+    void *stream;
+    if (B <= 0 || T <= 0 || C <= 0 || B > INT32_MAX || T > INT32_MAX || C > INT32_MAX || lower < INT32_MIN || upper > INT32_MAX ||
+        !pointers(args[1], 5, at::kFloat, C, x->device(), p) || !current(x->device(), stream))
+        Py_RETURN_NONE;
+    at::Tensor out, state, seq[2];
+    int rc;
+    try {
+        const auto f32 = x->options().dtype(at::kFloat);
+        out = at::empty({B, T, C}, x->options());
+        state = at::empty({2, B, C}, f32);
+        if (args[6] == Py_True)
+            for (at::Tensor &t : seq)
+                t = at::empty({B, T, C}, f32);
+        if (!out.has_storage() || !state.has_storage())
+            Py_RETURN_NONE;
+        void *op = out.mutable_data_ptr(), *zp = state.mutable_data_ptr(), *sc = (float *)zp + B * C;
+        void *sp[2] = {seq[0].defined() ? seq[0].mutable_data_ptr() : nullptr, seq[1].defined() ? seq[1].mutable_data_ptr() : nullptr};
+        const int type = x->scalar_type() == at::kFloat ? ADKV_DT_F32 : x->scalar_type() == at::kHalf ? ADKV_DT_F16 : ADKV_DT_BF16;
+        const double lo = PyFloat_AS_DOUBLE(args[4]), hi = PyFloat_AS_DOUBLE(args[5]);
+        Py_BEGIN_ALLOW_THREADS
+        rc = adkv_quant_f32(x->const_data_ptr(), op, nullptr, zp, sc, p[3], p[4], p[0], p[1], p[2], sp[0], sp[1], (int)B, (int)T, (int)C,
+                            T * C, C, type, (int)lower, (int)upper, (float)lo, (float)hi, stream);
+        Py_END_ALLOW_THREADS
+    } catch (const std::exception &) {
+        Py_RETURN_NONE;
+    }
+    if (rc)
+        return PyLong_FromLong(rc);
+    PyObject *o = THPVariable_Wrap(std::move(out));
+    PyObject *z = seq[0].defined() ? THPVariable_Wrap(std::move(seq[0])) : (Py_INCREF(Py_None), Py_None);
+    PyObject *c = seq[1].defined() ? THPVariable_Wrap(std::move(seq[1])) : (Py_INCREF(Py_None), Py_None);
+    PyObject *r = o && z && c ? PyTuple_Pack(3, o, z, c) : nullptr;
+    Py_XDECREF(o);
+    Py_XDECREF(z);
+    Py_XDECREF(c);
+    return r;
+}
+
+PyObject *init(PyObject *, PyObject *f)
+{
+    Py_INCREF(f);
+    Py_XSETREF(raw_stream, f);
+    Py_RETURN_NONE;
+}
+
+PyMethodDef methods[] = {
+    {"init", init, METH_O, "init(function from device index to raw stream)"},
+    {"rope_qk", (PyCFunction)(void (*)(void))rope_qk, METH_FASTCALL, nullptr},
+    {"decode", (PyCFunction)(void (*)(void))decode, METH_FASTCALL, nullptr},
+    {"append", (PyCFunction)(void (*)(void))append, METH_FASTCALL, nullptr},
+    {"quant_f32", (PyCFunction)(void (*)(void))quant_f32, METH_FASTCALL, nullptr},
+    {nullptr, nullptr, 0, nullptr}};
+PyModuleDef module = {PyModuleDef_HEAD_INIT, "_host", nullptr, -1, methods, nullptr, nullptr, nullptr, nullptr};
+
+} // namespace
+
+PyMODINIT_FUNC PyInit__host() { return PyModule_Create(&module); }

@@ -21,6 +21,7 @@ import math
 
 import torch
 
+from .. import _lib
 from ..kernel.gemv import append_kv_pair, decode_step, decode_step_workspace_bytes
 
 SCALE_MIN = math.exp(-4.0)  # kept for API parity; the fp16 recurrence never clamps
@@ -209,16 +210,13 @@ class KVCacheLayer_ADKV:
                        value_zp_init, value_scale_init, value_alpha, value_beta, value_quant_target,
                        fresh: bool = False):
         """Quantise ``[B, H, T, C]`` keys/values as tokens ``quant_len ..`` of the stream."""
-        v = self._view
-        S = self._ckpt_interval
         append_kv_pair(
             self._key_buf, self._value_buf,
             self._rows(key_states), self._rows(value_states),
-            (v(key_zp_init), v(key_scale_init), v(key_alpha), v(key_beta), v(key_quant_target)),
-            (v(value_zp_init), v(value_scale_init), v(value_alpha), v(value_beta),
-             v(value_quant_target)),
+            (key_zp_init, key_scale_init, key_alpha, key_beta, key_quant_target),
+            (value_zp_init, value_scale_init, value_alpha, value_beta, value_quant_target),
             self._quant_len, self._key_state, self._value_state,
-            k_ckpt=self._key_ckpt, v_ckpt=self._value_ckpt, ckpt_interval=S, bits=self._bits, fresh=fresh)
+            k_ckpt=self._key_ckpt, v_ckpt=self._value_ckpt, ckpt_interval=self._ckpt_interval, bits=self._bits, fresh=fresh)
         self._quant_len += key_states.shape[2]
 
     def prefill(self, key_states, value_states,
@@ -266,6 +264,19 @@ class KVCacheLayer_ADKV:
                scaling: float = 1.0) -> tuple[torch.Tensor, torch.Tensor]:
         """One causal decode step: attend over the cached tokens and the new one, append the new
         K/V codes, return ``(output [B,H,C] in the query's dtype, weights [B,H,ctx+1] fp16)``."""
+        ctx = self._quant_len
+        if self._key_buf is not None and ctx < self._cap_len:
+            r = _lib.host().decode(
+                query_states, key_states, value_states,
+                (key_zp_init, key_scale_init, key_alpha, key_beta, key_quant_target,
+                 value_zp_init, value_scale_init, value_alpha, value_beta, value_quant_target),
+                self._key_buf, self._value_buf, self._key_ckpt, self._value_ckpt, self._ckpt_interval, self._bits, ctx,
+                float(scaling), attention_mask, _workspaces)
+            if r is not None:      # None: something to check, convert, allocate or complain about below
+                if isinstance(r, int):
+                    _lib.check(r, "decode_step")
+                self._quant_len, self._state_valid = ctx + 1, False
+                return r
         B, Hq, Tq, C = query_states.shape
         H, Tk = key_states.shape[1], key_states.shape[2]
         if Tq != 1 or Tk != 1:
@@ -275,7 +286,6 @@ class KVCacheLayer_ADKV:
             raise ValueError("ADKV decode supports 1, 2, 4 or 8 query heads per KV head "
                              "(more than one only with head_dim 128)")
         self._check_geometry(B, H, C, query_states.device)
-        ctx = self._quant_len
         self._cap_buffers(ctx + 1)
 
         # fp16 and bf16 activations go in as they are; the kernels convert (see decode_step)

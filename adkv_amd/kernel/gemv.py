@@ -402,6 +402,11 @@ def append_kv_pair(
     ``fresh``: the caches, states and checkpoints are uninitialised memory (``torch.empty``) and the
     tokens are their first (``T0 == 0``); the launch also zeroes the slots and checkpoints past them.
     """
+    rc = _lib.host().append(k_cache, v_cache, k_new, v_new, tuple(k_params), tuple(v_params), T0, k_state, v_state,
+                            k_ckpt, v_ckpt, ckpt_interval, bits, fresh)
+    if rc is not None:      # None: something to check, convert or complain about below
+        _lib.check(rc, "append_kv_pair")
+        return
     _chk(k_new.dtype == v_new.dtype and k_new.dtype in (torch.float16, torch.bfloat16),
          "kv_new must be float16 or bfloat16 (K and V alike)")
     _chk(k_cache.dtype == torch.uint8 and v_cache.dtype == torch.uint8, "kv_cache must be uint8")
@@ -456,6 +461,11 @@ def rope_qk(q: torch.Tensor, k: torch.Tensor, cos: torch.Tensor, sin: torch.Tens
     type; ``cos`` / ``sin``: ``[B, T, D]`` (or ``[1, T, D]``).  Any batch / head / token strides with
     contiguous channels are read in place; the results are contiguous.
     """
+    r = _lib.host().rope_qk(q, k, cos, sin)      # None: something to check, convert or complain about below
+    if r is not None:
+        if isinstance(r, int):
+            _lib.check(r, "rope_qk")
+        return r
     _chk(q.dim() == 4 and k.dim() == 4 and cos.dim() == 3 and sin.dim() == 3,
          "q, k must be [B, H, T, D] and cos, sin [B, T, D]")
     B, Hq, T, D = q.shape

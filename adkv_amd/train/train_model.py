@@ -37,6 +37,13 @@ def quant_f32(x: torch.Tensor, alpha: torch.Tensor, beta: torch.Tensor, target: 
     (in-place, as the reference's eval cache does).  Returns ``(xhat, codes | None, zp_seq | None,
     sc_seq | None)``.
     """
+    if zp_state is None and sc_state is None and out is None and not want_codes:
+        r = _lib.host().quant_f32(x, (alpha, beta, target, zp_init, sc_init), lower_limit, upper_limit,
+                                  float(sc_min), float(sc_max), bool(output_states))
+        if r is not None:      # None: something to check, convert or complain about below
+            if isinstance(r, int):
+                _lib.check(r, "quant_f32")
+            return r[0], None, r[1], r[2]
     _chk(x.dim() == 3 and x.dtype in _DTYPES and x.stride(2) == 1, "x must be [B, T, C] with unit channel stride")
     B, T, C = x.shape
     dev = _need_device(x)

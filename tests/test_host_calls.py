@@ -1,0 +1,101 @@
+"""The host calls (csrc/host_calls.cpp): what they take gives what the Python functions give, and what they do
+not take goes to the Python functions."""
+import types
+
+import pytest
+import torch
+from torch.utils._python_dispatch import TorchDispatchMode
+
+from adkv_amd import _lib, synth
+from adkv_amd.hf import cache as C
+from adkv_amd.kernel import gemv
+from adkv_amd.train.train_model import quant_f32
+
+NOTHING = types.SimpleNamespace(**{n: (lambda *a: None) for n in ("rope_qk", "decode", "append", "quant_f32")})
+
+
+class _Sub(torch.Tensor):
+    pass
+
+
+def test_other_arguments_are_left_to_python():
+    h = _lib.host()
+    x = torch.zeros(1, 1, 1, 128, dtype=torch.float16)
+    assert h.rope_qk(x, x, x[0], x[0]) is None                                   # not on a device
+    for args in ((), (x,), (1, 2, 3, 4), (x, x, None, None)):
+        assert h.rope_qk(*args) is None
+    for f, n in ((h.decode, 14), (h.append, 14), (h.quant_f32, 7)):
+        assert f() is None and f(*[None] * n) is None and f(*[x] * n) is None and f(*[1 << 70] * n) is None
+    p = tuple(torch.zeros(128) for _ in range(5))
+    assert h.quant_f32(torch.zeros(1, 2, 128), p, -8, 7, 0.1, 2.0, False) is None
+
+
+class _Count(TorchDispatchMode):
+    seen = 0
+
+    def __torch_dispatch__(self, func, types, args=(), kwargs=None):
+        _Count.seen += 1
+        return func(*args, **(kwargs or {}))
+
+
+@pytest.mark.gpu
+def test_watched_or_unusual_tensors_are_left_to_python(gpu):
+    h = _lib.host()
+    q = torch.randn(2, 4, 3, 128, device=gpu).half()
+    cs = torch.randn(2, 3, 128, device=gpu).half()
+    took = lambda *a: h.rope_qk(*a) is not None
+    assert took(q, q, cs, cs)
+    assert took(q.transpose(1, 2).contiguous().transpose(1, 2), q, cs, cs) and took(q, q, cs[:1], cs[:1])
+    assert not took(q.as_subclass(_Sub), q, cs, cs) and not took(q, q.cpu(), cs, cs) and not took(q, q.bfloat16(), cs, cs)
+    assert not took(torch.randn(2, 4, 3, 129, device=gpu).half()[..., :128], q, cs, cs)     # odd strides
+    assert not took(q.float(), q.float(), cs.float(), cs.float()) and not took(q, q[:, :, :2], cs, cs)
+    with _Count():
+        assert not took(q, q, cs, cs)
+        gemv.rope_qk(q, q, cs, cs)
+    assert _Count.seen > 0                                                                     # the mode saw the Python function's work
+    got = []
+    torch.func.vmap(lambda a: (got.append(took(a, q, cs, cs)), a)[1])(q[None])
+    assert got == [False]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("D,Hq,H,bits,T,mask_dtype,mask_heads", [
+    (128, 4, 4, 4, 300, None, 1), (128, 8, 2, 2, 700, torch.bfloat16, 1), (256, 2, 2, 4, 300, torch.float32, 2), (128, 4, 1, 4, 0, None, 1)])
+def test_layer_calls_equal_the_python_functions(gpu, monkeypatch, dtype, D, Hq, H, bits, T, mask_dtype, mask_heads):
+    B = 2
+    params = [t.reshape(-1).to(gpu) for i in (1, 2) for t in synth.make_params(H, D, bits=bits, seed=i).astuple()]
+    g = torch.Generator(device=gpu).manual_seed(T)
+    heads = lambda n, t: torch.randn(B, t, n, D, generator=g, device=gpu).to(dtype).transpose(1, 2)
+    k, v, cos, sin = heads(H, T), heads(H, T), *(torch.randn(B, 1, D, generator=g, device=gpu).to(dtype) for _ in range(2))
+    new = [[heads(n, 1) for n in (Hq, H, H)] for _ in range(3)]
+    masks = [None if mask_dtype is None else torch.randn(B, mask_heads, 1, T + i + 1, generator=g, device=gpu).to(mask_dtype) for i in range(3)]
+    def run():
+        layer, res = C.KVCacheLayer_ADKV(bits), []
+        if T:
+            layer.prefill(k, v, *params)
+        for (q, kn, vn), m in zip(new, masks):
+            q, kn = gemv.rope_qk(q, kn, cos, sin)
+            out, w = layer.decode(q, kn, vn, *params, attention_mask=m, scaling=D ** -0.5)
+            assert out.dtype == dtype and w.shape == (B, Hq, layer.get_seq_length())
+            res += [q, kn, out, w.clone()]
+        used = -(-layer.get_seq_length() // (32 // bits))
+        return res + [t[:, :, :used] for t in (layer.key_states, layer.value_states)]
+    run()                                                                          # the workspace is there from now on
+    mine = run()
+    monkeypatch.setattr(_lib, "host", lambda: NOTHING)
+    for a, b in zip(mine, run()):
+        assert a.dtype == b.dtype and torch.equal(a, b)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("states", [False, True])
+def test_fp32_quantiser_equals_the_python_function(gpu, monkeypatch, dtype, states):
+    x = torch.randn(3, 77, 192, device=gpu).to(dtype)
+    a, b, t, z, s = (torch.rand(192, device=gpu) * 0.1 + 0.05 for _ in range(5))
+    f = lambda: quant_f32(x, a, b, t, -8, 7, 0.01, 50.0, zp_init=z, sc_init=s, output_states=states)
+    mine = f()
+    monkeypatch.setattr(_lib, "host", lambda: NOTHING)
+    for p, q in zip(mine, f()):
+        assert (p is None) == (q is None) and (p is None or torch.equal(p, q))
