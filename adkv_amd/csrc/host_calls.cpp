@@ -360,6 +360,54 @@ PyObject *quant_f32(PyObject *, PyObject *const *args, Py_ssize_t nargs)
     return r;
 }
 
+// quant_f32_pair(k rows, v rows, k out, v out, params (six), states (four), initial states (four) or None, lower,
+//                upper, sc_min, sc_max)
+PyObject *quant_f32_pair(PyObject *, PyObject *const *args, Py_ssize_t nargs)
+{
+    if (nargs != 11 || !unwatched() || !PyFloat_CheckExact(args[9]) || !PyFloat_CheckExact(args[10]))
+        Py_RETURN_NONE;
+    const at::Tensor *t[4];
+    for (int i = 0; i < 4; i++)
+        if (!(t[i] = plain(args[i])) || t[i]->dim() != 3 || t[i]->sizes() != t[0]->sizes() ||
+            t[i]->scalar_type() != t[0]->scalar_type() || t[i]->stride(2) != 1 || t[i]->device() != t[0]->device())
+            Py_RETURN_NONE;
+    const at::Tensor &x = *t[0];
+    const long lower = PyLong_AsLong(args[7]), upper = PyLong_AsLong(args[8]);
+    if (PyErr_Occurred()) {
+        PyErr_Clear();
+        Py_RETURN_NONE;
+    }
+    const int64_t B = x.size(0), T = x.size(1), C = x.size(2);
+    if ((!half_type(x) && x.scalar_type() != at::kFloat) || B <= 0 || T <= 0 || C <= 0 || B > INT32_MAX || T > INT32_MAX ||
+        C > INT32_MAX || lower < INT32_MIN || upper > INT32_MAX)
+        Py_RETURN_NONE;
+    const void *rows[4], *params[6], *state[4], *init[4];
+    int64_t strides[8];
+    for (int i = 0; i < 4; i++) { // of a single sequence or token the strides may be anything
+        rows[i] = t[i]->const_data_ptr();
+        strides[2 * i] = B > 1 ? t[i]->stride(0) : T * std::max(t[i]->stride(1), C);
+        strides[2 * i + 1] = T > 1 ? t[i]->stride(1) : C;
+    }
+    void *stream;
+    for (Py_ssize_t i = 0; PyTuple_CheckExact(args[5]) && i < PyTuple_GET_SIZE(args[5]); i++) {
+        const at::Tensor *st = plain(PyTuple_GET_ITEM(args[5], i));
+        if (!st || st->dim() != 2 || st->size(0) != B)
+            Py_RETURN_NONE;
+    }
+    if (!pointers(args[4], 6, at::kFloat, C, x.device(), params) || !pointers(args[5], 4, at::kFloat, B * C, x.device(), state) ||
+        (args[6] != Py_None && !pointers(args[6], 4, at::kFloat, C, x.device(), init)) || !current(x.device(), stream))
+        Py_RETURN_NONE;
+    const int type = x.scalar_type() == at::kFloat ? ADKV_DT_F32 : x.scalar_type() == at::kHalf ? ADKV_DT_F16 : ADKV_DT_BF16;
+    const double lo = PyFloat_AS_DOUBLE(args[9]), hi = PyFloat_AS_DOUBLE(args[10]);
+    int rc;
+    Py_BEGIN_ALLOW_THREADS
+    rc = adkv_quant_f32_pair(rows, strides, const_cast<void *const *>(rows + 2), strides + 4, const_cast<void *const *>(state),
+                             args[6] != Py_None ? init : nullptr, params, (int)B, (int)T, (int)C, type, (int)lower, (int)upper,
+                             (float)lo, (float)hi, stream);
+    Py_END_ALLOW_THREADS
+    return PyLong_FromLong(rc);
+}
+
 PyObject *init(PyObject *, PyObject *f)
 {
     Py_INCREF(f);
@@ -373,6 +421,7 @@ PyMethodDef methods[] = {
     {"decode", (PyCFunction)(void (*)(void))decode, METH_FASTCALL, nullptr},
     {"append", (PyCFunction)(void (*)(void))append, METH_FASTCALL, nullptr},
     {"quant_f32", (PyCFunction)(void (*)(void))quant_f32, METH_FASTCALL, nullptr},
+    {"quant_f32_pair", (PyCFunction)(void (*)(void))quant_f32_pair, METH_FASTCALL, nullptr},
     {nullptr, nullptr, 0, nullptr}};
 PyModuleDef module = {PyModuleDef_HEAD_INIT, "_host", nullptr, -1, methods, nullptr, nullptr, nullptr, nullptr};
 

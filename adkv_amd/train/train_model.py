@@ -88,6 +88,12 @@ def quant_f32_pair(x, params, lower_limit: int, upper_limit: int, sc_min: float,
     fp32 ``[B, C]`` tensors ``(zp, sc)`` updated in place, ``init`` optional ``[C]`` vectors ``(zp, sc)`` to
     start from instead.
     """
+    rc = _lib.host().quant_f32_pair(*x, *out, tuple(t for p in params for t in p), tuple(t for p in states for t in p),
+                                    tuple(t for p in init for t in p) if init else None, lower_limit, upper_limit,
+                                    float(sc_min), float(sc_max))
+    if rc is not None:      # None: something to check, convert or complain about below
+        _lib.check(rc, "quant_f32_pair")
+        return
     B, T, C = x[0].shape
     for t, o in zip(x, out):
         _chk(t.dtype == x[0].dtype and t.dtype in _DTYPES and t.shape == x[0].shape and t.stride(2) == 1, "x must be [B, T, C] with unit channel stride")

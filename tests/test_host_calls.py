@@ -11,7 +11,7 @@ from adkv_amd.hf import cache as C
 from adkv_amd.kernel import gemv
 from adkv_amd.train.train_model import quant_f32
 
-NOTHING = types.SimpleNamespace(**{n: (lambda *a: None) for n in ("rope_qk", "decode", "append", "quant_f32")})
+NOTHING = types.SimpleNamespace(**{n: (lambda *a: None) for n in ("rope_qk", "decode", "append", "quant_f32", "quant_f32_pair")})
 
 
 class _Sub(torch.Tensor):
@@ -24,7 +24,7 @@ def test_other_arguments_are_left_to_python():
     assert h.rope_qk(x, x, x[0], x[0]) is None                                   # not on a device
     for args in ((), (x,), (1, 2, 3, 4), (x, x, None, None)):
         assert h.rope_qk(*args) is None
-    for f, n in ((h.decode, 14), (h.append, 14), (h.quant_f32, 7)):
+    for f, n in ((h.decode, 14), (h.append, 14), (h.quant_f32, 7), (h.quant_f32_pair, 11)):
         assert f() is None and f(*[None] * n) is None and f(*[x] * n) is None and f(*[1 << 70] * n) is None
     p = tuple(torch.zeros(128) for _ in range(5))
     assert h.quant_f32(torch.zeros(1, 2, 128), p, -8, 7, 0.1, 2.0, False) is None
@@ -99,3 +99,20 @@ def test_fp32_quantiser_equals_the_python_function(gpu, monkeypatch, dtype, stat
     monkeypatch.setattr(_lib, "host", lambda: NOTHING)
     for p, q in zip(mine, f()):
         assert (p is None) == (q is None) and (p is None or torch.equal(p, q))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_evaluation_cache_equals_the_python_function(gpu, monkeypatch, dtype):
+    from adkv_amd.hf import llama_adkv_eval as E
+    x = [torch.randn(2, n, 256, device=gpu).to(dtype) for n in (77, 1, 30)]
+    p = [torch.rand(256, device=gpu) * 0.1 + 0.05 for _ in range(10)]
+    def run():
+        layer = E.KVCacheLayer_ADKV()
+        for t in x:
+            keys, values = layer.update(t, -t, *p)
+        return [t.clone() for t in (keys, values, layer.key_dc, layer.value_dc, layer.key_scale, layer.value_scale)]
+    mine = run()
+    monkeypatch.setattr(_lib, "host", lambda: NOTHING)
+    for a, b in zip(mine, run()):
+        assert torch.equal(a, b)
