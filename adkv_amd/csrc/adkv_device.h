@@ -342,6 +342,114 @@ __device__ __forceinline__ void enc_eight_tokens(Chan1 &c, const uint16_t *x, ui
 #undef ADKV_ENC_TOKEN
 }
 
+// Sixty-four tokens of one channel per lane, their rows in LDS: eight groups of eight rows of 64 channels,
+// 1 KB each from `addr` on.  ds_read_b64_tr_b16 hands every lane four tokens of its own channel (16 lanes read
+// four rows of 16 channels), two of them instead of eight narrow loads per group: a wave alone on its SIMD pays 12
+// cycles for any LDS read and 16 to 18 for any load from memory, against 4 or 5 for an arithmetic
+// instruction.  The reads of a group go out before the arithmetic of the one before it and are waited for
+// behind it, all inside one block, so that no register is handed over before its data is there.
+// The token is that of enc_eight_tokens with the scale kept NEGATED, in the low half of ss and in fp32
+// (nsc), and alpha negated with it: the remainder is then a plain multiply-add into d, and the conversion
+// of the next scale needs no half selected.  Negation is exact and products of two negated factors are the
+// same, NaNs aside; a run in which a quotient or the state it ends in is a NaN is done again (collect nsc and
+// zp behind the block).
+struct Chan1Neg {
+    uint32_t zp;  // low half; the high half is never read
+    uint32_t ss;  // low half: minus the scale
+    float nsc;    // minus the scale in fp32
+};
+#define ADKV_RUN_TOKEN(X, SEL, R, FILL, W)                                                               \
+    "v_rcp_f32_e64 %[rs], -%[ns]\n\t"                                                                    \
+    "v_fma_mix_f32 %[d], " X ", 1.0, -%[zp] op_sel:[" SEL ",0,0] op_sel_hi:[1,0,1]\n\t"                  \
+    "v_mul_f32 " R ", %[d], %[rs]\n\t"                                                                   \
+    "v_fmac_f32 %[d], " R ", %[ns]\n\t"                                                                  \
+    "v_fmac_f32 " R ", %[d], %[rs]\n\t"                                                                  \
+    "v_add_f32 %[u], %[magic], " R "\n\t"                                                                \
+    "v_med3_f32 %[u], %[u], %[lo], %[hi]\n\t"                                                            \
+    "v_cvt_f16_i16 %[q], %[u]\n\t"                                                                       \
+    "v_fma_f16 %[q], %[be], |%[q]|, %[omt] op_sel:[0,0,0,1]\n\t"                                         \
+    "v_alignbit_b32 " W ", %[u], " W ", %[bits]\n\t"                                                     \
+    "v_pk_mul_f16 %[ss], %[ss], %[q] op_sel:[0,1] op_sel_hi:[0,0]\n\t"                                   \
+    FILL "\n\t"                                                                                          \
+    "v_pk_fma_f16 %[zp], %[nal], %[ss], %[zp] op_sel:[0,1,0]\n\t"                                        \
+    "v_cvt_f32_f16 %[ns], %[ss]\n\t"
+#define ADKV_RUN_PAIR(X, W)                                                                              \
+    ADKV_RUN_TOKEN(X, "0", "%[r0]", "s_nop 0", W)                                                        \
+    ADKV_RUN_TOKEN(X, "1", "%[r1]", "v_maximum3_f32 %[nan], %[nan], %[r0], %[r1]", W)
+// bfloat16 pairs become fp16 pairs (nearest even) where they are
+#define ADKV_RUN_BF16(X)                                                                                 \
+    "v_lshlrev_b32 %[r0], 16, " X "\n\t"                                                                 \
+    "v_and_b32 %[r1], %[mask], " X "\n\t"                                                                \
+    "v_cvt_pk_f16_f32 " X ", %[r0], %[r1]\n\t"
+#define ADKV_RUN_F16(X) ""
+#define ADKV_RUN_READ(A, B, OFF0, OFF1)                                                                  \
+    "ds_read_b64_tr_b16 " A ", %[addr] offset:" OFF0 "\n\t"                                              \
+    "ds_read_b64_tr_b16 " B ", %[addr] offset:" OFF1 "\n\t"
+// (the pairs of the next two tokens are converted a pair ahead: a packed result is not read by the next instruction)
+#define ADKV_RUN_GROUP(C, X0, X1, X2, X3, NEXT, W)                                                       \
+    "s_waitcnt lgkmcnt(0)\n\t" NEXT C(X0) C(X1) ADKV_RUN_PAIR(X0, W) C(X2) ADKV_RUN_PAIR(X1, W)          \
+    C(X3) ADKV_RUN_PAIR(X2, W) ADKV_RUN_PAIR(X3, W)
+#define ADKV_RUN_A(C, NEXT, W) ADKV_RUN_GROUP(C, "v48", "v49", "v50", "v51", NEXT, W)
+#define ADKV_RUN_B(C, NEXT, W) ADKV_RUN_GROUP(C, "v52", "v53", "v54", "v55", NEXT, W)
+#define ADKV_RUN_INTO_A(OFF0, OFF1) ADKV_RUN_READ("v[48:49]", "v[50:51]", OFF0, OFF1)
+#define ADKV_RUN_INTO_B(OFF0, OFF1) ADKV_RUN_READ("v[52:53]", "v[54:55]", OFF0, OFF1)
+#define ADKV_RUN_ALL(C, W0, W1, W2, W3, W4, W5, W6, W7)                                                  \
+    ADKV_RUN_INTO_A("0", "512")                                                                          \
+    ADKV_RUN_A(C, ADKV_RUN_INTO_B("1024", "1536"), W0) ADKV_RUN_B(C, ADKV_RUN_INTO_A("2048", "2560"), W1) \
+    ADKV_RUN_A(C, ADKV_RUN_INTO_B("3072", "3584"), W2) ADKV_RUN_B(C, ADKV_RUN_INTO_A("4096", "4608"), W3) \
+    ADKV_RUN_A(C, ADKV_RUN_INTO_B("5120", "5632"), W4) ADKV_RUN_B(C, ADKV_RUN_INTO_A("6144", "6656"), W5) \
+    ADKV_RUN_A(C, ADKV_RUN_INTO_B("7168", "7680"), W6) ADKV_RUN_B(C, "", W7)
+#define ADKV_RUN_OPERANDS                                                                                \
+        : [zp] "+v"(c.zp), [ss] "+v"(c.ss), [ns] "+v"(c.nsc), [nan] "+v"(nan), [d] "=&v"(d), [rs] "=&v"(rs), [u] "=&v"(u), \
+          [q] "=&v"(q), [r0] "=&v"(r0), [r1] "=&v"(r1), [w0] "=&v"(w[0]), [w1] "=&v"(w[1]), [w2] "=&v"(w[2]), [w3] "=&v"(w[3])
+#define ADKV_RUN_INPUTS                                                                                  \
+        : [addr] "v"(addr), [nal] "v"(nal), [be] "v"(be), [omt] "v"(omt), [lo] "s"(lo), [hi] "v"(hi), [magic] "s"(magic), \
+          [mask] "s"(0xFFFF0000u), [bits] "n"(BITS)                                                      \
+        : "v48", "v49", "v50", "v51", "v52", "v53", "v54", "v55", "memory"
+#define ADKV_RUN_EIGHT_WORDS , [w4] "=&v"(w[4]), [w5] "=&v"(w[5]), [w6] "=&v"(w[6]), [w7] "=&v"(w[7])
+#define ADKV_RUN_4BIT(C) ADKV_RUN_ALL(C, "%[w0]", "%[w1]", "%[w2]", "%[w3]", "%[w4]", "%[w5]", "%[w6]", "%[w7]")
+#define ADKV_RUN_2BIT(C) ADKV_RUN_ALL(C, "%[w0]", "%[w0]", "%[w1]", "%[w1]", "%[w2]", "%[w2]", "%[w3]", "%[w3]")
+template <int BITS, bool BF16>
+__device__ __forceinline__ void enc_run64(Chan1Neg &c, uint32_t addr, uint32_t nal, uint32_t be, uint32_t omt, float magic,
+                                          float lo, float hi, uint32_t *w, float &nan)
+{
+    float d, r0, r1, rs;
+    uint32_t u, q;
+    if constexpr (BITS == 4 && BF16)
+        asm volatile(ADKV_RUN_4BIT(ADKV_RUN_BF16) ADKV_RUN_OPERANDS ADKV_RUN_EIGHT_WORDS ADKV_RUN_INPUTS);
+    else if constexpr (BITS == 4)
+        asm volatile(ADKV_RUN_4BIT(ADKV_RUN_F16) ADKV_RUN_OPERANDS ADKV_RUN_EIGHT_WORDS ADKV_RUN_INPUTS);
+    else if constexpr (BF16)
+        asm volatile(ADKV_RUN_2BIT(ADKV_RUN_BF16) ADKV_RUN_OPERANDS ADKV_RUN_INPUTS);
+    else
+        asm volatile(ADKV_RUN_2BIT(ADKV_RUN_F16) ADKV_RUN_OPERANDS ADKV_RUN_INPUTS);
+}
+#undef ADKV_RUN_2BIT
+#undef ADKV_RUN_4BIT
+#undef ADKV_RUN_EIGHT_WORDS
+#undef ADKV_RUN_INPUTS
+#undef ADKV_RUN_OPERANDS
+#undef ADKV_RUN_ALL
+#undef ADKV_RUN_INTO_B
+#undef ADKV_RUN_INTO_A
+#undef ADKV_RUN_B
+#undef ADKV_RUN_A
+#undef ADKV_RUN_GROUP
+#undef ADKV_RUN_READ
+#undef ADKV_RUN_F16
+#undef ADKV_RUN_BF16
+#undef ADKV_RUN_PAIR
+#undef ADKV_RUN_TOKEN
+
+// 64 lanes x 16 bytes from memory into 1 KB of LDS at `lds` (wave-uniform), without a register in between.
+// Counted by vmcnt like any load; the compiler does not know what it writes.
+typedef uint32_t rsrc4 __attribute__((ext_vector_type(4)));
+__device__ __forceinline__ void load_to_lds(uint32_t lds, uint32_t offset, rsrc4 buffer)
+{
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, 0 offen lds" ::"s"(lds), "v"(offset), "s"(buffer)
+                 : "memory"); // m0 is set before every use, by the compiler too
+}
+
 __device__ __forceinline__ h2 codes_to_h2(int q0, int q1) { return (h2){(h1)q0, (h1)q1}; }
 
 // Quantise one new token's channel pair with the current state and patch its two codes into the

@@ -513,6 +513,12 @@ struct SegLoads {
 constexpr int ENC_PF1 = 8;    // buffers of 8 rows in rotation, one channel per lane (one wave per SIMD: nothing else hides HBM)
 constexpr int ENC_AHEAD1 = 6; // groups loaded ahead: 56 loads and their groups' stores fit the 63 the counter holds
 constexpr int ENC_PF2 = 4; // two channels per lane (many waves)
+constexpr int ENC_RING = 16 * 1024; // a wave's LDS, one channel per lane: two runs of 64 rows of 64 channels
+template <int CPL>
+__device__ __forceinline__ char *enc_ring(uint4 *ring)
+{
+    return CPL == 1 ? reinterpret_cast<char *>(ring) + (threadIdx.x >> 6) * ENC_RING : nullptr;
+}
 
 // Where the new rows are: element strides between batches, heads and tokens (channels are
 // contiguous).  The encoder reads each row once, 256 bytes per head, so a [B, T, H, D] projection
@@ -533,7 +539,7 @@ __device__ __forceinline__ void encode_body(
     const h1 *__restrict__ zp, const h1 *__restrict__ sc, const h1 *__restrict__ al,
     const h1 *__restrict__ be, const h1 *__restrict__ tg,
     int BH, int H, int T0, int T, int D, int n_super_cap, const h1 *__restrict__ state_in,
-    h1 *__restrict__ state_out, const Seg &sa)
+    h1 *__restrict__ state_out, const Seg &sa, char *ring)
 {
     // Quantises tokens [T0, T) of a stream whose first T0 tokens are already in the cache; kv_new
     // holds the T - T0 new rows; state_in is the state after token T0-1 (ignored when T0 == 0).
@@ -716,10 +722,67 @@ __device__ __forceinline__ void encode_body(
     const int sg_end = T / TPW;
     const long span_words = (1L << 30) / (xs.t * 2 * TPW);
     int redo = PF / G8, resumed = -1; // words done with the plain division after a NaN; where the last such stretch ended
+    bool through_lds = CPL == 1 && ring != nullptr && ((uintptr_t)(xb + (long)sg * TPW * xs.t) & 15) == 0 && xs.t % 8 == 0 &&
+                       (sa.ckpt == nullptr || (sa.ckpt_interval % 64 == 0 && sg * TPW % 64 == 0));
     const int piece = (int)(span_words >= PF ? span_words / PF * PF : max(span_words, 1L)); // whole runs where it can
     while (sg < sg_end) {
         const int nw = min(piece, sg_end - sg), ng = nw * G8; // words, 8-token groups of this piece
         const uint32_t xbytes = (uint32_t)(((long)ng * 8 - 1) * xs.t * 2 + 128 * CPL);
+        if constexpr (CPL == 1) {
+            // Whole runs of 64 tokens whose rows come through the LDS (enc_run64), a run ahead: 64 tokens or 2 us.  Rows have
+            // to be 16-byte aligned; a run that meets a NaN, and all after it, go through the loop below.
+            if (through_lds && ng >= 8) {
+                constexpr int WORDS = 8 / G8;
+                const uint64_t base = wave_uniform((uint64_t)(xb + (long)sg * TPW * xs.t));
+                const rsrc4 rows = {(uint32_t)base, (uint32_t)(base >> 32), xbytes, 0x00027000u};
+                const uint32_t row = (uint32_t)(xs.t * 2), lds = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)(
+                    __attribute__((address_space(3))) char *)ring);
+                uint32_t off = (uint32_t)(lane >> 3) * row + (uint32_t)(lane & 7) * 16u, half = 0;
+                // lane i of 16 reads token i / 4, channels 4 * (i % 4).. of its 16-channel group
+                const uint32_t addr = lds + (uint32_t)((lane & 15) >> 2) * 128u + (uint32_t)(lane >> 4) * 32u + (uint32_t)(lane & 3) * 8u;
+                auto load_run = [&](uint32_t to) __attribute__((always_inline)) { // past the end: dropped by the bounds check
+#pragma unroll
+                    for (int k = 0; k < 8; k++) {
+                        load_to_lds(to + (uint32_t)k * 1024u, off, rows);
+                        off += row * 8u;
+                    }
+                };
+                uint32_t *dst = cw + (size_t)sg * D + lane;
+                const uint32_t nal = as_u32(st.al) ^ 0x80008000u;
+                load_run(lds);
+                for (int g = 0; g + 8 <= ng; g += 8) {
+                    load_run(lds + (half ^ 8192u));
+                    // everything but the next run's eight loads and, from the second run on, the codes just
+                    // stored (all of them complete in order)
+                    if (g == 0)
+                        asm volatile("s_waitcnt vmcnt(8)" ::: "memory");
+                    else if (WORDS == 8)
+                        asm volatile("s_waitcnt vmcnt(16)" ::: "memory");
+                    else
+                        asm volatile("s_waitcnt vmcnt(12)" ::: "memory");
+                    Chan1Neg ch = {as_u32(st.zp), as_u32((h2){-st.sc.x, (h1)0.0f}), -(float)st.sc.x};
+                    uint32_t w[WORDS];
+                    float nan = 0.0f;
+                    enc_run64<BITS, BF16>(ch, addr + half, nal, as_u32(st.be), as_u32(st.omt), MAGIC, ULO, uhi, w, nan);
+                    nan = enc_collect_nan(nan, ch.nsc, (float)as_h2(ch.zp).x);
+                    if (__builtin_expect(__any(nan != nan), 0)) {
+                        through_lds = false;
+                        break;
+                    }
+                    st.zp = splat(as_h2(ch.zp).x);
+                    st.sc = splat(-as_h2(ch.ss).x);
+#pragma unroll
+                    for (int k = 0; k < WORDS; k++)
+                        dst[(size_t)k * D] = w[k] ^ WORD_BIAS;
+                    dst += (size_t)WORDS * D;
+                    sg += WORDS;
+                    checkpoint(sg * TPW);
+                    half ^= 8192u;
+                }
+                asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); // nothing is on its way into the LDS any more
+                continue;
+            }
+        }
         const __amdgpu_buffer_rsrc_t xr = __builtin_amdgcn_make_buffer_rsrc(
             (void *)wave_uniform((uint64_t)(xb + (long)sg * TPW * xs.t)), 0, (int)xbytes, 0x00027000);
         uint32_t xoff = (uint32_t)lane * 2u * CPL;
@@ -869,8 +932,9 @@ __global__ __launch_bounds__(BLK, CPL == 2 ? 5 : 1) void encode_kernel(
     h1 *__restrict__ state_out, Seg sa)
 {
     const RowStrides packed = {(long)H * (T - T0) * D, (long)(T - T0) * D, (long)D};
+    __shared__ uint4 ring[CPL == 1 ? BLK / 64 * ENC_RING / 16 : 1];
     encode_body<BITS, CPL, BLK>(cache, kv_new, packed, zp, sc, al, be, tg, BH, H, T0, T, D, n_super_cap,
-                                state_in, state_out, sa);
+                                state_in, state_out, sa, enc_ring<CPL>(ring));
 }
 
 // Two tensors of one shape (the K and V rows of the same tokens) in one launch: blockIdx.y picks
@@ -891,8 +955,9 @@ __global__ __launch_bounds__(BLK, CPL == 2 ? 5 : 1) void encode_pair_kernel(EncT
 {
     const EncTensor e = blockIdx.y ? v : k;
     sa.ckpt = e.ckpt;
+    __shared__ uint4 ring[CPL == 1 ? BLK / 64 * ENC_RING / 16 : 1];
     encode_body<BITS, CPL, BLK, BF16>(e.cache, e.kv_new, e.xs, e.zp, e.sc, e.al, e.be, e.tg, BH, H, T0,
-                                      T, D, n_super_cap, e.state_in, e.state_out, sa);
+                                      T, D, n_super_cap, e.state_in, e.state_out, sa, enc_ring<CPL>(ring));
 }
 
 // Shared tail of the two decode kernels: quantise the new token with the state after token T-1,
