@@ -1,0 +1,57 @@
+"""Rows that reach the encoder through the LDS (one channel per lane, whole runs of 64 tokens, 16-byte aligned
+rows), where the runs, the pieces and the alignment end.  Codes, states and checkpoints are those of the
+oracle bit for bit."""
+import numpy as np
+import pytest
+import torch
+
+from adkv_amd import synth
+from adkv_amd.kernel import gemv
+from tests.test_encoder_forms import _np16, _same16
+
+pytestmark = pytest.mark.gpu
+
+D = 128
+
+
+@pytest.mark.parametrize("bits", (4, 2))
+@pytest.mark.parametrize("dtype", (torch.float16, torch.bfloat16))
+@pytest.mark.parametrize("cuts,S,pad,bad", [
+    ((0, 63), 0, 0, ()), ((0, 64), 64, 0, ()), ((0, 65), 0, 64, ()), ((0, 127), 64, 8, ()), ((0, 128), 128, 0, (127,)),
+    ((0, 129, 200), 64, 0, ()),             # resumed inside a word, checkpoints between runs that do not start at one
+    ((0, 128, 321), 64, 24, (191, 192)),    # resumed at a run, a run that fails at its last and first token
+    ((0, 200), 48, 0, ()),                  # checkpoints inside runs
+    ((0, 200), 64, 4, ()), ((0, 200), 64, 1, (64,)),   # rows 8 and 2 bytes off: not through the LDS
+    ((0, 7, 64, 576), 256, 16, (575,))])
+def test_runs_through_the_lds(gpu, oracle, bits, dtype, cuts, S, pad, bad):
+    B, H, T = 2, 3, cuts[-1]
+    params, rows, want = [], [], []
+    for i in range(2):
+        ps = [t.clone() for t in synth.make_params(H, D, bits=bits, seed=7 + i).astuple()]
+        x = (2.0 * torch.randn(B, T, H * D + pad, generator=torch.Generator().manual_seed(T + i))).to(dtype)
+        x[..., H * D:] = float("nan")                                # never read
+        for t in bad:
+            x[1, t, 17 + 64 * i] = float("inf")
+        xh = x[..., :H * D].view(B, T, H, D).transpose(1, 2)
+        rows.append(x.to(gpu)[..., :H * D].view(B, T, H, D).transpose(1, 2))
+        params.append([t.to(gpu) for t in ps])
+        pn, xn = [_np16(t) for t in ps], _np16(xh.to(torch.float16))
+        with oracle.code_bits(bits):
+            c = oracle.alloc_cache(B, H, T + 16, D)
+            st = oracle.encode_kv_f16(c, xn, *pn)
+            cks = []
+            for j in range(T // S if S else 0):
+                part = oracle.alloc_cache(B, H, (j + 1) * S, D)
+                cks.append(oracle.encode_kv_f16(part, xn[:, :, :(j + 1) * S], *pn))
+        want.append((c, st, cks))
+    caches = [synth.alloc_cache(B, H, T + 16, D, gpu, bits=bits) for _ in range(2)]
+    states = [torch.zeros(B, H, D, 2, dtype=torch.float16, device=gpu) for _ in range(2)]
+    cks = [torch.zeros(B, H, T // S + 1, D, 2, dtype=torch.float16, device=gpu) if S else None for _ in range(2)]
+    for a, b in zip(cuts, cuts[1:]):
+        gemv.append_kv_pair(*caches, *(r[:, :, a:b] for r in rows), *params, a, *states, k_ckpt=cks[0], v_ckpt=cks[1],
+                            ckpt_interval=S, bits=bits)
+    torch.cuda.synchronize()
+    for c, s, k, (wc, ws, wk) in zip(caches, states, cks, want):
+        assert np.array_equal(c.cpu().numpy(), wc) and _same16(_np16(s), ws)
+        for j, w in enumerate(wk):
+            assert _same16(_np16(k[:, :, j]), w), j
