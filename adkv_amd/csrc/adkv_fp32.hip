@@ -87,13 +87,18 @@ constexpr int GRP = 8; // tokens per speculative group
 struct Chan {
     float zp, sc, s, rs; // s = max(sc, 1e-8) (NaN kept), rs ~ 1/s
     float al, be, tg;
-    __device__ __forceinline__ void init(const Tensor &a, int b, int c, int C)
+    float sure; // no |off| reaches it: what step_spec returned is the reference's (below)
+    __device__ __forceinline__ void init(const Tensor &a, int b, int c, int C, const Limits &l)
     {
         zp = a.zp0 ? a.zp0[c] : a.zp_io[(long)b * C + c];
         set_scale(a.sc0 ? a.sc0[c] : a.sc_io[(long)b * C + c]);
         al = a.alpha[c];
         be = a.beta[c];
         tg = a.tgt[c];
+        // |sc*be| < 2^60 and |e| < 2^61: no scale of this channel can become a NaN before it is clamped.  A channel
+        // that is not known to be so has its groups repeated, every one (a NaN here as well).
+        const float most = fmaxf(fmaxf(l.sc_max, -l.sc_min), __builtin_fabsf(sc));
+        sure = most <= 0x1p100f && __builtin_fabsf(be) * most < 0x1p60f && __builtin_fabsf(tg) < 0x1p60f ? l.sure : -1.0f;
     }
     __device__ __forceinline__ void set_scale(float v)
     {
@@ -117,19 +122,18 @@ struct Chan {
         set_scale(clamp_keep_nan(sc + sbe, l.sc_min, l.sc_max));
         return xh;
     }
-    // The same token for a group that is checked afterwards: 16 instructions (rcp takes two slots).
+    // The same token for a group that is checked afterwards: 15 instructions (rcp takes two slots).
     //
     // The quotient is r = d*rs with the reciprocal kept from the token before.  |r - u| <= |u|*2^-22
     // for the IEEE quotient u (reciprocal 2^-23, two roundings 2^-24 each).  With L the largest code
     // magnitude, |u| > L + 1 is clamped either way, and below that rint(r) == rint(u) unless r lies
     // closer than (L + 1)*2^-22 to k + 1/2, that is unless |r - rint(r)| >= sure = 1/2 - (L + 1)*2^-21
-    // (twice the bound).  `off` returns r - rint(r), a NaN when r is infinite or one; `raw` the unclamped
-    // scale, whose NaN the clamp here drops and the reference's keeps.  The caller repeats the group
-    // with step() if any |off| is not below `sure` or any raw is a NaN: about one group of 8 tokens x 64
-    // channels in 120 with 4-bit codes.
+    // (twice the bound).  `off` returns r - rint(r), a NaN when r is infinite or one.  The caller repeats the
+    // group with step() if any |off| is not below `sure`: about one group of 8 tokens x 64 channels in 120 with
+    // 4-bit codes.  The clamp here drops a NaN that the reference's keeps: see init.
     // FLOOR: sc_min is below 1e-8 (otherwise s and sc are the same number).
     template <bool FLOOR>
-    __device__ __forceinline__ float step_spec(float xv, const Limits &l, float &q, float &off, float &raw)
+    __device__ __forceinline__ float step_spec(float xv, const Limits &l, float &q, float &off)
     {
         const float d = xv - zp;
         const float r = d * rs;
@@ -143,8 +147,7 @@ struct Chan {
         const float sb = sc * be;
         const float sbe = sb * e;
         zp = zp + ax;
-        raw = sc + sbe;
-        sc = __builtin_amdgcn_fmed3f(raw, l.sc_min, l.sc_max);
+        sc = __builtin_amdgcn_fmed3f(sc + sbe, l.sc_min, l.sc_max);
         s = FLOOR ? __builtin_amdgcn_fmed3f(sc, 1e-8f, __builtin_inff()) : sc;
         rs = __builtin_amdgcn_rcpf(s);
         return xh;
@@ -154,18 +157,16 @@ struct Chan {
     __device__ __forceinline__ void steps(const float *x, const Limits &l, float *xh, float *q, float *zs, float *ss)
     {
         const Chan saved = *this;
-        float off[GRP], raw[GRP], worst = 0.0f, nan = 0.0f;
+        float off[GRP], worst = 0.0f;
 #pragma unroll
         for (int k = 0; k < GRP; k++) {
             zs[k] = zp;
             ss[k] = sc;
-            xh[k] = step_spec<FLOOR>(x[k], l, q[k], off[k], raw[k]);
-            if (k & 1) {
+            xh[k] = step_spec<FLOOR>(x[k], l, q[k], off[k]);
+            if (k & 1)
                 worst = collect_abs(worst, off[k - 1], off[k]);
-                nan = adkv::enc_collect_nan(nan, raw[k - 1], raw[k]);
-            }
         }
-        if (__builtin_expect(__any(!(worst < l.sure) || nan != nan), 0)) {
+        if (__builtin_expect(__any(!(worst < sure)), 0)) {
             *this = saved;
 #pragma unroll
             for (int k = 0; k < GRP; k++) {
@@ -179,8 +180,10 @@ struct Chan {
 
 constexpr int CH = 32; // tokens per chunk, the unit in which the two waves of a workgroup hand rows over
 constexpr int NIN = 3, NOUT = 2;
+typedef float Quad __attribute__((ext_vector_type(4))); // four tokens of a channel
 
-// One array of rows a workgroup reads or writes: 64 channels from c0, rows `stride` elements apart.
+// One array of rows a workgroup reads or writes: 64 channels from c0, rows `stride` elements apart.  A lane has four
+// channels of rows 4*r0 .. 4*r0+3 of every 16.
 // WIDE: whole 4-channel vectors; the array has to be `aligned` and all 64 channels inside the row.
 template <typename T, bool WIDE>
 struct Rows {
@@ -191,14 +194,21 @@ struct Rows {
     Bits *base;
     long stride;
     int c, C; // this lane's first channel (of 4)
+    uint32_t lane; // bytes from row t of the array to this lane's first in row t + 4*r0 (WIDE)
     __device__ __forceinline__ Rows(void *p, long offset, long stride_, int c0, int C_)
         : stride(stride_), c(c0 + (threadIdx.x & 15) * 4), C(C_)
     {
         base = (Bits *)p + offset;
+        lane = ((uint32_t)stride * (((threadIdx.x & 63) >> 4) * 4) + (uint32_t)c) * (uint32_t)sizeof(Bits);
     }
     static __device__ __forceinline__ bool aligned(const void *p, long offset, long stride)
     {
-        return ((uintptr_t)p & (sizeof(Vec) - 1)) == 0 && offset % 4 == 0 && stride % 4 == 0;
+        return ((uintptr_t)p & (sizeof(Vec) - 1)) == 0 && offset % 4 == 0 && stride % 4 == 0 && stride <= 1L << 24;
+    }
+    // The lane's row k + 4*r0 of a chunk whose first row is at `rows`.
+    __device__ __forceinline__ Vec *quad(Bits *rows, int k) const
+    {
+        return reinterpret_cast<Vec *>(reinterpret_cast<char *>(rows + k * stride) + lane);
     }
     __device__ __forceinline__ void load(long row, Vec &d) const
     {
@@ -211,10 +221,14 @@ struct Rows {
                 d.v[k] = c + k < C ? p[k] : (Bits)0;
         }
     }
+    static __device__ __forceinline__ Vec down(const float4 &f)
+    {
+        return {{IO<T>::down(f.x), IO<T>::down(f.y), IO<T>::down(f.z), IO<T>::down(f.w)}};
+    }
     __device__ __forceinline__ void store(long row, const float4 &f) const
     {
         Bits *p = base + row * stride + c;
-        const Vec d = {{IO<T>::down(f.x), IO<T>::down(f.y), IO<T>::down(f.z), IO<T>::down(f.w)}};
+        const Vec d = down(f);
         if (WIDE) {
             *reinterpret_cast<Vec *>(p) = d;
         } else {
@@ -234,17 +248,21 @@ __device__ __forceinline__ void hand_over()
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
 }
 
+// Four tokens of a channel lie together: the recurrence reads and writes them in one instruction (an LDS read of
+// any width costs a wave that is alone 12 cycles, writes 16, 22 and 34 for one, two and four words).  Position
+// p of a row of 64 is channel p%16*4 + p/16, so that the mover, whose lane holds four neighbouring channels,
+// reads and writes without bank conflicts as well.
 // 40 KB without the optional outputs: four workgroups on a CU
 template <bool SEQ, bool CODES>
 struct Shared {
     static constexpr int Q = 1, ZP = CODES ? 2 : 1, SC = ZP + 1; // out[0] is xhat
-    float in[NIN][CH][64];
-    float out[1 + CODES + 2 * SEQ][NOUT][CH][64];
+    Quad in[NIN][CH / 4][64];
+    Quad out[1 + CODES + 2 * SEQ][NOUT][CH / 4][64];
 };
 
-// Chunk i is in `in[i % 3]` from the barrier before phase i-1 on (so the recurrence reads its first
-// group before the barrier that ends phase i-1); its results are in slot i % 2 of the output
-// buffers from the barrier after phase i on.  In phase i the mover
+// Chunk i is in `in[i % 3]` from the barrier before phase i-1 on (so the recurrence computes its first
+// group before the barrier that ends phase i-1, and writes those results after it); its results are in slot
+// i % 2 of the output buffers from the barrier after phase i on.  In phase i the mover
 //   writes chunk i+2 (loaded during phase i-1) to the slot chunk i-1 has left,
 //   issues the loads of chunk i+3, which have until phase i+2 (a phase is about 1 us) to arrive, and
 //   stores the results of chunk i-1.
@@ -256,107 +274,164 @@ __device__ __forceinline__ void move_rows(Shared<SEQ, CODES> &sm, const Tensor &
     const Rows<T, WIDE> xo(a.xhat, b * a.os_b, a.os_t, c0, C);
     const long dense = (long)b * Tn * C; // codes and state sequences are [B, T, C]
     const Rows<float, WIDE> zo(a.zp_seq, dense, C, c0, C), so(a.sc_seq, dense, C, c0, C);
-    const int r0 = (threadIdx.x & 63) >> 4, col = (threadIdx.x & 15) * 4;
+    const int r0 = (threadIdx.x & 63) >> 4, col = (threadIdx.x & 15) * 4; // rows 4*r0.. of every 16, channels col..
 
-    typename Rows<T, WIDE>::Vec v[CH / 4];
+    typedef typename Rows<T, WIDE>::Vec Vec;
+    typedef uint32_t Raw __attribute__((ext_vector_type(sizeof(Vec) / 4)));
+    Vec v[CH / 4];
+    // Chunk i, past the end the last row again.
     auto load = [&](int i) __attribute__((always_inline)) {
+        if (WIDE && (i + 1) * CH <= Tn) {
 #pragma unroll
-        for (int j = 0; j < CH / 4; j++)
-            x.load(min(i * CH + j * 4 + r0, Tn - 1), v[j]);
-    };
-    auto fill = [&](int slot) __attribute__((always_inline)) {
+            for (int j = 0; j < CH / 4; j++)
+                v[j] = *x.quad(x.base + i * CH * x.stride, j / 4 * 16 + j % 4);
+        } else {
 #pragma unroll
-        for (int j = 0; j < CH / 4; j++)
-            *reinterpret_cast<float4 *>(&sm.in[slot][j * 4 + r0][col]) =
-                make_float4(IO<T>::up(v[j].v[0]), IO<T>::up(v[j].v[1]), IO<T>::up(v[j].v[2]), IO<T>::up(v[j].v[3]));
-    };
-    auto drain = [&](int i) __attribute__((always_inline)) {
-        const int slot = i & 1;
-#pragma unroll
-        for (int j = 0; j < CH / 4; j++) {
-            const int row = j * 4 + r0;
-            const int t = i * CH + row;
-            if (t >= Tn)
-                break;
-            auto get = [&](const float *p) { return *reinterpret_cast<const float4 *>(p + col); };
-            if (a.xhat)
-                xo.store(t, get(sm.out[0][slot][row]));
-            if constexpr (SEQ) {
-                zo.store(t, get(sm.out[sm.ZP][slot][row]));
-                so.store(t, get(sm.out[sm.SC][slot][row]));
-            }
-            if constexpr (CODES) {
-                const float4 f = get(sm.out[sm.Q][slot][row]);
-                auto code = [](float q) { return (q != q) ? (int8_t)0 : (int8_t)q; };
-                const char4 k = make_char4(code(f.x), code(f.y), code(f.z), code(f.w));
-                int8_t *p = a.codes + dense + (long)t * C + c0 + col;
-                if (WIDE) {
-                    *reinterpret_cast<char4 *>(p) = k;
-                } else {
-                    const int8_t kk[4] = {k.x, k.y, k.z, k.w};
-#pragma unroll
-                    for (int e = 0; e < 4; e++)
-                        if (c0 + col + e < C)
-                            p[e] = kk[e];
-                }
-            }
+            for (int j = 0; j < CH / 4; j++)
+                x.load(min(i * CH + j / 4 * 16 + r0 * 4 + j % 4, Tn - 1), v[j]);
         }
     };
-    load(0);
-    fill(0);
-    if (nch > 1) {
+    auto fill = [&](int slot) __attribute__((always_inline)) {
+        // the rows are waited for here: without this they are put in order, and waited for, as soon as asked for
+#pragma unroll
+        for (int j = 0; j < CH / 4; j++) {
+            Raw raw = __builtin_bit_cast(Raw, v[j]);
+            asm volatile("" : "+v"(raw));
+            v[j] = __builtin_bit_cast(Vec, raw);
+        }
+#pragma unroll
+        for (int j = 0; j < CH / 4; j += 4)
+#pragma unroll
+            for (int k = 0; k < 4; k++)
+                sm.in[slot][j + r0][k * 16 + (threadIdx.x & 15)] =
+                    (Quad){IO<T>::up(v[j].v[k]), IO<T>::up(v[j + 1].v[k]), IO<T>::up(v[j + 2].v[k]), IO<T>::up(v[j + 3].v[k])};
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    // XHAT: a.xhat is there.  FULL: all of the chunk's tokens are.
+    auto drain = [&](int i, auto xhat, auto full) __attribute__((always_inline)) {
+        constexpr bool FULL = decltype(full)::value;
+        const int slot = i & 1;
+#pragma unroll
+        for (int j = 0; j < CH / 4; j += 4) {
+            // rows of four channels from four tokens of each
+            auto each_row = [&](int which, auto &&store) __attribute__((always_inline)) {
+                Quad f[4];
+#pragma unroll
+                for (int k = 0; k < 4; k++)
+                    f[k] = sm.out[which][slot][j + r0][k * 16 + (threadIdx.x & 15)];
+#pragma unroll
+                for (int e = 0; e < 4; e++)
+                    if (FULL || i * CH + (j + r0) * 4 + e < Tn)
+                        store(j * 4 + e, make_float4(f[0][e], f[1][e], f[2][e], f[3][e]));
+            };
+            // into row k + 4*r0 of the chunk
+            auto put = [&](auto &rows) {
+                return [&](int k, const float4 &f) __attribute__((always_inline)) {
+                    if (WIDE)
+                        *rows.quad(rows.base + i * CH * rows.stride, k) = rows.down(f);
+                    else
+                        rows.store(i * CH + k + r0 * 4, f);
+                };
+            };
+            if constexpr (decltype(xhat)::value)
+                each_row(0, put(xo));
+            if constexpr (SEQ) {
+                each_row(sm.ZP, put(zo));
+                each_row(sm.SC, put(so));
+            }
+            if constexpr (CODES)
+                each_row(sm.Q, [&](int k, const float4 &f) __attribute__((always_inline)) {
+                    auto code = [](float q) { return (q != q) ? (int8_t)0 : (int8_t)q; };
+                    const char4 q = make_char4(code(f.x), code(f.y), code(f.z), code(f.w));
+                    int8_t *p = a.codes + dense + (long)(i * CH + k + r0 * 4) * C + c0 + col;
+                    if (WIDE) {
+                        *reinterpret_cast<char4 *>(p) = q;
+                    } else {
+                        const int8_t kk[4] = {q.x, q.y, q.z, q.w};
+#pragma unroll
+                        for (int n = 0; n < 4; n++)
+                            if (c0 + col + n < C)
+                                p[n] = kk[n];
+                    }
+                });
+        }
+    };
+    // Every phase that repeats has the same loads and stores, a chunk that is not there is loaded as well: where
+    // paths with and without them met, more would be waited for than the loads.
+    auto phases = [&](auto xhat) __attribute__((always_inline)) {
+        load(0);
+        fill(0);
         load(1);
         fill(1);
-    }
-    if (nch > 2)
         load(2);
-    hand_over();
-    int slot = 2; // (i + 2) % 3
-    for (int i = 0; i < nch; i++) {
-        if (i + 2 < nch)
-            fill(slot);
-        if (i + 3 < nch)
-            load(i + 3);
-        if (i > 0)
-            drain(i - 1);
-        slot = slot == 2 ? 0 : slot + 1;
         hand_over();
-    }
-    drain(nch - 1);
+        fill(2);
+        load(3);
+        hand_over();
+        int slot = 0; // (i + 2) % 3
+        auto phase = [&](int i) __attribute__((always_inline)) {
+            fill(slot);
+            load(i + 3);
+            drain(i - 1, xhat, std::true_type());
+            slot = slot == 2 ? 0 : slot + 1;
+            hand_over();
+        };
+        if (nch > 1) {
+            phase(1);
+            for (int i = 2; i < nch; i++)
+                phase(i);
+        }
+        drain(nch - 1, xhat, std::false_type());
+    };
+    if (a.xhat)
+        phases(std::true_type());
+    else
+        phases(std::false_type());
 }
 
-// ~18 instructions per token: 16 of step_spec, half an LDS read and half an LDS write, the two halves of
-// the check.
+// ~16 instructions per token: 15 of step_spec, a quarter of an LDS read and of an LDS write, half of the check.  The
+// chain is the launch: a wave that is alone on its SIMD issues one of them in 4 cycles (the clamps 5, rcp 8, the
+// LDS read of four tokens 12, the write 34), 86 cycles or 36 ns per token; with rows read and written two
+// tokens at a time, NaNs of the scale looked for in every group and the mover waiting for its loads as it asked
+// for them 39.5.  64 blocks x 1024 tokens 45.3 -> 41.9 us, 1024 x 256 in bfloat16 25.4 -> 22.2.
 template <bool SEQ, bool CODES, bool FLOOR>
 __device__ __forceinline__ void recurrence(Shared<SEQ, CODES> &sm, const Tensor &a, int b, int c0, int Tn, int C, int nch,
                                            Limits l)
 {
     const int lane = threadIdx.x & 63;
-    const int c = c0 + lane;
+    const int c = c0 + (lane & 15) * 4 + (lane >> 4);
     Chan ch;
-    ch.init(a, b, min(c, C - 1), C);
+    ch.init(a, b, min(c, C - 1), C, l);
     // med3 takes one scalar operand: the other bound of each pair lives in a vector register
     asm volatile("" : "+v"(l.qu), "+v"(l.sc_max));
 
     // tokens `row`.. of a chunk: results of GRP tokens into slot `o`
-    auto group = [&](const float *x, int row, int o) __attribute__((always_inline)) {
+    auto group = [&](const float *x, int row, int o, auto &&before_results) __attribute__((always_inline)) {
         float xh[GRP], q[GRP], zs[GRP], ss[GRP];
         ch.template steps<FLOOR>(x, l, xh, q, zs, ss);
+        before_results();
+        auto put = [&](int which, const float *f) __attribute__((always_inline)) {
 #pragma unroll
-        for (int k = 0; k < GRP; k++) {
-            sm.out[0][o][row + k][lane] = xh[k];
-            if constexpr (CODES)
-                sm.out[sm.Q][o][row + k][lane] = q[k];
-            if constexpr (SEQ) {
-                sm.out[sm.ZP][o][row + k][lane] = zs[k];
-                sm.out[sm.SC][o][row + k][lane] = ss[k];
-            }
+            for (int k = 0; k < GRP; k += 4)
+                sm.out[which][o][(row + k) / 4][lane] = (Quad){f[k], f[k + 1], f[k + 2], f[k + 3]};
+        };
+        put(0, xh);
+        if constexpr (CODES)
+            put(sm.Q, q);
+        if constexpr (SEQ) {
+            put(sm.ZP, zs);
+            put(sm.SC, ss);
         }
     };
     auto read = [&](float *x, int slot, int row) __attribute__((always_inline)) {
 #pragma unroll
-        for (int k = 0; k < GRP; k++)
-            x[k] = sm.in[slot][row + k][lane];
+        for (int k = 0; k < GRP; k += 4) {
+            const Quad f = sm.in[slot][(row + k) / 4][lane];
+            x[k] = f.x;
+            x[k + 1] = f.y;
+            x[k + 2] = f.z;
+            x[k + 3] = f.w;
+        }
     };
 
     hand_over();
@@ -370,27 +445,33 @@ __device__ __forceinline__ void recurrence(Shared<SEQ, CODES> &sm, const Tensor 
         for (int g = 0; g < CH / GRP; g++) {
             // the next group's rows (past the last chunk: whatever the slot holds, never used)
             read(x[(g + 1) & 1], g + 1 < CH / GRP ? slot : next, (g + 1) * GRP % CH);
-            group(x[g & 1], g * GRP, i & 1);
+            __builtin_amdgcn_sched_barrier(0); // the reads first: they have a group's time
+            group(x[g & 1], g * GRP, i & 1, [&]() __attribute__((always_inline)) {
+                if (g == 0 && i > 0)
+                    hand_over(); // chunk i - 1: its last results are long written by now
+            });
         }
         slot = next;
-        hand_over();
     }
+    if (nfull > 0)
+        hand_over();
     if (nfull < nch) {
         const int o = nfull & 1, n = Tn - nfull * CH;
         int row = 0;
         for (; row + GRP <= n; row += GRP) {
             read(x[0], slot, row);
-            group(x[0], row, o);
+            group(x[0], row, o, []() {});
         }
+        auto word = [&](Quad (&rows)[CH / 4][64]) -> float & { return reinterpret_cast<float *>(&rows[row / 4][lane])[row % 4]; };
         for (; row < n; row++) {
             if constexpr (SEQ) {
-                sm.out[sm.ZP][o][row][lane] = ch.zp;
-                sm.out[sm.SC][o][row][lane] = ch.sc;
+                word(sm.out[sm.ZP][o]) = ch.zp;
+                word(sm.out[sm.SC][o]) = ch.sc;
             }
             float q;
-            sm.out[0][o][row][lane] = ch.step(sm.in[slot][row][lane], l, q);
+            word(sm.out[0][o]) = ch.step(word(sm.in[slot]), l, q);
             if constexpr (CODES)
-                sm.out[sm.Q][o][row][lane] = q;
+                word(sm.out[sm.Q][o]) = q;
         }
         hand_over();
     }
@@ -434,7 +515,7 @@ __global__ __launch_bounds__(64) void quant_direct_kernel(Tensor a0, Tensor a1, 
     if (c >= C)
         return;
     Chan ch;
-    ch.init(a, b, c, C);
+    ch.init(a, b, c, C, l);
     const Bits *xp = (const Bits *)a.x + b * a.xs_b + c;
     Bits *op = a.xhat ? (Bits *)a.xhat + b * a.os_b + c : nullptr;
     const long dense = (long)b * Tn * C + c;
@@ -495,8 +576,8 @@ __global__ __launch_bounds__(64) void quant_direct_kernel(Tensor a0, Tensor a1, 
 // Which kernel: quant_kernel while all its workgroups are resident at once (its LDS allows four on a
 // CU, two with codes or states, one with both), quant_direct_kernel beyond, where many waves hide what
 // quant_kernel moves out of the chain.  us, both kernels, one tensor of
-// fp32, 64-channel blocks x tokens, quant_kernel / quant_direct_kernel: 64 x 1024 45 / 121, 512 x 512
-// 30 / 66, 1024 x 64 9.5 / 12.1, 1024 x 256 23 / 37; 2048 x 64 20 / 12.7, 8192 x 32 36 / 23.
+// fp32, 64-channel blocks x tokens, quant_kernel / quant_direct_kernel: 64 x 1024 42 / 121, 512 x 512
+// 28 / 66, 1024 x 64 9.5 / 12.1, 1024 x 256 21 / 37; 2048 x 64 20 / 13.0, 8192 x 32 36 / 22.
 static int launch(const Tensor *a, int n, int B, int T, int C, int x_dtype, int lower_limit, int upper_limit,
                   float sc_min, float sc_max, hipStream_t st)
 {
