@@ -1643,6 +1643,48 @@ constexpr int SM_KEEP = SM_VEC * SM_NV;               // row elements a thread k
 constexpr int SM_CHUNK = SM_BLOCK * SM_KEEP;          // row elements a 256-thread workgroup holds
 constexpr int SM_ROW_MAX = 24576;                     // longest row a single workgroup keeps in registers
 
+// Rows [.., n] of an additive mask: fp32, fp16 or bfloat16, each widened as it is read (a conversion beforehand is
+// a launch, 3 us of a step that takes 25 to 65).  Rows are as aligned as their elements.
+struct MaskRow {
+    const char *p; // null: no mask
+    int dt;        // ADKV_DT_*
+    __device__ __forceinline__ explicit operator bool() const { return p != nullptr; }
+    __device__ __forceinline__ float widen(uint16_t v) const
+    {
+        return dt == ADKV_DT_F16 ? (float)__builtin_bit_cast(h1, v) : __uint_as_float((uint32_t)v << 16);
+    }
+    __device__ __forceinline__ float at(int i) const
+    {
+        if (dt == ADKV_DT_F32)
+            return reinterpret_cast<const float *>(p)[i];
+        return widen(reinterpret_cast<const uint16_t *>(p)[i]);
+    }
+    template <int V> __device__ __forceinline__ void load(int i, float *m) const
+    {
+        if (dt == ADKV_DT_F32) {
+            __builtin_memcpy(m, p + (size_t)i * 4, 4 * V);
+        } else {
+            uint16_t raw[V];
+            __builtin_memcpy(raw, p + (size_t)i * 2, 2 * V);
+#pragma unroll
+            for (int k = 0; k < V; k++)
+                m[k] = widen(raw[k]);
+        }
+    }
+};
+
+struct Mask {
+    const void *p; // [rows / rows_per_mask_row, n], or null
+    int rows_per_mask_row, dt;
+    // elements t0.. of the row of logits row `row`
+    __device__ __forceinline__ MaskRow of(size_t row, int n, int t0 = 0) const
+    {
+        if (p == nullptr)
+            return {nullptr, dt};
+        return {(const char *)p + (row / (unsigned)rows_per_mask_row * n + t0) * (dt == ADKV_DT_F32 ? 4 : 2), dt};
+    }
+};
+
 template <int NT = SM_BLOCK>
 __device__ __forceinline__ float block_reduce(float v, float *sm, bool is_max)
 {
@@ -1667,7 +1709,7 @@ __device__ __forceinline__ float block_reduce(float v, float *sm, bool is_max)
 // `base` (-inf past the end of the row); 16-byte accesses wherever a whole vector lies inside the
 // row (rows are only 2-byte aligned: the hardware takes unaligned vector accesses).
 template <int NV = SM_NV, int NT = SM_BLOCK>
-__device__ __forceinline__ void softmax_load_chunk(const h1 *l, const float *mk, int n, int base,
+__device__ __forceinline__ void softmax_load_chunk(const h1 *l, const MaskRow &mk, int n, int base,
                                                    float scaling, float *x, float &mx,
                                                    int tid = (int)threadIdx.x)
 {
@@ -1688,7 +1730,7 @@ __device__ __forceinline__ void softmax_load_chunk(const h1 *l, const float *mk,
             }
             if (mk) {
                 float m8[SM_VEC];
-                __builtin_memcpy(m8, mk + i0, 32);
+                mk.load<SM_VEC>(i0, m8);
 #pragma unroll
                 for (int k = 0; k < SM_VEC; k++)
                     xv[k] += m8[k];
@@ -1701,7 +1743,7 @@ __device__ __forceinline__ void softmax_load_chunk(const h1 *l, const float *mk,
                 if (i < n) {
                     xv[k] = (float)l[i] * scaling;
                     if (mk)
-                        xv[k] += mk[i];
+                        xv[k] += mk.at(i);
                 }
             }
         }
@@ -1741,8 +1783,8 @@ __device__ __forceinline__ void softmax_store_chunk(h1 *w, int n, int base, cons
 // elements per thread; rows of a few hundred tokens are the common decode case.
 template <int NV>
 __global__ __launch_bounds__(SM_BLOCK) void softmax_wave_kernel(
-    const h1 *__restrict__ logits, h1 *__restrict__ weights, const float *__restrict__ mask,
-    int rows, int n, long ld, int rows_per_mask_row, float scaling)
+    const h1 *__restrict__ logits, h1 *__restrict__ weights, Mask mask, int rows, int n,
+    long ld, float scaling)
 {
     const int row = blockIdx.x * (SM_BLOCK / 64) + (threadIdx.x >> 6);
     if (row >= rows)
@@ -1750,7 +1792,7 @@ __global__ __launch_bounds__(SM_BLOCK) void softmax_wave_kernel(
     const int lane = threadIdx.x & 63;
     const h1 *l = logits + (size_t)row * ld;
     h1 *w = weights + (size_t)row * ld;
-    const float *mk = mask ? mask + (size_t)(row / rows_per_mask_row) * n : nullptr;
+    const MaskRow mk = mask.of(row, n);
     float x[NV * SM_VEC], mx;
     softmax_load_chunk<NV, 64>(l, mk, n, 0, scaling, x, mx, lane);
 #pragma unroll
@@ -1773,14 +1815,13 @@ __global__ __launch_bounds__(SM_BLOCK) void softmax_wave_kernel(
 // are walked three times (the chunked kernels below avoid that when the caller gives a workspace).
 template <int NT, int NV>
 __global__ __launch_bounds__(NT) void softmax_kernel(
-    const h1 *__restrict__ logits, h1 *__restrict__ weights, const float *__restrict__ mask,
-    int n, long ld, int rows_per_mask_row, float scaling)
+    const h1 *__restrict__ logits, h1 *__restrict__ weights, Mask mask, int n, long ld, float scaling)
 {
     __shared__ float sm[NT / 64];
     const int row = blockIdx.x;
     const h1 *l = logits + (size_t)row * ld;
     h1 *w = weights + (size_t)row * ld;
-    const float *mk = mask ? mask + (size_t)(row / rows_per_mask_row) * n : nullptr;
+    const MaskRow mk = mask.of(row, n);
 
     if (n <= NT * NV * SM_VEC) {
         float x[NV * SM_VEC], mx;
@@ -1799,7 +1840,7 @@ __global__ __launch_bounds__(NT) void softmax_kernel(
     auto at = [&](int i) {
         float v = (float)l[i] * scaling;
         if (mk)
-            v += mk[i];
+            v += mk.at(i);
         return v;
     };
     float mx = -INFINITY;
@@ -1949,13 +1990,12 @@ __device__ __forceinline__ float2 softmax_wave_merge(float2 v)
 // goes to the first chunk's slot and the other slots get the neutral element.
 template <int SUB>
 __global__ __launch_bounds__(SM_BLOCK) void softmax_part_kernel(
-    const h1 *__restrict__ logits, const float *__restrict__ mask, float2 *__restrict__ part,
-    int n, long ld, int nchunk, int rows_per_mask_row, float scaling)
+    const h1 *__restrict__ logits, Mask mask, float2 *__restrict__ part, int n, long ld, int nchunk, float scaling)
 {
     __shared__ float2 sm[SM_BLOCK / 64];
     const int row = blockIdx.y, ck0 = blockIdx.x * SUB;
     const h1 *l = logits + (size_t)row * ld;
-    const float *mk = mask ? mask + (size_t)(row / rows_per_mask_row) * n : nullptr;
+    const MaskRow mk = mask.of(row, n);
     float mx = -INFINITY, sum = 0.0f;
     if (SUB > 1 && !mk && (ck0 + SUB) * SM_CHUNK <= n) {
         uint4 raw[SUB][SM_NV];
@@ -2018,14 +2058,14 @@ __global__ __launch_bounds__(SM_BLOCK) void softmax_part_kernel(
 }
 
 __global__ __launch_bounds__(SM_BLOCK) void softmax_norm_kernel(
-    const h1 *__restrict__ logits, h1 *__restrict__ weights, const float *__restrict__ mask,
-    const float2 *__restrict__ part, int n, long ld, int nchunk, int rows_per_mask_row, float scaling)
+    const h1 *__restrict__ logits, h1 *__restrict__ weights, Mask mask, const float2 *__restrict__ part,
+    int n, long ld, int nchunk, float scaling)
 {
     __shared__ float2 row_stats;
     const int row = blockIdx.y, ck = blockIdx.x;
     const h1 *l = logits + (size_t)row * ld;
     h1 *w = weights + (size_t)row * ld;
-    const float *mk = mask ? mask + (size_t)(row / rows_per_mask_row) * n : nullptr;
+    const MaskRow mk = mask.of(row, n);
     float x[SM_KEEP], mx;
     softmax_load_chunk(l, mk, n, ck * SM_CHUNK, scaling, x, mx);   // issued first: in flight meanwhile
     if (threadIdx.x < 64) {
@@ -3346,13 +3386,12 @@ int64_t adkv_row_pitch(int n)
     return k * 128;
 }
 
-int adkv_softmax_ex(const void *logits, void *weights, const void *mask,
-                    int rows, int n, int64_t ld, int rows_per_mask_row, float scaling,
-                    void *workspace, int64_t workspace_bytes, void *stream)
+static int softmax_launch(const void *logits, void *weights, const Mask &mask, int rows, int n, int64_t ld, float scaling,
+                          void *workspace, int64_t workspace_bytes, void *stream)
 {
     if (!logits || !weights)
         return ADKV_E_NULL;
-    if (rows <= 0 || n <= 0 || (mask && rows_per_mask_row <= 0) || (ld != 0 && ld < n))
+    if (rows <= 0 || n <= 0 || (mask.p && mask.rows_per_mask_row <= 0) || (ld != 0 && ld < n))
         return ADKV_E_SHAPE;
     if (ld == 0)
         ld = n;
@@ -3362,8 +3401,7 @@ int adkv_softmax_ex(const void *logits, void *weights, const void *mask,
         const dim3 grid((unsigned)((rows + SM_BLOCK / 64 - 1) / (SM_BLOCK / 64)));
 #define ADKV_SM_WAVE(NVW)                                                                           \
     hipLaunchKernelGGL(softmax_wave_kernel<NVW>, grid, dim3(SM_BLOCK), 0, (hipStream_t)stream,      \
-                       (const h1 *)logits, (h1 *)weights, (const float *)mask, rows, n, (long)ld,   \
-                       mask ? rows_per_mask_row : 1, scaling)
+                       (const h1 *)logits, (h1 *)weights, mask, rows, n, (long)ld, scaling)
         if (n <= 64 * SM_VEC)
             ADKV_SM_WAVE(1);
         else if (n <= 64 * SM_VEC * 2)
@@ -3374,7 +3412,7 @@ int adkv_softmax_ex(const void *logits, void *weights, const void *mask,
         return check_launch();
     }
     const int reg_nv = (n + 1024 * SM_VEC - 1) / (1024 * SM_VEC); // 16-byte vectors per thread
-    if (n > SM_ROW_MAX && !mask && n <= SM_REG_MAX && (rows >= SM_REG_MIN_ROWS || reg_nv <= 9) &&
+    if (n > SM_ROW_MAX && !mask.p && n <= SM_REG_MAX && (rows >= SM_REG_MIN_ROWS || reg_nv <= 9) &&
         scaling != 0.0f && scaling == scaling) {
         // long unmasked rows stay in registers, unless they are few and very long (32 rows of
         // 131 073: 14.6 us cut into chunks, 19.8 us this way; 128 rows: 28.1 and 24.8; 512 rows:
@@ -3401,8 +3439,7 @@ int adkv_softmax_ex(const void *logits, void *weights, const void *mask,
         // once); rows beyond 24576 elements without a workspace are read three times
 #define ADKV_SM_ROW(NT, NV)                                                                         \
     hipLaunchKernelGGL((softmax_kernel<NT, NV>), dim3((unsigned)rows), dim3(NT), 0,                 \
-                       (hipStream_t)stream, (const h1 *)logits, (h1 *)weights, (const float *)mask, \
-                       n, (long)ld, mask ? rows_per_mask_row : 1, scaling)
+                       (hipStream_t)stream, (const h1 *)logits, (h1 *)weights, mask, n, (long)ld, scaling)
         // (threads, 16-byte vectors per thread) per row length, measured on 4096 rows: 4097 elements
         // 18.4 us with 256 x 3 and 16.7 with 320 x 2; 8192: 35.5 with 512 x 3, 24.3 with 512 x 2;
         // 10000: 36.9 with 512 x 3, 33.0 with 256 x 6; 16384: 76.5 with 1024 x 3, 46.9 with 1024 x 2;
@@ -3428,22 +3465,26 @@ int adkv_softmax_ex(const void *logits, void *weights, const void *mask,
         return ADKV_E_ALIGN;
     const int nchunk = (n + SM_CHUNK - 1) / SM_CHUNK;
     const dim3 grid((unsigned)nchunk, (unsigned)rows);
-    if (nchunk >= 8 && !mask) {
+    if (nchunk >= 8 && !mask.p) {
         // long rows: four chunks per workgroup in the first pass
         const dim3 grid4((unsigned)((nchunk + 3) / 4), (unsigned)rows);
         hipLaunchKernelGGL(softmax_part_kernel<4>, grid4, dim3(SM_BLOCK), 0, (hipStream_t)stream,
-                           (const h1 *)logits, (const float *)mask, (float2 *)workspace, n, (long)ld, nchunk,
-                           1, scaling);
+                           (const h1 *)logits, mask, (float2 *)workspace, n, (long)ld, nchunk, scaling);
     } else {
         hipLaunchKernelGGL(softmax_part_kernel<1>, grid, dim3(SM_BLOCK), 0, (hipStream_t)stream,
-                           (const h1 *)logits, (const float *)mask, (float2 *)workspace, n, (long)ld, nchunk,
-                           mask ? rows_per_mask_row : 1, scaling);
+                           (const h1 *)logits, mask, (float2 *)workspace, n, (long)ld, nchunk, scaling);
     }
     hipLaunchKernelGGL(softmax_norm_kernel, grid, dim3(SM_BLOCK), 0, (hipStream_t)stream,
-                       (const h1 *)logits, (h1 *)weights, (const float *)mask,
-                       (const float2 *)workspace, n, (long)ld, nchunk, mask ? rows_per_mask_row : 1,
-                       scaling);
+                       (const h1 *)logits, (h1 *)weights, mask, (const float2 *)workspace, n, (long)ld, nchunk, scaling);
     return check_launch();
+}
+
+int adkv_softmax_ex(const void *logits, void *weights, const void *mask,
+                    int rows, int n, int64_t ld, int rows_per_mask_row, float scaling,
+                    void *workspace, int64_t workspace_bytes, void *stream)
+{
+    return softmax_launch(logits, weights, {mask, rows_per_mask_row, ADKV_DT_F32}, rows, n, ld, scaling, workspace,
+                          workspace_bytes, stream);
 }
 
 int adkv_softmax(const void *logits, void *weights, const void *mask,
@@ -3550,9 +3591,13 @@ int adkv_decode_step(const void *q, void *k_cache, void *v_cache, const void *k_
 {
     if (!k_params || !v_params || !workspace)
         return workspace ? ADKV_E_NULL : ADKV_E_WORKSPACE;
-    if (act_dtype != ADKV_DT_F16 && act_dtype != ADKV_DT_BF16)
+    const int mask_dtype = act_dtype >> 8;
+    act_dtype &= 255;
+    if ((act_dtype != ADKV_DT_F16 && act_dtype != ADKV_DT_BF16) ||
+        (mask_dtype != ADKV_DT_F32 && mask_dtype != ADKV_DT_F16 && mask_dtype != ADKV_DT_BF16))
         return ADKV_E_UNSUPPORTED;
     const int act_bf16 = act_dtype == ADKV_DT_BF16;
+    const Mask mk = {mask, rows_per_mask_row, mask_dtype};
     if (B <= 0 || H <= 0 || Hq <= 0 || Hq % H || T < 0)
         return ADKV_E_SHAPE;
     if (workspace_bytes < adkv_decode_step_workspace_bytes(B, Hq, H, T, D, n_ckpt_cap, ckpt_interval))
@@ -3605,8 +3650,7 @@ int adkv_decode_step(const void *q, void *k_cache, void *v_cache, const void *k_
             va.ckpt = (h1 *)v_ckpt;
             const FtParams kp = ft_params(k_params), vp = ft_params(v_params);
             hipLaunchKernelGGL(small_step_kernel, dim3((unsigned)(B * H)), dim3(256), 0, (hipStream_t)stream, (const h1 *)q,
-                               (uint4 *)k_cache, (const h1 *)k_new, (uint4 *)v_cache, (const h1 *)v_new, (const float *)mask,
-                               mask ? rows_per_mask_row : 1, (h1 *)weights, (h1 *)out, kp, vp, H, T,
+                               (uint4 *)k_cache, (const h1 *)k_new, (uint4 *)v_cache, (const h1 *)v_new, mk, (h1 *)weights, (h1 *)out, kp, vp, H, T,
                                n_super_cap, scaling, ka, va);
             return (rc = check_launch()) ? rc : mark_one_launch(stream);
         }
@@ -3625,7 +3669,6 @@ int adkv_decode_step(const void *q, void *k_cache, void *v_cache, const void *k_
             Seg va = ka;
             va.ckpt = (h1 *)v_ckpt;
             const long rows = (long)B * Hq;
-            const StepMask mk = {(const float *)mask, mask ? rows_per_mask_row : 1};
             float4 *ml = (float4 *)(ws + 2 * mat);
             float *partial = (float *)(ws + 2 * mat + pad256(ka.nseg * rows * 16));
             if ((rc = launch_step_segments(cpl, Hq / H, bits, D, B * H, ka.nseg, (hipStream_t)stream, (const h1 *)q, (uint4 *)k_cache,
@@ -3649,8 +3692,7 @@ int adkv_decode_step(const void *q, void *k_cache, void *v_cache, const void *k_
     if (rc || (rc = stage_mark(1, stream)))
         return rc;
     const int64_t smb = pad256(adkv_softmax_workspace_bytes(B * Hq, T + 1));
-    rc = adkv_softmax_ex(logits, weights, mask, B * Hq, T + 1, ld, rows_per_mask_row, scaling,
-                         smb ? ws + 2 * mat : nullptr, smb, stream);
+    rc = softmax_launch(logits, weights, mk, B * Hq, T + 1, ld, scaling, smb ? ws + 2 * mat : nullptr, smb, stream);
     if (rc || (rc = stage_mark(2, stream)))
         return rc;
     rc = forward_ov_impl(weights, v_cache, v_new, out, v_params[0], v_params[1], v_params[2],

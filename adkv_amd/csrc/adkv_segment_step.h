@@ -20,11 +20,6 @@ namespace adkv {
 // query heads) and one, in whole 16-byte vectors.
 template <int GQ> constexpr int step_cap() { return GQ == 8 ? 264 : 520; }
 
-struct StepMask {
-    const float *mask; // [rows / rows_per_mask_row, n], or null
-    int rows_per_mask_row;
-};
-
 // max or sum over the LPH lanes of a head, in registers: four rotations within the row of 16 lanes, then
 // the row and half swaps.  (Through the LDS, as __shfl_xor goes, the dozen trips per head took 4 of the 55
 // us of a step of 256-token segments with four query heads.)
@@ -66,7 +61,7 @@ __device__ __forceinline__ float head_reduce(float v)
 // rounding, go to ml[g].  logits: the first head's row at
 // the segment's first token, 16-byte aligned, its pitch a multiple of 8.
 template <int LPH, int GQ>
-__device__ __forceinline__ void segment_weights(const h1 *logits, long pitch, const StepMask &mk, long row0, int n, int t0,
+__device__ __forceinline__ void segment_weights(const h1 *logits, long pitch, const Mask &mk, long row0, int n, int t0,
                                                 int ntok, float scaling, h1 *p, float4 *ml, int lh, bool active)
 {
     constexpr int V = 256 / LPH, CAP = step_cap<GQ>(), NC = (CAP + 255) / 256; // values per lane, chunks of 256 tokens
@@ -83,7 +78,7 @@ __device__ __forceinline__ void segment_weights(const h1 *logits, long pitch, co
         }
 #pragma unroll
     for (int g = 0; g < GQ; g++) {
-        const float *mrow = mk.mask ? mk.mask + (size_t)((row0 + g) / mk.rows_per_mask_row) * n + t0 : nullptr;
+        const MaskRow mrow = mk.of(row0 + g, n, t0);
         float x[NC][V], mx = -INFINITY;
 #pragma unroll
         for (int c = 0; c < NC; c++) {
@@ -93,20 +88,20 @@ __device__ __forceinline__ void segment_weights(const h1 *logits, long pitch, co
             vec_words(raw[g][c], w);
             const int t = c * 256 + lh * V;
             float add[V];
-            if (mrow != nullptr) {
+            if (mrow) {
                 if (t + V <= ntok) {
-                    __builtin_memcpy(add, mrow + t, 4 * V);
+                    mrow.load<V>(t, add);
                 } else {
 #pragma unroll
                     for (int k = 0; k < V; k++)
-                        add[k] = t + k < ntok ? mrow[t + k] : 0.0f;
+                        add[k] = t + k < ntok ? mrow.at(t + k) : 0.0f;
                 }
             }
 #pragma unroll
             for (int k = 0; k < V; k++) {
                 const h2 pair = as_h2(w[k / 2]);
                 float v = (float)(k & 1 ? pair.y : pair.x) * scaling;
-                if (mrow != nullptr)
+                if (mrow)
                     v += add[k];
                 x[c][k] = t + k < ntok ? v : -INFINITY;
                 mx = fmaxf(mx, x[c][k]);
@@ -150,7 +145,7 @@ struct StepShape {
 
 template <int D, int CPL, int BITS, int GQ, int BLK>
 __global__ __launch_bounds__(BLK) void step_segments_kernel(
-    const h1 *q, uint4 *__restrict__ k_cache, const h1 *k_new, uint4 *__restrict__ v_cache, const h1 *v_new, StepMask mk,
+    const h1 *q, uint4 *__restrict__ k_cache, const h1 *k_new, uint4 *__restrict__ v_cache, const h1 *v_new, Mask mk,
     h1 *logits, float *__restrict__ partial, float4 *__restrict__ ml, FtParams kp, FtParams vp, int BH, int H, int T,
     int n_super_cap, float scaling, Seg ka, Seg va)
 {
@@ -236,7 +231,7 @@ __global__ __launch_bounds__(BLK) void step_segments_kernel(
 // outputs: all 128 channels in two groups of segments, or, with many segments, 16 channels in 16 groups.
 // Sums are taken in a fixed order.
 __global__ __launch_bounds__(256) void step_combine_kernel(
-    const h1 *__restrict__ logits, h1 *__restrict__ weights, h1 *__restrict__ out, StepMask mk,
+    const h1 *__restrict__ logits, h1 *__restrict__ weights, h1 *__restrict__ out, Mask mk,
     const float *__restrict__ partial, const float4 *__restrict__ ml, long rows, int n, long pitch, int D, int nseg,
     float scaling, int out_waves, int act_bf16)
 {
@@ -267,15 +262,15 @@ __global__ __launch_bounds__(256) void step_combine_kernel(
         if (t >= n)
             return;
         const uint32_t w[4] = {raw.x, raw.y, raw.z, raw.w};
-        const float *mrow = mk.mask ? mk.mask + (size_t)(row / mk.rows_per_mask_row) * n : nullptr;
+        const MaskRow mrow = mk.of(row, n);
         uint32_t o[4];
 #pragma unroll
         for (int k = 0; k < 4; k++) {
             const h2 l = as_h2(w[k]);
             float a = (float)l.x * scaling, b = (float)l.y * scaling;
-            if (mrow != nullptr) {
-                a += mrow[min(t + 2 * k, n - 1)];
-                b += mrow[min(t + 2 * k + 1, n - 1)];
+            if (mrow) {
+                a += mrow.at(min(t + 2 * k, n - 1));
+                b += mrow.at(min(t + 2 * k + 1, n - 1));
             }
             o[k] = as_u32((h2){(h1)(__expf(a - M) * inv), (h1)(__expf(b - M) * inv)});
         }

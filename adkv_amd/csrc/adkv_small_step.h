@@ -15,7 +15,7 @@ constexpr int SMALL_ROW = 3 * 64 * SM_VEC; // longest row of logits: three vecto
 
 __global__ __launch_bounds__(256) void small_step_kernel(
     const h1 *q, uint4 *__restrict__ k_cache, const h1 *k_new, uint4 *__restrict__ v_cache,
-    const h1 *v_new, const float *__restrict__ mask, int rows_per_mask_row, h1 *__restrict__ weights,
+    const h1 *v_new, Mask mask, h1 *__restrict__ weights,
     h1 *__restrict__ out, FtParams kp, FtParams vp, int H, int T, int n_super_cap, float scaling, Seg ka, Seg va)
 {
     constexpr int D = 128, CPL = 2;
@@ -84,7 +84,7 @@ __global__ __launch_bounds__(256) void small_step_kernel(
         // for another, and the copy it reads from is its own.
         h1 *w = reinterpret_cast<h1 *>(tile);
         float x[SMALL_ROW / 64], mx;
-        softmax_load_chunk<SMALL_ROW / 512, 64>(logits, mask ? mask + (size_t)(bx / rows_per_mask_row) * n : nullptr, n, 0,
+        softmax_load_chunk<SMALL_ROW / 512, 64>(logits, mask.of(bx, n), n, 0,
                                                 scaling, x, mx, lane);
 #pragma unroll
         for (int m = 1; m < 64; m <<= 1)

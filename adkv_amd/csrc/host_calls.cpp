@@ -7,6 +7,8 @@
 // of one current device, of the right shapes, dtypes and layouts, a workspace that is large enough) and
 // returns None for all others: the Python function that called it then goes its own way, with its own
 // conversions and error messages.  A number is the library's return code.
+#include <algorithm>
+
 #include <torch/csrc/autograd/python_variable.h>
 
 #include <ATen/ATen.h>
@@ -197,7 +199,7 @@ PyObject *decode(PyObject *, PyObject *const *args, Py_ssize_t nargs)
         Py_RETURN_NONE;
     const int64_t n = T + 1;
     const at::Tensor *mask = nullptr;
-    int rows_per_mask_row = 1;
+    int rows_per_mask_row = 1, mask_type = -1; // the type as the kernels read it, -1: to fp32 first
     if (args[12] != Py_None) {
         mask = plain(args[12]);
         if (!mask || mask->device() != q.device() || !at::isFloatingType(mask->scalar_type()) ||
@@ -205,6 +207,8 @@ PyObject *decode(PyObject *, PyObject *const *args, Py_ssize_t nargs)
             (mask->size(1) != 1 && mask->size(1) != Hq) || mask->size(-1) != n)
             Py_RETURN_NONE;
         rows_per_mask_row = mask->size(1) == 1 ? (int)Hq : 1;
+        mask_type = mask->scalar_type() == at::kFloat ? ADKV_DT_F32 : mask->scalar_type() == at::kHalf ? ADKV_DT_F16
+                    : mask->scalar_type() == at::kBFloat16 ? ADKV_DT_BF16 : -1;
     }
     void *stream;
     if (!current(q.device(), stream))
@@ -216,12 +220,12 @@ PyObject *decode(PyObject *, PyObject *const *args, Py_ssize_t nargs)
     const int64_t need = adkv_decode_step_workspace_bytes((int)B, (int)Hq, (int)H, (int)T, (int)D, (int)n_ckpt, (int)interval);
     if (!ws || ws->scalar_type() != at::kByte || ws->numel() < need || !ws->is_contiguous() || ws->device() != q.device())
         Py_RETURN_NONE;
-    at::Tensor out, weights, m32, scratch = *ws; // held: another thread may replace the dictionary's entry
+    at::Tensor out, weights, m, scratch = *ws; // held: another thread may replace the dictionary's entry
     int rc;
     try {
         if (mask) {
-            m32 = mask->to(at::kFloat).contiguous();
-            if (!m32.has_storage())
+            m = (mask_type >= 0 ? *mask : mask->to(at::kFloat)).contiguous();
+            if (!m.has_storage())
                 Py_RETURN_NONE;
         }
         const int64_t pitch = adkv_row_pitch((int)n);
@@ -230,13 +234,14 @@ PyObject *decode(PyObject *, PyObject *const *args, Py_ssize_t nargs)
         if (!out.has_storage() || !weights.has_storage())
             Py_RETURN_NONE;
         void *op = out.mutable_data_ptr(), *wp = weights.mutable_data_ptr();
-        const void *mp = mask ? m32.const_data_ptr() : nullptr;
+        const void *mp = mask ? m.const_data_ptr() : nullptr;
         const double scaling = PyFloat_AS_DOUBLE(args[11]);
         Py_BEGIN_ALLOW_THREADS
         rc = adkv_decode_step(q.const_data_ptr(), kc->mutable_data_ptr(), vc->mutable_data_ptr(), kn->const_data_ptr(),
                               vn->const_data_ptr(), params, params + 5, mp, rows_per_mask_row, (float)scaling, op, wp, pitch, (int)B,
                               (int)Hq, (int)H, (int)T, (int)D, (int)n_super, (int)bits,
-                              q.scalar_type() == at::kBFloat16 ? ADKV_DT_BF16 : ADKV_DT_F16, ck[0], ck[1], (int)n_ckpt, (int)interval,
+                              (q.scalar_type() == at::kBFloat16 ? ADKV_DT_BF16 : ADKV_DT_F16) | ADKV_MASK_DT(std::max(mask_type, ADKV_DT_F32)),
+                              ck[0], ck[1], (int)n_ckpt, (int)interval,
                               scratch.mutable_data_ptr(), scratch.numel(), stream);
         Py_END_ALLOW_THREADS
         const int64_t sizes[3] = {B, Hq, n}, strides[3] = {Hq * pitch, pitch, 1};

@@ -355,6 +355,7 @@ def append_kv(
 
 
 _DT_F16, _DT_BF16 = 1, 2     # ADKV_DT_F16 / ADKV_DT_BF16 of include/adkv_hip.h
+_MASK_DT = {torch.float16: _DT_F16, torch.bfloat16: _DT_BF16}     # masks read as they are; any other becomes fp32
 
 
 def _row_strides(t: torch.Tensor):
@@ -587,13 +588,14 @@ def decode_step(
     _chk(DIM in _DIMS, "DIM must be 128, 256 or 512")
     dev = _need_device(q, k_cache, v_cache, k_new, v_new, *kp, *vp)
     n = T + 1
-    rpm, mptr, mk = 1, None, None
+    rpm, mptr, mk, mdt = 1, None, None, 0
     if mask is not None:
         mk = mask[:, :, 0, :] if mask.dim() == 4 else mask
         _chk(mk.dim() == 3 and mk.shape[0] == B and mk.shape[2] == n and mk.shape[1] in (1, nq),
              "mask must broadcast to [B, nh, n]")
         rpm = nq if mk.shape[1] == 1 else 1
-        mk = mk.to(device=dev, dtype=torch.float32).contiguous()
+        mdt = _MASK_DT.get(mk.dtype, 0)
+        mk = mk.to(device=dev, dtype=mk.dtype if mdt else torch.float32).contiguous()
         mptr = mk.data_ptr()
     kcp, ccap, civ = _ckpt_args(k_ckpt, ckpt_interval, B, nh, DIM, bits)
     vcp, vcap, _ = _ckpt_args(v_ckpt, ckpt_interval, B, nh, DIM, bits)
@@ -617,7 +619,7 @@ def decode_step(
             qf.data_ptr(), k_cache.data_ptr(), v_cache.data_ptr(), knf.data_ptr(), vnf.data_ptr(),
             arr(*[t.data_ptr() for t in kp]), arr(*[t.data_ptr() for t in vp]),
             mptr, rpm, float(scaling), out.data_ptr(), weights.data_ptr(), wld,
-            B, nq, nh, T, DIM, n_super_cap, bits, _DT_BF16 if act == torch.bfloat16 else _DT_F16,
+            B, nq, nh, T, DIM, n_super_cap, bits, (_DT_BF16 if act == torch.bfloat16 else _DT_F16) | mdt << 8,
             kcp, vcp, ccap, civ,
             workspace.data_ptr(), workspace.numel(), _lib.current_stream_ptr(dev))
     _lib.check(rc, "decode_step")

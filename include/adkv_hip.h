@@ -287,13 +287,14 @@ int adkv_forward_ov_noalloc(const void *attn, void *v_cache, const void *v_new, 
  * Replaces the body of KVCacheLayer_ADKV.decode (src/adkv/hf/llama_adkv.py:245-276).
  * q: fp16 [B, Hq, D] with Hq a multiple of the H KV heads (Hq == H is the reference's case).
  * k_params / v_params: host arrays of five device pointers {zp, sc, alpha, beta, tgt}, each
- * fp16 [H, D].  mask: optional fp32 additive mask as in adkv_softmax.  out: fp16 [B, Hq, D].
+ * fp16 [H, D].  mask: optional additive mask as in adkv_softmax, fp32 or of the type given in act_dtype.  out: fp16 [B, Hq, D].
  * weights_out: optional fp16 [B, Hq, weights_ld] with weights_ld == adkv_row_pitch(T + 1), columns
  * 0..T valid (the attention weights the reference returns); when NULL they live in the workspace.  Checkpoint tensors as in the _ex entry points (NULL = none).
  * act_dtype: ADKV_DT_F16, or ADKV_DT_BF16 when q, k_new, v_new and out are bfloat16: they are
  * rounded to fp16 as they are read and the fp16 result to bf16 as it is written, the values of
  * the reference's .to(torch.float16) / .to(q.dtype) around its kernels (llama_adkv.py:248-250, 274)
- * without the four conversion launches.  Logits and weights stay fp16.
+ * without the four conversion launches.  Logits and weights stay fp16.  act_dtype | ADKV_MASK_DT(dt): a mask
+ * of fp16 or bfloat16 (dt ADKV_DT_F16 or ADKV_DT_BF16) is widened as it is read.
  * workspace: >= adkv_decode_step_workspace_bytes(...) bytes, 256-byte aligned.
  */
 int64_t adkv_decode_step_workspace_bytes(int B, int Hq, int H, int T, int D, int n_ckpt_cap,
@@ -356,6 +357,7 @@ void adkv_set_stage_events(void *const *events);
 #define ADKV_DT_F32 0
 #define ADKV_DT_F16 1
 #define ADKV_DT_BF16 2
+#define ADKV_MASK_DT(dt) ((dt) << 8) /* in act_dtype of adkv_decode_step: the mask's type */
 int adkv_quant_f32(const void *x, void *xhat, void *codes, void *zp_state, void *sc_state,
                    const void *zp_init, const void *sc_init, const void *alpha,
                    const void *beta, const void *tgt, void *zp_seq, void *sc_seq,
