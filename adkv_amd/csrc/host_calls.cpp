@@ -311,11 +311,11 @@ PyObject *append(PyObject *, PyObject *const *args, Py_ssize_t nargs)
     return PyLong_FromLong(rc);
 }
 
-// quant_f32(x, (alpha, beta, target, zp_init, sc_init), lower, upper, sc_min, sc_max, output_states)
+// quant_f32(x, (alpha, beta, target, zp_init, sc_init), lower, upper, sc_min, sc_max, output_states, free_params)
 //   -> (xhat, zp sequence or None, sc sequence or None)
 PyObject *quant_f32(PyObject *, PyObject *const *args, Py_ssize_t nargs)
 {
-    if (nargs != 7 || !unwatched() || !PyFloat_CheckExact(args[4]) || !PyFloat_CheckExact(args[5]))
+    if (nargs != 8 || !unwatched() || !PyFloat_CheckExact(args[4]) || !PyFloat_CheckExact(args[5]))
         Py_RETURN_NONE;
     const at::Tensor *x = plain(args[0]);
     const long lower = PyLong_AsLong(args[2]), upper = PyLong_AsLong(args[3]);
@@ -344,7 +344,8 @@ PyObject *quant_f32(PyObject *, PyObject *const *args, Py_ssize_t nargs)
             Py_RETURN_NONE;
         void *op = out.mutable_data_ptr(), *zp = state.mutable_data_ptr(), *sc = (float *)zp + B * C;
         void *sp[2] = {seq[0].defined() ? seq[0].mutable_data_ptr() : nullptr, seq[1].defined() ? seq[1].mutable_data_ptr() : nullptr};
-        const int type = x->scalar_type() == at::kFloat ? ADKV_DT_F32 : x->scalar_type() == at::kHalf ? ADKV_DT_F16 : ADKV_DT_BF16;
+        const int type = (x->scalar_type() == at::kFloat ? ADKV_DT_F32 : x->scalar_type() == at::kHalf ? ADKV_DT_F16 : ADKV_DT_BF16) |
+                         (args[7] == Py_True ? ADKV_PARAMS_FREE : 0);
         const double lo = PyFloat_AS_DOUBLE(args[4]), hi = PyFloat_AS_DOUBLE(args[5]);
         Py_BEGIN_ALLOW_THREADS
         rc = adkv_quant_f32(x->const_data_ptr(), op, nullptr, zp, sc, p[3], p[4], p[0], p[1], p[2], sp[0], sp[1], (int)B, (int)T, (int)C,

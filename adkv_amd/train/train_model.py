@@ -17,6 +17,7 @@ from .. import _lib
 from ..kernel.gemv import _chk, _need_device
 
 _DTYPES = {torch.float32: 0, torch.float16: 1, torch.bfloat16: 2}
+_PARAMS_FREE = 256     # ADKV_PARAMS_FREE of include/adkv_hip.h
 
 
 def _f32vec(t: torch.Tensor, n: int, name: str) -> torch.Tensor:
@@ -29,17 +30,18 @@ def quant_f32(x: torch.Tensor, alpha: torch.Tensor, beta: torch.Tensor, target: 
               zp_state: torch.Tensor | None = None, sc_state: torch.Tensor | None = None,
               zp_init: torch.Tensor | None = None, sc_init: torch.Tensor | None = None,
               out: torch.Tensor | None = None, want_codes: bool = False,
-              output_states: bool = False):
+              output_states: bool = False, free_params: bool = False):
     """Fake-quantise ``x [B, T, C]`` (fp32 / fp16 / bf16, channel stride 1) along ``T``.
 
     State: ``zp_state`` / ``sc_state`` fp32 ``[B, C]`` are updated in place; they are also the
     starting state unless ``zp_init`` / ``sc_init`` ``[C]`` are given.  ``out`` may be ``x`` itself
-    (in-place, as the reference's eval cache does).  Returns ``(xhat, codes | None, zp_seq | None,
+    (in-place, as the reference's eval cache does).  With ``free_params`` the unconstrained parameters of
+    training are given: ``sigmoid(alpha)``, ``0.1 * sigmoid(beta)`` and ``exp(sc_init)`` are used.  Returns ``(xhat, codes | None, zp_seq | None,
     sc_seq | None)``.
     """
     if zp_state is None and sc_state is None and out is None and not want_codes:
         r = _lib.host().quant_f32(x, (alpha, beta, target, zp_init, sc_init), lower_limit, upper_limit,
-                                  float(sc_min), float(sc_max), bool(output_states))
+                                  float(sc_min), float(sc_max), bool(output_states), bool(free_params))
         if r is not None:      # None: something to check, convert or complain about below
             if isinstance(r, int):
                 _lib.check(r, "quant_f32")
@@ -74,7 +76,7 @@ def quant_f32(x: torch.Tensor, alpha: torch.Tensor, beta: torch.Tensor, target: 
         rc = _lib.lib().adkv_quant_f32(
             x.data_ptr(), out.data_ptr(), p(codes), zp_state.data_ptr(), sc_state.data_ptr(),
             p(zi), p(si), al.data_ptr(), be.data_ptr(), tg.data_ptr(), p(zs), p(ss),
-            B, T, C, sb, st, _DTYPES[x.dtype], int(lower_limit), int(upper_limit),
+            B, T, C, sb, st, _DTYPES[x.dtype] | (_PARAMS_FREE if free_params else 0), int(lower_limit), int(upper_limit),
             float(sc_min), float(sc_max), _lib.current_stream_ptr(dev))
     _lib.check(rc, "quant_f32")
     return out, codes, zs, ss
@@ -170,8 +172,13 @@ class ADKVTrainModel(nn.Module):
         B, T, C = kv_cache.shape
         assert C == self.num_hidden_states
         assert self.truncation % CHUNK == 0
-        out, _, zs, ss = quant_f32(kv_cache, self.get_alpha(), self.get_beta(), self.target,
+        # The launch constrains fp32 parameters itself; a subclass's or an instance's own way stays in force.
+        free = (self.alpha.dtype == self.beta.dtype == self.init_log_sc.dtype == torch.float32
+                and all(getattr(type(self), f) is getattr(ADKVTrainModel, f) and f not in self.__dict__
+                        for f in ("get_alpha", "get_beta", "get_sc")))
+        out, _, zs, ss = quant_f32(kv_cache, self.alpha if free else self.get_alpha(),
+                                   self.beta if free else self.get_beta(), self.target,
                                    self.lower_limit, self.upper_limit, self.sc_min, self.sc_max,
-                                   zp_init=self.init_zp, sc_init=self.get_sc(),
-                                   output_states=output_states)
+                                   zp_init=self.init_zp, sc_init=self.init_log_sc if free else self.get_sc(),
+                                   output_states=output_states, free_params=free)
         return (out, zs, ss) if output_states else out

@@ -353,11 +353,14 @@ void adkv_set_stage_events(void *const *events);
  *             (train_model.py:66-68)
  *   lower_limit/upper_limit   integer code range (train_model.py:96-97), sc_min/sc_max the
  *             clamp of the scale (train_model.py:98-99).
+ * x_dtype | ADKV_PARAMS_FREE: alpha, beta and sc_init (then required, with zp_init) are the unconstrained
+ * parameters; sigmoid(alpha), 0.1*sigmoid(beta) and exp(sc_init) of them are used (train_model.py:127-134).
  */
 #define ADKV_DT_F32 0
 #define ADKV_DT_F16 1
 #define ADKV_DT_BF16 2
 #define ADKV_MASK_DT(dt) ((dt) << 8) /* in act_dtype of adkv_decode_step: the mask's type */
+#define ADKV_PARAMS_FREE 256         /* in x_dtype of adkv_quant_f32 */
 int adkv_quant_f32(const void *x, void *xhat, void *codes, void *zp_state, void *sc_state,
                    const void *zp_init, const void *sc_init, const void *alpha,
                    const void *beta, const void *tgt, void *zp_seq, void *sc_seq,
