@@ -491,13 +491,16 @@ struct SegLoads {
 // The state at token t depends on every code before it, so the encoder is one serial chain per
 // channel and nothing but B*H*D is parallel.  A lane owns CPL consecutive channels (1 or 2, the
 // launcher's choice).  With few channels a wave has its SIMD to itself, and a wave alone issues one
-// instruction every 4 cycles whether or not it depends on the one before (8 for v_rcp_f32 and
-// v_fma_f16; s_nop, s_waitcnt and scalar instructions take a slot as well): the time per token is
-// the NUMBER of instructions, and the loop below is written for that number.
-//  * rows come through buffer loads (16 bits per lane with one channel, 32 with two): one
-//    instruction per token and nothing else, because the row offsets within a group of 8 tokens
-//    sit in scalar registers and loads past the end of the stream are dropped by the bounds check
-//    instead of being guarded;
+// instruction every 4 cycles whether or not it depends on the one before (5 for 8-byte encodings, 8 for
+// v_rcp_f32 and v_fma_f16, 16 and more for a load, 24 and more for a store): the time per token is the
+// sum over its instructions, and the loops below are written for that sum.
+//  * one channel per lane, rows 16-byte aligned: 8 rows come into the LDS with one buffer load, a run of
+//    64 tokens ahead, and a lane reads four tokens of its channel with one transposing LDS read (a load
+//    per token was 4 of 39 ns);
+//  * otherwise rows come through buffer loads into registers (16 bits per lane with one channel, 32 with
+//    two): one instruction per token and nothing else, because the row offsets within a group of 8 tokens
+//    sit in scalar registers.  Loads past the end of the stream are dropped by the bounds check instead of
+//    being guarded;
 //  * the quotient takes three instructions on top of the reciprocal and is the IEEE one
 //    (enc_quotient), so nothing has to be checked or repeated for finite values: a form that takes
 //    the reciprocal product alone and repeats the groups of 8 tokens in which it comes near a
@@ -875,7 +878,7 @@ __device__ __forceinline__ void encode_body(
         // during this one's steps; then the loop above starts anew behind it.  A channel whose scale is
         // zero, or whose state is a NaN, meets one in every run: as long as no run is clean, twice as many
         // words are taken here each time (up to 16 runs), so that such a wave hardly tries the fast form:
-        // 86 ns per token of one channel against 38 in the loop above (145 with a load per token).
+        // 83 ns per token of one channel against 34 of whole runs (145 with a load per token).
         redo = sg == resumed ? min(redo * 2, 16 * (PF / G8)) : PF / G8;
         dst = cw + (size_t)sg * D + lane * CPL;
         xoff = (uint32_t)lane * 2u * CPL + row * 8u * (uint32_t)g;
@@ -2825,13 +2828,24 @@ static int encode_common(void *cache, const void *kv_new,
     seg.fresh = fresh ? 1 : 0;
     // Lane width: one channel per lane while every wave then has a SIMD to itself (its time per token is
     // its instruction count, 17 against 30 with two channels), two channels beyond (they share the
-    // packed updates and the wave's fixed cost).  ns per token, fp16 rows of 8192 tokens, 4-bit codes, at
-    // 0.25 / 1 / 1.5 / 2 one-channel waves per SIMD: one channel 37 / 42 / 67 / 71, two - / - / 64 / 69
-    // (4.8 TB/s; with 8 two-channel waves per SIMD 4.5 TB/s and the vector pipe 85 % busy).  Before the
-    // loop was written for its instruction count: 61 at one wave per SIMD.
+    // packed updates and the wave's fixed cost), but for launches of two to three one-channel waves per
+    // SIMD: two channels per lane put two waves on some SIMDs and one on others, and take as long as two
+    // everywhere; one channel per lane takes a round of two waves (their LDS) and a round of one, which
+    // is less from some 300 tokens on, where rows come through the LDS.  us, bf16 rows, 4-bit codes, one
+    // channel / two, at 2.12, 2.5 and 3 one-channel waves per SIMD: 128 tokens 18.9 / 19.5, 19.9 / 20.0,
+    // 21.3 / 19.8; 500 tokens 57 / 62, 58 / 62, 59 / 62; 2048 tokens 200 / 232, 205 / 234, 214 / 238.  Outside: 1.25
+    // 41 / 37 (500 tokens) and 137 / 135 (2048), 2 42 / 38 and 282 / 278 (4096), 3.25 76 / 65 and 267 / 247,
+    // 16 290 / 285 (512; 4.5 TB/s and the vector pipe 85 % busy).
     const long channels = (long)BH * D;
     const long tensors = second ? 2 : 1;
-    int cpl = tensors * channels > 64L * n_simd() ? 2 : 1;
+    const long one_per_simd = 64L * n_simd(), all = tensors * channels;
+    auto lds_rows = [](const void *x, const RowStrides &s) {
+        return ((uintptr_t)x & 15) == 0 && s.t % 8 == 0 && s.h % 8 == 0 && s.b % 8 == 0;
+    };
+    const bool two_and_one = all > 2 * one_per_simd && all <= 3 * one_per_simd && T - T0 >= 384 && lds_rows(kv_new, xs1) &&
+                             (!second || lds_rows(second->kv_new, second->xs)) &&
+                             (!ckpt_out || (ckpt_interval % 64 == 0 && T0 % 64 == 0));
+    int cpl = all > one_per_simd && !two_and_one ? 2 : 1;
     const long lanes = channels / cpl;
     const dim3 grid((unsigned)((lanes + 255) / 256), (unsigned)tensors), block(256);
     EncTensor first;

@@ -55,3 +55,31 @@ def test_runs_through_the_lds(gpu, oracle, bits, dtype, cuts, S, pad, bad):
         assert np.array_equal(c.cpu().numpy(), wc) and _same16(_np16(s), ws)
         for j, w in enumerate(wk):
             assert _same16(_np16(k[:, :, j]), w), j
+
+
+@pytest.mark.parametrize("bits", (4, 2))
+@pytest.mark.parametrize("B,T,S", [(17, 384, 64), (24, 449, 0), (21, 400, 48), (25, 385, 64), (17, 383, 64)])
+def test_two_rounds_of_one_channel_per_lane(gpu, bits, B, T, S):
+    """32 heads: 17 to 24 sequences are more than two and at most three waves per SIMD.  Sequences 0 and B - 1 are
+    what they are alone, where their few channels take one channel per lane with a wave to a SIMD."""
+    H = 32
+    params = [[t.to(gpu) for t in synth.make_params(H, D, bits=bits, seed=7 + i).astuple()] for i in range(2)]
+    rows = [torch.randn(B, T, H * D, generator=torch.Generator().manual_seed(i)).to(torch.bfloat16) for i in range(2)]
+    rows[1][B - 1, T - 2, 77] = float("nan")
+    rows = [r.to(gpu).view(B, T, H, D).transpose(1, 2) for r in rows]
+
+    def run(rs):
+        n = rs[0].shape[0]
+        caches = [synth.alloc_cache(n, H, T + 16, D, gpu, bits=bits) for _ in range(2)]
+        states = [torch.zeros(n, H, D, 2, dtype=torch.float16, device=gpu) for _ in range(2)]
+        cks = [torch.zeros(n, H, T // S + 1, D, 2, dtype=torch.float16, device=gpu) if S else None for _ in range(2)]
+        gemv.append_kv_pair(*caches, *rs, *params, 0, *states, k_ckpt=cks[0], v_ckpt=cks[1], ckpt_interval=S, bits=bits)
+        return caches, states, cks
+
+    got, torch_nan = run(rows), lambda t: torch.nan_to_num(t.float(), nan=123.0)
+    for b in (0, B - 1):
+        want = run([r[b:b + 1] for r in rows])
+        for g, w in zip(got[0], want[0]):
+            assert torch.equal(g[b:b + 1], w)
+        for g, w in [*zip(got[1], want[1]), *(zip(got[2], want[2]) if S else ())]:
+            assert torch.equal(torch_nan(g[b:b + 1]), torch_nan(w))
