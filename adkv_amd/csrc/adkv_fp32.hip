@@ -10,13 +10,13 @@
 //
 // The recurrence is serial in t and only channels are parallel (64 to 1024 waves in the sizes this
 // form is used at, at most one per SIMD).  A wave alone on its SIMD issues one instruction every 4
-// cycles whether or not it depends on the one before, so the time per token is the NUMBER of
-// instructions of the wave that carries the chain.  quant_kernel therefore gives a workgroup two
-// waves: one does nothing but the recurrence, out of LDS and into LDS (two tokens per LDS
-// instruction); the other moves rows between memory and LDS, four channels per lane and a 16-byte
-// access per four rows, and converts types.  4096 channels x 1024 tokens of fp32 take 45 us, 44 ns per
-// token (18.5 issue slots at the 2.0-2.3 ns a lone wave pays for one); with everything in one wave it
-// was 65 us, the rest being loads, stores, their addresses and the guards of the rounding.
+// cycles whether or not it depends on the one before (more for some, see recurrence), so the time per
+// token is the sum over the instructions of the wave that carries the chain.  quant_kernel therefore
+// gives a workgroup two waves: one does nothing but the recurrence, out of LDS and into LDS (four tokens
+// per LDS instruction); the other moves rows between memory and LDS, 16 bytes per access, and converts
+// types.  4096 channels x 1024 tokens of fp32 take 42 us, 36 ns per token and 5 us for the launch and its
+// first rows; with everything in one wave it was 65 us, the rest being loads, stores, their addresses and
+// the guards of the rounding.
 #include <hip/hip_runtime.h>
 #include <hip/hip_bf16.h>
 #include <stdint.h>
