@@ -729,12 +729,12 @@ __device__ __forceinline__ void encode_body(
                        (sa.ckpt == nullptr || (sa.ckpt_interval % 64 == 0 && sg * TPW % 64 == 0));
     const int piece = (int)(span_words >= PF ? span_words / PF * PF : max(span_words, 1L)); // whole runs where it can
     while (sg < sg_end) {
-        const int nw = min(piece, sg_end - sg), ng = nw * G8; // words, 8-token groups of this piece
+        const int sg_piece = sg, nw = min(piece, sg_end - sg), ng = nw * G8; // words, 8-token groups of this piece
         const uint32_t xbytes = (uint32_t)(((long)ng * 8 - 1) * xs.t * 2 + 128 * CPL);
         if constexpr (CPL == 1) {
             // Whole runs of 64 tokens whose rows come through the LDS (enc_run64), a run ahead: 64 tokens or 2 us.  Rows have
             // to be 16-byte aligned; a run that meets a NaN, and all after it, go through the loop below.
-            if (through_lds && ng >= 8) {
+            if (through_lds && ng >= 8 && (sa.ckpt == nullptr || sg * TPW % 64 == 0)) {
                 constexpr int WORDS = 8 / G8;
                 const uint64_t base = wave_uniform((uint64_t)(xb + (long)sg * TPW * xs.t));
                 const rsrc4 rows = {(uint32_t)base, (uint32_t)(base >> 32), xbytes, 0x00027000u};
@@ -783,6 +783,33 @@ __device__ __forceinline__ void encode_body(
                     half ^= 8192u;
                 }
                 asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); // nothing is on its way into the LDS any more
+                // The words behind the last whole run: their rows are in the LDS already, and no checkpoint lies
+                // inside them.  (Loaded again for the loop below they cost a short stream 1 of its 13 to 25 us.)
+                const int words = (sg_piece + nw) - sg;
+                if (through_lds && words > 0) {
+                    typedef const volatile __attribute__((address_space(3))) uint16_t *LdsRows;
+                    const LdsRows tail = (LdsRows)(lds + half) + lane;
+                    const Pair saved = st;
+                    enter();
+                    for (int k = 0; k < words * G8; k++) {
+                        XW x[8];
+#pragma unroll
+                        for (int tt = 0; tt < 8; tt++)
+                            x[tt] = (XW)tail[(k * 8 + tt) * 64];
+                        tokens8(x);
+                        if (k % G8 == G8 - 1) {
+                            *dst = w[0] ^ WORD_BIAS;
+                            dst += D;
+                        }
+                    }
+                    leave();
+                    if (__builtin_expect(__any(nan != nan), 0)) {
+                        st = saved;
+                        through_lds = false;
+                    } else {
+                        sg += words;
+                    }
+                }
                 continue;
             }
         }

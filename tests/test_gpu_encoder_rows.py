@@ -22,6 +22,7 @@ D = 128
     ((0, 128, 321), 64, 24, (191, 192)),    # resumed at a run, a run that fails at its last and first token
     ((0, 200), 48, 0, ()),                  # checkpoints inside runs
     ((0, 200), 64, 4, ()), ((0, 200), 64, 1, (64,)),   # rows 8 and 2 bytes off: not through the LDS
+    ((0, 120), 0, 0, (70,)), ((0, 190), 64, 0, (150, 188)), ((0, 66, 250), 64, 8, ()),   # words behind the last run, and a NaN there
     ((0, 7, 64, 576), 256, 16, (575,))])
 def test_runs_through_the_lds(gpu, oracle, bits, dtype, cuts, S, pad, bad):
     B, H, T = 2, 3, cuts[-1]
