@@ -1130,6 +1130,10 @@ struct PairScores {
     template <typename PUT>
     __device__ __forceinline__ void emit(int token, int ntok, PUT &&put)
     {
+        // All of d is held up to here: registers of it that nobody reads would go to the hand-laid block behind
+        // multiply() while the matrix cores have yet to write them, and the compiler waits for no block.  (With 2-bit
+        // codes the block wrote one of them an instruction later; at two waves per SIMD its value was lost.)
+        asm volatile("" ::"v"(d));
         const int t = lane & 15, quarter = lane >> 4;
         if (t >= ntok || (GQ == 1 && quarter) || (GQ == 2 && (quarter & 1)))
             return;

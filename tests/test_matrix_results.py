@@ -1,0 +1,89 @@
+"""Registers that a matrix instruction still has to write are left alone until it has, in the library as built.
+
+The hardware does not hold back a vector instruction that reads or overwrites such a register; the compiler keeps
+the distance between its own instructions, but not to a hand-laid block, and it hands registers of a result that
+nobody reads to the next block at once: what the block has left there is then overwritten behind its back, now
+and then, as the waves of a SIMD happen to interleave."""
+import os
+import re
+import shutil
+import struct
+import subprocess
+
+import pytest
+
+from adkv_amd.build import LIB_PATH
+
+LLVM = "/opt/rocm/llvm/bin"
+# Wait states between a matrix instruction (of 2 and of 4 passes) and a vector instruction that reads, overwrites its
+# result, as the compiler keeps them between its own.
+WAIT = {"v_mfma_f32_4x4x4_16b_f16": (5, 5), "v_mfma_f32_16x16x32_f16": (8, 7)}
+
+
+def _registers(text):
+    regs = {(k, int(i)) for k, i in re.findall(r"\b([va])(\d+)\b", text)}
+    for k, lo, hi in re.findall(r"\b([va])\[(\d+):(\d+)\]", text):
+        regs |= {(k, i) for i in range(int(lo), int(hi) + 1)}
+    return regs
+
+
+def violations(listing):
+    """(kernel, wait states, matrix instruction, vector instruction) of every pair that is too close, along every path."""
+    for name, body in re.findall(r"^[0-9a-f]+ <(\S+)>:\n(.*?)(?=^[0-9a-f]+ <|\Z)", listing, re.S | re.M):
+        if "v_mfma" not in body:
+            continue
+        code = re.findall(r"^\t(\S+)(?: +([^/\n]*?))? *// ([0-9A-F]+):.*$", body, re.M)
+        at = {int(a, 16): i for i, (_, _, a) in enumerate(code)}
+
+        def after(i):                                                      # where the wave goes next
+            op, args, addr = code[i]
+            if op == "s_endpgm":
+                return []
+            if op.startswith(("s_branch", "s_cbranch")):
+                off = int(args)
+                to = at.get(int(addr, 16) + 4 + 4 * (off - 65536 if off > 32767 else off))
+                return [to] if op == "s_branch" else [to, i + 1]
+            return [i + 1]
+
+        for i, (op, args, _) in enumerate(code):
+            if not op.startswith("v_mfma"):
+                continue
+            result, seen, todo = _registers(args.split(",")[0]), {}, [(j, 0) for j in after(i)]
+            read, write = WAIT[op]
+            while todo:
+                j, waited = todo.pop()
+                if j is None or j >= len(code) or waited >= read or seen.get(j, 99) <= waited:
+                    continue
+                seen[j] = waited
+                o, a, _ = code[j]
+                if o.startswith("v_") and not o.startswith("v_mfma"):
+                    dst, src = (_registers(x) for x in (a.split(",")[0], ",".join(a.split(",")[1:])))
+                    if src & result or (dst & result and waited < write):
+                        yield name, waited, f"{op} {args}", f"{o} {a}"
+                    if (dst | src) & result:
+                        continue
+                todo += [(k, waited + (int(a, 0) + 1 if o == "s_nop" else 1)) for k in after(j)]
+
+
+@pytest.fixture(scope="module")
+def listings(tmp_path_factory):
+    if not os.path.exists(LIB_PATH) or not os.path.exists(f"{LLVM}/llvm-objdump"):
+        pytest.skip("no library or no disassembler")
+    d, found = tmp_path_factory.mktemp("code"), []
+    subprocess.run([shutil.which("llvm-objcopy", path=LLVM), f"--dump-section=.hip_fatbin={d}/fat", LIB_PATH, f"{d}/copy"], check=True)
+    fat = (d / "fat").read_bytes()
+    for m in re.finditer(b"__CLANG_OFFLOAD_BUNDLE__", fat):
+        p = m.start() + 32
+        for _ in range(struct.unpack_from("<Q", fat, m.start() + 24)[0]):
+            offset, size, n = struct.unpack_from("<QQQ", fat, p)
+            if b"gfx950" in fat[p + 24:p + 24 + n]:
+                (d / "code").write_bytes(fat[m.start() + offset:m.start() + offset + size])
+                found.append(subprocess.run([f"{LLVM}/llvm-objdump", "-d", "--no-show-raw-insn", f"{d}/code"], check=True,
+                                            capture_output=True, text=True).stdout)
+            p += 24 + n
+    return found
+
+
+def test_results_of_matrix_instructions_are_left_alone_until_written(listings):
+    assert sum(t.count("\tv_mfma") for t in listings) > 1000               # the listings are what they should be
+    assert not [v for t in listings for v in violations(t)][:5]
