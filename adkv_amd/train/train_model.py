@@ -172,13 +172,17 @@ class ADKVTrainModel(nn.Module):
         B, T, C = kv_cache.shape
         assert C == self.num_hidden_states
         assert self.truncation % CHUNK == 0
-        # The launch constrains fp32 parameters itself; a subclass's or an instance's own way stays in force.
+        # The launch constrains fp32 parameters itself; another way, of a subclass or an instance or set on the
+        # class afterwards, stays in force.
         free = (self.alpha.dtype == self.beta.dtype == self.init_log_sc.dtype == torch.float32
-                and all(getattr(type(self), f) is getattr(ADKVTrainModel, f) and f not in self.__dict__
-                        for f in ("get_alpha", "get_beta", "get_sc")))
+                and all(getattr(type(self), name) is f and name not in self.__dict__ for name, f in _CONSTRAINTS.items()))
         out, _, zs, ss = quant_f32(kv_cache, self.alpha if free else self.get_alpha(),
                                    self.beta if free else self.get_beta(), self.target,
                                    self.lower_limit, self.upper_limit, self.sc_min, self.sc_max,
                                    zp_init=self.init_zp, sc_init=self.init_log_sc if free else self.get_sc(),
                                    output_states=output_states, free_params=free)
         return (out, zs, ss) if output_states else out
+
+
+# the functions that ADKV_PARAMS_FREE stands for
+_CONSTRAINTS = {name: getattr(ADKVTrainModel, name) for name in ("get_alpha", "get_beta", "get_sc")}

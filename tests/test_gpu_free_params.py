@@ -7,8 +7,6 @@ from adkv_amd import _lib
 from adkv_amd.train import ADKVTrainModel, quant_f32
 from tests.test_host_calls import NOTHING
 
-pytestmark = pytest.mark.gpu
-
 
 def _model(C, cls=ADKVTrainModel):
     m = cls(C)
@@ -26,6 +24,7 @@ def _want(m, x, states):
                      zp_init=m.init_zp, sc_init=m.get_sc(), output_states=states)
 
 
+@pytest.mark.gpu
 @pytest.mark.parametrize("dtype", (torch.float32, torch.bfloat16))
 @pytest.mark.parametrize("B,T", [(1, 1), (2, 77), (600, 9)])          # 600: a lane per channel straight from memory
 @pytest.mark.parametrize("in_python", (False, True))
@@ -40,6 +39,7 @@ def test_same_bits_as_torch(gpu, monkeypatch, dtype, B, T, in_python):
     assert torch.equal(torch.nan_to_num(m(x).float()), torch.nan_to_num(out.float()))
 
 
+@pytest.mark.gpu
 def test_own_constraints_stay(gpu):
     class Own(ADKVTrainModel):
         def get_beta(self):
@@ -51,3 +51,19 @@ def test_own_constraints_stay(gpu):
     m = _model(64)
     m.get_alpha = lambda: torch.full((64,), 0.5, device=gpu)
     assert torch.equal(torch.nan_to_num(m(x)), torch.nan_to_num(_want(m, x, False)[0]))
+
+
+@pytest.mark.parametrize("name", ("get_alpha", "get_beta", "get_sc"))
+def test_constraints_set_on_the_class_stay(monkeypatch, name):
+    """What the forward gives the quantiser, without a device."""
+    from adkv_amd.train import train_model
+    given = {}
+    monkeypatch.setattr(train_model, "quant_f32", lambda x, *a, **kw: given.update(kw, a=a) or (x, None, None, None))
+    m, x = ADKVTrainModel(64), torch.zeros(1, 2, 64)
+    m(x)
+    assert given["free_params"] and given["a"][0] is m.alpha and given["sc_init"] is m.init_log_sc
+    own = torch.full((64,), 0.5)
+    monkeypatch.setattr(ADKVTrainModel, name, lambda self: own)
+    m(x)
+    assert not given["free_params"]
+    assert {"get_alpha": given["a"][0], "get_beta": given["a"][1], "get_sc": given["sc_init"]}[name] is own
