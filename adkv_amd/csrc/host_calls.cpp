@@ -256,7 +256,7 @@ PyObject *decode(PyObject *, PyObject *const *args, Py_ssize_t nargs)
 //        value state, key checkpoints, value checkpoints, interval, bits, fresh)
 PyObject *append(PyObject *, PyObject *const *args, Py_ssize_t nargs)
 {
-    if (nargs != 14 || !unwatched())
+    if (nargs != 14 || !unwatched() || (args[13] != Py_True && args[13] != Py_False)) // any other truth value: Python's
         Py_RETURN_NONE;
     const at::Tensor *t[6];
     const int at_arg[6] = {0, 1, 2, 3, 7, 8};

@@ -116,3 +116,18 @@ def test_evaluation_cache_equals_the_python_function(gpu, monkeypatch, dtype):
     monkeypatch.setattr(_lib, "host", lambda: NOTHING)
     for a, b in zip(mine, run()):
         assert torch.equal(a, b)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("fresh", [True, 1, torch.ones(1, dtype=torch.bool)])
+def test_any_truth_value_makes_a_cache_fresh(gpu, fresh):
+    """Slots and checkpoints behind the prompt are zeroed, whatever says that the memory is uninitialised."""
+    B, H, D, T, S = 1, 2, 128, 70, 64
+    p = [t.to(gpu) for t in synth.make_params(H, D, seed=1).astuple()]
+    x = torch.randn(B, H, T, D, device=gpu).half()
+    junk = lambda *shape: torch.full(shape, 0x5A, dtype=torch.uint8, device=gpu)
+    caches = [junk(B, H, 16, D // 4, 4, 4) for _ in range(2)]
+    state, ckpt = ([junk(B, H, *n, D, 4).view(torch.float16) for _ in range(2)] for n in ((), (3,)))
+    gemv.append_kv_pair(*caches, x, x, p, p, 0, *state, k_ckpt=ckpt[0], v_ckpt=ckpt[1], ckpt_interval=S, fresh=fresh)
+    for c, k in zip(caches, ckpt):
+        assert not torch.any(c[:, :, 9:]) and not torch.any(k[:, :, 1:].view(torch.int16)) and torch.any(k[:, :, 0] != 0)
