@@ -108,25 +108,23 @@ PyObject *rope_qk(PyObject *, PyObject *const *args, Py_ssize_t n)
         Py_RETURN_NONE;
     at::Tensor qo, ko;
     int rc;
-    try {
-        qo = at::empty({B, Hq, T, D}, q.options());
-        ko = at::empty({B, H, T, D}, q.options());
-        if (!qo.has_storage() || !ko.has_storage())
-            Py_RETURN_NONE;
-        void *qp = qo.mutable_data_ptr(), *kp = ko.mutable_data_ptr();
-        Py_BEGIN_ALLOW_THREADS
-        rc = adkv_rope_qk(q.const_data_ptr(), k.const_data_ptr(), c.const_data_ptr(), s.const_data_ptr(), qp, kp, (int)B, (int)Hq,
-                          (int)H, (int)T, (int)D, q.stride(0), q.stride(1), q.stride(2), k.stride(0), k.stride(1), k.stride(2),
-                          c.size(0) == B && B > 1 ? c.stride(0) : 0, c.stride(1), q.scalar_type() == at::kBFloat16, stream);
-        Py_END_ALLOW_THREADS
-    } catch (const std::exception &) {
-        Py_RETURN_NONE; // out of memory, or a mode that allocates otherwise: the Python function meets it too
-    }
+    qo = at::empty({B, Hq, T, D}, q.options());
+    ko = at::empty({B, H, T, D}, q.options());
+    if (!qo.has_storage() || !ko.has_storage())
+        Py_RETURN_NONE;
+    void *qp = qo.mutable_data_ptr(), *kp = ko.mutable_data_ptr();
+    Py_BEGIN_ALLOW_THREADS
+    rc = adkv_rope_qk(q.const_data_ptr(), k.const_data_ptr(), c.const_data_ptr(), s.const_data_ptr(), qp, kp, (int)B, (int)Hq,
+                      (int)H, (int)T, (int)D, q.stride(0), q.stride(1), q.stride(2), k.stride(0), k.stride(1), k.stride(2),
+                      c.size(0) == B && B > 1 ? c.stride(0) : 0, c.stride(1), q.scalar_type() == at::kBFloat16, stream);
+    Py_END_ALLOW_THREADS
     return rc ? PyLong_FromLong(rc) : pair(std::move(qo), std::move(ko));
 }
 
 // n contiguous tensors of `type` and `numel` elements each on `device` in a tuple -> their addresses
-bool pointers(PyObject *tuple, Py_ssize_t n, at::ScalarType type, int64_t numel, c10::Device device, const void **out)
+// (written: in place, so a storage shared by a lazy copy becomes the tensor's own)
+bool pointers(PyObject *tuple, Py_ssize_t n, at::ScalarType type, int64_t numel, c10::Device device, const void **out,
+              bool written = false)
 {
     if (!PyTuple_CheckExact(tuple) || PyTuple_GET_SIZE(tuple) != n)
         return false;
@@ -134,7 +132,7 @@ bool pointers(PyObject *tuple, Py_ssize_t n, at::ScalarType type, int64_t numel,
         const at::Tensor *p = plain(PyTuple_GET_ITEM(tuple, i));
         if (!p || p->scalar_type() != type || p->numel() != numel || !p->is_contiguous() || p->device() != device)
             return false;
-        out[i] = p->const_data_ptr();
+        out[i] = written ? p->mutable_data_ptr() : p->const_data_ptr();
     }
     return true;
 }
@@ -222,33 +220,28 @@ PyObject *decode(PyObject *, PyObject *const *args, Py_ssize_t nargs)
         Py_RETURN_NONE;
     at::Tensor out, weights, m, scratch = *ws; // held: another thread may replace the dictionary's entry
     int rc;
-    try {
-        if (mask) {
-            m = (mask_type >= 0 ? *mask : mask->to(at::kFloat)).contiguous();
-            if (!m.has_storage())
-                Py_RETURN_NONE;
-        }
-        const int64_t pitch = adkv_row_pitch((int)n);
-        out = at::empty({B, Hq, D}, q.options());
-        weights = at::empty({B, Hq, pitch}, q.options().dtype(at::kHalf));
-        if (!out.has_storage() || !weights.has_storage())
+    if (mask) {
+        m = (mask_type >= 0 ? *mask : mask->to(at::kFloat)).contiguous();
+        if (!m.has_storage())
             Py_RETURN_NONE;
-        void *op = out.mutable_data_ptr(), *wp = weights.mutable_data_ptr();
-        const void *mp = mask ? m.const_data_ptr() : nullptr;
-        const double scaling = PyFloat_AS_DOUBLE(args[11]);
-        Py_BEGIN_ALLOW_THREADS
-        rc = adkv_decode_step(q.const_data_ptr(), kc->mutable_data_ptr(), vc->mutable_data_ptr(), kn->const_data_ptr(),
-                              vn->const_data_ptr(), params, params + 5, mp, rows_per_mask_row, (float)scaling, op, wp, pitch, (int)B,
-                              (int)Hq, (int)H, (int)T, (int)D, (int)n_super, (int)bits,
-                              (q.scalar_type() == at::kBFloat16 ? ADKV_DT_BF16 : ADKV_DT_F16) | ADKV_MASK_DT(std::max(mask_type, ADKV_DT_F32)),
-                              ck[0], ck[1], (int)n_ckpt, (int)interval,
-                              scratch.mutable_data_ptr(), scratch.numel(), stream);
-        Py_END_ALLOW_THREADS
-        const int64_t sizes[3] = {B, Hq, n}, strides[3] = {Hq * pitch, pitch, 1};
-        weights.unsafeGetTensorImpl()->set_sizes_and_strides(at::IntArrayRef(sizes), at::IntArrayRef(strides));
-    } catch (const std::exception &) {
-        Py_RETURN_NONE;
     }
+    const int64_t pitch = adkv_row_pitch((int)n);
+    out = at::empty({B, Hq, D}, q.options());
+    weights = at::empty({B, Hq, pitch}, q.options().dtype(at::kHalf));
+    if (!out.has_storage() || !weights.has_storage())
+        Py_RETURN_NONE;
+    void *op = out.mutable_data_ptr(), *wp = weights.mutable_data_ptr(), *kcp = kc->mutable_data_ptr(), *vcp = vc->mutable_data_ptr(),
+         *work = scratch.mutable_data_ptr(); // before the lock is given up: these may throw
+    const void *mp = mask ? m.const_data_ptr() : nullptr;
+    const double scaling = PyFloat_AS_DOUBLE(args[11]);
+    Py_BEGIN_ALLOW_THREADS
+    rc = adkv_decode_step(q.const_data_ptr(), kcp, vcp, kn->const_data_ptr(), vn->const_data_ptr(), params, params + 5, mp, rows_per_mask_row, (float)scaling, op, wp, pitch, (int)B,
+                          (int)Hq, (int)H, (int)T, (int)D, (int)n_super, (int)bits,
+                          (q.scalar_type() == at::kBFloat16 ? ADKV_DT_BF16 : ADKV_DT_F16) | ADKV_MASK_DT(std::max(mask_type, ADKV_DT_F32)),
+                          ck[0], ck[1], (int)n_ckpt, (int)interval, work, scratch.numel(), stream);
+    Py_END_ALLOW_THREADS
+    const int64_t sizes[3] = {B, Hq, n}, strides[3] = {Hq * pitch, pitch, 1};
+    weights.unsafeGetTensorImpl()->set_sizes_and_strides(at::IntArrayRef(sizes), at::IntArrayRef(strides));
     return rc ? PyLong_FromLong(rc) : pair(std::move(out), std::move(weights));
 }
 
@@ -333,27 +326,23 @@ PyObject *quant_f32(PyObject *, PyObject *const *args, Py_ssize_t nargs)
         Py_RETURN_NONE;
     at::Tensor out, state, seq[2];
     int rc;
-    try {
-        const auto f32 = x->options().dtype(at::kFloat);
-        out = at::empty({B, T, C}, x->options());
-        state = at::empty({2, B, C}, f32);
-        if (args[6] == Py_True)
-            for (at::Tensor &t : seq)
-                t = at::empty({B, T, C}, f32);
-        if (!out.has_storage() || !state.has_storage())
-            Py_RETURN_NONE;
-        void *op = out.mutable_data_ptr(), *zp = state.mutable_data_ptr(), *sc = (float *)zp + B * C;
-        void *sp[2] = {seq[0].defined() ? seq[0].mutable_data_ptr() : nullptr, seq[1].defined() ? seq[1].mutable_data_ptr() : nullptr};
-        const int type = (x->scalar_type() == at::kFloat ? ADKV_DT_F32 : x->scalar_type() == at::kHalf ? ADKV_DT_F16 : ADKV_DT_BF16) |
-                         (args[7] == Py_True ? ADKV_PARAMS_FREE : 0);
-        const double lo = PyFloat_AS_DOUBLE(args[4]), hi = PyFloat_AS_DOUBLE(args[5]);
-        Py_BEGIN_ALLOW_THREADS
-        rc = adkv_quant_f32(x->const_data_ptr(), op, nullptr, zp, sc, p[3], p[4], p[0], p[1], p[2], sp[0], sp[1], (int)B, (int)T, (int)C,
-                            T * C, C, type, (int)lower, (int)upper, (float)lo, (float)hi, stream);
-        Py_END_ALLOW_THREADS
-    } catch (const std::exception &) {
+    const auto f32 = x->options().dtype(at::kFloat);
+    out = at::empty({B, T, C}, x->options());
+    state = at::empty({2, B, C}, f32);
+    if (args[6] == Py_True)
+        for (at::Tensor &t : seq)
+            t = at::empty({B, T, C}, f32);
+    if (!out.has_storage() || !state.has_storage())
         Py_RETURN_NONE;
-    }
+    void *op = out.mutable_data_ptr(), *zp = state.mutable_data_ptr(), *sc = (float *)zp + B * C;
+    void *sp[2] = {seq[0].defined() ? seq[0].mutable_data_ptr() : nullptr, seq[1].defined() ? seq[1].mutable_data_ptr() : nullptr};
+    const int type = (x->scalar_type() == at::kFloat ? ADKV_DT_F32 : x->scalar_type() == at::kHalf ? ADKV_DT_F16 : ADKV_DT_BF16) |
+                     (args[7] == Py_True ? ADKV_PARAMS_FREE : 0);
+    const double lo = PyFloat_AS_DOUBLE(args[4]), hi = PyFloat_AS_DOUBLE(args[5]);
+    Py_BEGIN_ALLOW_THREADS
+    rc = adkv_quant_f32(x->const_data_ptr(), op, nullptr, zp, sc, p[3], p[4], p[0], p[1], p[2], sp[0], sp[1], (int)B, (int)T, (int)C,
+                        T * C, C, type, (int)lower, (int)upper, (float)lo, (float)hi, stream);
+    Py_END_ALLOW_THREADS
     if (rc)
         return PyLong_FromLong(rc);
     PyObject *o = THPVariable_Wrap(std::move(out));
@@ -389,8 +378,8 @@ PyObject *quant_f32_pair(PyObject *, PyObject *const *args, Py_ssize_t nargs)
         Py_RETURN_NONE;
     const void *rows[4], *params[6], *state[4], *init[4];
     int64_t strides[8];
-    for (int i = 0; i < 4; i++) { // of a single sequence or token the strides may be anything
-        rows[i] = t[i]->const_data_ptr();
+    for (int i = 3; i >= 0; i--) { // outputs first (they may be the inputs); of a single sequence or token the strides may be anything
+        rows[i] = i >= 2 ? t[i]->mutable_data_ptr() : t[i]->const_data_ptr();
         strides[2 * i] = B > 1 ? t[i]->stride(0) : T * std::max(t[i]->stride(1), C);
         strides[2 * i + 1] = T > 1 ? t[i]->stride(1) : C;
     }
@@ -400,7 +389,7 @@ PyObject *quant_f32_pair(PyObject *, PyObject *const *args, Py_ssize_t nargs)
         if (!st || st->dim() != 2 || st->size(0) != B)
             Py_RETURN_NONE;
     }
-    if (!pointers(args[4], 6, at::kFloat, C, x.device(), params) || !pointers(args[5], 4, at::kFloat, B * C, x.device(), state) ||
+    if (!pointers(args[4], 6, at::kFloat, C, x.device(), params) || !pointers(args[5], 4, at::kFloat, B * C, x.device(), state, true) ||
         (args[6] != Py_None && !pointers(args[6], 4, at::kFloat, C, x.device(), init)) || !current(x.device(), stream))
         Py_RETURN_NONE;
     const int type = x.scalar_type() == at::kFloat ? ADKV_DT_F32 : x.scalar_type() == at::kHalf ? ADKV_DT_F16 : ADKV_DT_BF16;
@@ -414,6 +403,17 @@ PyObject *quant_f32_pair(PyObject *, PyObject *const *args, Py_ssize_t nargs)
     return PyLong_FromLong(rc);
 }
 
+// No C++ exception reaches Python's frames.
+template <PyObject *(*CALL)(PyObject *, PyObject *const *, Py_ssize_t)>
+PyObject *guarded(PyObject *self, PyObject *const *args, Py_ssize_t n)
+{
+    try {
+        return CALL(self, args, n);
+    } catch (const std::exception &) {
+        Py_RETURN_NONE; // out of memory, or a mode that allocates otherwise: the Python function meets it too
+    }
+}
+
 PyObject *init(PyObject *, PyObject *f)
 {
     Py_INCREF(f);
@@ -423,11 +423,11 @@ PyObject *init(PyObject *, PyObject *f)
 
 PyMethodDef methods[] = {
     {"init", init, METH_O, "init(function from device index to raw stream)"},
-    {"rope_qk", (PyCFunction)(void (*)(void))rope_qk, METH_FASTCALL, nullptr},
-    {"decode", (PyCFunction)(void (*)(void))decode, METH_FASTCALL, nullptr},
-    {"append", (PyCFunction)(void (*)(void))append, METH_FASTCALL, nullptr},
-    {"quant_f32", (PyCFunction)(void (*)(void))quant_f32, METH_FASTCALL, nullptr},
-    {"quant_f32_pair", (PyCFunction)(void (*)(void))quant_f32_pair, METH_FASTCALL, nullptr},
+    {"rope_qk", (PyCFunction)(void (*)(void))guarded<rope_qk>, METH_FASTCALL, nullptr},
+    {"decode", (PyCFunction)(void (*)(void))guarded<decode>, METH_FASTCALL, nullptr},
+    {"append", (PyCFunction)(void (*)(void))guarded<append>, METH_FASTCALL, nullptr},
+    {"quant_f32", (PyCFunction)(void (*)(void))guarded<quant_f32>, METH_FASTCALL, nullptr},
+    {"quant_f32_pair", (PyCFunction)(void (*)(void))guarded<quant_f32_pair>, METH_FASTCALL, nullptr},
     {nullptr, nullptr, 0, nullptr}};
 PyModuleDef module = {PyModuleDef_HEAD_INIT, "_host", nullptr, -1, methods, nullptr, nullptr, nullptr, nullptr};
 

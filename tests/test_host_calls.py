@@ -131,3 +131,18 @@ def test_any_truth_value_makes_a_cache_fresh(gpu, fresh):
     gemv.append_kv_pair(*caches, x, x, p, p, 0, *state, k_ckpt=ckpt[0], v_ckpt=ckpt[1], ckpt_interval=S, fresh=fresh)
     for c, k in zip(caches, ckpt):
         assert not torch.any(c[:, :, 9:]) and not torch.any(k[:, :, 1:].view(torch.int16)) and torch.any(k[:, :, 0] != 0)
+
+
+@pytest.mark.gpu
+def test_written_tensors_that_share_their_storage_lazily_become_their_own(gpu):
+    from adkv_amd.train.train_model import quant_f32_pair
+    B, T, C = 2, 9, 64
+    x = [torch.randn(B, T, C, device=gpu) for _ in range(2)]
+    p = [tuple(torch.rand(C, device=gpu) * 0.1 + 0.05 for _ in range(3)) for _ in range(2)]
+    shared = [torch.ones(n, device=gpu).view(*s) for n, s in [(B * T * C, (B, T, C))] * 2 + [(B * C, (B, C))] * 4]
+    mine = [torch._lazy_clone(t) for t in shared]
+    plain = [t.clone() for t in shared]
+    for out in (mine, plain):
+        quant_f32_pair(x, p, -8, 7, 0.1, 2.0, states=[tuple(out[2:4]), tuple(out[4:])], out=out[:2])
+    for t, a, b in zip(shared, mine, plain):
+        assert torch.all(t == 1.0) and torch.equal(a, b)
