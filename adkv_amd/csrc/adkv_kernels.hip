@@ -3129,6 +3129,19 @@ const char *adkv_decode_kernel_name(int B, int Hq, int H, int T, int D, int bits
     return decode_kernel_name(B, Hq, H, T, D, bits, n_ckpt_cap, ckpt_interval);
 }
 
+int adkv_decode_step_launches(int B, int Hq, int H, int T, int D, int bits, int n_ckpt_cap, int ckpt_interval,
+                              int masked)
+{
+    if (adkv_decode_step_is_fused(B, Hq, H, T, D, bits, n_ckpt_cap, ckpt_interval, masked))
+        return 1;
+    if (adkv_decode_segments(B, Hq, H, T, D, bits, n_ckpt_cap, ckpt_interval, nullptr, 0, nullptr) < 0)
+        return 3;
+    int dummy = 0, cpl;
+    Seg seg;
+    void *ck = n_ckpt_cap > 0 && ckpt_interval > 0 ? &dummy : nullptr;
+    return segment_step_plan(seg, cpl, B, Hq, H, T, D, bits, ck, ck, n_ckpt_cap, ckpt_interval) ? 2 : 3;
+}
+
 int adkv_decode_segments(int B, int Hq, int H, int T, int D, int bits, int n_ckpt_cap,
                          int ckpt_interval, int *bounds, int max_bounds, int *info)
 {

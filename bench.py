@@ -336,6 +336,18 @@ def quant_f32_record(args, B, T, steps, warmup):
     return res
 
 
+def step_kernels(L, B, Hq, H, T, D, bits, n_ckpt_cap, S):
+    """The kernels of one decode_step call: one launch; short segments and their combination; or forward_qk, the
+    softmax and forward_ov.  The library's first pair of events brackets the first of them, the last pair the last."""
+    n = L.adkv_decode_step_launches(B, Hq, H, T, D, bits, n_ckpt_cap, S, 0)
+    if n == 1:                     # few short sequences
+        return ("small_step_kernel",)
+    if n == 2:
+        return ("step_segments_kernel", "step_combine_kernel")
+    name = L.adkv_decode_kernel_name(B, Hq, H, T, D, bits, n_ckpt_cap, S).decode()
+    return "qk_" + name, "softmax", "ov_" + name
+
+
 def decode_record(args, B, Hq, H, D, T, bits, S, NL, steps, warmup, headline=True, bf16=False):
     """Times `steps` decode_step calls (the product path) over NL rotating layer caches and returns
     the bench record.  headline=False leaves out the comparator, the CPU baseline and the graph
@@ -385,9 +397,7 @@ def decode_record(args, B, Hq, H, D, T, bits, S, NL, steps, warmup, headline=Tru
     from adkv_amd import _lib
     L = _lib.lib()
     ncap_arg = ncap if S else 0
-    kernel = L.adkv_decode_kernel_name(B, Hq, H, T, D, bits, ncap_arg, S).decode()
-    # few short sequences: the whole step is one launch, and what its events bracket is that launch
-    one_launch = L.adkv_decode_step_is_fused(B, Hq, H, T, D, bits, ncap_arg, S, 0) == 1
+    kernels = step_kernels(L, B, Hq, H, T, D, bits, ncap_arg, S)
     ws = torch.empty(gemv.decode_step_workspace_bytes(B, Hq, H, T, D, ncap_arg, S), dtype=torch.uint8, device=dev)
 
     def fused(l):
@@ -469,9 +479,9 @@ def decode_record(args, B, Hq, H, D, T, bits, S, NL, steps, warmup, headline=Tru
         torch.cuda.synchronize()
         graph_ms = (time.perf_counter() - t0) * 1e3 / steps
 
-    qk_kernel, ov_kernel = ("small_step_kernel", None) if one_launch else ("qk_" + kernel, "ov_" + kernel)
+    qk_kernel = kernels[0]                              # what the first pair of events brackets
     code_bytes = B * H * T * D * bits / 8.0             # one tensor's codes: bytes per QK launch
-    achieved = (2 if one_launch else 1) * code_bytes / (qk_ms * 1e-3) / 1e9
+    achieved = (1 if len(kernels) == 3 else 2) * code_bytes / (qk_ms * 1e-3) / 1e9
     tokens_s = B / (N_LAYERS_MODEL * ms_step * 1e-3)
     workload_key = f"decode B={B} Hq={Hq} H={H} d={D} ctx={T} bits={bits} ckpt={S}"
     traffic = None
@@ -519,10 +529,12 @@ def decode_record(args, B, Hq, H, D, T, bits, S, NL, steps, warmup, headline=Tru
             "traffic": traffic,
         },
     }
-    if one_launch:
+    if len(kernels) == 1:
         res["kernel_ms"] = {"one_launch": qk_ms, "step_device_median": dev_ms, "steps_with_events": len(marks)}
+    elif len(kernels) == 2:
+        res["kernel_ms"] = {"segments": qk_ms, "combine": ov_ms, "step_device_median": dev_ms, "steps_with_events": len(marks)}
     else:  # the second big launch of the step, same algorithmic bytes (the V codes)
-        res["roofline_ov"] = {"kernel": ov_kernel, "bound": "hbm", "achieved": code_bytes / (ov_ms * 1e-3) / 1e9,
+        res["roofline_ov"] = {"kernel": kernels[2], "bound": "hbm", "achieved": code_bytes / (ov_ms * 1e-3) / 1e9,
                               "peak": HBM_PEAK_GBPS, "unit": "GB/s", "frac": code_bytes / (ov_ms * 1e-3) / 1e9 / HBM_PEAK_GBPS,
                               "note": "forward_ov stage incl. the partial-sum kernel"}
     # what the memory system itself delivers for these kernels' access pattern with nothing else

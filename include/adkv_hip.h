@@ -56,9 +56,14 @@ void adkv_set_mha_kernel(int use_matrix_cores);
  * device has CUs, at most four segments and 1535 cached tokens, mask or not; not while
  * adkv_set_mha_kernel or ADKV_MFMA picks a family).
  * adkv_decode_step_is_fused: 1 if a call with these sizes, masked or not, is one launch of either
- * kind under the current settings, else 0. */
+ * kind under the current settings, else 0.
+ * adkv_decode_step_launches: 1 for those; 2 if the call runs as step_segments_kernel and step_combine_kernel
+ * (steps of short segments, see adkv_decode_step); 3 if forward_qk, the softmax and forward_ov are launched
+ * one after the other, also for sizes that the call refuses. */
 void adkv_set_fused_step(int mode);
 int adkv_decode_step_is_fused(int B, int Hq, int H, int T, int D, int bits, int n_ckpt_cap,
+                              int ckpt_interval, int masked);
+int adkv_decode_step_launches(int B, int Hq, int H, int T, int D, int bits, int n_ckpt_cap,
                               int ckpt_interval, int masked);
 const char *adkv_strerror(int code);
 /* hipError_t (as int) of the last failed launch in this thread, 0 if none. */
@@ -307,10 +312,10 @@ int adkv_decode_step(const void *q, void *k_cache, void *v_cache, const void *k_
                       void *k_ckpt, void *v_ckpt, int n_ckpt_cap, int ckpt_interval,
                       void *workspace, int64_t workspace_bytes, void *stream);
 
-/* Which of the library's decode kernels adkv_forward_qk_gqa / adkv_forward_ov_gqa /
- * adkv_decode_step launch for these sizes ("qk_" / "ov_" + the returned text): a static string,
- * for benchmark records and tests; "invalid" for sizes the entry points reject.  An adkv_decode_step
- * that adkv_decode_step_is_fused reports runs in one launch instead of these. */
+/* Which of the library's decode kernels adkv_forward_qk_gqa / adkv_forward_ov_gqa launch for these
+ * sizes ("qk_" / "ov_" + the returned text), and adkv_decode_step where adkv_decode_step_launches is 3
+ * (otherwise it runs other kernels): a static string, for benchmark records and tests; "invalid" for sizes
+ * the entry points reject. */
 const char *adkv_decode_kernel_name(int B, int Hq, int H, int T, int D, int bits, int n_ckpt_cap,
                                     int ckpt_interval);
 

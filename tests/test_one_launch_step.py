@@ -79,6 +79,32 @@ def test_library_says_which_steps_are_one_launch():
         L.adkv_set_fused_step(0)
 
 
+def test_library_says_in_how_many_launches_a_step_runs():
+    """Without a GPU, and what the benchmark calls the kernels of such a step."""
+    import bench
+    L = _lib.lib()
+    launches = lambda B, Hq, H, T, S=256, D=D, bits=4, masked=0: L.adkv_decode_step_launches(
+        B, Hq, H, T, D, bits, T // S + 1 if S else 0, S, masked)
+    names = lambda B, Hq, H, T, D=D, bits=4, S=256: bench.step_kernels(L, B, Hq, H, T, D, bits, T // S + 1, S)
+    for masked in (0, 1):
+        assert launches(1, 32, 32, 603, masked=masked) == 1
+        for n, sizes in ((2, (8, 32, 8, 16001)), (2, (4, 32, 32, 8000)), (2, (64, 32, 32, 663)), (2, (1, 64, 8, 300)),
+                         (3, (128, 32, 32, 4096)), (3, (16, 32, 8, 131072)), (3, (1, 64, 8, 300, 0)), (3, (2, 3, 3, 4000, 64))):
+            assert launches(*sizes, masked=masked) == n, sizes
+        assert launches(4, 8, 8, 8190, D=256, masked=masked) == 2 and launches(2, 8, 2, 5000, bits=2, masked=masked) == 2
+    for bad in ((2, 6, 4, 100), (2, 6, 2, 100), (0, 8, 8, 100), (1, 8, 8, -1)):
+        assert launches(*bad) == 3
+    assert launches(2, 16, 8, 100, D=256) == 3 and launches(1, 8, 8, 100, bits=3) == 3
+    assert names(1, 32, 32, 603) == ("small_step_kernel",)
+    assert names(8, 32, 8, 16001) == ("step_segments_kernel", "step_combine_kernel")
+    assert names(128, 32, 32, 4096)[0].startswith("qk_ft_kernel (") and len(names(128, 32, 32, 4096)) == 3
+    L.adkv_set_mha_kernel(0)
+    try:
+        assert launches(8, 32, 8, 16001) == 3
+    finally:
+        L.adkv_set_mha_kernel(-1)
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("H,T,S", [(4, 200, 64), (3, 600, 256)])
 def test_one_launch_step_replays_from_a_captured_graph(gpu, H, T, S):
