@@ -2670,6 +2670,12 @@ static bool small_step_plan(Seg &seg, int B, int Hq, int H, int T, int D, int bi
 // 4000 93.6 / 90.0, 1 x 8 x 1000 34.5 / 30.6; head dim 512, 8 x 8 x 2000 57.3 / 50.1.
 // With one query head two channels per lane are taken as long as four waves per SIMD hold them (12 x 32 heads x
 // 2000 tokens: 48.4 with four channels, 40.6 with two), four beyond.
+// Of the launches that a table per head pays for (use_head_table) two kinds stay with the three kernels, where
+// forward_qk's workgroups are more than half of the CUs and segments longer than 128 tokens: those whose forward_ov
+// adds its segments inside the workgroup, and segments beyond 256 tokens.  Three launches / two, 32 heads, every
+// 256: 128 x 300 60.0 / 60.7, 128 x 511 89.8 / 93.0, 64 x 1024 90.4 / 93.8; every 512: 100 x 1000 135.4 / 145.1; every
+// 128: 16 x 8000 152.7 / 161.2.  The others: 40 x 1100 80.3 / 78.6, 32 x 2048 (half the CUs) 114.4 / 91.3, every
+// 128: 128 x 150 36.6 / 35.3, 32 x 2000 85.2 / 83.7, every 512: 32 x 4000 (half) 195.4 / 161.9.
 // Segments cut finer than 128 tokens (by checkpoints closer than that) with one query head per KV head stay
 // with the separate launches: such a step is the three calls bit for bit, where here a weight is rounded
 // before it is divided by its row's sum, at 15.0 us instead of 11.0 (2 x 3 heads x 530, every 64).
@@ -2691,6 +2697,13 @@ static bool segment_step_plan(Seg &seg, int &cpl, int B, int Hq, int H, int T, i
     if (waves > room && GQ == 1 && bits == 4 && D == 128) {
         cpl = 4;
         waves = padded_units<32>(BH, seg.nseg) / 2;
+        if (waves <= room && longest > 128 && use_head_table(B, H, 1, bits, D, seg)) {
+            Seg k = seg, v = seg;
+            plan_ft(k, B, H, T, FT_SKEW_QK, FT16_QK);
+            const int lanes = plan_ft_ov(v, B, H, T);
+            if (2L * H * k.phys_per_head > cus() && (longest > 256 || ft_ov_combines(v, B, lanes)))
+                return false;
+        }
     }
     return waves <= room;
 }

@@ -92,6 +92,12 @@ def test_library_says_in_how_many_launches_a_step_runs():
                          (3, (128, 32, 32, 4096)), (3, (16, 32, 8, 131072)), (3, (1, 64, 8, 300, 0)), (3, (2, 3, 3, 4000, 64))):
             assert launches(*sizes, masked=masked) == n, sizes
         assert launches(4, 8, 8, 8190, D=256, masked=masked) == 2 and launches(2, 8, 2, 5000, bits=2, masked=masked) == 2
+    # a table per head pays: its forward_ov adds two or four segments in the workgroup, or does not; half of the CUs
+    for n, sizes in ((3, (128, 32, 32, 300)), (3, (64, 32, 32, 1024)), (3, (40, 40, 40, 1000)), (2, (40, 32, 32, 1100)),
+                     (2, (64, 40, 40, 600)), (2, (32, 32, 32, 2048)), (2, (8, 32, 32, 8000)), (2, (128, 32, 32, 256)),
+                     (2, (128, 32, 32, 150, 128)), (2, (128, 32, 32, 250, 128)), (3, (128, 32, 32, 500, 128)), (3, (16, 32, 32, 8000, 128)), (3, (100, 32, 32, 1000, 512)),
+                     (2, (32, 32, 32, 4000, 512)), (2, (64, 32, 32, 1500, 512))):
+        assert launches(*sizes) == n, sizes
     for bad in ((2, 6, 4, 100), (2, 6, 2, 100), (0, 8, 8, 100), (1, 8, 8, -1)):
         assert launches(*bad) == 3
     assert launches(2, 16, 8, 100, D=256) == 3 and launches(1, 8, 8, 100, bits=3) == 3
