@@ -1678,7 +1678,12 @@ constexpr int SM_CHUNK = SM_BLOCK * SM_KEEP;          // row elements a 256-thre
 constexpr int SM_ROW_MAX = 24576;                     // longest row a single workgroup keeps in registers
 
 // Rows [.., n] of an additive mask: fp32, fp16 or bfloat16, each widened as it is read (a conversion beforehand is
-// a launch, 3 us of a step that takes 25 to 65).  Rows are as aligned as their elements.
+// a launch, 3 us of a step that takes 25 to 65).  Rows are as aligned as their elements.  HALF: whether the
+// 16-bit types may come.  The kernels that keep a row in registers are there with and without: both ways of reading in
+// one kernel took 138 registers instead of 109, three waves to a SIMD instead of four (16 384 rows of 1025 with an
+// fp32 mask or none 22.5 / 19.0 us, in one kernel 28.5 / 22.8).  The chunked pair takes 2 registers less with both
+// (512 rows of 131 073 with an fp32 mask 99 us, 105 without the 16-bit types).
+template <bool HALF>
 struct MaskRow {
     const char *p; // null: no mask
     int dt;        // ADKV_DT_*
@@ -1689,13 +1694,13 @@ struct MaskRow {
     }
     __device__ __forceinline__ float at(int i) const
     {
-        if (dt == ADKV_DT_F32)
+        if (!HALF || dt == ADKV_DT_F32)
             return reinterpret_cast<const float *>(p)[i];
         return widen(reinterpret_cast<const uint16_t *>(p)[i]);
     }
     template <int V> __device__ __forceinline__ void load(int i, float *m) const
     {
-        if (dt == ADKV_DT_F32) {
+        if (!HALF || dt == ADKV_DT_F32) {
             __builtin_memcpy(m, p + (size_t)i * 4, 4 * V);
         } else {
             uint16_t raw[V];
@@ -1711,11 +1716,11 @@ struct Mask {
     const void *p; // [rows / rows_per_mask_row, n], or null
     int rows_per_mask_row, dt;
     // elements t0.. of the row of logits row `row`
-    __device__ __forceinline__ MaskRow of(size_t row, int n, int t0 = 0) const
+    template <bool HALF> __device__ __forceinline__ MaskRow<HALF> of(unsigned row, int n, int t0 = 0) const
     {
         if (p == nullptr)
             return {nullptr, dt};
-        return {(const char *)p + (row / (unsigned)rows_per_mask_row * n + t0) * (dt == ADKV_DT_F32 ? 4 : 2), dt};
+        return {(const char *)p + ((size_t)(row / (unsigned)rows_per_mask_row) * n + t0) * (!HALF || dt == ADKV_DT_F32 ? 4 : 2), dt};
     }
 };
 
@@ -1742,8 +1747,8 @@ __device__ __forceinline__ float block_reduce(float v, float *sm, bool is_max)
 // x[k] = logits*scaling + mask for the SM_KEEP elements of this thread in the chunk that starts at
 // `base` (-inf past the end of the row); 16-byte accesses wherever a whole vector lies inside the
 // row (rows are only 2-byte aligned: the hardware takes unaligned vector accesses).
-template <int NV = SM_NV, int NT = SM_BLOCK>
-__device__ __forceinline__ void softmax_load_chunk(const h1 *l, const MaskRow &mk, int n, int base,
+template <int NV = SM_NV, int NT = SM_BLOCK, bool HALF>
+__device__ __forceinline__ void softmax_load_chunk(const h1 *l, const MaskRow<HALF> &mk, int n, int base,
                                                    float scaling, float *x, float &mx,
                                                    int tid = (int)threadIdx.x)
 {
@@ -1764,7 +1769,7 @@ __device__ __forceinline__ void softmax_load_chunk(const h1 *l, const MaskRow &m
             }
             if (mk) {
                 float m8[SM_VEC];
-                mk.load<SM_VEC>(i0, m8);
+                mk.template load<SM_VEC>(i0, m8);
 #pragma unroll
                 for (int k = 0; k < SM_VEC; k++)
                     xv[k] += m8[k];
@@ -1815,7 +1820,7 @@ __device__ __forceinline__ void softmax_store_chunk(h1 *w, int n, int base, cons
 // Short rows: one wave per row (four rows per workgroup), the row in registers, reductions across
 // the wave only.  A workgroup per row would spend most of its time on two barriers for a handful of
 // elements per thread; rows of a few hundred tokens are the common decode case.
-template <int NV>
+template <int NV, bool HALF>
 __global__ __launch_bounds__(SM_BLOCK) void softmax_wave_kernel(
     const h1 *__restrict__ logits, h1 *__restrict__ weights, Mask mask, int rows, int n,
     long ld, float scaling)
@@ -1826,7 +1831,7 @@ __global__ __launch_bounds__(SM_BLOCK) void softmax_wave_kernel(
     const int lane = threadIdx.x & 63;
     const h1 *l = logits + (size_t)row * ld;
     h1 *w = weights + (size_t)row * ld;
-    const MaskRow mk = mask.of(row, n);
+    const MaskRow<HALF> mk = mask.of<HALF>(row, n);
     float x[NV * SM_VEC], mx;
     softmax_load_chunk<NV, 64>(l, mk, n, 0, scaling, x, mx, lane);
 #pragma unroll
@@ -1847,7 +1852,7 @@ __global__ __launch_bounds__(SM_BLOCK) void softmax_wave_kernel(
 // One workgroup of NT threads per row.  A row of up to NT * NV * 8 elements is read once and kept
 // in registers (the launcher picks NT and NV by the row length, up to 24576 elements); longer rows
 // are walked three times (the chunked kernels below avoid that when the caller gives a workspace).
-template <int NT, int NV>
+template <int NT, int NV, bool HALF>
 __global__ __launch_bounds__(NT) void softmax_kernel(
     const h1 *__restrict__ logits, h1 *__restrict__ weights, Mask mask, int n, long ld, float scaling)
 {
@@ -1855,7 +1860,7 @@ __global__ __launch_bounds__(NT) void softmax_kernel(
     const int row = blockIdx.x;
     const h1 *l = logits + (size_t)row * ld;
     h1 *w = weights + (size_t)row * ld;
-    const MaskRow mk = mask.of(row, n);
+    const MaskRow<HALF> mk = mask.of<HALF>(row, n);
 
     if (n <= NT * NV * SM_VEC) {
         float x[NV * SM_VEC], mx;
@@ -2029,7 +2034,7 @@ __global__ __launch_bounds__(SM_BLOCK) void softmax_part_kernel(
     __shared__ float2 sm[SM_BLOCK / 64];
     const int row = blockIdx.y, ck0 = blockIdx.x * SUB;
     const h1 *l = logits + (size_t)row * ld;
-    const MaskRow mk = mask.of(row, n);
+    const MaskRow<true> mk = mask.of<true>(row, n);
     float mx = -INFINITY, sum = 0.0f;
     if (SUB > 1 && !mk && (ck0 + SUB) * SM_CHUNK <= n) {
         uint4 raw[SUB][SM_NV];
@@ -2099,7 +2104,7 @@ __global__ __launch_bounds__(SM_BLOCK) void softmax_norm_kernel(
     const int row = blockIdx.y, ck = blockIdx.x;
     const h1 *l = logits + (size_t)row * ld;
     h1 *w = weights + (size_t)row * ld;
-    const MaskRow mk = mask.of(row, n);
+    const MaskRow<true> mk = mask.of<true>(row, n);
     float x[SM_KEEP], mx;
     softmax_load_chunk(l, mk, n, ck * SM_CHUNK, scaling, x, mx);   // issued first: in flight meanwhile
     if (threadIdx.x < 64) {
@@ -3035,6 +3040,100 @@ int adkv_encode_kv(void *cache, const void *kv_new,
 
 } // extern "C"
 
+template <bool HALF>
+static int softmax_launch(const void *logits, void *weights, const Mask &mask, int rows, int n, int64_t ld, float scaling,
+                          void *workspace, int64_t workspace_bytes, void *stream)
+{
+    if (!logits || !weights)
+        return ADKV_E_NULL;
+    if (rows <= 0 || n <= 0 || (mask.p && mask.rows_per_mask_row <= 0) || (ld != 0 && ld < n))
+        return ADKV_E_SHAPE;
+    if (ld == 0)
+        ld = n;
+    if (n <= 64 * SM_VEC * 4) {
+        // short rows: a wave per row, the row in 8, 16 or 32 registers per lane (longer rows were
+        // measured slower this way: 27 us against 22 us for 4096 rows of 4097 elements)
+        const dim3 grid((unsigned)((rows + SM_BLOCK / 64 - 1) / (SM_BLOCK / 64)));
+#define ADKV_SM_WAVE(NVW)                                                                           \
+    hipLaunchKernelGGL((softmax_wave_kernel<NVW, HALF>), grid, dim3(SM_BLOCK), 0, (hipStream_t)stream,      \
+                       (const h1 *)logits, (h1 *)weights, mask, rows, n, (long)ld, scaling)
+        if (n <= 64 * SM_VEC)
+            ADKV_SM_WAVE(1);
+        else if (n <= 64 * SM_VEC * 2)
+            ADKV_SM_WAVE(2);
+        else
+            ADKV_SM_WAVE(4);
+#undef ADKV_SM_WAVE
+        return check_launch();
+    }
+    const int reg_nv = (n + 1024 * SM_VEC - 1) / (1024 * SM_VEC); // 16-byte vectors per thread
+    if (n > SM_ROW_MAX && !mask.p && n <= SM_REG_MAX && (rows >= SM_REG_MIN_ROWS || reg_nv <= 9) &&
+        scaling != 0.0f && scaling == scaling) {
+        // long unmasked rows stay in registers, unless they are few and very long (32 rows of
+        // 131 073: 14.6 us cut into chunks, 19.8 us this way; 128 rows: 28.1 and 24.8; 512 rows:
+        // 74.8 and 56.7; 64 rows of 32 769: 11.4 and 9.4; 4096 rows of 24 577: 148 and 80)
+#define ADKV_SM_REG(NV)                                                                             \
+    case NV:                                                                                        \
+        hipLaunchKernelGGL(softmax_regrow_kernel<NV>, dim3((unsigned)rows), dim3(1024), 0,          \
+                           (hipStream_t)stream, (const h1 *)logits, (h1 *)weights, n, (long)ld,     \
+                           scaling);                                                                \
+        break
+        switch (reg_nv) {
+            ADKV_SM_REG(4); ADKV_SM_REG(5); ADKV_SM_REG(6); ADKV_SM_REG(7); ADKV_SM_REG(8);
+            ADKV_SM_REG(9); ADKV_SM_REG(10); ADKV_SM_REG(11); ADKV_SM_REG(12); ADKV_SM_REG(13);
+            ADKV_SM_REG(14); ADKV_SM_REG(15); ADKV_SM_REG(16);
+        default:
+            ADKV_SM_REG(17);
+        }
+#undef ADKV_SM_REG
+        return check_launch();
+    }
+    const int64_t need = adkv_softmax_workspace_bytes(rows, n);
+    if (need == 0 || !workspace || rows > 65535) {
+        // one workgroup per row, sized so that the row stays in its registers (read once, written
+        // once); rows beyond 24576 elements without a workspace are read three times
+#define ADKV_SM_ROW(NT, NV)                                                                         \
+    hipLaunchKernelGGL((softmax_kernel<NT, NV, HALF>), dim3((unsigned)rows), dim3(NT), 0,                 \
+                       (hipStream_t)stream, (const h1 *)logits, (h1 *)weights, mask, n, (long)ld, scaling)
+        // (threads, 16-byte vectors per thread) per row length, measured on 4096 rows: 4097 elements
+        // 18.4 us with 256 x 3 and 16.7 with 320 x 2; 8192: 35.5 with 512 x 3, 24.3 with 512 x 2;
+        // 10000: 36.9 with 512 x 3, 33.0 with 256 x 6; 16384: 76.5 with 1024 x 3, 46.9 with 1024 x 2;
+        // 2048 rows of 24576: 42.1 with 1024 x 3, 37.4 with 512 x 6
+        if (n <= 5120)
+            ADKV_SM_ROW(320, 2);
+        else if (n <= SM_CHUNK || n > SM_ROW_MAX)
+            ADKV_SM_ROW(SM_BLOCK, SM_NV);
+        else if (n <= 8192)
+            ADKV_SM_ROW(512, 2);
+        else if (n <= 12288)
+            ADKV_SM_ROW(256, 6);
+        else if (n <= 16384)
+            ADKV_SM_ROW(1024, 2);
+        else
+            ADKV_SM_ROW(512, 6);
+#undef ADKV_SM_ROW
+        return check_launch();
+    }
+    if (workspace_bytes < need)
+        return ADKV_E_WORKSPACE;
+    if ((uintptr_t)workspace & 7)
+        return ADKV_E_ALIGN;
+    const int nchunk = (n + SM_CHUNK - 1) / SM_CHUNK;
+    const dim3 grid((unsigned)nchunk, (unsigned)rows);
+    if (nchunk >= 8 && !mask.p) {
+        // long rows: four chunks per workgroup in the first pass
+        const dim3 grid4((unsigned)((nchunk + 3) / 4), (unsigned)rows);
+        hipLaunchKernelGGL(softmax_part_kernel<4>, grid4, dim3(SM_BLOCK), 0, (hipStream_t)stream,
+                           (const h1 *)logits, mask, (float2 *)workspace, n, (long)ld, nchunk, scaling);
+    } else {
+        hipLaunchKernelGGL(softmax_part_kernel<1>, grid, dim3(SM_BLOCK), 0, (hipStream_t)stream,
+                           (const h1 *)logits, mask, (float2 *)workspace, n, (long)ld, nchunk, scaling);
+    }
+    hipLaunchKernelGGL(softmax_norm_kernel, grid, dim3(SM_BLOCK), 0, (hipStream_t)stream,
+                       (const h1 *)logits, (h1 *)weights, mask, (const float2 *)workspace, n, (long)ld, nchunk, scaling);
+    return check_launch();
+}
+
 // Which decode kernel family and shape a launch of these sizes takes (the dispatch below, as text).
 static const char *decode_kernel_name(int B, int Hq, int H, int T, int D, int bits, int n_ckpt_cap,
                                       int ckpt_interval)
@@ -3457,104 +3556,11 @@ int64_t adkv_row_pitch(int n)
     return k * 128;
 }
 
-static int softmax_launch(const void *logits, void *weights, const Mask &mask, int rows, int n, int64_t ld, float scaling,
-                          void *workspace, int64_t workspace_bytes, void *stream)
-{
-    if (!logits || !weights)
-        return ADKV_E_NULL;
-    if (rows <= 0 || n <= 0 || (mask.p && mask.rows_per_mask_row <= 0) || (ld != 0 && ld < n))
-        return ADKV_E_SHAPE;
-    if (ld == 0)
-        ld = n;
-    if (n <= 64 * SM_VEC * 4) {
-        // short rows: a wave per row, the row in 8, 16 or 32 registers per lane (longer rows were
-        // measured slower this way: 27 us against 22 us for 4096 rows of 4097 elements)
-        const dim3 grid((unsigned)((rows + SM_BLOCK / 64 - 1) / (SM_BLOCK / 64)));
-#define ADKV_SM_WAVE(NVW)                                                                           \
-    hipLaunchKernelGGL(softmax_wave_kernel<NVW>, grid, dim3(SM_BLOCK), 0, (hipStream_t)stream,      \
-                       (const h1 *)logits, (h1 *)weights, mask, rows, n, (long)ld, scaling)
-        if (n <= 64 * SM_VEC)
-            ADKV_SM_WAVE(1);
-        else if (n <= 64 * SM_VEC * 2)
-            ADKV_SM_WAVE(2);
-        else
-            ADKV_SM_WAVE(4);
-#undef ADKV_SM_WAVE
-        return check_launch();
-    }
-    const int reg_nv = (n + 1024 * SM_VEC - 1) / (1024 * SM_VEC); // 16-byte vectors per thread
-    if (n > SM_ROW_MAX && !mask.p && n <= SM_REG_MAX && (rows >= SM_REG_MIN_ROWS || reg_nv <= 9) &&
-        scaling != 0.0f && scaling == scaling) {
-        // long unmasked rows stay in registers, unless they are few and very long (32 rows of
-        // 131 073: 14.6 us cut into chunks, 19.8 us this way; 128 rows: 28.1 and 24.8; 512 rows:
-        // 74.8 and 56.7; 64 rows of 32 769: 11.4 and 9.4; 4096 rows of 24 577: 148 and 80)
-#define ADKV_SM_REG(NV)                                                                             \
-    case NV:                                                                                        \
-        hipLaunchKernelGGL(softmax_regrow_kernel<NV>, dim3((unsigned)rows), dim3(1024), 0,          \
-                           (hipStream_t)stream, (const h1 *)logits, (h1 *)weights, n, (long)ld,     \
-                           scaling);                                                                \
-        break
-        switch (reg_nv) {
-            ADKV_SM_REG(4); ADKV_SM_REG(5); ADKV_SM_REG(6); ADKV_SM_REG(7); ADKV_SM_REG(8);
-            ADKV_SM_REG(9); ADKV_SM_REG(10); ADKV_SM_REG(11); ADKV_SM_REG(12); ADKV_SM_REG(13);
-            ADKV_SM_REG(14); ADKV_SM_REG(15); ADKV_SM_REG(16);
-        default:
-            ADKV_SM_REG(17);
-        }
-#undef ADKV_SM_REG
-        return check_launch();
-    }
-    const int64_t need = adkv_softmax_workspace_bytes(rows, n);
-    if (need == 0 || !workspace || rows > 65535) {
-        // one workgroup per row, sized so that the row stays in its registers (read once, written
-        // once); rows beyond 24576 elements without a workspace are read three times
-#define ADKV_SM_ROW(NT, NV)                                                                         \
-    hipLaunchKernelGGL((softmax_kernel<NT, NV>), dim3((unsigned)rows), dim3(NT), 0,                 \
-                       (hipStream_t)stream, (const h1 *)logits, (h1 *)weights, mask, n, (long)ld, scaling)
-        // (threads, 16-byte vectors per thread) per row length, measured on 4096 rows: 4097 elements
-        // 18.4 us with 256 x 3 and 16.7 with 320 x 2; 8192: 35.5 with 512 x 3, 24.3 with 512 x 2;
-        // 10000: 36.9 with 512 x 3, 33.0 with 256 x 6; 16384: 76.5 with 1024 x 3, 46.9 with 1024 x 2;
-        // 2048 rows of 24576: 42.1 with 1024 x 3, 37.4 with 512 x 6
-        if (n <= 5120)
-            ADKV_SM_ROW(320, 2);
-        else if (n <= SM_CHUNK || n > SM_ROW_MAX)
-            ADKV_SM_ROW(SM_BLOCK, SM_NV);
-        else if (n <= 8192)
-            ADKV_SM_ROW(512, 2);
-        else if (n <= 12288)
-            ADKV_SM_ROW(256, 6);
-        else if (n <= 16384)
-            ADKV_SM_ROW(1024, 2);
-        else
-            ADKV_SM_ROW(512, 6);
-#undef ADKV_SM_ROW
-        return check_launch();
-    }
-    if (workspace_bytes < need)
-        return ADKV_E_WORKSPACE;
-    if ((uintptr_t)workspace & 7)
-        return ADKV_E_ALIGN;
-    const int nchunk = (n + SM_CHUNK - 1) / SM_CHUNK;
-    const dim3 grid((unsigned)nchunk, (unsigned)rows);
-    if (nchunk >= 8 && !mask.p) {
-        // long rows: four chunks per workgroup in the first pass
-        const dim3 grid4((unsigned)((nchunk + 3) / 4), (unsigned)rows);
-        hipLaunchKernelGGL(softmax_part_kernel<4>, grid4, dim3(SM_BLOCK), 0, (hipStream_t)stream,
-                           (const h1 *)logits, mask, (float2 *)workspace, n, (long)ld, nchunk, scaling);
-    } else {
-        hipLaunchKernelGGL(softmax_part_kernel<1>, grid, dim3(SM_BLOCK), 0, (hipStream_t)stream,
-                           (const h1 *)logits, mask, (float2 *)workspace, n, (long)ld, nchunk, scaling);
-    }
-    hipLaunchKernelGGL(softmax_norm_kernel, grid, dim3(SM_BLOCK), 0, (hipStream_t)stream,
-                       (const h1 *)logits, (h1 *)weights, mask, (const float2 *)workspace, n, (long)ld, nchunk, scaling);
-    return check_launch();
-}
-
 int adkv_softmax_ex(const void *logits, void *weights, const void *mask,
                     int rows, int n, int64_t ld, int rows_per_mask_row, float scaling,
                     void *workspace, int64_t workspace_bytes, void *stream)
 {
-    return softmax_launch(logits, weights, {mask, rows_per_mask_row, ADKV_DT_F32}, rows, n, ld, scaling, workspace,
+    return softmax_launch<false>(logits, weights, {mask, rows_per_mask_row, ADKV_DT_F32}, rows, n, ld, scaling, workspace,
                           workspace_bytes, stream);
 }
 
@@ -3763,7 +3769,8 @@ int adkv_decode_step(const void *q, void *k_cache, void *v_cache, const void *k_
     if (rc || (rc = stage_mark(1, stream)))
         return rc;
     const int64_t smb = pad256(adkv_softmax_workspace_bytes(B * Hq, T + 1));
-    rc = softmax_launch(logits, weights, mk, B * Hq, T + 1, ld, scaling, smb ? ws + 2 * mat : nullptr, smb, stream);
+    rc = (mask && mask_dtype != ADKV_DT_F32 ? softmax_launch<true> : softmax_launch<false>)(
+        logits, weights, mk, B * Hq, T + 1, ld, scaling, smb ? ws + 2 * mat : nullptr, smb, stream);
     if (rc || (rc = stage_mark(2, stream)))
         return rc;
     rc = forward_ov_impl(weights, v_cache, v_new, out, v_params[0], v_params[1], v_params[2],

@@ -78,7 +78,7 @@ __device__ __forceinline__ void segment_weights(const h1 *logits, long pitch, co
         }
 #pragma unroll
     for (int g = 0; g < GQ; g++) {
-        const MaskRow mrow = mk.of(row0 + g, n, t0);
+        const MaskRow<true> mrow = mk.of<true>((unsigned)row0 + g, n, t0);
         float x[NC][V], mx = -INFINITY;
 #pragma unroll
         for (int c = 0; c < NC; c++) {
@@ -262,7 +262,7 @@ __global__ __launch_bounds__(256) void step_combine_kernel(
         if (t >= n)
             return;
         const uint32_t w[4] = {raw.x, raw.y, raw.z, raw.w};
-        const MaskRow mrow = mk.of(row, n);
+        const MaskRow<true> mrow = mk.of<true>((unsigned)row, n);
         uint32_t o[4];
 #pragma unroll
         for (int k = 0; k < 4; k++) {

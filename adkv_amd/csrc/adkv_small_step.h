@@ -84,7 +84,7 @@ __global__ __launch_bounds__(256) void small_step_kernel(
         // for another, and the copy it reads from is its own.
         h1 *w = reinterpret_cast<h1 *>(tile);
         float x[SMALL_ROW / 64], mx;
-        softmax_load_chunk<SMALL_ROW / 512, 64>(logits, mask.of(bx, n), n, 0,
+        softmax_load_chunk<SMALL_ROW / 512, 64>(logits, mask.of<true>(bx, n), n, 0,
                                                 scaling, x, mx, lane);
 #pragma unroll
         for (int m = 1; m < 64; m <<= 1)

@@ -1,9 +1,11 @@
-"""Registers that a matrix instruction still has to write are left alone until it has, in the library as built.
+"""The device code of the library as built.
 
-The hardware does not hold back a vector instruction that reads or overwrites such a register; the compiler keeps
+Registers that a matrix instruction still has to write are left alone until it has: the hardware does not hold back a vector instruction that reads or overwrites such a register; the compiler keeps
 the distance between its own instructions, but not to a hand-laid block, and it hands registers of a result that
 nobody reads to the next block at once: what the block has left there is then overwritten behind its back, now
-and then, as the waves of a SIMD happen to interleave."""
+and then, as the waves of a SIMD happen to interleave.
+
+Kernels that live from the number of their waves leave room for them."""
 import os
 import re
 import shutil
@@ -78,12 +80,19 @@ def listings(tmp_path_factory):
             offset, size, n = struct.unpack_from("<QQQ", fat, p)
             if b"gfx950" in fat[p + 24:p + 24 + n]:
                 (d / "code").write_bytes(fat[m.start() + offset:m.start() + offset + size])
-                found.append(subprocess.run([f"{LLVM}/llvm-objdump", "-d", "--no-show-raw-insn", f"{d}/code"], check=True,
-                                            capture_output=True, text=True).stdout)
+                found.append([subprocess.run([f"{LLVM}/{tool}", *how, f"{d}/code"], check=True, capture_output=True, text=True).stdout
+                              for tool, *how in (("llvm-objdump", "-d", "--no-show-raw-insn"), ("llvm-readelf", "--notes"))])
             p += 24 + n
     return found
 
 
 def test_results_of_matrix_instructions_are_left_alone_until_written(listings):
-    assert sum(t.count("\tv_mfma") for t in listings) > 1000               # the listings are what they should be
-    assert not [v for t in listings for v in violations(t)][:5]
+    assert sum(t.count("\tv_mfma") for t, _ in listings) > 1000            # the listings are what they should be
+    assert not [v for t, _ in listings for v in violations(t)][:5]
+
+
+def test_rows_without_16_bit_masks_keep_four_waves_to_a_simd(listings):
+    """Of 512 registers, in steps of 8: at most 128 each."""
+    found = [(name, int(vgprs)) for _, notes in listings
+             for name, vgprs in re.findall(r"\.name: +(\S*softmax_(?:wave_)?kernel\S*Lb0E\S*)\n.*?\.vgpr_count: +(\d+)", notes, re.S)]
+    assert len(found) == 9 and not [f for f in found if f[1] > 128], found
