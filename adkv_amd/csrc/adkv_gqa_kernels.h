@@ -490,10 +490,14 @@ __device__ __forceinline__ void ov_gqa_segment(const uint2 *lut, uint32_t lane_c
 
     if (last) {
         // ragged tail, then the appended token: a handful of tokens, plain fp32 multiply-adds
-        auto add_token = [&](const h2 *vd, int t) {
+        h1 wT[GQ]; // before the stores: they may not be loaded ahead of them afterwards, and cost 0.5 us
+#pragma unroll
+        for (int g = 0; g < GQ; g++)
+            wT[g] = w1(g, T - t0);
+        auto add_token = [&](const h2 *vd, auto &&weight) {
 #pragma unroll
             for (int g = 0; g < GQ; g++) {
-                const float wt = (float)w1(g, t);
+                const float wt = (float)weight(g);
 #pragma unroll
                 for (int p = 0; p < G::NP; p++) {
                     acc[g >> 2][2 * p][g & 3] = __builtin_fmaf(wt, (float)vd[p].x, acc[g >> 2][2 * p][g & 3]);
@@ -516,14 +520,14 @@ __device__ __forceinline__ void ov_gqa_segment(const uint2 *lut, uint32_t lane_c
                     vd[pp] = qs + s.zp;
                     update_pair(s, qc, qs);
                 }
-                add_token(vd, nfull * TPW + tt);
+                add_token(vd, [&](int g) { return w1(g, nfull * TPW + tt); });
             }
         }
         if (active)
             publish_state<D, CPL>(st, state_out, sa, bx, c0, T);
         h2 deq[G::NP];
         append_new_token<D, CPL, BITS>(cbh, T, v_new + (size_t)bx * D + c0, st, deq, active, sa.act_bf16);
-        add_token(deq, T - t0);
+        add_token(deq, [&](int g) { return wT[g]; });
     }
 }
 

@@ -422,6 +422,21 @@ struct Unit {
     }
 };
 
+// Parameters plus the state this segment starts from.
+template <int D, int CPL>
+__device__ __forceinline__ void init_pairs(Pair *st, const h1 *zp, const h1 *sc, const h1 *al,
+                                           const h1 *be, const h1 *tg, int h, int bx, int c0, int seg,
+                                           const Seg &sa)
+{
+#pragma unroll
+    for (int p = 0; p < CPL / 2; p++)
+        load_pair(st[p], zp, sc, al, be, tg, h * D + c0 + 2 * p);
+    if (seg_begin(sa, seg) > 0) {
+        const int j = seg_begin(sa, seg) / sa.ckpt_interval - 1;
+        load_state<CPL>(sa.ckpt + (((size_t)bx * sa.n_ckpt_cap + j) * D + c0) * 2, st);
+    }
+}
+
 // What a unit reads before it can decode: parameters, the state its segment starts from, the first
 // supergroups of codes.  start() issues the loads and waits for none of them, so they travel while
 // the workgroup writes its table; state() is for after it.  One after the other behind the table (parameters, the
@@ -1558,45 +1573,187 @@ __device__ __forceinline__ void ov_segment(const uint2 *lut, uint32_t lane_copy,
     }
 }
 
+// forward_ov by itself keeps its loads behind the table and the loop to itself: built from ov_segment with the loads
+// on their way meanwhile it was 0.5 to 1 us longer in launches of few waves (1 x 32 heads x 256 tokens 9.4 / 10.4 us)
+// and 3 to 8 % in long ones of wide heads (4 x 8 heads of 256 channels x 5000 tokens, no checkpoints, 188 / 202 us): the
+// compiler orders and waits otherwise.
 template <int D, int CPL, int BLK>
 __global__ __launch_bounds__(BLK) void ov_kernel(
-    const h1 *attn, uint4 *__restrict__ cache, const h1 *v_new,
+    const h1 *__restrict__ attn, uint4 *__restrict__ cache, const h1 *__restrict__ v_new,
     h1 *__restrict__ out, float *__restrict__ partial,
-    const h1 *zp, const h1 *sc, const h1 *al,
-    const h1 *be, const h1 *tg,
+    const h1 *__restrict__ zp, const h1 *__restrict__ sc, const h1 *__restrict__ al,
+    const h1 *__restrict__ be, const h1 *__restrict__ tg,
     int BH, int H, int T, int n_super_cap, h1 *__restrict__ state_out, Seg sa)
 {
     using G = Geo<D, CPL>;
     constexpr int AHEAD = CPL == 2 ? PF_PAIR : PF;
     sa.groups = 0; // only even plans come here
     __shared__ uint2 lut[LUT_WORDS64];
+    lut_fill<BLK>(lut, threadIdx.x);
+    __syncthreads();
     const uint32_t lane_copy = (uint32_t)(threadIdx.x & (LUT_COPIES - 1)) * 8u;
 
     const Unit<D, CPL, BLK> un(BH, sa.nseg);
+    if (!un.wave_active)
+        return; // padding waves
     const int bx = un.bx, lh = un.lh, c0 = un.c0;
     const bool active = un.active;
-    SegLoads<D, CPL, 4, AHEAD> s;
-    s.start(cache, zp, sc, al, be, tg, bx % H, bx, lh, un.seg, T, n_super_cap, sa);
-    const int nfull = s.nfull;
-    const h1 *wb = attn + (size_t)bx * sa.row_pitch + s.t0;
+    const bool last = seg_is_last(sa, un.seg);
+    const int h = bx % H;
+
+    Pair st[G::NP];
+    float acc[CPL];
+    init_pairs<D, CPL>(st, zp, sc, al, be, tg, h, bx, c0, un.seg, sa);
+#pragma unroll
+    for (int c = 0; c < CPL; c++)
+        acc[c] = 0.0f;
+    // Four-channel (and wider) lanes contract on the matrix cores, as ov_ft_kernel does and for the
+    // reason given there: B = the lane's dequantised pair at two tokens, A = (w[t], 0, w[t+1], 0)
+    // from lane 0 of each group of four, (0, w[t], 0, w[t+1]) from lane 1, zeros from lanes 2, 3.
+    constexpr bool MM = CPL >= 4;
+    f4v acc4[G::NP];
+#pragma unroll
+    for (int p = 0; p < G::NP; p++)
+        acc4[p] = (f4v){0.0f, 0.0f, 0.0f, 0.0f};
+    const int role = threadIdx.x & 3;
+    const uint32_t sel_a0 = role == 0 ? 0x0C0C0100u : role == 1 ? 0x01000C0Cu : 0x0C0C0C0Cu;
+    const uint32_t sel_a1 = role == 0 ? 0x0C0C0302u : role == 1 ? 0x03020C0Cu : 0x0C0C0C0Cu;
+
+    const int t0 = seg_begin(sa, un.seg);
+    const int t1 = last ? T : seg_end(sa, un.seg);
+    using Vec = typename G::Vec;
+    Vec *cbh = reinterpret_cast<Vec *>(cache) + (size_t)bx * n_super_cap * G::VPS + lh * G::NV;
+    const Vec *cb = cbh + (size_t)(t0 >> 3) * G::VPS;
+    const h1 *wrow = attn + (size_t)bx * sa.row_pitch;
+    const h1 *wb = wrow + t0;
+    const int nfull = (t1 - t0) >> 3;
+
     auto load_w = [&](int sg) {
         uint4 r;
         __builtin_memcpy(&r, wb + (size_t)sg * 8, 16); // row base is only 2-byte aligned
         return r;
     };
-    uint4 wbuf[AHEAD];
-    if (nfull > 0)
+    // two tokens of the current supergroup on the matrix cores, then the lookups of the same two
+    // slots of the next one
+    auto token2 = [&](int t, uint2 (*e)[8], const uint32_t (*nb)[2], const uint4 wv) {
+        const uint32_t ww[4] = {wv.x, wv.y, wv.z, wv.w};
+        const uint32_t w2 = ww[t >> 1];
+        const h4v a = as_h4(__builtin_amdgcn_perm(w2, w2, sel_a0), __builtin_amdgcn_perm(w2, w2, sel_a1));
+        uint32_t vd[G::NP][2];
 #pragma unroll
-        for (int i = 0; i < AHEAD; i++)
-            wbuf[i] = load_w(min(i, nfull - 1));
-    lut_fill<BLK>(lut, threadIdx.x);
-    __syncthreads();
-    if (!un.wave_active)
-        return; // padding waves
+        for (int k = 0; k < 2; k++)
+#pragma unroll
+            for (int p = 0; p < G::NP; p++) {
+                Pair &s = st[p];
+                const h2 qs = as_h2(e[p][t + k].x) * s.sc;
+                vd[p][k] = as_u32(qs + s.zp);
+                update_pair_abs(s, as_h2(e[p][t + k].y), qs);
+            }
+#pragma unroll
+        for (int p = 0; p < G::NP; p++)
+            acc4[p] = __builtin_amdgcn_mfma_f32_4x4x4f16(a, as_h4(vd[p][0], vd[p][1]), acc4[p], 0, 0, 0);
+#pragma unroll
+        for (int k = 0; k < 2; k++)
+#pragma unroll
+            for (int p = 0; p < G::NP; p++)
+                e[p][t + k] = lut_get(lut, nb[p][(t + k) & 1], lane_copy, (t + k) >> 1);
+        __builtin_amdgcn_sched_barrier(0);
+    };
 
-    float acc[CPL];
-    ov_segment<D, CPL, AHEAD>(lut, lane_copy, bx, c0, active, s, wbuf, load_w, [&](int t) { return wb[t]; }, v_new, T,
-                              state_out, sa, acc);
+    Vec buf[AHEAD][G::NV];
+    uint4 wbuf[AHEAD];
+    uint2 lk[MM ? G::NP : 2][8]; // two channels per lane: this supergroup's lookups and the next one's
+    uint32_t nb[G::NP][2];
+    if (nfull > 0) {
+        // unconditional, in the loop's order: see qk_kernel
+#pragma unroll
+        for (int i = 0; i < AHEAD; i++) {
+            const int sg = min(i, nfull - 1);
+#pragma unroll
+            for (int v = 0; v < G::NV; v++)
+                buf[i][v] = load_codes(cb + (size_t)sg * G::VPS + v);
+            wbuf[i] = load_w(sg);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        pair_bytes_of<D, CPL>(buf[0], nb);
+#pragma unroll
+        for (int t = 0; t < 8; t++)
+#pragma unroll
+            for (int p = 0; p < G::NP; p++)
+                lk[p][t] = lut_get(lut, nb[p][t & 1], lane_copy, t >> 1);
+        wait_lgkm();
+    }
+    // one supergroup, nothing conditional in it (see qk_kernel); i = its buffer in the rotation
+    auto body = [&](int sg, auto ic) {
+        constexpr int i = decltype(ic)::value;
+        pair_bytes_of<D, CPL>(buf[(i + 1) % AHEAD], nb);
+        const int sgp = min(sg + AHEAD, nfull - 1);
+#pragma unroll
+        for (int v = 0; v < G::NV; v++)
+            buf[i][v] = load_codes(cb + (size_t)sgp * G::VPS + v);
+        __builtin_amdgcn_sched_barrier(0);
+        if constexpr (MM) {
+#pragma unroll
+            for (int t = 0; t < 8; t += 2)
+                token2(t, lk, nb, wbuf[i]);
+        } else {
+            // a wave (nearly) alone on its SIMD: see replay_eight
+#pragma unroll
+            for (int t = 0; t < 8; t++)
+                lk[(i & 1) ^ 1][t] = lut_get(lut, nb[0][t & 1], lane_copy, t >> 1);
+            replay_eight_weighted(st[0], lk[i & 1], wbuf[i], acc);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        // the weights are reloaded once their last token is done: loading them earlier into a
+        // second register set costs copies at the loop edge, which wait for the load they move
+        wbuf[i] = load_w(sgp);
+    };
+    rotate_over<AHEAD>(nfull, body);
+    if (MM) {
+#pragma unroll
+        for (int p = 0; p < G::NP; p++) {
+            acc[2 * p] = acc4[p].x;
+            acc[2 * p + 1] = acc4[p].y;
+        }
+    }
+
+    if (last) {
+        const int ntail = (t1 - t0) & 7;
+        if (ntail) {
+#pragma unroll
+            for (int v = 0; v < G::NV; v++) {
+                uint32_t w[G::WPV];
+                vec_words(cb[(size_t)nfull * G::VPS + v], w);
+#pragma unroll
+                for (int pp = 0; pp < G::WPV / 2; pp++) {
+                    Pair &s = st[(G::WPV / 2) * v + pp];
+                    for (int tt = 0; tt < ntail; tt++) {
+                        const uint32_t na = (w[2 * pp] >> (4 * tt)) & 0xFu;
+                        const uint32_t nbb = (w[2 * pp + 1] >> (4 * tt)) & 0xFu;
+                        const h2 qc = codes_to_h2((int)na - 8, (int)nbb - 8);
+                        const h2 qs = qc * s.sc;
+                        const h2 vd = qs + s.zp;
+                        const float wt = (float)wb[nfull * 8 + tt];
+                        const int c = G::WPV * v + 2 * pp;
+                        acc[c] = __builtin_fmaf(wt, (float)vd.x, acc[c]);
+                        acc[c + 1] = __builtin_fmaf(wt, (float)vd.y, acc[c + 1]);
+                        update_pair(s, qc, qs);
+                    }
+                }
+            }
+        }
+        if (active)
+            publish_state<D, CPL>(st, state_out, sa, bx, c0, T);
+
+        h2 deq[G::NP];
+        append_new_token<D, CPL>(cbh, T, v_new + (size_t)bx * D + c0, st, deq, active, sa.act_bf16);
+        const float wT = (float)wrow[T];
+#pragma unroll
+        for (int p = 0; p < G::NP; p++) {
+            acc[2 * p] = __builtin_fmaf(wT, (float)deq[p].x, acc[2 * p]);
+            acc[2 * p + 1] = __builtin_fmaf(wT, (float)deq[p].y, acc[2 * p + 1]);
+        }
+    }
     if (!active)
         return;
     if (sa.nseg == 1) {

@@ -5,7 +5,8 @@ the distance between its own instructions, but not to a hand-laid block, and it 
 nobody reads to the next block at once: what the block has left there is then overwritten behind its back, now
 and then, as the waves of a SIMD happen to interleave.
 
-Kernels that live from the number of their waves leave room for them."""
+Kernels that live from the number of their waves leave room for them, and those that live from their loads in flight
+do not wait for the youngest of them."""
 import os
 import re
 import shutil
@@ -29,15 +30,15 @@ def _registers(text):
     return regs
 
 
-def violations(listing):
-    """(kernel, wait states, matrix instruction, vector instruction) of every pair that is too close, along every path."""
+def kernels(listing, with_):
+    """(name, [(instruction, operands, address)], function from an index to those that may follow it)."""
     for name, body in re.findall(r"^[0-9a-f]+ <(\S+)>:\n(.*?)(?=^[0-9a-f]+ <|\Z)", listing, re.S | re.M):
-        if "v_mfma" not in body:
+        if with_ not in name + body:
             continue
         code = re.findall(r"^\t(\S+)(?: +([^/\n]*?))? *// ([0-9A-F]+):.*$", body, re.M)
         at = {int(a, 16): i for i, (_, _, a) in enumerate(code)}
 
-        def after(i):                                                      # where the wave goes next
+        def after(i, code=code, at=at):
             op, args, addr = code[i]
             if op == "s_endpgm":
                 return []
@@ -46,7 +47,12 @@ def violations(listing):
                 to = at.get(int(addr, 16) + 4 + 4 * (off - 65536 if off > 32767 else off))
                 return [to] if op == "s_branch" else [to, i + 1]
             return [i + 1]
+        yield name, code, after
 
+
+def violations(listing):
+    """(kernel, wait states, matrix instruction, vector instruction) of every pair that is too close, along every path."""
+    for name, code, after in kernels(listing, "v_mfma"):
         for i, (op, args, _) in enumerate(code):
             if not op.startswith("v_mfma"):
                 continue
@@ -96,3 +102,12 @@ def test_rows_without_16_bit_masks_keep_four_waves_to_a_simd(listings):
     found = [(name, int(vgprs)) for _, notes in listings
              for name, vgprs in re.findall(r"\.name: +(\S*softmax_(?:wave_)?kernel\S*Lb0E\S*)\n.*?\.vgpr_count: +(\d+)", notes, re.S)]
     assert len(found) == 9 and not [f for f in found if f[1] > 128], found
+
+
+def test_the_weights_loop_keeps_its_loads_in_flight(listings):
+    """Codes and weights of seven supergroups, two loads each."""
+    (name, code, after), = [k for t, _ in listings for k in kernels(t, "9ov_kernelILi128ELi2ELi256E")]
+    loops = [code[min(after(i)):i + 1] for i in range(len(code)) if code[i][0].startswith("s_cbranch") and min(after(i)) < i]
+    loop = max(loops, key=lambda b: sum(o.startswith("v_pk") for o, _, _ in b) / len(b) if len(b) > 100 else 0)
+    waits = [int(n) for o, a, _ in loop if o == "s_waitcnt" for n in re.findall(r"vmcnt\((\d+)\)", a)]
+    assert len(waits) == 8 and min(waits) == 14, waits
