@@ -2472,16 +2472,29 @@ static int threads_per_workgroup(long threads)
 // 2-bit ones), ov_gqa_kernel spills accumulators and loses (421 -> 533 us, 346 -> 747 us), so BIG8 says
 // which of the two this is, and the latter takes 8-wave workgroups.
 // A launch that would leave at most two waves on a SIMD takes two channels per lane instead (a KV head
-// per wave): twice the waves, forward_qk without the reduction over the quarters of a head.  8 x 8 KV
-// heads x 16001 tokens, four query heads each (16 waves per CU instead of 8), kernel times: forward_qk
-// 31.3 / 28.3 us, forward_ov 27.9 / 27.5.  With more waves than that the four-channel lanes have enough
-// of them and spend fewer instructions on what a wave does once per token.
+// per wave): twice the waves, forward_qk without the reduction over the quarters of a head.  With more waves than
+// that the four-channel lanes have enough of them and spend fewer instructions on what a wave does once per token.
+// forward_ov has nothing to reduce and pays for its weights once per wave: 16 bytes per lane and eight tokens, as often
+// with half of the channels, and several times that from rows that are not 16-byte aligned.  So it takes two
+// channels up to this many waves of them per SIMD: four with one query head, and with two where rows are aligned,
+// three with four heads, two with eight; from other rows two with two heads, less than two with more.  us, four channels
+// per lane / two, 16 x 8 KV heads: aligned, four heads x 4000 tokens (two waves) 25.0 / 18.6, 5000 (2.5) 26.1 / 23.0,
+// 8000 (four) 29.0 / 29.3, eight heads 30.9 / 27.5, 32.5 / 35.5, 34.2 / 45.4; other rows, two heads 25.1 / 19.1,
+// 25.8 / 26.1, 27.5 / 41.0, four 29.7 / 29.5, 30.9 / 41.3, 38.4 / 63.7; 128 x 8 x 300, four heads 19.7 / 25.4.
 static bool gqa_pair(long BH, int nseg) { return padded_units<64>((int)BH, nseg) <= 4L * n_simd(); }
+static bool ov_gqa_pair(long BH, int nseg, int GQ, bool aligned)
+{
+    const long waves = padded_units<64>((int)BH, nseg);
+    if (GQ == 1 || (GQ == 2 && aligned))
+        return waves <= 4L * n_simd();
+    if (aligned)
+        return waves <= (GQ == 4 ? 3L : 2L) * n_simd();
+    return GQ == 2 ? waves <= 2L * n_simd() : waves < 2L * n_simd();
+}
 #define ADKV_LAUNCH_GQA_(KERNEL, BB, GQV, BLK, CPLV, ...)                                          \
     hipLaunchKernelGGL((KERNEL<BB, GQV, BLK, CPLV>), dim3((unsigned)((threads + (BLK)-1) / (BLK))), dim3(BLK), 0, st, __VA_ARGS__)
 #define ADKV_LAUNCH_GQA(KERNEL, BIG8, BB, GQV, ...)                                                \
     do {                                                                                            \
-        const bool pair = gqa_pair(BH, seg.nseg);                                                   \
         const long threads = pair ? padded_units<64>(BH, seg.nseg) * 64 : padded_units<32>(BH, seg.nseg) * 32; \
         const int blk = threads_per_workgroup(threads);                                             \
         constexpr bool BIG = GQV <= 4 || BIG8;                                                      \
@@ -2493,8 +2506,10 @@ static bool gqa_pair(long BH, int nseg) { return padded_units<64>((int)BH, nseg)
             ADKV_LAUNCH_GQA_(KERNEL, BB, GQV, 256, 2, __VA_ARGS__);                                 \
         else if (blk == 1024 || !BIG)                                                               \
             ADKV_LAUNCH_GQA_(KERNEL, BB, GQV, (BIG ? 1024 : 512), 4, __VA_ARGS__);                  \
-        else /* more than eight waves per CU: never 256 */                                          \
+        else if (blk == 768 || BIG8) /* forward_qk: more than eight waves per CU, never 256 */      \
             ADKV_LAUNCH_GQA_(KERNEL, BB, GQV, (BIG ? 768 : 512), 4, __VA_ARGS__);                   \
+        else                                                                                        \
+            ADKV_LAUNCH_GQA_(KERNEL, BB, GQV, (BIG8 ? 768 : 512), 4, __VA_ARGS__);                  \
     } while (0)
 
 #define ADKV_DISPATCH_GQ_BITS(KERNEL, BIG8, BB, ...)                                               \
@@ -3369,6 +3384,7 @@ static int forward_qk_impl(const void *q, void *k_cache, const void *k_new, void
     if (D == 128 && (GQ > 1 || bits != 4 || mfma_for_mha())) {
         if (GQ <= 4) // eight query heads per KV head may fall back to 8-wave workgroups
             plan_uneven(seg, T, padded_units<32>(BH, seg.nseg) * 32, GQA_SKEW_QK);
+        const bool pair = gqa_pair(BH, seg.nseg);
         ADKV_DISPATCH_GQ(qk_gqa_kernel, true, (const h1 *)q, (uint4 *)k_cache, (const h1 *)k_new,
                          (h1 *)logits, (const h1 *)zp, (const h1 *)sc, (const h1 *)alpha,
                          (const h1 *)beta, (const h1 *)tgt, BH, H, T, n_super_cap, (h1 *)state_out,
@@ -3540,6 +3556,7 @@ static int forward_ov_impl(const void *attn, void *v_cache, const void *v_new, v
     if (matrix_cores) {
         if (GQ <= 4)
             plan_uneven(seg, T, padded_units<32>(BH, seg.nseg) * 32, GQA_SKEW_OV);
+        const bool pair = ov_gqa_pair(BH, seg.nseg, GQ, ((uintptr_t)attn & 15) == 0 && seg.row_pitch % 8 == 0);
         ADKV_DISPATCH_GQ(ov_gqa_kernel, false, (const h1 *)attn, (uint4 *)v_cache, (const h1 *)v_new,
                          (h1 *)out, (float *)workspace, (const h1 *)zp, (const h1 *)sc,
                          (const h1 *)alpha, (const h1 *)beta, (const h1 *)tgt, BH, H, T, n_super_cap,

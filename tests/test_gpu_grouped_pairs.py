@@ -55,3 +55,22 @@ def test_two_channels_per_lane(gpu, oracle, bits, G, T, pair):
     lg, og = _np16(lg[0]).astype(np.float64), _np16(og[0]).astype(np.float64)
     assert np.all(np.abs(lg - lw) <= _ulp16(lw) + 1e-3)
     assert np.all(np.abs(og - ow) <= _ulp16(ow) + 1e-3)
+
+
+@pytest.mark.parametrize("bits", [4, 2])
+@pytest.mark.parametrize("G", [2, 4, 8])
+@pytest.mark.parametrize("segments", [127, 128, 129, 192, 193])          # two and three waves per SIMD, and either side
+def test_values_from_rows_of_any_alignment(gpu, bits, G, segments):
+    """Two or four channels per lane, which the rows' alignment decides as well: the same sums, bit for bit."""
+    S = 32 // bits
+    T = S * segments - 3
+    x, p = _inputs(B, H, T + 1, D, seed=segments, bits=bits)
+    p = [t.to(gpu) for t in p.astuple()]
+    cache = synth.alloc_cache(B, H, T + S, D, gpu, bits=bits)
+    ckpt = torch.zeros(B, H, T // S + 1, D, 2, dtype=torch.float16, device=gpu)
+    state = torch.zeros(B, H, D, 2, dtype=torch.float16, device=gpu)
+    gemv.append_kv(cache, x[:, :, :T].contiguous().to(gpu), *p, 0, state, ckpt=ckpt, ckpt_interval=S, bits=bits)
+    rows = torch.rand(B, H * G, (T + 8) // 8 * 8, generator=torch.Generator().manual_seed(G)).half().to(gpu)[:, :, :T + 1]
+    got = [gemv.forward_ov(w, cache.clone(), x[:, :, T:].contiguous().to(gpu), *p, SMIN, SMAX, ckpt=ckpt.clone(), ckpt_interval=S, bits=bits)
+           for w in (rows, rows.contiguous())]
+    assert torch.equal(*got) and torch.all(torch.isfinite(got[0]))
