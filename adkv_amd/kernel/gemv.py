@@ -403,8 +403,9 @@ def append_kv_pair(
     ``fresh``: the caches, states and checkpoints are uninitialised memory (``torch.empty``) and the
     tokens are their first (``T0 == 0``); the launch also zeroes the slots and checkpoints past them.
     """
-    rc = _lib.host().append(k_cache, v_cache, k_new, v_new, tuple(k_params), tuple(v_params), T0, k_state, v_state,
-                            k_ckpt, v_ckpt, ckpt_interval, bits, fresh)
+    k_params, v_params = tuple(k_params), tuple(v_params)      # read twice: they may be iterators
+    rc = _lib.host().append(k_cache, v_cache, k_new, v_new, k_params, v_params, T0, k_state, v_state, k_ckpt,
+                            v_ckpt, ckpt_interval, bits, fresh)
     if rc is not None:      # None: something to check, convert or complain about below
         _lib.check(rc, "append_kv_pair")
         return

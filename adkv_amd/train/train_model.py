@@ -90,6 +90,8 @@ def quant_f32_pair(x, params, lower_limit: int, upper_limit: int, sc_min: float,
     fp32 ``[B, C]`` tensors ``(zp, sc)`` updated in place, ``init`` optional ``[C]`` vectors ``(zp, sc)`` to
     start from instead.
     """
+    params, states = ([tuple(p) for p in pair] for pair in (params, states))      # read twice: they may be iterators
+    init = [tuple(p) for p in init] if init else None
     rc = _lib.host().quant_f32_pair(*x, *out, tuple(t for p in params for t in p), tuple(t for p in states for t in p),
                                     tuple(t for p in init for t in p) if init else None, lower_limit, upper_limit,
                                     float(sc_min), float(sc_max))

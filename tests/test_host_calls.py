@@ -30,6 +30,23 @@ def test_other_arguments_are_left_to_python():
     assert h.quant_f32(torch.zeros(1, 2, 128), p, -8, 7, 0.1, 2.0, False) is None
 
 
+def test_iterators_that_are_left_to_python_still_hold_their_tensors(monkeypatch):
+    """CPU tensors are refused by the device check, which sees every tensor of the call."""
+    from adkv_amd.train import train_model
+    seen = []
+    for m in (gemv, train_model):
+        monkeypatch.setattr(m, "_need_device", lambda *t: (seen.append(len(t)), gemv._chk(False, "no device"))[0])
+    p = synth.make_params(1, 128).astuple()
+    k, caches = torch.zeros(1, 1, 8, 128).half(), [synth.alloc_cache(1, 1, 8, 128, "cpu") for _ in range(2)]
+    with pytest.raises(RuntimeError, match="no device"):
+        gemv.append_kv_pair(*caches, k, k, iter(p), iter(p), 0, *[torch.zeros(1, 1, 128, 2).half() for _ in range(2)])
+    x, three, two = [torch.zeros(1, 8, 128)] * 2, [torch.ones(128)] * 3, [torch.zeros(1, 128)] * 2
+    twice = lambda t: iter([iter(t), iter(t)])
+    with pytest.raises(RuntimeError, match="no device"):
+        train_model.quant_f32_pair(x, twice(three), -8, 7, 0.1, 2.0, states=twice(two), out=x, init=twice([t[0] for t in two]))
+    assert seen == [16, 18]
+
+
 class _Count(TorchDispatchMode):
     seen = 0
 
