@@ -24,10 +24,10 @@ def test_other_arguments_are_left_to_python():
     assert h.rope_qk(x, x, x[0], x[0]) is None                                   # not on a device
     for args in ((), (x,), (1, 2, 3, 4), (x, x, None, None)):
         assert h.rope_qk(*args) is None
-    for f, n in ((h.decode, 14), (h.append, 14), (h.quant_f32, 7), (h.quant_f32_pair, 11)):
+    for f, n in ((h.decode, 14), (h.append, 14), (h.quant_f32, 8), (h.quant_f32_pair, 11)):
         assert f() is None and f(*[None] * n) is None and f(*[x] * n) is None and f(*[1 << 70] * n) is None
     p = tuple(torch.zeros(128) for _ in range(5))
-    assert h.quant_f32(torch.zeros(1, 2, 128), p, -8, 7, 0.1, 2.0, False) is None
+    assert h.quant_f32(torch.zeros(1, 2, 128), p, -8, 7, 0.1, 2.0, False, False) is None       # not on a device
 
 
 def test_iterators_that_are_left_to_python_still_hold_their_tensors(monkeypatch):
@@ -116,6 +116,21 @@ def test_fp32_quantiser_equals_the_python_function(gpu, monkeypatch, dtype, stat
     monkeypatch.setattr(_lib, "host", lambda: NOTHING)
     for p, q in zip(mine, f()):
         assert (p is None) == (q is None) and (p is None or torch.equal(p, q))
+
+
+@pytest.mark.gpu
+def test_fp32_calls_that_are_left_to_python(gpu):
+    """quant_f32 with all of its arguments: taken as it should be, refused for one of them at a time."""
+    h = _lib.host()
+    x = torch.randn(2, 5, 128, device=gpu)
+    p = tuple(torch.rand(128, device=gpu) * 0.1 + 0.05 for _ in range(5))
+    took = lambda x=x, p=p, lower=-8, upper=7, lo=0.1, hi=2.0, states=False, free=False: (
+        h.quant_f32(x, p, lower, upper, lo, hi, states, free) is not None)
+    assert took() and took(states=True) and took(free=True) and took(x=x.half()) and took(x=x.bfloat16())
+    assert not took(x=x.cpu()) and not took(x=x.double()) and not took(x=x[0]) and not took(x=x[:, ::2]) and not took(x=x[:0])
+    assert not took(x=x.as_subclass(_Sub)) and not took(p=p[:4]) and not took(p=list(p)) and not took(p=(p[0].half(), *p[1:]))
+    assert not took(p=(p[0][:64], *p[1:])) and not took(p=(p[0].cpu(), *p[1:])) and not took(lo=1) and not took(hi=None)
+    assert not took(lower=1 << 70) and not took(upper=1 << 40) and not took(lower=-(1 << 40)) and not took(lower=0.5)
 
 
 @pytest.mark.gpu
