@@ -97,11 +97,40 @@ def test_rows_that_a_buffer_descriptor_cannot_span(gpu, oracle, bits):
         assert np.array_equal(c.cpu().numpy(), want) and _same16(_np16(s), st)
 
 
+@pytest.mark.parametrize("bits", (4, 2))
+@pytest.mark.parametrize("mib", (10, 11, 12, 13))
+def test_checkpoints_of_pieces_that_start_inside_a_run(gpu, oracle, bits, mib):
+    """Rows 10 to 13 MiB apart: a piece of 2-bit codes is 96, 80 or 64 tokens, and checkpoints every 64 lie inside
+    the runs that such a piece counts from its own start."""
+    T, S, pitch = 300, 64, mib << 19
+    params = synth.make_params(1, D, bits=bits, seed=2).astuple()
+    x = torch.randn(1, 1, T, D, generator=torch.Generator().manual_seed(mib)).half()
+    big = torch.empty(T, pitch, dtype=torch.float16, device=gpu)
+    big[:, :D] = x[0, 0].to(gpu)
+    rows = big.as_strided((1, 1, T, D), (T * pitch, T * pitch, pitch, 1))
+    pg = tuple(t.to(gpu) for t in params)
+    caches = [synth.alloc_cache(1, 1, T + 16, D, gpu, bits=bits) for _ in range(2)]
+    states = [torch.zeros(1, 1, D, 2, dtype=torch.float16, device=gpu) for _ in range(2)]
+    cks = [torch.zeros(1, 1, T // S + 1, D, 2, dtype=torch.float16, device=gpu) for _ in range(2)]
+    gemv.append_kv_pair(*caches, rows, rows, pg, pg, 0, *states, k_ckpt=cks[0], v_ckpt=cks[1], ckpt_interval=S, bits=bits)
+    torch.cuda.synchronize()
+    pn, xn = [_np16(t) for t in params], _np16(x)
+    with oracle.code_bits(bits):
+        want = oracle.alloc_cache(1, 1, T + 16, D)
+        st = oracle.encode_kv_f16(want, xn, *pn)
+        at = [oracle.encode_kv_f16(oracle.alloc_cache(1, 1, (j + 1) * S, D), xn[:, :, :(j + 1) * S], *pn) for j in range(T // S)]
+    for c, s, k in zip(caches, states, cks):
+        assert np.array_equal(c.cpu().numpy(), want) and _same16(_np16(s), st)
+        for j, a in enumerate(at):
+            assert _same16(_np16(k[:, :, j]), a), j
+        assert not torch.any(k[:, :, T // S:])
+
+
 @pytest.mark.parametrize("form,T", [("one_channel", 8192), ("two_channels", 2048)])
 def test_one_bad_channel_does_not_stall_the_launch(gpu, form, T):
     """A channel with a zero scale sends its wave through the plain division for the whole stream, and the
-    launch waits for that wave: 2.2 times as long as without it (86 ns per token against 38, one channel per
-    lane), 3.8 times when every token waits for a load of its own."""
+    launch waits for that wave: some 2.4 times as long as without it (83 ns per token against 34, one channel per
+    lane).  When every token waits for a load of its own it is 3.8 times."""
     B, H = FORMS[form]
     params = [t.to(gpu) for t in synth.make_params(H, D, seed=2).astuple()]
     x = synth.make_k(B, H, T, D, dtype=torch.float16, device=gpu)
