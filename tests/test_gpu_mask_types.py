@@ -3,7 +3,7 @@ the same mask in fp32 gives, rows of odd lengths included."""
 import pytest
 import torch
 
-from adkv_amd import synth
+from adkv_amd import _lib, synth
 from adkv_amd.kernel import gemv
 
 pytestmark = pytest.mark.gpu
@@ -11,13 +11,13 @@ pytestmark = pytest.mark.gpu
 
 @pytest.mark.parametrize("mask_dtype", (torch.float16, torch.bfloat16, torch.float64))
 @pytest.mark.parametrize("per_head", (False, True))
-@pytest.mark.parametrize("B,Hq,H,T,S", [
-    (2, 3, 3, 0, 0), (2, 3, 3, 6, 256), (2, 3, 3, 530, 256),         # one launch
-    (2, 8, 2, 300, 256), (2, 8, 1, 1201, 256), (3, 4, 4, 777, 256),  # two launches
-    (2, 2, 2, 530, 64), (3, 32, 32, 1030, 64),                       # three: a wave per row
-    (1, 3, 3, 4096, 64), (2, 2, 2, 9001, 0),                         # a workgroup per row
-    (1, 2, 2, 30001, 0), (1, 2, 2, 61003, 64)])                      # rows in chunks
-def test_same_bits_as_fp32(gpu, mask_dtype, per_head, B, Hq, H, T, S):
+@pytest.mark.parametrize("launches,B,Hq,H,T,S", [
+    (1, 2, 3, 3, 0, 0), (1, 2, 3, 3, 6, 256), (1, 2, 3, 3, 530, 256), (1, 3, 4, 4, 777, 256),
+    (2, 2, 8, 2, 300, 256), (2, 2, 8, 1, 1201, 256), (2, 3, 4, 4, 1777, 256),
+    (3, 2, 2, 2, 530, 64), (3, 3, 32, 32, 1030, 64),                 # a wave per row
+    (3, 1, 3, 3, 4096, 64), (3, 2, 2, 2, 9001, 0),                   # a workgroup per row
+    (3, 1, 2, 2, 30001, 0), (3, 1, 2, 2, 61003, 64)])                # rows in chunks
+def test_same_bits_as_fp32(gpu, mask_dtype, per_head, launches, B, Hq, H, T, S):
     D, n = 128, T + 1
     g = torch.Generator().manual_seed(T)
     kp, vp = ([t.to(gpu) for t in synth.make_params(H, D, seed=i).astuple()] for i in (3, 4))
@@ -33,6 +33,7 @@ def test_same_bits_as_fp32(gpu, mask_dtype, per_head, B, Hq, H, T, S):
     mask[0, :, :, : n // 3] = torch.finfo(torch.float16).min
     mask[-1, :, :, n - 1 - n // 5:n - 1] = -float("inf")
     mask = mask.to(mask_dtype).to(gpu)
+    assert _lib.lib().adkv_decode_step_launches(B, Hq, H, T, D, 4, cks[0].shape[2] if S else 0, S, 1) == launches
     got = []
     for m in (mask, mask.float()):
         c = [t.clone() for t in caches]

@@ -1,19 +1,20 @@
 """adkv_decode_step in two launches (every segment through keys, softmax and values, then the segments put
-together) against the three calls that it stands for: every shape of its kernel, ragged and one-token last
-segments, masks that leave a segment or a row nothing, non-finite logits."""
+together) against the three calls that it stands for and against 64 bits: every shape of its kernel, ragged and
+one-token last segments, masks that leave a segment or a row nothing, non-finite logits."""
 import math
 
+import numpy as np
 import pytest
 import torch
 
-from adkv_amd import synth
+from adkv_amd import _lib, synth
 from adkv_amd.kernel import gemv
 
 pytestmark = pytest.mark.gpu
 SMIN, SMAX = math.exp(-4.0), math.exp(4.0)
 
 
-def _case(gpu, B, Hq, H, D, T, bits=4, S=256, dtype=torch.float16, mask=None, scaling=None, q_scale=1.0):
+def _case(gpu, B, Hq, H, D, T, bits=4, S=256, dtype=torch.float16, mask=None, scaling=None, q_scale=1.0, more=None):
     g = torch.Generator(device=gpu).manual_seed(T + Hq)
     kp, vp = ([t.to(gpu) for t in synth.make_params(H, D, bits=bits, seed=i).astuple()] for i in (3, 4))
     tps = 32 // bits
@@ -29,6 +30,7 @@ def _case(gpu, B, Hq, H, D, T, bits=4, S=256, dtype=torch.float16, mask=None, sc
                             ckpt_interval=S, bits=bits)
     c2, ck2 = [c.clone() for c in caches], [c.clone() if S else None for c in cks]
     scaling = D ** -0.5 if scaling is None else scaling
+    assert _lib.lib().adkv_decode_step_launches(B, Hq, H, T, D, bits, cks[0].shape[2] if S else 0, S, mask is not None) == 2
     out, w = gemv.decode_step(q, *caches, kn, vn, kp, vp, T, scaling, mask, k_ckpt=cks[0], v_ckpt=cks[1], ckpt_interval=S, bits=bits)
     logits = gemv.forward_qk(q.half(), c2[0], kn.half(), *kp, T, SMIN, SMAX, ckpt=ck2[0], ckpt_interval=S, bits=bits)
     w_want = gemv.softmax_scale_mask(logits, scaling, mask)
@@ -38,7 +40,17 @@ def _case(gpu, B, Hq, H, D, T, bits=4, S=256, dtype=torch.float16, mask=None, sc
         assert torch.equal(a, b)
     for a, b in zip(cks, ck2):
         assert not S or torch.equal(a.view(torch.int16), b.view(torch.int16))
+    if more is not None:
+        more.update(q=q.half(), caches=caches, params=(kp, vp))
     return out.float(), w.float(), o_want.float(), w_want.float()
+
+
+def _replayed(oracle, cache, params, bits, n, heads):
+    """float64 [len(heads), n, D]: the oracle's values of `n` tokens of these (sequence, head)s."""
+    np16 = lambda t: t.detach().cpu().contiguous().view(torch.int16).numpy().view(np.float16)
+    with oracle.code_bits(bits):
+        return torch.stack([torch.from_numpy(oracle.replay_f16(
+            cache[b:b + 1, h:h + 1].cpu().numpy(), *[np16(p[h:h + 1]) for p in params], n)[0][0, 0]).double() for b, h in heads])
 
 
 def _compare(out, w, o_want, w_want, bf16=False):
@@ -59,8 +71,38 @@ def _compare(out, w, o_want, w_want, bf16=False):
     (1, 1, 1, 512, 519, 4, 0), (2, 3, 3, 512, 770, 4, 256), (9, 8, 8, 512, 1790, 4, 256),
 ])
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
-def test_against_the_three_calls(gpu, B, Hq, H, D, T, bits, S, dtype):
-    _compare(*_case(gpu, B, Hq, H, D, T, bits, S, dtype), bf16=dtype == torch.bfloat16)
+def test_against_the_three_calls(gpu, oracle, B, Hq, H, D, T, bits, S, dtype):
+    more = {}
+    out, w, o_want, w_want = _case(gpu, B, Hq, H, D, T, bits, S, dtype, more=more)
+    _compare(out, w, o_want, w_want, bf16=dtype == torch.bfloat16)
+    # The outputs are sums over the returned weights, up to roundings that know nothing of each other: of the weights
+    # there and here (2^-12 of each at most, or 2^-25 below 2^-14: a variance of a third of the square) and of
+    # the output.  Seven deviations of the sum; a token left out is tens of them.
+    heads = sorted({(0, 0), (B - 1, H - 1)})
+    v = _replayed(oracle, more["caches"][1], more["params"][1], bits, T + 1, heads)
+    rows = lambda t: torch.stack([t[b, h * (Hq // H):(h + 1) * (Hq // H)] for b, h in heads]).double().cpu()
+    w, out = rows(w), rows(out)
+    sigma = torch.sqrt(2 / 3 * (torch.clamp(w * 2.0 ** -11, min=2.0 ** -25) ** 2) @ v ** 2)
+    tol = 7 * sigma + (2.0 ** -8 if dtype == torch.bfloat16 else 2.0 ** -11) * (w @ v).abs() + 2.0 ** -25
+    err = (out - w @ v).abs()
+    assert torch.all(err <= tol), (err / tol).max()
+
+
+@pytest.mark.parametrize("B,Hq,H,D,T,bits", [(24, 16, 2, 128, 700, 4), (24, 8, 2, 128, 2063, 2), (12, 8, 8, 256, 1290, 4),
+                                             (13, 32, 32, 128, 1100, 4)])
+@pytest.mark.parametrize("q_scale", [0.3, 1.0])
+def test_error_against_64_bits(gpu, oracle, B, Hq, H, D, T, bits, q_scale):
+    """Outputs are no further from softmax and sum in 64 bits over the cache's values than those of the three
+    calls: both round a logit and a weight to fp16, by independent amounts; 5 % covers the chance in 10^5 outputs."""
+    more = {}
+    out, _, o_want, _ = _case(gpu, B, Hq, H, D, T, bits, q_scale=q_scale, more=more)
+    heads = [(b, h) for b in range(B) for h in range(0, H, max(1, H // 4))]
+    k, v = (_replayed(oracle, c, p, bits, T + 1, heads) for c, p in zip(more["caches"], more["params"]))
+    rows = lambda t: torch.stack([t[b, h * (Hq // H):(h + 1) * (Hq // H)] for b, h in heads]).double().cpu()
+    want = torch.softmax(rows(more["q"][:, :, 0]) @ k.transpose(1, 2).contiguous() * D ** -0.5, -1) @ v
+    rms = [float(((rows(o) - want) ** 2).mean().sqrt()) for o in (out, o_want)]
+    print(f"rms error {rms[0]:.3e}, of the three calls {rms[1]:.3e}, of a value of {float((want ** 2).mean().sqrt()):.3e}")
+    assert rms[0] <= 1.05 * rms[1]
 
 
 @pytest.mark.parametrize("low", [torch.finfo(torch.float32).min, torch.finfo(torch.bfloat16).min, -math.inf])
