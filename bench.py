@@ -550,8 +550,9 @@ def decode_record(args, B, Hq, H, D, T, bits, S, NL, steps, warmup, headline=Tru
     if fused_ms is not None:
         res["one_launch_step"] = {"ms_per_step": fused_ms, "tokens_per_s": B / (N_LAYERS_MODEL * fused_ms * 1e-3),
                                   "note": "adkv_decode_step with adkv_set_fused_step(1): forward_qk, softmax and forward_ov "
-                                          "in one launch (decode_ft_kernel), no stage events; the default three launches "
-                                          "are the headline"}
+                                          "in one launch (decode_ft_kernel), no stage events, timed after the default three "
+                                          "launches, which are the headline, on a device that has come up to its clock "
+                                          "since (in turn with them it is the slower one)"}
     if graph_ms is not None:
         res["graph_replay"] = {"ms_per_step": graph_ms, "tokens_per_s": B / (N_LAYERS_MODEL * graph_ms * 1e-3),
                                "note": "the same decode_step step captured once per layer cache and replayed"}
