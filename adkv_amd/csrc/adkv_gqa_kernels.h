@@ -152,9 +152,9 @@ __device__ __forceinline__ uint32_t table_lane_offset(int lane)
 }
 
 // forward_qk of one segment, two channels per lane: a KV head fills the wave (see PairScores).
-template <int BITS, int GQ>
-__device__ __forceinline__ void qk_gqa_pair_segment(const uint2 *lut, int lane, int bx, PairScores<BITS, GQ> &scores,
-                                                    SegLoads<GQA_D, 2, BITS, PairScores<BITS, GQ>::AHEAD> &s,
+template <int BITS, int GQ, bool LONE>
+__device__ __forceinline__ void qk_gqa_pair_segment(const uint2 *lut, int lane, int bx, PairScores<BITS, GQ, LONE> &scores,
+                                                    SegLoads<GQA_D, 2, BITS, PairScores<BITS, GQ, LONE>::AHEAD> &s,
                                                     const h1 *k_new, h1 *out, int T, h1 *state_out, const Seg &sa)
 {
     constexpr int D = GQA_D, CPL = 2, TPW = Code<BITS>::TPW;
@@ -207,9 +207,10 @@ __global__ __launch_bounds__(BLK) void qk_gqa_kernel(
         sa.groups = 0; // only even plans come here
         __shared__ uint2 smem[LUT_WORDS64 + (BLK / 64) * PAIR_TILE / 8];
         const Unit<GQA_D, 2, BLK> un(BH, sa.nseg);
-        PairScores<BITS, GQ> scores(reinterpret_cast<char *>(smem + LUT_WORDS64) + (threadIdx.x >> 6) * PAIR_TILE, un.lh,
-                                    q + (size_t)un.bx * GQ * GQA_D);
-        SegLoads<GQA_D, 2, BITS, PairScores<BITS, GQ>::AHEAD> s;
+        using Scores = PairScores<BITS, GQ, BLK == 256>;
+        Scores scores(reinterpret_cast<char *>(smem + LUT_WORDS64) + (threadIdx.x >> 6) * PAIR_TILE, un.lh,
+                      q + (size_t)un.bx * GQ * GQA_D);
+        SegLoads<GQA_D, 2, BITS, Scores::AHEAD> s;
         s.start(cache, zp, sc, al, be, tg, un.bx % H, un.bx, un.lh, un.seg, T, n_super_cap, sa);
         fill_table<BITS, BLK>(smem, threadIdx.x);
         __syncthreads();

@@ -1083,7 +1083,9 @@ constexpr int PAIR_TILE = 16 * 256; // bytes of a wave's key tile
 // 38 -> 32).
 // The tile: row t = token t, 256 bytes; its 16-byte pieces are permuted by (t / 2) % 8 so that
 // both halves of an access to 16 rows at once spread over the banks.
-template <int BITS, int GQ>
+// LONE: workgroups of 256 threads, a wave with a SIMD's registers to itself; the compiler keeps products in
+// accumulation registers there and in vector registers elsewhere.
+template <int BITS, int GQ, bool LONE>
 struct PairScores {
     using G = Geo<128, 2>;
     using Vec = G::Vec;
@@ -1147,8 +1149,13 @@ struct PairScores {
     {
         // All of d is held up to here: registers of it that nobody reads would go to the hand-laid block behind
         // multiply() while the matrix cores have yet to write them, and the compiler waits for no block.  (With 2-bit
-        // codes the block wrote one of them an instruction later; at two waves per SIMD its value was lost.)
-        asm volatile("" ::"v"(d));
+        // codes the block wrote one of them an instruction later; at two waves per SIMD its value was lost.)  In the
+        // registers where it is: moved into the others, it took a lone wave 12 instructions per 64 tokens (1 x 32 heads x
+        // 603 tokens with the rotary embedding 21.19 us, 21.08 where they are).
+        if constexpr (LONE)
+            asm volatile("" ::"a"(d));
+        else
+            asm volatile("" ::"v"(d));
         const int t = lane & 15, quarter = lane >> 4;
         if (t >= ntok || (GQ == 1 && quarter) || (GQ == 2 && (quarter & 1)))
             return;
@@ -1242,9 +1249,9 @@ struct PairScores {
 
 // forward_qk of one (head, segment), from the loads that s.start() and the caller have sent off.
 // Writes the segment's logits to out + bx * row_pitch and, with the context's last segment, appends.
-template <int D, int CPL>
+template <int D, int CPL, bool LONE>
 __device__ __forceinline__ void qk_segment(const uint2 *lut, uint32_t lane_copy, int lane, int bx, int lh, int c0, bool active,
-                                           PairScores<4, 1> &scores, SegLoads<D, CPL, 4, CPL == 2 ? PF_PAIR : PF> &s,
+                                           PairScores<4, 1, LONE> &scores, SegLoads<D, CPL, 4, CPL == 2 ? PF_PAIR : PF> &s,
                                            const uint32_t *qw, const h1 *k_new, h1 *out, int T, h1 *state_out, const Seg &sa)
 {
     using G = Geo<D, CPL>;
@@ -1411,7 +1418,7 @@ __global__ __launch_bounds__(BLK) void qk_kernel(
     const bool active = un.active;
     uint32_t qw[G::NP];
     __builtin_memcpy(qw, q + (size_t)bx * D + c0, 2 * CPL);
-    PairScores<4, 1> scores(reinterpret_cast<char *>(smem + LUT_WORDS64) + (threadIdx.x >> 6) * PAIR_TILE, lane,
+    PairScores<4, 1, BLK == 256> scores(reinterpret_cast<char *>(smem + LUT_WORDS64) + (threadIdx.x >> 6) * PAIR_TILE, lane,
                             q + (size_t)bx * D); // two channels per lane only
     SegLoads<D, CPL, 4, PAIR ? PF_PAIR : PF> s;
     s.start(cache, zp, sc, al, be, tg, bx % H, bx, lh, un.seg, T, n_super_cap, sa);

@@ -169,8 +169,9 @@ __global__ __launch_bounds__(BLK) void step_segments_kernel(
 
     uint32_t qw[G::NP];
     __builtin_memcpy(qw, q + (size_t)bx * GQ * D + c0, 2 * CPL);
-    PairScores<BITS, GQ> scores(slot, lane, q + (size_t)bx * GQ * D); // two channels per lane only
-    SegLoads<D, CPL, BITS, PAIR ? PairScores<BITS, GQ>::AHEAD : PF> s;
+    using Scores = PairScores<BITS, GQ, BLK == 256>;
+    Scores scores(slot, lane, q + (size_t)bx * GQ * D); // two channels per lane only
+    SegLoads<D, CPL, BITS, PAIR ? Scores::AHEAD : PF> s;
     s.start(k_cache, kp.zp, kp.sc, kp.al, kp.be, kp.tg, h, bx, lh, un.seg, T, n_super_cap, ka);
     fill_table<BITS, BLK>(lut, threadIdx.x);
     __syncthreads();

@@ -34,7 +34,7 @@ __global__ __launch_bounds__(256) void small_step_kernel(
     const int bx = blockIdx.x, h = bx % H, c0 = lane * 2, n = T + 1;
     const bool works = seg < ka.nseg;
     const uint32_t lane_copy = (uint32_t)(lane & (LUT_COPIES - 1)) * 8u;
-    PairScores<4, 1> scores(tile, lane, q + (size_t)bx * D);
+    PairScores<4, 1, true> scores(tile, lane, q + (size_t)bx * D);
     SegLoads<D, CPL, 4, PF_PAIR> s;
     s.start(k_cache, kp.zp, kp.sc, kp.al, kp.be, kp.tg, h, bx, lane, works ? seg : 0, T, n_super_cap, ka);
     const bool last = works && s.last;
