@@ -1583,7 +1583,9 @@ __device__ __forceinline__ void ov_segment(const uint2 *lut, uint32_t lane_copy,
 // forward_ov by itself keeps its loads behind the table and the loop to itself: built from ov_segment with the loads
 // on their way meanwhile it was 0.5 to 1 us longer in launches of few waves (1 x 32 heads x 256 tokens 9.4 / 10.4 us)
 // and 3 to 8 % in long ones of wide heads (4 x 8 heads of 256 channels x 5000 tokens, no checkpoints, 188 / 202 us): the
-// compiler orders and waits otherwise.
+// compiler orders and waits otherwise.  (One wave per SIMD and more of 1024 tokens are the other way round by less: 32 x 32
+// 28.8 / 28.6 us, 60 x 32 42.2 / 41.7.)  The loads ahead of the table in the order of the loop were slower throughout:
+// 1 x 32 x 256 10.4 us, 32 x 32 x 1024 29.5, 16 x 32 x 1500 40.6 instead of 38.9.
 template <int D, int CPL, int BLK>
 __global__ __launch_bounds__(BLK) void ov_kernel(
     const h1 *__restrict__ attn, uint4 *__restrict__ cache, const h1 *__restrict__ v_new,
