@@ -1,9 +1,10 @@
 """The device code of the library as built.
 
-Registers that a matrix instruction still has to write are left alone until it has: the hardware does not hold back a vector instruction that reads or overwrites such a register; the compiler keeps
-the distance between its own instructions, but not to a hand-laid block, and it hands registers of a result that
-nobody reads to the next block at once: what the block has left there is then overwritten behind its back, now
-and then, as the waves of a SIMD happen to interleave.
+Registers that a matrix instruction still has to write are left alone until it has: the hardware does not hold back a
+vector instruction that reads or overwrites such a register; the compiler keeps the distance between its own
+instructions, but not to a hand-laid block, and it hands registers of a result that nobody reads to the next block at
+once: what the block has left there is then overwritten behind its back, now and then, as the waves of a SIMD happen
+to interleave.
 
 Kernels that live from the number of their waves leave room for them, and those that live from their loads in flight
 do not wait for the youngest of them."""
