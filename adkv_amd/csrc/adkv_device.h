@@ -235,6 +235,102 @@ __device__ __forceinline__ void replay_eight_weighted(Pair &p, const uint2 *e, c
 #undef ADKV_REPLAY_F
 #undef ADKV_REPLAY_TOKEN
 
+// ---------------------------------------------------------------------------------------------
+// One channel per lane: both halves of the packed instructions work for the same channel.  The table is indexed by a
+// byte of the channel's word as it is (two tokens, the earlier one in the low nibble) and returns (q, |q|) of each, so
+// no bytes are merged and one LDS read serves two tokens.  With f = be*|q| + omt beside q, one packed multiply gives the
+// code's value q*sc and the next scale sc*f, and one packed fma by (al, 1) the next zero-point and the token's
+// value: three packed instructions per token and channel, the arithmetic of update_pair bit for bit (a product by one
+// and a sum with zero are exact).
+// ---------------------------------------------------------------------------------------------
+struct Lone {
+    uint32_t z;  // low half: the zero-point; high half: the last token's value
+    uint32_t r;  // high half: the scale; low half: the last token's q*sc
+    uint32_t ca; // (al, 1)
+    uint32_t cf; // (1, be)
+    uint32_t c0; // (0, omt)
+};
+__device__ __forceinline__ h1 lone_zp(const Lone &s) { return as_h2(s.z).x; }
+__device__ __forceinline__ h1 lone_sc(const Lone &s) { return as_h2(s.r).y; }
+
+template <int NT>
+__device__ __forceinline__ void lone_fill(uint2 *lut, int tid)
+{
+    static_assert(NT % 256 == 0, "whole groups of 256 entries' 16 lanes");
+    uint4 *l4 = reinterpret_cast<uint4 *>(lut);
+    const h1 lo = (h1)(((tid >> 4) & 15) - 8);
+    const uint32_t x = as_u32(splat(lo)) & 0x7FFFFFFFu;
+#pragma unroll
+    for (int i = 0; i < LUT_WORDS64 / 2; i += NT) {
+        if (LUT_WORDS64 / 2 % NT != 0 && i + tid >= LUT_WORDS64 / 2)
+            break;
+        const uint32_t y = as_u32(splat((h1)(((i + tid) >> 8) - 8))) & 0x7FFFFFFFu;
+        l4[i + tid] = make_uint4(x, y, x, y);
+    }
+}
+
+// Eight tokens, entries e[0..3] of two tokens each; x[k] = the values of tokens 2k and 2k + 1.  As in replay_eight no
+// packed result is read by the very next instruction.
+#define ADKV_LONE_F(E) "v_pk_fma_f16 %[f], " E ", %[cf], %[c0]\n\t"
+#define ADKV_LONE_R "v_pk_mul_f16 %[r], %[f], %[r] op_sel:[0,1] op_sel_hi:[1,1]\n\t"
+#define ADKV_LONE_Z(TO, FROM) "v_pk_fma_f16 " TO ", %[r], %[ca], " FROM " op_sel_hi:[0,1,0]\n\t"
+#define ADKV_LONE_P(X) "v_perm_b32 " X ", %[z], " X ", %[hi]\n\t"
+__device__ __forceinline__ void lone_eight(Lone &s, const uint2 *e, uint32_t *x)
+{
+    uint32_t f;
+    asm(ADKV_LONE_F("%[a0]") "s_nop 0\n\t"
+        ADKV_LONE_R ADKV_LONE_F("%[b0]") ADKV_LONE_Z("%[x0]", "%[z]")
+        ADKV_LONE_R ADKV_LONE_F("%[a1]") ADKV_LONE_Z("%[z]", "%[x0]")
+        ADKV_LONE_R ADKV_LONE_F("%[b1]") ADKV_LONE_Z("%[x1]", "%[z]")
+        ADKV_LONE_R ADKV_LONE_F("%[a2]") ADKV_LONE_P("%[x0]") ADKV_LONE_Z("%[z]", "%[x1]")
+        ADKV_LONE_R ADKV_LONE_F("%[b2]") ADKV_LONE_Z("%[x2]", "%[z]")
+        ADKV_LONE_R ADKV_LONE_F("%[a3]") ADKV_LONE_P("%[x1]") ADKV_LONE_Z("%[z]", "%[x2]")
+        ADKV_LONE_R ADKV_LONE_F("%[b3]") ADKV_LONE_Z("%[x3]", "%[z]")
+        ADKV_LONE_R ADKV_LONE_P("%[x2]") ADKV_LONE_Z("%[z]", "%[x3]")
+        "s_nop 0\n\t" ADKV_LONE_P("%[x3]")
+        : [z] "+v"(s.z), [r] "+v"(s.r), [f] "=&v"(f), [x0] "=&v"(x[0]), [x1] "=&v"(x[1]), [x2] "=&v"(x[2]), [x3] "=&v"(x[3])
+        : [a0] "v"(e[0].x), [b0] "v"(e[0].y), [a1] "v"(e[1].x), [b1] "v"(e[1].y), [a2] "v"(e[2].x), [b2] "v"(e[2].y),
+          [a3] "v"(e[3].x), [b3] "v"(e[3].y), [ca] "v"(s.ca), [cf] "v"(s.cf), [c0] "v"(s.c0), [hi] "s"(0x07060302u));
+}
+// The same, each value multiplied by its token's weight (two per word of w) and added to acc in fp32.
+#define ADKV_LONE_M(W, HI) "v_fma_mix_f32 %[c], " W ", %[z], %[c] op_sel:[" HI ",1,0] op_sel_hi:[1,1,0]\n\t"
+#define ADKV_LONE_TOKEN(NEXT, ADD) ADKV_LONE_R NEXT ADD ADKV_LONE_Z("%[z]", "%[z]")
+__device__ __forceinline__ void lone_eight_weighted(Lone &s, const uint2 *e, const uint4 &w, float &acc)
+{
+    uint32_t f;
+    asm(ADKV_LONE_F("%[a0]") "s_nop 0\n\t"
+        ADKV_LONE_TOKEN(ADKV_LONE_F("%[b0]"), "")
+        ADKV_LONE_TOKEN(ADKV_LONE_F("%[a1]"), ADKV_LONE_M("%[w0]", "0"))
+        ADKV_LONE_TOKEN(ADKV_LONE_F("%[b1]"), ADKV_LONE_M("%[w0]", "1"))
+        ADKV_LONE_TOKEN(ADKV_LONE_F("%[a2]"), ADKV_LONE_M("%[w1]", "0"))
+        ADKV_LONE_TOKEN(ADKV_LONE_F("%[b2]"), ADKV_LONE_M("%[w1]", "1"))
+        ADKV_LONE_TOKEN(ADKV_LONE_F("%[a3]"), ADKV_LONE_M("%[w2]", "0"))
+        ADKV_LONE_TOKEN(ADKV_LONE_F("%[b3]"), ADKV_LONE_M("%[w2]", "1"))
+        ADKV_LONE_TOKEN("", ADKV_LONE_M("%[w3]", "0"))
+        "s_nop 0\n\t" ADKV_LONE_M("%[w3]", "1")
+        : [z] "+v"(s.z), [r] "+v"(s.r), [f] "=&v"(f), [c] "+v"(acc)
+        : [a0] "v"(e[0].x), [b0] "v"(e[0].y), [a1] "v"(e[1].x), [b1] "v"(e[1].y), [a2] "v"(e[2].x), [b2] "v"(e[2].y),
+          [a3] "v"(e[3].x), [b3] "v"(e[3].y), [w0] "v"(w.x), [w1] "v"(w.y), [w2] "v"(w.z), [w3] "v"(w.w), [ca] "v"(s.ca),
+          [cf] "v"(s.cf), [c0] "v"(s.c0));
+}
+#undef ADKV_LONE_TOKEN
+#undef ADKV_LONE_M
+#undef ADKV_LONE_P
+#undef ADKV_LONE_Z
+#undef ADKV_LONE_R
+#undef ADKV_LONE_F
+
+// One token with code q (ragged tails): returns its value.
+__device__ __forceinline__ h1 lone_token(Lone &s, int q)
+{
+    const h1 qh = (h1)q, qs = qh * lone_sc(s), v = qs + lone_zp(s);
+    const h1 f = __builtin_fmaf16(as_h2(s.cf).y, (h1)(q < 0 ? -q : q), as_h2(s.c0).y);
+    const h1 zp = __builtin_fmaf16(as_h2(s.ca).x, qs, lone_zp(s)), sc = lone_sc(s) * f;
+    s.z = as_u32((h2){zp, v});
+    s.r = as_u32((h2){qs, sc});
+    return v;
+}
+
 // Code width.  4 bits is the reference's format (8 tokens per 32-bit channel word, codes in
 // [-8, 7], stored as q + 8).  2 bits is the same recurrence over codes in [-2, 1] (the range the
 // reference's train model uses for bits = 2, train_model.py:96-97), stored as q + 2, 16 tokens per

@@ -2325,6 +2325,7 @@ static inline int lanes_per_head(int D) { return D == 128 ? 32 : 64; }
 
 #include "adkv_gqa_kernels.h"
 #include "adkv_ft_kernels.h"
+#include "adkv_lone.h"
 #include "adkv_small_step.h"
 #include "adkv_segment_step.h"
 
@@ -2473,6 +2474,30 @@ static int threads_per_workgroup(long threads)
         break;                                        \
     }                                                 \
     }
+
+// Head dim 128 in launches that leave SIMDs empty: one channel per lane, a head over two waves (adkv_lone.h), as long as
+// two channels per lane would leave at most two waves on a SIMD (forward_ov: four of these) or one and a half
+// (forward_qk, whose keys take more of the LDS: with four waves it is the two-channel form's equal).  us, two channels per
+// lane / one, 32 heads, no checkpoints: 1 x 1024 tokens qk 29.5 / 19.3, ov 28.8 / 14.9, 16 x 1024 30.2 / 20.9 and 28.0 / 16.6,
+// 32 x 1024 30.7 / 29.0 and 28.3 / 24.7, 48 x 1024 45.2 / 37.7 and 44.3 / 33.5, 48 x 200 12.3 / 10.6 and 12.5 / 9.0, 64 x 1024
+// 48.9 / 48.6 and 47.5 / 43.0, 64 x 200 12.7 / 12.9 and 12.7 / 10.9; every 256: 1 x 4096 10.4 / 8.1 and 12.4 / 8.3, 2 x 8192
+// 15.3 / 15.0 and 17.8 / 15.1.
+// A buffer descriptor holds a segment's codes: rows of 2^24 tokens and more stay with the other kernels.
+static bool qk_lone(int BH, int nseg, int T) { return 2 * padded_units<64>(BH, nseg) <= 3L * n_simd() && T < 1 << 24; }
+static bool ov_lone(int BH, int nseg, int T) { return padded_units<64>(BH, nseg) <= 2L * n_simd() && T < 1 << 24; }
+#define ADKV_LAUNCH_LONE_(KERNEL, BLK, ...) \
+    hipLaunchKernelGGL(KERNEL<BLK>, dim3((unsigned)((threads + (BLK)-1) / (BLK))), dim3(BLK), 0, st, __VA_ARGS__)
+#define ADKV_LAUNCH_LONE(KERNEL, ...)                                  \
+    do {                                                               \
+        const long threads = padded_units<64>(BH, seg.nseg) * 128;     \
+        const int blk = threads_per_workgroup(threads);                \
+        if (blk == 1024)                                               \
+            ADKV_LAUNCH_LONE_(KERNEL, 1024, __VA_ARGS__);              \
+        else if (blk == 768)                                           \
+            ADKV_LAUNCH_LONE_(KERNEL, 768, __VA_ARGS__);               \
+        else                                                           \
+            ADKV_LAUNCH_LONE_(KERNEL, 256, __VA_ARGS__);               \
+    } while (0)
 
 // Matrix-core kernels (head dim 128), four channels per lane: 12- or 16-wave workgroups by the same
 // rule.  Eight query heads per KV head need ~138 registers per lane, more than the 128 a 16-wave
@@ -2830,12 +2855,11 @@ static int fused_step_plan(Seg &ka, Seg &va, int B, int Hq, int H, int T, int D,
     return lanes;
 }
 
-// Whether a step runs as small_step_kernel, and its plan: a workgroup per (sequence, head), one per CU, a
-// wave per segment.  us per step on the device, three or four launches /
-// one, sequences x heads x tokens: 1 x 32 x 603 25.6 / 20.3 (and 15 us of host time / 5), 8 x 32 x 1000
-// 27.7 / 22.4, 4 x 32 x 200 20.4 / 18.1, 2 x 8 x 64 12.8 / 11.4.  With five to eight segments two waves
-// share a SIMD while other CUs idle, and beyond one workgroup per CU (its LDS allows no second) a launch
-// takes two rounds: those stay with the separate launches.
+// Whether a step runs as small_step_kernel, and its plan: a workgroup per (sequence, head), one per CU, two
+// waves per segment.  us per step on the device, three or four launches / one, sequences x heads x tokens: 1 x 32 x 603
+// 25.6 / 13.2 (and 15 us of host time / 5), 8 x 32 x 1000 27.7 / 20.0, 4 x 32 x 200 20.4 / 12.8, 2 x 8 x 64 12.8 / 8.8.
+// With five to eight segments four waves share a SIMD while other CUs idle, and beyond one workgroup per CU (its LDS
+// allows no second) a launch takes two rounds: those stay with the separate launches.
 static bool small_step_plan(Seg &seg, int B, int Hq, int H, int T, int D, int bits, void *k_ckpt, void *v_ckpt,
                             int n_ckpt_cap, int ckpt_interval)
 {
@@ -3346,6 +3370,8 @@ static const char *decode_kernel_name(int B, int Hq, int H, int T, int D, int bi
     }
     if (D == 128) {
         const long units = padded_units<32>(B * H, seg.nseg);
+        if (qk_lone(B * H, seg.nseg, T))
+            return "lone_kernel (shared table, one channel per lane)";
         if (units / 2 <= n_simd())
             return "kernel<128,2,256> (shared table, two channels per lane)";
         const int blk = threads_per_workgroup(units * 32);
@@ -3407,6 +3433,12 @@ static int forward_qk_impl(const void *q, void *k_cache, const void *k_new, void
                            (const h1 *)q, (uint4 *)k_cache, (const h1 *)k_new, (h1 *)logits,
                            (const h1 *)zp, (const h1 *)sc, (const h1 *)alpha, (const h1 *)beta,
                            (const h1 *)tgt, B, H, T, n_super_cap, (h1 *)state_out, seg);
+        return check_launch();
+    }
+    if (D == 128 && qk_lone(BH, seg.nseg, T)) {
+        const FtParams p = {(const h1 *)zp, (const h1 *)sc, (const h1 *)alpha, (const h1 *)beta, (const h1 *)tgt};
+        ADKV_LAUNCH_LONE(qk_lone_kernel, (const h1 *)q,
+                           (uint4 *)k_cache, (const h1 *)k_new, (h1 *)logits, p, BH, H, T, n_super_cap, (h1 *)state_out, seg);
         return check_launch();
     }
     ADKV_DISPATCH_D(qk_kernel, (const h1 *)q, (uint4 *)k_cache, (const h1 *)k_new, (h1 *)logits,
@@ -3576,6 +3608,11 @@ static int forward_ov_impl(const void *attn, void *v_cache, const void *v_new, v
                            dim3(FT_BLK), 0, st, (const h1 *)attn, (uint4 *)v_cache, (const h1 *)v_new, (h1 *)out,
                            (float *)workspace, (const h1 *)zp, (const h1 *)sc, (const h1 *)alpha,
                            (const h1 *)beta, (const h1 *)tgt, B, H, T, n_super_cap, (h1 *)state_out, seg);
+    } else if (D == 128 && ov_lone(BH, seg.nseg, T)) {
+        const FtParams p = {(const h1 *)zp, (const h1 *)sc, (const h1 *)alpha, (const h1 *)beta, (const h1 *)tgt};
+        ADKV_LAUNCH_LONE(ov_lone_kernel, (const h1 *)attn,
+                           (uint4 *)v_cache, (const h1 *)v_new, (h1 *)out, (float *)workspace, p, BH, H, T, n_super_cap,
+                           (h1 *)state_out, seg);
     } else {
         ADKV_DISPATCH_D(ov_kernel, (const h1 *)attn, (uint4 *)v_cache, (const h1 *)v_new, (h1 *)out,
                         (float *)workspace, (const h1 *)zp, (const h1 *)sc, (const h1 *)alpha,
@@ -3909,7 +3946,7 @@ int adkv_decode_step(const void *q, void *k_cache, void *v_cache, const void *k_
             Seg va = ka;
             va.ckpt = (h1 *)v_ckpt;
             const FtParams kp = ft_params(k_params), vp = ft_params(v_params);
-            hipLaunchKernelGGL(small_step_kernel, dim3((unsigned)(B * H)), dim3(256), 0, (hipStream_t)stream, (const h1 *)q,
+            hipLaunchKernelGGL(small_step_kernel, dim3((unsigned)(B * H)), dim3(512), 0, (hipStream_t)stream, (const h1 *)q,
                                (uint4 *)k_cache, (const h1 *)k_new, (uint4 *)v_cache, (const h1 *)v_new, mk, (h1 *)weights, (h1 *)out, kp, vp, H, T,
                                n_super_cap, scaling, ka, va);
             return (rc = check_launch()) ? rc : mark_one_launch(stream);

@@ -1,0 +1,405 @@
+// forward_qk and forward_ov of launches that leave SIMDs empty: head dim 128, 4-bit codes, one query head per KV
+// head, one channel per lane, a head over two waves.  Included by adkv_kernels.hip after the shared device helpers.
+//
+// Such a launch takes as long as one wave's instructions per token: a wave alone on its SIMD issues one every four
+// or five cycles, LDS reads twelve, whatever the other lanes do.  With two channels per lane that is a lookup and
+// five packed instructions per token, nine with the outputs'; with one (lone_eight) half a lookup and three,
+// four with them, and twice the waves.
+#pragma once
+
+namespace adkv {
+
+constexpr int LONE_PF = 8;          // supergroups of codes in flight
+constexpr int LONE_TILE = 64 * 32;  // bytes of a wave's key tile: 64 channels x 16 tokens
+constexpr int LONE_CHUNK = 512;     // tokens between two exchanges of partial logits
+
+// Wave w of the launch is half w % 2 of unit w / 2; units are ordered like the waves of a head per wave.
+struct LoneUnit {
+    int bx, seg, half, c;
+    bool active;
+    __device__ __forceinline__ LoneUnit(int BH, int nseg, int wave)
+    {
+        int wis;
+        interleave_segment(wave >> 1, nseg, seg, wis);
+        half = wave & 1;
+        c = half * 64 + (int)(threadIdx.x & 63);
+        active = wis < BH;
+        bx = min(wis, BH - 1);
+    }
+};
+
+// See SegLoads; also the word that the appended token goes to and the token itself.
+struct LoneLoads {
+    uint32_t *cbh;      // this head, this channel
+    // this segment's whole supergroups: reads past them are dropped, and a load takes no address arithmetic (with a
+    // clamped index it was five instructions)
+    __amdgpu_buffer_rsrc_t codes;
+    int lane4;
+    int t0, t1, nfull, ntail;
+    bool last, from_ckpt;
+    h1 zp, sc, al, be, tg;
+    uint32_t ck, tail, buf[LONE_PF];
+    uint16_t fresh;
+
+    __device__ __forceinline__ void start(void *cache, const FtParams &p, const h1 *x_new, int h, int bx, int c, int seg, int T,
+                                          int n_super_cap, const Seg &sa)
+    {
+        const int iv = seg_first_interval(sa, seg), pi = h * 128 + c;
+        last = seg_is_last(sa, seg);
+        t0 = iv * sa.ckpt_interval;
+        t1 = last ? T : seg_end(sa, seg);
+        nfull = (t1 - t0) >> 3;
+        ntail = (t1 - t0) & 7; // of the last segment only: the others are whole intervals
+        cbh = reinterpret_cast<uint32_t *>(cache) + (size_t)bx * n_super_cap * 128 + c;
+        codes = __builtin_amdgcn_make_buffer_rsrc(cbh - c + (size_t)(t0 >> 3) * 128, 0, nfull * 512, 0x00027000);
+        lane4 = c * 4;
+        from_ckpt = iv > 0;
+        ck = 0;
+        if (from_ckpt)
+            ck = *reinterpret_cast<const uint32_t *>(sa.ckpt + (((size_t)bx * sa.n_ckpt_cap + iv - 1) * 128 + c) * 2);
+        zp = p.zp[pi];
+        sc = p.sc[pi];
+        al = p.al[pi];
+        be = p.be[pi];
+        tg = p.tg[pi];
+#pragma unroll
+        for (int i = 0; i < LONE_PF; i++)
+            buf[i] = load(0, i);
+        tail = cbh[(size_t)(last ? T >> 3 : 0) * 128];
+        fresh = reinterpret_cast<const uint16_t *>(x_new)[(size_t)bx * 128 + c];
+    }
+    // supergroup sg + i, i < LONE_PF; read once: not kept in the caches
+    __device__ __forceinline__ uint32_t load(int sg, int i) const
+    {
+        return __builtin_amdgcn_raw_buffer_load_b32(codes, lane4 + i * 512, sg * 512, 2);
+    }
+    __device__ __forceinline__ Lone state() const
+    {
+        const h2 s = from_ckpt ? as_h2(ck) : (h2){zp, sc};
+        const h1 one = (h1)1.0f, bt = be * tg; // omt = 1 - beta*target, both steps rounded (gemv.cu:220-221)
+        Lone r;
+        r.z = as_u32((h2){s.x, (h1)0.0f});
+        r.r = as_u32((h2){(h1)0.0f, s.y});
+        r.ca = as_u32((h2){al, one});
+        r.cf = as_u32((h2){one, be});
+        r.c0 = as_u32((h2){(h1)0.0f, one - bt});
+        return r;
+    }
+};
+
+__device__ __forceinline__ void lone_lookup(uint2 *e, const uint2 *lut, uint32_t word, uint32_t lane_copy)
+{
+#pragma unroll
+    for (int k = 0; k < 4; k++)
+        e[k] = lut_get(lut, word, lane_copy, k);
+}
+
+// The last segment's end: hands out the state after token T - 1, records it where token T opens an interval,
+// quantises token T into its word (gemv.cu:744-798, 1105-1157) and returns its value r16(q*sc + zp).
+__device__ __forceinline__ h1 lone_append(const LoneLoads &s, const Lone &st, int bx, int c, int T, h1 *state_out, const Seg &sa,
+                                          bool active)
+{
+    const uint32_t zs = as_u32((h2){lone_zp(st), lone_sc(st)});
+    if (active && state_out != nullptr)
+        *reinterpret_cast<uint32_t *>(state_out + ((size_t)bx * 128 + c) * 2) = zs;
+    if (active && sa.ckpt != nullptr && T > 0 && T % sa.ckpt_interval == 0) {
+        const int j = T / sa.ckpt_interval - 1;
+        if (j < sa.n_ckpt_cap)
+            *reinterpret_cast<uint32_t *>(sa.ckpt + (((size_t)bx * sa.n_ckpt_cap + j) * 128 + c) * 2) = zs;
+    }
+    const h1 x = act2(s.fresh, sa.act_bf16).x;
+    const int q = quantize<4>(x, lone_zp(st), lone_sc(st));
+    const int sh = 4 * s.ntail;
+    if (active)
+        s.cbh[(size_t)(T >> 3) * 128] = (s.tail & ~(0xFu << sh)) | ((uint32_t)(q + 8) << sh);
+    return __builtin_fmaf16((h1)q, lone_sc(st), lone_zp(st));
+}
+
+// forward_qk of a wave's 64 channels.  The values of 16 tokens go to an LDS tile, 32 bytes per channel, from
+// which transposing reads hand every lane eight channels of its token as a column for the matrix cores; all rows are
+// the query.  Columns of four tiles are put side by side, a lane per token, and written as the half's share of
+// the logits (fp32); the two halves of a head are added by who reads them.
+// ACC: at most eight waves to a workgroup; the compiler then keeps products in accumulation registers.
+// The tile's 16-byte pieces change places with every fourth channel, so that eight lanes' writes spread over the banks.
+template <bool ACC>
+struct LoneScores {
+    char *tile;
+    int lane, wr[2], rd[2];
+    h8v qa[2], kv[2];
+    f4v d;
+    float hold;
+
+    // loads the queries (rows are 8-byte aligned); ready() once the rest of the workgroup's loads are out
+    __device__ __forceinline__ LoneScores(char *tile_, int lane_, const h1 *q) : tile(tile_), lane(lane_)
+    {
+#pragma unroll
+        for (int m = 0; m < 2; m++) {
+            const uint2 *src = reinterpret_cast<const uint2 *>(q + m * 32 + (lane >> 4) * 8);
+            const uint2 a = src[0], b = src[1];
+            qa[m] = __builtin_bit_cast(h8v, make_uint4(a.x, a.y, b.x, b.y));
+        }
+    }
+    __device__ __forceinline__ void ready(int act_bf16)
+    {
+#pragma unroll
+        for (int m = 0; m < 2; m++) {
+            if (act_bf16) {
+                const uint4 u = __builtin_bit_cast(uint4, qa[m]);
+                qa[m] = __builtin_bit_cast(h8v, make_uint4(as_u32(act2(u.x, 1)), as_u32(act2(u.y, 1)),
+                                                           as_u32(act2(u.z, 1)), as_u32(act2(u.w, 1))));
+            }
+            kv[m] = (h8v){};
+            wr[m] = lane * 32 + ((m ^ (lane >> 2 & 1)) << 4);
+            // rows 4 * m.. of a quarter's eight channels; lane i of 16 reads row i / 4, tokens 4 * (i % 4)..
+            rd[m] = ((lane >> 4) * 8 + m * 4 + (lane >> 2 & 3)) * 32 + (((lane >> 1 & 1) ^ m) << 4) + (lane & 1) * 8;
+        }
+        d = (f4v){0.0f, 0.0f, 0.0f, 0.0f};
+        hold = 0.0f;
+    }
+    __device__ __forceinline__ void write(int half, const uint32_t *x)
+    {
+        *reinterpret_cast<uint4 *>(tile + wr[half]) = make_uint4(x[0], x[1], x[2], x[3]);
+    }
+    __device__ __forceinline__ void fetch()
+    {
+        typedef short s4v __attribute__((ext_vector_type(4)));
+        typedef __attribute__((address_space(3))) s4v *Lds;
+        const auto base = (__attribute__((address_space(3))) char *)tile;
+#pragma unroll
+        for (int m = 0; m < 2; m++) {
+            const s4v a = __builtin_amdgcn_ds_read_tr16_b64_v4i16((Lds)(base + m * 1024 + rd[0]));
+            const s4v b = __builtin_amdgcn_ds_read_tr16_b64_v4i16((Lds)(base + m * 1024 + rd[1]));
+            const uint2 x = __builtin_bit_cast(uint2, a), y = __builtin_bit_cast(uint2, b);
+            kv[m] = __builtin_bit_cast(h8v, make_uint4(x.x, x.y, y.x, y.y));
+        }
+    }
+    __device__ __forceinline__ void multiply()
+    {
+        d = (f4v){0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+        for (int m = 0; m < 2; m++)
+            d = __builtin_amdgcn_mfma_f32_16x16x32_f16(qa[m], kv[m], d, 0, 0, 0);
+    }
+    // the column of the u-th tile of four goes to the lanes of quarter u
+    __device__ __forceinline__ void keep(int u)
+    {
+        if constexpr (ACC) // all of d is held up to here: see PairScores::emit
+            asm volatile("" ::"a"(d));
+        else
+            asm volatile("" ::"v"(d));
+        hold = (lane >> 4) == u ? d.x : hold;
+    }
+
+    // supergroups sg0 .. sg0 + n of the segment, sg0 a multiple of LONE_PF; the shares of their logits to part[0..8n)
+    __device__ __forceinline__ void run(const uint2 *lut, uint32_t lane_copy, Lone &st, LoneLoads &s, int sg0, int n, float *part)
+    {
+        if (n <= 0)
+            return;
+        uint2 e[2][4];
+        lone_lookup(e[0], lut, s.buf[0], lane_copy);
+        wait_lgkm();
+        // tile i / 2 of a group of eight supergroups is written after its two, fetched with the second, multiplied
+        // half a tile later and kept another half later
+        auto body = [&](int sg, auto ic, auto &&group_done) __attribute__((always_inline)) {
+            constexpr int i = decltype(ic)::value;
+            lone_lookup(e[(i & 1) ^ 1], lut, s.buf[(i + 1) % LONE_PF], lane_copy); // stale past the end: looked up, never used
+            s.buf[i] = s.load(sg0 + sg - i + LONE_PF, i);
+            __builtin_amdgcn_sched_barrier(0);
+            uint32_t x[4];
+            lone_eight(st, e[i & 1], x);
+            write(i & 1, x);
+            __builtin_amdgcn_sched_barrier(0);
+            if constexpr (i & 1) {
+                keep((i / 2 + 3) & 3);
+                if constexpr (i == 1)
+                    group_done();
+                fetch();
+            } else {
+                multiply();
+            }
+            __builtin_amdgcn_sched_barrier(0);
+        };
+        int g0 = 0;
+        for (; g0 + LONE_PF <= n; g0 += LONE_PF)
+            static_for<LONE_PF>([&](auto ic) __attribute__((always_inline)) {
+                // the group before this one; at the first what is stored is overwritten by the second's or the end's
+                body(g0 + decltype(ic)::value, ic, [&]() __attribute__((always_inline)) { part[max(g0 - LONE_PF, 0) * 8 + lane] = hold; });
+            });
+        static_for<LONE_PF - 1>([&](auto ic) __attribute__((always_inline)) {
+            if (g0 + decltype(ic)::value < n)
+                body(g0 + decltype(ic)::value, ic, [&]() __attribute__((always_inline)) {
+                    if (g0 > 0)
+                        part[(g0 - LONE_PF) * 8 + lane] = hold;
+                });
+        });
+        const int end = n - 1, base = (end & ~7) * 8;
+        if (end & 1) {
+            multiply();
+        } else { // half a tile, and the one before it is still to be kept
+            keep((end / 2 + 3) & 3);
+            if ((end & 7) == 0 && end > 0)
+                part[base - 64 + lane] = hold;
+            fetch();
+            multiply();
+        }
+        keep((end / 2) & 3);
+        if (lane < 8 * n - base)
+            part[base + lane] = hold;
+    }
+    // up to eight tokens by themselves
+    __device__ __forceinline__ void few(const uint32_t *x, int ntok, float *part)
+    {
+        write(0, x);
+        fetch();
+        multiply();
+        keep(0);
+        if (lane < ntok)
+            part[lane] = hold;
+    }
+    // the last segment's ragged tail and the appended token; their shares of the logits to part[0..ntail]
+    __device__ __forceinline__ void finish(const LoneLoads &s, Lone &st, int bx, int c, int T, h1 *state_out, const Seg &sa, bool active,
+                                           float *part)
+    {
+        uint32_t v[8] = {0, 0, 0, 0, 0, 0, 0, 0};
+#pragma unroll
+        for (int t = 0; t < 7; t++)
+            if (t < s.ntail)
+                v[t] = __builtin_bit_cast(uint16_t, lone_token(st, (int)(s.tail >> (4 * t) & 15) - 8));
+        const uint32_t self = __builtin_bit_cast(uint16_t, lone_append(s, st, bx, c, T, state_out, sa, active));
+#pragma unroll
+        for (int t = 0; t < 8; t++)
+            v[t] = t == s.ntail ? self : v[t];
+        const uint32_t x[4] = {v[0] | v[1] << 16, v[2] | v[3] << 16, v[4] | v[5] << 16, v[6] | v[7] << 16};
+        few(x, s.ntail + 1, part);
+    }
+};
+
+// forward_ov of a wave's 64 channels: adds supergroups sg0 .. sg0 + n of the segment to acc, sg0 a multiple of
+// LONE_PF.  w: their weights, in LDS.
+__device__ __forceinline__ void lone_values(const uint2 *lut, uint32_t lane_copy, LoneLoads &s, Lone &st, int sg0, int n, const h1 *w,
+                                            float &acc)
+{
+    if (n <= 0)
+        return;
+    const uint4 *w4 = reinterpret_cast<const uint4 *>(w);
+    uint2 e[2][4];
+    uint4 wv[2];
+    lone_lookup(e[0], lut, s.buf[0], lane_copy);
+    wv[0] = w4[0];
+    wait_lgkm();
+    rotate_over<LONE_PF>(n, [&](int sg, auto ic) __attribute__((always_inline)) {
+        constexpr int i = decltype(ic)::value, half = i & 1;
+        lone_lookup(e[half ^ 1], lut, s.buf[(i + 1) % LONE_PF], lane_copy); // stale past the end: looked up, never used
+        wv[half ^ 1] = w4[sg + 1]; // so are these: the caller's LDS goes on behind them
+        s.buf[i] = s.load(sg0 + sg - i + LONE_PF, i);
+        __builtin_amdgcn_sched_barrier(0);
+        lone_eight_weighted(st, e[half], wv[half], acc);
+        __builtin_amdgcn_sched_barrier(0);
+    });
+}
+// The last segment's ragged tail and the appended token.  w1(t): the weight of the segment's token t.
+template <typename W1>
+__device__ __forceinline__ void lone_values_end(const LoneLoads &s, Lone &st, W1 &&w1, int bx, int c, int T, h1 *state_out, const Seg &sa,
+                                                bool active, float &acc)
+{
+    if (!s.last)
+        return;
+#pragma unroll
+    for (int t = 0; t < 7; t++)
+        if (t < s.ntail)
+            acc = __builtin_fmaf((float)w1(8 * s.nfull + t), (float)lone_token(st, (int)(s.tail >> (4 * t) & 15) - 8), acc);
+    acc = __builtin_fmaf((float)w1(T - s.t0), (float)lone_append(s, st, bx, c, T, state_out, sa, active), acc);
+}
+
+template <int BLK>
+__global__ __launch_bounds__(BLK) void qk_lone_kernel(const h1 *q, uint4 *cache, const h1 *k_new, h1 *__restrict__ out, FtParams p, int BH,
+                                                      int H, int T, int n_super_cap, h1 *__restrict__ state_out, Seg sa)
+{
+    constexpr int WAVES = BLK / 64;
+    sa.groups = 0; // only even plans come here
+    // the table at LDS offset 0, a tile per wave, a chunk of partial logits per wave: half of a CU's LDS
+    __shared__ uint4 smem[(LUT_WORDS64 * 8 + WAVES * LONE_TILE + WAVES * LONE_CHUNK * 4) / 16];
+    uint2 *lut = reinterpret_cast<uint2 *>(smem);
+    char *lds = reinterpret_cast<char *>(smem) + LUT_WORDS64 * 8;
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    const uint32_t lane_copy = (uint32_t)(lane & (LUT_COPIES - 1)) * 8u;
+    const LoneUnit un(BH, sa.nseg, (int)blockIdx.x * WAVES + wave);
+    LoneScores<BLK <= 512> scores(lds + wave * LONE_TILE, lane, q + (size_t)un.bx * 128 + un.half * 64);
+    LoneLoads s;
+    s.start(cache, p, k_new, un.bx % H, un.bx, un.c, un.seg, T, n_super_cap, sa);
+    lone_fill<BLK>(lut, threadIdx.x);
+    __syncthreads();
+
+    float *unit_part = reinterpret_cast<float *>(lds + WAVES * LONE_TILE) + (wave >> 1) * 2 * LONE_CHUNK;
+    float *part = unit_part + un.half * LONE_CHUNK;
+    h1 *ob = out + (size_t)un.bx * sa.row_pitch + s.t0;
+    // the unit's logits from t on, n of them: the shares of its two waves added
+    auto flush = [&](int t, int n) __attribute__((always_inline)) {
+        __syncthreads();
+        if (un.active)
+            for (int i = un.c; i < n; i += 128)
+                ob[t + i] = (h1)(unit_part[i] + unit_part[LONE_CHUNK + i]);
+        __syncthreads();
+    };
+    Lone st = s.state();
+    scores.ready(sa.act_bf16);
+    const int longest = sa.nseg > 1 ? sa.seg_tokens : T; // every wave of the workgroup takes part in every exchange
+    for (int t = 0; t < longest; t += LONE_CHUNK) {
+        const int n = max(0, min(LONE_CHUNK / 8, s.nfull - t / 8));
+        scores.run(lut, lane_copy, st, s, t / 8, n, part);
+        flush(t, 8 * n);
+    }
+    if (s.last)
+        scores.finish(s, st, un.bx, un.c, T, state_out, sa, un.active, part);
+    flush(s.nfull * 8, s.last ? s.ntail + 1 : 0);
+}
+
+template <int BLK>
+__global__ __launch_bounds__(BLK) void ov_lone_kernel(const h1 *attn, uint4 *cache, const h1 *v_new, h1 *__restrict__ out,
+                                                      float *__restrict__ partial, FtParams p, int BH, int H, int T, int n_super_cap,
+                                                      h1 *__restrict__ state_out, Seg sa)
+{
+    constexpr int WAVES = BLK / 64;
+    sa.groups = 0;
+    // the table at LDS offset 0; per wave the weights of a chunk (and a vector that is read behind them, never used)
+    __shared__ uint4 smem[LUT_WORDS64 / 2 + WAVES * (LONE_CHUNK / 8 + 1)];
+    const uint2 *lut = reinterpret_cast<const uint2 *>(smem);
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    uint4 *weights = smem + LUT_WORDS64 / 2 + wave * (LONE_CHUNK / 8 + 1);
+    const uint32_t lane_copy = (uint32_t)(lane & (LUT_COPIES - 1)) * 8u;
+    const LoneUnit un(BH, sa.nseg, (int)blockIdx.x * WAVES + wave);
+    LoneLoads s;
+    s.start(cache, p, v_new, un.bx % H, un.bx, un.c, un.seg, T, n_super_cap, sa);
+    const h1 *wb = attn + (size_t)un.bx * sa.row_pitch + s.t0;
+    // a chunk's weights, eight tokens per lane, a chunk ahead: as a load of eight for all lanes alike, one per supergroup,
+    // they were a tenth of a lone wave's time (more where rows are only 2-byte aligned)
+    uint4 ahead = make_uint4(0, 0, 0, 0);
+    auto load_chunk = [&](int sg) __attribute__((always_inline)) {
+        if (s.nfull > 0)
+            __builtin_memcpy(&ahead, wb + (size_t)min(sg + lane, s.nfull - 1) * 8, 16);
+    };
+    load_chunk(0);
+    lone_fill<BLK>(reinterpret_cast<uint2 *>(smem), threadIdx.x);
+    __syncthreads();
+    if (!un.active)
+        return;
+    Lone st = s.state();
+    float acc = 0.0f;
+    for (int sg = 0; sg < s.nfull; sg += LONE_CHUNK / 8) {
+        weights[lane] = ahead;
+        load_chunk(sg + LONE_CHUNK / 8);
+        lone_values(lut, lane_copy, s, st, sg, min(LONE_CHUNK / 8, s.nfull - sg), reinterpret_cast<const h1 *>(weights), acc);
+    }
+    lone_values_end(s, st, [&](int t) { return wb[t]; }, un.bx, un.c, T, state_out, sa, true, acc);
+    if (sa.nseg == 1) {
+        h1 *o = out + (size_t)un.bx * 128 + un.c;
+        if (sa.act_bf16)
+            *reinterpret_cast<uint16_t *>(o) = (uint16_t)bf16_bits((h1)acc);
+        else
+            *o = (h1)acc;
+    } else {
+        partial[((size_t)un.seg * BH + un.bx) * 128 + un.c] = acc;
+    }
+}
+
+} // namespace adkv
