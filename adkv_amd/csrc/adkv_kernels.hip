@@ -2949,10 +2949,75 @@ static int launch_step_grouped(int GQ, long waves, hipStream_t st, Args... args)
     }
 }
 
+// Whether step_lone_kernel takes a step of the two launches, and with which workgroups: a wave's 64 channels bring
+// twice the waves of two channels per lane and four or eight times those of wide heads, and pay as long as a CU holds
+// them at once: 16 waves, and 12 / 8 with four / eight query heads, whose logits take more of the LDS; with one or two
+// query heads of 128 channels, whose other form has its waves' LDS reads covered by then, 12.  us per step on the device,
+// step_segments_kernel / this, waves per CU in brackets: head dim 512, 9 x 8 heads x 80 (2) 22.8 / 11.8, 2 x 8 x 1000 (2)
+// 47.7 / 18.7, 8 x 8 x 2000 (16) 48.8 / 28.9, 10 x 8 x 2000 (20) 48.9 / 49.1; head dim 256, 1 x 8 x 300 30.3 / 14.1, 2 x 16 x
+// 5021 (10) 31.7 / 23.2, 4 x 8 x 8190 (16) 33.7 / 30.4, 5 x 8 x 8000 (20) 44.6 / 49.2; head dim 128, 1 x 32 x 2000 (2)
+// 20.7 / 15.7, 4 x 32 x 2000 (8) 21.3 / 19.5, 6 x 32 x 2000 (12) 27.3 / 24.1, 8 x 32 x 2000 (16) 27.4 / 28.0; two query heads, 4 x 16
+// x 2000 (4) 22.6 / 16.3, 8 x 16 x 2000 (8) 23.3 / 20.3, 12 x 16 x 2000 (12) 30.0 / 25.6, 16 x 16 x 2000 (16) 31.1 / 30.7; four, 1 x 8
+// x 603 22.2 / 15.3, 28 x 8 x 936 (7) 24.5 / 21.3, 8 x 8 x 6000 (12) 33.5 / 28.4, 8 x 8 x 7000 (14) 34.1 / 46; eight, 3 x 8 x
+// 113 18.9 / 13.7, 3 x 8 x 4799 (4) 29.4 / 19.8, 8 x 8 x 4000 (8) 35.1 / 29.4, 8 x 8 x 8000 (16) 45.4 / 46.1.
+// Small workgroups spread best; what they leave free of a CU's LDS (the table takes 64 KB) holds a second one only with
+// one query head.  A workgroup of as many waves as the CU is to hold otherwise: 2 x 16 x 5021 of 256 channels with 4, 8, 12
+// and 16 waves 26.5, 32.6, 23.3, 27.4; 28 x 8 x 936 with four query heads 28.1, 21.3, 25.4.
+static int step_lone_threads(long units, int D, int GQ, int bits, int longest)
+{
+    const long per_cu = (units * (D / 64) + cus() - 1) / cus();
+    const int most = GQ == 8 ? 8 : D == 128 ? 12 : 16;
+    if (bits != 4 || longest > 256 || per_cu > most)
+        return 0;
+    if (D == 512)
+        return per_cu <= 8 ? 512 : 1024;
+    if (per_cu <= (GQ == 1 ? 8 : 4))
+        return 256;
+    return per_cu <= 8 ? 512 : per_cu <= 12 ? 768 : 1024;
+}
+
+template <int D, int GQ, typename... Args>
+static int launch_step_lone(int blk, long units, hipStream_t st, Args... args)
+{
+    const int per_block = blk / D; // units: a wave per 64 channels
+    const dim3 grid((unsigned)((units + per_block - 1) / per_block));
+#define ADKV_STEP(BLK) hipLaunchKernelGGL((step_lone_kernel<D, GQ, BLK>), grid, dim3(BLK), 0, st, args...)
+    if constexpr (D != 512) {
+        if (blk == 256)
+            ADKV_STEP(256);
+        if constexpr (GQ != 8) {
+            if (blk == 768)
+                ADKV_STEP(768);
+        }
+    }
+    if constexpr (D == 512 || GQ > 1) {
+        if (blk == 512)
+            ADKV_STEP(512);
+    }
+    if constexpr (D != 128) {
+        if (blk == 1024)
+            ADKV_STEP(1024);
+    }
+#undef ADKV_STEP
+    return check_launch();
+}
+
 template <typename... Args>
-static int launch_step_segments(int cpl, int GQ, int bits, int D, int BH, int nseg, hipStream_t st, Args... args)
+static int launch_step_segments(int cpl, int GQ, int bits, int D, int BH, int nseg, int longest, hipStream_t st, Args... args)
 {
     const long units = padded_units<64>(BH, nseg);
+    if (const int blk = step_lone_threads(units, D, GQ, bits, longest)) {
+        if (D == 512)
+            return launch_step_lone<512, 1>(blk, units, st, args...);
+        if (D == 256)
+            return launch_step_lone<256, 1>(blk, units, st, args...);
+        switch (GQ) {
+        case 1: return launch_step_lone<128, 1>(blk, units, st, args...);
+        case 2: return launch_step_lone<128, 2>(blk, units, st, args...);
+        case 4: return launch_step_lone<128, 4>(blk, units, st, args...);
+        default: return launch_step_lone<128, 8>(blk, units, st, args...);
+        }
+    }
     if (D == 512)
         return launch_step_shape<512, 8, 4, 1>(units, st, args...);
     if (D == 256)
@@ -3968,7 +4033,7 @@ int adkv_decode_step(const void *q, void *k_cache, void *v_cache, const void *k_
             const long rows = (long)B * Hq;
             float4 *ml = (float4 *)(ws + 2 * mat);
             float *partial = (float *)(ws + 2 * mat + pad256(ka.nseg * rows * 16));
-            if ((rc = launch_step_segments(cpl, Hq / H, bits, D, B * H, ka.nseg, (hipStream_t)stream, (const h1 *)q, (uint4 *)k_cache,
+            if ((rc = launch_step_segments(cpl, Hq / H, bits, D, B * H, ka.nseg, ka.nseg > 1 ? ka.seg_tokens : T, (hipStream_t)stream, (const h1 *)q, (uint4 *)k_cache,
                                            (const h1 *)k_new, (uint4 *)v_cache, (const h1 *)v_new, mk, (h1 *)logits, partial, ml,
                                            ft_params(k_params), ft_params(v_params), B * H, H, T, n_super_cap, scaling, ka, va)))
                 return rc;

@@ -1,5 +1,6 @@
 // forward_qk and forward_ov of launches that leave SIMDs empty: head dim 128, 4-bit codes, one query head per KV
-// head, one channel per lane, a head over two waves.  Included by adkv_kernels.hip after the shared device helpers.
+// head, one channel per lane, a head over two waves; and their parts for steps of any head dim D, a head over D / 64
+// waves, with GQ query heads (adkv_segment_step.h).  Included by adkv_kernels.hip after the shared device helpers.
 //
 // Such a launch takes as long as one wave's instructions per token: a wave alone on its SIMD issues one every four
 // or five cycles, LDS reads twelve, whatever the other lanes do.  With two channels per lane that is a lookup and
@@ -11,6 +12,7 @@ namespace adkv {
 
 constexpr int LONE_PF = 8;          // supergroups of codes in flight
 constexpr int LONE_TILE = 64 * 32;  // bytes of a wave's key tile: 64 channels x 16 tokens
+constexpr int LONE_SEG = 264;       // tokens of a segment of a step, and one vector behind them
 constexpr int LONE_CHUNK = 512;     // tokens between two exchanges of partial logits
 
 // Wave w of the launch is half w % 2 of unit w / 2; units are ordered like the waves of a head per wave.
@@ -29,7 +31,9 @@ struct LoneUnit {
 };
 
 // See SegLoads; also the word that the appended token goes to and the token itself.
+template <int D = 128>
 struct LoneLoads {
+    static constexpr int HEAD = D;
     uint32_t *cbh;      // this head, this channel
     // this segment's whole supergroups: reads past them are dropped, and a load takes no address arithmetic (with a
     // clamped index it was five instructions)
@@ -44,19 +48,19 @@ struct LoneLoads {
     __device__ __forceinline__ void start(void *cache, const FtParams &p, const h1 *x_new, int h, int bx, int c, int seg, int T,
                                           int n_super_cap, const Seg &sa)
     {
-        const int iv = seg_first_interval(sa, seg), pi = h * 128 + c;
+        const int iv = seg_first_interval(sa, seg), pi = h * D + c;
         last = seg_is_last(sa, seg);
         t0 = iv * sa.ckpt_interval;
         t1 = last ? T : seg_end(sa, seg);
         nfull = (t1 - t0) >> 3;
         ntail = (t1 - t0) & 7; // of the last segment only: the others are whole intervals
-        cbh = reinterpret_cast<uint32_t *>(cache) + (size_t)bx * n_super_cap * 128 + c;
-        codes = __builtin_amdgcn_make_buffer_rsrc(cbh - c + (size_t)(t0 >> 3) * 128, 0, nfull * 512, 0x00027000);
+        cbh = reinterpret_cast<uint32_t *>(cache) + (size_t)bx * n_super_cap * D + c;
+        codes = __builtin_amdgcn_make_buffer_rsrc(cbh - c + (size_t)(t0 >> 3) * D, 0, nfull * D * 4, 0x00027000);
         lane4 = c * 4;
         from_ckpt = iv > 0;
         ck = 0;
         if (from_ckpt)
-            ck = *reinterpret_cast<const uint32_t *>(sa.ckpt + (((size_t)bx * sa.n_ckpt_cap + iv - 1) * 128 + c) * 2);
+            ck = *reinterpret_cast<const uint32_t *>(sa.ckpt + (((size_t)bx * sa.n_ckpt_cap + iv - 1) * D + c) * 2);
         zp = p.zp[pi];
         sc = p.sc[pi];
         al = p.al[pi];
@@ -65,13 +69,13 @@ struct LoneLoads {
 #pragma unroll
         for (int i = 0; i < LONE_PF; i++)
             buf[i] = load(0, i);
-        tail = cbh[(size_t)(last ? T >> 3 : 0) * 128];
-        fresh = reinterpret_cast<const uint16_t *>(x_new)[(size_t)bx * 128 + c];
+        tail = cbh[(size_t)(last ? T >> 3 : 0) * D];
+        fresh = reinterpret_cast<const uint16_t *>(x_new)[(size_t)bx * D + c];
     }
     // supergroup sg + i, i < LONE_PF; read once: not kept in the caches
     __device__ __forceinline__ uint32_t load(int sg, int i) const
     {
-        return __builtin_amdgcn_raw_buffer_load_b32(codes, lane4 + i * 512, sg * 512, 2);
+        return __builtin_amdgcn_raw_buffer_load_b32(codes, lane4 + i * D * 4, sg * D * 4, 2);
     }
     __device__ __forceinline__ Lone state() const
     {
@@ -96,22 +100,23 @@ __device__ __forceinline__ void lone_lookup(uint2 *e, const uint2 *lut, uint32_t
 
 // The last segment's end: hands out the state after token T - 1, records it where token T opens an interval,
 // quantises token T into its word (gemv.cu:744-798, 1105-1157) and returns its value r16(q*sc + zp).
-__device__ __forceinline__ h1 lone_append(const LoneLoads &s, const Lone &st, int bx, int c, int T, h1 *state_out, const Seg &sa,
+template <int D>
+__device__ __forceinline__ h1 lone_append(const LoneLoads<D> &s, const Lone &st, int bx, int c, int T, h1 *state_out, const Seg &sa,
                                           bool active)
 {
     const uint32_t zs = as_u32((h2){lone_zp(st), lone_sc(st)});
     if (active && state_out != nullptr)
-        *reinterpret_cast<uint32_t *>(state_out + ((size_t)bx * 128 + c) * 2) = zs;
+        *reinterpret_cast<uint32_t *>(state_out + ((size_t)bx * D + c) * 2) = zs;
     if (active && sa.ckpt != nullptr && T > 0 && T % sa.ckpt_interval == 0) {
         const int j = T / sa.ckpt_interval - 1;
         if (j < sa.n_ckpt_cap)
-            *reinterpret_cast<uint32_t *>(sa.ckpt + (((size_t)bx * sa.n_ckpt_cap + j) * 128 + c) * 2) = zs;
+            *reinterpret_cast<uint32_t *>(sa.ckpt + (((size_t)bx * sa.n_ckpt_cap + j) * D + c) * 2) = zs;
     }
     const h1 x = act2(s.fresh, sa.act_bf16).x;
     const int q = quantize<4>(x, lone_zp(st), lone_sc(st));
     const int sh = 4 * s.ntail;
     if (active)
-        s.cbh[(size_t)(T >> 3) * 128] = (s.tail & ~(0xFu << sh)) | ((uint32_t)(q + 8) << sh);
+        s.cbh[(size_t)(T >> 3) * D] = (s.tail & ~(0xFu << sh)) | ((uint32_t)(q + 8) << sh);
     return __builtin_fmaf16((h1)q, lone_sc(st), lone_zp(st));
 }
 
@@ -120,8 +125,10 @@ __device__ __forceinline__ h1 lone_append(const LoneLoads &s, const Lone &st, in
 // the query.  Columns of four tiles are put side by side, a lane per token, and written as the half's share of
 // the logits (fp32); the two halves of a head are added by who reads them.
 // ACC: at most eight waves to a workgroup; the compiler then keeps products in accumulation registers.
+// GQ: query heads per KV head.  Row r of the product is head r * GQ / 16, so that a lane has the share of its token and of the
+// head of its quarter (of two heads with eight): a store per tile where a single head's columns are collected first.
 // The tile's 16-byte pieces change places with every fourth channel, so that eight lanes' writes spread over the banks.
-template <bool ACC>
+template <bool ACC, int GQ = 1, int D = 128>
 struct LoneScores {
     char *tile;
     int lane, wr[2], rd[2];
@@ -134,7 +141,7 @@ struct LoneScores {
     {
 #pragma unroll
         for (int m = 0; m < 2; m++) {
-            const uint2 *src = reinterpret_cast<const uint2 *>(q + m * 32 + (lane >> 4) * 8);
+            const uint2 *src = reinterpret_cast<const uint2 *>(q + ((lane & 15) * GQ >> 4) * D + m * 32 + (lane >> 4) * 8);
             const uint2 a = src[0], b = src[1];
             qa[m] = __builtin_bit_cast(h8v, make_uint4(a.x, a.y, b.x, b.y));
         }
@@ -190,8 +197,23 @@ struct LoneScores {
         hold = (lane >> 4) == u ? d.x : hold;
     }
 
+    // several query heads: the first ntok tokens of a tile, a row of LONE_SEG per head
+    __device__ __forceinline__ void put(float *part, int ntok)
+    {
+        if constexpr (ACC)
+            asm volatile("" ::"a"(d));
+        else
+            asm volatile("" ::"v"(d));
+        const int t = lane & 15, quarter = lane >> 4;
+        if (t < ntok) {
+            part[(GQ == 8 ? 2 * quarter : quarter * GQ >> 2) * LONE_SEG + t] = d.x;
+            if constexpr (GQ == 8)
+                part[(2 * quarter + 1) * LONE_SEG + t] = d.z;
+        }
+    }
+
     // supergroups sg0 .. sg0 + n of the segment, sg0 a multiple of LONE_PF; the shares of their logits to part[0..8n)
-    __device__ __forceinline__ void run(const uint2 *lut, uint32_t lane_copy, Lone &st, LoneLoads &s, int sg0, int n, float *part)
+    __device__ __forceinline__ void run(const uint2 *lut, uint32_t lane_copy, Lone &st, LoneLoads<D> &s, int sg0, int n, float *part)
     {
         if (n <= 0)
             return;
@@ -210,9 +232,13 @@ struct LoneScores {
             write(i & 1, x);
             __builtin_amdgcn_sched_barrier(0);
             if constexpr (i & 1) {
-                keep((i / 2 + 3) & 3);
-                if constexpr (i == 1)
-                    group_done();
+                if constexpr (GQ > 1) {
+                    put(part + max(sg - 3, 0) * 8, 16); // at the first what is stored is overwritten
+                } else {
+                    keep((i / 2 + 3) & 3);
+                    if constexpr (i == 1)
+                        group_done();
+                }
                 fetch();
             } else {
                 multiply();
@@ -233,6 +259,16 @@ struct LoneScores {
                 });
         });
         const int end = n - 1, base = (end & ~7) * 8;
+        if constexpr (GQ > 1) {
+            if (!(end & 1)) {
+                if (end > 0)
+                    put(part + (end - 2) * 8, 16);
+                fetch();
+            }
+            multiply();
+            put(part + (end & ~1) * 8, end & 1 ? 16 : 8);
+            return;
+        }
         if (end & 1) {
             multiply();
         } else { // half a tile, and the one before it is still to be kept
@@ -252,12 +288,16 @@ struct LoneScores {
         write(0, x);
         fetch();
         multiply();
+        if constexpr (GQ > 1) {
+            put(part, ntok);
+            return;
+        }
         keep(0);
         if (lane < ntok)
             part[lane] = hold;
     }
     // the last segment's ragged tail and the appended token; their shares of the logits to part[0..ntail]
-    __device__ __forceinline__ void finish(const LoneLoads &s, Lone &st, int bx, int c, int T, h1 *state_out, const Seg &sa, bool active,
+    __device__ __forceinline__ void finish(const LoneLoads<D> &s, Lone &st, int bx, int c, int T, h1 *state_out, const Seg &sa, bool active,
                                            float *part)
     {
         uint32_t v[8] = {0, 0, 0, 0, 0, 0, 0, 0};
@@ -276,7 +316,8 @@ struct LoneScores {
 
 // forward_ov of a wave's 64 channels: adds supergroups sg0 .. sg0 + n of the segment to acc, sg0 a multiple of
 // LONE_PF.  w: their weights, in LDS.
-__device__ __forceinline__ void lone_values(const uint2 *lut, uint32_t lane_copy, LoneLoads &s, Lone &st, int sg0, int n, const h1 *w,
+template <int D>
+__device__ __forceinline__ void lone_values(const uint2 *lut, uint32_t lane_copy, LoneLoads<D> &s, Lone &st, int sg0, int n, const h1 *w,
                                             float &acc)
 {
     if (n <= 0)
@@ -298,8 +339,8 @@ __device__ __forceinline__ void lone_values(const uint2 *lut, uint32_t lane_copy
     });
 }
 // The last segment's ragged tail and the appended token.  w1(t): the weight of the segment's token t.
-template <typename W1>
-__device__ __forceinline__ void lone_values_end(const LoneLoads &s, Lone &st, W1 &&w1, int bx, int c, int T, h1 *state_out, const Seg &sa,
+template <int D, typename W1>
+__device__ __forceinline__ void lone_values_end(const LoneLoads<D> &s, Lone &st, W1 &&w1, int bx, int c, int T, h1 *state_out, const Seg &sa,
                                                 bool active, float &acc)
 {
     if (!s.last)
@@ -309,6 +350,47 @@ __device__ __forceinline__ void lone_values_end(const LoneLoads &s, Lone &st, W1
         if (t < s.ntail)
             acc = __builtin_fmaf((float)w1(8 * s.nfull + t), (float)lone_token(st, (int)(s.tail >> (4 * t) & 15) - 8), acc);
     acc = __builtin_fmaf((float)w1(T - s.t0), (float)lone_append(s, st, bx, c, T, state_out, sa, active), acc);
+}
+
+// The same for GQ query heads: the values of four tokens of a lane's channel are a column for the matrix cores as
+// they are, the weights of the query heads the rows (see ov_gqa_segment); element i of acc[n] is head 4n + i.
+// w: a row of LONE_SEG weights per head.
+template <int GQ, int D>
+__device__ __forceinline__ void lone_values_grouped(const uint2 *lut, uint32_t lane_copy, LoneLoads<D> &s, Lone &st, const h1 *w, int lane,
+                                                    f4v *acc)
+{
+    constexpr int NB = (GQ + 3) / 4;
+    if (s.nfull <= 0)
+        return;
+    const uint4 *w4[NB];
+    uint2 e[2][4];
+    uint4 wv[2][NB];
+    lone_lookup(e[0], lut, s.buf[0], lane_copy);
+#pragma unroll
+    for (int n = 0; n < NB; n++) {
+        w4[n] = reinterpret_cast<const uint4 *>(w + min(4 * n + (lane & 3), GQ - 1) * LONE_SEG);
+        wv[0][n] = w4[n][0];
+    }
+    wait_lgkm();
+    rotate_over<LONE_PF>(s.nfull, [&](int sg, auto ic) __attribute__((always_inline)) {
+        constexpr int i = decltype(ic)::value, half = i & 1;
+        lone_lookup(e[half ^ 1], lut, s.buf[(i + 1) % LONE_PF], lane_copy); // stale past the end: looked up, never used
+#pragma unroll
+        for (int n = 0; n < NB; n++)
+            wv[half ^ 1][n] = w4[n][sg + 1]; // so are these: a row goes on for a vector
+        s.buf[i] = s.load(sg - i + LONE_PF, i);
+        __builtin_amdgcn_sched_barrier(0);
+        uint32_t x[4];
+        lone_eight(st, e[half], x);
+        asm volatile("s_nop 1" ::: "memory"); // the block's results, as the matrix cores need them: two slots later
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int n = 0; n < NB; n++) {
+            acc[n] = __builtin_amdgcn_mfma_f32_4x4x4f16(as_h4(wv[half][n].x, wv[half][n].y), as_h4(x[0], x[1]), acc[n], 0, 0, 0);
+            acc[n] = __builtin_amdgcn_mfma_f32_4x4x4f16(as_h4(wv[half][n].z, wv[half][n].w), as_h4(x[2], x[3]), acc[n], 0, 0, 0);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+    });
 }
 
 template <int BLK>
@@ -325,7 +407,7 @@ __global__ __launch_bounds__(BLK) void qk_lone_kernel(const h1 *q, uint4 *cache,
     const uint32_t lane_copy = (uint32_t)(lane & (LUT_COPIES - 1)) * 8u;
     const LoneUnit un(BH, sa.nseg, (int)blockIdx.x * WAVES + wave);
     LoneScores<BLK <= 512> scores(lds + wave * LONE_TILE, lane, q + (size_t)un.bx * 128 + un.half * 64);
-    LoneLoads s;
+    LoneLoads<> s;
     s.start(cache, p, k_new, un.bx % H, un.bx, un.c, un.seg, T, n_super_cap, sa);
     lone_fill<BLK>(lut, threadIdx.x);
     __syncthreads();
@@ -368,7 +450,7 @@ __global__ __launch_bounds__(BLK) void ov_lone_kernel(const h1 *attn, uint4 *cac
     uint4 *weights = smem + LUT_WORDS64 / 2 + wave * (LONE_CHUNK / 8 + 1);
     const uint32_t lane_copy = (uint32_t)(lane & (LUT_COPIES - 1)) * 8u;
     const LoneUnit un(BH, sa.nseg, (int)blockIdx.x * WAVES + wave);
-    LoneLoads s;
+    LoneLoads<> s;
     s.start(cache, p, v_new, un.bx % H, un.bx, un.c, un.seg, T, n_super_cap, sa);
     const h1 *wb = attn + (size_t)un.bx * sa.row_pitch + s.t0;
     // a chunk's weights, eight tokens per lane, a chunk ahead: as a load of eight for all lanes alike, one per supergroup,

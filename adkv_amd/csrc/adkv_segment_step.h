@@ -231,6 +231,171 @@ __global__ __launch_bounds__(BLK) void step_segments_kernel(
     }
 }
 
+// The weights of one head of a unit of step_lone_kernel (see segment_weights): a token's logit is the sum of its shares in HW
+// rows, `stride` apart; four tokens per lane, and the one behind 256.  writes: this wave leaves the logits, m and the sums too.
+template <int HW>
+__device__ __forceinline__ void lone_weights(const float *share, int stride, h1 *logits, const MaskRow<true> &mrow, int ntok,
+                                             float scaling, h1 *p, float4 *ml, int lane, bool writes)
+{
+    const int t = lane * 4;
+    float4 a = *reinterpret_cast<const float4 *>(share + t);
+    float extra = share[256];
+#pragma unroll
+    for (int i = 1; i < HW; i++) {
+        const float4 b = *reinterpret_cast<const float4 *>(share + i * stride + t);
+        a = make_float4(a.x + b.x, a.y + b.y, a.z + b.z, a.w + b.w);
+        extra += share[i * stride + 256];
+    }
+    const h1 l[5] = {(h1)a.x, (h1)a.y, (h1)a.z, (h1)a.w, (h1)extra};
+    if (writes) {
+        if (t + 4 <= ntok) { // t0 and the pitch are multiples of 8
+            *reinterpret_cast<uint2 *>(logits + t) = make_uint2(as_u32((h2){l[0], l[1]}), as_u32((h2){l[2], l[3]}));
+        } else {
+#pragma unroll
+            for (int k = 0; k < 4; k++)
+                if (t + k < ntok)
+                    logits[t + k] = l[k];
+        }
+        if (lane == 0 && ntok > 256)
+            logits[256] = l[4];
+    }
+    float add[5] = {0.0f, 0.0f, 0.0f, 0.0f, 0.0f}, x[5], mx = -INFINITY;
+    if (mrow) {
+        if (t + 4 <= ntok) {
+            mrow.load<4>(t, add);
+        } else {
+#pragma unroll
+            for (int k = 0; k < 4; k++)
+                add[k] = t + k < ntok ? mrow.at(t + k) : 0.0f;
+        }
+        if (ntok > 256)
+            add[4] = mrow.at(256);
+    }
+#pragma unroll
+    for (int k = 0; k < 5; k++) {
+        const float v = (float)l[k] * scaling + add[k];
+        x[k] = (k < 4 ? t + k : 256) < ntok ? v : -INFINITY;
+        mx = fmaxf(mx, x[k]);
+    }
+    mx = head_reduce<64, true>(mx);
+    const float ref = mx == -INFINITY ? 0.0f : mx; // nothing but -inf: all weights are zero
+    float e[5];
+    h1 w[5];
+#pragma unroll
+    for (int k = 0; k < 5; k++) {
+        e[k] = __expf(x[k] - ref);
+        w[k] = (h1)e[k];
+    }
+    const float sum = head_reduce<64, false>((e[0] + e[1]) + (e[2] + e[3])) + e[4];
+    const float rounded = head_reduce<64, false>(((float)w[0] + (float)w[1]) + ((float)w[2] + (float)w[3])) + (float)w[4];
+    *reinterpret_cast<uint2 *>(p + t) = make_uint2(as_u32((h2){w[0], w[1]}), as_u32((h2){w[2], w[3]}));
+    if (lane == 0)
+        *reinterpret_cast<uint4 *>(p + 256) = make_uint4(as_u32((h2){w[4], (h1)0.0f}), 0, 0, 0);
+    if (writes && lane == 0)
+        *ml = make_float4(mx, sum, rounded, 0.0f);
+}
+
+// The same launch with one channel per lane, a KV head over D / 64 waves (adkv_lone.h): 4-bit codes, segments of at
+// most 256 tokens.  With few waves per SIMD a step takes as long as one wave's instructions per token, and a lane with
+// four or eight channels has two and four times as many of them; the waves of a head meet once, behind the keys, where
+// each has left its share of the logits (fp32) in the LDS, and with several query heads again behind the weights.
+// Of the 256 + 256 tokens of a full segment a lone wave takes some 9 us (19 ns per token, step_segments_kernel 27 with two
+// channels per lane, 50 with four and 90 with eight); from four waves per SIMD on vector issue holds it, 23 cycles per
+// wave and token.  us per step: 2 x 8 heads x 1000 of 512 channels 47.7 / 18.7, 2 x 16 x 5021 of 256 31.7 / 23.2, 3 x 8 x 4799 with
+// eight query heads 29.4 / 19.8; step_lone_threads has the rest.
+template <int D, int GQ, int BLK>
+__global__ __launch_bounds__(BLK) void step_lone_kernel(
+    const h1 *q, uint4 *k_cache, const h1 *k_new, uint4 *v_cache, const h1 *v_new, Mask mk, h1 *logits, float *__restrict__ partial,
+    float4 *__restrict__ ml, FtParams kp, FtParams vp, int BH, int H, int T, int n_super_cap, float scaling, Seg ka, Seg va)
+{
+    constexpr int WAVES = BLK / 64, HW = D / 64, UNITS = WAVES / HW;
+    static_assert(WAVES % HW == 0, "whole heads");
+    // a wave's key tile; then its copy of the weights, or its share of those that the waves of a unit write together
+    constexpr int WEIGHTS = GQ == 1 ? 0 : GQ * LONE_SEG * 2 / HW, SLOT = WEIGHTS > LONE_TILE ? WEIGHTS : LONE_TILE;
+    static_assert(SLOT % 16 == 0, "vectors");
+    __shared__ uint4 smem[(LUT_WORDS64 * 8 + WAVES * (SLOT + GQ * LONE_SEG * 4)) / 16];
+    ka.groups = va.groups = 0; // only even plans come here
+    uint2 *lut = reinterpret_cast<uint2 *>(smem);
+    char *lds = reinterpret_cast<char *>(smem) + LUT_WORDS64 * 8;
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    const int u = wave / HW, part = wave % HW, c = part * 64 + lane;
+    const uint32_t lane_copy = (uint32_t)(lane & (LUT_COPIES - 1)) * 8u;
+    int seg, wis;
+    interleave_segment((int)blockIdx.x * UNITS + u, ka.nseg, seg, wis);
+    const bool active = wis < BH;
+    const int bx = min(wis, BH - 1), h = bx % H;
+    float *shares = reinterpret_cast<float *>(lds + WAVES * SLOT) + u * HW * GQ * LONE_SEG;
+    LoneScores<BLK <= 512, GQ, D> scores(lds + wave * SLOT, lane, q + (size_t)bx * GQ * D + part * 64);
+    LoneLoads<D> s;
+    s.start(k_cache, kp, k_new, h, bx, c, seg, T, n_super_cap, ka);
+    lone_fill<BLK>(lut, threadIdx.x);
+    __syncthreads();
+
+    const int t0 = s.t0, ntok = s.t1 - s.t0 + (s.last ? 1 : 0); // the appended token is the last segment's
+    if (active) {
+        Lone st = s.state();
+        float *mine = shares + part * GQ * LONE_SEG;
+        scores.ready(ka.act_bf16);
+        scores.run(lut, lane_copy, st, s, 0, s.nfull, mine);
+        if (s.last)
+            scores.finish(s, st, bx, c, T, nullptr, ka, true, mine + s.nfull * 8);
+        // the values' state and codes travel while the weights are made
+        s.start(v_cache, vp, v_new, h, bx, c, seg, T, n_super_cap, va);
+    }
+    __syncthreads();
+
+    const long row0 = (long)bx * GQ, rows = (long)BH * GQ;
+    h1 *p = reinterpret_cast<h1 *>(lds + (GQ == 1 ? wave : u * HW) * SLOT);
+    if (active) {
+        // one query head: every wave of the unit by itself, no wave waits for another
+        constexpr int EACH = GQ == 1 ? 1 : GQ / HW;
+#pragma unroll
+        for (int i = 0; i < EACH; i++) {
+            const int g = GQ == 1 ? 0 : part * EACH + i;
+            lone_weights<HW>(shares + g * LONE_SEG, GQ * LONE_SEG, logits + (row0 + g) * ka.row_pitch + t0,
+                             mk.of<true>((unsigned)row0 + g, T + 1, t0), ntok, scaling, p + g * LONE_SEG, ml + seg * rows + row0 + g,
+                             lane, GQ > 1 || part == 0);
+        }
+    }
+    if constexpr (GQ > 1)
+        __syncthreads();
+    if (!active)
+        return;
+
+    Lone st = s.state();
+    float *o = partial + (seg * rows + row0) * D + c;
+    if constexpr (GQ == 1 && D != 512) {
+        // measured, adding on the vector pipe / on the matrix cores: 4 x 8 x 8190 of 256 channels 30.4 / 31.3, 8 x 32 x 2000
+        // 28.0 / 29.2, 4 x 32 x 2000 19.6 / 19.3; 8 x 8 x 2000 of 512 30.5 / 28.9
+        float acc = 0.0f;
+        lone_values(lut, lane_copy, s, st, 0, s.nfull, p, acc);
+        lone_values_end(s, st, [&](int t) { return p[t]; }, bx, c, T, nullptr, va, true, acc);
+        *o = acc;
+        return;
+    }
+    constexpr int NB = (GQ + 3) / 4;
+    f4v acc[NB];
+#pragma unroll
+    for (int n = 0; n < NB; n++)
+        acc[n] = (f4v){0.0f, 0.0f, 0.0f, 0.0f};
+    lone_values_grouped<GQ>(lut, lane_copy, s, st, p, lane, acc);
+    if (s.last) {
+        auto token = [&](int t, float v) __attribute__((always_inline)) {
+#pragma unroll
+            for (int g = 0; g < GQ; g++)
+                acc[g >> 2][g & 3] = __builtin_fmaf((float)p[g * LONE_SEG + t], v, acc[g >> 2][g & 3]);
+        };
+#pragma unroll
+        for (int t = 0; t < 7; t++)
+            if (t < s.ntail)
+                token(8 * s.nfull + t, (float)lone_token(st, (int)(s.tail >> (4 * t) & 15) - 8));
+        token(T - t0, (float)lone_append(s, st, bx, c, T, nullptr, va, true));
+    }
+#pragma unroll
+    for (int g = 0; g < GQ; g++)
+        o[g * D] = acc[g >> 2][g & 3];
+}
+
 // The segments of a row put together, by waves of two kinds: 512 of its weights each, or a share of its
 // outputs: all 128 channels in two groups of segments, or, with many segments, 16 channels in 16 groups.
 // Sums are taken in a fixed order.

@@ -36,7 +36,7 @@ __global__ __launch_bounds__(512) void small_step_kernel(
     const bool works = seg < ka.nseg;
     const uint32_t lane_copy = (uint32_t)(lane & (LUT_COPIES - 1)) * 8u;
     LoneScores<true> scores(mine, lane, q + (size_t)bx * D + half * 64);
-    LoneLoads s;
+    LoneLoads<> s;
     s.start(k_cache, kp, k_new, h, bx, c, works ? seg : 0, T, n_super_cap, ka);
     lone_fill<512>(lut, threadIdx.x);
     __syncthreads();

@@ -1,0 +1,36 @@
+"""Steps in two launches with one channel per lane (a KV head over two, four or eight waves): its workgroup sizes and the
+sizes just beyond it, and the ends of supergroups, tiles and groups of tiles."""
+import pytest
+import torch
+
+from tests.test_gpu_segment_step import test_against_the_three_calls, test_masked_segments_and_rows
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("B,Hq,H,D,T,S", [
+    (4, 32, 32, 128, 1300, 256), (5, 32, 32, 128, 1800, 256), (6, 32, 32, 128, 2041, 256),                # 4, 12 waves, beyond
+    (4, 32, 16, 128, 1500, 256), (8, 32, 16, 128, 1793, 256), (9, 32, 16, 128, 2047, 256), (13, 32, 16, 128, 2047, 256),
+    (2, 32, 8, 128, 6000, 256), (3, 32, 8, 128, 9001, 256), (6, 32, 8, 128, 7680, 256),                   # 4, 8, 12 waves
+    (3, 64, 8, 128, 4799, 256), (5, 64, 8, 128, 5632, 256), (9, 64, 8, 128, 3800, 256),                   # 4, 8 waves, beyond
+    (2, 16, 16, 256, 3900, 256), (2, 16, 16, 256, 5021, 256), (4, 8, 8, 256, 7171, 256), (5, 8, 8, 256, 7170, 256),
+    (1, 8, 8, 512, 3333, 256), (3, 8, 8, 512, 3584, 256), (10, 8, 8, 512, 1799, 256),
+])
+def test_workgroup_sizes(gpu, oracle, B, Hq, H, D, T, S):
+    test_against_the_three_calls(gpu, oracle, B, Hq, H, D, T, 4, S, torch.float16)
+
+
+@pytest.mark.parametrize("Hq,H,D", [(2, 2, 256), (3, 3, 512), (4, 2, 128), (4, 1, 128), (8, 1, 128)])
+@pytest.mark.parametrize("T,S", [(0, 0), (1, 0), (7, 0), (8, 256), (63, 0), (72, 256), (80, 256), (129, 0), (255, 256), (256, 0),
+                                 (257, 256), (264, 256), (281, 256), (330, 256), (512, 256), (200, 64)])
+def test_ends_of_segments(gpu, oracle, Hq, H, D, T, S):
+    """No supergroup, a half tile, a tile, a group of four and one more; 256 tokens and the appended one; segments of 64."""
+    if S == 64 and Hq == H:
+        pytest.skip("segments below 128 tokens of one query head per KV head keep the separate launches")
+    test_against_the_three_calls(gpu, oracle, 2, Hq, H, D, T, 4, S, torch.bfloat16)
+
+
+@pytest.mark.parametrize("low", [torch.finfo(torch.float32).min, float("-inf")])
+@pytest.mark.parametrize("Hq,H,D", [(4, 4, 512), (8, 1, 128), (4, 2, 128)])
+def test_masks(gpu, Hq, H, D, low):
+    test_masked_segments_and_rows(gpu, 3, Hq, H, D, 768, low)
