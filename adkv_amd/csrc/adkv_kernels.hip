@@ -4041,8 +4041,11 @@ int adkv_decode_step(const void *q, void *k_cache, void *v_cache, const void *k_
                 if ((rc = stage_mark(i, stream)))
                     return rc;
             const int out_waves = ka.nseg > 16 ? D / 16 : D / 128;
-            const long waves = rows * ((T + 1 + 511) / 512 + out_waves);
-            hipLaunchKernelGGL(step_combine_kernel, dim3((unsigned)((waves + 3) / 4)), dim3(256), 0, (hipStream_t)stream,
+            // two vectors of weights per lane where one would give more waves than the device holds at once
+            const int vecs = rows * ((T + 1 + 511) / 512 + out_waves) > 32L * cus() ? 2 : 1;
+            const long waves = rows * ((T + 1 + 512 * vecs - 1) / (512 * vecs) + out_waves);
+            const auto combine = vecs == 2 ? step_combine_kernel<2> : step_combine_kernel<1>;
+            hipLaunchKernelGGL(combine, dim3((unsigned)((waves + 3) / 4)), dim3(256), 0, (hipStream_t)stream,
                                (const h1 *)logits, (h1 *)weights, (h1 *)out, mk, partial, ml, rows, T + 1, (long)ld, D, ka.nseg,
                                scaling, out_waves, act_bf16);
             return (rc = check_launch()) ? rc : stage_mark(3, stream);
