@@ -2959,15 +2959,17 @@ static int launch_step_grouped(int GQ, long waves, hipStream_t st, Args... args)
 // 20.7 / 15.7, 4 x 32 x 2000 (8) 21.3 / 19.5, 6 x 32 x 2000 (12) 27.3 / 24.1, 8 x 32 x 2000 (16) 27.4 / 28.0; two query heads, 4 x 16
 // x 2000 (4) 22.6 / 16.3, 8 x 16 x 2000 (8) 23.3 / 20.3, 12 x 16 x 2000 (12) 30.0 / 25.6, 16 x 16 x 2000 (16) 31.1 / 30.7; four, 1 x 8
 // x 603 22.2 / 15.3, 28 x 8 x 936 (7) 24.5 / 21.3, 8 x 8 x 6000 (12) 33.5 / 28.4, 8 x 8 x 7000 (14) 34.1 / 46; eight, 3 x 8 x
-// 113 18.9 / 13.7, 3 x 8 x 4799 (4) 29.4 / 19.8, 8 x 8 x 4000 (8) 35.1 / 29.4, 8 x 8 x 8000 (16) 45.4 / 46.1.
+// 113 18.9 / 13.7, 3 x 8 x 4799 (4) 29.4 / 19.8, 8 x 8 x 4000 (8) 35.1 / 29.4, 8 x 8 x 8000 (16) 45.4 / 46.1.  2-bit codes:
+// 1 x 32 x 2000 20.1 / 13.8, 6 x 32 x 2000 26.1 / 21.8, 12 x 16 x 2000 27.7 / 22.9, 2 x 8 x 8664 22.9 / 20.6, 8 x 8 x 6000 30.9 / 26.6, 8 x 8
+// x 4000 with eight 31.0 / 26.1.
 // Small workgroups spread best; what they leave free of a CU's LDS (the table takes 64 KB) holds a second one only with
 // one query head.  A workgroup of as many waves as the CU is to hold otherwise: 2 x 16 x 5021 of 256 channels with 4, 8, 12
 // and 16 waves 26.5, 32.6, 23.3, 27.4; 28 x 8 x 936 with four query heads 28.1, 21.3, 25.4.
-static int step_lone_threads(long units, int D, int GQ, int bits, int longest)
+static int step_lone_threads(long units, int D, int GQ, int longest)
 {
     const long per_cu = (units * (D / 64) + cus() - 1) / cus();
     const int most = GQ == 8 ? 8 : D == 128 ? 12 : 16;
-    if (bits != 4 || longest > 256 || per_cu > most)
+    if (longest > 256 || per_cu > most)
         return 0;
     if (D == 512)
         return per_cu <= 8 ? 512 : 1024;
@@ -2976,12 +2978,12 @@ static int step_lone_threads(long units, int D, int GQ, int bits, int longest)
     return per_cu <= 8 ? 512 : per_cu <= 12 ? 768 : 1024;
 }
 
-template <int D, int GQ, typename... Args>
+template <int D, int BITS, int GQ, typename... Args>
 static int launch_step_lone(int blk, long units, hipStream_t st, Args... args)
 {
     const int per_block = blk / D; // units: a wave per 64 channels
     const dim3 grid((unsigned)((units + per_block - 1) / per_block));
-#define ADKV_STEP(BLK) hipLaunchKernelGGL((step_lone_kernel<D, GQ, BLK>), grid, dim3(BLK), 0, st, args...)
+#define ADKV_STEP(BLK) hipLaunchKernelGGL((step_lone_kernel<D, BITS, GQ, BLK>), grid, dim3(BLK), 0, st, args...)
     if constexpr (D != 512) {
         if (blk == 256)
             ADKV_STEP(256);
@@ -3002,21 +3004,28 @@ static int launch_step_lone(int blk, long units, hipStream_t st, Args... args)
     return check_launch();
 }
 
+template <int BITS, typename... Args>
+static int launch_step_lone_grouped(int GQ, int blk, long units, hipStream_t st, Args... args)
+{
+    switch (GQ) {
+    case 1: return launch_step_lone<128, BITS, 1>(blk, units, st, args...);
+    case 2: return launch_step_lone<128, BITS, 2>(blk, units, st, args...);
+    case 4: return launch_step_lone<128, BITS, 4>(blk, units, st, args...);
+    default: return launch_step_lone<128, BITS, 8>(blk, units, st, args...);
+    }
+}
+
 template <typename... Args>
 static int launch_step_segments(int cpl, int GQ, int bits, int D, int BH, int nseg, int longest, hipStream_t st, Args... args)
 {
     const long units = padded_units<64>(BH, nseg);
-    if (const int blk = step_lone_threads(units, D, GQ, bits, longest)) {
+    if (const int blk = step_lone_threads(units, D, GQ, longest)) {
         if (D == 512)
-            return launch_step_lone<512, 1>(blk, units, st, args...);
+            return launch_step_lone<512, 4, 1>(blk, units, st, args...);
         if (D == 256)
-            return launch_step_lone<256, 1>(blk, units, st, args...);
-        switch (GQ) {
-        case 1: return launch_step_lone<128, 1>(blk, units, st, args...);
-        case 2: return launch_step_lone<128, 2>(blk, units, st, args...);
-        case 4: return launch_step_lone<128, 4>(blk, units, st, args...);
-        default: return launch_step_lone<128, 8>(blk, units, st, args...);
-        }
+            return launch_step_lone<256, 4, 1>(blk, units, st, args...);
+        return bits == 4 ? launch_step_lone_grouped<4>(GQ, blk, units, st, args...)
+                         : launch_step_lone_grouped<2>(GQ, blk, units, st, args...);
     }
     if (D == 512)
         return launch_step_shape<512, 8, 4, 1>(units, st, args...);

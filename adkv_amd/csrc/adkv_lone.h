@@ -10,7 +10,7 @@
 
 namespace adkv {
 
-constexpr int LONE_PF = 8;          // supergroups of codes in flight
+constexpr int LONE_PF = 8;          // units of eight tokens whose codes are in flight
 constexpr int LONE_TILE = 64 * 32;  // bytes of a wave's key tile: 64 channels x 16 tokens
 constexpr int LONE_SEG = 264;       // tokens of a segment of a step, and one vector behind them
 constexpr int LONE_CHUNK = 512;     // tokens between two exchanges of partial logits
@@ -31,9 +31,9 @@ struct LoneUnit {
 };
 
 // See SegLoads; also the word that the appended token goes to and the token itself.
-template <int D = 128>
+template <int D = 128, int BITS = 4>
 struct LoneLoads {
-    static constexpr int HEAD = D;
+    static constexpr int TPW = Code<BITS>::TPW, UPS = TPW / 8, PF = LONE_PF / UPS; // units, words of codes in flight
     uint32_t *cbh;      // this head, this channel
     // this segment's whole supergroups: reads past them are dropped, and a load takes no address arithmetic (with a
     // clamped index it was five instructions)
@@ -42,7 +42,7 @@ struct LoneLoads {
     int t0, t1, nfull, ntail;
     bool last, from_ckpt;
     h1 zp, sc, al, be, tg;
-    uint32_t ck, tail, buf[LONE_PF];
+    uint32_t ck, tail, buf[PF];
     uint16_t fresh;
 
     __device__ __forceinline__ void start(void *cache, const FtParams &p, const h1 *x_new, int h, int bx, int c, int seg, int T,
@@ -52,10 +52,10 @@ struct LoneLoads {
         last = seg_is_last(sa, seg);
         t0 = iv * sa.ckpt_interval;
         t1 = last ? T : seg_end(sa, seg);
-        nfull = (t1 - t0) >> 3;
-        ntail = (t1 - t0) & 7; // of the last segment only: the others are whole intervals
+        nfull = (unsigned)(t1 - t0) / TPW;
+        ntail = (unsigned)(t1 - t0) % TPW; // of the last segment only: the others are whole intervals
         cbh = reinterpret_cast<uint32_t *>(cache) + (size_t)bx * n_super_cap * D + c;
-        codes = __builtin_amdgcn_make_buffer_rsrc(cbh - c + (size_t)(t0 >> 3) * D, 0, nfull * D * 4, 0x00027000);
+        codes = __builtin_amdgcn_make_buffer_rsrc(cbh - c + (size_t)((unsigned)t0 / TPW) * D, 0, nfull * D * 4, 0x00027000);
         lane4 = c * 4;
         from_ckpt = iv > 0;
         ck = 0;
@@ -67,16 +67,23 @@ struct LoneLoads {
         be = p.be[pi];
         tg = p.tg[pi];
 #pragma unroll
-        for (int i = 0; i < LONE_PF; i++)
+        for (int i = 0; i < PF; i++)
             buf[i] = load(0, i);
-        tail = cbh[(size_t)(last ? T >> 3 : 0) * D];
+        tail = cbh[(size_t)(last ? (unsigned)T / TPW : 0) * D];
         fresh = reinterpret_cast<const uint16_t *>(x_new)[(size_t)bx * D + c];
     }
-    // supergroup sg + i, i < LONE_PF; read once: not kept in the caches
+    // supergroup sg + i, i < PF; read once: not kept in the caches
     __device__ __forceinline__ uint32_t load(int sg, int i) const
     {
         return __builtin_amdgcn_raw_buffer_load_b32(codes, lane4 + i * D * 4, sg * D * 4, 2);
     }
+    // behind unit i of LONE_PF (at that unit of `first` on): the word that it was the last of, PF words further
+    __device__ __forceinline__ void refill(int first, int i)
+    {
+        if (i % UPS == UPS - 1)
+            buf[i / UPS] = load((unsigned)first / UPS + PF, i / UPS);
+    }
+    __device__ __forceinline__ int code(int t) const { return (int)(tail >> (BITS * t) & Code<BITS>::FIELD) + Code<BITS>::QLO; }
     __device__ __forceinline__ Lone state() const
     {
         const h2 s = from_ckpt ? as_h2(ck) : (h2){zp, sc};
@@ -91,17 +98,43 @@ struct LoneLoads {
     }
 };
 
-__device__ __forceinline__ void lone_lookup(uint2 *e, const uint2 *lut, uint32_t word, uint32_t lane_copy)
+// The entries of unit i of the words in flight, two tokens each; with 2-bit codes a byte of a word is four tokens and
+// an LDS read returns two entries.
+template <int BITS>
+__device__ __forceinline__ void lone_lookup(uint2 *e, const uint2 *lut, const uint32_t *buf, int i, uint32_t lane_copy)
 {
+    if constexpr (BITS == 4) {
 #pragma unroll
-    for (int k = 0; k < 4; k++)
-        e[k] = lut_get(lut, word, lane_copy, k);
+        for (int k = 0; k < 4; k++)
+            e[k] = lut_get(lut, buf[i], lane_copy, k);
+    } else {
+#pragma unroll
+        for (int k = 0; k < 2; k++) {
+            const uint4 v = lut2_get(lut, buf[i / 2], lane_copy, i % 2 * 2 + k);
+            e[2 * k] = make_uint2(v.x, v.y);
+            e[2 * k + 1] = make_uint2(v.z, v.w);
+        }
+    }
+}
+// The table for them (see lone_fill for 4 bits): 16 copies of 16-byte entries.
+template <int NT>
+__device__ __forceinline__ void lone_fill2(uint2 *lut, int tid)
+{
+    uint4 *l4 = reinterpret_cast<uint4 *>(lut);
+#pragma unroll
+    for (int i = 0; i < LUT_ENTRIES * LUT2_COPIES; i += NT) {
+        if (LUT_ENTRIES * LUT2_COPIES % NT != 0 && i + tid >= LUT_ENTRIES * LUT2_COPIES)
+            break;
+        const int b = (i + tid) / LUT2_COPIES;
+        const auto entry = [](int code) { return as_u32(splat((h1)(code - 2))) & 0x7FFFFFFFu; };
+        l4[i + tid] = make_uint4(entry(b & 3), entry(b >> 2 & 3), entry(b >> 4 & 3), entry(b >> 6));
+    }
 }
 
 // The last segment's end: hands out the state after token T - 1, records it where token T opens an interval,
 // quantises token T into its word (gemv.cu:744-798, 1105-1157) and returns its value r16(q*sc + zp).
-template <int D>
-__device__ __forceinline__ h1 lone_append(const LoneLoads<D> &s, const Lone &st, int bx, int c, int T, h1 *state_out, const Seg &sa,
+template <int D, int BITS>
+__device__ __forceinline__ h1 lone_append(const LoneLoads<D, BITS> &s, const Lone &st, int bx, int c, int T, h1 *state_out, const Seg &sa,
                                           bool active)
 {
     const uint32_t zs = as_u32((h2){lone_zp(st), lone_sc(st)});
@@ -113,10 +146,10 @@ __device__ __forceinline__ h1 lone_append(const LoneLoads<D> &s, const Lone &st,
             *reinterpret_cast<uint32_t *>(sa.ckpt + (((size_t)bx * sa.n_ckpt_cap + j) * D + c) * 2) = zs;
     }
     const h1 x = act2(s.fresh, sa.act_bf16).x;
-    const int q = quantize<4>(x, lone_zp(st), lone_sc(st));
-    const int sh = 4 * s.ntail;
+    const int q = quantize<BITS>(x, lone_zp(st), lone_sc(st));
+    const int sh = BITS * s.ntail;
     if (active)
-        s.cbh[(size_t)(T >> 3) * D] = (s.tail & ~(0xFu << sh)) | ((uint32_t)(q + 8) << sh);
+        s.cbh[(size_t)((unsigned)T / Code<BITS>::TPW) * D] = (s.tail & ~(Code<BITS>::FIELD << sh)) | ((uint32_t)(q - Code<BITS>::QLO) << sh);
     return __builtin_fmaf16((h1)q, lone_sc(st), lone_zp(st));
 }
 
@@ -128,7 +161,7 @@ __device__ __forceinline__ h1 lone_append(const LoneLoads<D> &s, const Lone &st,
 // GQ: query heads per KV head.  Row r of the product is head r * GQ / 16, so that a lane has the share of its token and of the
 // head of its quarter (of two heads with eight): a store per tile where a single head's columns are collected first.
 // The tile's 16-byte pieces change places with every fourth channel, so that eight lanes' writes spread over the banks.
-template <bool ACC, int GQ = 1, int D = 128>
+template <bool ACC, int GQ = 1, int D = 128, int BITS = 4>
 struct LoneScores {
     char *tile;
     int lane, wr[2], rd[2];
@@ -212,20 +245,20 @@ struct LoneScores {
         }
     }
 
-    // supergroups sg0 .. sg0 + n of the segment, sg0 a multiple of LONE_PF; the shares of their logits to part[0..8n)
-    __device__ __forceinline__ void run(const uint2 *lut, uint32_t lane_copy, Lone &st, LoneLoads<D> &s, int sg0, int n, float *part)
+    // units sg0 .. sg0 + n of the segment, sg0 a multiple of LONE_PF; the shares of their logits to part[0..8n)
+    __device__ __forceinline__ void run(const uint2 *lut, uint32_t lane_copy, Lone &st, LoneLoads<D, BITS> &s, int sg0, int n, float *part)
     {
         if (n <= 0)
             return;
         uint2 e[2][4];
-        lone_lookup(e[0], lut, s.buf[0], lane_copy);
+        lone_lookup<BITS>(e[0], lut, s.buf, 0, lane_copy);
         wait_lgkm();
         // tile i / 2 of a group of eight supergroups is written after its two, fetched with the second, multiplied
         // half a tile later and kept another half later
         auto body = [&](int sg, auto ic, auto &&group_done) __attribute__((always_inline)) {
             constexpr int i = decltype(ic)::value;
-            lone_lookup(e[(i & 1) ^ 1], lut, s.buf[(i + 1) % LONE_PF], lane_copy); // stale past the end: looked up, never used
-            s.buf[i] = s.load(sg0 + sg - i + LONE_PF, i);
+            lone_lookup<BITS>(e[(i & 1) ^ 1], lut, s.buf, (i + 1) % LONE_PF, lane_copy); // stale past the end: looked up, never used
+            s.refill(sg0 + sg - i, i);
             __builtin_amdgcn_sched_barrier(0);
             uint32_t x[4];
             lone_eight(st, e[i & 1], x);
@@ -282,10 +315,12 @@ struct LoneScores {
         if (lane < 8 * n - base)
             part[base + lane] = hold;
     }
-    // up to eight tokens by themselves
+    // up to eight tokens by themselves, sixteen with 2-bit codes
     __device__ __forceinline__ void few(const uint32_t *x, int ntok, float *part)
     {
         write(0, x);
+        if constexpr (BITS == 2)
+            write(1, x + 4);
         fetch();
         multiply();
         if constexpr (GQ > 1) {
@@ -297,27 +332,30 @@ struct LoneScores {
             part[lane] = hold;
     }
     // the last segment's ragged tail and the appended token; their shares of the logits to part[0..ntail]
-    __device__ __forceinline__ void finish(const LoneLoads<D> &s, Lone &st, int bx, int c, int T, h1 *state_out, const Seg &sa, bool active,
+    __device__ __forceinline__ void finish(const LoneLoads<D, BITS> &s, Lone &st, int bx, int c, int T, h1 *state_out, const Seg &sa, bool active,
                                            float *part)
     {
-        uint32_t v[8] = {0, 0, 0, 0, 0, 0, 0, 0};
+        constexpr int TPW = Code<BITS>::TPW;
+        uint32_t v[TPW] = {}, x[TPW / 2];
 #pragma unroll
-        for (int t = 0; t < 7; t++)
+        for (int t = 0; t < TPW - 1; t++)
             if (t < s.ntail)
-                v[t] = __builtin_bit_cast(uint16_t, lone_token(st, (int)(s.tail >> (4 * t) & 15) - 8));
+                v[t] = __builtin_bit_cast(uint16_t, lone_token(st, s.code(t)));
         const uint32_t self = __builtin_bit_cast(uint16_t, lone_append(s, st, bx, c, T, state_out, sa, active));
 #pragma unroll
-        for (int t = 0; t < 8; t++)
+        for (int t = 0; t < TPW; t++)
             v[t] = t == s.ntail ? self : v[t];
-        const uint32_t x[4] = {v[0] | v[1] << 16, v[2] | v[3] << 16, v[4] | v[5] << 16, v[6] | v[7] << 16};
+#pragma unroll
+        for (int k = 0; k < TPW / 2; k++)
+            x[k] = v[2 * k] | v[2 * k + 1] << 16;
         few(x, s.ntail + 1, part);
     }
 };
 
-// forward_ov of a wave's 64 channels: adds supergroups sg0 .. sg0 + n of the segment to acc, sg0 a multiple of
+// forward_ov of a wave's 64 channels: adds units sg0 .. sg0 + n of the segment to acc, sg0 a multiple of
 // LONE_PF.  w: their weights, in LDS.
-template <int D>
-__device__ __forceinline__ void lone_values(const uint2 *lut, uint32_t lane_copy, LoneLoads<D> &s, Lone &st, int sg0, int n, const h1 *w,
+template <int D, int BITS>
+__device__ __forceinline__ void lone_values(const uint2 *lut, uint32_t lane_copy, LoneLoads<D, BITS> &s, Lone &st, int sg0, int n, const h1 *w,
                                             float &acc)
 {
     if (n <= 0)
@@ -325,38 +363,38 @@ __device__ __forceinline__ void lone_values(const uint2 *lut, uint32_t lane_copy
     const uint4 *w4 = reinterpret_cast<const uint4 *>(w);
     uint2 e[2][4];
     uint4 wv[2];
-    lone_lookup(e[0], lut, s.buf[0], lane_copy);
+    lone_lookup<BITS>(e[0], lut, s.buf, 0, lane_copy);
     wv[0] = w4[0];
     wait_lgkm();
     rotate_over<LONE_PF>(n, [&](int sg, auto ic) __attribute__((always_inline)) {
         constexpr int i = decltype(ic)::value, half = i & 1;
-        lone_lookup(e[half ^ 1], lut, s.buf[(i + 1) % LONE_PF], lane_copy); // stale past the end: looked up, never used
+        lone_lookup<BITS>(e[half ^ 1], lut, s.buf, (i + 1) % LONE_PF, lane_copy); // stale past the end: looked up, never used
         wv[half ^ 1] = w4[sg + 1]; // so are these: the caller's LDS goes on behind them
-        s.buf[i] = s.load(sg0 + sg - i + LONE_PF, i);
+        s.refill(sg0 + sg - i, i);
         __builtin_amdgcn_sched_barrier(0);
         lone_eight_weighted(st, e[half], wv[half], acc);
         __builtin_amdgcn_sched_barrier(0);
     });
 }
 // The last segment's ragged tail and the appended token.  w1(t): the weight of the segment's token t.
-template <int D, typename W1>
-__device__ __forceinline__ void lone_values_end(const LoneLoads<D> &s, Lone &st, W1 &&w1, int bx, int c, int T, h1 *state_out, const Seg &sa,
+template <int D, int BITS, typename W1>
+__device__ __forceinline__ void lone_values_end(const LoneLoads<D, BITS> &s, Lone &st, W1 &&w1, int bx, int c, int T, h1 *state_out, const Seg &sa,
                                                 bool active, float &acc)
 {
     if (!s.last)
         return;
 #pragma unroll
-    for (int t = 0; t < 7; t++)
+    for (int t = 0; t < s.TPW - 1; t++)
         if (t < s.ntail)
-            acc = __builtin_fmaf((float)w1(8 * s.nfull + t), (float)lone_token(st, (int)(s.tail >> (4 * t) & 15) - 8), acc);
+            acc = __builtin_fmaf((float)w1(s.TPW * s.nfull + t), (float)lone_token(st, s.code(t)), acc);
     acc = __builtin_fmaf((float)w1(T - s.t0), (float)lone_append(s, st, bx, c, T, state_out, sa, active), acc);
 }
 
 // The same for GQ query heads: the values of four tokens of a lane's channel are a column for the matrix cores as
 // they are, the weights of the query heads the rows (see ov_gqa_segment); element i of acc[n] is head 4n + i.
 // w: a row of LONE_SEG weights per head.
-template <int GQ, int D>
-__device__ __forceinline__ void lone_values_grouped(const uint2 *lut, uint32_t lane_copy, LoneLoads<D> &s, Lone &st, const h1 *w, int lane,
+template <int GQ, int D, int BITS>
+__device__ __forceinline__ void lone_values_grouped(const uint2 *lut, uint32_t lane_copy, LoneLoads<D, BITS> &s, Lone &st, const h1 *w, int lane,
                                                     f4v *acc)
 {
     constexpr int NB = (GQ + 3) / 4;
@@ -365,20 +403,20 @@ __device__ __forceinline__ void lone_values_grouped(const uint2 *lut, uint32_t l
     const uint4 *w4[NB];
     uint2 e[2][4];
     uint4 wv[2][NB];
-    lone_lookup(e[0], lut, s.buf[0], lane_copy);
+    lone_lookup<BITS>(e[0], lut, s.buf, 0, lane_copy);
 #pragma unroll
     for (int n = 0; n < NB; n++) {
         w4[n] = reinterpret_cast<const uint4 *>(w + min(4 * n + (lane & 3), GQ - 1) * LONE_SEG);
         wv[0][n] = w4[n][0];
     }
     wait_lgkm();
-    rotate_over<LONE_PF>(s.nfull, [&](int sg, auto ic) __attribute__((always_inline)) {
+    rotate_over<LONE_PF>(s.nfull * s.UPS, [&](int sg, auto ic) __attribute__((always_inline)) {
         constexpr int i = decltype(ic)::value, half = i & 1;
-        lone_lookup(e[half ^ 1], lut, s.buf[(i + 1) % LONE_PF], lane_copy); // stale past the end: looked up, never used
+        lone_lookup<BITS>(e[half ^ 1], lut, s.buf, (i + 1) % LONE_PF, lane_copy); // stale past the end: looked up, never used
 #pragma unroll
         for (int n = 0; n < NB; n++)
             wv[half ^ 1][n] = w4[n][sg + 1]; // so are these: a row goes on for a vector
-        s.buf[i] = s.load(sg - i + LONE_PF, i);
+        s.refill(sg - i, i);
         __builtin_amdgcn_sched_barrier(0);
         uint32_t x[4];
         lone_eight(st, e[half], x);

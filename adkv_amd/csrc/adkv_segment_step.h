@@ -295,15 +295,14 @@ __device__ __forceinline__ void lone_weights(const float *share, int stride, h1 
         *ml = make_float4(mx, sum, rounded, 0.0f);
 }
 
-// The same launch with one channel per lane, a KV head over D / 64 waves (adkv_lone.h): 4-bit codes, segments of at
-// most 256 tokens.  With few waves per SIMD a step takes as long as one wave's instructions per token, and a lane with
+// The same launch with one channel per lane, a KV head over D / 64 waves (adkv_lone.h): segments of at most 256 tokens.  With few waves per SIMD a step takes as long as one wave's instructions per token, and a lane with
 // four or eight channels has two and four times as many of them; the waves of a head meet once, behind the keys, where
 // each has left its share of the logits (fp32) in the LDS, and with several query heads again behind the weights.
 // Of the 256 + 256 tokens of a full segment a lone wave takes some 9 us (19 ns per token, step_segments_kernel 27 with two
 // channels per lane, 50 with four and 90 with eight); from four waves per SIMD on vector issue holds it, 23 cycles per
 // wave and token.  us per step: 2 x 8 heads x 1000 of 512 channels 47.7 / 18.7, 2 x 16 x 5021 of 256 31.7 / 23.2, 3 x 8 x 4799 with
 // eight query heads 29.4 / 19.8; step_lone_threads has the rest.
-template <int D, int GQ, int BLK>
+template <int D, int BITS, int GQ, int BLK>
 __global__ __launch_bounds__(BLK) void step_lone_kernel(
     const h1 *q, uint4 *k_cache, const h1 *k_new, uint4 *v_cache, const h1 *v_new, Mask mk, h1 *logits, float *__restrict__ partial,
     float4 *__restrict__ ml, FtParams kp, FtParams vp, int BH, int H, int T, int n_super_cap, float scaling, Seg ka, Seg va)
@@ -319,16 +318,19 @@ __global__ __launch_bounds__(BLK) void step_lone_kernel(
     char *lds = reinterpret_cast<char *>(smem) + LUT_WORDS64 * 8;
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
     const int u = wave / HW, part = wave % HW, c = part * 64 + lane;
-    const uint32_t lane_copy = (uint32_t)(lane & (LUT_COPIES - 1)) * 8u;
+    const uint32_t lane_copy = table_lane_offset<BITS>(lane);
     int seg, wis;
     interleave_segment((int)blockIdx.x * UNITS + u, ka.nseg, seg, wis);
     const bool active = wis < BH;
     const int bx = min(wis, BH - 1), h = bx % H;
     float *shares = reinterpret_cast<float *>(lds + WAVES * SLOT) + u * HW * GQ * LONE_SEG;
-    LoneScores<BLK <= 512, GQ, D> scores(lds + wave * SLOT, lane, q + (size_t)bx * GQ * D + part * 64);
-    LoneLoads<D> s;
+    LoneScores<BLK <= 512, GQ, D, BITS> scores(lds + wave * SLOT, lane, q + (size_t)bx * GQ * D + part * 64);
+    LoneLoads<D, BITS> s;
     s.start(k_cache, kp, k_new, h, bx, c, seg, T, n_super_cap, ka);
-    lone_fill<BLK>(lut, threadIdx.x);
+    if constexpr (BITS == 4)
+        lone_fill<BLK>(lut, threadIdx.x);
+    else
+        lone_fill2<BLK>(lut, threadIdx.x);
     __syncthreads();
 
     const int t0 = s.t0, ntok = s.t1 - s.t0 + (s.last ? 1 : 0); // the appended token is the last segment's
@@ -336,9 +338,9 @@ __global__ __launch_bounds__(BLK) void step_lone_kernel(
         Lone st = s.state();
         float *mine = shares + part * GQ * LONE_SEG;
         scores.ready(ka.act_bf16);
-        scores.run(lut, lane_copy, st, s, 0, s.nfull, mine);
+        scores.run(lut, lane_copy, st, s, 0, s.nfull * s.UPS, mine);
         if (s.last)
-            scores.finish(s, st, bx, c, T, nullptr, ka, true, mine + s.nfull * 8);
+            scores.finish(s, st, bx, c, T, nullptr, ka, true, mine + s.nfull * s.TPW);
         // the values' state and codes travel while the weights are made
         s.start(v_cache, vp, v_new, h, bx, c, seg, T, n_super_cap, va);
     }
@@ -368,7 +370,7 @@ __global__ __launch_bounds__(BLK) void step_lone_kernel(
         // measured, adding on the vector pipe / on the matrix cores: 4 x 8 x 8190 of 256 channels 30.4 / 31.3, 8 x 32 x 2000
         // 28.0 / 29.2, 4 x 32 x 2000 19.6 / 19.3; 8 x 8 x 2000 of 512 30.5 / 28.9
         float acc = 0.0f;
-        lone_values(lut, lane_copy, s, st, 0, s.nfull, p, acc);
+        lone_values(lut, lane_copy, s, st, 0, s.nfull * s.UPS, p, acc);
         lone_values_end(s, st, [&](int t) { return p[t]; }, bx, c, T, nullptr, va, true, acc);
         *o = acc;
         return;
@@ -386,9 +388,9 @@ __global__ __launch_bounds__(BLK) void step_lone_kernel(
                 acc[g >> 2][g & 3] = __builtin_fmaf((float)p[g * LONE_SEG + t], v, acc[g >> 2][g & 3]);
         };
 #pragma unroll
-        for (int t = 0; t < 7; t++)
+        for (int t = 0; t < s.TPW - 1; t++)
             if (t < s.ntail)
-                token(8 * s.nfull + t, (float)lone_token(st, (int)(s.tail >> (4 * t) & 15) - 8));
+                token(s.TPW * s.nfull + t, (float)lone_token(st, s.code(t)));
         token(T - t0, (float)lone_append(s, st, bx, c, T, nullptr, va, true));
     }
 #pragma unroll

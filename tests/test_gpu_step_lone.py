@@ -30,6 +30,20 @@ def test_ends_of_segments(gpu, oracle, Hq, H, D, T, S):
     test_against_the_three_calls(gpu, oracle, 2, Hq, H, D, T, 4, S, torch.bfloat16)
 
 
+@pytest.mark.parametrize("Hq,H", [(2, 2), (4, 2), (4, 1), (8, 1)])
+@pytest.mark.parametrize("T,S", [(0, 0), (1, 0), (15, 0), (16, 256), (17, 0), (40, 0), (144, 256), (255, 256), (256, 0), (257, 256),
+                                 (271, 256), (272, 256), (330, 256), (512, 256), (200, 64)])
+def test_two_bits(gpu, oracle, Hq, H, T, S):
+    """A word of codes is a whole tile: no word, ragged ones of one to fifteen tokens, an odd and an even number of them."""
+    test_against_the_three_calls(gpu, oracle, 2, Hq, H, 128, T, 2, S, torch.float16)
+
+
+@pytest.mark.parametrize("B,Hq,H,T", [(4, 32, 32, 1300), (6, 32, 32, 1900), (8, 32, 16, 1793), (12, 32, 16, 1800), (3, 32, 8, 9001),
+                                      (6, 32, 8, 7680), (2, 64, 8, 4000), (5, 64, 8, 5632), (8, 64, 8, 8000)])
+def test_two_bits_workgroup_sizes(gpu, oracle, B, Hq, H, T):
+    test_against_the_three_calls(gpu, oracle, B, Hq, H, 128, T, 2, 256, torch.bfloat16)
+
+
 @pytest.mark.parametrize("low", [torch.finfo(torch.float32).min, float("-inf")])
 @pytest.mark.parametrize("Hq,H,D", [(4, 4, 512), (8, 1, 128), (4, 2, 128)])
 def test_masks(gpu, Hq, H, D, low):
