@@ -34,6 +34,7 @@ struct LoneUnit {
 template <int D = 128, int BITS = 4>
 struct LoneLoads {
     static constexpr int TPW = Code<BITS>::TPW, UPS = TPW / 8, PF = LONE_PF / UPS; // units, words of codes in flight
+    static constexpr int SHIFT = BITS == 4 ? 3 : 4;                                // of tokens to words
     uint32_t *cbh;      // this head, this channel
     // this segment's whole supergroups: reads past them are dropped, and a load takes no address arithmetic (with a
     // clamped index it was five instructions)
@@ -52,10 +53,10 @@ struct LoneLoads {
         last = seg_is_last(sa, seg);
         t0 = iv * sa.ckpt_interval;
         t1 = last ? T : seg_end(sa, seg);
-        nfull = (unsigned)(t1 - t0) / TPW;
-        ntail = (unsigned)(t1 - t0) % TPW; // of the last segment only: the others are whole intervals
+        nfull = (t1 - t0) >> SHIFT;
+        ntail = (t1 - t0) & (TPW - 1); // of the last segment only: the others are whole intervals
         cbh = reinterpret_cast<uint32_t *>(cache) + (size_t)bx * n_super_cap * D + c;
-        codes = __builtin_amdgcn_make_buffer_rsrc(cbh - c + (size_t)((unsigned)t0 / TPW) * D, 0, nfull * D * 4, 0x00027000);
+        codes = __builtin_amdgcn_make_buffer_rsrc(cbh - c + (size_t)(t0 >> SHIFT) * D, 0, nfull * D * 4, 0x00027000);
         lane4 = c * 4;
         from_ckpt = iv > 0;
         ck = 0;
@@ -69,7 +70,7 @@ struct LoneLoads {
 #pragma unroll
         for (int i = 0; i < PF; i++)
             buf[i] = load(0, i);
-        tail = cbh[(size_t)(last ? (unsigned)T / TPW : 0) * D];
+        tail = cbh[(size_t)(last ? T >> SHIFT : 0) * D];
         fresh = reinterpret_cast<const uint16_t *>(x_new)[(size_t)bx * D + c];
     }
     // supergroup sg + i, i < PF; read once: not kept in the caches
@@ -81,7 +82,7 @@ struct LoneLoads {
     __device__ __forceinline__ void refill(int first, int i)
     {
         if (i % UPS == UPS - 1)
-            buf[i / UPS] = load((unsigned)first / UPS + PF, i / UPS);
+            buf[i / UPS] = load((first >> (SHIFT - 3)) + PF, i / UPS);
     }
     __device__ __forceinline__ int code(int t) const { return (int)(tail >> (BITS * t) & Code<BITS>::FIELD) + Code<BITS>::QLO; }
     __device__ __forceinline__ Lone state() const
@@ -149,7 +150,7 @@ __device__ __forceinline__ h1 lone_append(const LoneLoads<D, BITS> &s, const Lon
     const int q = quantize<BITS>(x, lone_zp(st), lone_sc(st));
     const int sh = BITS * s.ntail;
     if (active)
-        s.cbh[(size_t)((unsigned)T / Code<BITS>::TPW) * D] = (s.tail & ~(Code<BITS>::FIELD << sh)) | ((uint32_t)(q - Code<BITS>::QLO) << sh);
+        s.cbh[(size_t)(T >> s.SHIFT) * D] = (s.tail & ~(Code<BITS>::FIELD << sh)) | ((uint32_t)(q - Code<BITS>::QLO) << sh);
     return __builtin_fmaf16((h1)q, lone_sc(st), lone_zp(st));
 }
 
