@@ -36,8 +36,9 @@ struct LoneLoads {
     static constexpr int TPW = Code<BITS>::TPW, UPS = TPW / 8, PF = LONE_PF / UPS; // units, words of codes in flight
     static constexpr int SHIFT = BITS == 4 ? 3 : 4;                                // of tokens to words
     uint32_t *cbh;      // this head, this channel
-    // this segment's whole supergroups: reads past them are dropped, and a load takes no address arithmetic (with a
-    // clamped index it was five instructions)
+    // this segment's whole supergroups.  Reads past them are dropped: a load's whole position is in its vector offset, which
+    // is what the range check looks at (of the scalar offset the check is not documented to take account), one
+    // addition for PF of them (with a clamped index it was five instructions a load)
     __amdgpu_buffer_rsrc_t codes;
     int lane4;
     int t0, t1, nfull, ntail;
@@ -76,7 +77,7 @@ struct LoneLoads {
     // supergroup sg + i, i < PF; read once: not kept in the caches
     __device__ __forceinline__ uint32_t load(int sg, int i) const
     {
-        return __builtin_amdgcn_raw_buffer_load_b32(codes, lane4 + i * D * 4, sg * D * 4, 2);
+        return __builtin_amdgcn_raw_buffer_load_b32(codes, lane4 + sg * D * 4 + i * D * 4, 0, 2);
     }
     // behind unit i of LONE_PF (at that unit of `first` on): the word that it was the last of, PF words further
     __device__ __forceinline__ void refill(int first, int i)

@@ -112,3 +112,13 @@ def test_the_weights_loop_keeps_its_loads_in_flight(listings):
     loop = max(loops, key=lambda b: sum(o.startswith("v_pk") for o, _, _ in b) / len(b) if len(b) > 100 else 0)
     waits = [int(n) for o, a, _ in loop if o == "s_waitcnt" for n in re.findall(r"vmcnt\((\d+)\)", a)]
     assert len(waits) == 8 and min(waits) == 14, waits
+
+
+def test_code_loads_keep_their_position_where_the_range_check_sees_it(listings):
+    """Of one channel per lane: up to eight loads a lane run past the segment and have to be dropped; the check looks at the
+    vector offset, and a scalar one beyond the range is nobody's promise."""
+    found = [(name, args) for t, _ in listings for with_ in ("lone_kernel", "small_step_kernel")
+             for name, code, _ in kernels(t, with_) if with_ in name
+             for op, args, _ in code if op.startswith("buffer_load_dword")]
+    assert len(found) > 600                                                # the listings are what they should be
+    assert not [f for f in found if not re.search(r"\], 0 offen", f[1])][:5]
