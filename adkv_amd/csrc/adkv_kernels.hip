@@ -3413,29 +3413,32 @@ static int softmax_launch(const void *logits, void *weights, const Mask &mask, i
     return check_launch();
 }
 
-// Which decode kernel family and shape a launch of these sizes takes (the dispatch below, as text).
-static const char *decode_kernel_name(int B, int Hq, int H, int T, int D, int bits, int n_ckpt_cap,
+// Which decode kernel family and shape forward_qk (ov: forward_ov, of 16-byte aligned rows) takes for these sizes: the
+// dispatch below, as text.
+static const char *decode_kernel_name(bool ov, int B, int Hq, int H, int T, int D, int bits, int n_ckpt_cap,
                                       int ckpt_interval)
 {
     if (B <= 0 || H <= 0 || Hq <= 0 || Hq % H || T < 0 || (D != 128 && D != 256 && D != 512) ||
         (bits != 2 && bits != 4))
         return "invalid";
-    const int GQ = Hq / H;
+    const int GQ = Hq / H, BH = B * H;
     if ((GQ > 1 || bits != 4) && D != 128)
         return "invalid";
     int dummy = 0;
     const Seg seg = plan_segments(n_ckpt_cap > 0 && ckpt_interval > 0 ? &dummy : nullptr, n_ckpt_cap,
-                                  ckpt_interval, B * H, T, D);
+                                  ckpt_interval, BH, T, D);
     if (D == 128 && (GQ > 1 || bits != 4 || mfma_for_mha())) {
-        if (gqa_pair(B * H, seg.nseg))
+        if (ov ? ov_gqa_pair(BH, seg.nseg, GQ, true) : gqa_pair(BH, seg.nseg))
             return "gqa_kernel, two channels per lane (matrix cores)";
-        return threads_per_workgroup(padded_units<32>(B * H, seg.nseg) * 32) == 1024
-                   ? "gqa_kernel, 16-wave workgroups (matrix cores)"
-                   : "gqa_kernel, 12-wave workgroups (matrix cores)";
+        const int blk = threads_per_workgroup(padded_units<32>(BH, seg.nseg) * 32);
+        if (ov && (GQ > 4 || blk == 256))
+            return "gqa_kernel, 8-wave workgroups (matrix cores)";
+        return blk == 1024 ? "gqa_kernel, 16-wave workgroups (matrix cores)"
+                           : "gqa_kernel, 12-wave workgroups (matrix cores)";
     }
     if (use_head_table(B, H, GQ, bits, D, seg)) {
         Seg s2 = seg;
-        const int lanes = plan_ft(s2, B, H, T, FT_SKEW_QK, FT16_QK);
+        const int lanes = ov ? plan_ft_ov(s2, B, H, T) : plan_ft(s2, B, H, T, FT_SKEW_QK, FT16_QK);
         if (lanes == 16)
             return s2.groups ? "ft_kernel (per-head table, 16 lanes per head, 16-wave workgroups, uneven segments)"
                              : "ft_kernel (per-head table, 16 lanes per head, 16-wave workgroups)";
@@ -3443,8 +3446,8 @@ static const char *decode_kernel_name(int B, int Hq, int H, int T, int D, int bi
                          : "ft_kernel (per-head table, 16-wave workgroups)";
     }
     if (D == 128) {
-        const long units = padded_units<32>(B * H, seg.nseg);
-        if (qk_lone(B * H, seg.nseg, T))
+        const long units = padded_units<32>(BH, seg.nseg);
+        if (ov ? ov_lone(BH, seg.nseg, T) : qk_lone(BH, seg.nseg, T))
             return "lone_kernel (shared table, one channel per lane)";
         if (units / 2 <= n_simd())
             return "kernel<128,2,256> (shared table, two channels per lane)";
@@ -3526,7 +3529,13 @@ extern "C" {
 const char *adkv_decode_kernel_name(int B, int Hq, int H, int T, int D, int bits, int n_ckpt_cap,
                                     int ckpt_interval)
 {
-    return decode_kernel_name(B, Hq, H, T, D, bits, n_ckpt_cap, ckpt_interval);
+    return decode_kernel_name(false, B, Hq, H, T, D, bits, n_ckpt_cap, ckpt_interval);
+}
+
+const char *adkv_decode_ov_kernel_name(int B, int Hq, int H, int T, int D, int bits, int n_ckpt_cap,
+                                       int ckpt_interval)
+{
+    return decode_kernel_name(true, B, Hq, H, T, D, bits, n_ckpt_cap, ckpt_interval);
 }
 
 int adkv_decode_step_launches(int B, int Hq, int H, int T, int D, int bits, int n_ckpt_cap, int ckpt_interval,

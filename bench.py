@@ -344,8 +344,8 @@ def step_kernels(L, B, Hq, H, T, D, bits, n_ckpt_cap, S):
         return ("small_step_kernel",)
     if n == 2:
         return ("step_segments_kernel", "step_combine_kernel")
-    name = L.adkv_decode_kernel_name(B, Hq, H, T, D, bits, n_ckpt_cap, S).decode()
-    return "qk_" + name, "softmax", "ov_" + name
+    qk, ov = (f(B, Hq, H, T, D, bits, n_ckpt_cap, S).decode() for f in (L.adkv_decode_kernel_name, L.adkv_decode_ov_kernel_name))
+    return "qk_" + qk, "softmax", "ov_" + ov
 
 
 def decode_record(args, B, Hq, H, D, T, bits, S, NL, steps, warmup, headline=True, bf16=False):

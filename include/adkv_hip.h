@@ -312,12 +312,14 @@ int adkv_decode_step(const void *q, void *k_cache, void *v_cache, const void *k_
                       void *k_ckpt, void *v_ckpt, int n_ckpt_cap, int ckpt_interval,
                       void *workspace, int64_t workspace_bytes, void *stream);
 
-/* Which of the library's decode kernels adkv_forward_qk_gqa / adkv_forward_ov_gqa launch for these
- * sizes ("qk_" / "ov_" + the returned text), and adkv_decode_step where adkv_decode_step_launches is 3
- * (otherwise it runs other kernels): a static string, for benchmark records and tests; "invalid" for sizes
- * the entry points reject. */
+/* Which of the library's decode kernels adkv_forward_qk_gqa / adkv_forward_ov_gqa launch for these sizes ("qk_" + the
+ * first text, "ov_" + the second: forward_ov takes some shapes up to other sizes, here for rows of weights that are 16-byte
+ * aligned, as adkv_decode_step lays them), and adkv_decode_step where adkv_decode_step_launches is 3 (otherwise it runs
+ * other kernels): static strings, for benchmark records and tests; "invalid" for sizes the entry points reject. */
 const char *adkv_decode_kernel_name(int B, int Hq, int H, int T, int D, int bits, int n_ckpt_cap,
                                     int ckpt_interval);
+const char *adkv_decode_ov_kernel_name(int B, int Hq, int H, int T, int D, int bits, int n_ckpt_cap,
+                                       int ckpt_interval);
 
 /* How the context of such a launch is cut into independently replayed segments (no counterpart
  * in the reference, whose kernels replay every sequence from token 0: gemv.cu:565).  Returns the

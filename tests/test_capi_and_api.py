@@ -137,6 +137,28 @@ def test_segment_plans_cut_at_checkpoints_and_cover_the_context():
         L.adkv_set_mha_kernel(-1)
 
 
+def test_library_names_the_kernels_of_keys_and_of_values():
+    """Without a GPU (256 CUs): forward_ov takes one channel per lane, and two with grouped queries, up to other sizes."""
+    L = _lib.lib()
+
+    def names(B, Hq, H, T, S=256, D=128, bits=4):
+        args = (B, Hq, H, T, D, bits, T // S + 1 if S else 0, S)
+        return tuple(f(*args).decode().split(" (")[0] for f in (L.adkv_decode_kernel_name, L.adkv_decode_ov_kernel_name))
+
+    lone, two, gqa, pair = "lone_kernel", "kernel<128,2,256>", "gqa_kernel, %d-wave workgroups", "gqa_kernel, two channels per lane"
+    assert names(48, 32, 32, 1024, 0) == (lone, lone)
+    assert names(60, 32, 32, 1024, 0) == names(64, 32, 32, 200) == (two, lone)
+    assert names(65, 32, 32, 200) == ("kernel<128,4,256>",) * 2
+    assert names(128, 64, 8, 300, 0) == (pair, pair)
+    # eight query heads from two waves of two channels per SIMD on, four from three
+    assert names(16, 64, 8, 4096) == (pair, pair) and names(16, 64, 8, 5000) == (pair, gqa % 8)
+    assert names(16, 32, 8, 6000) == (pair, pair) and names(16, 32, 8, 7000) == (pair, gqa % 8)
+    assert names(16, 32, 8, 131072) == (gqa % 16, gqa % 16)
+    for k, v in (names(128, 32, 32, 4096), names(100, 32, 32, 4096), names(8, 32, 32, 65536)):
+        assert k.startswith("ft_kernel") and v.startswith("ft_kernel")
+    assert names(4, 8, 8, 8190, D=256) == ("kernel<256,4,*>",) * 2 and names(2, 6, 4, 100) == ("invalid",) * 2
+
+
 def test_segment_plans_of_random_shapes_stay_inside_the_checkpoints():
     """Seeded sweep of batch sizes, head counts, context lengths, checkpoint intervals and capacities,
     under the library's own choice of kernels and with every kernel family forced: every plan covers
