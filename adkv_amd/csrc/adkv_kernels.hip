@@ -2870,6 +2870,8 @@ static bool small_step_plan(Seg &seg, int B, int Hq, int H, int T, int D, int bi
     return seg.nseg <= 4;
 }
 
+static int longest_segment(const Seg &seg, int T) { return seg.nseg > 1 ? seg.seg_tokens : T; } // of an even plan
+
 // Whether a step runs as step_segments_kernel + step_combine_kernel, its plan and its channels per lane.
 // Every segment has to fit the LDS of its wave and all waves have to be resident: at most four per SIMD
 // (two with 184 registers at head dim 512).  us per step on the device, three to four launches / two,
@@ -2898,7 +2900,7 @@ static bool segment_step_plan(Seg &seg, int &cpl, int B, int Hq, int H, int T, i
         return false;
     const int BH = B * H;
     seg = plan_segments(k_ckpt, n_ckpt_cap, ckpt_interval, BH, T, D);
-    const int longest = seg.nseg > 1 ? seg.seg_tokens : T;
+    const int longest = longest_segment(seg, T);
     if (longest + 1 > (GQ == 8 ? step_cap<8>() : step_cap<1>()) || (GQ == 1 && bits == 4 && seg.nseg > 1 && longest < 128))
         return false;
     const long room = (D == 512 ? 2L : 4L) * n_simd();
@@ -3551,6 +3553,30 @@ int adkv_decode_step_launches(int B, int Hq, int H, int T, int D, int bits, int 
     return segment_step_plan(seg, cpl, B, Hq, H, T, D, bits, ck, ck, n_ckpt_cap, ckpt_interval) ? 2 : 3;
 }
 
+const char *adkv_decode_step_kernel_name(int B, int Hq, int H, int T, int D, int bits, int n_ckpt_cap, int ckpt_interval,
+                                         int masked)
+{
+    int dummy = 0, cpl;
+    Seg seg, vseg;
+    void *ck = n_ckpt_cap > 0 && ckpt_interval > 0 ? &dummy : nullptr;
+    switch (adkv_decode_step_launches(B, Hq, H, T, D, bits, n_ckpt_cap, ckpt_interval, masked)) {
+    case 1:
+        return !masked && fused_step_plan(seg, vseg, B, Hq, H, T, D, bits, ck, ck, n_ckpt_cap, ckpt_interval) ? "decode_ft_kernel"
+                                                                                                             : "small_step_kernel";
+    case 2:
+        segment_step_plan(seg, cpl, B, Hq, H, T, D, bits, ck, ck, n_ckpt_cap, ckpt_interval);
+        switch (step_lone_threads(padded_units<64>(B * H, seg.nseg), D, Hq / H, longest_segment(seg, T))) {
+        case 0: return "step_segments_kernel";
+        case 256: return "step_lone_kernel, 4-wave workgroups";
+        case 512: return "step_lone_kernel, 8-wave workgroups";
+        case 768: return "step_lone_kernel, 12-wave workgroups";
+        default: return "step_lone_kernel, 16-wave workgroups";
+        }
+    default:
+        return nullptr;
+    }
+}
+
 int adkv_decode_segments(int B, int Hq, int H, int T, int D, int bits, int n_ckpt_cap,
                          int ckpt_interval, int *bounds, int max_bounds, int *info)
 {
@@ -4051,9 +4077,10 @@ int adkv_decode_step(const void *q, void *k_cache, void *v_cache, const void *k_
             const long rows = (long)B * Hq;
             float4 *ml = (float4 *)(ws + 2 * mat);
             float *partial = (float *)(ws + 2 * mat + pad256(ka.nseg * rows * 16));
-            if ((rc = launch_step_segments(cpl, Hq / H, bits, D, B * H, ka.nseg, ka.nseg > 1 ? ka.seg_tokens : T, (hipStream_t)stream, (const h1 *)q, (uint4 *)k_cache,
-                                           (const h1 *)k_new, (uint4 *)v_cache, (const h1 *)v_new, mk, (h1 *)logits, partial, ml,
-                                           ft_params(k_params), ft_params(v_params), B * H, H, T, n_super_cap, scaling, ka, va)))
+            if ((rc = launch_step_segments(cpl, Hq / H, bits, D, B * H, ka.nseg, longest_segment(ka, T), (hipStream_t)stream,
+                                           (const h1 *)q, (uint4 *)k_cache, (const h1 *)k_new, (uint4 *)v_cache, (const h1 *)v_new,
+                                           mk, (h1 *)logits, partial, ml, ft_params(k_params), ft_params(v_params), B * H, H, T,
+                                           n_super_cap, scaling, ka, va)))
                 return rc;
             for (int i = 1; i <= 2; i++)
                 if ((rc = stage_mark(i, stream)))

@@ -339,12 +339,12 @@ def quant_f32_record(args, B, T, steps, warmup):
 def step_kernels(L, B, Hq, H, T, D, bits, n_ckpt_cap, S):
     """The kernels of one decode_step call: one launch; short segments and their combination; or forward_qk, the
     softmax and forward_ov.  The library's first pair of events brackets the first of them, the last pair the last."""
-    n = L.adkv_decode_step_launches(B, Hq, H, T, D, bits, n_ckpt_cap, S, 0)
-    if n == 1:                     # few short sequences
-        return ("small_step_kernel",)
-    if n == 2:
-        return ("step_segments_kernel", "step_combine_kernel")
-    qk, ov = (f(B, Hq, H, T, D, bits, n_ckpt_cap, S).decode() for f in (L.adkv_decode_kernel_name, L.adkv_decode_ov_kernel_name))
+    sizes = (B, Hq, H, T, D, bits, n_ckpt_cap, S)
+    n = L.adkv_decode_step_launches(*sizes, 0)
+    if n < 3:                      # few short sequences; short segments
+        first = L.adkv_decode_step_kernel_name(*sizes, 0).decode()
+        return (first,) if n == 1 else (first, "step_combine_kernel")
+    qk, ov = (f(*sizes).decode() for f in (L.adkv_decode_kernel_name, L.adkv_decode_ov_kernel_name))
     return "qk_" + qk, "softmax", "ov_" + ov
 
 

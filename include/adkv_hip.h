@@ -57,14 +57,18 @@ void adkv_set_mha_kernel(int use_matrix_cores);
  * adkv_set_mha_kernel or ADKV_MFMA picks a family).
  * adkv_decode_step_is_fused: 1 if a call with these sizes, masked or not, is one launch of either
  * kind under the current settings, else 0.
- * adkv_decode_step_launches: 1 for those; 2 if the call runs as step_segments_kernel and step_combine_kernel
- * (steps of short segments, see adkv_decode_step); 3 if forward_qk, the softmax and forward_ov are launched
- * one after the other, also for sizes that the call refuses. */
+ * adkv_decode_step_launches: 1 for those; 2 if the call runs as step_segments_kernel or step_lone_kernel (one channel
+ * per lane) and step_combine_kernel (steps of short segments, see adkv_decode_step); 3 if forward_qk, the softmax and
+ * forward_ov are launched one after the other, also for sizes that the call refuses.
+ * adkv_decode_step_kernel_name: the first kernel of a call in one or two launches, a static string for benchmark records
+ * and tests; NULL for the others (adkv_decode_kernel_name and adkv_decode_ov_kernel_name have theirs). */
 void adkv_set_fused_step(int mode);
 int adkv_decode_step_is_fused(int B, int Hq, int H, int T, int D, int bits, int n_ckpt_cap,
                               int ckpt_interval, int masked);
 int adkv_decode_step_launches(int B, int Hq, int H, int T, int D, int bits, int n_ckpt_cap,
                               int ckpt_interval, int masked);
+const char *adkv_decode_step_kernel_name(int B, int Hq, int H, int T, int D, int bits, int n_ckpt_cap,
+                                         int ckpt_interval, int masked);
 const char *adkv_strerror(int code);
 /* hipError_t (as int) of the last failed launch in this thread, 0 if none. */
 int adkv_last_hip_error(void);

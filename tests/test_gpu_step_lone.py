@@ -1,22 +1,33 @@
 """Steps in two launches with one channel per lane (a KV head over two, four or eight waves): its workgroup sizes and the
 sizes just beyond it, and the ends of supergroups, tiles and groups of tiles."""
+import re
+
 import pytest
 import torch
 
+from adkv_amd import _lib
 from tests.test_gpu_segment_step import test_against_the_three_calls, test_masked_segments_and_rows
 
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("B,Hq,H,D,T,S", [
-    (4, 32, 32, 128, 1300, 256), (5, 32, 32, 128, 1800, 256), (6, 32, 32, 128, 2041, 256),                # 4, 12 waves, beyond
-    (4, 32, 16, 128, 1500, 256), (8, 32, 16, 128, 1793, 256), (9, 32, 16, 128, 2047, 256), (13, 32, 16, 128, 2047, 256),
-    (2, 32, 8, 128, 6000, 256), (3, 32, 8, 128, 9001, 256), (6, 32, 8, 128, 7680, 256),                   # 4, 8, 12 waves
-    (3, 64, 8, 128, 4799, 256), (5, 64, 8, 128, 5632, 256), (9, 64, 8, 128, 3800, 256),                   # 4, 8 waves, beyond
-    (2, 16, 16, 256, 3900, 256), (2, 16, 16, 256, 5021, 256), (4, 8, 8, 256, 7171, 256), (5, 8, 8, 256, 7170, 256),
-    (1, 8, 8, 512, 3333, 256), (3, 8, 8, 512, 3584, 256), (10, 8, 8, 512, 1799, 256),
+def _runs(B, Hq, H, D, T, bits, S):
+    """What the library says a step starts with: the waves of a step_lone_kernel's workgroup, 0 for the other kernel."""
+    tps = 32 // bits
+    name = _lib.lib().adkv_decode_step_kernel_name(B, Hq, H, T, D, bits, (T + tps) // S + 1 if S else 0, S, 0).decode()
+    return 0 if name == "step_segments_kernel" else int(re.fullmatch(r"step_lone_kernel, (\d+)-wave workgroups", name)[1])
+
+
+@pytest.mark.parametrize("B,Hq,H,D,T,S,waves", [
+    (4, 32, 32, 128, 1300, 256, 4), (5, 32, 32, 128, 1800, 256, 12), (6, 32, 32, 128, 2041, 256, 12), (7, 32, 32, 128, 2041, 256, 0),
+    (4, 32, 16, 128, 1500, 256, 4), (8, 32, 16, 128, 1793, 256, 8), (9, 32, 16, 128, 2047, 256, 12), (13, 32, 16, 128, 2047, 256, 0),
+    (2, 32, 8, 128, 6000, 256, 4), (3, 32, 8, 128, 9001, 256, 8), (6, 32, 8, 128, 7680, 256, 12), (7, 32, 8, 128, 7169, 256, 0),
+    (3, 64, 8, 128, 4799, 256, 4), (5, 64, 8, 128, 5632, 256, 8), (9, 64, 8, 128, 3800, 256, 0),
+    (2, 16, 16, 256, 3900, 256, 4), (2, 16, 16, 256, 5021, 256, 12), (4, 8, 8, 256, 7171, 256, 16), (5, 8, 8, 256, 7170, 256, 0),
+    (1, 8, 8, 512, 3333, 256, 8), (3, 8, 8, 512, 3584, 256, 16), (10, 8, 8, 512, 1799, 256, 0),
 ])
-def test_workgroup_sizes(gpu, oracle, B, Hq, H, D, T, S):
+def test_workgroup_sizes(gpu, oracle, B, Hq, H, D, T, S, waves):
+    assert _runs(B, Hq, H, D, T, 4, S) == waves
     test_against_the_three_calls(gpu, oracle, B, Hq, H, D, T, 4, S, torch.float16)
 
 
@@ -27,6 +38,7 @@ def test_ends_of_segments(gpu, oracle, Hq, H, D, T, S):
     """No supergroup, a half tile, a tile, a group of four and one more; 256 tokens and the appended one; segments of 64."""
     if S == 64 and Hq == H:
         pytest.skip("segments below 128 tokens of one query head per KV head keep the separate launches")
+    assert _runs(2, Hq, H, D, T, 4, S) > 0
     test_against_the_three_calls(gpu, oracle, 2, Hq, H, D, T, 4, S, torch.bfloat16)
 
 
@@ -35,16 +47,20 @@ def test_ends_of_segments(gpu, oracle, Hq, H, D, T, S):
                                  (271, 256), (272, 256), (330, 256), (512, 256), (200, 64)])
 def test_two_bits(gpu, oracle, Hq, H, T, S):
     """A word of codes is a whole tile: no word, ragged ones of one to fifteen tokens, an odd and an even number of them."""
+    assert _runs(2, Hq, H, 128, T, 2, S) > 0
     test_against_the_three_calls(gpu, oracle, 2, Hq, H, 128, T, 2, S, torch.float16)
 
 
-@pytest.mark.parametrize("B,Hq,H,T", [(4, 32, 32, 1300), (6, 32, 32, 1900), (8, 32, 16, 1793), (12, 32, 16, 1800), (3, 32, 8, 9001),
-                                      (6, 32, 8, 7680), (2, 64, 8, 4000), (5, 64, 8, 5632), (8, 64, 8, 8000)])
-def test_two_bits_workgroup_sizes(gpu, oracle, B, Hq, H, T):
+@pytest.mark.parametrize("B,Hq,H,T,waves", [(4, 32, 32, 1300, 4), (6, 32, 32, 1900, 12), (7, 32, 32, 1900, 0), (8, 32, 16, 1793, 8),
+                                            (12, 32, 16, 1800, 12), (3, 32, 8, 9001, 8), (6, 32, 8, 7680, 12), (2, 64, 8, 4000, 4),
+                                            (5, 64, 8, 5632, 8), (8, 64, 8, 8000, 0)])
+def test_two_bits_workgroup_sizes(gpu, oracle, B, Hq, H, T, waves):
+    assert _runs(B, Hq, H, 128, T, 2, 256) == waves
     test_against_the_three_calls(gpu, oracle, B, Hq, H, 128, T, 2, 256, torch.bfloat16)
 
 
 @pytest.mark.parametrize("low", [torch.finfo(torch.float32).min, float("-inf")])
 @pytest.mark.parametrize("Hq,H,D", [(4, 4, 512), (8, 1, 128), (4, 2, 128)])
 def test_masks(gpu, Hq, H, D, low):
+    assert _runs(3, Hq, H, D, 768, 4, 256) > 0
     test_masked_segments_and_rows(gpu, 3, Hq, H, D, 768, low)

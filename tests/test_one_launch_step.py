@@ -111,6 +111,39 @@ def test_library_says_in_how_many_launches_a_step_runs():
         L.adkv_set_mha_kernel(-1)
 
 
+def test_library_and_benchmark_name_the_first_kernel_of_a_step():
+    """Without a GPU (256 CUs): one channel per lane up to 12 waves of 64 channels per CU (wide heads 16, eight query heads 8),
+    the other kernel beyond, longer segments and in one launch."""
+    import bench
+    L = _lib.lib()
+
+    def name(B, Hq, H, T, D=D, bits=4, S=256, masked=0):
+        n = T // S + 1 if S else 0
+        first = L.adkv_decode_step_kernel_name(B, Hq, H, T, D, bits, n, S, masked)
+        if not masked and L.adkv_decode_step_launches(B, Hq, H, T, D, bits, n, S, 0) < 3:
+            assert bench.step_kernels(L, B, Hq, H, T, D, bits, n, S)[0] == first.decode()
+        return first.decode() if first else None
+
+    lone = "step_lone_kernel, %d-wave workgroups"
+    for bits in (4, 2):
+        for waves, sizes in ((4, (4, 32, 32, 2048)), (12, (6, 32, 32, 2048)), (0, (7, 32, 32, 2048)), (4, (4, 32, 16, 2048)),
+                             (8, (8, 32, 16, 2048)), (12, (12, 32, 16, 2048)), (0, (13, 32, 16, 2048)), (4, (8, 32, 8, 2048)),
+                             (8, (16, 32, 8, 2048)), (12, (24, 32, 8, 2048)), (0, (25, 32, 8, 2048)), (4, (8, 64, 8, 2048)),
+                             (8, (16, 64, 8, 2048)), (0, (17, 64, 8, 2048))):
+            assert name(*sizes, bits=bits) == name(*sizes, bits=bits, masked=1) == (lone % waves if waves else "step_segments_kernel")
+    for waves, sizes in ((4, (4, 16, 16, 2048, 256)), (12, (6, 16, 16, 2048, 256)), (16, (8, 16, 16, 2048, 256)),
+                         (0, (9, 16, 16, 2048, 256)), (8, (4, 8, 8, 2048, 512)), (16, (8, 8, 8, 2048, 512)), (0, (9, 8, 8, 2048, 512))):
+        assert name(*sizes) == (lone % waves if waves else "step_segments_kernel"), sizes
+    assert name(2, 8, 2, 1500, S=512) == "step_segments_kernel"               # segments beyond 256 tokens
+    assert name(1, 32, 32, 603) == name(1, 32, 32, 603, masked=1) == "small_step_kernel"
+    assert name(128, 32, 32, 4096) is None and name(1, 6, 4, 100) is None
+    L.adkv_set_fused_step(1)
+    try:
+        assert name(128, 32, 32, 4096) == "decode_ft_kernel" and name(128, 32, 32, 4096, masked=1) is None
+    finally:
+        L.adkv_set_fused_step(0)
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("H,T,S", [(4, 200, 64), (3, 600, 256)])
 def test_one_launch_step_replays_from_a_captured_graph(gpu, H, T, S):
