@@ -270,27 +270,34 @@ __device__ __forceinline__ void lone_fill(uint2 *lut, int tid)
 }
 
 // Eight tokens, entries e[0..3] of two tokens each; x[k] = the values of tokens 2k and 2k + 1.  As in replay_eight no
-// packed result is read by the very next instruction.
+// packed result is read by the very next instruction.  TO_MATRIX: the next one may be a matrix instruction that reads x,
+// two states later; the wait is the block's own (as a statement behind the block the compiler put it in front of it).
 #define ADKV_LONE_F(E) "v_pk_fma_f16 %[f], " E ", %[cf], %[c0]\n\t"
 #define ADKV_LONE_R "v_pk_mul_f16 %[r], %[f], %[r] op_sel:[0,1] op_sel_hi:[1,1]\n\t"
 #define ADKV_LONE_Z(TO, FROM) "v_pk_fma_f16 " TO ", %[r], %[ca], " FROM " op_sel_hi:[0,1,0]\n\t"
 #define ADKV_LONE_P(X) "v_perm_b32 " X ", %[z], " X ", %[hi]\n\t"
+#define ADKV_LONE_EIGHT(END)                                                                                                \
+    asm(ADKV_LONE_F("%[a0]") "s_nop 0\n\t"                                                                                  \
+        ADKV_LONE_R ADKV_LONE_F("%[b0]") ADKV_LONE_Z("%[x0]", "%[z]")                                                       \
+        ADKV_LONE_R ADKV_LONE_F("%[a1]") ADKV_LONE_Z("%[z]", "%[x0]")                                                       \
+        ADKV_LONE_R ADKV_LONE_F("%[b1]") ADKV_LONE_Z("%[x1]", "%[z]")                                                       \
+        ADKV_LONE_R ADKV_LONE_F("%[a2]") ADKV_LONE_P("%[x0]") ADKV_LONE_Z("%[z]", "%[x1]")                                  \
+        ADKV_LONE_R ADKV_LONE_F("%[b2]") ADKV_LONE_Z("%[x2]", "%[z]")                                                       \
+        ADKV_LONE_R ADKV_LONE_F("%[a3]") ADKV_LONE_P("%[x1]") ADKV_LONE_Z("%[z]", "%[x2]")                                  \
+        ADKV_LONE_R ADKV_LONE_F("%[b3]") ADKV_LONE_Z("%[x3]", "%[z]")                                                       \
+        ADKV_LONE_R ADKV_LONE_P("%[x2]") ADKV_LONE_Z("%[z]", "%[x3]")                                                       \
+        "s_nop 0\n\t" ADKV_LONE_P("%[x3]") END                                                                              \
+        : [z] "+v"(s.z), [r] "+v"(s.r), [f] "=&v"(f), [x0] "=&v"(x[0]), [x1] "=&v"(x[1]), [x2] "=&v"(x[2]), [x3] "=&v"(x[3])\
+        : [a0] "v"(e[0].x), [b0] "v"(e[0].y), [a1] "v"(e[1].x), [b1] "v"(e[1].y), [a2] "v"(e[2].x), [b2] "v"(e[2].y),       \
+          [a3] "v"(e[3].x), [b3] "v"(e[3].y), [ca] "v"(s.ca), [cf] "v"(s.cf), [c0] "v"(s.c0), [hi] "s"(0x07060302u))
+template <bool TO_MATRIX = false>
 __device__ __forceinline__ void lone_eight(Lone &s, const uint2 *e, uint32_t *x)
 {
     uint32_t f;
-    asm(ADKV_LONE_F("%[a0]") "s_nop 0\n\t"
-        ADKV_LONE_R ADKV_LONE_F("%[b0]") ADKV_LONE_Z("%[x0]", "%[z]")
-        ADKV_LONE_R ADKV_LONE_F("%[a1]") ADKV_LONE_Z("%[z]", "%[x0]")
-        ADKV_LONE_R ADKV_LONE_F("%[b1]") ADKV_LONE_Z("%[x1]", "%[z]")
-        ADKV_LONE_R ADKV_LONE_F("%[a2]") ADKV_LONE_P("%[x0]") ADKV_LONE_Z("%[z]", "%[x1]")
-        ADKV_LONE_R ADKV_LONE_F("%[b2]") ADKV_LONE_Z("%[x2]", "%[z]")
-        ADKV_LONE_R ADKV_LONE_F("%[a3]") ADKV_LONE_P("%[x1]") ADKV_LONE_Z("%[z]", "%[x2]")
-        ADKV_LONE_R ADKV_LONE_F("%[b3]") ADKV_LONE_Z("%[x3]", "%[z]")
-        ADKV_LONE_R ADKV_LONE_P("%[x2]") ADKV_LONE_Z("%[z]", "%[x3]")
-        "s_nop 0\n\t" ADKV_LONE_P("%[x3]")
-        : [z] "+v"(s.z), [r] "+v"(s.r), [f] "=&v"(f), [x0] "=&v"(x[0]), [x1] "=&v"(x[1]), [x2] "=&v"(x[2]), [x3] "=&v"(x[3])
-        : [a0] "v"(e[0].x), [b0] "v"(e[0].y), [a1] "v"(e[1].x), [b1] "v"(e[1].y), [a2] "v"(e[2].x), [b2] "v"(e[2].y),
-          [a3] "v"(e[3].x), [b3] "v"(e[3].y), [ca] "v"(s.ca), [cf] "v"(s.cf), [c0] "v"(s.c0), [hi] "s"(0x07060302u));
+    if constexpr (TO_MATRIX)
+        ADKV_LONE_EIGHT("s_nop 1");
+    else
+        ADKV_LONE_EIGHT("");
 }
 // The same, each value multiplied by its token's weight (two per word of w) and added to acc in fp32.
 #define ADKV_LONE_M(W, HI) "v_fma_mix_f32 %[c], " W ", %[z], %[c] op_sel:[" HI ",1,0] op_sel_hi:[1,1,0]\n\t"
@@ -315,6 +322,7 @@ __device__ __forceinline__ void lone_eight_weighted(Lone &s, const uint2 *e, con
 }
 #undef ADKV_LONE_TOKEN
 #undef ADKV_LONE_M
+#undef ADKV_LONE_EIGHT
 #undef ADKV_LONE_P
 #undef ADKV_LONE_Z
 #undef ADKV_LONE_R

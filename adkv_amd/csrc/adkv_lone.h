@@ -421,8 +421,7 @@ __device__ __forceinline__ void lone_values_grouped(const uint2 *lut, uint32_t l
         s.refill(sg - i, i);
         __builtin_amdgcn_sched_barrier(0);
         uint32_t x[4];
-        lone_eight(st, e[half], x);
-        asm volatile("s_nop 1" ::: "memory"); // the block's results, as the matrix cores need them: two slots later
+        lone_eight<true>(st, e[half], x);
         __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
         for (int n = 0; n < NB; n++) {

@@ -12,6 +12,7 @@ PROBE = """
 #include "%s"
 using namespace adkv;
 __global__ void keys(Lone *s, const uint2 *e, uint32_t *x) { lone_eight(s[threadIdx.x], e + 4 * threadIdx.x, x + 4 * threadIdx.x); }
+__global__ void columns(Lone *s, const uint2 *e, uint32_t *x) { lone_eight<true>(s[threadIdx.x], e + 4 * threadIdx.x, x + 4 * threadIdx.x); }
 __global__ void values(Lone *s, const uint2 *e, const uint4 *w, float *acc) {
     lone_eight_weighted(s[threadIdx.x], e + 4 * threadIdx.x, w[threadIdx.x], acc[threadIdx.x]);
 }
@@ -28,7 +29,8 @@ def test_results_are_waited_for(tmp_path):
     found = re.findall(r"#ASMSTART\n(.*?)\n\s*;;?#ASMEND", (tmp_path / "probe.s").read_text(), re.S)
     found = [[l.strip() for l in b.strip().split("\n")] for b in found]
     found = [b for b in found if len(b) > 8]
-    assert len(found) == 2
+    assert len(found) == 3
+    assert [b[-1] for b in found].count("s_nop 1") == 1        # ahead of a matrix instruction
     for b in found:
         assert sum(i.startswith("v_pk_") for i in b) == 24
         for a, nxt in zip(b, b[1:]):

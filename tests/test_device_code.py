@@ -74,6 +74,27 @@ def violations(listing):
                 todo += [(k, waited + (int(a, 0) + 1 if o == "s_nop" else 1)) for k in after(j)]
 
 
+def early_sources(listing):
+    """(kernel, wait states, vector instruction, matrix instruction) of every matrix instruction that reads what a vector
+    instruction has written less than two wait states before it, along every path."""
+    for name, code, after in kernels(listing, "v_mfma"):
+        for i, (op, args, _) in enumerate(code):
+            if not op.startswith("v_") or op.startswith(("v_mfma", "v_cmp")):
+                continue
+            both = op.startswith(("v_permlane", "v_swap"))                  # these write their second operand as well
+            result, todo = _registers(",".join(args.split(",")[:2 if both else 1])), [(j, 0) for j in after(i)]
+            while todo:
+                j, waited = todo.pop()
+                if j is None or j >= len(code) or waited >= 2:
+                    continue
+                o, a, _ = code[j]
+                if o.startswith("v_mfma"):
+                    if result & _registers(",".join(a.split(",")[1:])):
+                        yield name, waited, f"{op} {args}", f"{o} {a}"
+                    continue
+                todo += [(k, waited + (int(a, 0) + 1 if o == "s_nop" else 1)) for k in after(j)]
+
+
 @pytest.fixture(scope="module")
 def listings(tmp_path_factory):
     if not os.path.exists(LIB_PATH) or not os.path.exists(f"{LLVM}/llvm-objdump"):
@@ -96,6 +117,17 @@ def listings(tmp_path_factory):
 def test_results_of_matrix_instructions_are_left_alone_until_written(listings):
     assert sum(t.count("\tv_mfma") for t, _ in listings) > 1000            # the listings are what they should be
     assert not [v for t, _ in listings for v in violations(t)][:5]
+
+
+def test_matrix_instructions_read_vector_results_two_states_later(listings):
+    """The distance that the compiler keeps between its own instructions, and not to a hand-laid block."""
+    code = ["v_perm_b32 v7, v3, v2, s4", "s_nop 1", "s_nop 0", "v_mfma_f32_4x4x4_16b_f16 v[8:11], v[0:1], v[6:7], v[8:11]", "s_endpgm"]
+
+    def found(order):
+        return len([*early_sources("0000 <k>:\n" + "".join(f"\t{code[i]} // {4 * n:08X}: 0\n" for n, i in enumerate(order)))])
+    assert found((0, 1, 3, 4)) == found((2, 0, 1, 3, 4)) == 0 and found((1, 0, 3, 4)) == found((1, 0, 2, 3, 4)) == 1
+    assert sum(t.count("\tv_mfma") for t, _ in listings) > 1000            # the listings are what they should be
+    assert not [v for t, _ in listings for v in early_sources(t)][:5]
 
 
 def test_rows_without_16_bit_masks_keep_four_waves_to_a_simd(listings):
