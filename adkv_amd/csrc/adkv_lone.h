@@ -508,6 +508,7 @@ __global__ __launch_bounds__(BLK) void ov_lone_kernel(const h1 *attn, uint4 *cac
     float acc = 0.0f;
     for (int sg = 0; sg < s.nfull; sg += LONE_CHUNK / 8) {
         weights[lane] = ahead;
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront"); // read by the wave's other lanes
         load_chunk(sg + LONE_CHUNK / 8);
         lone_values(lut, lane_copy, s, st, sg, min(LONE_CHUNK / 8, s.nfull - sg), reinterpret_cast<const h1 *>(weights), acc);
     }

@@ -361,6 +361,8 @@ __global__ __launch_bounds__(BLK) void step_lone_kernel(
     }
     if constexpr (GQ > 1)
         __syncthreads();
+    else
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront"); // the wave's own weights, read by its other lanes
     if (!active)
         return;
 

@@ -78,6 +78,7 @@ __global__ __launch_bounds__(512) void small_step_kernel(
         softmax_store_chunk<SMALL_ROW / 512, 64>(w, n, 0, x, 1.0f / sum, lane);
         if (wave == 0)
             softmax_store_chunk<SMALL_ROW / 512, 64>(weights + (size_t)bx * ka.row_pitch, n, 0, x, 1.0f / sum, lane);
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront"); // w is read by the wave's other lanes
 
         const h1 *wb = w + s.t0;
         Lone st = s.state();
