@@ -367,7 +367,7 @@ __global__ __launch_bounds__(FT_BLK) void qk_ft_kernel(
 // and zp separately would save the packed add; the outputs would then lack that rounding, up to
 // half an fp16 ulp of the largest value, for 1 % of the kernel's time: not done.)
 // A non-finite cached value makes both outputs of its channel PAIR non-finite (0 * inf inside the
-// product); the vector form of ov_kernel's two-channel lanes confines it to its own channel.
+// product); the vector form of ov_lone_kernel confines it to its own channel.
 //
 // One virtual workgroup per workgroup (forward_ov's plans never need more).  sa.combine: the two
 // or four segments of a wave's sequences sit in the same workgroup and are added there; otherwise

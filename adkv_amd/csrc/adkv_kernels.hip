@@ -1079,8 +1079,7 @@ constexpr int PAIR_TILE = 16 * 256; // bytes of a wave's key tile
 // rows.  Row r is head r * GQ / 16, so that lane (token, quarter of the rows) receives its head's
 // logit of its token as it is, and nothing is summed across lanes.  ~10 issue slots per token
 // where the dot product, its reduction over the lanes and the wait states made it 19
-// (32 x 32 heads x 1024 tokens, one segment: 49 -> 34 us; ov_kernel with replay_eight_weighted
-// 38 -> 32).
+// (32 x 32 heads x 1024 tokens, one segment: 49 -> 34 us).
 // The tile: row t = token t, 256 bytes; its 16-byte pieces are permuted by (t / 2) % 8 so that
 // both halves of an access to 16 rows at once spread over the banks.
 // LONE: workgroups of 256 threads, a wave with a SIMD's registers to itself; the compiler keeps products in
@@ -1581,11 +1580,8 @@ __device__ __forceinline__ void ov_segment(const uint2 *lut, uint32_t lane_copy,
 }
 
 // forward_ov by itself keeps its loads behind the table and the loop to itself: built from ov_segment with the loads
-// on their way meanwhile it was 0.5 to 1 us longer in launches of few waves (1 x 32 heads x 256 tokens 9.4 / 10.4 us)
-// and 3 to 8 % in long ones of wide heads (4 x 8 heads of 256 channels x 5000 tokens, no checkpoints, 188 / 202 us): the
-// compiler orders and waits otherwise.  (One wave per SIMD and more of 1024 tokens are the other way round by less: 32 x 32
-// 28.8 / 28.6 us, 60 x 32 42.2 / 41.7.)  The loads ahead of the table in the order of the loop were slower throughout:
-// 1 x 32 x 256 10.4 us, 32 x 32 x 1024 29.5, 16 x 32 x 1500 40.6 instead of 38.9.
+// on their way meanwhile it was 3 to 8 % longer in long launches of wide heads (4 x 8 heads of 256 channels x 5000 tokens,
+// no checkpoints, 188 / 202 us): the compiler orders and waits otherwise.
 template <int D, int CPL, int BLK>
 __global__ __launch_bounds__(BLK) void ov_kernel(
     const h1 *__restrict__ attn, uint4 *__restrict__ cache, const h1 *__restrict__ v_new,
@@ -1595,7 +1591,7 @@ __global__ __launch_bounds__(BLK) void ov_kernel(
     int BH, int H, int T, int n_super_cap, h1 *__restrict__ state_out, Seg sa)
 {
     using G = Geo<D, CPL>;
-    constexpr int AHEAD = CPL == 2 ? PF_PAIR : PF;
+    static_assert(CPL >= 4, "fewer channels per lane: ov_lone_kernel");
     sa.groups = 0; // only even plans come here
     __shared__ uint2 lut[LUT_WORDS64];
     lut_fill<BLK>(lut, threadIdx.x);
@@ -1613,13 +1609,8 @@ __global__ __launch_bounds__(BLK) void ov_kernel(
     Pair st[G::NP];
     float acc[CPL];
     init_pairs<D, CPL>(st, zp, sc, al, be, tg, h, bx, c0, un.seg, sa);
-#pragma unroll
-    for (int c = 0; c < CPL; c++)
-        acc[c] = 0.0f;
-    // Four-channel (and wider) lanes contract on the matrix cores, as ov_ft_kernel does and for the
-    // reason given there: B = the lane's dequantised pair at two tokens, A = (w[t], 0, w[t+1], 0)
+    // The contraction is the matrix cores', as in ov_ft_kernel and for the reason given there: B = the lane's dequantised pair at two tokens, A = (w[t], 0, w[t+1], 0)
     // from lane 0 of each group of four, (0, w[t], 0, w[t+1]) from lane 1, zeros from lanes 2, 3.
-    constexpr bool MM = CPL >= 4;
     f4v acc4[G::NP];
 #pragma unroll
     for (int p = 0; p < G::NP; p++)
@@ -1669,14 +1660,14 @@ __global__ __launch_bounds__(BLK) void ov_kernel(
         __builtin_amdgcn_sched_barrier(0);
     };
 
-    Vec buf[AHEAD][G::NV];
-    uint4 wbuf[AHEAD];
-    uint2 lk[MM ? G::NP : 2][8]; // two channels per lane: this supergroup's lookups and the next one's
+    Vec buf[PF][G::NV];
+    uint4 wbuf[PF];
+    uint2 lk[G::NP][8];
     uint32_t nb[G::NP][2];
     if (nfull > 0) {
         // unconditional, in the loop's order: see qk_kernel
 #pragma unroll
-        for (int i = 0; i < AHEAD; i++) {
+        for (int i = 0; i < PF; i++) {
             const int sg = min(i, nfull - 1);
 #pragma unroll
             for (int v = 0; v < G::NV; v++)
@@ -1695,35 +1686,24 @@ __global__ __launch_bounds__(BLK) void ov_kernel(
     // one supergroup, nothing conditional in it (see qk_kernel); i = its buffer in the rotation
     auto body = [&](int sg, auto ic) {
         constexpr int i = decltype(ic)::value;
-        pair_bytes_of<D, CPL>(buf[(i + 1) % AHEAD], nb);
-        const int sgp = min(sg + AHEAD, nfull - 1);
+        pair_bytes_of<D, CPL>(buf[(i + 1) % PF], nb);
+        const int sgp = min(sg + PF, nfull - 1);
 #pragma unroll
         for (int v = 0; v < G::NV; v++)
             buf[i][v] = load_codes(cb + (size_t)sgp * G::VPS + v);
         __builtin_amdgcn_sched_barrier(0);
-        if constexpr (MM) {
 #pragma unroll
-            for (int t = 0; t < 8; t += 2)
-                token2(t, lk, nb, wbuf[i]);
-        } else {
-            // a wave (nearly) alone on its SIMD: see replay_eight
-#pragma unroll
-            for (int t = 0; t < 8; t++)
-                lk[(i & 1) ^ 1][t] = lut_get(lut, nb[0][t & 1], lane_copy, t >> 1);
-            replay_eight_weighted(st[0], lk[i & 1], wbuf[i], acc);
-            __builtin_amdgcn_sched_barrier(0);
-        }
+        for (int t = 0; t < 8; t += 2)
+            token2(t, lk, nb, wbuf[i]);
         // the weights are reloaded once their last token is done: loading them earlier into a
         // second register set costs copies at the loop edge, which wait for the load they move
         wbuf[i] = load_w(sgp);
     };
-    rotate_over<AHEAD>(nfull, body);
-    if (MM) {
+    rotate_over<PF>(nfull, body);
 #pragma unroll
-        for (int p = 0; p < G::NP; p++) {
-            acc[2 * p] = acc4[p].x;
-            acc[2 * p + 1] = acc4[p].y;
-        }
+    for (int p = 0; p < G::NP; p++) {
+        acc[2 * p] = acc4[p].x;
+        acc[2 * p + 1] = acc4[p].y;
     }
 
     if (last) {
@@ -2452,18 +2432,10 @@ static int threads_per_workgroup(long threads)
             ADKV_LAUNCH_(KERNEL, DD, CC, 256, __VA_ARGS__);                                         \
     } while (0)
 
-// Head dim 128 has a second shape, two channels per lane (a head per wave): twice the waves, each
-// with half the instruction stream per token.  It pays when every wave has a SIMD to itself and
-// the launch is bound by the length of that stream (small batches, or no checkpoints to cut the
-// context with); with more waves per SIMD the four-channel lanes do less work in total.
 #define ADKV_DISPATCH_D(KERNEL, ...)                  \
     switch (D) {                                      \
     case 128:                                         \
-        if (padded_units<32>(BH, seg.nseg) / 2 <= n_simd()) { \
-            const long threads = padded_units<64>(BH, seg.nseg) * 64; \
-            ADKV_LAUNCH_(KERNEL, 128, 2, 256, __VA_ARGS__); \
-        } else                                        \
-            ADKV_LAUNCH(KERNEL, 128, 4, __VA_ARGS__); \
+        ADKV_LAUNCH(KERNEL, 128, 4, __VA_ARGS__);     \
         break;                                        \
     case 256:                                         \
         ADKV_LAUNCH(KERNEL, 256, 4, __VA_ARGS__);     \
@@ -2483,7 +2455,11 @@ static int threads_per_workgroup(long threads)
 // 48.9 / 48.6 and 47.5 / 43.0, 64 x 200 12.7 / 12.9 and 12.7 / 10.9; every 256: 1 x 4096 10.4 / 8.1 and 12.4 / 8.3, 2 x 8192
 // 15.3 / 15.0 and 17.8 / 15.1.
 // A buffer descriptor holds a segment's codes: rows of 2^24 tokens and more stay with the other kernels.
+// forward_qk's launches of more waves than that, up to two per SIMD, take two channels per lane (a head per wave, see
+// PairScores): twice the waves of four channels, each with half the instruction stream per token; with more waves per SIMD
+// the four-channel lanes do less work in total.
 static bool qk_lone(int BH, int nseg, int T) { return 2 * padded_units<64>(BH, nseg) <= 3L * n_simd() && T < 1 << 24; }
+static bool qk_pair(int BH, int nseg) { return padded_units<32>(BH, nseg) <= 2L * n_simd(); }
 static bool ov_lone(int BH, int nseg, int T) { return padded_units<64>(BH, nseg) <= 2L * n_simd() && T < 1 << 24; }
 #define ADKV_LAUNCH_LONE_(KERNEL, BLK, ...) \
     hipLaunchKernelGGL(KERNEL<BLK>, dim3((unsigned)((threads + (BLK)-1) / (BLK))), dim3(BLK), 0, st, __VA_ARGS__)
@@ -3451,7 +3427,7 @@ static const char *decode_kernel_name(bool ov, int B, int Hq, int H, int T, int 
         const long units = padded_units<32>(BH, seg.nseg);
         if (ov ? ov_lone(BH, seg.nseg, T) : qk_lone(BH, seg.nseg, T))
             return "lone_kernel (shared table, one channel per lane)";
-        if (units / 2 <= n_simd())
+        if (!ov && qk_pair(BH, seg.nseg))
             return "kernel<128,2,256> (shared table, two channels per lane)";
         const int blk = threads_per_workgroup(units * 32);
         return blk == 1024 ? "kernel<128,4,1024> (shared table)"
@@ -3518,6 +3494,12 @@ static int forward_qk_impl(const void *q, void *k_cache, const void *k_new, void
         const FtParams p = {(const h1 *)zp, (const h1 *)sc, (const h1 *)alpha, (const h1 *)beta, (const h1 *)tgt};
         ADKV_LAUNCH_LONE(qk_lone_kernel, (const h1 *)q,
                            (uint4 *)k_cache, (const h1 *)k_new, (h1 *)logits, p, BH, H, T, n_super_cap, (h1 *)state_out, seg);
+        return check_launch();
+    }
+    if (D == 128 && qk_pair(BH, seg.nseg)) {
+        const long threads = padded_units<64>(BH, seg.nseg) * 64;
+        ADKV_LAUNCH_(qk_kernel, 128, 2, 256, (const h1 *)q, (uint4 *)k_cache, (const h1 *)k_new, (h1 *)logits, (const h1 *)zp,
+                     (const h1 *)sc, (const h1 *)alpha, (const h1 *)beta, (const h1 *)tgt, BH, H, T, n_super_cap, (h1 *)state_out, seg);
         return check_launch();
     }
     ADKV_DISPATCH_D(qk_kernel, (const h1 *)q, (uint4 *)k_cache, (const h1 *)k_new, (h1 *)logits,

@@ -149,6 +149,8 @@ def test_library_names_the_kernels_of_keys_and_of_values():
     assert names(48, 32, 32, 1024, 0) == (lone, lone)
     assert names(60, 32, 32, 1024, 0) == names(64, 32, 32, 200) == (two, lone)
     assert names(65, 32, 32, 200) == ("kernel<128,4,256>",) * 2
+    # beyond what a buffer descriptor covers
+    assert names(1, 2, 2, (1 << 24) - 1, 0) == (lone, lone) and names(1, 2, 2, 1 << 24, 0) == (two, "kernel<128,4,256>")
     assert names(128, 64, 8, 300, 0) == (pair, pair)
     # eight query heads from two waves of two channels per SIMD on, four from three
     assert names(16, 64, 8, 4096) == (pair, pair) and names(16, 64, 8, 5000) == (pair, gqa % 8)
