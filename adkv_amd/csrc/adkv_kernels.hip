@@ -2463,16 +2463,17 @@ static bool qk_pair(int BH, int nseg) { return padded_units<32>(BH, nseg) <= 2L 
 static bool ov_lone(int BH, int nseg, int T) { return padded_units<64>(BH, nseg) <= 2L * n_simd() && T < 1 << 24; }
 #define ADKV_LAUNCH_LONE_(KERNEL, BLK, ...) \
     hipLaunchKernelGGL(KERNEL<BLK>, dim3((unsigned)((threads + (BLK)-1) / (BLK))), dim3(BLK), 0, st, __VA_ARGS__)
-#define ADKV_LAUNCH_LONE(KERNEL, ...)                                  \
+// MOST: the largest workgroup that the rule above asks for
+#define ADKV_LAUNCH_LONE(KERNEL, MOST, ...)                            \
     do {                                                               \
         const long threads = padded_units<64>(BH, seg.nseg) * 128;     \
         const int blk = threads_per_workgroup(threads);                \
-        if (blk == 1024)                                               \
-            ADKV_LAUNCH_LONE_(KERNEL, 1024, __VA_ARGS__);              \
+        if (blk == 256)                                                \
+            ADKV_LAUNCH_LONE_(KERNEL, 256, __VA_ARGS__);               \
         else if (blk == 768)                                           \
             ADKV_LAUNCH_LONE_(KERNEL, 768, __VA_ARGS__);               \
         else                                                           \
-            ADKV_LAUNCH_LONE_(KERNEL, 256, __VA_ARGS__);               \
+            ADKV_LAUNCH_LONE_(KERNEL, MOST, __VA_ARGS__);              \
     } while (0)
 
 // Matrix-core kernels (head dim 128), four channels per lane: 12- or 16-wave workgroups by the same
@@ -3492,7 +3493,7 @@ static int forward_qk_impl(const void *q, void *k_cache, const void *k_new, void
     }
     if (D == 128 && qk_lone(BH, seg.nseg, T)) {
         const FtParams p = {(const h1 *)zp, (const h1 *)sc, (const h1 *)alpha, (const h1 *)beta, (const h1 *)tgt};
-        ADKV_LAUNCH_LONE(qk_lone_kernel, (const h1 *)q,
+        ADKV_LAUNCH_LONE(qk_lone_kernel, 768, (const h1 *)q,
                            (uint4 *)k_cache, (const h1 *)k_new, (h1 *)logits, p, BH, H, T, n_super_cap, (h1 *)state_out, seg);
         return check_launch();
     }
@@ -3701,7 +3702,7 @@ static int forward_ov_impl(const void *attn, void *v_cache, const void *v_new, v
                            (const h1 *)beta, (const h1 *)tgt, B, H, T, n_super_cap, (h1 *)state_out, seg);
     } else if (D == 128 && ov_lone(BH, seg.nseg, T)) {
         const FtParams p = {(const h1 *)zp, (const h1 *)sc, (const h1 *)alpha, (const h1 *)beta, (const h1 *)tgt};
-        ADKV_LAUNCH_LONE(ov_lone_kernel, (const h1 *)attn,
+        ADKV_LAUNCH_LONE(ov_lone_kernel, 1024, (const h1 *)attn,
                            (uint4 *)v_cache, (const h1 *)v_new, (h1 *)out, (float *)workspace, p, BH, H, T, n_super_cap,
                            (h1 *)state_out, seg);
     } else {
