@@ -6,7 +6,7 @@ import torch
 
 from adkv_amd import _lib, synth
 from adkv_amd.kernel import gemv
-from tests.test_gpu_parity import _np16, test_checkpointed_segments, test_forward_qk_and_ov
+from tests.test_gpu_parity import _bf16_case, test_checkpointed_segments, test_forward_qk_and_ov
 
 pytestmark = pytest.mark.gpu
 
@@ -51,3 +51,12 @@ def test_the_step_and_the_calls_agree_bit_for_bit(gpu, T, S):
     assert torch.equal(w.contiguous().view(torch.int16), w2.contiguous().view(torch.int16))
     assert torch.equal(out.view(torch.int16), out2.view(torch.int16))
     assert torch.equal(caches[0], two[0]) and torch.equal(caches[1], two[1])
+
+
+@pytest.mark.parametrize("B,H,T", [(2, 4, 1600), (3, 5, 1541), (65, 4, 520)])
+def test_bfloat16_results_of_rows_in_one_piece(gpu, B, H, T):
+    """Steps that are neither one launch nor two, without checkpoints: forward_ov's waves write the results themselves."""
+    L = _lib.lib()
+    assert L.adkv_decode_step_launches(B, H, H, T, 128, 4, 0, 0, 0) == 3
+    assert L.adkv_decode_ov_kernel_name(B, H, H, T, 128, 4, 0, 0).startswith(b"lone_kernel")
+    _bf16_case(gpu, B, H, H, T, 0, 4)

@@ -670,12 +670,12 @@ def test_decode_step_replays_from_a_captured_graph(gpu, H, Hq, T, S, bits):
 
 
 @pytest.mark.parametrize("B,H,Hq,T,S,bits", [
-    (2, 4, 4, 257, 0, 4),        # vector kernels, one segment
-    (2, 3, 3, 530, 64, 4),       # vector kernels, a few segments (narrow partial-sum kernel)
+    (2, 4, 4, 257, 0, 4),        # one launch
+    (2, 3, 3, 530, 64, 4),       # one channel per lane, a few segments (narrow partial-sum kernel)
     (1, 2, 2, 2100, 64, 4),      # many segments (wide partial-sum kernel)
-    (40, 32, 32, 300, 64, 4),    # enough units for four channels per lane
-    (2, 2, 8, 530, 64, 4),       # matrix-core kernels, 4 query heads per KV head
-    (1, 2, 16, 200, 32, 2),      # 2-bit codes, 8 query heads per KV head
+    (40, 32, 32, 300, 64, 4),    # the per-head-table kernels by the library's choice
+    (2, 2, 8, 530, 64, 4),       # two launches, 4 query heads per KV head
+    (1, 2, 16, 200, 32, 2),      # two launches, 2-bit codes, 8 query heads per KV head
     (3, 2, -2, 530, 64, 4),      # the per-head-table kernels (forced, 32 lanes per head), a few segments
     (5, 3, -3, 257, 0, 4),       # the per-head-table kernels (forced, 32 lanes per head), one segment
     (3, 2, -102, 530, 64, 4),    # the per-head-table kernels (forced, 16 lanes per head), a few segments

@@ -6,7 +6,7 @@ import pytest
 import torch
 
 from adkv_amd import _lib
-from tests.test_gpu_segment_step import test_against_the_three_calls, test_masked_segments_and_rows
+from tests.test_gpu_segment_step import test_against_the_three_calls, test_error_against_64_bits, test_masked_segments_and_rows
 
 pytestmark = pytest.mark.gpu
 
@@ -64,3 +64,12 @@ def test_two_bits_workgroup_sizes(gpu, oracle, B, Hq, H, T, waves):
 def test_masks(gpu, Hq, H, D, low):
     assert _runs(3, Hq, H, D, 768, 4, 256) > 0
     test_masked_segments_and_rows(gpu, 3, Hq, H, D, 768, low)
+
+
+@pytest.mark.parametrize("q_scale", [0.3, 1.0])
+@pytest.mark.parametrize("B,Hq,H,D,T,bits", [(9, 8, 8, 512, 700, 4), (6, 16, 16, 256, 1290, 4), (4, 32, 32, 128, 1100, 4), (12, 8, 2, 128, 1100, 4),
+                                             (12, 16, 2, 128, 1500, 2)])
+def test_no_further_from_64_bits(gpu, oracle, B, Hq, H, D, T, bits, q_scale):
+    """One query head on the vector pipe and, with 512 channels, on the matrix cores; four and eight of them."""
+    assert _runs(B, Hq, H, D, T, bits, 256) > 0
+    test_error_against_64_bits(gpu, oracle, B, Hq, H, D, T, bits, q_scale)
