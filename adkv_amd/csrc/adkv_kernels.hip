@@ -2931,16 +2931,23 @@ static int launch_step_grouped(int GQ, long waves, hipStream_t st, Args... args)
 // Whether step_lone_kernel takes a step of the two launches, and with which workgroups: a wave's 64 channels bring
 // twice the waves of two channels per lane and four or eight times those of wide heads, and pay as long as a CU holds
 // them at once: 16 waves, and 12 / 8 with four / eight query heads, whose logits take more of the LDS; with one or two
-// query heads of 128 channels, whose other form has its waves' LDS reads covered by then, 12.  us per step on the device,
-// step_segments_kernel / this, waves per CU in brackets: head dim 512, 9 x 8 heads x 80 (2) 22.8 / 11.8, 2 x 8 x 1000 (2)
-// 47.7 / 18.7, 8 x 8 x 2000 (16) 48.8 / 28.9, 10 x 8 x 2000 (20) 48.9 / 49.1; head dim 256, 1 x 8 x 300 30.3 / 14.1, 2 x 16 x
-// 5021 (10) 31.7 / 23.2, 4 x 8 x 8190 (16) 33.7 / 30.4, 5 x 8 x 8000 (20) 44.6 / 49.2; head dim 128, 1 x 32 x 2000 (2)
-// 20.7 / 15.7, 4 x 32 x 2000 (8) 21.3 / 19.5, 6 x 32 x 2000 (12) 27.3 / 24.1, 8 x 32 x 2000 (16) 27.4 / 28.0; two query heads, 4 x 16
-// x 2000 (4) 22.6 / 16.3, 8 x 16 x 2000 (8) 23.3 / 20.3, 12 x 16 x 2000 (12) 30.0 / 25.6, 16 x 16 x 2000 (16) 31.1 / 30.7; four, 1 x 8
-// x 603 22.2 / 15.3, 28 x 8 x 936 (7) 24.5 / 21.3, 8 x 8 x 6000 (12) 33.5 / 28.4, 8 x 8 x 7000 (14) 34.1 / 46; eight, 3 x 8 x
-// 113 18.9 / 13.7, 3 x 8 x 4799 (4) 29.4 / 19.8, 8 x 8 x 4000 (8) 35.1 / 29.4, 8 x 8 x 8000 (16) 45.4 / 46.1.  2-bit codes:
-// 1 x 32 x 2000 20.1 / 13.8, 6 x 32 x 2000 26.1 / 21.8, 12 x 16 x 2000 27.7 / 22.9, 2 x 8 x 8664 22.9 / 20.6, 8 x 8 x 6000 30.9 / 26.6, 8 x 8
-// x 4000 with eight 31.0 / 26.1.
+// query heads of 128 channels, whose other form has its waves' LDS reads covered by then, 12.  us per step on the
+// device, step_segments_kernel / this, waves per CU in brackets:
+//   512 channels: 9 x 8 heads x 80 (2) 22.8 / 11.8, 2 x 8 x 1000 (2) 47.7 / 18.7, 8 x 8 x 2000 (16) 48.8 / 28.9
+//   256: 1 x 8 x 300 30.3 / 14.1, 2 x 16 x 5021 (10) 31.7 / 23.2, 4 x 8 x 8190 (16) 33.7 / 30.4
+//   128: 1 x 32 x 2000 (2) 20.7 / 15.7, 4 x 32 x 2000 (8) 21.3 / 19.5, 6 x 32 x 2000 (12) 27.3 / 24.1, 8 x 32 x 2000 (16)
+//     27.4 / 28.0
+//   two query heads: 4 x 16 x 2000 (4) 22.6 / 16.3, 8 x 16 x 2000 (8) 23.3 / 20.3, 12 x 16 x 2000 (12) 30.0 / 25.6,
+//     16 x 16 x 2000 (16) 31.1 / 30.7
+//   four: 1 x 8 x 603 22.2 / 15.3, 28 x 8 x 936 (7) 24.5 / 21.3, 8 x 8 x 6000 (12) 33.5 / 28.4, 8 x 8 x 7000 (14) 34.1 / 46
+//   eight: 3 x 8 x 113 18.9 / 13.7, 3 x 8 x 4799 (4) 29.4 / 19.8, 8 x 8 x 4000 (8) 35.1 / 29.4, 8 x 8 x 8000 (16) 45.4 / 46.1
+//   2-bit codes: 1 x 32 x 2000 20.1 / 13.8, 6 x 32 x 2000 26.1 / 21.8, 12 x 16 x 2000 27.7 / 22.9, 2 x 8 x 8664 22.9 / 20.6,
+//     8 x 8 x 6000 30.9 / 26.6, 8 x 8 x 4000 with eight query heads 31.0 / 26.1
+// Beyond 16 waves of wide heads the launch takes two rounds or more, and the line is a cautious one: up to 24 workgroups
+// smaller than the CU are still the faster ones, by 32 they are not.  step_segments_kernel / this in workgroups of 4,
+// 12 and 16 waves (512 channels: 8 and 16): 256 channels, 5 x 8 x 8000 (20) 47.0 / 43.2, 44.3, 51.5, 6 x 8 x 8000 (24) 47.5
+// / 47.4, 44.9, 51.8, 8 x 8 x 8000 (32) 49.2 / 60.2, 62.7, 56.7; 512, 10 x 8 x 2000 (20) 50.7 / 48.5, 51.8, 12 x 8 x 2000 (24)
+// 51.1 / 49.8, 51.9, 16 x 8 x 2000 (32) 51.8 / 64.2, 56.7 (these with the rotary embedding's launch, some 2 us).
 // Small workgroups spread best; what they leave free of a CU's LDS (the table takes 64 KB) holds a second one only with
 // one query head.  A workgroup of as many waves as the CU is to hold otherwise: 2 x 16 x 5021 of 256 channels with 4, 8, 12
 // and 16 waves 26.5, 32.6, 23.3, 27.4; 28 x 8 x 936 with four query heads 28.1, 21.3, 25.4.

@@ -493,7 +493,9 @@ __global__ __launch_bounds__(BLK) void ov_lone_kernel(const h1 *attn, uint4 *cac
     s.start(cache, p, v_new, un.bx % H, un.bx, un.c, un.seg, T, n_super_cap, sa);
     const h1 *wb = attn + (size_t)un.bx * sa.row_pitch + s.t0;
     // a chunk's weights, eight tokens per lane, a chunk ahead: as a load of eight for all lanes alike, one per supergroup,
-    // they were a tenth of a lone wave's time (more where rows are only 2-byte aligned)
+    // they were a tenth of a lone wave's time (more where rows are only 2-byte aligned).  As built the wave waits at each
+    // chunk for its code loads too; with whole chunks in a loop of their own, which waits for the weights alone, it
+    // was slower: 1 x 32 heads x 1024 tokens 14.8 / 15.7 us, 2 x 8 x 700 12.0 / 13.1, 3 x 40 x 5000 61.8 / 66.0.
     uint4 ahead = make_uint4(0, 0, 0, 0);
     auto load_chunk = [&](int sg) __attribute__((always_inline)) {
         if (s.nfull > 0)

@@ -295,9 +295,10 @@ __device__ __forceinline__ void lone_weights(const float *share, int stride, h1 
         *ml = make_float4(mx, sum, rounded, 0.0f);
 }
 
-// The same launch with one channel per lane, a KV head over D / 64 waves (adkv_lone.h): segments of at most 256 tokens.  With few waves per SIMD a step takes as long as one wave's instructions per token, and a lane with
-// four or eight channels has two and four times as many of them; the waves of a head meet once, behind the keys, where
-// each has left its share of the logits (fp32) in the LDS, and with several query heads again behind the weights.
+// The same launch with one channel per lane, a KV head over D / 64 waves (adkv_lone.h): segments of at most 256 tokens.
+// With few waves per SIMD a step takes as long as one wave's instructions per token, and a lane with four or eight
+// channels has two and four times as many of them; the waves of a head meet once, behind the keys, where each has left
+// its share of the logits (fp32) in the LDS, and with several query heads again behind the weights.
 // Of the 256 + 256 tokens of a full segment a lone wave takes some 9 us (19 ns per token, step_segments_kernel 27 with two
 // channels per lane, 50 with four and 90 with eight); from four waves per SIMD on vector issue holds it, 23 cycles per
 // wave and token.  us per step: 2 x 8 heads x 1000 of 512 channels 47.7 / 18.7, 2 x 16 x 5021 of 256 31.7 / 23.2, 3 x 8 x 4799 with
@@ -402,9 +403,10 @@ __global__ __launch_bounds__(BLK) void step_lone_kernel(
 
 // The segments of a row put together, by waves of two kinds: VECS x 512 of its weights each, or a share of its
 // outputs: all 128 channels in two groups of segments, or, with many segments, 16 channels in 16 groups.
-// Sums are taken in a fixed order.  A wave's chain of loads holds it, then the bytes: a row's maxima and sums lie side by side
-// (a line each, as they lay, a wave of 64 segments touched 64 lines for them), and long rows give a wave two vectors of weights per
-// lane, so that all waves are resident.  us per step, 8 x 8 heads x 16 001 with four query heads 58.8 / 58.2.
+// Sums are taken in a fixed order.  A wave's chain of loads holds it, then the bytes.  us of this kernel, other form / this:
+// a row's maxima and sums side by side (a segment's beside each other, a wave of 64 segments touches 64 lines for them):
+// 1 x 8 heads x 60 000 with four query heads 8.8 / 7.4, 8 x 8 x 16 001 equal; long rows with two vectors of weights per
+// lane, so that all waves are resident: 8 x 8 x 16 001 8.0 / 7.5; masks read as vectors: 64 x 32 x 663 5.5 / 5.1.
 template <int VECS>
 __global__ __launch_bounds__(256) void step_combine_kernel(
     const h1 *__restrict__ logits, h1 *__restrict__ weights, h1 *__restrict__ out, Mask mk,
