@@ -37,10 +37,11 @@ struct LoneLoads {
     static constexpr int SHIFT = BITS == 4 ? 3 : 4;                                // of tokens to words
     uint32_t *cbh;      // this head, this channel
     // this segment's whole supergroups.  Reads past them are dropped: a load's whole position is in its vector offset, which
-    // is what the range check looks at (of the scalar offset the check is not documented to take account), one
-    // addition for PF of them (with a clamped index it was five instructions a load)
+    // is what the range check looks at (of the scalar offset the check is not documented to take account).  The offset
+    // moves on once for PF loads, whose places behind it are in the instructions (with an addition per load a step of
+    // 1 x 32 heads x 603 tokens took 15.8 us instead of 15.4; with a clamped index it was five instructions a load)
     __amdgpu_buffer_rsrc_t codes;
-    int lane4;
+    int next; // where in it this lane's next PF words are
     int t0, t1, nfull, ntail;
     bool last, from_ckpt;
     h1 zp, sc, al, be, tg;
@@ -58,7 +59,7 @@ struct LoneLoads {
         ntail = (t1 - t0) & (TPW - 1); // of the last segment only: the others are whole intervals
         cbh = reinterpret_cast<uint32_t *>(cache) + (size_t)bx * n_super_cap * D + c;
         codes = __builtin_amdgcn_make_buffer_rsrc(cbh - c + (size_t)(t0 >> SHIFT) * D, 0, nfull * D * 4, 0x00027000);
-        lane4 = c * 4;
+        next = c * 4;
         from_ckpt = iv > 0;
         ck = 0;
         if (from_ckpt)
@@ -70,20 +71,29 @@ struct LoneLoads {
         tg = p.tg[pi];
 #pragma unroll
         for (int i = 0; i < PF; i++)
-            buf[i] = load(0, i);
+            buf[i] = load(i);
+        move_on();
         tail = cbh[(size_t)(last ? T >> SHIFT : 0) * D];
         fresh = reinterpret_cast<const uint16_t *>(x_new)[(size_t)bx * D + c];
     }
-    // supergroup sg + i, i < PF; read once: not kept in the caches
-    __device__ __forceinline__ uint32_t load(int sg, int i) const
+    // the i-th of the next PF words; read once: not kept in the caches
+    __device__ __forceinline__ uint32_t load(int i) const
     {
-        return __builtin_amdgcn_raw_buffer_load_b32(codes, lane4 + sg * D * 4 + i * D * 4, 0, 2);
+        return __builtin_amdgcn_raw_buffer_load_b32(codes, next + i * D * 4, 0, 2);
     }
-    // behind unit i of LONE_PF (at that unit of `first` on): the word that it was the last of, PF words further
-    __device__ __forceinline__ void refill(int first, int i)
+    // behind unit i of LONE_PF: the word that it was the last of, PF words further
+    __device__ __forceinline__ void refill(int i)
     {
         if (i % UPS == UPS - 1)
-            buf[i / UPS] = load((first >> (SHIFT - 3)) + PF, i / UPS);
+            buf[i / UPS] = load(i / UPS);
+        if (i == LONE_PF - 1)
+            move_on();
+    }
+    // hidden from the loop's optimiser, which would count from the last of the places, and add for each of the others
+    __device__ __forceinline__ void move_on()
+    {
+        next += PF * D * 4;
+        asm("" : "+v"(next));
     }
     __device__ __forceinline__ int code(int t) const { return (int)(tail >> (BITS * t) & Code<BITS>::FIELD) + Code<BITS>::QLO; }
     __device__ __forceinline__ Lone state() const
@@ -247,8 +257,8 @@ struct LoneScores {
         }
     }
 
-    // units sg0 .. sg0 + n of the segment, sg0 a multiple of LONE_PF; the shares of their logits to part[0..8n)
-    __device__ __forceinline__ void run(const uint2 *lut, uint32_t lane_copy, Lone &st, LoneLoads<D, BITS> &s, int sg0, int n, float *part)
+    // the segment's next n units, of all calls but the last a multiple of LONE_PF; the shares of their logits to part[0..8n)
+    __device__ __forceinline__ void run(const uint2 *lut, uint32_t lane_copy, Lone &st, LoneLoads<D, BITS> &s, int n, float *part)
     {
         if (n <= 0)
             return;
@@ -260,7 +270,7 @@ struct LoneScores {
         auto body = [&](int sg, auto ic, auto &&group_done) __attribute__((always_inline)) {
             constexpr int i = decltype(ic)::value;
             lone_lookup<BITS>(e[(i & 1) ^ 1], lut, s.buf, (i + 1) % LONE_PF, lane_copy); // stale past the end: looked up, never used
-            s.refill(sg0 + sg - i, i);
+            s.refill(i);
             __builtin_amdgcn_sched_barrier(0);
             uint32_t x[4];
             lone_eight(st, e[i & 1], x);
@@ -354,10 +364,10 @@ struct LoneScores {
     }
 };
 
-// forward_ov of a wave's 64 channels: adds units sg0 .. sg0 + n of the segment to acc, sg0 a multiple of
+// forward_ov of a wave's 64 channels: adds the segment's next n units to acc, of all calls but the last a multiple of
 // LONE_PF.  w: their weights, in LDS.
 template <int D, int BITS>
-__device__ __forceinline__ void lone_values(const uint2 *lut, uint32_t lane_copy, LoneLoads<D, BITS> &s, Lone &st, int sg0, int n, const h1 *w,
+__device__ __forceinline__ void lone_values(const uint2 *lut, uint32_t lane_copy, LoneLoads<D, BITS> &s, Lone &st, int n, const h1 *w,
                                             float &acc)
 {
     if (n <= 0)
@@ -372,7 +382,7 @@ __device__ __forceinline__ void lone_values(const uint2 *lut, uint32_t lane_copy
         constexpr int i = decltype(ic)::value, half = i & 1;
         lone_lookup<BITS>(e[half ^ 1], lut, s.buf, (i + 1) % LONE_PF, lane_copy); // stale past the end: looked up, never used
         wv[half ^ 1] = w4[sg + 1]; // so are these: the caller's LDS goes on behind them
-        s.refill(sg0 + sg - i, i);
+        s.refill(i);
         __builtin_amdgcn_sched_barrier(0);
         lone_eight_weighted(st, e[half], wv[half], acc);
         __builtin_amdgcn_sched_barrier(0);
@@ -418,7 +428,7 @@ __device__ __forceinline__ void lone_values_grouped(const uint2 *lut, uint32_t l
 #pragma unroll
         for (int n = 0; n < NB; n++)
             wv[half ^ 1][n] = w4[n][sg + 1]; // so are these: a row goes on for a vector
-        s.refill(sg - i, i);
+        s.refill(i);
         __builtin_amdgcn_sched_barrier(0);
         uint32_t x[4];
         lone_eight<true>(st, e[half], x);
@@ -467,7 +477,7 @@ __global__ __launch_bounds__(BLK) void qk_lone_kernel(const h1 *q, uint4 *cache,
     const int longest = sa.nseg > 1 ? sa.seg_tokens : T; // every wave of the workgroup takes part in every exchange
     for (int t = 0; t < longest; t += LONE_CHUNK) {
         const int n = max(0, min(LONE_CHUNK / 8, s.nfull - t / 8));
-        scores.run(lut, lane_copy, st, s, t / 8, n, part);
+        scores.run(lut, lane_copy, st, s, n, part);
         flush(t, 8 * n);
     }
     if (s.last)
@@ -512,7 +522,7 @@ __global__ __launch_bounds__(BLK) void ov_lone_kernel(const h1 *attn, uint4 *cac
         weights[lane] = ahead;
         __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront"); // read by the wave's other lanes
         load_chunk(sg + LONE_CHUNK / 8);
-        lone_values(lut, lane_copy, s, st, sg, min(LONE_CHUNK / 8, s.nfull - sg), reinterpret_cast<const h1 *>(weights), acc);
+        lone_values(lut, lane_copy, s, st, min(LONE_CHUNK / 8, s.nfull - sg), reinterpret_cast<const h1 *>(weights), acc);
     }
     lone_values_end(s, st, [&](int t) { return wb[t]; }, un.bx, un.c, T, state_out, sa, true, acc);
     if (sa.nseg == 1) {

@@ -339,7 +339,7 @@ __global__ __launch_bounds__(BLK) void step_lone_kernel(
         Lone st = s.state();
         float *mine = shares + part * GQ * LONE_SEG;
         scores.ready(ka.act_bf16);
-        scores.run(lut, lane_copy, st, s, 0, s.nfull * s.UPS, mine);
+        scores.run(lut, lane_copy, st, s, s.nfull * s.UPS, mine);
         if (s.last)
             scores.finish(s, st, bx, c, T, nullptr, ka, true, mine + s.nfull * s.TPW);
         // the values' state and codes travel while the weights are made
@@ -373,7 +373,7 @@ __global__ __launch_bounds__(BLK) void step_lone_kernel(
         // measured, adding on the vector pipe / on the matrix cores: 4 x 8 x 8190 of 256 channels 30.4 / 31.3, 8 x 32 x 2000
         // 28.0 / 29.2, 4 x 32 x 2000 19.6 / 19.3; 8 x 8 x 2000 of 512 30.5 / 28.9
         float acc = 0.0f;
-        lone_values(lut, lane_copy, s, st, 0, s.nfull * s.UPS, p, acc);
+        lone_values(lut, lane_copy, s, st, s.nfull * s.UPS, p, acc);
         lone_values_end(s, st, [&](int t) { return p[t]; }, bx, c, T, nullptr, va, true, acc);
         *o = acc;
         return;

@@ -45,7 +45,7 @@ __global__ __launch_bounds__(512) void small_step_kernel(
         Lone st = s.state();
         float *part = share + half * SMALL_ROW + s.t0;
         scores.ready(ka.act_bf16);
-        scores.run(lut, lane_copy, st, s, 0, s.nfull, part);
+        scores.run(lut, lane_copy, st, s, s.nfull, part);
         if (s.last)
             scores.finish(s, st, bx, c, T, nullptr, ka, true, part + s.nfull * 8);
         // the V segment's state and codes are on their way while the other waves finish
@@ -83,7 +83,7 @@ __global__ __launch_bounds__(512) void small_step_kernel(
         const h1 *wb = w + s.t0;
         Lone st = s.state();
         float acc = 0.0f;
-        lone_values(lut, lane_copy, s, st, 0, s.nfull, wb, acc);
+        lone_values(lut, lane_copy, s, st, s.nfull, wb, acc);
         lone_values_end(s, st, [&](int t) { return wb[t]; }, bx, c, T, nullptr, va, true, acc);
         partial[seg * D + c] = acc;
     }

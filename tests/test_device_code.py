@@ -154,3 +154,4 @@ def test_code_loads_keep_their_position_where_the_range_check_sees_it(listings):
              for op, args, _ in code if op.startswith("buffer_load_dword")]
     assert len(found) > 600                                                # the listings are what they should be
     assert not [f for f in found if not re.search(r"\], 0 offen", f[1])][:5]
+    assert sum("offset:" in args for _, args in found) > len(found) / 2    # and the places of a group in the instructions
