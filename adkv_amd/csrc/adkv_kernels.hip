@@ -4046,8 +4046,8 @@ int adkv_decode_step(const void *q, void *k_cache, void *v_cache, const void *k_
             va.ckpt = (h1 *)v_ckpt;
             const FtParams kp = ft_params(k_params), vp = ft_params(v_params);
             hipLaunchKernelGGL(small_step_kernel, dim3((unsigned)(B * H)), dim3(512), 0, (hipStream_t)stream, (const h1 *)q,
-                               (uint4 *)k_cache, (const h1 *)k_new, (uint4 *)v_cache, (const h1 *)v_new, mk, (h1 *)weights, (h1 *)out, kp, vp, H, T,
-                               n_super_cap, scaling, ka, va);
+                               (uint4 *)k_cache, (const h1 *)k_new, (uint4 *)v_cache, (const h1 *)v_new, mk, (h1 *)weights,
+                               (h1 *)out, kp, vp, H, T, n_super_cap, scaling, ka, va);
             return (rc = check_launch()) ? rc : mark_one_launch(stream);
         }
     }
