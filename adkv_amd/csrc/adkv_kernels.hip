@@ -2832,9 +2832,9 @@ static int fused_step_plan(Seg &ka, Seg &va, int B, int Hq, int H, int T, int D,
     return lanes;
 }
 
-// Whether a step runs as small_step_kernel, and its plan: a workgroup per (sequence, head), one per CU, two
+// Whether a step runs as small_step_kernel, and its plan: a workgroup per (sequence, head), one per CU, four
 // waves per segment.  us per step on the device, three or four launches / one, sequences x heads x tokens: 1 x 32 x 603
-// 25.6 / 13.2 (and 15 us of host time / 5), 8 x 32 x 1000 27.7 / 20.0, 4 x 32 x 200 20.4 / 12.8, 2 x 8 x 64 12.8 / 8.8.
+// 25.6 / 11.9 (and 15 us of host time / 5), 8 x 32 x 1000 27.7 / 17.3, 4 x 32 x 200 20.4 / 11.0, 2 x 8 x 64 12.8 / 7.8.
 // With five to eight segments four waves share a SIMD while other CUs idle, and beyond one workgroup per CU (its LDS
 // allows no second) a launch takes two rounds: those stay with the separate launches.
 static bool small_step_plan(Seg &seg, int B, int Hq, int H, int T, int D, int bits, void *k_ckpt, void *v_ckpt,
@@ -4045,7 +4045,9 @@ int adkv_decode_step(const void *q, void *k_cache, void *v_cache, const void *k_
             Seg va = ka;
             va.ckpt = (h1 *)v_ckpt;
             const FtParams kp = ft_params(k_params), vp = ft_params(v_params);
-            hipLaunchKernelGGL(small_step_kernel, dim3((unsigned)(B * H)), dim3(512), 0, (hipStream_t)stream, (const h1 *)q,
+            const auto kernel = ka.nseg == 1 ? small_step_kernel<1> : ka.nseg == 2 ? small_step_kernel<2>
+                              : ka.nseg == 3 ? small_step_kernel<3> : small_step_kernel<4>;
+            hipLaunchKernelGGL(kernel, dim3((unsigned)(B * H)), dim3((unsigned)ka.nseg * 256), 0, (hipStream_t)stream, (const h1 *)q,
                                (uint4 *)k_cache, (const h1 *)k_new, (uint4 *)v_cache, (const h1 *)v_new, mk, (h1 *)weights,
                                (h1 *)out, kp, vp, H, T, n_super_cap, scaling, ka, va);
             return (rc = check_launch()) ? rc : mark_one_launch(stream);

@@ -388,6 +388,48 @@ __device__ __forceinline__ void lone_values(const uint2 *lut, uint32_t lane_copy
         __builtin_amdgcn_sched_barrier(0);
     });
 }
+// The values of a segment's first tokens before their weights are there: whole groups of LONE_PF units, at most UNITS; x[4u..]
+// are unit u's.  Returns the units done, with which lone_values goes on.
+template <int UNITS, int D, int BITS>
+__device__ __forceinline__ int lone_values_ahead(const uint2 *lut, uint32_t lane_copy, LoneLoads<D, BITS> &s, Lone &st, int n, uint32_t *x)
+{
+    static_assert(UNITS % LONE_PF == 0, "whole groups");
+    uint2 e[2][4];
+    lone_lookup<BITS>(e[0], lut, s.buf, 0, lane_copy);
+    wait_lgkm();
+#pragma unroll
+    for (int g = 0; g < UNITS; g += LONE_PF)
+        if (g + LONE_PF <= n)
+            static_for<LONE_PF>([&](auto ic) __attribute__((always_inline)) {
+                constexpr int i = decltype(ic)::value, half = i & 1;
+                lone_lookup<BITS>(e[half ^ 1], lut, s.buf, (i + 1) % LONE_PF, lane_copy); // stale past the end: looked up, never used
+                s.refill(i);
+                __builtin_amdgcn_sched_barrier(0);
+                lone_eight(st, e[half], x + (g + i) * 4);
+                __builtin_amdgcn_sched_barrier(0);
+            });
+    return min(UNITS, n & ~(LONE_PF - 1));
+}
+// Those values by their weights, in the order of lone_values.  done: what lone_values_ahead returned.
+template <int UNITS>
+__device__ __forceinline__ void lone_weigh(const uint32_t *x, int done, const h1 *w, float &acc)
+{
+    const uint4 *w4 = reinterpret_cast<const uint4 *>(w);
+#pragma unroll
+    for (int g = 0; g < UNITS; g += LONE_PF)
+        if (g < done) {
+#pragma unroll
+            for (int u = g; u < g + LONE_PF; u++) {
+                const uint4 wv = w4[u];
+                const uint32_t ww[4] = {wv.x, wv.y, wv.z, wv.w};
+#pragma unroll
+                for (int k = 0; k < 4; k++) {
+                    acc = __builtin_fmaf((float)as_h2(ww[k]).x, (float)as_h2(x[u * 4 + k]).x, acc);
+                    acc = __builtin_fmaf((float)as_h2(ww[k]).y, (float)as_h2(x[u * 4 + k]).y, acc);
+                }
+            }
+        }
+}
 // The last segment's ragged tail and the appended token.  w1(t): the weight of the segment's token t.
 template <int D, int BITS, typename W1>
 __device__ __forceinline__ void lone_values_end(const LoneLoads<D, BITS> &s, Lone &st, W1 &&w1, int bx, int c, int T, h1 *state_out, const Seg &sa,
