@@ -212,6 +212,37 @@ __device__ __forceinline__ float xor32_add(float s)
     return __builtin_bit_cast(float, x) + __builtin_bit_cast(float, y);
 }
 
+// v + v[lane ^ 1], + that of lane ^ 2, ^ 4 .. ^ 32 of the sums (or the largest of them), in registers: inside 4, 8 and 16 lanes that
+// agree a mirrored lane has what the exchanged one has.  The sums of a butterfly through __shfl_xor bit for bit, without its six trips
+// through the LDS.
+template <int CTRL, bool MAX>
+__device__ __forceinline__ float mirror_fold(float v)
+{
+    const float o = __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), CTRL, 0xF, 0xF, false));
+    return MAX ? fmaxf(v, o) : v + o;
+}
+template <bool MAX>
+__device__ __forceinline__ float wave_reduce(float v)
+{
+    v = mirror_fold<0xB1, MAX>(v);  // quad_perm [1, 0, 3, 2]
+    v = mirror_fold<0x4E, MAX>(v);  // quad_perm [2, 3, 0, 1]
+    v = mirror_fold<0x141, MAX>(v); // row_half_mirror
+    v = mirror_fold<0x140, MAX>(v); // row_mirror
+    unsigned a = __builtin_bit_cast(unsigned, v), b; // see xor16_add
+    asm volatile("v_mov_b32 %0, %1" : "=v"(b) : "v"(a));
+    const u2v r = __builtin_amdgcn_permlane16_swap(a, b, false, false);
+    unsigned x = r.x, y = r.y;
+    asm volatile("" : "+v"(x), "+v"(y));
+    v = MAX ? fmaxf(__builtin_bit_cast(float, x), __builtin_bit_cast(float, y)) : __builtin_bit_cast(float, x) + __builtin_bit_cast(float, y);
+    a = __builtin_bit_cast(unsigned, v);
+    asm volatile("v_mov_b32 %0, %1" : "=v"(b) : "v"(a));
+    const u2v h = __builtin_amdgcn_permlane32_swap(a, b, false, false);
+    x = h.x;
+    y = h.y;
+    asm volatile("" : "+v"(x), "+v"(y));
+    return MAX ? fmaxf(__builtin_bit_cast(float, x), __builtin_bit_cast(float, y)) : __builtin_bit_cast(float, x) + __builtin_bit_cast(float, y);
+}
+
 // Sum over the LPH lanes of a head; every lane of the head gets the total.
 template <int LPH>
 __device__ __forceinline__ float head_allreduce(float v)
@@ -1980,18 +2011,14 @@ __global__ __launch_bounds__(SM_BLOCK) void softmax_wave_kernel(
     const MaskRow<HALF> mk = mask.of<HALF>(row, n);
     float x[NV * SM_VEC], mx;
     softmax_load_chunk<NV, 64>(l, mk, n, 0, scaling, x, mx, lane);
-#pragma unroll
-    for (int m = 1; m < 64; m <<= 1)
-        mx = fmaxf(mx, __shfl_xor(mx, m, 64));
+    mx = wave_reduce<true>(mx);
     float sum = 0.0f;
 #pragma unroll
     for (int k = 0; k < NV * SM_VEC; k++) {
         x[k] = __expf(x[k] - mx);
         sum += x[k];
     }
-#pragma unroll
-    for (int m = 1; m < 64; m <<= 1)
-        sum += __shfl_xor(sum, m, 64);
+    sum = wave_reduce<false>(sum);
     softmax_store_chunk<NV, 64>(w, n, 0, x, 1.0f / sum, lane);
 }
 
@@ -2834,7 +2861,7 @@ static int fused_step_plan(Seg &ka, Seg &va, int B, int Hq, int H, int T, int D,
 
 // Whether a step runs as small_step_kernel, and its plan: a workgroup per (sequence, head), one per CU, four
 // waves per segment.  us per step on the device, three or four launches / one, sequences x heads x tokens: 1 x 32 x 603
-// 25.6 / 11.9 (and 15 us of host time / 5), 8 x 32 x 1000 27.7 / 17.3, 4 x 32 x 200 20.4 / 11.0, 2 x 8 x 64 12.8 / 7.8.
+// 25.6 / 11.0 (and 15 us of host time / 5), 8 x 32 x 1000 27.7 / 16.3, 4 x 32 x 200 20.4 / 11.0, 2 x 8 x 64 12.8 / 7.8.
 // With five to eight segments four waves share a SIMD while other CUs idle, and beyond one workgroup per CU (its LDS
 // allows no second) a launch takes two rounds: those stay with the separate launches.
 static bool small_step_plan(Seg &seg, int B, int Hq, int H, int T, int D, int bits, void *k_ckpt, void *v_ckpt,
