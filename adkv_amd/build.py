@@ -46,7 +46,7 @@ def build_host(verbose: bool = False) -> str:
     cmd = [os.environ.get("CXX", "g++"), "-O2", "-std=c++17", "-fPIC", "-shared", "-Wall",
            f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
            "-isystem", os.path.join(t, "include"), "-I", sysconfig.get_paths()["include"], HOST_SOURCE, "-o", HOST_PATH,
-           "-L", os.path.join(t, "lib"), "-ltorch_python", "-ltorch_cpu", "-lc10", "-L", _DIR, "-l:libadkv_hip.so",
+           "-L", os.path.join(t, "lib"), "-ltorch_python", "-ltorch_cpu", "-ltorch_hip", "-lc10", "-L", _DIR, "-l:libadkv_hip.so",
            "-Wl,-rpath,$ORIGIN", "-Wl,--allow-shlib-undefined"]
     if verbose:
         print(" ".join(cmd), file=sys.stderr)

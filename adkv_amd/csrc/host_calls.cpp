@@ -13,6 +13,7 @@
 
 #include <ATen/ATen.h>
 #include <ATen/PythonTorchFunctionTLS.h>
+#include <ATen/ops/empty_cuda_dispatch.h>
 #include <c10/core/impl/LocalDispatchKeySet.h>
 #include <c10/core/impl/DeviceGuardImplInterface.h>
 
@@ -67,6 +68,14 @@ bool current(c10::Device device, void *&stream)
     return true;
 }
 
+// at::empty where its dispatch ends for an ordinary thread (unwatched), on like's device.  The host's part of a step of
+// 1 x 32 heads x 603 tokens with its rotary embedding, four tensors: 14.4 us, 13.6 without the dispatcher, 13.1 without working out
+// the workspace's size a second time (see decode).
+at::Tensor fresh(at::IntArrayRef sizes, const at::Tensor &like, at::ScalarType type)
+{
+    return at::cuda::empty(sizes, type, at::kStrided, like.device(), false, c10::nullopt);
+}
+
 PyObject *pair(at::Tensor &&a, at::Tensor &&b)
 {
     PyObject *x = THPVariable_Wrap(std::move(a)), *y = THPVariable_Wrap(std::move(b));
@@ -108,8 +117,8 @@ PyObject *rope_qk(PyObject *, PyObject *const *args, Py_ssize_t n)
         Py_RETURN_NONE;
     at::Tensor qo, ko;
     int rc;
-    qo = at::empty({B, Hq, T, D}, q.options());
-    ko = at::empty({B, H, T, D}, q.options());
+    qo = fresh({B, Hq, T, D}, q, q.scalar_type());
+    ko = fresh({B, H, T, D}, q, q.scalar_type());
     if (!qo.has_storage() || !ko.has_storage())
         Py_RETURN_NONE;
     void *qp = qo.mutable_data_ptr(), *kp = ko.mutable_data_ptr();
@@ -215,8 +224,7 @@ PyObject *decode(PyObject *, PyObject *const *args, Py_ssize_t nargs)
     PyObject *w = key ? PyDict_GetItem(args[13], key) : nullptr; // borrowed
     Py_XDECREF(key);
     const at::Tensor *ws = w ? plain(w) : nullptr;
-    const int64_t need = adkv_decode_step_workspace_bytes((int)B, (int)Hq, (int)H, (int)T, (int)D, (int)n_ckpt, (int)interval);
-    if (!ws || ws->scalar_type() != at::kByte || ws->numel() < need || !ws->is_contiguous() || ws->device() != q.device())
+    if (!ws || ws->scalar_type() != at::kByte || !ws->is_contiguous() || ws->device() != q.device())
         Py_RETURN_NONE;
     at::Tensor out, weights, m, scratch = *ws; // held: another thread may replace the dictionary's entry
     int rc;
@@ -226,8 +234,8 @@ PyObject *decode(PyObject *, PyObject *const *args, Py_ssize_t nargs)
             Py_RETURN_NONE;
     }
     const int64_t pitch = adkv_row_pitch((int)n);
-    out = at::empty({B, Hq, D}, q.options());
-    weights = at::empty({B, Hq, pitch}, q.options().dtype(at::kHalf));
+    out = fresh({B, Hq, D}, q, q.scalar_type());
+    weights = fresh({B, Hq, pitch}, q, at::kHalf);
     if (!out.has_storage() || !weights.has_storage())
         Py_RETURN_NONE;
     void *op = out.mutable_data_ptr(), *wp = weights.mutable_data_ptr(), *kcp = kc->mutable_data_ptr(), *vcp = vc->mutable_data_ptr(),
@@ -240,6 +248,8 @@ PyObject *decode(PyObject *, PyObject *const *args, Py_ssize_t nargs)
                           (q.scalar_type() == at::kBFloat16 ? ADKV_DT_BF16 : ADKV_DT_F16) | ADKV_MASK_DT(std::max(mask_type, ADKV_DT_F32)),
                           ck[0], ck[1], (int)n_ckpt, (int)interval, work, scratch.numel(), stream);
     Py_END_ALLOW_THREADS
+    if (rc == ADKV_E_WORKSPACE) // too small: said before anything is launched, and the Python function gets a larger one
+        Py_RETURN_NONE;
     const int64_t sizes[3] = {B, Hq, n}, strides[3] = {Hq * pitch, pitch, 1};
     weights.unsafeGetTensorImpl()->set_sizes_and_strides(at::IntArrayRef(sizes), at::IntArrayRef(strides));
     return rc ? PyLong_FromLong(rc) : pair(std::move(out), std::move(weights));
@@ -326,12 +336,11 @@ PyObject *quant_f32(PyObject *, PyObject *const *args, Py_ssize_t nargs)
         Py_RETURN_NONE;
     at::Tensor out, state, seq[2];
     int rc;
-    const auto f32 = x->options().dtype(at::kFloat);
-    out = at::empty({B, T, C}, x->options());
-    state = at::empty({2, B, C}, f32);
+    out = fresh({B, T, C}, *x, x->scalar_type());
+    state = fresh({2, B, C}, *x, at::kFloat);
     if (args[6] == Py_True)
         for (at::Tensor &t : seq)
-            t = at::empty({B, T, C}, f32);
+            t = fresh({B, T, C}, *x, at::kFloat);
     if (!out.has_storage() || !state.has_storage())
         Py_RETURN_NONE;
     void *op = out.mutable_data_ptr(), *zp = state.mutable_data_ptr(), *sc = (float *)zp + B * C;
