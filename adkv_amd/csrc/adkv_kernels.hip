@@ -2991,6 +2991,13 @@ static int step_lone_threads(long units, int D, int GQ, int longest)
     return per_cu <= 8 ? 512 : per_cu <= 12 ? 768 : 1024;
 }
 
+// Whether the values of such a step have waves beside the keys' (step_beside_lone_kernel): as long as both kinds together are
+// two waves per SIMD, whose registers hold most of a segment's values.  us per step, step_lone_kernel / this, sequences x KV heads x
+// tokens: one query head, 1 x 32 x 2000 14.8 / 12.8, x 4096 16.0 / 14.3; two, 2 x 8 x 3000 16.1 / 13.3; four, 1 x 8 x 603 15.5 / 12.6,
+// 1 x 8 x 4000 16.2 / 13.2, 1 x 8 x 16000 18.1 / 15.6, 4 x 8 x 1000 16.2 / 13.1, 1 x 2 x 30000 18.6 / 15.8; eight, 1 x 8 x 4000
+// 17.5 / 14.2, 2 x 8 x 3000 18.1 / 14.9; 2-bit, four, 1 x 8 x 4000 15.0 / 12.3; 256 channels, 1 x 8 x 2000 14.4 / 12.2, 2 x 8 x 4000 15.7 / 14.1.
+static bool step_beside(long units, int D) { return D != 512 && units * (D / 64) <= 4L * cus(); }
+
 template <int D, int BITS, int GQ, typename... Args>
 static int launch_step_lone(int blk, long units, hipStream_t st, Args... args)
 {
@@ -2998,7 +3005,9 @@ static int launch_step_lone(int blk, long units, hipStream_t st, Args... args)
     const dim3 grid((unsigned)((units + per_block - 1) / per_block));
 #define ADKV_STEP(BLK) hipLaunchKernelGGL((step_lone_kernel<D, BITS, GQ, BLK>), grid, dim3(BLK), 0, st, args...)
     if constexpr (D != 512) {
-        if (blk == 256)
+        if (blk == 256 && step_beside(units, D))
+            hipLaunchKernelGGL((step_beside_lone_kernel<D, BITS, GQ>), grid, dim3(512), 0, st, args...);
+        else if (blk == 256)
             ADKV_STEP(256);
         if constexpr (GQ != 8) {
             if (blk == 768)
@@ -3584,7 +3593,7 @@ const char *adkv_decode_step_kernel_name(int B, int Hq, int H, int T, int D, int
         segment_step_plan(seg, cpl, B, Hq, H, T, D, bits, ck, ck, n_ckpt_cap, ckpt_interval);
         switch (step_lone_threads(padded_units<64>(B * H, seg.nseg), D, Hq / H, longest_segment(seg, T))) {
         case 0: return "step_segments_kernel";
-        case 256: return "step_lone_kernel, 4-wave workgroups";
+        case 256: return "step_lone_kernel, 4-wave workgroups"; // of keys; values may have theirs beside them
         case 512: return "step_lone_kernel, 8-wave workgroups";
         case 768: return "step_lone_kernel, 12-wave workgroups";
         default: return "step_lone_kernel, 16-wave workgroups";

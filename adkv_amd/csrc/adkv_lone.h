@@ -446,13 +446,13 @@ __device__ __forceinline__ void lone_values_end(const LoneLoads<D, BITS> &s, Lon
 
 // The same for GQ query heads: the values of four tokens of a lane's channel are a column for the matrix cores as
 // they are, the weights of the query heads the rows (see ov_gqa_segment); element i of acc[n] is head 4n + i.
-// w: a row of LONE_SEG weights per head.
+// w: a row of LONE_SEG weights per head, from the first of the n units on.
 template <int GQ, int D, int BITS>
-__device__ __forceinline__ void lone_values_grouped(const uint2 *lut, uint32_t lane_copy, LoneLoads<D, BITS> &s, Lone &st, const h1 *w, int lane,
-                                                    f4v *acc)
+__device__ __forceinline__ void lone_values_grouped(const uint2 *lut, uint32_t lane_copy, LoneLoads<D, BITS> &s, Lone &st, int n_units, const h1 *w,
+                                                    int lane, f4v *acc)
 {
     constexpr int NB = (GQ + 3) / 4;
-    if (s.nfull <= 0)
+    if (n_units <= 0)
         return;
     const uint4 *w4[NB];
     uint2 e[2][4];
@@ -464,7 +464,7 @@ __device__ __forceinline__ void lone_values_grouped(const uint2 *lut, uint32_t l
         wv[0][n] = w4[n][0];
     }
     wait_lgkm();
-    rotate_over<LONE_PF>(s.nfull * s.UPS, [&](int sg, auto ic) __attribute__((always_inline)) {
+    rotate_over<LONE_PF>(n_units, [&](int sg, auto ic) __attribute__((always_inline)) {
         constexpr int i = decltype(ic)::value, half = i & 1;
         lone_lookup<BITS>(e[half ^ 1], lut, s.buf, (i + 1) % LONE_PF, lane_copy); // stale past the end: looked up, never used
 #pragma unroll
@@ -482,6 +482,26 @@ __device__ __forceinline__ void lone_values_grouped(const uint2 *lut, uint32_t l
         }
         __builtin_amdgcn_sched_barrier(0);
     });
+}
+
+// What lone_values_ahead has left, by the weights of GQ query heads (see lone_weigh).
+template <int GQ, int UNITS>
+__device__ __forceinline__ void lone_weigh_grouped(const uint32_t *x, int done, const h1 *w, int lane, f4v *acc)
+{
+#pragma unroll
+    for (int n = 0; n < (GQ + 3) / 4; n++) {
+        const uint4 *w4 = reinterpret_cast<const uint4 *>(w + min(4 * n + (lane & 3), GQ - 1) * LONE_SEG);
+#pragma unroll
+        for (int g = 0; g < UNITS; g += LONE_PF)
+            if (g < done) {
+#pragma unroll
+                for (int u = g; u < g + LONE_PF; u++) {
+                    const uint4 wv = w4[u];
+                    acc[n] = __builtin_amdgcn_mfma_f32_4x4x4f16(as_h4(wv.x, wv.y), as_h4(x[4 * u], x[4 * u + 1]), acc[n], 0, 0, 0);
+                    acc[n] = __builtin_amdgcn_mfma_f32_4x4x4f16(as_h4(wv.z, wv.w), as_h4(x[4 * u + 2], x[4 * u + 3]), acc[n], 0, 0, 0);
+                }
+            }
+    }
 }
 
 template <int BLK>

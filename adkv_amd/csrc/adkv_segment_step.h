@@ -295,6 +295,48 @@ __device__ __forceinline__ void lone_weights(const float *share, int stride, h1 
         *ml = make_float4(mx, sum, rounded, 0.0f);
 }
 
+// A wave's channels of a segment's values by its weights p (a row of LONE_SEG per query head), to o.  ahead: the first `done` units
+// of the AHEAD that lone_values_ahead was to hold.
+template <int D, int BITS, int GQ, int AHEAD>
+__device__ __forceinline__ void lone_step_values(const uint2 *lut, uint32_t lane_copy, LoneLoads<D, BITS> &s, Lone &st, const uint32_t *ahead, int done,
+                                                 const h1 *p, int bx, int c, int T, int lane, const Seg &va, float *o)
+{
+    if constexpr (GQ == 1 && D != 512) {
+        // measured, adding on the vector pipe / on the matrix cores: 4 x 8 x 8190 of 256 channels 30.4 / 31.3, 8 x 32 x 2000
+        // 28.0 / 29.2, 4 x 32 x 2000 19.6 / 19.3; 8 x 8 x 2000 of 512 30.5 / 28.9
+        float acc = 0.0f;
+        if constexpr (AHEAD > 0)
+            lone_weigh<AHEAD>(ahead, done, p, acc);
+        lone_values(lut, lane_copy, s, st, s.nfull * s.UPS - done, p + done * 8, acc);
+        lone_values_end(s, st, [&](int t) { return p[t]; }, bx, c, T, nullptr, va, true, acc);
+        *o = acc;
+        return;
+    }
+    constexpr int NB = (GQ + 3) / 4;
+    f4v acc[NB];
+#pragma unroll
+    for (int n = 0; n < NB; n++)
+        acc[n] = (f4v){0.0f, 0.0f, 0.0f, 0.0f};
+    if constexpr (AHEAD > 0)
+        lone_weigh_grouped<GQ, AHEAD>(ahead, done, p, lane, acc);
+    lone_values_grouped<GQ>(lut, lane_copy, s, st, s.nfull * s.UPS - done, p + done * 8, lane, acc);
+    if (s.last) {
+        auto token = [&](int t, float v) __attribute__((always_inline)) {
+#pragma unroll
+            for (int g = 0; g < GQ; g++)
+                acc[g >> 2][g & 3] = __builtin_fmaf((float)p[g * LONE_SEG + t], v, acc[g >> 2][g & 3]);
+        };
+#pragma unroll
+        for (int t = 0; t < s.TPW - 1; t++)
+            if (t < s.ntail)
+                token(s.TPW * s.nfull + t, (float)lone_token(st, s.code(t)));
+        token(T - s.t0, (float)lone_append(s, st, bx, c, T, nullptr, va, true));
+    }
+#pragma unroll
+    for (int g = 0; g < GQ; g++)
+        o[g * D] = acc[g >> 2][g & 3];
+}
+
 // The same launch with one channel per lane, a KV head over D / 64 waves (adkv_lone.h): segments of at most 256 tokens.
 // With few waves per SIMD a step takes as long as one wave's instructions per token, and a lane with four or eight
 // channels has two and four times as many of them; the waves of a head meet once, behind the keys, where each has left
@@ -368,37 +410,96 @@ __global__ __launch_bounds__(BLK) void step_lone_kernel(
         return;
 
     Lone st = s.state();
-    float *o = partial + (seg * rows + row0) * D + c;
-    if constexpr (GQ == 1 && D != 512) {
-        // measured, adding on the vector pipe / on the matrix cores: 4 x 8 x 8190 of 256 channels 30.4 / 31.3, 8 x 32 x 2000
-        // 28.0 / 29.2, 4 x 32 x 2000 19.6 / 19.3; 8 x 8 x 2000 of 512 30.5 / 28.9
-        float acc = 0.0f;
-        lone_values(lut, lane_copy, s, st, s.nfull * s.UPS, p, acc);
-        lone_values_end(s, st, [&](int t) { return p[t]; }, bx, c, T, nullptr, va, true, acc);
-        *o = acc;
-        return;
+    lone_step_values<D, BITS, GQ, 0>(lut, lane_copy, s, st, nullptr, 0, p, bx, c, T, lane, va, partial + (seg * rows + row0) * D + c);
+}
+
+// The same for launches that leave SIMDs empty (at most four waves per CU): the values have waves of their own, which hold a
+// segment's in their registers (see small_step_kernel) while the keys' waves, the older ones, are at work, and
+// multiply them by the weights when those are there.  A workgroup is four waves of keys and four of values.  (Registers for all
+// of a segment, 32 units, keep the softmax waiting for the last of them: 1 to 2 % slower than 24.)
+template <int D, int BITS, int GQ>
+__global__ __launch_bounds__(512) void step_beside_lone_kernel(
+    const h1 *q, uint4 *k_cache, const h1 *k_new, uint4 *v_cache, const h1 *v_new, Mask mk, h1 *logits, float *__restrict__ partial,
+    float4 *__restrict__ ml, FtParams kp, FtParams vp, int BH, int H, int T, int n_super_cap, float scaling, Seg ka, Seg va)
+{
+    constexpr int WAVES = 4, HW = D / 64, UNITS = WAVES / HW, AHEAD = 24;
+    static_assert(WAVES % HW == 0, "whole heads");
+    constexpr int ROWS = GQ == 1 ? WAVES : UNITS * GQ; // of weights: a copy per values' wave, or those that a unit's waves write together
+    __shared__ uint4 smem[(LUT_WORDS64 * 8 + WAVES * (LONE_TILE + GQ * LONE_SEG * 4) + ROWS * LONE_SEG * 2) / 16];
+    static_assert(LONE_SEG * 2 % 16 == 0, "vectors");
+    ka.groups = va.groups = 0; // only even plans come here
+    uint2 *lut = reinterpret_cast<uint2 *>(smem);
+    char *lds = reinterpret_cast<char *>(smem) + LUT_WORDS64 * 8;
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    const bool values = wave >= WAVES;
+    const int w = values ? wave - WAVES : wave, u = w / HW, part = w % HW, c = part * 64 + lane;
+    const uint32_t lane_copy = table_lane_offset<BITS>(lane);
+    int seg, wis;
+    interleave_segment((int)blockIdx.x * UNITS + u, ka.nseg, seg, wis);
+    const bool active = wis < BH;
+    const int bx = min(wis, BH - 1), h = bx % H;
+    float *shares = reinterpret_cast<float *>(lds + WAVES * LONE_TILE) + u * HW * GQ * LONE_SEG;
+    h1 *rows_of_weights = reinterpret_cast<h1 *>(lds + WAVES * (LONE_TILE + GQ * LONE_SEG * 4));
+    LoneLoads<D, BITS> s;
+    s.start(values ? v_cache : k_cache, values ? vp : kp, values ? v_new : k_new, h, bx, c, seg, T, n_super_cap, values ? va : ka);
+    if constexpr (BITS == 4)
+        lone_fill<512>(lut, threadIdx.x);
+    else
+        lone_fill2<512>(lut, threadIdx.x);
+    __syncthreads();
+
+    const int t0 = s.t0, ntok = s.t1 - s.t0 + (s.last ? 1 : 0); // the appended token is the last segment's
+    const long row0 = (long)bx * GQ, rows = (long)BH * GQ;
+    auto weigh = [&](int g, h1 *p, bool writes) __attribute__((always_inline)) {
+        lone_weights<HW>(shares + g * LONE_SEG, GQ * LONE_SEG, logits + (row0 + g) * ka.row_pitch + t0,
+                         mk.of<true>((unsigned)row0 + g, T + 1, t0), ntok, scaling, p, ml + (row0 + g) * ka.nseg + seg, lane, writes);
+    };
+    // several query heads: a unit's waves, of both kinds, share them out
+    auto weigh_mine = [&]() __attribute__((always_inline)) {
+#pragma unroll
+        for (int i = 0; i < (GQ + 2 * HW - 1) / (2 * HW); i++) {
+            const int g = i * 2 * HW + (values ? HW : 0) + part;
+            if (active && g < GQ)
+                weigh(g, rows_of_weights + (u * GQ + g) * LONE_SEG, true);
+        }
+    };
+    Lone st = s.state();
+    if (values) {
+        uint32_t ahead[AHEAD * 4];
+        const int done = active ? lone_values_ahead<AHEAD>(lut, lane_copy, s, st, s.nfull * s.UPS, ahead) : 0;
+        __syncthreads();
+        const h1 *p;
+        if constexpr (GQ == 1) { // every wave by itself, no wave waits for another
+            h1 *mine = rows_of_weights + w * LONE_SEG;
+            if (active)
+                weigh(0, mine, false);
+            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront"); // the wave's own weights, read by its other lanes
+            p = mine;
+        } else {
+            weigh_mine();
+            __syncthreads();
+            p = rows_of_weights + u * GQ * LONE_SEG;
+        }
+        if (active)
+            lone_step_values<D, BITS, GQ, AHEAD>(lut, lane_copy, s, st, ahead, done, p, bx, c, T, lane, va, partial + (seg * rows + row0) * D + c);
+    } else {
+        if (active) {
+            LoneScores<true, GQ, D, BITS> scores(lds + w * LONE_TILE, lane, q + (size_t)bx * GQ * D + part * 64);
+            float *mine = shares + part * GQ * LONE_SEG;
+            scores.ready(ka.act_bf16);
+            scores.run(lut, lane_copy, st, s, s.nfull * s.UPS, mine);
+            if (s.last)
+                scores.finish(s, st, bx, c, T, nullptr, ka, true, mine + s.nfull * s.TPW);
+        }
+        __syncthreads();
+        if constexpr (GQ == 1) {
+            if (active && part == 0)
+                weigh(0, reinterpret_cast<h1 *>(lds + w * LONE_TILE), true);
+        } else {
+            weigh_mine();
+            __syncthreads();
+        }
     }
-    constexpr int NB = (GQ + 3) / 4;
-    f4v acc[NB];
-#pragma unroll
-    for (int n = 0; n < NB; n++)
-        acc[n] = (f4v){0.0f, 0.0f, 0.0f, 0.0f};
-    lone_values_grouped<GQ>(lut, lane_copy, s, st, p, lane, acc);
-    if (s.last) {
-        auto token = [&](int t, float v) __attribute__((always_inline)) {
-#pragma unroll
-            for (int g = 0; g < GQ; g++)
-                acc[g >> 2][g & 3] = __builtin_fmaf((float)p[g * LONE_SEG + t], v, acc[g >> 2][g & 3]);
-        };
-#pragma unroll
-        for (int t = 0; t < s.TPW - 1; t++)
-            if (t < s.ntail)
-                token(s.TPW * s.nfull + t, (float)lone_token(st, s.code(t)));
-        token(T - t0, (float)lone_append(s, st, bx, c, T, nullptr, va, true));
-    }
-#pragma unroll
-    for (int g = 0; g < GQ; g++)
-        o[g * D] = acc[g >> 2][g & 3];
 }
 
 // The segments of a row put together, by waves of two kinds: VECS x 512 of its weights each, or a share of its

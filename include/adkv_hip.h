@@ -61,7 +61,8 @@ void adkv_set_mha_kernel(int use_matrix_cores);
  * per lane) and step_combine_kernel (steps of short segments, see adkv_decode_step); 3 if forward_qk, the softmax and
  * forward_ov are launched one after the other, also for sizes that the call refuses.
  * adkv_decode_step_kernel_name: the first kernel of a call in one or two launches, a static string for benchmark records
- * and tests; NULL for the others (adkv_decode_kernel_name and adkv_decode_ov_kernel_name have theirs). */
+ * and tests; NULL for the others (adkv_decode_kernel_name and adkv_decode_ov_kernel_name have theirs).  A step_lone_kernel's
+ * waves are those that take a segment's keys: with few of them its values have as many of their own beside them. */
 void adkv_set_fused_step(int mode);
 int adkv_decode_step_is_fused(int B, int Hq, int H, int T, int D, int bits, int n_ckpt_cap,
                               int ckpt_interval, int masked);
