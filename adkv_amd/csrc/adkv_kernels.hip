@@ -2955,7 +2955,7 @@ static int launch_step_grouped(int GQ, long waves, hipStream_t st, Args... args)
     }
 }
 
-// Whether step_lone_kernel takes a step of the two launches, and with which workgroups: a wave's 64 channels bring
+// Whether a step of the two launches is of one channel per lane, and how many waves of keys a workgroup has: a wave's 64 channels bring
 // twice the waves of two channels per lane and four or eight times those of wide heads, and pay as long as a CU holds
 // them at once: 16 waves, and 12 / 8 with four / eight query heads, whose logits take more of the LDS; with one or two
 // query heads of 128 channels, whose other form has its waves' LDS reads covered by then, 12.  us per step on the
@@ -2991,24 +2991,27 @@ static int step_lone_threads(long units, int D, int GQ, int longest)
     return per_cu <= 8 ? 512 : per_cu <= 12 ? 768 : 1024;
 }
 
-// Whether the values of such a step have waves beside the keys' (step_beside_lone_kernel): as long as both kinds together are
-// two waves per SIMD, whose registers hold most of a segment's values.  us per step, step_lone_kernel / this, sequences x KV heads x
-// tokens: one query head, 1 x 32 x 2000 14.8 / 12.8, x 4096 16.0 / 14.3; two, 2 x 8 x 3000 16.1 / 13.3; four, 1 x 8 x 603 15.5 / 12.6,
-// 1 x 8 x 4000 16.2 / 13.2, 1 x 8 x 16000 18.1 / 15.6, 4 x 8 x 1000 16.2 / 13.1, 1 x 2 x 30000 18.6 / 15.8; eight, 1 x 8 x 4000
-// 17.5 / 14.2, 2 x 8 x 3000 18.1 / 14.9; 2-bit, four, 1 x 8 x 4000 15.0 / 12.3; 256 channels, 1 x 8 x 2000 14.4 / 12.2, 2 x 8 x 4000 15.7 / 14.1.
-static bool step_beside(long units, int D) { return D != 512 && units * (D / 64) <= 4L * cus(); }
-
+// Up to eight waves per CU the values of such a step have waves beside the keys' (step_beside_lone_kernel): as many again, up to two
+// per SIMD with registers for 24 units of a segment's values, up to four with registers for 16.  With more both kinds together are
+// more than a CU holds.  us per step, one behind the other (step_lone_kernel) / beside, sequences x KV heads x tokens (waves of keys
+// per CU): one query head, 1 x 32 x 2000 (2) 14.8 / 12.8, 2 x 32 x 2048 (4) 15.9 / 14.1, 4 x 32 x 2048 (8) 19.3 / 18.4; two, 2 x 8 x 3000 16.1 /
+// 13.3, 8 x 16 x 2048 (8) 20.6 / 18.7; four, 1 x 8 x 603 15.5 / 12.6, 1 x 8 x 4000 16.2 / 13.2, 1 x 8 x 16000 (4) 18.1 / 15.6, 1 x 2 x 30000 18.6 /
+// 15.8, 3 x 8 x 6000 (5) 20.7 / 18.4, 8 x 8 x 4096 (8) 22.7 / 20.5; eight, 1 x 8 x 4000 17.5 / 14.2, 5 x 8 x 5632 (8) 26.4 / 24.1; 2-bit,
+// four, 1 x 8 x 4000 15.0 / 12.3, 6 x 8 x 4096 (6) 20.3 / 18.2, one, 4 x 32 x 2048 (8) 18.4 / 17.8; 256 channels, 1 x 8 x 2000 14.4 / 12.2, 4 x 8 x
+// 4000 (8) 18.8 / 18.2; 512, 1 x 8 x 1000 18.4 / 16.6, 2 x 8 x 2000 (4) 18.5 / 17.0.
 template <int D, int BITS, int GQ, typename... Args>
 static int launch_step_lone(int blk, long units, hipStream_t st, Args... args)
 {
     const int per_block = blk / D; // units: a wave per 64 channels
     const dim3 grid((unsigned)((units + per_block - 1) / per_block));
 #define ADKV_STEP(BLK) hipLaunchKernelGGL((step_lone_kernel<D, BITS, GQ, BLK>), grid, dim3(BLK), 0, st, args...)
+#define ADKV_BESIDE(BLK, AHEAD) hipLaunchKernelGGL((step_beside_lone_kernel<D, BITS, GQ, (BLK) / 64, AHEAD>), grid, dim3(2 * (BLK)), 0, st, args...)
     if constexpr (D != 512) {
-        if (blk == 256 && step_beside(units, D))
-            hipLaunchKernelGGL((step_beside_lone_kernel<D, BITS, GQ>), grid, dim3(512), 0, st, args...);
-        else if (blk == 256)
-            ADKV_STEP(256);
+        if (blk == 256 && units * (D / 64) <= 4L * cus())
+            ADKV_BESIDE(256, 24);
+        else if constexpr (GQ == 1)
+            if (blk == 256)
+                ADKV_BESIDE(256, 16);
         if constexpr (GQ != 8) {
             if (blk == 768)
                 ADKV_STEP(768);
@@ -3016,12 +3019,13 @@ static int launch_step_lone(int blk, long units, hipStream_t st, Args... args)
     }
     if constexpr (D == 512 || GQ > 1) {
         if (blk == 512)
-            ADKV_STEP(512);
+            ADKV_BESIDE(512, 16);
     }
     if constexpr (D != 128) {
         if (blk == 1024)
             ADKV_STEP(1024);
     }
+#undef ADKV_BESIDE
 #undef ADKV_STEP
     return check_launch();
 }
@@ -3593,7 +3597,7 @@ const char *adkv_decode_step_kernel_name(int B, int Hq, int H, int T, int D, int
         segment_step_plan(seg, cpl, B, Hq, H, T, D, bits, ck, ck, n_ckpt_cap, ckpt_interval);
         switch (step_lone_threads(padded_units<64>(B * H, seg.nseg), D, Hq / H, longest_segment(seg, T))) {
         case 0: return "step_segments_kernel";
-        case 256: return "step_lone_kernel, 4-wave workgroups"; // of keys; values may have theirs beside them
+        case 256: return "step_lone_kernel, 4-wave workgroups"; // of keys, the values have theirs beside them
         case 512: return "step_lone_kernel, 8-wave workgroups";
         case 768: return "step_lone_kernel, 12-wave workgroups";
         default: return "step_lone_kernel, 16-wave workgroups";

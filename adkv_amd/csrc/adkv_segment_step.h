@@ -367,7 +367,7 @@ __global__ __launch_bounds__(BLK) void step_lone_kernel(
     const bool active = wis < BH;
     const int bx = min(wis, BH - 1), h = bx % H;
     float *shares = reinterpret_cast<float *>(lds + WAVES * SLOT) + u * HW * GQ * LONE_SEG;
-    LoneScores<BLK <= 512, GQ, D, BITS> scores(lds + wave * SLOT, lane, q + (size_t)bx * GQ * D + part * 64);
+    LoneScores<false, GQ, D, BITS> scores(lds + wave * SLOT, lane, q + (size_t)bx * GQ * D + part * 64);
     LoneLoads<D, BITS> s;
     s.start(k_cache, kp, k_new, h, bx, c, seg, T, n_super_cap, ka);
     if constexpr (BITS == 4)
@@ -413,19 +413,22 @@ __global__ __launch_bounds__(BLK) void step_lone_kernel(
     lone_step_values<D, BITS, GQ, 0>(lut, lane_copy, s, st, nullptr, 0, p, bx, c, T, lane, va, partial + (seg * rows + row0) * D + c);
 }
 
-// The same for launches that leave SIMDs empty (at most four waves per CU): the values have waves of their own, which hold a
+// The same for launches of at most eight waves per CU: the values have waves of their own, which hold the first AHEAD units of a
 // segment's in their registers (see small_step_kernel) while the keys' waves, the older ones, are at work, and
-// multiply them by the weights when those are there.  A workgroup is four waves of keys and four of values.  (Registers for all
-// of a segment, 32 units, keep the softmax waiting for the last of them: 1 to 2 % slower than 24.)
-template <int D, int BITS, int GQ>
-__global__ __launch_bounds__(512) void step_beside_lone_kernel(
+// multiply them by the weights when those are there.  A workgroup is WAVES waves of keys and as many of values; the SIMD has two of
+// them with AHEAD = 24 and four with 16.  (Registers for all of a segment, 32 units, keep the softmax waiting for the last of
+// them: 1 to 2 % slower than 24.)
+template <int D, int BITS, int GQ, int WAVES, int AHEAD>
+__global__ __launch_bounds__(WAVES * 128, AHEAD > 16 ? 2 : 4) void step_beside_lone_kernel(
     const h1 *q, uint4 *k_cache, const h1 *k_new, uint4 *v_cache, const h1 *v_new, Mask mk, h1 *logits, float *__restrict__ partial,
     float4 *__restrict__ ml, FtParams kp, FtParams vp, int BH, int H, int T, int n_super_cap, float scaling, Seg ka, Seg va)
 {
-    constexpr int WAVES = 4, HW = D / 64, UNITS = WAVES / HW, AHEAD = 24;
+    constexpr int HW = D / 64, UNITS = WAVES / HW;
     static_assert(WAVES % HW == 0, "whole heads");
-    constexpr int ROWS = GQ == 1 ? WAVES : UNITS * GQ; // of weights: a copy per values' wave, or those that a unit's waves write together
-    __shared__ uint4 smem[(LUT_WORDS64 * 8 + WAVES * (LONE_TILE + GQ * LONE_SEG * 4) + ROWS * LONE_SEG * 2) / 16];
+    // key tiles, the weights, the shares.  Weights: a copy per values' wave, or, where the tiles were, those that a unit's waves write together
+    constexpr int TILES = WAVES * LONE_TILE, WEIGHTS = (GQ == 1 ? WAVES : UNITS * GQ) * LONE_SEG * 2, AT = GQ == 1 ? TILES : 0;
+    constexpr int SHARES = AT + WEIGHTS > TILES ? AT + WEIGHTS : TILES;
+    __shared__ uint4 smem[(LUT_WORDS64 * 8 + SHARES + WAVES * GQ * LONE_SEG * 4) / 16];
     static_assert(LONE_SEG * 2 % 16 == 0, "vectors");
     ka.groups = va.groups = 0; // only even plans come here
     uint2 *lut = reinterpret_cast<uint2 *>(smem);
@@ -438,14 +441,14 @@ __global__ __launch_bounds__(512) void step_beside_lone_kernel(
     interleave_segment((int)blockIdx.x * UNITS + u, ka.nseg, seg, wis);
     const bool active = wis < BH;
     const int bx = min(wis, BH - 1), h = bx % H;
-    float *shares = reinterpret_cast<float *>(lds + WAVES * LONE_TILE) + u * HW * GQ * LONE_SEG;
-    h1 *rows_of_weights = reinterpret_cast<h1 *>(lds + WAVES * (LONE_TILE + GQ * LONE_SEG * 4));
+    float *shares = reinterpret_cast<float *>(lds + SHARES) + u * HW * GQ * LONE_SEG;
+    h1 *rows_of_weights = reinterpret_cast<h1 *>(lds + AT);
     LoneLoads<D, BITS> s;
     s.start(values ? v_cache : k_cache, values ? vp : kp, values ? v_new : k_new, h, bx, c, seg, T, n_super_cap, values ? va : ka);
     if constexpr (BITS == 4)
-        lone_fill<512>(lut, threadIdx.x);
+        lone_fill<WAVES * 128>(lut, threadIdx.x);
     else
-        lone_fill2<512>(lut, threadIdx.x);
+        lone_fill2<WAVES * 128>(lut, threadIdx.x);
     __syncthreads();
 
     const int t0 = s.t0, ntok = s.t1 - s.t0 + (s.last ? 1 : 0); // the appended token is the last segment's
@@ -484,7 +487,7 @@ __global__ __launch_bounds__(512) void step_beside_lone_kernel(
             lone_step_values<D, BITS, GQ, AHEAD>(lut, lane_copy, s, st, ahead, done, p, bx, c, T, lane, va, partial + (seg * rows + row0) * D + c);
     } else {
         if (active) {
-            LoneScores<true, GQ, D, BITS> scores(lds + w * LONE_TILE, lane, q + (size_t)bx * GQ * D + part * 64);
+            LoneScores<(AHEAD > 16), GQ, D, BITS> scores(lds + w * LONE_TILE, lane, q + (size_t)bx * GQ * D + part * 64);
             float *mine = shares + part * GQ * LONE_SEG;
             scores.ready(ka.act_bf16);
             scores.run(lut, lane_copy, st, s, s.nfull * s.UPS, mine);
