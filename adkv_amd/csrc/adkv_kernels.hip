@@ -92,8 +92,9 @@ struct Seg {
     long row_pitch;     // elements between rows of the logits / attention-weight matrix (>= T + 1)
     int act_bf16;       // q, the new token and the output are bfloat16 (see load_act2 / store_act2)
     int combine;        // ov_ft_kernel: the segments' partial outputs are added inside the workgroup
-    // Per-head-table kernels only.  groups > 0: the context's `intervals` checkpoint intervals are
-    // cut into `groups` groups of four segments of unequal length (uneven_cut).  phys_per_head:
+    // Per-head-table and matrix-core kernels only.  groups > 0: the context's `intervals` checkpoint intervals are
+    // cut into `groups` groups of four segments of unequal length (uneven_cut).  groups < 0: into nseg segments that
+    // differ by one interval at most.  phys_per_head (per-head table):
     // workgroups launched per KV head; each walks through the head's virtual workgroups pw,
     // pw + phys_per_head, ... one after the other (same table, no barrier between them).
     int groups;
@@ -151,23 +152,27 @@ __host__ __device__ inline int uneven_cut(int seg, int groups, int intervals, un
 // the work after the loop is (ragged tail, appended token, published state: a chain of dependent
 // memory operations), and the oldest slot's waves are the first to finish their loop, so that
 // work runs while the other slots are still in theirs instead of at the very end of the launch.
-__host__ __device__ inline int segment_of_slot(const Seg &sa, int seg) { return sa.groups ? seg ^ 3 : seg; }
+__host__ __device__ inline int segment_of_slot(const Seg &sa, int seg) { return sa.groups > 0 ? seg ^ 3 : seg; }
 
-// first token of the segment of slot index `seg` / of the one after it in time; whether it is the
-// last of the context
-__host__ __device__ inline int seg_begin(const Seg &sa, int seg)
-{
-    return sa.groups ? uneven_cut(seg ^ 3, sa.groups, sa.intervals, sa.skew) * sa.ckpt_interval : seg * sa.seg_tokens;
-}
-// the same in checkpoint intervals (0 when there is one segment)
+// first interval of the seg-th of nseg segments as equal as they can be
+__host__ __device__ inline int balanced_cut(const Seg &sa, int seg) { return (int)((long)sa.intervals * seg / sa.nseg); }
+// first token of the segment of slot index `seg` / of the one after it in time, in checkpoint intervals (0 when there is one segment)
 __host__ __device__ inline int seg_first_interval(const Seg &sa, int seg)
 {
-    return sa.groups ? uneven_cut(seg ^ 3, sa.groups, sa.intervals, sa.skew) : seg * sa.seg_intervals;
+    return sa.groups > 0   ? uneven_cut(seg ^ 3, sa.groups, sa.intervals, sa.skew)
+           : sa.groups < 0 ? balanced_cut(sa, seg)
+                           : seg * sa.seg_intervals;
+}
+// the same in tokens; whether it is the last of the context
+__host__ __device__ inline int seg_begin(const Seg &sa, int seg)
+{
+    return sa.groups ? seg_first_interval(sa, seg) * sa.ckpt_interval : seg * sa.seg_tokens;
 }
 __host__ __device__ inline int seg_end(const Seg &sa, int seg)
 {
-    return sa.groups ? uneven_cut((seg ^ 3) + 1, sa.groups, sa.intervals, sa.skew) * sa.ckpt_interval
-                     : (seg + 1) * sa.seg_tokens;
+    return sa.groups > 0   ? uneven_cut((seg ^ 3) + 1, sa.groups, sa.intervals, sa.skew) * sa.ckpt_interval
+           : sa.groups < 0 ? balanced_cut(sa, seg + 1) * sa.ckpt_interval
+                           : (seg + 1) * sa.seg_tokens;
 }
 __host__ __device__ inline bool seg_is_last(const Seg &sa, int seg) { return segment_of_slot(sa, seg) == sa.nseg - 1; }
 
@@ -2814,6 +2819,65 @@ static void plan_uneven(Seg &seg, int T, long threads, unsigned skew)
     seg.intervals = avail;
 }
 
+// The plan of a matrix-core launch of up to four query heads, four channels per lane (`seg` comes in as the even plan).  The even
+// plan's segments are whole multiples of an interval, all the same, and leave what they leave: 17 x 8 KV heads x 15467 tokens are 61
+// segments of one interval in 260 workgroups, two rounds for four of them, and 128 x 2 x 20219 27 segments of three in 216 of 256
+// CUs.  So the number of segments is chosen for the workgroups that it makes: as groups of four uneven ones where an interval more or
+// less is little of a group, else nearly equal ones of as many intervals as it takes.  The length of a launch is modelled as rounds of
+// workgroups x the intervals of a SIMD's three or four waves, over the part of the time that its vector pipe is busy then: 0.80
+// with three waves, 0.83 with four alike, 0.89 with four uneven ones (SQ_ACTIVE_INST_VALU).  Another plan has to be 5 % shorter.
+// us per step, the even plan (uneven where its segments are a multiple of four) / this: 17 x 8 x 15467 175 / 116, 128 x 2 x 20219 240 / 226, 69 x 2 x
+// 46577 307 / 282 (four query heads), 24 x 32 x 12000 2-bit 331 / 318, 48 x 8 x 9000 (two) 159 / 155; the others of eleven such sizes
+// keep theirs.
+static void plan_gqa(Seg &seg, int BH, int T, unsigned skew)
+{
+    plan_uneven(seg, T, padded_units<32>(BH, seg.nseg) * 32, skew);
+    const int n_cus = cus(), per_seg = pad4((BH + 1) / 2); // waves
+    if (!seg.ckpt || seg.ckpt_interval <= 0 || seg.nseg < 2 || (long)per_seg * seg.nseg <= 8L * n_cus)
+        return;
+    const int avail = (T + seg.ckpt_interval - 1) / seg.ckpt_interval;
+    auto rounds = [&](long waves, int &slots) { // of workgroups; the waves of one on a SIMD, as threads_per_workgroup has them
+        slots = (waves + n_cus - 1) / n_cus <= 12 ? 3 : 4;
+        return (double)(((waves + slots * 4 - 1) / (slots * 4) + n_cus - 1) / n_cus);
+    };
+    auto cost = [&](const Seg &s) {
+        int slots;
+        const double r = rounds((long)per_seg * s.nseg, slots);
+        if (s.groups > 0)
+            return r * ((avail + s.groups - 1) / s.groups) / 0.89;
+        const long sum = s.groups < 0 ? ((long)slots * avail + s.nseg - 1) / s.nseg : (long)slots * s.seg_intervals;
+        return r * sum / (slots == 4 ? 0.83 : 0.80);
+    };
+    double best = 0.95 * cost(seg);
+    const Seg even = seg;
+    auto consider = [&](int groups, int nseg) {
+        Seg s = even;
+        s.groups = groups;
+        s.nseg = nseg;
+        s.intervals = avail;
+        s.seg_tokens = s.ckpt_interval; // not read
+        // the last segment starts from a checkpoint
+        const int last = groups > 0 ? uneven_cut(nseg - 1, groups, avail, skew) : balanced_cut(s, nseg - 1);
+        if (last - 1 >= s.n_ckpt_cap)
+            return;
+        const double c = cost(s);
+        if (c < best) {
+            best = c;
+            seg = s;
+        }
+    };
+    for (int round = 1; round <= 2; round++)
+        for (int slots = 4; slots >= 3; slots--) {
+            const long most = (long)round * n_cus * slots * 4 / per_seg; // segments in that many rounds
+            const int groups = (int)std::min(most / 4, (long)avail / FT_MIN_GROUP);
+            if (slots == 4 && groups >= 1 && (long)per_seg * 4 * groups > 12L * n_cus)
+                consider(groups, 4 * groups);
+            const int n = (int)std::min(most, (long)avail);
+            if (n >= 2 && (long)per_seg * n > 8L * n_cus)
+                consider(-1, n);
+        }
+}
+
 // How many segments the forward_ov partial sums of a launch can have under either plan (what a
 // workspace must be sized for: the kernel family can be switched between sizing and launch).
 static int max_plan_segments(void *ckpt, int n_ckpt_cap, int ckpt_interval, int B, int H, int T, int D)
@@ -2826,6 +2890,8 @@ static int max_plan_segments(void *ckpt, int n_ckpt_cap, int ckpt_interval, int 
         plan_ft(b, B, H, T, FT_SKEW_QK, true);
         plan_ft_ov(c, B, H, T);
         n = std::max(std::max(n, a.nseg), std::max(b.nseg, c.nseg));
+        plan_gqa(seg, B * H, T, GQA_SKEW_OV);
+        n = std::max(n, seg.nseg);
     }
     return n;
 }
@@ -3456,7 +3522,10 @@ static const char *decode_kernel_name(bool ov, int B, int Hq, int H, int T, int 
     if (D == 128 && (GQ > 1 || bits != 4 || mfma_for_mha())) {
         if (ov ? ov_gqa_pair(BH, seg.nseg, GQ, true) : gqa_pair(BH, seg.nseg))
             return "gqa_kernel, two channels per lane (matrix cores)";
-        const int blk = threads_per_workgroup(padded_units<32>(BH, seg.nseg) * 32);
+        Seg s = seg;
+        if (GQ <= 4)
+            plan_gqa(s, BH, T, ov ? GQA_SKEW_OV : GQA_SKEW_QK);
+        const int blk = threads_per_workgroup(padded_units<32>(BH, s.nseg) * 32);
         if (ov && (GQ > 4 || blk == 256))
             return "gqa_kernel, 8-wave workgroups (matrix cores)";
         return blk == 1024 ? "gqa_kernel, 16-wave workgroups (matrix cores)"
@@ -3520,9 +3589,9 @@ static int forward_qk_impl(const void *q, void *k_cache, const void *k_new, void
     if (ld)
         seg.row_pitch = ld;
     if (D == 128 && (GQ > 1 || bits != 4 || mfma_for_mha())) {
-        if (GQ <= 4) // eight query heads per KV head may fall back to 8-wave workgroups
-            plan_uneven(seg, T, padded_units<32>(BH, seg.nseg) * 32, GQA_SKEW_QK);
         const bool pair = gqa_pair(BH, seg.nseg);
+        if (GQ <= 4 && !pair) // eight query heads per KV head may fall back to 8-wave workgroups
+            plan_gqa(seg, BH, T, GQA_SKEW_QK);
         ADKV_DISPATCH_GQ(qk_gqa_kernel, true, (const h1 *)q, (uint4 *)k_cache, (const h1 *)k_new,
                          (h1 *)logits, (const h1 *)zp, (const h1 *)sc, (const h1 *)alpha,
                          (const h1 *)beta, (const h1 *)tgt, BH, H, T, n_super_cap, (h1 *)state_out,
@@ -3623,8 +3692,8 @@ int adkv_decode_segments(int B, int Hq, int H, int T, int D, int bits, int n_ckp
     const bool head_table = !matrix_cores && use_head_table(B, H, GQ, bits, D, seg);
     long wgs = 0;
     int virt = 1;
-    if (matrix_cores && GQ <= 4)
-        plan_uneven(seg, T, padded_units<32>(B * H, seg.nseg) * 32, GQA_SKEW_QK);
+    if (matrix_cores && GQ <= 4 && !gqa_pair((long)B * H, seg.nseg))
+        plan_gqa(seg, B * H, T, GQA_SKEW_QK);
     if (head_table) {
         const int lanes = plan_ft(seg, B, H, T, FT_SKEW_QK, FT16_QK);
         const int W = ft_wgs_per_head(B, seg.nseg, 64 / lanes);
@@ -3633,8 +3702,9 @@ int adkv_decode_segments(int B, int Hq, int H, int T, int D, int bits, int n_ckp
     }
     if (bounds != nullptr && max_bounds > seg.nseg) {
         for (int s = 0; s < seg.nseg; s++)
-            bounds[s] = seg.groups ? uneven_cut(s, seg.groups, seg.intervals, seg.skew) * seg.ckpt_interval
-                                   : s * seg.seg_tokens; // in time order
+            bounds[s] = seg.groups > 0   ? uneven_cut(s, seg.groups, seg.intervals, seg.skew) * seg.ckpt_interval
+                        : seg.groups < 0 ? balanced_cut(seg, s) * seg.ckpt_interval
+                                         : s * seg.seg_tokens; // in time order
         bounds[seg.nseg] = T;
     }
     if (info != nullptr) {
@@ -3727,6 +3797,15 @@ static int forward_ov_impl(const void *attn, void *v_cache, const void *v_new, v
     // sequence pair sit in the same workgroup (interleave_segment) and add their partial outputs
     // there; no second launch and nothing in the workspace
     seg.combine = (head_table && ft_ov_combines(seg, B, ft_lanes)) ? 1 : 0;
+    const bool pair = matrix_cores && ov_gqa_pair(BH, seg.nseg, GQ, ((uintptr_t)attn & 15) == 0 && seg.row_pitch % 8 == 0);
+    if (matrix_cores && GQ <= 4 && !pair) {
+        Seg s = seg;
+        plan_gqa(s, BH, T, GQA_SKEW_OV);
+        if (workspace_bytes >= (int64_t)s.nseg * BH * GQ * D * 4)
+            seg = s;
+        else // a workspace for fewer segments keeps the even plan's number of them
+            plan_uneven(seg, T, padded_units<32>(BH, seg.nseg) * 32, GQA_SKEW_OV);
+    }
     if (seg.nseg > 1 && !seg.combine) {
         if (!workspace || workspace_bytes < (int64_t)seg.nseg * BH * GQ * D * 4)
             return ADKV_E_WORKSPACE;
@@ -3734,9 +3813,6 @@ static int forward_ov_impl(const void *attn, void *v_cache, const void *v_new, v
             return ADKV_E_ALIGN;
     }
     if (matrix_cores) {
-        if (GQ <= 4)
-            plan_uneven(seg, T, padded_units<32>(BH, seg.nseg) * 32, GQA_SKEW_OV);
-        const bool pair = ov_gqa_pair(BH, seg.nseg, GQ, ((uintptr_t)attn & 15) == 0 && seg.row_pitch % 8 == 0);
         ADKV_DISPATCH_GQ(ov_gqa_kernel, false, (const h1 *)attn, (uint4 *)v_cache, (const h1 *)v_new,
                          (h1 *)out, (float *)workspace, (const h1 *)zp, (const h1 *)sc,
                          (const h1 *)alpha, (const h1 *)beta, (const h1 *)tgt, BH, H, T, n_super_cap,
