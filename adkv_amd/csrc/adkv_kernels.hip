@@ -1440,7 +1440,7 @@ __global__ __launch_bounds__(BLK) void qk_kernel(
     int BH, int H, int T, int n_super_cap, h1 *__restrict__ state_out, Seg sa)
 {
     using G = Geo<D, CPL>;
-    sa.groups = 0; // only even plans come here (a fifth of the code was the other kind's cuts)
+    sa.groups = sa.groups < 0 ? -1 : 0; // no uneven plans come here (a fifth of the code was their cuts)
     constexpr bool PAIR = CPL == 2;
     // the only LDS object: the table sits at LDS offset 0 (its byte address is used as is)
     __shared__ uint2 smem[LUT_WORDS64 + (PAIR ? (BLK / 64) * PAIR_TILE / 8 : 0)];
@@ -1628,7 +1628,7 @@ __global__ __launch_bounds__(BLK) void ov_kernel(
 {
     using G = Geo<D, CPL>;
     static_assert(CPL >= 4, "fewer channels per lane: ov_lone_kernel");
-    sa.groups = 0; // only even plans come here
+    sa.groups = sa.groups < 0 ? -1 : 0; // no uneven plans come here
     __shared__ uint2 lut[LUT_WORDS64];
     lut_fill<BLK>(lut, threadIdx.x);
     __syncthreads();
@@ -2819,7 +2819,7 @@ static void plan_uneven(Seg &seg, int T, long threads, unsigned skew)
     seg.intervals = avail;
 }
 
-// The plan of a matrix-core launch of up to four query heads, four channels per lane (`seg` comes in as the even plan).  The even
+// The plan of a launch of four channels per lane, of matrix-core ones up to four query heads (`seg` comes in as the even plan).  The even
 // plan's segments are whole multiples of an interval, all the same, and leave what they leave: 17 x 8 KV heads x 15467 tokens are 61
 // segments of one interval in 260 workgroups, two rounds for four of them, and 128 x 2 x 20219 27 segments of three in 216 of 256
 // CUs.  So the number of segments is chosen for the workgroups that it makes: as groups of four uneven ones where an interval more or
@@ -2829,10 +2829,9 @@ static void plan_uneven(Seg &seg, int T, long threads, unsigned skew)
 // us per step, the even plan (uneven where its segments are a multiple of four) / this: 17 x 8 x 15467 175 / 116, 128 x 2 x 20219 240 / 226, 69 x 2 x
 // 46577 307 / 282 (four query heads), 24 x 32 x 12000 2-bit 331 / 318, 48 x 8 x 9000 (two) 159 / 155; the others of eleven such sizes
 // keep theirs.
-static void plan_gqa(Seg &seg, int BH, int T, unsigned skew)
+static void plan_rounds(Seg &seg, int per_seg, int T, unsigned skew) // per_seg: waves per segment; skew: 0, no uneven groups
 {
-    plan_uneven(seg, T, padded_units<32>(BH, seg.nseg) * 32, skew);
-    const int n_cus = cus(), per_seg = pad4((BH + 1) / 2); // waves
+    const int n_cus = cus();
     if (!seg.ckpt || seg.ckpt_interval <= 0 || seg.nseg < 2 || (long)per_seg * seg.nseg <= 8L * n_cus)
         return;
     const int avail = (T + seg.ckpt_interval - 1) / seg.ckpt_interval;
@@ -2870,12 +2869,24 @@ static void plan_gqa(Seg &seg, int BH, int T, unsigned skew)
         for (int slots = 4; slots >= 3; slots--) {
             const long most = (long)round * n_cus * slots * 4 / per_seg; // segments in that many rounds
             const int groups = (int)std::min(most / 4, (long)avail / FT_MIN_GROUP);
-            if (slots == 4 && groups >= 1 && (long)per_seg * 4 * groups > 12L * n_cus)
+            if (skew && slots == 4 && groups >= 1 && (long)per_seg * 4 * groups > 12L * n_cus)
                 consider(groups, 4 * groups);
             const int n = (int)std::min(most, (long)avail);
             if (n >= 2 && (long)per_seg * n > 8L * n_cus)
                 consider(-1, n);
         }
+}
+static void plan_gqa(Seg &seg, int BH, int T, unsigned skew)
+{
+    plan_uneven(seg, T, padded_units<32>(BH, seg.nseg) * 32, skew);
+    plan_rounds(seg, pad4((BH + 1) / 2), T, skew);
+}
+// Shared-table launches of head dim 128: nearly equal segments only.  us per step, 32 heads, the even plan / this: 10 x 20000 284 / 260, 6 x
+// 68692 518 / 505.  (256 channels, 3 x 16 x 93341, 73 segments / 85: 367 / 362, where two runs of one side differ by as much.)
+static void plan_shared(Seg &seg, int BH, int T, int D)
+{
+    if (D == 128)
+        plan_rounds(seg, pad4((BH + 1) / 2), T, 0);
 }
 
 // How many segments the forward_ov partial sums of a launch can have under either plan (what a
@@ -2890,10 +2901,12 @@ static int max_plan_segments(void *ckpt, int n_ckpt_cap, int ckpt_interval, int 
         plan_ft(b, B, H, T, FT_SKEW_QK, true);
         plan_ft_ov(c, B, H, T);
         n = std::max(std::max(n, a.nseg), std::max(b.nseg, c.nseg));
-        plan_gqa(seg, B * H, T, GQA_SKEW_OV);
-        n = std::max(n, seg.nseg);
+        Seg d = seg;
+        plan_gqa(d, B * H, T, GQA_SKEW_OV);
+        n = std::max(n, d.nseg);
     }
-    return n;
+    plan_shared(seg, B * H, T, D);
+    return std::max(n, seg.nseg);
 }
 
 // Whether adkv_decode_step may run its three stages as ONE launch (decode_ft_kernel): off unless
@@ -3541,12 +3554,13 @@ static const char *decode_kernel_name(bool ov, int B, int Hq, int H, int T, int 
                          : "ft_kernel (per-head table, 16-wave workgroups)";
     }
     if (D == 128) {
-        const long units = padded_units<32>(BH, seg.nseg);
         if (ov ? ov_lone(BH, seg.nseg, T) : qk_lone(BH, seg.nseg, T))
             return "lone_kernel (shared table, one channel per lane)";
         if (!ov && qk_pair(BH, seg.nseg))
             return "kernel<128,2,256> (shared table, two channels per lane)";
-        const int blk = threads_per_workgroup(units * 32);
+        Seg s2 = seg;
+        plan_shared(s2, BH, T, D);
+        const int blk = threads_per_workgroup(padded_units<32>(BH, s2.nseg) * 32);
         return blk == 1024 ? "kernel<128,4,1024> (shared table)"
                : blk == 768 ? "kernel<128,4,768> (shared table)"
                             : "kernel<128,4,256> (shared table)";
@@ -3619,6 +3633,7 @@ static int forward_qk_impl(const void *q, void *k_cache, const void *k_new, void
                      (const h1 *)sc, (const h1 *)alpha, (const h1 *)beta, (const h1 *)tgt, BH, H, T, n_super_cap, (h1 *)state_out, seg);
         return check_launch();
     }
+    plan_shared(seg, BH, T, D);
     ADKV_DISPATCH_D(qk_kernel, (const h1 *)q, (uint4 *)k_cache, (const h1 *)k_new, (h1 *)logits,
                     (const h1 *)zp, (const h1 *)sc, (const h1 *)alpha, (const h1 *)beta,
                     (const h1 *)tgt, BH, H, T, n_super_cap, (h1 *)state_out, seg);
@@ -3699,6 +3714,8 @@ int adkv_decode_segments(int B, int Hq, int H, int T, int D, int bits, int n_ckp
         const int W = ft_wgs_per_head(B, seg.nseg, 64 / lanes);
         wgs = (long)H * seg.phys_per_head;
         virt = (W + seg.phys_per_head - 1) / seg.phys_per_head;
+    } else if (!matrix_cores && !(D == 128 && (qk_lone(B * H, seg.nseg, T) || qk_pair(B * H, seg.nseg)))) {
+        plan_shared(seg, B * H, T, D);
     }
     if (bounds != nullptr && max_bounds > seg.nseg) {
         for (int s = 0; s < seg.nseg; s++)
@@ -3798,12 +3815,16 @@ static int forward_ov_impl(const void *attn, void *v_cache, const void *v_new, v
     // there; no second launch and nothing in the workspace
     seg.combine = (head_table && ft_ov_combines(seg, B, ft_lanes)) ? 1 : 0;
     const bool pair = matrix_cores && ov_gqa_pair(BH, seg.nseg, GQ, ((uintptr_t)attn & 15) == 0 && seg.row_pitch % 8 == 0);
-    if (matrix_cores && GQ <= 4 && !pair) {
+    const bool lone = !matrix_cores && !head_table && D == 128 && ov_lone(BH, seg.nseg, T);
+    if (matrix_cores ? GQ <= 4 && !pair : !head_table && !lone) {
         Seg s = seg;
-        plan_gqa(s, BH, T, GQA_SKEW_OV);
+        if (matrix_cores)
+            plan_gqa(s, BH, T, GQA_SKEW_OV);
+        else
+            plan_shared(s, BH, T, D);
         if (workspace_bytes >= (int64_t)s.nseg * BH * GQ * D * 4)
             seg = s;
-        else // a workspace for fewer segments keeps the even plan's number of them
+        else if (matrix_cores) // a workspace for fewer segments keeps the even plan's number of them
             plan_uneven(seg, T, padded_units<32>(BH, seg.nseg) * 32, GQA_SKEW_OV);
     }
     if (seg.nseg > 1 && !seg.combine) {
@@ -3823,7 +3844,7 @@ static int forward_ov_impl(const void *attn, void *v_cache, const void *v_new, v
                            dim3(FT_BLK), 0, st, (const h1 *)attn, (uint4 *)v_cache, (const h1 *)v_new, (h1 *)out,
                            (float *)workspace, (const h1 *)zp, (const h1 *)sc, (const h1 *)alpha,
                            (const h1 *)beta, (const h1 *)tgt, B, H, T, n_super_cap, (h1 *)state_out, seg);
-    } else if (D == 128 && ov_lone(BH, seg.nseg, T)) {
+    } else if (lone) {
         const FtParams p = {(const h1 *)zp, (const h1 *)sc, (const h1 *)alpha, (const h1 *)beta, (const h1 *)tgt};
         ADKV_LAUNCH_LONE(ov_lone_kernel, 1024, (const h1 *)attn,
                            (uint4 *)v_cache, (const h1 *)v_new, (h1 *)out, (float *)workspace, p, BH, H, T, n_super_cap,

@@ -1,5 +1,5 @@
-"""Matrix-core launches whose segments are nearly equal, or more groups of uneven ones than the even plan has: against the same
-calls without checkpoints, one segment."""
+"""Launches of four channels per lane whose segments are nearly equal, or more groups of uneven ones than the even plan has: against
+the same calls without checkpoints, one segment.  The last shape is a shared-table launch, the others are matrix-core ones."""
 import ctypes
 import math
 
@@ -12,7 +12,8 @@ from adkv_amd.kernel import gemv
 SMIN, SMAX = math.exp(-4.0), math.exp(4.0)
 # sequences, query heads, KV heads, tokens, interval, bits -> segments, balanced
 SHAPES = [((17, 32, 8, 3899, 64, 4), 60, True), ((17, 16, 8, 3904, 64, 2), 60, True), ((17, 8, 8, 3841, 64, 2), 60, True),
-          ((34, 32, 8, 961, 16, 4), 28, False), ((128, 8, 2, 1257, 16, 4), 32, False), ((69, 8, 2, 2912, 16, 4), 56, False)]
+          ((34, 32, 8, 961, 16, 4), 28, False), ((128, 8, 2, 1257, 16, 4), 32, False), ((69, 8, 2, 2912, 16, 4), 56, False),
+          ((10, 32, 32, 1257, 16, 4), 25, True)]
 
 
 def _bounds(B, Hq, H, T, S, bits):
