@@ -1108,6 +1108,25 @@ __device__ __forceinline__ void pair_bytes_of(const typename Geo<D, CPL>::Vec *u
 typedef _Float16 h8v __attribute__((ext_vector_type(8))); // operand of v_mfma_f32_16x16x32_f16
 constexpr int PAIR_TILE = 16 * 256; // bytes of a wave's key tile
 
+// Entries of one unit of eight tokens of a lane's channel pair: e[t] for token t.
+template <int BITS>
+__device__ __forceinline__ void pair_lookup(uint2 *e, const uint2 *lut, const uint32_t *nb, uint32_t lane_copy, int unit)
+{
+    if constexpr (BITS == 4) {
+#pragma unroll
+        for (int t = 0; t < 8; t++)
+            e[t] = lut_get(lut, nb[t & 1], lane_copy, t >> 1);
+    } else { // an entry is tokens s and s + 2
+#pragma unroll
+        for (int s = 0; s < 4; s++) {
+            const int t = 4 * (s >> 1) + (s & 1);
+            const uint4 v = lut2_get(lut, nb[s & 1], lane_copy, 2 * unit + (s >> 1));
+            e[t] = make_uint2(v.x, v.y);
+            e[t + 2] = make_uint2(v.z, v.w);
+        }
+    }
+}
+
 // forward_qk of a segment with the head over a whole wave, two channels per lane, for GQ query heads.
 // A wave has its SIMD (nearly) to itself and pays for every instruction, so what is left per
 // token is the lookup, the replay (replay_eight) and half a write: the values of 16 tokens go
@@ -1219,21 +1238,7 @@ struct PairScores {
             else
                 pair_bytes2(u.x, u.y, nb[0], nb[1]);
         };
-        auto lookup = [&](uint2 *l, int unit) __attribute__((always_inline)) {
-            if constexpr (BITS == 4) {
-#pragma unroll
-                for (int t = 0; t < 8; t++)
-                    l[t] = lut_get(lut, nb[t & 1], lane_copy, t >> 1);
-            } else { // an entry is tokens s and s + 2
-#pragma unroll
-                for (int s = 0; s < 4; s++) {
-                    const int t = 4 * (s >> 1) + (s & 1);
-                    const uint4 v = lut2_get(lut, nb[s & 1], lane_copy, 2 * unit + (s >> 1));
-                    l[t] = make_uint2(v.x, v.y);
-                    l[t + 2] = make_uint2(v.z, v.w);
-                }
-            }
-        };
+        auto lookup = [&](uint2 *l, int unit) __attribute__((always_inline)) { pair_lookup<BITS>(l, lut, nb, lane_copy, unit); };
         // no scalar load in flight when the loop starts: its waits would have to cover it
         bytes(buf[0][0]);
         lookup(e[0], 0);
