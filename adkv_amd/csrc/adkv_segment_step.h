@@ -538,7 +538,8 @@ __global__ __launch_bounds__(256) void step_combine_kernel(
     }
     // What else a wave reads travels meanwhile: the mask, or its share of the first AHEAD segments' partial outputs.  (Behind the
     // reductions it was a second trip to memory: steps of 1 x 8 KV heads x 16000 tokens with four query heads 15.6 us instead of 14.5, 10 x 8 x
-    // 9000 with eight 55.6 instead of 54.0, 6 x 8 x 9000 33.5 instead of 32.8, 4 x 8 x 8190 of 256 channels 32.8 instead of 32.5.)
+    // 9000 with eight 55.6 instead of 54.0, 6 x 8 x 9000 33.5 instead of 32.8, 4 x 8 x 8190 of 256 channels 32.8 instead of 32.5.  Only what is there
+    // is read: rows of three segments read four, and tokens behind the row's end, 0.4 us more for 64 x 32 x 663 with a mask.)
     constexpr int AHEAD = 4;
     const MaskRow<true> mrow = mk.of<true>((unsigned)row, n);
     float add[VECS][8] = {};
@@ -548,7 +549,7 @@ __global__ __launch_bounds__(256) void step_combine_kernel(
             const int t = t0 + i * 512;
             if (t + 8 <= n) {
                 mrow.load<8>(t, add[i]);
-            } else {
+            } else if (t < n) {
 #pragma unroll
                 for (int k = 0; k < 8; k++)
                     add[i][k] = mrow.at(min(t + k, n - 1));
@@ -564,9 +565,11 @@ __global__ __launch_bounds__(256) void step_combine_kernel(
     if (!writes_weights) {
 #pragma unroll
         for (int i = 0; i < AHEAD; i++) {
-            const int k = min(lane / lanes + i * groups, nseg - 1);
-            ahead[i] = part(k);
-            max_ahead[i] = ml[k].x;
+            const int k = lane / lanes + i * groups;
+            if (k < nseg) {
+                ahead[i] = part(k);
+                max_ahead[i] = ml[k].x;
+            }
         }
     }
     float M = first.x;
