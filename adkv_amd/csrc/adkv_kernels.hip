@@ -3821,6 +3821,13 @@ static int forward_ov_impl(const void *attn, void *v_cache, const void *v_new, v
     seg.combine = (head_table && ft_ov_combines(seg, B, ft_lanes)) ? 1 : 0;
     const bool pair = matrix_cores && ov_gqa_pair(BH, seg.nseg, GQ, ((uintptr_t)attn & 15) == 0 && seg.row_pitch % 8 == 0);
     const bool lone = !matrix_cores && !head_table && D == 128 && ov_lone(BH, seg.nseg, T);
+    // a workspace has to hold the even plan's sums, whichever plan runs
+    if (seg.nseg > 1 && !seg.combine) {
+        if (!workspace || workspace_bytes < (int64_t)seg.nseg * BH * GQ * D * 4)
+            return ADKV_E_WORKSPACE;
+        if ((uintptr_t)workspace & 15)
+            return ADKV_E_ALIGN;
+    }
     if (matrix_cores ? GQ <= 4 && !pair : !head_table && !lone) {
         Seg s = seg;
         if (matrix_cores)
@@ -3829,14 +3836,8 @@ static int forward_ov_impl(const void *attn, void *v_cache, const void *v_new, v
             plan_shared(s, BH, T, D);
         if (workspace_bytes >= (int64_t)s.nseg * BH * GQ * D * 4)
             seg = s;
-        else if (matrix_cores) // a workspace for fewer segments keeps the even plan's number of them
+        else if (matrix_cores) // one that holds no more keeps the even plan's number of segments
             plan_uneven(seg, T, padded_units<32>(BH, seg.nseg) * 32, GQA_SKEW_OV);
-    }
-    if (seg.nseg > 1 && !seg.combine) {
-        if (!workspace || workspace_bytes < (int64_t)seg.nseg * BH * GQ * D * 4)
-            return ADKV_E_WORKSPACE;
-        if ((uintptr_t)workspace & 15)
-            return ADKV_E_ALIGN;
     }
     if (matrix_cores) {
         ADKV_DISPATCH_GQ(ov_gqa_kernel, false, (const h1 *)attn, (uint4 *)v_cache, (const h1 *)v_new,

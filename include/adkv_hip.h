@@ -218,7 +218,11 @@ int adkv_forward_qk_ex(const void *q, void *k_cache, const void *k_new, void *lo
                        void *state_out, void *ckpt, int n_ckpt_cap, int ckpt_interval,
                        void *stream);
 
-/* Bytes of fp32 workspace adkv_forward_ov_ex needs for these sizes (0 when it runs one segment). */
+/* Bytes of fp32 workspace with which adkv_forward_ov_ex cuts the context as it is fastest for these sizes (0 when it runs
+ * one segment).  The call refuses a workspace that does not hold a partial output for each of as many equal segments of whole
+ * checkpoint intervals as fill the device (ADKV_E_WORKSPACE).  Some launches are faster in a few more segments than that;
+ * with a workspace between the two sizes they run in the equal ones: the same sums of the same products, added in another
+ * order.  adkv_decode_step's workspace always holds the larger number. */
 int64_t adkv_forward_ov_workspace_bytes(int B, int H, int T, int D, int n_ckpt_cap,
                                         int ckpt_interval);
 
