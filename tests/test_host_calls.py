@@ -178,3 +178,18 @@ def test_written_tensors_that_share_their_storage_lazily_become_their_own(gpu):
         quant_f32_pair(x, p, -8, 7, 0.1, 2.0, states=[tuple(out[2:4]), tuple(out[4:])], out=out[:2])
     for t, a, b in zip(shared, mine, plain):
         assert torch.all(t == 1.0) and torch.equal(a, b)
+
+
+@pytest.mark.gpu
+def test_a_profiler_sees_the_tensors_that_a_call_makes(gpu):
+    h = _lib.host()
+    q, cs = torch.randn(2, 4, 3, 128, device=gpu).half(), torch.randn(2, 3, 128, device=gpu).half()
+    x, p = torch.randn(1, 8, 128, device=gpu), tuple(torch.full((128,), 0.5, device=gpu) for _ in range(5))
+    for call in (lambda: h.rope_qk(q, q, cs, cs), lambda: h.quant_f32(x, p, -8, 7, 0.1, 2.0, False, False)):
+        want = call()
+        assert want is not None
+        with torch.profiler.profile(activities=[torch.profiler.ProfilerActivity.CPU]) as seen:
+            got = call()
+        assert [e.count for e in seen.key_averages() if e.key == "aten::empty"] == [2]
+        for a, b in zip(want, got):
+            assert not isinstance(a, torch.Tensor) or torch.equal(a, b)
