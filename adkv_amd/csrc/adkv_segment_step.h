@@ -246,6 +246,10 @@ __device__ __forceinline__ void lone_weights(const float *share, int stride, h1 
         a = make_float4(a.x + b.x, a.y + b.y, a.z + b.z, a.w + b.w);
         extra += share[i * stride + 256];
     }
+    // Eight shares are added here: the compiler puts the additions behind the mask's loads and keeps all 40 registers until then, beside
+    // the units that the values' waves hold (18 spilled; 2 x 8 heads x 2000 of 512 channels 16.9 us, 16.6 like this, 1 x 8 x 8000 19.0 / 18.7).
+    if constexpr (HW == 8)
+        asm volatile("" : "+v"(a.x), "+v"(a.y), "+v"(a.z), "+v"(a.w), "+v"(extra));
     const h1 l[5] = {(h1)a.x, (h1)a.y, (h1)a.z, (h1)a.w, (h1)extra};
     if (writes) {
         if (t + 4 <= ntok) { // t0 and the pitch are multiples of 8

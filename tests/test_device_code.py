@@ -137,6 +137,14 @@ def test_rows_without_16_bit_masks_keep_four_waves_to_a_simd(listings):
     assert len(found) == 9 and not [f for f in found if f[1] > 128], found
 
 
+def test_waves_beside_each_other_keep_what_they_hold_in_registers(listings):
+    """The values' waves of a step live from the units that they hold: none of it in memory."""
+    found = [(name, int(private), int(spilled)) for _, notes in listings for name, private, spilled in
+             re.findall(r"\.name: +(\S*(?:step_beside_lone|small_step)_kernel\S*)\n.*?\.private_segment_fixed_size: +(\d+).*?\.vgpr_spill_count: +(\d+)",
+                        notes, re.S)]
+    assert len(found) == 23 and not [f for f in found if f[1] or f[2]], found
+
+
 def test_the_weights_loop_keeps_its_loads_in_flight(listings):
     """Codes of seven supergroups."""
     (name, code, after), = [k for t, _ in listings for k in kernels(t, "14ov_lone_kernelILi256E")]
