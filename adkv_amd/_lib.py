@@ -25,6 +25,7 @@ PROTOTYPES = {
     "adkv_decode_step_is_fused": (_i, [_i] * 9),
     "adkv_decode_step_launches": (_i, [_i] * 9),
     "adkv_decode_step_kernel_name": (C.c_char_p, [_i] * 9),
+    "adkv_decode_step_values_ahead": (_i, [_i] * 8),
     "adkv_strerror": (C.c_char_p, [_i]),
     "adkv_last_hip_error": (_i, []),
     "adkv_encode_kv": (_i, [_vp] * 7 + [_i] * 5 + [_f, _f, _vp, _vp]),

@@ -3083,26 +3083,34 @@ static int step_lone_threads(long units, int D, int GQ, int longest)
 // 15.8, 3 x 8 x 6000 (5) 20.7 / 18.4, 8 x 8 x 4096 (8) 22.7 / 20.5; eight, 1 x 8 x 4000 17.5 / 14.2, 5 x 8 x 5632 (8) 26.4 / 24.1; 2-bit,
 // four, 1 x 8 x 4000 15.0 / 12.3, 6 x 8 x 4096 (6) 20.3 / 18.2, one, 4 x 32 x 2048 (8) 18.4 / 17.8; 256 channels, 1 x 8 x 2000 14.4 / 12.2, 4 x 8 x
 // 4000 (8) 18.8 / 18.2; 512, 1 x 8 x 1000 18.4 / 16.6, 2 x 8 x 2000 (4) 18.5 / 17.0.
+// Returns the units that a values' wave holds; 0: a wave takes keys and values.  blk: of step_lone_threads.
+static int step_values_ahead(int blk, long units, int D)
+{
+    if (blk == 256)
+        return units * (D / 64) <= 4L * cus() ? 24 : 16;
+    return blk == 512 ? 16 : 0;
+}
 template <int D, int BITS, int GQ, typename... Args>
 static int launch_step_lone(int blk, long units, hipStream_t st, Args... args)
 {
-    const int per_block = blk / D; // units: a wave per 64 channels
+    const int per_block = blk / D, ahead = step_values_ahead(blk, units, D); // units: a wave per 64 channels
     const dim3 grid((unsigned)((units + per_block - 1) / per_block));
 #define ADKV_STEP(BLK) hipLaunchKernelGGL((step_lone_kernel<D, BITS, GQ, BLK>), grid, dim3(BLK), 0, st, args...)
 #define ADKV_BESIDE(BLK, AHEAD) hipLaunchKernelGGL((step_beside_lone_kernel<D, BITS, GQ, (BLK) / 64, AHEAD>), grid, dim3(2 * (BLK)), 0, st, args...)
     if constexpr (D != 512) {
-        if (blk == 256 && units * (D / 64) <= 4L * cus())
+        if (ahead == 24)
             ADKV_BESIDE(256, 24);
-        else if constexpr (GQ == 1)
-            if (blk == 256)
+        if constexpr (GQ == 1) {
+            if (blk == 256 && ahead == 16)
                 ADKV_BESIDE(256, 16);
+        }
         if constexpr (GQ != 8) {
             if (blk == 768)
                 ADKV_STEP(768);
         }
     }
     if constexpr (D == 512 || GQ > 1) {
-        if (blk == 512)
+        if (ahead == 16 && blk == 512)
             ADKV_BESIDE(512, 16);
     }
     if constexpr (D != 128) {
@@ -3686,7 +3694,7 @@ const char *adkv_decode_step_kernel_name(int B, int Hq, int H, int T, int D, int
         segment_step_plan(seg, cpl, B, Hq, H, T, D, bits, ck, ck, n_ckpt_cap, ckpt_interval);
         switch (step_lone_threads(padded_units<64>(B * H, seg.nseg), D, Hq / H, longest_segment(seg, T))) {
         case 0: return "step_segments_kernel";
-        case 256: return "step_lone_kernel, 4-wave workgroups"; // of keys, the values have theirs beside them
+        case 256: return "step_lone_kernel, 4-wave workgroups"; // of keys, see adkv_decode_step_values_ahead
         case 512: return "step_lone_kernel, 8-wave workgroups";
         case 768: return "step_lone_kernel, 12-wave workgroups";
         default: return "step_lone_kernel, 16-wave workgroups";
@@ -3694,6 +3702,18 @@ const char *adkv_decode_step_kernel_name(int B, int Hq, int H, int T, int D, int
     default:
         return nullptr;
     }
+}
+
+int adkv_decode_step_values_ahead(int B, int Hq, int H, int T, int D, int bits, int n_ckpt_cap, int ckpt_interval)
+{
+    int dummy = 0, cpl;
+    Seg seg;
+    void *ck = n_ckpt_cap > 0 && ckpt_interval > 0 ? &dummy : nullptr;
+    if (adkv_decode_step_launches(B, Hq, H, T, D, bits, n_ckpt_cap, ckpt_interval, 0) != 2 ||
+        !segment_step_plan(seg, cpl, B, Hq, H, T, D, bits, ck, ck, n_ckpt_cap, ckpt_interval))
+        return 0;
+    const long units = padded_units<64>(B * H, seg.nseg);
+    return step_values_ahead(step_lone_threads(units, D, Hq / H, longest_segment(seg, T)), units, D);
 }
 
 int adkv_decode_segments(int B, int Hq, int H, int T, int D, int bits, int n_ckpt_cap,

@@ -533,6 +533,8 @@ def decode_record(args, B, Hq, H, D, T, bits, S, NL, steps, warmup, headline=Tru
         res["kernel_ms"] = {"one_launch": qk_ms, "step_device_median": dev_ms, "steps_with_events": len(marks)}
     elif len(kernels) == 2:
         res["kernel_ms"] = {"segments": qk_ms, "combine": ov_ms, "step_device_median": dev_ms, "steps_with_events": len(marks)}
+        # units of eight tokens that waves of the values' own hold beside the keys'; 0: a wave takes both
+        res["step_values_ahead"] = L.adkv_decode_step_values_ahead(B, Hq, H, T, D, bits, ncap_arg, S)
     else:  # the second big launch of the step, same algorithmic bytes (the V codes)
         res["roofline_ov"] = {"kernel": kernels[2], "bound": "hbm", "achieved": code_bytes / (ov_ms * 1e-3) / 1e9,
                               "peak": HBM_PEAK_GBPS, "unit": "GB/s", "frac": code_bytes / (ov_ms * 1e-3) / 1e9 / HBM_PEAK_GBPS,

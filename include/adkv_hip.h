@@ -62,7 +62,10 @@ void adkv_set_mha_kernel(int use_matrix_cores);
  * forward_ov are launched one after the other, also for sizes that the call refuses.
  * adkv_decode_step_kernel_name: the first kernel of a call in one or two launches, a static string for benchmark records
  * and tests; NULL for the others (adkv_decode_kernel_name and adkv_decode_ov_kernel_name have theirs).  A step_lone_kernel's
- * waves are those that take a segment's keys: with few of them its values have as many of their own beside them. */
+ * waves are those that take a segment's keys: with few of them its values have as many of their own beside them
+ * (step_beside_lone_kernel).
+ * adkv_decode_step_values_ahead: for a call in two launches whose values have, how many units of eight tokens each of their waves
+ * holds until the weights are there, 24 or 16; 0 for all other calls.  A mask makes no difference to it. */
 void adkv_set_fused_step(int mode);
 int adkv_decode_step_is_fused(int B, int Hq, int H, int T, int D, int bits, int n_ckpt_cap,
                               int ckpt_interval, int masked);
@@ -70,6 +73,7 @@ int adkv_decode_step_launches(int B, int Hq, int H, int T, int D, int bits, int 
                               int ckpt_interval, int masked);
 const char *adkv_decode_step_kernel_name(int B, int Hq, int H, int T, int D, int bits, int n_ckpt_cap,
                                          int ckpt_interval, int masked);
+int adkv_decode_step_values_ahead(int B, int Hq, int H, int T, int D, int bits, int n_ckpt_cap, int ckpt_interval);
 const char *adkv_strerror(int code);
 /* hipError_t (as int) of the last failed launch in this thread, 0 if none. */
 int adkv_last_hip_error(void);

@@ -144,6 +144,30 @@ def test_library_and_benchmark_name_the_first_kernel_of_a_step():
         L.adkv_set_fused_step(0)
 
 
+def test_library_says_whether_the_values_have_waves_beside_the_keys():
+    """Without a GPU (256 CUs): 24 units held with up to four waves of keys per CU, 16 up to eight, none beyond and in the other
+    kernels.  The rows of test_gpu_step_beside.test_most_waves, then what lies behind them."""
+    L = _lib.lib()
+    ahead = lambda B, Hq, H, D, T, bits, S=256: L.adkv_decode_step_values_ahead(B, Hq, H, T, D, bits, T // S + 1 if S else 0, S)
+    for n, rows in ((24, ((2, 32, 32, 128, 2000, 4), (4, 32, 16, 128, 2048, 4), (8, 64, 8, 128, 2000, 4), (2, 32, 32, 128, 1999, 2),
+                          (2, 16, 16, 256, 2000, 4))),
+                    (16, ((2, 32, 32, 128, 2100, 4), (4, 32, 16, 128, 2049, 4), (2, 16, 16, 256, 2064, 4), (4, 32, 32, 128, 2047, 4),
+                          (4, 32, 32, 128, 1800, 2), (8, 32, 16, 128, 2048, 4), (5, 32, 8, 128, 6400, 4), (5, 64, 8, 128, 5633, 4),
+                          (4, 16, 16, 256, 2040, 4), (3, 8, 8, 512, 2500, 4), (1, 8, 8, 512, 8192, 4), (1, 8, 8, 512, 300, 4))),
+                    (0, ((4, 32, 32, 128, 2049, 4), (8, 32, 16, 128, 2049, 4), (16, 64, 8, 128, 2049, 4), (4, 16, 16, 256, 2049, 4),
+                         (2, 8, 8, 512, 4097, 4), (8, 32, 8, 128, 16001, 4), (1, 32, 32, 128, 603, 4), (128, 32, 32, 128, 4096, 4)))):
+        for row in rows:
+            assert ahead(*row) == n, row
+    assert ahead(2, 8, 2, 128, 1500, 4, 512) == 0                              # segments beyond 256 tokens
+    for bad in ((0, 8, 8, 128, 100, 4), (1, 6, 4, 128, 100, 4), (1, 8, 8, 128, -1, 4), (1, 8, 8, 128, 100, 3), (2, 16, 8, 256, 100, 4)):
+        assert ahead(*bad) == 0
+    L.adkv_set_mha_kernel(0)
+    try:
+        assert ahead(2, 32, 32, 128, 2000, 4) == 0
+    finally:
+        L.adkv_set_mha_kernel(-1)
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("H,T,S", [(4, 200, 64), (3, 600, 256)])
 def test_one_launch_step_replays_from_a_captured_graph(gpu, H, T, S):
