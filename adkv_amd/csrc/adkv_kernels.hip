@@ -92,9 +92,9 @@ struct Seg {
     long row_pitch;     // elements between rows of the logits / attention-weight matrix (>= T + 1)
     int act_bf16;       // q, the new token and the output are bfloat16 (see load_act2 / store_act2)
     int combine;        // ov_ft_kernel: the segments' partial outputs are added inside the workgroup
-    // Per-head-table and matrix-core kernels only.  groups > 0: the context's `intervals` checkpoint intervals are
-    // cut into `groups` groups of four segments of unequal length (uneven_cut).  groups < 0: into nseg segments that
-    // differ by one interval at most.  phys_per_head (per-head table):
+    // groups > 0 (per-head-table and matrix-core kernels): the context's `intervals` checkpoint intervals are
+    // cut into `groups` groups of four segments of unequal length (uneven_cut).  groups < 0 (matrix-core and shared-table
+    // ones of head dim 128): into nseg segments that differ by one interval at most.  phys_per_head (per-head table):
     // workgroups launched per KV head; each walks through the head's virtual workgroups pw,
     // pw + phys_per_head, ... one after the other (same table, no barrier between them).
     int groups;
@@ -2514,11 +2514,11 @@ static bool ov_lone(int BH, int nseg, int T) { return padded_units<64>(BH, nseg)
     } while (0)
 
 // Matrix-core kernels (head dim 128), four channels per lane: 12- or 16-wave workgroups by the same
-// rule.  Eight query heads per KV head need ~138 registers per lane, more than the 128 a 16-wave
-// workgroup leaves: qk_gqa_kernel still gains from four waves per SIMD with a dozen cold values spilled
-// (16 x 8 KV heads x 131072 tokens, 64 query heads: 563 -> 530 us with 4-bit codes, 518 -> 425 us with
-// 2-bit ones), ov_gqa_kernel spills accumulators and loses (421 -> 533 us, 346 -> 747 us), so BIG8 says
-// which of the two this is, and the latter takes 8-wave workgroups.
+// rule.  With eight query heads per KV head ov_gqa_kernel needs 142 registers per lane, more than the 128 a 16-wave
+// workgroup leaves: there it spills accumulators and loses (16 x 8 KV heads x 131072 tokens, 64 query heads: 421 -> 533 us
+// with 4-bit codes, 346 -> 747 us with 2-bit ones), and takes 8-wave workgroups.  qk_gqa_kernel fits into 118, and gained from
+// four waves per SIMD when it still needed 138 and spilled a dozen (563 -> 530 us, 518 -> 425 us).  BIG8 says which of the two
+// this is.
 // A launch that would leave at most two waves on a SIMD takes two channels per lane instead (a KV head
 // per wave): twice the waves, forward_qk without the reduction over the quarters of a head.  With more waves than
 // that the four-channel lanes have enough of them and spend fewer instructions on what a wave does once per token.
@@ -2833,7 +2833,10 @@ static void plan_uneven(Seg &seg, int T, long threads, unsigned skew)
 // with three waves, 0.83 with four alike, 0.89 with four uneven ones (SQ_ACTIVE_INST_VALU).  Another plan has to be 5 % shorter.
 // us per step, the even plan (uneven where its segments are a multiple of four) / this: 17 x 8 x 15467 175 / 116, 128 x 2 x 20219 240 / 226, 69 x 2 x
 // 46577 307 / 282 (four query heads), 24 x 32 x 12000 2-bit 331 / 318, 48 x 8 x 9000 (two) 159 / 155; the others of eleven such sizes
-// keep theirs.
+// keep theirs.  Of 82 sizes drawn at random among those that take another plan than the even one: 29 of one query head in 2 bits 0.90 of
+// the even plan's time, 27 of four 0.94, in 2 bits (26) 0.90; the worst 1.010 (20 x 2 x 58865, 136.8 / 138.2, runs 1.8 apart), the others below 1.
+// Eight query heads are not planned like this: forward_ov's workgroups have eight waves then, which is not what the model counts.  For
+// forward_qk alone it would hold: 17 x 8 x 15467 193 / 161, 24 x 8 x 12000 187 / 185, 16 x 8 x 131072 2-bit 732 / 726, five others the same.
 static void plan_rounds(Seg &seg, int per_seg, int T, unsigned skew) // per_seg: waves per segment; skew: 0, no uneven groups
 {
     const int n_cus = cus();
@@ -2887,7 +2890,7 @@ static void plan_gqa(Seg &seg, int BH, int T, unsigned skew)
     plan_rounds(seg, pad4((BH + 1) / 2), T, skew);
 }
 // Shared-table launches of head dim 128: nearly equal segments only.  us per step, 32 heads, the even plan / this: 10 x 20000 284 / 260, 6 x
-// 68692 518 / 505.  (256 channels, 3 x 16 x 93341, 73 segments / 85: 367 / 362, where two runs of one side differ by as much.)
+// 68692 518 / 505; 26 sizes drawn at random 0.82 to 0.995 of the even plan's time, 0.95 in the mean.  (256 channels, 3 x 16 x 93341, 73 segments / 85: 367 / 362, where two runs of one side differ by as much.)
 static void plan_shared(Seg &seg, int BH, int T, int D)
 {
     if (D == 128)
@@ -2944,8 +2947,11 @@ static int fused_step_plan(Seg &ka, Seg &va, int B, int Hq, int H, int T, int D,
 }
 
 // Whether a step runs as small_step_kernel, and its plan: a workgroup per (sequence, head), one per CU, four
-// waves per segment.  us per step on the device, three or four launches / one, sequences x heads x tokens: 1 x 32 x 603
-// 25.6 / 11.0 (and 15 us of host time / 5), 8 x 32 x 1000 27.7 / 16.3, 4 x 32 x 200 20.4 / 11.0, 2 x 8 x 64 12.8 / 7.8.
+// waves per segment.  us per step on the device, one launch / the two that it would be otherwise (step_beside_lone_kernel), sequences x
+// heads x tokens: 1 x 32 x 603 10.7 / 12.2, 4 x 32 x 200 9.4 / 11.0, 8 x 32 x 500 11.9 / 13.5, 8 x 32 x 1000 16.0 / 18.6, 5 x 40 x 700
+// 13.2 / 17.3, 2 x 8 x 64 6.3 / 7.8; the second launch costs the host 3 us more.  Four segments of few heads are the other way round,
+// 1 x 32 x 1000 14.6 / 12.7, 4 x 32 x 1000 15.3 / 13.2, 1 x 8 x 1024 14.9 / 12.3 (with the rotary embedding and the host's part 17.5 / 16.4,
+// 17.3 / 16.4, 17.4 / 15.9): the line does not lie there yet.
 // With five to eight segments four waves share a SIMD while other CUs idle, and beyond one workgroup per CU (its LDS
 // allows no second) a launch takes two rounds: those stay with the separate launches.
 static bool small_step_plan(Seg &seg, int B, int Hq, int H, int T, int D, int bits, void *k_ckpt, void *v_ckpt,
@@ -3043,17 +3049,19 @@ static int launch_step_grouped(int GQ, long waves, hipStream_t st, Args... args)
 // twice the waves of two channels per lane and four or eight times those of wide heads, and pay as long as a CU holds
 // them at once: 16 waves, and 12 / 8 with four / eight query heads, whose logits take more of the LDS; with one or two
 // query heads of 128 channels, whose other form has its waves' LDS reads covered by then, 12.  us per step on the
-// device, step_segments_kernel / this, waves per CU in brackets:
-//   512 channels: 9 x 8 heads x 80 (2) 22.8 / 11.8, 2 x 8 x 1000 (2) 47.7 / 18.7, 8 x 8 x 2000 (16) 48.8 / 28.9
-//   256: 1 x 8 x 300 30.3 / 14.1, 2 x 16 x 5021 (10) 31.7 / 23.2, 4 x 8 x 8190 (16) 33.7 / 30.4
-//   128: 1 x 32 x 2000 (2) 20.7 / 15.7, 4 x 32 x 2000 (8) 21.3 / 19.5, 6 x 32 x 2000 (12) 27.3 / 24.1, 8 x 32 x 2000 (16)
+// device, step_segments_kernel / this, waves per CU in brackets (up to eight: with the values beside the keys, see launch_step_lone):
+//   512 channels: 9 x 8 heads x 80 (3) 21.5 / 10.3, 2 x 8 x 1000 (2) 47.0 / 16.3, 8 x 8 x 2000 (16) 48.0 / 29.6
+//   256: 1 x 8 x 300 30.1 / 11.6, 2 x 16 x 5021 (10) 31.2 / 23.7, 4 x 8 x 8190 (16) 32.8 / 29.2
+//   128: 1 x 32 x 2000 (2) 19.5 / 12.4, 4 x 32 x 2000 (8) 20.5 / 18.3, 6 x 32 x 2000 (12) 26.0 / 23.1, 8 x 32 x 2000 (16)
 //     27.4 / 28.0
-//   two query heads: 4 x 16 x 2000 (4) 22.6 / 16.3, 8 x 16 x 2000 (8) 23.3 / 20.3, 12 x 16 x 2000 (12) 30.0 / 25.6,
+//   two query heads: 4 x 16 x 2000 (4) 20.2 / 12.8, 8 x 16 x 2000 (8) 21.1 / 17.8, 12 x 16 x 2000 (12) 28.8 / 25.6,
 //     16 x 16 x 2000 (16) 31.1 / 30.7
-//   four: 1 x 8 x 603 22.2 / 15.3, 28 x 8 x 936 (7) 24.5 / 21.3, 8 x 8 x 6000 (12) 33.5 / 28.4, 8 x 8 x 7000 (14) 34.1 / 46
-//   eight: 3 x 8 x 113 18.9 / 13.7, 3 x 8 x 4799 (4) 29.4 / 19.8, 8 x 8 x 4000 (8) 35.1 / 29.4, 8 x 8 x 8000 (16) 45.4 / 46.1
-//   2-bit codes: 1 x 32 x 2000 20.1 / 13.8, 6 x 32 x 2000 26.1 / 21.8, 12 x 16 x 2000 27.7 / 22.9, 2 x 8 x 8664 22.9 / 20.6,
-//     8 x 8 x 6000 30.9 / 26.6, 8 x 8 x 4000 with eight query heads 31.0 / 26.1
+//   four: 1 x 8 x 603 21.4 / 12.1, 28 x 8 x 936 (7) 23.6 / 19.0, 8 x 8 x 6000 (12) 32.3 / 28.1, 8 x 8 x 7000 (14) 34.1 / 46
+//   eight: 3 x 8 x 113 18.6 / 11.2, 3 x 8 x 4799 (4) 29.0 / 17.0, 8 x 8 x 4000 (8) 33.3 / 24.9, 8 x 8 x 8000 (16) 45.4 / 46.1
+//   2-bit codes: 1 x 32 x 2000 17.8 / 11.6, 6 x 32 x 2000 24.7 / 21.9, 12 x 16 x 2000 26.6 / 23.2, 2 x 8 x 8664 21.2 / 17.3,
+//     8 x 8 x 6000 30.6 / 26.6, 8 x 8 x 4000 with eight query heads 29.0 / 23.9
+// (The sizes beyond the line, of 14 and 16 waves with 128 channels, and the two paragraphs below: before the second launch read ahead, and with
+// the values behind the keys.)
 // Beyond 16 waves of wide heads the launch takes two rounds or more, and the line is a cautious one: up to 24 workgroups
 // smaller than the CU are still the faster ones, by 32 they are not.  step_segments_kernel / this in workgroups of 4,
 // 12 and 16 waves (512 channels: 8 and 16): 256 channels, 5 x 8 x 8000 (20) 47.0 / 43.2, 44.3, 51.5, 6 x 8 x 8000 (24) 47.5
@@ -3617,7 +3625,7 @@ static int forward_qk_impl(const void *q, void *k_cache, const void *k_new, void
         seg.row_pitch = ld;
     if (D == 128 && (GQ > 1 || bits != 4 || mfma_for_mha())) {
         const bool pair = gqa_pair(BH, seg.nseg);
-        if (GQ <= 4 && !pair) // eight query heads per KV head may fall back to 8-wave workgroups
+        if (GQ <= 4 && !pair)
             plan_gqa(seg, BH, T, GQA_SKEW_QK);
         ADKV_DISPATCH_GQ(qk_gqa_kernel, true, (const h1 *)q, (uint4 *)k_cache, (const h1 *)k_new,
                          (h1 *)logits, (const h1 *)zp, (const h1 *)sc, (const h1 *)alpha,

@@ -541,9 +541,9 @@ __global__ __launch_bounds__(256) void step_combine_kernel(
             raw[i] = *reinterpret_cast<const uint4 *>(logits + row * pitch + t0 + i * 512);
     }
     // What else a wave reads travels meanwhile: the mask, or its share of the first AHEAD segments' partial outputs.  (Behind the
-    // reductions it was a second trip to memory: steps of 1 x 8 KV heads x 16000 tokens with four query heads 15.6 us instead of 14.5, 10 x 8 x
-    // 9000 with eight 55.6 instead of 54.0, 6 x 8 x 9000 33.5 instead of 32.8, 4 x 8 x 8190 of 256 channels 32.8 instead of 32.5.  Only what is there
-    // is read: rows of three segments read four, and tokens behind the row's end, 0.4 us more for 64 x 32 x 663 with a mask.)
+    // reductions it was a second trip to memory: steps of 1 x 8 KV heads x 16000 tokens with four query heads 15.4 us instead of 14.4, 6 x 8 x
+    // 9000 33.7 instead of 33.1; 10 x 8 x 9000 with eight (55 to 58) and 4 x 8 x 8190 of 256 channels (29.5) are the same either way.  Only
+    // what is there is read: rows of three segments read four, and tokens behind the row's end, 0.4 us more for 64 x 32 x 663 with a mask.)
     constexpr int AHEAD = 4;
     const MaskRow<true> mrow = mk.of<true>((unsigned)row, n);
     float add[VECS][8] = {};

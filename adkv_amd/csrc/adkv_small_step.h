@@ -21,7 +21,9 @@ namespace adkv {
 constexpr int SMALL_ROW = 3 * 64 * SM_VEC; // longest row of logits: three vectors per lane
 
 // Units of eight tokens that a values' wave holds: four registers each, of 256 / 168 / 128 with two / three / four waves per SIMD.
-// (With three segments 24 units fit as well, and keep the keys waiting: 1 x 32 x 603 12.2 us, with 16 11.9.)
+// (With three segments 24 units fit as well, and keep the keys waiting where the last segment is a part of one: 1 x 32 x 603 11.0 us, with 16
+// 10.7, 4 x 32 x 650 11.7 / 11.5.  Three whole ones gain from them, 2 x 8 x 768 12.7 / 13.6; 8 x 32 x 700 13.5 / 13.6, 5 x 40 x 700 12.8 / 13.0,
+// 1 x 32 x 520 10.5 / 10.7.)
 template <int SEGS> constexpr int small_ahead() { return SEGS == 1 ? 32 : SEGS == 2 ? 24 : SEGS == 3 ? 16 : 8; }
 
 template <int SEGS>

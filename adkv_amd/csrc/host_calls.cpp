@@ -1,7 +1,7 @@
 // The library calls of an attention layer, and of the fp32 quantiser, from Python without Python: rotary embedding,
-// attention of one token, quantising of new tokens.  On few sequences a step is over on the device in some 20 us,
+// attention of one token, quantising of new tokens.  On few sequences a step is over on the device in 10 to 20 us,
 // and the checks, views, allocations and argument conversions of the Python functions took twice that on the host
-// (1 x 32 heads x 603 tokens: 38.2 us per step, now 21.0 and bound by the device).
+// (1 x 32 heads x 603 tokens with its rotary embedding: 38.2 us per step in Python, now 13.1, as long as the device is busy with it).
 //
 // Each function here takes exactly the arguments that need nothing done to them first (plain device tensors
 // of one current device, of the right shapes, dtypes and layouts, a workspace that is large enough) and
